@@ -1,0 +1,98 @@
+"""The wide context-encoding GEMM (gemm_wide_kernel, gemm_wide16_kernel) at the edges of its tiles, K-steps and K-slices, for every weight type;
+and, with the epilogues of the layer stacks, against the 128 x 128 kernel.  Products of bf16 activations with bf16, e4m3 or int8 weights are
+exact in fp32, so two runs differ by their summation order alone."""
+import os
+import subprocess
+import sys
+
+import pytest
+import torch
+
+from oracle.quant import dequantize_weight, quantize_weight
+from tests.test_ops_gpu import WD, dev, quantize_on_device
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from vllm_neuron_amd import _native
+    _native.load_library()
+    return _native
+
+
+# one, two and three K-steps (fewer than the ring has stages); a ring's length and one more; slices of uneven length (5 and 11 K-steps over 2 .. 10
+# slices); rows and columns one tile more than a block, one row short of it, a single 16-row tile behind the last block
+@pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
+@pytest.mark.parametrize("M,N,K", [(129, 32, 64), (255, 272, 128), (257, 528, 192), (300, 272, 320), (385, 256, 704), (130, 8208, 2112),
+                                   (33, 4112, 4224), (100, 2064, 8640), (513, 1040, 1088), (1100, 6160, 576), (2031, 1296, 1984)])
+def test_edges_of_the_wide_gemm(lib, wd, M, N, K):
+    g = torch.Generator().manual_seed(M + N + K)
+    w = torch.randn(N, K, generator=g) * 0.05
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    bias = torch.randn(N, generator=g) * 0.1
+    tiled, scale = quantize_on_device(lib, w, wd, "per_channel_symmetric")
+    wq = w.to(torch.bfloat16).float() if wd == "bf16" else dequantize_weight(*quantize_weight(w, wd, "per_channel_symmetric"))
+    ref = (x.float() @ wq.t()).double() if M * N * K > 1 << 31 else x.double() @ wq.double().t()
+    ref += bias.double()
+    y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    xd, bd = dev(x), dev(bias)
+    lib.check(lib.load_library().mi_op_qlinear(xd.data_ptr(), M, tiled.data_ptr(), scale.data_ptr(), bd.data_ptr(), N, K, WD[wd], y.data_ptr(), 8, None))
+    torch.cuda.synchronize()
+    err = (y.cpu().double() - ref).abs().max().item()
+    tol = 2e-5 * ref.abs().max().item() + 1e-5 * (K ** 0.5)     # as the other linear tests: fp32 sums in another order
+    assert err < tol, (err, tol)
+
+
+_CHILD = r"""
+import sys, torch
+sys.path.insert(0, %(root)r)
+from vllm_neuron_amd._native import NativeModel
+from vllm_neuron_amd.models import config_from_dict, fill_sizes
+from tests.helpers import prefill_inputs
+out = sys.argv[1]
+dense = {"kind": "dense", "ff": 1200}
+att = {"heads": 8, "kv_heads": 2, "dim": 64, "vdim": 64, "mask": {"size": 256}, "scale": 0.125}
+common = {"width": 500, "vocab": 1010, "norm": {"eps": 1e-5}}
+designs = {
+    "vimesun": {"architecture": "Vimesun", **common, "layers": [{"type": "attention", "mixer": att, "mlp": dense}] * 2, "residual_mult": 0.5,
+                "max_positions": 1024},
+    "rapodra": {"architecture": "Rapodra", **common, "norm": {"eps": 1e-5, "groups": 4}, "canon": {"taps": 4}, "logit_softcap": 30.0, "layers": [
+        {"type": "latent_attention", "mixer": {"heads": 4, "dim": 64, "vdim": 64, "kv_rank": 192, "mask": {"size": 256}, "scale": 0.125},
+         "mlp": dict(dense, limit=7.0)}] * 2},
+    "nusovik": {"architecture": "Nusovik", **common, "embedding": {"scale": 1.0}, "logit_scale": 1.0, "layers": [{"type": "parallel", "mixer": {
+        "left": dict(att, bias_max=128), "right": {"heads": 8, "vdim": 64, "state": 64, "groups": 1, "norm_groups": 1, "conv": 4},
+        "left_scale": 1.0, "right_scale": 1.0}, "mlp": dense}] * 2},
+}
+g, res = torch.Generator().manual_seed(5), {}
+for name, config in designs.items():
+    c = config_from_dict(config)
+    fill_sizes(c, lambda n: (32, 500))
+    m = NativeModel(stack=dict(c.stack, compute_dtype=1), num_blocks=65, block_size=16, max_num_seqs=4, max_model_len=1024, device_id=0,
+                    use_graphs=1, ctx_buckets=[1024])
+    m.init_synthetic_weights(1, 0.05)
+    m.finalize()
+    for n in (40, 150, 300, 777):
+        prompt = torch.randint(0, 1010, (n,), generator=g).tolist()
+        inp = prefill_inputs(prompt, list(range(1, 2 + n // 16)), 16, 1024)
+        res[name + str(n)] = m.forward(**inp).float().clone()
+        print(name, n, flush=True)
+    m.close()
+torch.save(res, out)
+print("CHILD_OK", flush=True)
+"""
+
+
+def test_stack_epilogues_agree_with_the_128x128_kernel(tmp_path):
+    """Squared relu, clipped gate, soft cap, keys and values by head; widths that are no multiple of a tile.  The switch is read once per process."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    got = {}
+    for wide in ("0", "1"):
+        out = str(tmp_path / f"logits_{wide}.pt")
+        r = subprocess.run([sys.executable, "-c", _CHILD % {"root": root}, out], env=dict(os.environ, MI355X_GEMM_WIDE=wide), capture_output=True,
+                           text=True, timeout=300)
+        assert r.returncode == 0 and "CHILD_OK" in r.stdout, (r.stdout[-1500:], r.stderr[-1500:])
+        got[wide] = torch.load(out, weights_only=True)
+    for k, want in got["0"].items():
+        d = got["1"][k] - want
+        assert torch.isfinite(d).all() and d.pow(2).mean().sqrt() < 0.02 * want.std(), k    # the bar of the other dispatch test

@@ -69,7 +69,7 @@ int launch_gemv(const LinearW& w, int M, int pro, const ProArgs& p, int epi, con
 int launch_gemm(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e,
                 hipStream_t s, float* splitk_ws = nullptr, size_t splitk_ws_bytes = 0, SlabSum* defer = nullptr);
 int launch_splitk_flush(const SlabSum& sl, const float* resid_in, float* out, int ld_out, hipStream_t s);
-// the wide-N LDS-DMA variant of launch_gemm (1-byte weights); launch_gemm picks it by size
+// the wide-N LDS-DMA variant of launch_gemm; launch_gemm picks it by size
 int launch_gemm_wide(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
                      float* splitk_ws = nullptr, size_t splitk_ws_bytes = 0, SlabSum* defer = nullptr, int force_bm = 0,
                      int force_ks = 0);   // force_*: tests (token block 128 / 256, K slices)

@@ -227,70 +227,97 @@ static int launch_gemm_wd(const LinearW& w, int T, const uint16_t* x, int ldx, i
 
 
 // =====================================================================================
-// GEMM, wide-N tile with an LDS-DMA ring and two wave groups half a K-step apart (context encoding, 1-byte weights)
+// GEMM, wide-N tile with an LDS-DMA ring and two wave groups half a K-step apart (context encoding)
 // =====================================================================================
-// The 128 x 128 kernel above is L1-fill bound: per 64-deep K-step a work-group pulls
-// 16 KiB of bf16 activations + 8 KiB of fp8 weights for 2.1 MFLOP.  Weights are half the bytes per
-// element of the activations, so the tile grows along N: 128 tokens x 256 weight rows = 16 + 16 KiB
-// for 4.2 MFLOP (1.5 x the flops per byte), 256 x 256 = 32 + 16 KiB for 8.4.  Eight waves as 2 (tokens) x 4 (weight
+// The 128 x 128 kernel above pulls 16 KiB of activations + 8 (16) KiB of weights per 64-deep K-step for 2.1 MFLOP.  A CU takes in 55 - 65 GB/s
+// once half of it comes from HBM (64 KiB of requests in flight, 1.2 us each; from L2 it takes 125 GB/s), so the tile grows: 128 tokens x 256
+// weight rows = 16 + 16 (32) KiB for 4.2 MFLOP, 256 x 256 = 32 + 16 (32) KiB for 8.4.  Eight waves as 2 (tokens) x 4 (weight
 // rows): activation fragments are shared by four waves, weight fragments by two.  Both operands arrive by LDS-DMA
 // (global_load_lds, 1 KiB per wave-instruction: the weight tiles land lane-linear = fragment
 // order; the activation rows land in the XOR-swizzled image of the kernel above, the swizzle being
-// applied to the per-lane SOURCE address) into a ring of three stages: two K-steps are in
-// flight while one is multiplied, retired by counted vmcnt waits in front of raw barriers -- no ordinary global
-// load in the loop, so hipcc has nothing to drain.  Round 3: a wave's K-step is a READ phase (fragments LDS -> registers,
-// weight codes decoded on the way) and a MULTIPLY phase (MFMAs only), and the two waves of a SIMD are in opposite phases
-// (see "Schedule" in the kernel): gate|up at 2048 tokens 436.6 -> 373.4 us (1.10 -> 1.29 PF/s), down 220 -> 198 us.
-constexpr int kWideBN = 256, kWideWBytes = 16 * 1024, kWideStages = 3;
+// applied to the per-lane SOURCE address) into a ring of stages: all but the one being multiplied are in
+// flight, retired by counted vmcnt waits in front of raw barriers -- no ordinary global
+// load in the loop, so hipcc has nothing to drain.  A wave's K-step is a READ phase (fragments LDS -> registers, then the requests of a later
+// K-step) and a MULTIPLY phase (MFMAs, the weight codes decoded between them), and the two waves of a SIMD are in opposite phases
+// (see "Schedule" in the kernel).
+// What it holds on full grids (gate|up of the 8B model, 2031 tokens): bf16 1.22, fp8 1.27, int8 1.22 PF/s (1.16 before the codes were decoded
+// between the MFMAs), where a library product of 8192^3 in bf16 runs at 1.28 on this card; 128-token blocks 1.13 / 1.18 / 1.05.
+constexpr int kWideBN = 256;
+template <int WD> constexpr int kWideWBytes = (WD == MI_W_BF16 ? 32 : 16) * 1024;   // 256 weight rows of a 64-deep K-step
+// as many stages as the LDS holds: 144 or 160 KiB
+template <int WD, int BM> constexpr int kWideStages = 160 * 1024 / (kWideWBytes<WD> + BM * 128);
 
+// Waits until at most the youngest min(left, MOST) K-steps' DMAs (PER each) of this wave are in flight.
+template <int PER, int MOST>
+__device__ __forceinline__ void wait_dma(int left) {
+  if (left >= MOST) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER * MOST) : "memory");
+  else if constexpr (MOST > 0) wait_dma<PER, MOST - 1>(left);
+}
+
+// The tile of this work-group.  Work-group b runs on XCD b % 8: an XCD takes an eighth of the tiles, one after the other with the token
+// blocks of a weight slab in a row, so that a slab comes into its L2 once.  (Every eighth slab to an XCD, as in gemm_kernel, left the XCDs
+// up to a slab apart: 44 slabs of 11 token blocks put 66 work-groups on the 32 CUs of four of them, three rounds in place of two.)
+template <int BM>
+__device__ __forceinline__ bool wide_tile(int T, int NT, int& m0, int& nt0) {
+  const int mtiles = ceil_div(T, BM), tiles = mtiles * ceil_div(NT, kWideBN / 16), per = ceil_div(tiles, 8);
+  const int seq = blockIdx.x >> 3, t = (blockIdx.x & 7) * per + seq;
+  if (seq >= per || t >= tiles) return false;
+  nt0 = t / mtiles * (kWideBN / 16);
+  m0 = t % mtiles * BM;
+  return true;
+}
+// the K-steps of grid.z slice blockIdx.z: equal ones, the last may be shorter (the launch leaves none empty)
+template <bool SPLIT>
+__device__ __forceinline__ void wide_slice(int K, int& ks0, int& nks) {
+  const int all = K / 64, per = SPLIT ? ceil_div(all, (int)gridDim.z) : all;
+  ks0 = SPLIT ? (int)blockIdx.z * per : 0;
+  nks = min(per, all - ks0);
+}
 
 // BM = 128: each wave 64 x 64 (64 accumulator registers).  BM = 256: each 128 x 64 (128 accumulator registers, 246 VGPRs
 // with the decoded fragments of one K-step).
-// SPLIT: grid.z K-slices write raw fp32 accumulators to slab[z][m][n] (see gemm_a8_kernel); K / 64 is a multiple of grid.z.
+// SPLIT: grid.z K-slices write raw fp32 accumulators to slab[z][m][n] (see gemm_a8_kernel).
 template <int WD, int EPI, int BM, bool SPLIT>
 __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict__ W, int NT, int KT, int T, int K,
                                                         const uint16_t* __restrict__ x, int ldx, EpiArgs e,
                                                         float* __restrict__ slab) {
-  static_assert(WD != MI_W_BF16, "1-byte weight tiles (64 k per tile)");
-  static_assert(BM == 128 || BM == 256, "token block");
-  // waves as 2 (tokens) x 4 (weight rows), each MT 16-token tiles x 4 16-row weight tiles.  (4 x 2 waves of 64 x 128 read
-  // 16 instead of 20 KiB of fragments per K-step but decode every weight code four times instead of twice: measured slower,
-  // 401 against 387 us on the gate-up shape -- the decode, not the LDS read, is what the schedule has to hide.)
+  static_assert(BM == 128 || (BM == 256 && WD != MI_W_BF16), "token block");   // 256 tokens of bf16 weights: gemm_wide16_kernel
+  // waves as 2 (tokens) x 4 (weight rows), each MT 16-token tiles x 4 16-row weight tiles (4 x 2 waves would read 16 instead of 20 KiB of
+  // fragments per K-step but decode every weight code four times instead of twice)
   constexpr int MT = BM / 32;                 // 16-token tiles per wave
   constexpr int WM = 2, NTW = 4;
   constexpr int XP = BM / 64;                 // 8-row activation pieces per wave and stage
-  constexpr int kStage = kWideWBytes + BM * 128;
-  constexpr int kDma = 2 + XP;                // DMAs per wave and stage
+  constexpr int WP = kWideWBytes<WD> / 8192;  // 1 KiB weight tiles per wave and stage
+  constexpr int WPK = WP / 2;                 // weight tiles per 16 rows and K-step
+  constexpr int kStages = kWideStages<WD, BM>, kStage = kWideWBytes<WD> + BM * 128;
+  constexpr int kDma = WP + XP;               // DMAs per wave and stage
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int g = lane >> 4, c = lane & 15;
   const int wm = wave % WM, wn = wave / WM;
-  // XCD-aware tile order (see gemm_a8_kernel): an XCD walks all token blocks of a weight slab back to back
-  const int mtiles = ceil_div(T, BM), ntiles = ceil_div(NT, kWideBN / 16);
-  const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
-  const int mblk = seq % mtiles, nblk = (seq / mtiles) * 8 + xcd;
-  if (nblk >= ntiles) return;
-  const int m0 = mblk * BM, ntb = nblk * (kWideBN / 16);
-  const int nks = SPLIT ? K / 64 / (int)gridDim.z : K / 64;     // this slice's K-steps, from K-step ks0 on
-  const int ks0 = SPLIT ? (int)blockIdx.z * nks : 0;
+  int m0, ntb;
+  if (!wide_tile<BM>(T, NT, m0, ntb)) return;
+  int ks0, nks;                               // this slice's K-steps, from K-step ks0 on
+  wide_slice<SPLIT>(K, ks0, nks);
 
   // this lane's DMA sources: wave w brings weight tiles 2w, 2w + 1 of the work-group's 16 (fragment
   // order) and XP 8-row pieces of the activation tile
   const uint4* wsrc[2];
   const uint16_t* xsrc[XP];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) wsrc[i] = W + ((size_t)min(ntb + 2 * wave + i, NT - 1) * KT + ks0) * 64 + lane;
+  for (int i = 0; i < 2; ++i) wsrc[i] = W + ((size_t)min(ntb + 2 * wave + i, NT - 1) * KT + ks0 * WPK) * 64 + lane;
 #pragma unroll
   for (int i = 0; i < XP; ++i) {
     const int r = (XP * wave + i) * 8 + (lane >> 3), sl = lane & 7;
     xsrc[i] = x + (size_t)min(m0 + r, T - 1) * ldx + (size_t)ks0 * 64 + ((sl ^ xs_swz<WD>(r)) * 8);   // LDS slot sl of row r holds chunk sl ^ swz(r)
   }
-  auto issue = [&](int ks) {
-    unsigned char* st = smem + (ks % kWideStages) * kStage;
+  auto issue = [&](int ks, int stage) {
+    unsigned char* st = smem + stage * kStage;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) glds16(wsrc[i] + (size_t)ks * 64, st + (2 * wave + i) * 1024);
+    for (int i = 0; i < WP; ++i)   // tile (row tile i / WPK, k tile i % WPK)
+      glds16(wsrc[i / WPK] + ((size_t)ks * WPK + i % WPK) * 64, st + (WP * wave + i) * 1024);
 #pragma unroll
-    for (int i = 0; i < XP; ++i) glds16(xsrc[i] + (size_t)ks * 64, st + kWideWBytes + (XP * wave + i) * 1024);
+    for (int i = 0; i < XP; ++i) glds16(xsrc[i] + (size_t)ks * 64, st + kWideWBytes<WD> + (XP * wave + i) * 1024);
   };
 
   f32x4_t acc[NTW][MT];
@@ -299,7 +326,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
 #pragma unroll
     for (int j = 0; j < MT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  // Schedule.  A K-step of a wave is two phases: READ (its fragments, 20 KiB at BM = 256, from LDS into registers, the weight codes decoded to bf16 on the way) and MULTIPLY
+  // Schedule.  A K-step of a wave is two phases: READ (its fragments, 20 KiB at BM = 256, from LDS into registers) and MULTIPLY
   // (2 NTW MT MFMAs from registers).  With one barrier per K-step every wave is in the same phase at the same time, the two waves
   // of a SIMD included, and LDS-read time and MFMA time add up: 1.7 us per K-step at BM = 256 against 1.0 us of MFMAs.  Here
   // the two wave groups (waves 0-3 / 4-7 = the two waves of every SIMD) run half a K-step apart -- group 1 executes one
@@ -307,58 +334,76 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
   //     physical barrier:      P0        P1        P2        P3        P4  ...
   //     group 0 (waves 0-3):   | READ 0  | MUL 0   | READ 1  | MUL 1   | ...
   //     group 1 (waves 4-7):   |         | READ 0  | MUL 0   | READ 1  | MUL 1 ...
-  // Stage k is read in [P2k, P2k+2]; K-step k + 2 goes into the stage of K-step k - 1 (read until P2k), requested by every wave
-  // behind its top barrier of iteration k: two K-steps ahead of its first read, as before.  A wave waits for ITS pieces of a
+  // Stage k is read in [P2k, P2k+2]; K-step k + kStages - 1 goes into the stage of K-step k - 1 (read until P2k), requested by every wave
+  // behind its top barrier of iteration k, kStages - 1 K-steps ahead of its first read.  A wave waits for ITS pieces of a
   // stage before the barrier in front of the stage's first read by anyone (group 0: its top barrier; group 1: its second one).
   const int grp = __builtin_amdgcn_readfirstlane(wave >> 2);
-  issue(0);
-  if (nks > 1) issue(1);
+#pragma unroll
+  for (int k = 0; k + 1 < kStages; ++k)
+    if (k < nks) issue(k, k);
   if (grp == 1) {   // its pieces of stage 0 are in before P0
-    if (nks > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kDma) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    wait_dma<kDma, kStages - 2>(nks - 1);
     __builtin_amdgcn_s_barrier();           // P0
   }
+  int cur = 0, fill = kStages - 1;          // the stages of K-step ks and of K-step ks + kStages - 1
   for (int ks = 0; ks < nks; ++ks) {
-    if (grp == 0) {   // own pieces of stage ks (at most those of stage ks + 1 are younger)
-      if (ks + 1 < nks) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kDma) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
+    if (grp == 0) wait_dma<kDma, kStages - 2>(nks - 1 - ks);   // own pieces of stage ks
     __builtin_amdgcn_s_barrier();           // group 0: P2ks | group 1: P2ks+1 -- either way nobody reads stage ks - 1 any more
-    if (ks + 2 < nks) issue(ks + 2);
-    const unsigned char* st = smem + (ks % kWideStages) * kStage;
-    const uint4* xs = reinterpret_cast<const uint4*>(st + kWideWBytes);
-    u32x4_t b0[MT], b1[MT];
-    bf16x8_t a0[NTW], a1[NTW];
+    const unsigned char* st = smem + cur * kStage;
+    const uint4* xs = reinterpret_cast<const uint4*>(st + kWideWBytes<WD>);
+    u32x4_t b0[MT], b1[MT], w0[NTW], w1[NTW];
+#pragma unroll
+    for (int i = 0; i < NTW; ++i) {
+      const u32x4_t* w = reinterpret_cast<const u32x4_t*>(st + (wn * NTW + i) * (WPK * 1024) + lane * 16);
+      w0[i] = w[0];
+      if constexpr (WD == MI_W_BF16) w1[i] = w[64];
+    }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const int r = wm * (BM / 2) + mt * 16 + c;
-      b0[mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + ((2 * g) ^ xs_swz<WD>(r))]);
-      b1[mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + ((2 * g + 1) ^ xs_swz<WD>(r))]);
+      const int ch0 = WD == MI_W_BF16 ? g : 2 * g, ch1 = WD == MI_W_BF16 ? 4 + g : 2 * g + 1;
+      b0[mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + (ch0 ^ xs_swz<WD>(r))]);
+      b1[mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + (ch1 ^ xs_swz<WD>(r))]);
     }
-#pragma unroll
-    for (int i = 0; i < NTW; ++i) {   // decoded here, in the READ phase, while the SIMD's other wave multiplies: the MULTIPLY phase is MFMAs only
-      const u32x4_t w4 = *reinterpret_cast<const u32x4_t*>(st + (wn * NTW + i) * 1024 + lane * 16);
-      a0[i] = decode8<WD>(w4[0], w4[1]);
-      a1[i] = decode8<WD>(w4[2], w4[3]);
-    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (ks + kStages - 1 < nks) issue(ks + kStages - 1, fill);
+    __builtin_amdgcn_sched_barrier(0);
+    cur = cur + 1 == kStages ? 0 : cur + 1;
+    fill = fill + 1 == kStages ? 0 : fill + 1;
     // the fragments are in registers (the empty asm takes them as operands: the compiler's wait for the reads sits in front of it)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) { asm volatile("" : "+v"(b0[mt])); asm volatile("" : "+v"(b1[mt])); }
-#pragma unroll
-    for (int i = 0; i < NTW; ++i) { asm volatile("" : "+v"(a0[i])); asm volatile("" : "+v"(a1[i])); }
-    if (grp == 1 && ks + 1 < nks) {   // own pieces of stage ks + 1: group 0 reads it behind the next barrier
-      if (ks + 2 < nks) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kDma) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    for (int i = 0; i < NTW; ++i) {
+      asm volatile("" : "+v"(w0[i]));
+      if constexpr (WD == MI_W_BF16) asm volatile("" : "+v"(w1[i]));
     }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) { asm volatile("" : "+v"(b0[mt])); asm volatile("" : "+v"(b1[mt])); }
+    if (grp == 1 && ks + 1 < nks) wait_dma<kDma, kStages - 2>(nks - 2 - ks);   // own pieces of stage ks + 1: group 0 reads it behind the next barrier
     __builtin_amdgcn_s_barrier();           // group 0: P2ks+1 | group 1: P2ks+2
     __builtin_amdgcn_sched_barrier(0);
+    // the codes of weight tile i + 1 are decoded between the MFMAs of tile i, whose 16 cycles leave room for three vector instructions each
+    u32x4_t a[2], an[2];
+    auto piece = [&](const u32x4_t& w, int q) { const uint32_t v = w[q >> 1]; return decode2<WD>(v, q & 1); };
+    if constexpr (WD != MI_W_BF16) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) a[q >> 2][q & 3] = piece(w0[0], q);
+    }
 #pragma unroll
     for (int i = 0; i < NTW; ++i) {
+      if constexpr (WD == MI_W_BF16) { a[0] = w0[i]; a[1] = w1[i]; }
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        acc[i][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[i], __builtin_bit_cast(bf16x8_t, b0[mt]), acc[i][mt], 0, 0, 0);
-        acc[i][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[i], __builtin_bit_cast(bf16x8_t, b1[mt]), acc[i][mt], 0, 0, 0);
+      for (int m2 = 0; m2 < 2 * MT; ++m2) {   // both halves of a K-step one after the other: two MFMAs in a row never meet in an accumulator
+        const int h = m2 / MT, mt = m2 % MT;
+        acc[i][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[h]), __builtin_bit_cast(bf16x8_t, h ? b1[mt] : b0[mt]), acc[i][mt], 0, 0, 0);
+        if constexpr (WD != MI_W_BF16) {
+          if (i + 1 < NTW) {
+#pragma unroll
+            for (int q = m2 * 4 / MT; q < (m2 + 1) * 4 / MT; ++q) an[q >> 2][q & 3] = piece(w0[i + 1], q);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
+      if constexpr (WD != MI_W_BF16) { a[0] = an[0]; a[1] = an[1]; }
     }
   }
   if (grp == 0) __builtin_amdgcn_s_barrier();   // the barrier group 1 executed first
@@ -380,67 +425,199 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
   }
 }
 
+// The same for bf16 weights at 256 tokens x 256 weight rows.  A 64-deep stage of it is 64 KiB, and the LDS holds two; the stagger
+// needs a third.  So a K-step is 32 deep (one weight tile per 16 rows; 32 MFMAs a wave), the weights ride in four stages of 16 KiB, and the
+// activations, whose rows are fetched 128 bytes at a time, in three of 64-deep pairs of K-steps (32 KiB): 160 KiB.  K-step s requests the weights
+// of s + 3 and one half of the rows of the pair behind the next, four DMAs a wave, so what K-step s reads was requested by K-step s - 3 at
+// the latest and eight younger DMAs stay in flight.
+template <int EPI, bool SPLIT>
+__global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restrict__ W, int NT, int KT, int T, int K,
+                                                          const uint16_t* __restrict__ x, int ldx, EpiArgs e,
+                                                          float* __restrict__ slab) {
+  constexpr int BM = 256, MT = 8, WM = 2, NTW = 4, kW = 16 * 1024, kX = 32 * 1024, kXs = 4 * kW;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int g = lane >> 4, c = lane & 15;
+  const int wm = wave % WM, wn = wave / WM;
+  int m0, ntb;
+  if (!wide_tile<BM>(T, NT, m0, ntb)) return;
+  int ks0, nks;
+  wide_slice<SPLIT>(K, ks0, nks);
+  const int s0 = 2 * ks0, n = 2 * nks;        // this slice's 32-deep K-steps
+
+  const uint4* wsrc[2];
+  const uint16_t* xsrc[4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) wsrc[i] = W + ((size_t)min(ntb + 2 * wave + i, NT - 1) * KT + s0) * 64 + lane;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = (4 * wave + i) * 8 + (lane >> 3), sl = lane & 7;
+    xsrc[i] = x + (size_t)min(m0 + r, T - 1) * ldx + (size_t)s0 * 32 + ((sl ^ xs_swz<MI_W_BF16>(r)) * 8);
+  }
+  auto issue_w = [&](int s) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) glds16(wsrc[i] + (size_t)s * 64, smem + (s & 3) * kW + (2 * wave + i) * 1024);
+  };
+  auto issue_x = [&](int p, int half, int stage) {   // half of this wave's rows of pair p
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int q = 2 * half + i;
+      glds16((half ? xsrc[2 + i] : xsrc[i]) + (size_t)p * 64, smem + kXs + stage * kX + (4 * wave + q) * 1024);
+    }
+  };
+  // own pieces of K-step s are in: the requests of the last two K-steps may be out, fewer of them at the end
+  auto wait_for = [&](int s) {
+    const int left = n - 1 - s;
+    if (left >= 3) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    else if (left == 2) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+    else if (left == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  };
+
+  f32x4_t acc[NTW][MT];
+#pragma unroll
+  for (int i = 0; i < NTW; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  const int grp = __builtin_amdgcn_readfirstlane(wave >> 2);
+  issue_x(0, 0, 0);
+  issue_x(0, 1, 0);
+  issue_w(0);
+  issue_w(1);
+  if (n > 2) {
+    issue_x(1, 0, 1);
+    issue_w(2);
+    issue_x(1, 1, 1);
+  }
+  if (grp == 1) {
+    wait_for(0);
+    __builtin_amdgcn_s_barrier();           // P0
+  }
+  auto step = [&](int s, int half, int xcur, int xfill) {
+    if (grp == 0) wait_for(s);
+    __builtin_amdgcn_s_barrier();           // group 0: P2s | group 1: P2s+1
+    const unsigned char* st = smem + (s & 3) * kW;
+    const uint4* xs = reinterpret_cast<const uint4*>(smem + kXs + xcur * kX);
+    u32x4_t b[MT], a[NTW];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int r = wm * (BM / 2) + mt * 16 + c;
+      b[mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + ((4 * half + g) ^ xs_swz<MI_W_BF16>(r))]);
+    }
+#pragma unroll
+    for (int i = 0; i < NTW; ++i) a[i] = *reinterpret_cast<const u32x4_t*>(st + (wn * NTW + i) * 1024 + lane * 16);
+    __builtin_amdgcn_sched_barrier(0);
+    if (s + 3 < n) issue_w(s + 3);
+    if ((s >> 1) + 2 < (n >> 1)) issue_x((s >> 1) + 2, half, xfill);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(b[mt]));
+#pragma unroll
+    for (int i = 0; i < NTW; ++i) asm volatile("" : "+v"(a[i]));
+    if (grp == 1 && s + 1 < n) wait_for(s + 1);
+    __builtin_amdgcn_s_barrier();           // group 0: P2s+1 | group 1: P2s+2
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NTW; ++i)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+        acc[i][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[i]), __builtin_bit_cast(bf16x8_t, b[mt]), acc[i][mt], 0, 0, 0);
+  };
+  int xcur = 0, xfill = 2;
+  for (int s = 0; s < n; s += 2) {
+    step(s, 0, xcur, xfill);
+    step(s + 1, 1, xcur, xfill);
+    xcur = xcur == 2 ? 0 : xcur + 1;
+    xfill = xfill == 2 ? 0 : xfill + 1;
+  }
+  if (grp == 0) __builtin_amdgcn_s_barrier();   // the barrier group 1 executed first
+#pragma unroll
+  for (int i = 0; i < NTW; ++i) {
+    const int nt = ntb + wn * NTW + i;
+    if (nt >= NT) continue;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int m = m0 + wm * (BM / 2) + mt * 16 + c;
+      if (m >= T) continue;
+      if constexpr (SPLIT) {
+        *reinterpret_cast<float4*>(slab + ((size_t)blockIdx.z * T + m) * (NT * 16) + nt * 16 + g * 4) =
+            make_float4(acc[i][mt][0], acc[i][mt][1], acc[i][mt][2], acc[i][mt][3]);
+      } else {
+        epilogue<EPI>(e, m, nt * 16 + g * 4, acc[i][mt]);
+      }
+    }
+  }
+}
+
+template <int WD, int EPI, int BM, bool SPLIT>
+static auto gemm_wide_fn() {
+  if constexpr (WD == MI_W_BF16 && BM == 256) return gemm_wide16_kernel<EPI, SPLIT>;
+  else return gemm_wide_kernel<WD, EPI, BM, SPLIT>;
+}
+
 template <int WD, int BM>
 static int launch_gemm_wide_bm(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
                                int KS, float* splitk_ws, SlabSum* defer) {
-  const int NT = w.N / 16, KT = w.K / 64;
-  const int mtiles = ceil_div(T, BM), ntiles = ceil_div(w.N, kWideBN);
-  dim3 grid(8 * mtiles * ceil_div(ntiles, 8), 1, KS);
+  const int NT = w.N / 16, KT = w.K / tile_k(WD);
+  dim3 grid(8 * ceil_div(ceil_div(T, BM) * ceil_div(w.N, kWideBN), 8), 1, KS);
   const uint4* W = reinterpret_cast<const uint4*>(w.w);
-  constexpr int lds = kWideStages * (kWideWBytes + BM * 128);
+  constexpr int lds = WD == MI_W_BF16 && BM == 256 ? 160 * 1024 : kWideStages<WD, BM> * (kWideWBytes<WD> + BM * 128);
 #define MI_GW(EPI_) \
   do { \
     if (KS == 1) { \
-      MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_wide_kernel<WD, EPI_, BM, false>), lds)); \
-      hipLaunchKernelGGL((gemm_wide_kernel<WD, EPI_, BM, false>), grid, dim3(512), lds, s, W, NT, KT, T, w.K, x, ldx, e, nullptr); \
+      const auto fn = gemm_wide_fn<WD, EPI_, BM, false>(); \
+      MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)); \
+      hipLaunchKernelGGL(fn, grid, dim3(512), lds, s, W, NT, KT, T, w.K, x, ldx, e, nullptr); \
     } else { \
-      MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_wide_kernel<WD, EPI_, BM, true>), lds)); \
-      hipLaunchKernelGGL((gemm_wide_kernel<WD, EPI_, BM, true>), grid, dim3(512), lds, s, W, NT, KT, T, w.K, x, ldx, e, splitk_ws); \
-      if (defer && EPI_ == EPI_RESID) { *defer = SlabSum{splitk_ws, KS, T, w.N, e.scale, e.bias, e.row_scale}; } \
+      const auto fn = gemm_wide_fn<WD, EPI_, BM, true>(); \
+      MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)); \
+      hipLaunchKernelGGL(fn, grid, dim3(512), lds, s, W, NT, KT, T, w.K, x, ldx, e, splitk_ws); \
+      if (defer && (EPI_ == EPI_RESID || EPI_ == EPI_F32)) { *defer = SlabSum{splitk_ws, KS, T, w.N, e.scale, e.bias, e.row_scale}; } \
       else hipLaunchKernelGGL((splitk_reduce_kernel<EPI_>), dim3(ceil_div(T * (w.N / 4), 256)), dim3(256), 0, s, splitk_ws, KS, T, w.N, e); \
     } \
   } while (0)
   if (epi == EPI_QKV) MI_GW(EPI_QKV);
   else if (epi == EPI_SWIGLU) MI_GW(EPI_SWIGLU);
   else if (epi == EPI_RESID) MI_GW(EPI_RESID);
-  else MI_GW(EPI_F32);
+  else if (epi >= EPI_RELU2) {
+    if constexpr (WD == MI_W_BF16) {
+      if (epi == EPI_RELU2) MI_GW(EPI_RELU2);
+      else if (epi == EPI_GLU_CLIP) MI_GW(EPI_GLU_CLIP);
+      else if (epi == EPI_SOFTCAP) MI_GW(EPI_SOFTCAP);
+      else MI_GW(EPI_HEADS_KV);
+    } else { set_error("gemm_wide: this epilogue is built for bf16 weights"); return MI_EINVAL; }
+  } else MI_GW(EPI_F32);
 #undef MI_GW
   MI_HIP(hipGetLastError());
   return MI_OK;
 }
-// The wide kernel runs ONE work-group per CU (96 / 144 KiB of LDS), so what decides is how full its rounds of the chip are,
-// and between the two token blocks, rounds x time per K-step (measured on full grids: 0.90 us at 128 tokens, 1.45 us at 256 --
-// twice the flops).  Measured on the Llama-8B shapes (round 3, staggered schedule; wide against the 128 x 128 kernel, us):
-//     gate|up  256 tokens: 224 work-groups of 128 tokens (one round, 88 %)   62.0 vs  73.4      512: 448 (two rounds)  115.3 vs 141.6
-//     gate|up 1024 tokens: 896 (3.5 rounds)                                 224.5 vs 227.6      QKV 1024: 192 (one round, 75 %) 66.6 vs 84.2
-//     QKV  512: 96 work-groups   64.6 vs 40.1      O / down 1024: 128   57.1 vs 40.7 / 166.6 vs 116.2 (K-split on the other side)
-//     QKV 2048: 384 (1.5 rounds, 75 %)  134.5 vs 112.4;  gate|up 2048: 403.6 at 128 tokens (7 rounds), 373.4 at 256 (3.5)
-// -> a shape is eligible with one partial round from 70 % of the CUs on or several rounds at 80 % fill; the cheapest eligible
-// (token block, K-split) runs: rounds x K-steps x time per K-step, plus, for a K-split, the slabs written and read once more
-// (~4 bytes/ns) and the launch that sums them.
-struct WidePlan { int bm, ks; };   // bm 0: not wanted
-static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd) {
+// Which token block and K-split: the cheapest of a model of the kernel, us, fitted to 113 shapes (60 .. 4000 tokens, the projections of TinyLlama,
+// Llama-8B, Qwen2.5-7B and of the layer stacks; every block and split of each timed; the choice is 1.3 % from the fastest, 18 % at worst).  The
+// kernel holds 144 - 160 KiB of LDS, i.e. ONE work-group per CU, so a launch is rounds of 32 work-groups on each of the eight XCDs: 6.5 us, and
+// a round 2.6 us of ramp and epilogue beside its K-steps.  Time per 64-deep K-step, on an almost empty and on a full chip:
+//     128 tokens: fp8 0.49 / 0.77, bf16 0.68 / 0.80, int8 0.66 / 0.88;  256 tokens: fp8 0.95 / 1.36, bf16 0.93 / 1.51, int8 0.99 / 1.43
+// A K-split writes its slabs, and a second launch sums them (0.215 us per MB both ways), or the row norm that follows reads them.
+// Against the rule before it and the 128 x 128 kernel, us: bf16 gate|up of the 8B model 1000 tokens 298 -> 200, 350 tokens 151 -> 104, 128 tokens
+// 80 -> 64; its down projection 1000 tokens 199 -> 98, 350 tokens 104 -> 62; fp8 gate|up 128 tokens 55 -> 44, 33 tokens 48 -> 36.
+struct WidePlan { int bm, ks; };   // bm 0: the shape has no plan
+static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, bool deferred) {
   int cus = 256;
-  if (device_num_cu(&cus) != MI_OK || cus < 1) cus = 256;
+  if (device_num_cu(&cus) != MI_OK || cus < 8) cus = 256;
+  static const double kStep[3][2][2] = {{{0.68, 0.80}, {0.93, 1.51}}, {{0.49, 0.77}, {0.95, 1.36}}, {{0.66, 0.88}, {0.99, 1.43}}};
   const int nks = K / 64;
   WidePlan best{0, 1};
   double best_cost = 0.;
   for (int bm = 128; bm <= 256; bm *= 2) {
-    for (int ks = 1; ks <= 8; ks *= 2) {
-      if (nks % ks != 0 || nks / ks < 8) continue;
-      if (ks > 1 && (size_t)ks * T * N * sizeof(float) > ws_bytes) continue;
-      const int wgs = ceil_div(T, bm) * ceil_div(N, kWideBN) * ks, rounds = ceil_div(wgs, cus);
-      const bool ok = wgs < cus ? wgs * 10 >= cus * 7 : wgs * 5 >= rounds * cus * 4;
-      if (!ok) continue;
-      // INT8 codes cost the READ phase ~6 x the VALU work of the fp8 hardware convert: 1.38 / 1.73 us per K-step measured on
-      // the Qwen2.5-7B shapes (gate|up at 1024 tokens 387.8 us at 128-token blocks against 303.5 on the 128 x 128 kernel;
-      // at 2048 tokens 485 at 256-token blocks against 592) -- there the wide tile must also beat what the 128 x 128 kernel
-      // holds: 0.9 PF/s on grids that keep three work-groups per CU resident, 0.65 on its K-split grids
-      const bool i8 = wd == MI_W_INT8;
-      double cost = (double)rounds * (nks / ks) * (bm == 128 ? (i8 ? 1.38 : 0.90) : (i8 ? 1.73 : 1.45));
-      if (ks > 1) cost += 4.0 + (double)(ks + 1) * T * N * 4.0 / 4.0e6 * 1.0;   // slabs out and in, the sum out
-      const double alt_pf = ceil_div(T, 128) * ceil_div(N, 128) >= 3 * cus ? 0.9e9 : 0.65e9;   // flops per us: full residency / a K-split grid
-      if (i8 && cost > 2.0 * T * N * (double)K / alt_pf) continue;
+    const int tiles = ceil_div(T, bm) * ceil_div(N, kWideBN);
+    for (int ks = 1; ks <= 10; ++ks) {
+      const int per = ceil_div(nks, ks);
+      if (ks > 1 && (per < 4 || (ks - 1) * per >= nks || (size_t)ks * T * N * sizeof(float) > ws_bytes)) continue;
+      const double fill = std::min(1.0, (double)tiles * ks / cus), *st = kStep[wd][bm / 256];
+      const int rounds = ceil_div(ceil_div(tiles, 8) * ks, std::max(1, cus / 8));
+      double cost = 6.5 + rounds * (2.6 + per * (st[0] + (st[1] - st[0]) * fill));
+      const double mb = (double)T * N * 4e-6;
+      if (ks > 1) cost += deferred ? 0.15 * ks * mb : 2.7 + 0.215 * (ks + 1) * mb;
       if (best.bm == 0 || cost < best_cost) { best = WidePlan{bm, ks}; best_cost = cost; }
     }
   }
@@ -461,31 +638,34 @@ static int gemm_wide_ks() {      // MI355X_GEMM_WIDE_KS: 1 = never split K in th
 template <int WD>
 static int launch_gemm_wide_wd(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
                                float* splitk_ws, size_t splitk_ws_bytes, SlabSum* defer, int force_bm, int force_ks) {
-  WidePlan pl = gemm_wide_plan(T, w.N, w.K, gemm_wide_ks() == 1 || !splitk_ws ? 0 : splitk_ws_bytes, w.wd);
+  WidePlan pl = gemm_wide_plan(T, w.N, w.K, gemm_wide_ks() == 1 || !splitk_ws ? 0 : splitk_ws_bytes, w.wd, defer && (epi == EPI_RESID || epi == EPI_F32));
   const int forced_bm = force_bm ? force_bm : gemm_wide_bm();
   if (forced_bm == 128 || forced_bm == 256) pl = WidePlan{forced_bm, 1};
-  if (pl.bm == 0) pl = WidePlan{ceil_div(T, 256) * ceil_div(w.N, kWideBN) >= 512 ? 256 : 128, 1};   // forced onto a shape the plan would not take
   if (force_ks) {
-    MI_CHECK(force_ks >= 1 && (w.K / 64) % force_ks == 0 && (force_ks == 1 || (splitk_ws && (size_t)force_ks * T * w.N * 4 <= splitk_ws_bytes)),
-             "gemm_wide: forced K-split must divide K / 64 and fit the workspace");
+    MI_CHECK(force_ks >= 1 && (force_ks - 1) * ceil_div(w.K / 64, force_ks) < w.K / 64 && (force_ks == 1 || (splitk_ws && (size_t)force_ks * T * w.N * 4 <= splitk_ws_bytes)),
+             "gemm_wide: forced K-split must leave no slice empty and fit the workspace");
     pl.ks = force_ks;
   }
   if (pl.bm == 256) return launch_gemm_wide_bm<WD, 256>(w, T, x, ldx, epi, e, s, pl.ks, splitk_ws, defer);
   return launch_gemm_wide_bm<WD, 128>(w, T, x, ldx, epi, e, s, pl.ks, splitk_ws, defer);
 }
-// the wide tile needs 1-byte weights
+// The 128 x 128 kernel keeps what is small on both sides: up to 128 tokens of a matrix of up to 17 M weights (33 .. 128 tokens, us: 4096 x 4096
+// fp8 16.3 / 18.4 / 19.5 against 15.8 / 18.8 / 20.9, 3584 x 3584 int8 15.3 / 17.3 / 20.9 against 16.2 / 18.8 / 22.7, 2560 x 2048 bf16
+// 12.6 / - / 17.4 against 12.1 / - / 18.1; 8448 x 2048 bf16 at 100 tokens is past it: 27.7 against 19.7), and grids of less than half the chip where there is no workspace to split K into.
 static bool gemm_wide_wanted(const LinearW& w, int T, size_t ws_bytes) {
-  if (w.wd == MI_W_BF16 || w.K % 64 != 0 || (w.N / 16) < 2) return false;
+  if (w.K % 64 != 0 || (w.N / 16) < 2) return false;
   const int mode = gemm_wide_mode();
   if (mode == 1) return true;
   if (mode == 0) return false;
-  if (T <= 128) return false;   // up to one 128-token block: the 128 x 128 kernel and its K-split (also the 33 .. 128-row decode batches)
-  return gemm_wide_plan(T, w.N, w.K, gemm_wide_ks() == 1 ? 0 : ws_bytes, w.wd).bm != 0;
+  if (T <= 128 && (int64_t)w.N * w.K <= 17000000) return false;
+  return ws_bytes > 0 || ceil_div(T, 128) * ceil_div(w.N, kWideBN) >= 128;
 }
 int launch_gemm_wide(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
                      float* splitk_ws, size_t splitk_ws_bytes, SlabSum* defer, int force_bm, int force_ks) {
   if (defer) *defer = SlabSum();
-  MI_CHECK(w.wd != MI_W_BF16 && w.K % 64 == 0 && ldx % 8 == 0, "gemm_wide: 1-byte weights, K % 64 == 0");
+  MI_CHECK(w.K % 64 == 0 && ldx % 8 == 0, "gemm_wide: K % 64 == 0");
+  if (w.wd == MI_W_BF16)
+    return launch_gemm_wide_wd<MI_W_BF16>(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer, force_bm, force_ks);
   if (w.wd == MI_W_F8E4M3)
     return launch_gemm_wide_wd<MI_W_F8E4M3>(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer, force_bm, force_ks);
   return launch_gemm_wide_wd<MI_W_INT8>(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer, force_bm, force_ks);
@@ -495,7 +675,7 @@ int launch_gemm(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, co
                 float* splitk_ws, size_t splitk_ws_bytes, SlabSum* defer) {
   if (defer) *defer = SlabSum();
   MI_CHECK(T >= 1, "gemm: T must be >= 1");
-  if (epi < EPI_RELU2 && gemm_wide_wanted(w, T, splitk_ws ? splitk_ws_bytes : 0) && ldx % 8 == 0)
+  if (gemm_wide_wanted(w, T, splitk_ws ? splitk_ws_bytes : 0) && ldx % 8 == 0)
     return launch_gemm_wide(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer);
   MI_CHECK(w.N % 16 == 0 && w.K % 64 == 0, "gemm: N % 16 == 0 and K % 64 == 0 required");
   MI_CHECK(ldx % 8 == 0, "gemm: x row stride must be a multiple of 8 elements");
@@ -649,7 +829,7 @@ __global__ __launch_bounds__(256) void gemm_a8_kernel(const uint4* __restrict__ 
 // 64 KiB a stage: two stages in 160 KiB, and two stages cannot carry the stagger -- profiles/r03_a8_wide_experiment.txt.)
 // A stage: [16 n-tiles][2 k-tiles][64 lanes x 16 B] weight fragments as stored, then 128 activation rows x 128 B with
 // 16-byte chunk ch of row r at slot ch ^ (r & 7) (the lane reads chunks g and 4 + g: conflict-free with that key).
-constexpr int kA8wStage = 32 * 1024 + 128 * 128, kA8wDma = 6;
+constexpr int kA8wStage = 32 * 1024 + 128 * 128, kA8wDma = 6, kA8WideStages = 3;
 // (A ninth wave touching the lines of the K-step four ahead, to make the ring's DMAs L2 hits, cost 27 %: 260 -> 330 us on
 // gate|up at 2048 tokens -- profiles/r03_a8_wide_experiment.txt.)
 template <int EPI, bool SPLIT>
@@ -680,7 +860,7 @@ __global__ __launch_bounds__(512) void gemm_a8_wide_kernel(const uint4* __restri
     xsrc[i] = x8 + ((size_t)ks0 * ldx + min(m0 + r, T - 1)) * 128 + ((sl ^ (r & 7)) * 16);
   }
   auto issue = [&](int ks) {
-    unsigned char* st = smem + (ks % kWideStages) * kA8wStage;
+    unsigned char* st = smem + (ks % kA8WideStages) * kA8wStage;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -711,7 +891,7 @@ __global__ __launch_bounds__(512) void gemm_a8_wide_kernel(const uint4* __restri
     }
     __builtin_amdgcn_s_barrier();
     if (ks + 2 < nks) issue(ks + 2);
-    const unsigned char* st = smem + (ks % kWideStages) * kA8wStage;
+    const unsigned char* st = smem + (ks % kA8WideStages) * kA8wStage;
     const uint4* xs = reinterpret_cast<const uint4*>(st + 32 * 1024);
     u32x4_t b0[4], b1[4], a0[4], a1[4];
 #pragma unroll
@@ -825,7 +1005,7 @@ int launch_gemm_a8(const LinearW& w, int T, const uint8_t* x8, int ldx, int epi,
       const int KS = best_ks;
       dim3 grid(8 * ceil_div(T, 128) * ceil_div(ceil_div(w.N, 256), 8), 1, KS);
       const uint4* W = reinterpret_cast<const uint4*>(w.w);
-      constexpr int lds = kWideStages * kA8wStage;
+      constexpr int lds = kA8WideStages * kA8wStage;
 #define MI_A8W_L(EPI_, SPLIT_, WS_) \
   do { \
     MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_a8_wide_kernel<EPI_, SPLIT_>), lds)); \

@@ -84,6 +84,14 @@ __device__ __forceinline__ bf16x8_t decode8<MI_W_INT8>(uint32_t lo, uint32_t hi)
   return u.v;
 }
 
+// two neighbouring codes of a word: its low half or its high half
+template <int WD>
+__device__ __forceinline__ uint32_t decode2(uint32_t w, int half) {
+  if constexpr (WD == MI_W_F8E4M3)
+    return __builtin_bit_cast(uint32_t, half ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, true) : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, false));
+  else return i8x2_to_bf16x2(w, 2 * half, 2 * half + 1);
+}
+
 // ---- cross-lane sums inside an aligned group of 4, 8 or 16 lanes (DPP, no LDS) ------------
 template <int CTRL>
 __device__ __forceinline__ float dpp_add(float v) {

@@ -2022,9 +2022,20 @@ int mi_op_qlinear(const void* x, int32_t M, const void* w_tiled, const float* sc
   p.x = reinterpret_cast<const uint16_t*>(x); p.ldx = K;
   const bool gemv = force_path == 1 || (force_path == 0 && gemv_fits(M, K));
   if (gemv) return launch_gemv(W, M, PRO_BF16, p, EPI_F32, e, (hipStream_t)stream);
+  MI_CHECK(wd != MI_W_BF16 || force_path < 3 || force_path > 7, "qlinear: paths 3 .. 7 are for 1-byte weights");
+  if (force_path == 8) {   // as the model runs it: with a workspace of the model's size for K slices
+    float* slab = nullptr;
+    const size_t bytes = (size_t)64 << 20;
+    MI_HIP(hipMalloc(reinterpret_cast<void**>(&slab), bytes));
+    int rc = launch_gemm(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes);
+    hipStreamSynchronize((hipStream_t)stream);
+    hipFree(slab);
+    return rc;
+  }
   if (force_path == 3) return launch_gemm_wide(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream);
   if (force_path >= 4 && force_path <= 7) {   // the wide GEMM with its K dimension split: 4 / 5 = 2 / 4 slices at 128-token blocks, 6 / 7 at 256
     const int ks = (force_path & 1) ? 4 : 2, bm = force_path >= 6 ? 256 : 128;
+    MI_CHECK(K / 64 % ks == 0, "qlinear: paths 4 .. 7 need K / 64 a multiple of their slices");
     float* slab = nullptr;
     const size_t bytes = (size_t)ks * M * N * 4;
     MI_HIP(hipMalloc(reinterpret_cast<void**>(&slab), bytes));
