@@ -19,12 +19,8 @@ struct QdRow {
     return v * sl.scale[c];
   }
   __device__ __forceinline__ float4 at4(int c) const {      // c % 4 == 0
-    float4 v = *reinterpret_cast<const float4*>(p + c);
-    if (!sl.slab) return v;
-    for (int z = 1; z < sl.KS; ++z) {
-      const float4 q = *reinterpret_cast<const float4*>(p + (size_t)z * sl.T * sl.N + c);
-      v.x += q.x; v.y += q.y; v.z += q.z; v.w += q.w;
-    }
+    if (!sl.slab) return *reinterpret_cast<const float4*>(p + c);
+    const float4 v = slab_sum4(p + c, (size_t)sl.T * sl.N, sl.KS);
     const float4 s = *reinterpret_cast<const float4*>(sl.scale + c);
     return make_float4(v.x * s.x, v.y * s.y, v.z * s.z, v.w * s.w);
   }

@@ -951,12 +951,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   const int nq = N >> 2;
   if (q >= T * nq) return;
   const int m = q / nq, n0 = (q - m * nq) * 4;
-  f32x4_t v = {0.f, 0.f, 0.f, 0.f};
-  for (int z = 0; z < KS; ++z) {
-    const float4 p = *reinterpret_cast<const float4*>(slab + ((size_t)z * T + m) * N + n0);
-    v[0] += p.x; v[1] += p.y; v[2] += p.z; v[3] += p.w;
-  }
-  epilogue<EPI>(e, m, n0, v);
+  const float4 v = slab_sum4(slab + (size_t)m * N + n0, (size_t)T * N, KS);
+  epilogue<EPI>(e, m, n0, f32x4_t{v.x, v.y, v.z, v.w});
 }
 
 // sum a deferred K-split (SlabSum) the plain way: splitk_reduce + residual epilogue

@@ -181,6 +181,23 @@ struct SlabSum {
   const float* bias = nullptr;      // [N] or null
   const float* row_scale = nullptr; // [T] or null (FP8 activations)
 };
+#ifdef __HIPCC__
+// The sum of KS slabs' four numbers at p, `stride` numbers apart, in slice order.  Five requests leave before the first is waited for: one after the
+// other they cost a trip to memory each (the row norm over 8 slabs of 242 x 4096: 13.9 us that way, 9.3 now, of which the bytes take 6.3).
+__device__ __forceinline__ float4 slab_sum4(const float* __restrict__ p, size_t stride, int KS) {
+  constexpr int U = 5;
+  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int z = 0; z < KS; z += U) {
+    float4 q[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) q[u] = *reinterpret_cast<const float4*>(p + (size_t)min(z + u, KS - 1) * stride);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (z + u < KS) { v.x += q[u].x; v.y += q[u].y; v.z += q[u].z; v.w += q[u].w; }
+  }
+  return v;
+}
+#endif
 int device_num_cu(int* out);                                  // CUs of the current device
 int ensure_dynamic_lds(const void* kernel, int bytes);        // hipFuncSetAttribute where (device, kernel) has fewer so far
 

@@ -73,27 +73,23 @@ int launch_gather_rows(const float* src, const int32_t* rows, int n, int H, floa
 // to bf16, then e4m3 with the per-token scale amax / 448 -- as the K-step-major image
 // [H / 128][T][128 B] the FP8 GEMM reads (same arithmetic, one launch and one bf16 round trip less).
 template <bool FP8>
-__global__ __launch_bounds__(256) void norm_rows_kernel(const float* __restrict__ resid_in, const float* __restrict__ partial,
+__global__ __launch_bounds__(1024) void norm_rows_kernel(const float* __restrict__ resid_in, const float* __restrict__ partial,
                                                         float* __restrict__ resid_out, const float* __restrict__ gain,
                                                         int H, float eps, uint16_t* __restrict__ y,
                                                         uint8_t* __restrict__ x8, float* __restrict__ row_scale, SlabSum sl) {
-  extern __shared__ __attribute__((aligned(16))) float hrow[];  // H floats + 8
-  const int t = blockIdx.x, tid = threadIdx.x;
+  extern __shared__ __attribute__((aligned(16))) float hrow[];  // H floats + 32
+  const int t = blockIdx.x, tid = threadIdx.x, nthr = blockDim.x;
   const size_t o = (size_t)t * H;
   float ss = 0.f;
   const float sl_rs = (sl.slab && sl.row_scale) ? sl.row_scale[t] : 1.f;   // read before this launch may overwrite it (FP8: same array)
-  for (int c4 = tid; c4 < H / 4; c4 += 256) {
+  for (int c4 = tid; c4 < H / 4; c4 += nthr) {
     float4 a = *reinterpret_cast<const float4*>(resid_in + o + c4 * 4);
     if (partial) {
       const float4 p = *reinterpret_cast<const float4*>(partial + o + c4 * 4);
       a.x += p.x; a.y += p.y; a.z += p.z; a.w += p.w;
     }
     if (sl.slab) {   // the residual add of a K-split projection: slabs in slice order, scale, bias, + residual
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      for (int z = 0; z < sl.KS; ++z) {
-        const float4 q = *reinterpret_cast<const float4*>(sl.slab + ((size_t)z * sl.T + t) * sl.N + c4 * 4);
-        v.x += q.x; v.y += q.y; v.z += q.z; v.w += q.w;
-      }
+      float4 v = slab_sum4(sl.slab + (size_t)t * sl.N + c4 * 4, (size_t)sl.T * sl.N, sl.KS);
       float4 sc = *reinterpret_cast<const float4*>(sl.scale + c4 * 4);
       if (sl.row_scale) { sc.x *= sl_rs; sc.y *= sl_rs; sc.z *= sl_rs; sc.w *= sl_rs; }
       v.x *= sc.x; v.y *= sc.y; v.z *= sc.z; v.w *= sc.w;
@@ -111,9 +107,11 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const float* __restrict_
   float* red = hrow + H;
   if ((tid & 63) == 0) red[tid >> 6] = ss;
   __syncthreads();
-  const float rinv = rsqrtf((red[0] + red[1] + red[2] + red[3]) / (float)H + eps);
+  ss = red[0];
+  for (int w = 1; w < nthr >> 6; ++w) ss += red[w];
+  const float rinv = rsqrtf(ss / (float)H + eps);
   float amax = 0.f;
-  for (int c4 = tid; c4 < H / 4; c4 += 256) {
+  for (int c4 = tid; c4 < H / 4; c4 += nthr) {
     const float4 a = *reinterpret_cast<const float4*>(hrow + c4 * 4);
     const float4 g = *reinterpret_cast<const float4*>(gain + c4 * 4);
     const uint2 pk = make_uint2(pack_bf16x2(a.x * rinv * g.x, a.y * rinv * g.y), pack_bf16x2(a.z * rinv * g.z, a.w * rinv * g.w));
@@ -128,12 +126,13 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const float* __restrict_
   if constexpr (FP8) {
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
-    if ((tid & 63) == 0) red[4 + (tid >> 6)] = amax;
+    if ((tid & 63) == 0) red[16 + (tid >> 6)] = amax;
     __syncthreads();
-    amax = fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7]));
+    amax = red[16];
+    for (int w = 1; w < nthr >> 6; ++w) amax = fmaxf(amax, red[16 + w]);
     const float scale = amax > 0.f ? amax / 448.f : 1.f;
     if (tid == 0) row_scale[t] = scale;
-    for (int c4 = tid; c4 < H / 4; c4 += 256) {
+    for (int c4 = tid; c4 < H / 4; c4 += nthr) {
       const uint2 pk = *reinterpret_cast<const uint2*>(hrow + c4 * 4);
       const float v0 = fminf(fmaxf(bf16lo_to_f32(pk.x) / scale, -448.f), 448.f);
       const float v1 = fminf(fmaxf(bf16hi_to_f32(pk.x) / scale, -448.f), 448.f);
@@ -145,11 +144,13 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const float* __restrict_
     }
   }
 }
+// up to 512 rows (two per CU): a float4 per thread, one round of requests; more rows: 256 threads, several rows per CU
+static int norm_threads(int T, int H) { return T <= 512 ? std::min(1024, ceil_div(H / 4, 64) * 64) : 256; }
 int launch_norm_rows(const float* resid_in, const float* partial, float* resid_out, const float* gain, int T,
                      int H, float eps, uint16_t* y, hipStream_t s, const SlabSum* slabs) {
   MI_CHECK(H % 4 == 0 && H <= 32768, "rmsnorm: H % 4 == 0 and H <= 32768 required");
   MI_CHECK(!slabs || (slabs->T == T && slabs->N == H && resid_out), "rmsnorm: pending K-split sum of another shape");
-  hipLaunchKernelGGL(norm_rows_kernel<false>, dim3(T), dim3(256), (H + 8) * sizeof(float), s, resid_in, partial, resid_out,
+  hipLaunchKernelGGL(norm_rows_kernel<false>, dim3(T), dim3(norm_threads(T, H)), (H + 32) * sizeof(float), s, resid_in, partial, resid_out,
                      gain, H, eps, y, nullptr, nullptr, slabs ? *slabs : SlabSum());
   MI_HIP(hipGetLastError());
   return MI_OK;
@@ -158,7 +159,7 @@ int launch_norm_rows_fp8(const float* resid_in, const float* partial, float* res
                          int H, float eps, uint8_t* x8, float* row_scale, hipStream_t s, const SlabSum* slabs) {
   MI_CHECK(H % 128 == 0 && H <= 32768, "rmsnorm + fp8: H % 128 == 0 and H <= 32768 required");
   MI_CHECK(!slabs || (slabs->T == T && slabs->N == H && resid_out), "rmsnorm: pending K-split sum of another shape");
-  hipLaunchKernelGGL(norm_rows_kernel<true>, dim3(T), dim3(256), (H + 8) * sizeof(float), s, resid_in, partial, resid_out,
+  hipLaunchKernelGGL(norm_rows_kernel<true>, dim3(T), dim3(norm_threads(T, H)), (H + 32) * sizeof(float), s, resid_in, partial, resid_out,
                      gain, H, eps, nullptr, x8, row_scale, slabs ? *slabs : SlabSum());
   MI_HIP(hipGetLastError());
   return MI_OK;

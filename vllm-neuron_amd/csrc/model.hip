@@ -134,9 +134,9 @@ int run_linear(mi_ctx* c, const Linear& L, int rows, int pro, ProArgs p, int epi
   }
   // a residual projection whose K-split sum the next norm can take over (one work-group per row there)
   static const bool fuse = [] { const char* v = getenv("MI355X_FUSE_SPLITK_NORM"); return !v || v[0] != '0'; }();
-  // (from 384 rows on -- the 512 bucket holds 495: the norm runs one work-group per row -- with few rows the K-split sum is the wider kernel on its
-  //  own; measured at 32 rows: 14.2 us fused against 5.0 + 4.6 us)
-  static const int fuse_min_rows = [] { const char* v = getenv("MI355X_FUSE_SPLITK_MIN_ROWS"); return v ? atoi(v) : 384; }();
+  // (at every length: with the slabs' requests in flight together the sum inside the norm costs less than a launch of its own; prompts of 70 tokens of
+  //  the 8B model in fp8 2077 -> 2036 us, 242 tokens 3114 -> 3062, 300 tokens of TinyLlama 2602 -> 2520)
+  static const int fuse_min_rows = [] { const char* v = getenv("MI355X_FUSE_SPLITK_MIN_ROWS"); return v ? atoi(v) : 0; }();
   SlabSum* defer = (fuse && epi == EPI_RESID && rows >= fuse_min_rows && !c->pend.slab) ? &c->pend : nullptr;
   auto note_deferred = [&]() {
     if (defer && c->pend.slab) { c->pend_in = e.resid_in; c->pend_out = e.out_f32; }

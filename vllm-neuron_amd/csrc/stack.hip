@@ -1357,7 +1357,7 @@ int latent_mixer(mi_ctx* c, const StackLayer& W, size_t kv_at, const Batch& b, R
   EpiArgs e{};
   e.out_f32 = S->qkv_out; e.ld_out = W.qkv.N;
   SlabSum slabs;       // (many rows: a K-split's sum is left to the scatter)
-  MI_TRY(apply(c, W.qkv, b.rows, S->n1, S->Kd, EPI_F32, e, b.rows >= 384 ? &slabs : nullptr));
+  MI_TRY(apply(c, W.qkv, b.rows, S->n1, S->Kd, EPI_F32, e, b.rows > 32 ? &slabs : nullptr));
   unsigned char* pool = reinterpret_cast<unsigned char*>(c->kv_pool) + kv_at * S->elem();
   const LatentRowsIn in{S->qkv_out, S->qkv_out + g.H * g.dk, W.qkv.N, W.qkv.N};
   if (b.decode && W.fast() && latent_token_supported(g)) {
@@ -1374,7 +1374,7 @@ int latent_mixer(mi_ctx* c, const StackLayer& W, size_t kv_at, const Batch& b, R
   EpiArgs o{};
   o.out_f32 = S->y; o.ld_out = S->ld;
   out.y = S->y; out.ld = S->ld;
-  return apply(c, W.out, b.rows, S->cat, S->cat_ld, EPI_F32, o, b.rows >= 384 ? &out.slabs : nullptr);
+  return apply(c, W.out, b.rows, S->cat, S->cat_ld, EPI_F32, o, b.rows > 32 ? &out.slabs : nullptr);
 }
 
 int gated_ff(mi_ctx* c, const StackLayer& W, int rows, RowSource& out) {
@@ -1386,7 +1386,7 @@ int gated_ff(mi_ctx* c, const StackLayer& W, int rows, RowSource& out) {
   EpiArgs o{};
   o.out_f32 = S->y; o.ld_out = S->ld;
   out.y = S->y; out.ld = S->ld;
-  return apply(c, W.down, rows, S->act, S->act_ld, EPI_F32, o, rows >= 384 ? &out.slabs : nullptr);
+  return apply(c, W.down, rows, S->act, S->act_ld, EPI_F32, o, rows > 32 ? &out.slabs : nullptr);
 }
 
 // few rows stream the weights of the experts they chose; many are grouped by expert
@@ -1565,7 +1565,7 @@ int one_norm_trunk(mi_ctx* c, const Batch& b, int& cur) {
     MI_TRY(W.s.mixer_kind == MI_MIX_DELTA ? one_norm_delta(c, W, S->state_at[i], b) : one_norm_latent(c, W, S->kv_at[i], b));
     EpiArgs e{};
     e.out_f32 = c->resid[cur ^ 1]; e.resid_in = c->resid[cur]; e.ld_out = S->ld;
-    MI_TRY(apply(c, W.out, b.rows, S->cat, S->cat_ld, EPI_RESID, e, b.rows >= 384 ? &src.slabs : nullptr));
+    MI_TRY(apply(c, W.out, b.rows, S->cat, S->cat_ld, EPI_RESID, e, b.rows > 32 ? &src.slabs : nullptr));
     if (!src.slabs.slab) cur ^= 1;
   }
   MI_TRY(row(nullptr));
@@ -1683,7 +1683,7 @@ int post_norm_trunk(mi_ctx* c, const Batch& b, int& cur) {
     e.out_f32 = S->y; e.ld_out = S->ld;
     src.y = S->y; src.ld = S->ld;
     w_post = w;
-    return apply(c, m, b.rows, x, ldx, EPI_F32, e, b.rows >= 384 ? &src.slabs : nullptr);
+    return apply(c, m, b.rows, x, ldx, EPI_F32, e, b.rows > 32 ? &src.slabs : nullptr);
   };
   for (size_t i = 0; i < S->runs.size(); ++i) {
     const StackLayer& W = S->layers[S->runs[i].layer];
@@ -1774,7 +1774,7 @@ int stack_trunk(mi_ctx* c, int rows, bool decode, int MB, const AttnSeg* segs, i
       EpiArgs e{};
       e.out_f32 = c->resid[cur ^ 1]; e.resid_in = c->resid[cur]; e.ld_out = S->ld;
       // (many rows: the K-split sum is left to the next norm, which passes over the row anyway)
-      MI_TRY(apply(c, W.out, rows, S->cat, S->cat_ld, EPI_RESID, e, rows >= 384 && !S->residuals ? &S->pend : nullptr));
+      MI_TRY(apply(c, W.out, rows, S->cat, S->cat_ld, EPI_RESID, e, rows > 32 && !S->residuals ? &S->pend : nullptr));
       cur ^= 1;
     }
     if (S->residuals)

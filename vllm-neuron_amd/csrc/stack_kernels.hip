@@ -79,11 +79,7 @@ __global__ __launch_bounds__(1024) void layernorm_rows_kernel(const float* __res
   for (int c4 = tid; c4 < ld / 4; c4 += nthr) {
     float4 a = *reinterpret_cast<const float4*>(resid_in + o + c4 * 4);
     if (sl.slab) {   // slabs in slice order, scale, + residual: the arithmetic of splitk_reduce + the residual epilogue
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      for (int z = 0; z < sl.KS; ++z) {
-        const float4 q = *reinterpret_cast<const float4*>(sl.slab + ((size_t)z * sl.T + t) * sl.N + c4 * 4);
-        v.x += q.x; v.y += q.y; v.z += q.z; v.w += q.w;
-      }
+      const float4 v = slab_sum4(sl.slab + (size_t)t * sl.N + c4 * 4, (size_t)sl.T * sl.N, sl.KS);
       const float4 sc = *reinterpret_cast<const float4*>(sl.scale + c4 * 4);
       a.x += v.x * sc.x; a.y += v.y * sc.y; a.z += v.z * sc.z; a.w += v.w * sc.w;
       *reinterpret_cast<float4*>(resid_out + o + c4 * 4) = a;
@@ -151,10 +147,7 @@ __device__ __forceinline__ float4 part_rstd(const float* rstd, int d, int G, flo
 __device__ __forceinline__ float4 source_row4(const RowSource& src, int t, int d) {
   float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
   if (src.slabs.slab) {
-    for (int z = 0; z < src.slabs.KS; ++z) {
-      const float4 q = *reinterpret_cast<const float4*>(src.slabs.slab + ((size_t)z * src.slabs.T + t) * src.slabs.N + d);
-      v.x += q.x; v.y += q.y; v.z += q.z; v.w += q.w;
-    }
+    v = slab_sum4(src.slabs.slab + (size_t)t * src.slabs.N + d, (size_t)src.slabs.T * src.slabs.N, src.slabs.KS);
     const float4 sc = *reinterpret_cast<const float4*>(src.slabs.scale + d);
     v.x *= sc.x; v.y *= sc.y; v.z *= sc.z; v.w *= sc.w;
   }
@@ -674,8 +667,8 @@ int launch_layernorm_rows(const float* resid_in, float* resid_out, int T, int D,
   MI_CHECK(ld % 4 == 0 && ld >= D && ld <= 32768 && ldy >= ld, "layer norm: row stride must be a multiple of 4, at least the width, at most 32768");
   MI_CHECK(!slabs || (slabs->T == T && slabs->N == ld && resid_out && !slabs->bias && !slabs->row_scale), "layer norm: pending K-split sum of another shape");
   const size_t lds = (size_t)(ld + 32) * sizeof(float);
-  // few rows (token generation): one float4 per thread, the row is one round of loads; many rows: 256 threads, several rows per CU
-  const int threads = T <= 32 ? std::min(1024, ceil_div(ld / 4, 64) * 64) : 256;
+  // few rows (up to two per CU): one float4 per thread, the row is one round of loads; many rows: 256 threads, several rows per CU
+  const int threads = T <= 512 ? std::min(1024, ceil_div(ld / 4, 64) * 64) : 256;
   const SlabSum sl = slabs ? *slabs : SlabSum();
   if (lds > 64 * 1024)
     MI_HIP(f32 ? hipFuncSetAttribute(reinterpret_cast<const void*>(layernorm_rows_kernel<float>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)
@@ -724,7 +717,7 @@ int launch_sandwich_rows(const float* resid_in, float* resid_out, const RowSourc
     return MI_OK;
   }
   const size_t lds = (size_t)(ld + std::max(groups, 16) + groups) * sizeof(float);
-  const int threads = T <= 32 ? std::min(1024, ceil_div(ld / 4, 64) * 64) : 256;
+  const int threads = T <= 512 ? std::min(1024, ceil_div(ld / 4, 64) * 64) : 256;   // one float4 per thread up to two rows per CU
   const void* kern = f32 ? reinterpret_cast<const void*>(sandwich_rows_kernel<float>) : reinterpret_cast<const void*>(sandwich_rows_kernel<uint16_t>);
   MI_CHECK(lds <= 160 * 1024, "sandwich rows: row too long");
   if (lds > 64 * 1024) { int rc = ensure_dynamic_lds(kern, 160 * 1024); if (rc != MI_OK) return rc; }
