@@ -734,11 +734,13 @@ __device__ __forceinline__ int kv_swz(int key) {   // XOR key of the 16-byte chu
   else return (((key >> 1) & 1) << 2) | ((key >> 2) & 3);                        // 128-byte rows,  8 chunks
 }
 
+constexpr int kPrefillSlices = 6;   // of the keys, at most
+
 template <int HD, int NW>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill2_kernel(
     const uint16_t* __restrict__ q, int T, int q_pos0, const uint16_t* __restrict__ kpool,
     const uint16_t* __restrict__ vpool, int bs, int bs_shift, const int32_t* __restrict__ block_table, int nh, int nkv,
-    int G, int Gp, int nblk, uint16_t* __restrict__ out, float scale_log2e) {
+    int G, int Gp, int nblk, int paired, float* __restrict__ o_part, float* __restrict__ ml_part, uint16_t* __restrict__ out, float scale_log2e) {
   constexpr int TK = 64;                       // keys per tile
   constexpr int ROWB = HD * 2;                 // bytes per K/V row
   constexpr int CPR = HD / 8;                  // 16-byte chunks per row
@@ -789,12 +791,16 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
       vaddr[db][u] = key * ROWB + ((chunk ^ kv_swz<HD>(key)) * 16) + 8 * (pc & 1);
     }
 
-  const int passes = QB == 1 ? 2 : 1;
+  const int passes = QB == 1 && paired ? 2 : 1;
   for (int pass = 0; pass < passes; ++pass) {
     // ---- which query block this wave owns --------------------------------------------------------
     int blk_q, pair;
     bool blk_ok;
-    if (QB == 1) {                       // one block at a time: the heavy one of pair blockIdx.x, then the light one
+    if (QB == 1 && !paired) {            // a work-group per block, the heavy ones first
+      pair = blockIdx.x;
+      blk_q = nblk - 1 - pair;
+      blk_ok = pair < nblk;
+    } else if (QB == 1) {                // one block at a time: the heavy one of pair blockIdx.x, then the light one
       pair = blockIdx.x;
       blk_q = pass == 0 ? nblk - 1 - pair : pair;
       blk_ok = pair < npair && !(pass == 1 && pair == nblk - 1 - pair);
@@ -811,7 +817,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     int wg_pair0 = QB == 1 ? (int)blockIdx.x : (int)blockIdx.x * (QB >> 1);
     int wg_blk = QB == 1 ? (pass == 0 ? nblk - 1 - wg_pair0 : wg_pair0) : nblk - 1 - wg_pair0;   // heaviest block of the work-group
     wg_blk = max(min(wg_blk, nblk - 1), 0);
-    const int nt = (q_pos0 + min(wg_blk * 32 + 31, T - 1)) / TK + 1;
+    const int nt_all = (q_pos0 + min(wg_blk * 32 + 31, T - 1)) / TK + 1;
+    // this slice of them: all, or the blockIdx.z-th of gridDim.z slices of the keys
+    const int t_per = ceil_div(nt_all, (int)gridDim.z), t0 = (int)blockIdx.z * t_per, nt = min(nt_all, t0 + t_per);
 
     // ---- Q fragments (B operand of S^T): Q[q0 + qq][16 ks + 8 h ..] ---------------------------------
     const int qi = min(q0 + qq, T - 1);
@@ -853,16 +861,15 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     };
 
     int st_issue = 0, st_read = 0;
-    fetch_ids(0);
-    issue(0);
-    if (nt > 1) { fetch_ids(1); issue(1); }
-    fetch_ids(2);
+    if (t0 < nt) { fetch_ids(t0); issue(0); }
+    if (t0 + 1 < nt) { fetch_ids(t0 + 1); issue(1); }
+    fetch_ids(t0 + 2);
     st_issue = 2;
     // hipcc waits for a plain load at its first use -- inside the tile loop, as vmcnt(0) on every iteration, which would drain
     // the two tiles in flight each time.  Taking the Q fragments through an empty asm here puts that wait in front of the loop.
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) asm volatile("" : "+v"(qf[ks]));
-    for (int t = 0; t < nt; ++t) {
+    for (int t = t0; t < nt; ++t) {
       if (t + 1 < nt) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CNT) : "memory");
       else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();            // every wave's pieces of tile t are in; everyone is done reading tile t - 1
@@ -920,7 +927,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
         const f32x2_t sw = swap32_pair(mx);
         mx = fmaxf(sw[0], sw[1]);
       }
-      const float ms = mx * scale_log2e;         // key 0 is visible to every query: finite from the first tile on
+      const float ms = mx * scale_log2e;         // key 0 is visible to every query: finite from the first tile on, but for a later slice of the keys
       const bool moved = ms > m_used + kDeferLog2;
       if (__any(moved)) {
         const float mn = moved ? ms : m_used;
@@ -952,12 +959,13 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
       MI_VREAD(0); MI_VREAD(1); MI_VREAD(2); MI_VREAD(3);
       static_assert(kVAhead == 4, "the prefetch above is written out for 4");
       bf16x8_t pb[4];
+      const float m_exp = gridDim.z > 1 && m_used == -INFINITY ? 0.f : m_used;   // (a slice whose keys so far all lie ahead of this query)
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
         float pv[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          pv[r] = fexp2(fmaf(sc[b][r], scale_log2e, -m_used));   // masked: exp2(-inf) = 0
+          pv[r] = fexp2(fmaf(sc[b][r], scale_log2e, -m_exp));    // masked: exp2(-inf) = 0
           lsum += pv[r];
         }
 #pragma unroll
@@ -992,6 +1000,20 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     }
     const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
     const bool st_ok = active && q0 + qq < T;
+    if (gridDim.z > 1) {   // unnormalised, with its maximum and sum: attn_prefill_combine_kernel puts the slices together
+      const size_t row = ((size_t)blockIdx.z * T + q0 + qq) * nh + head;
+      if (st_ok && h == 0) *reinterpret_cast<float2*>(ml_part + 2 * row) = make_float2(m_used, lsum);
+      if (st_ok && m_used != -INFINITY) {
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            *reinterpret_cast<float4*>(o_part + row * HD + 32 * db + 8 * k + 4 * h) =
+                make_float4(o[db][4 * k], o[db][4 * k + 1], o[db][4 * k + 2], o[db][4 * k + 3]);
+      }
+      __syncthreads();
+      continue;
+    }
     uint16_t* orow = out + ((size_t)(q0 + qq) * nh + head) * HD;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -1011,6 +1033,36 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
   }
 }
 
+// the slices of the keys put together: out = sum_z 2^(m_z - M) O_z / sum_z 2^(m_z - M) l_z; four elements of a head per thread
+template <int HD>
+__global__ __launch_bounds__(256) void attn_prefill_combine_kernel(const float* __restrict__ o_part, const float* __restrict__ ml_part, int ns, int rows,
+                                                                   uint16_t* __restrict__ out) {
+  const int i = blockIdx.x * 256 + threadIdx.x, row = i / (HD / 4), d = i % (HD / 4) * 4;
+  if (row >= rows) return;                     // rows = tokens x heads
+  float2 ml[kPrefillSlices];
+  float4 o[kPrefillSlices];
+  float M = -INFINITY;
+#pragma unroll
+  for (int z = 0; z < kPrefillSlices; ++z) {   // requests of every slice leave together; those behind the last are copies of it and count nothing
+    const size_t r = (size_t)min(z, ns - 1) * rows + row;
+    ml[z] = *reinterpret_cast<const float2*>(ml_part + 2 * r);
+    o[z] = *reinterpret_cast<const float4*>(o_part + r * HD + d);
+  }
+#pragma unroll
+  for (int z = 0; z < kPrefillSlices; ++z) M = fmaxf(M, ml[z].x);
+  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+  float l = 0.f;
+#pragma unroll
+  for (int z = 0; z < kPrefillSlices; ++z) {
+    if (z >= ns || ml[z].x == -INFINITY) continue;   // (a slice without a key for this query wrote no O)
+    const float w = fexp2(ml[z].x - M);
+    l = fmaf(w, ml[z].y, l);
+    v.x = fmaf(w, o[z].x, v.x); v.y = fmaf(w, o[z].y, v.y); v.z = fmaf(w, o[z].z, v.z); v.w = fmaf(w, o[z].w, v.w);
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  *reinterpret_cast<uint2*>(out + (size_t)row * HD + d) = make_uint2(pack_bf16x2(v.x * inv, v.y * inv), pack_bf16x2(v.z * inv, v.w * inv));
+}
+
 static bool attn_prefill_v1() {   // MI355X_ATTN_PREFILL_V1=1: the first-generation kernel (A/B)
   static const bool on = [] { const char* v = getenv("MI355X_ATTN_PREFILL_V1"); return v && v[0] == '1'; }();
   return on;
@@ -1018,7 +1070,7 @@ static bool attn_prefill_v1() {   // MI355X_ATTN_PREFILL_V1=1: the first-generat
 
 int launch_attn_prefill(const uint16_t* q, int T, int q_pos0, const uint16_t* kpool, const uint16_t* vpool,
                         int block_size, const int32_t* block_table, int nh, int nkv, int hd, uint16_t* out,
-                        hipStream_t s) {
+                        hipStream_t s, float* ws, size_t ws_bytes) {
   MI_CHECK(hd == 64 || hd == 128, "attention: head_dim must be 64 or 128");
   MI_CHECK(T >= 1 && q_pos0 >= 0, "attention: bad T / q_pos0");
   MI_CHECK(nh % nkv == 0 && nh / nkv <= 8, "attention: q heads per kv head must be 1..8");
@@ -1031,17 +1083,35 @@ int launch_attn_prefill(const uint16_t* q, int T, int q_pos0, const uint16_t* kp
     const int nblk = ceil_div(T, 32), npair = (nblk + 1) / 2, qb = 8 / Gp;
     int bs_shift = -1;
     for (int sh = 4; sh < 20; ++sh) if ((1 << sh) == block_size) bs_shift = sh;
-    const dim3 grid2(ceil_div(npair, qb >= 2 ? qb / 2 : 1), nkv);
+    // One block per work-group (5 .. 8 heads on a kv head): pairs only where single blocks would not all run at once.
+    const int paired = qb > 1 || nblk * nkv > 256;
+    const int gx = paired ? ceil_div(npair, qb >= 2 ? qb / 2 : 1) : nblk;
+    // A short prompt, or the rest of one behind cached keys, leaves most of the chip idle while each work-group walks its tiles, 1.75 us each:
+    // slices of the keys then, at least two tiles each, the cheapest by that and the second launch, which moves every slice's O out and in.
+    // 188 tokens behind 512 cached ones, 28 heads on 4: 40.8 us in 12 work-groups of two passes, 16.7 + 4.8 now.
+    int ns = 1;
+    const int tiles = ceil_div(q_pos0 + T, 64);
+    double best = 1.75 * tiles * ceil_div(gx * nkv, 256);
+    for (int z = 2; ws && z <= kPrefillSlices; ++z) {
+      const size_t part = (size_t)z * T * nh;
+      if (ceil_div(tiles, z) < 2 || part * (hd + 2) * sizeof(float) > ws_bytes) break;
+      const double cost = 1.75 * ceil_div(tiles, z) * ceil_div(gx * nkv * z, 256) + 4.5 + (double)part * hd * 8.0 / 4e6;
+      if (cost < best) { best = cost; ns = z; }
+    }
+    float *o_part = ns > 1 ? ws : nullptr, *ml_part = ns > 1 ? ws + (size_t)ns * T * nh * hd : nullptr;
+    const dim3 grid2(gx, nkv, ns);
     if (hd == 128) {
       constexpr int lds = 3 * 2 * 64 * 256;
       MI_TRY_A(ensure_dynamic_lds(reinterpret_cast<const void*>(attn_prefill2_kernel<128, 8>), lds));
       hipLaunchKernelGGL((attn_prefill2_kernel<128, 8>), grid2, dim3(512), lds, s, q, T, q_pos0, kpool, vpool, block_size, bs_shift,
-                         block_table, nh, nkv, G, Gp, nblk, out, scale_log2e);
+                         block_table, nh, nkv, G, Gp, nblk, paired, o_part, ml_part, out, scale_log2e);
+      if (ns > 1) hipLaunchKernelGGL((attn_prefill_combine_kernel<128>), dim3(ceil_div(T * nh * (128 / 4), 256)), dim3(256), 0, s, o_part, ml_part, ns, T * nh, out);
     } else {
       constexpr int lds = 3 * 2 * 64 * 128;
       MI_TRY_A(ensure_dynamic_lds(reinterpret_cast<const void*>(attn_prefill2_kernel<64, 8>), lds));
       hipLaunchKernelGGL((attn_prefill2_kernel<64, 8>), grid2, dim3(512), lds, s, q, T, q_pos0, kpool, vpool, block_size, bs_shift,
-                         block_table, nh, nkv, G, Gp, nblk, out, scale_log2e);
+                         block_table, nh, nkv, G, Gp, nblk, paired, o_part, ml_part, out, scale_log2e);
+      if (ns > 1) hipLaunchKernelGGL((attn_prefill_combine_kernel<64>), dim3(ceil_div(T * nh * (64 / 4), 256)), dim3(256), 0, s, o_part, ml_part, ns, T * nh, out);
     }
     MI_HIP(hipGetLastError());
     return MI_OK;

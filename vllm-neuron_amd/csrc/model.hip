@@ -271,13 +271,13 @@ int run_trunk(mi_ctx* c, int rows, bool decode, int B, int MB, int q_pos0, const
         }
         MI_TRY(launch_attn_prefill(c->qbuf + (size_t)segs[i].row0 * c->q_dim, segs[i].n, segs[i].pos0, kpool, vpool,
                                    k.block_size, c->d_bt + (size_t)i * MB, c->nh_l, c->nkv_l, c->hd,
-                                   c->attn_out + (size_t)segs[i].row0 * c->q_dim, s));
+                                   c->attn_out + (size_t)segs[i].row0 * c->q_dim, s, c->splitk_ws, c->splitk_ws_bytes));
         ++i;
       }
     } else {
       Scope sc(c, MI_K_ATTN_PREFILL);
       MI_TRY(launch_attn_prefill(c->qbuf, rows, q_pos0, kpool, vpool, k.block_size, c->d_bt, c->nh_l,
-                                 c->nkv_l, c->hd, c->attn_out, s));
+                                 c->nkv_l, c->hd, c->attn_out, s, c->splitk_ws, c->splitk_ws_bytes));
     }
     const bool tp = c->collective();  // a communicator (even of one rank) selects the collective path
     {  // O projection.  TP = 1: straight into the residual stream (resid' = resid + y);
