@@ -354,7 +354,7 @@ int run_head(mi_ctx* c, int logits_rows, int logits_row0, bool gather) {
     p.resid_out = nullptr;
     p.gain = c->g_final; p.eps = k.rms_norm_eps;
     EpiArgs e{};
-    e.out_f32 = c->logits; e.ld_out = c->V_l;
+    e.out_f32 = c->head_out ? c->head_out : c->logits; e.ld_out = c->V_l;
     MI_TRY(run_linear(c, c->lm_head, logits_rows, PRO_NORM, p, EPI_F32, e));
   }
   if (c->grp) {
@@ -382,11 +382,20 @@ int run_layers(mi_ctx* c, int rows, bool decode, int B, int MB, int q_pos0, int 
   return run_head(c, logits_rows, logits_row0, segs != nullptr);
 }
 
+// Where the head of a call for `nrows` rows of host logits writes: straight into the pinned buffer the caller reads, over PCIe under its own weight stream.
+// The weight-streaming kernels' 64-byte pieces go out at 40 - 44 GB/s (a copy kernel: 42 - 55), so 4 rows of 128256 take 51 us under the head's 87 where
+// head, gap and copy took 87 + 19 + 37; 32 rows 369 against 127 + 19 + 300.  The GEMMs of larger batches, and shards, keep the copy.
+struct HeadToHost {
+  mi_ctx* c;
+  HeadToHost(mi_ctx* c_, int nrows, bool wanted) : c(c_) { c->head_out = wanted && !c->collective() && gemv_fits(nrows, c->H) ? c->h_logits : nullptr; }
+  ~HeadToHost() { c->head_out = nullptr; }
+};
+
 int fetch_logits(mi_ctx* c, int nrows, float* out) {
   const mi_model_config& k = c->cfg;
   const int V = k.vocab_size;
   if (!c->collective()) {
-    MI_HIP(hipMemcpyAsync(c->h_logits, c->logits, (size_t)nrows * V * 4, hipMemcpyDeviceToHost, c->stream));
+    if (!c->head_out) MI_HIP(hipMemcpyAsync(c->h_logits, c->logits, (size_t)nrows * V * 4, hipMemcpyDeviceToHost, c->stream));
     g_ht.lap(3);
     MI_HIP(hipStreamSynchronize(c->stream));
     g_ht.lap(4);
@@ -545,7 +554,7 @@ float bf16_bits_to_f32(uint16_t h) {
 }
 
 int capture_or_launch_decode(mi_ctx* c, int B, int MB) {
-  const int key = (B * 65536 + MB) ^ (int)((c->class_mask & 0xff) << 24) ^ ((c->attn_rows_per_seq - 1) << 12);
+  const int64_t key = (int64_t)(uint32_t)((B * 65536 + MB) ^ (int)((c->class_mask & 0xff) << 24) ^ ((c->attn_rows_per_seq - 1) << 12)) | (int64_t)(c->head_out != nullptr) << 40;
   // a caller-supplied transport runs on the host thread: never captured
   if (!c->cfg.use_graphs || c->prof.on || c->xport_allreduce || (c->stack && c->stack->residuals)) return run_layers(c, B, true, B, MB, 0, B, 0);
   auto it = c->graphs.find(key);
@@ -1425,6 +1434,7 @@ static int forward_impl(mi_ctx* c, int32_t B, int32_t S, const int64_t* input_id
     MI_TRY(push_inputs());
     guard.pushed = true;
     g_ht.lap(1);
+    HeadToHost to(c, B, logits_out != nullptr);
     MI_TRY(capture_or_launch_decode(c, B, MB));
     g_ht.lap(2);
     c->last_B = B;
@@ -1463,6 +1473,7 @@ static int forward_impl(mi_ctx* c, int32_t B, int32_t S, const int64_t* input_id
     MI_TRY(stage_state(c, 1, seq_ids ? seq_ids + b : nullptr));
     memcpy(c->h_segs, std::array<int32_t, 4>{0, n_new, comp, 0}.data(), 16);
     MI_TRY(push_inputs());
+    HeadToHost to(c, 1, logits_out != nullptr);
     MI_TRY(run_layers(c, n_new, false, 1, MB, comp, 1, n_new - 1));
     // (the copy engine reads the pinned block asynchronously: the next row's staging must not
     //  start before this row's copy has been consumed -- both fetch paths synchronize the stream)
@@ -1565,6 +1576,7 @@ int mi_forward_chunked(mi_ctx* c, int32_t n_req, int32_t total, const int64_t* i
     return forward_impl(c, n_req, 1, input_ids, position_ids, seq_ids, block_table, MB, slot_mapping, 1, full_context_lens,
                         computed_context_lens, logits_out, sampling_params, seed, tokens_out);
   MI_TRY(ragged_trunk(c, n_req, total, input_ids, position_ids, seq_ids, slot_mapping, block_table, MB, full_context_lens, computed_context_lens));
+  HeadToHost to(c, n_req, logits_out != nullptr);
   MI_TRY(run_head(c, n_req, 0, true));
   if (tokens_out) MI_TRY(sample_on_device(c, n_req, 0, sampling_params, seed, tokens_out));
   else MI_TRY(fetch_logits(c, n_req, logits_out));
@@ -1599,6 +1611,7 @@ int mi_forward_rows(mi_ctx* c, int32_t n_req, int32_t total, const int64_t* inpu
     MI_HIP(hipStreamSynchronize(c->stream));       // the pinned list behind d_ctx is free to be rewritten
     for (int i = 0; i < n; ++i) c->h_ctx[i] = (int32_t)rows[i0 + i];
     MI_HIP(hipMemcpyAsync(c->d_ctx, c->h_ctx, (size_t)n * 4, hipMemcpyHostToDevice, c->stream));
+    HeadToHost to(c, n, true);
     MI_TRY(run_head(c, n, 0, true));
     MI_TRY(fetch_logits(c, n, logits_out + (size_t)i0 * V));
   }

@@ -107,7 +107,8 @@ struct mi_ctx {
   int32_t *d_spec = nullptr, *h_spec = nullptr;   // fused speculation (mi_forward_spec): candidates, limits, outputs
   int MB_cap = 0;
   size_t weight_bytes = 0, workspace_bytes = 0, kv_bytes = 0;
-  std::map<int, hipGraphExec_t> graphs;  // token-generation graph per (B * 65536 + MB)
+  std::map<int64_t, hipGraphExec_t> graphs;  // token-generation graph per (B * 65536 + MB) and per where its logits go
+  float* head_out = nullptr;      // where the head writes its logits: h_logits, or (null) logits on the device
   int last_B = 0, last_MB = 0;           // shape of the last token-generation call (mi_replay_decode)
   Prof prof;
   // kernel classes the token-generation step launches (mi_replay_decode_classes measures a step with

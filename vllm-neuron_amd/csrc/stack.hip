@@ -1796,13 +1796,14 @@ int stack_head(mi_ctx* c, const float* resid, int nrows) {
   }
   const bool direct = c->V_l % 16 == 0;
   EpiArgs e{};
-  e.out_f32 = direct ? c->logits : S->logits_pad;
+  float* out = c->head_out ? c->head_out : c->logits;
+  e.out_f32 = direct ? out : S->logits_pad;
   e.ld_out = S->head.N;
   e.softcap = S->cfg.logit_softcap;
   MI_TRY(apply(c, S->head, nrows, S->n1, S->Kd, e.softcap > 0.f ? EPI_SOFTCAP : EPI_F32, e));
   if (!direct) {
     Scope sc(c, MI_K_OTHER);
-    MI_TRY(launch_pack_rows(S->logits_pad, S->head.N, nrows, c->V_l, c->logits, c->stream));
+    MI_TRY(launch_pack_rows(S->logits_pad, S->head.N, nrows, c->V_l, out, c->stream));
   }
   return MI_OK;
 }
