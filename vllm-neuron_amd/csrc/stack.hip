@@ -1356,11 +1356,12 @@ int latent_mixer(mi_ctx* c, const StackLayer& W, size_t kv_at, const Batch& b, R
   hipStream_t s = c->stream;
   EpiArgs e{};
   e.out_f32 = S->qkv_out; e.ld_out = W.qkv.N;
-  SlabSum slabs;       // (many rows: a K-split's sum is left to the scatter)
-  MI_TRY(apply(c, W.qkv, b.rows, S->n1, S->Kd, EPI_F32, e, b.rows > 32 ? &slabs : nullptr));
+  const bool token = b.decode && W.fast() && latent_token_supported(g);
+  SlabSum slabs;       // (many rows: a K-split's sum is left to the scatter; the token kernel reads summed rows)
+  MI_TRY(apply(c, W.qkv, b.rows, S->n1, S->Kd, EPI_F32, e, b.rows > 32 && !token ? &slabs : nullptr));
   unsigned char* pool = reinterpret_cast<unsigned char*>(c->kv_pool) + kv_at * S->elem();
   const LatentRowsIn in{S->qkv_out, S->qkv_out + g.H * g.dk, W.qkv.N, W.qkv.N};
-  if (b.decode && W.fast() && latent_token_supported(g)) {
+  if (token) {
     if (runs_other(c)) {
       Scope sc(c, MI_K_OTHER);
       MI_TRY(launch_latent_token(in, b.rows, g, Rotation(), W.w_uk, W.c_norm, S->cfg.norm_eps, c->d_slots, reinterpret_cast<uint16_t*>(S->qa),
