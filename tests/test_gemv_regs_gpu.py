@@ -1,0 +1,70 @@
+"""Token generation of 5 .. 32 rows: the weight stream with the activations in registers (gemv_regs_kernel) at the edges of its splits, and the
+sums it leaves to the next norm inside the models."""
+import pytest
+import torch
+
+from oracle.quant import dequantize_weight, quantize_weight
+from tests.test_ops_gpu import WD, dev, quantize_on_device
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from vllm_neuron_amd import _native
+    _native.load_library()
+    return _native
+
+
+# rows: the first and last of each column group; K: fewer k-tiles than waves, an odd share per wave, the first beyond 4 / 8 / 16 tiles a wave, two to eight
+# slices of uneven length; N: one row-tile, one more than the CUs, several passes, more than the passes whose scales fit
+@pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
+@pytest.mark.parametrize("M", [5, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(16, 64), (4112, 320), (272, 1088), (528, 2112), (144, 4096), (48, 4160), (2048, 6208), (16, 28672), (263680, 64), (8208, 1152)])
+def test_edges_of_the_register_gemv(lib, wd, M, N, K):
+    g = torch.Generator().manual_seed(M + N + K)
+    w = torch.randn(N, K, generator=g) * 0.05
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    bias = torch.randn(N, generator=g) * 0.1
+    tiled, scale = quantize_on_device(lib, w, wd, "per_channel_symmetric")
+    wq = w.to(torch.bfloat16).float() if wd == "bf16" else dequantize_weight(*quantize_weight(w, wd, "per_channel_symmetric"))
+    ref = x.double() @ wq.double().t() + bias.double()
+    y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    xd, bd = dev(x), dev(bias)
+    lib.check(lib.load_library().mi_op_qlinear(xd.data_ptr(), M, tiled.data_ptr(), scale.data_ptr(), bd.data_ptr(), N, K, WD[wd], y.data_ptr(), 8, None))
+    torch.cuda.synchronize()
+    err = (y.cpu().double() - ref).abs().max().item()
+    tol = 2e-5 * ref.abs().max().item() + 1e-5 * (K ** 0.5)     # as the other linear tests: fp32 sums in another order
+    assert err < tol, (err, tol)
+
+
+def _rapodra():
+    from tests import test_rapodra_gpu as T
+    from tests.rapodra_cases import config, dense, latent
+    cfg = config(256, 160, [latent(4, 32, 32, 64, 40, dense(6144)), latent(4, 32, 32, 64, 48, dense(6144), kv_from=0)], groups=2)
+    return T, cfg
+
+
+def _vimesun():
+    from tests import test_vimesun_gpu as T
+    from tests.vimesun_cases import att, config
+    return T, config(256, 160, [att(4, 2, 32, 32, 40, 6144), att(4, 1, 32, 32, 48, 6144)])
+
+
+# a feed-forward 24 times as deep as the row is wide: K goes over several slices, and the row norm behind it takes the sum over
+@pytest.mark.parametrize("family", [_rapodra, _vimesun])
+@pytest.mark.parametrize("rows", [5, 12, 32])
+def test_sums_left_to_the_next_norm(family, rows):
+    T, cfg = family()
+    w = T.weights(cfg, 9)
+    r = T.replay(cfg, w, "bfloat16", max_tokens=rows * 48, max_live=rows)
+    toks = [T.tokens(cfg, w, n, 7000 + n) if family is _rapodra else T.tokens(cfg, n, 7000 + n) for n in (30, 31, 32)]
+    refs = [T.reference(f"deep{i}", cfg, w, t, "bfloat16") for i, t in enumerate(toks)]
+    ids = [T.uid() for _ in range(rows)]
+    r.step([{"id": rid, "tokens": toks[i % 3][:20], "want": []} for i, rid in enumerate(ids)], [])
+    worst = 0.0
+    for p in range(20, 28):
+        outs = r.step([{"id": rid, "tokens": [toks[i % 3][p]], "want": [0]} for i, rid in enumerate(ids)], ids if p == 27 else [])
+        worst = max([worst] + [T.error(o, refs[i % 3][p:p + 1]) for i, o in enumerate(outs)])
+    assert worst <= T.LIMIT["bfloat16"], worst
+    r.engine.close()

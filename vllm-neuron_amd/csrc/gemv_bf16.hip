@@ -1,6 +1,8 @@
 // Token-generation weight stream, BF16 weights (templates: linear_device.h).
-#include "linear_device.h"
+#include "gemv_regs.h"
 
 namespace mi {
 template int launch_gemv_wd<MI_W_BF16>(const LinearW&, int, int, const ProArgs&, int, const EpiArgs&, hipStream_t);
+template int launch_gemv_regs_wd<MI_W_BF16>(const LinearW&, int, const uint16_t*, int, int, const EpiArgs&, hipStream_t, float*, size_t, SlabSum*, bool);
+template bool gemv_regs_fits_wd<MI_W_BF16>(int, int, int, size_t);
 }

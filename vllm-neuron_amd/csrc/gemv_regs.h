@@ -1,0 +1,251 @@
+// Token-generation weight stream for 5 .. 32 rows: the activations live in registers.
+//
+// The kernels of linear_device.h keep the activations in LDS.  From 5 rows on that is what their time goes to: rows x K does not fit
+// beside the reduction buffers, so it is staged in chunks between barriers, or streamed beside the weights and read back by every wave.  Here a
+// work-group's eight waves split its K-slice and a wave takes its eighth of the activations into registers once, as MFMA operands (4096 deep and 32
+// rows: 128 registers a lane).  After that a wave only requests weight tiles, one row-tile ahead, and multiplies them; per row-tile the eight
+// partial sums meet in LDS, and the waves take turns at adding them up (in wave order) and running the epilogue, so that no wave has stores
+// of every row-tile in front of its requests (vector memory retires in order).  K beyond what fits the registers goes over grid.y: raw sums to
+// slabs, added by the next row norm or by splitk_reduce.
+// Bound by the weight bytes (117 MB of gate|up of the 8B model in fp8 in 22.7 us at 8 rows, 5.2 TB/s; 27.3 at 32).  us a launch, LDS kernels -> these,
+// 8B fp8 at 32 rows: gate|up 35.8 -> 27.3, QKV 23 -> 15.7, and 4.8 for each norm that was a part of them; 7B int8 at 24 rows: gate|up 57.8, lm_head 261
+// against 25.4 and 139 here at 5 rows (the logits' way over PCIe included).
+#pragma once
+#include "linear_device.h"
+
+namespace mi {
+
+// k-tiles a wave holds: 4 or 8 of 64 k (1-byte weights), 4, 8 or 16 of 32 k
+constexpr int kRegsMaxPasses = 64;   // row-tiles of a work-group: their scales and biases wait in LDS
+template <int WD> constexpr int kRegsMaxTiles = WD == MI_W_BF16 ? 16 : 8;
+
+template <int WD, int EPI, int MG, int NK, bool SLAB>
+__global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4* __restrict__ W, int NT, int KT, int M, int G,
+                                                                   const uint16_t* __restrict__ x, int ldx, EpiArgs e, float* __restrict__ slab) {
+  constexpr int FR = WD == MI_W_BF16 ? 1 : 2;         // MFMAs per weight tile and column group
+  constexpr int BT = NK < 8 ? NK : 8, NB = NK / BT;   // weight tiles per request batch (8 KiB a wave), batches per row-tile
+  constexpr int TK = WD == MI_W_BF16 ? 32 : 64;
+  static_assert(NB == 1 || NB == 2, "one or two batches per row-tile");
+  __shared__ f32x4_t red[2][kGemvWaves][MG][64];
+  __shared__ __attribute__((aligned(16))) float sc_lds[SLAB ? 4 : kRegsMaxPasses * 16], bi_lds[SLAB ? 4 : kRegsMaxPasses * 16];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int g = lane >> 4, c = lane & 15;
+  const int kper = ceil_div(KT, (int)gridDim.y), k_lo = (int)blockIdx.y * kper, k_hi = min(k_lo + kper, KT);
+  const int ktw = ceil_div(k_hi - k_lo, kGemvWaves);
+  const int kbeg = min(k_lo + wave * ktw, k_hi), kend = min(kbeg + ktw, k_hi), klast = max(kend - 1, k_lo);
+  const int passes = ceil_div(NT - (int)blockIdx.x, G);
+
+  // ---- this wave's activations: row c (and 16 + c) of every k-tile it owns; tiles it does not own multiply zeros ----
+  u32x4_t xf[NK * FR * MG];
+#pragma unroll
+  for (int mg = 0; mg < MG; ++mg) {
+    const uint16_t* row = x + (size_t)min(mg * 16 + c, M - 1) * ldx + g * (8 * FR);
+#pragma unroll
+    for (int j = 0; j < NK; ++j) {
+      const int kt = min(kbeg + j, klast);
+#pragma unroll
+      for (int f = 0; f < FR; ++f) xf[(j * FR + f) * MG + mg] = *reinterpret_cast<const u32x4_t*>(row + (size_t)kt * TK + f * 8);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  float rmul[MG];                                     // the row's own factor: 1 / rms where the norm left it to the output
+#pragma unroll
+  for (int mg = 0; mg < MG; ++mg) rmul[mg] = !SLAB && e.row_scale ? e.row_scale[min(mg * 16 + c, M - 1)] : 1.f;
+  // operands of the epilogue of the first row-tile (every wave asks: see gemv_priv_kernel)
+  constexpr bool kPre = !SLAB && !(EPI == EPI_QKV && MG == 2);   // (two groups' rotary factors would not fit the registers)
+  EpiPre<kPre ? EPI : EPI_F32> epre[MG];
+  if constexpr (kPre) {
+#pragma unroll
+    for (int mg = 0; mg < MG; ++mg) epi_prefetch<EPI>(e, min(mg * 16 + c, M - 1), (int)blockIdx.x * 16 + g * 4, epre[mg]);
+  }
+  u32x4_t bufA[BT], bufB[BT];
+  const int total = passes * NB;
+  auto issue = [&](u32x4_t (&buf)[BT], int i) {
+    const bool live = i < total;                      // (a batch that does not exist: one line, the same for every lane)
+    const int ii = min(i, total - 1), tile = (int)blockIdx.x + (ii / NB) * G, k0 = kbeg + (ii % NB) * BT;
+    const uint4* base = live ? W + (size_t)tile * KT * 64 : W;
+    const int kstep = live ? 64 : 0;
+    const unsigned at = live ? lane : 0;
+#pragma unroll
+    for (int u = 0; u < BT; ++u) stream_load16(buf[u], base + (size_t)(min(k0 + u, klast) * kstep) + at);
+  };
+  issue(bufA, 0);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < NK; ++j)
+    if (kbeg + j >= kend) {
+#pragma unroll
+      for (int q = 0; q < FR * MG; ++q) xf[j * FR * MG + q] = u32x4_t{0, 0, 0, 0};
+    }
+  if constexpr (kPre) {
+#pragma unroll
+    for (int mg = 0; mg < MG; ++mg) epi_prefetch_dependent<EPI>(e, (int)blockIdx.x * 16 + g * 4, epre[mg]);
+  }
+  if constexpr (!SLAB) {
+    const int n = passes * 16;
+#pragma unroll
+    for (int q = 0; q < kRegsMaxPasses * 16 / (kGemvWaves * 64); ++q) {
+      const int i = tid + q * kGemvWaves * 64;
+      if (i < n) {
+        const int at = ((int)blockIdx.x + (i >> 4) * G) * 16 + (i & 15);
+        sc_lds[i] = e.scale[at];
+        bi_lds[i] = e.bias ? e.bias[at] : 0.f;
+      }
+    }
+  }
+  issue(bufB, 1);
+
+  f32x4_t acc[MG];
+#pragma unroll
+  for (int mg = 0; mg < MG; ++mg) acc[mg] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](u32x4_t (&buf)[BT], auto j0) {
+#pragma unroll
+    for (int u = 0; u < BT; ++u) {
+      const u32x4_t w = buf[u];
+#pragma unroll
+      for (int f = 0; f < FR; ++f) {
+        bf16x8_t a;
+        if constexpr (WD == MI_W_BF16) a = __builtin_bit_cast(bf16x8_t, w);
+        else a = f ? decode8<WD>(w[2], w[3]) : decode8<WD>(w[0], w[1]);
+#pragma unroll
+        for (int mg = 0; mg < MG; ++mg)
+          acc[mg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8_t, xf[((decltype(j0)::value + u) * FR + f) * MG + mg]), acc[mg], 0, 0, 0);
+      }
+    }
+  };
+  // the row-tile's partial sums to LDS; everybody's are there behind the barrier.  Two buffers: a wave reads one before it meets the next barrier,
+  // and it is written again behind that one.
+  auto meet = [&](int par) {
+#pragma unroll
+    for (int mg = 0; mg < MG; ++mg) {
+      red[par][wave][mg][lane] = acc[mg];
+      acc[mg] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  auto finish = [&](int pass, int par) {
+#pragma unroll
+    for (int mg = 0; mg < MG; ++mg) {
+      if (wave != ((pass * MG + mg) & (kGemvWaves - 1))) continue;
+      f32x4_t s = red[par][0][mg][lane];
+#pragma unroll
+      for (int w = 1; w < kGemvWaves; ++w) {
+        const f32x4_t t = red[par][w][mg][lane];
+        s[0] += t[0]; s[1] += t[1]; s[2] += t[2]; s[3] += t[3];
+      }
+      const int m = mg * 16 + c, n0 = ((int)blockIdx.x + pass * G) * 16 + g * 4;
+      if (m >= M) continue;
+      if constexpr (SLAB) {
+        *reinterpret_cast<float4*>(slab + ((size_t)blockIdx.y * M + m) * (NT * 16) + n0) = make_float4(s[0], s[1], s[2], s[3]);
+      } else {
+        const float *sc4 = sc_lds + pass * 16 + g * 4, *b4 = e.bias ? bi_lds + pass * 16 + g * 4 : nullptr;
+        bool done = false;
+        if constexpr (kPre) {
+          if (pass == 0) { epilogue_pre<EPI>(e, m, n0, sc4, b4, s, epre[mg], rmul[mg]); done = true; }
+        }
+        if (!done) epilogue_lds<EPI>(e, m, n0, sc4, b4, s, rmul[mg]);
+      }
+    }
+  };
+  using First = std::integral_constant<int, 0>;
+  using Second = std::integral_constant<int, (NB - 1) * BT>;
+  if constexpr (NB == 1) {
+    for (int pass = 0; pass < passes; pass += 2) {
+      multiply(bufA, First());
+      meet(0);
+      issue(bufA, pass + 2);
+      finish(pass, 0);
+      if (pass + 1 < passes) {
+        multiply(bufB, First());
+        meet(1);
+        issue(bufB, pass + 3);
+        finish(pass + 1, 1);
+      }
+    }
+  } else {
+    for (int pass = 0; pass < passes; ++pass) {
+      multiply(bufA, First());
+      issue(bufA, 2 * pass + 2);
+      multiply(bufB, Second());
+      meet(pass & 1);
+      issue(bufB, 2 * pass + 3);
+      finish(pass, pass & 1);
+    }
+  }
+}
+
+template <int WD, int EPI, int MG, bool SLAB>
+static int launch_gemv_regs_k(const LinearW& w, int M, const uint16_t* x, int ldx, const EpiArgs& e, hipStream_t s, int slices, float* slab) {
+  const int NT = w.N / 16, KT = w.K / tile_k(WD);
+  int num_cu = 0;
+  MI_TRY_(device_num_cu(&num_cu));
+  const int tiles = ceil_div(ceil_div(KT, slices), kGemvWaves), per = std::max(1, num_cu / slices);
+  // every work-group the same number of row-tiles, or one less; at most kRegsMaxPasses
+  const int G = ceil_div(NT, std::min(kRegsMaxPasses, ceil_div(NT, std::min(NT, per))));
+  const dim3 grid(G, slices);
+  const uint4* W = reinterpret_cast<const uint4*>(w.w);
+  if (tiles <= 4) hipLaunchKernelGGL((gemv_regs_kernel<WD, EPI, MG, 4, SLAB>), grid, dim3(kGemvWaves * 64), 0, s, W, NT, KT, M, G, x, ldx, e, slab);
+  else if (tiles <= 8) hipLaunchKernelGGL((gemv_regs_kernel<WD, EPI, MG, 8, SLAB>), grid, dim3(kGemvWaves * 64), 0, s, W, NT, KT, M, G, x, ldx, e, slab);
+  else if constexpr (WD == MI_W_BF16) hipLaunchKernelGGL((gemv_regs_kernel<WD, EPI, MG, 16, SLAB>), grid, dim3(kGemvWaves * 64), 0, s, W, NT, KT, M, G, x, ldx, e, slab);
+  MI_HIP(hipGetLastError());
+  return MI_OK;
+}
+
+// Over how many slices K goes: what the registers need at least, and more where whole rows of K would leave CUs idle (2048 x 2048: 128 row-tiles) if the
+// sums have a taker.  us: a work-group's bytes at 24 GB/s, the slabs, and a launch that adds them where no row norm does.
+template <int WD>
+static int gemv_regs_slices(int M, int N, int K, size_t ws_bytes, bool deferred, int num_cu) {
+  const int NT = N / 16, KT = K / tile_k(WD);
+  int best = 0;
+  double best_cost = 0.;
+  for (int z = ceil_div(KT, kGemvWaves * kRegsMaxTiles<WD>); z <= 8; ++z) {
+    const int per = ceil_div(KT, z);
+    if (z > 1 && ((z - 1) * per >= KT || (size_t)z * M * N * sizeof(float) > ws_bytes)) continue;
+    double cost = ceil_div(NT, std::max(1, num_cu / z)) * (per / 24.0 + 0.3);
+    if (z > 1) cost += (deferred ? 0.5 : 4.5) + z * (double)M * N * 8e-6 / 4.0;
+    if (best == 0 || cost < best_cost) { best = z; best_cost = cost; }
+  }
+  return best;
+}
+
+template <int WD>
+int launch_gemv_regs_wd(const LinearW& w, int M, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s, float* ws, size_t ws_bytes, SlabSum* defer,
+                        bool split_as_deferred) {
+  int num_cu = 0;
+  MI_TRY_(device_num_cu(&num_cu));
+  const bool deferred = defer && (epi == EPI_RESID || epi == EPI_F32);
+  const int slices = gemv_regs_slices<WD>(M, w.N, w.K, ws ? ws_bytes : 0, deferred || split_as_deferred, num_cu);
+  MI_CHECK(slices > 0, "gemv_regs: no split of K fits the workspace");
+  if (slices > 1) {
+    MI_TRY_(M <= 16 ? (launch_gemv_regs_k<WD, EPI_F32, 1, true>(w, M, x, ldx, e, s, slices, ws)) : (launch_gemv_regs_k<WD, EPI_F32, 2, true>(w, M, x, ldx, e, s, slices, ws)));
+    const SlabSum sum{ws, slices, M, w.N, e.scale, e.bias, e.row_scale};
+    if (deferred) { *defer = sum; return MI_OK; }
+    return launch_splitk_reduce(sum, epi, e, s);
+  }
+#define MI_R(EPI_) return M <= 16 ? launch_gemv_regs_k<WD, EPI_, 1, false>(w, M, x, ldx, e, s, 1, nullptr) : launch_gemv_regs_k<WD, EPI_, 2, false>(w, M, x, ldx, e, s, 1, nullptr)
+  switch (epi) {
+    case EPI_QKV: MI_R(EPI_QKV);
+    case EPI_SWIGLU: MI_R(EPI_SWIGLU);
+    case EPI_RESID: MI_R(EPI_RESID);
+    case EPI_F32: MI_R(EPI_F32);
+  }
+  if constexpr (WD == MI_W_BF16)
+    switch (epi) {
+      case EPI_RELU2: MI_R(EPI_RELU2);
+      case EPI_GLU_CLIP: MI_R(EPI_GLU_CLIP);
+      case EPI_SOFTCAP: MI_R(EPI_SOFTCAP);
+    }
+#undef MI_R
+  set_error("gemv_regs: this epilogue is not built for this weight type");
+  return MI_EINVAL;
+}
+
+template <int WD>
+bool gemv_regs_fits_wd(int M, int N, int K, size_t ws_bytes) {
+  int num_cu = 0;
+  return device_num_cu(&num_cu) == MI_OK && gemv_regs_slices<WD>(M, N, K, ws_bytes, false, num_cu) > 0;
+}
+
+}  // namespace mi

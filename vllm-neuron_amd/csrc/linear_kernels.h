@@ -13,7 +13,7 @@ enum { PRO_BF16 = 0, PRO_NORM = 1, PRO_NORM_PARTIAL = 2 };  // callers pass PRO_
 
 struct EpiArgs {
   const float* scale;  // [N] per-output-row dequant scale
-  const float* row_scale;  // [M] per-token activation scale (FP8-activation GEMM) or nullptr
+  const float* row_scale;  // [M] factor per row (per-token activation scale of the FP8-activation GEMM; launch_gemv_regs) or nullptr
   const float* bias;   // [N] or nullptr
   // EPI_F32: out[m * ld_out + n] = y;  EPI_RESID: out = resid_in[m * ld_out + n] + y
   float* out_f32;
@@ -63,16 +63,25 @@ struct LinearW {
 // M <= 16 token-generation path (HBM-bound weight streaming).
 int launch_gemv(const LinearW& w, int M, int pro, const ProArgs& p, int epi, const EpiArgs& e,
                 hipStream_t s);
+// The same for 5 .. 32 rows of bf16 activations, with those in registers (gemv_regs.h).  ws: room for the slabs of a split K; defer as launch_gemm.
+// EpiArgs::row_scale: a factor per row of the product (1 / rms where launch_norm_rows left it out).
+int launch_gemv_regs(const LinearW& w, int M, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s, float* ws, size_t ws_bytes,
+                     SlabSum* defer = nullptr, bool split_as_deferred = false);
+// whether M rows of w take it (K beyond 8 slices of the registers, or slabs that do not fit: launch_gemv up to 16 rows, launch_gemm)
+bool gemv_in_regs(const LinearW& w, int M, size_t ws_bytes);
+// sums the slabs and runs the epilogue
+int launch_splitk_reduce(const SlabSum& sl, int epi, const EpiArgs& e, hipStream_t s);
 // M > 16 context-encoding path (MFMA-bound).  x is always bf16 [T, K].
 // defer != null: a K-split projection (EPI_RESID, EPI_F32) leaves its slabs unsummed and describes them in *defer
 // (slab == null: nothing deferred); the caller hands them to the next row norm or to launch_splitk_flush
+// split_as_deferred: K is split as if the sum were deferred, though it is not (a shard's partial sums: the same additions as one GPU's)
 int launch_gemm(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e,
-                hipStream_t s, float* splitk_ws = nullptr, size_t splitk_ws_bytes = 0, SlabSum* defer = nullptr);
+                hipStream_t s, float* splitk_ws = nullptr, size_t splitk_ws_bytes = 0, SlabSum* defer = nullptr, bool split_as_deferred = false);
 int launch_splitk_flush(const SlabSum& sl, const float* resid_in, float* out, int ld_out, hipStream_t s);
 // the wide-N LDS-DMA variant of launch_gemm; launch_gemm picks it by size
 int launch_gemm_wide(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
                      float* splitk_ws = nullptr, size_t splitk_ws_bytes = 0, SlabSum* defer = nullptr, int force_bm = 0,
-                     int force_ks = 0);   // force_*: tests (token block 128 / 256, K slices)
+                     int force_ks = 0, bool split_as_deferred = false);   // force_*: tests (token block 128 / 256, K slices)
 // M > 16 with FP8 activations: x8 = K-step-major e4m3 image [K / 128][ldx >= T rows][128 B] as
 // launch_rowquant_fp8 writes it (per-token scale in EpiArgs::row_scale), FP8 weights,
 // MX-scaled MFMA (v_mfma_scale_f32_16x16x128_f8f6f4, unit block scales) at twice the bf16 rate.

@@ -37,11 +37,44 @@ extern template int launch_gemv_wd<MI_W_BF16>(const LinearW&, int, int, const Pr
 extern template int launch_gemv_wd<MI_W_F8E4M3>(const LinearW&, int, int, const ProArgs&, int, const EpiArgs&, hipStream_t);
 extern template int launch_gemv_wd<MI_W_INT8>(const LinearW&, int, int, const ProArgs&, int, const EpiArgs&, hipStream_t);
 
+template <int WD>
+int launch_gemv_regs_wd(const LinearW& w, int M, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s, float* ws, size_t ws_bytes, SlabSum* defer, bool split_as_deferred);
+template <int WD> bool gemv_regs_fits_wd(int M, int N, int K, size_t ws_bytes);
+
+// From 5 rows on (us per call; the LDS kernels with the norm in front of them / these behind a norm kernel; contexts of 500, TinyLlama 200):
+//   8B fp8, 16 layers:  8 rows 1472 / 1332, 16 rows 1758 / 1527, 32 rows 2282 / 2117;   4 rows 1191 / 1277
+//   8B bf16:            8 rows 1949 / 1857, 24 rows 2526 / 2298
+//   7B int8, 14 layers: 5 rows 1454 / 1330, 14 rows 1699 / 1446, 24 rows 2332 / 1789
+//   TinyLlama bf16:     1 row 876 / 1034, 16 rows 1389 / 1210, 30 rows 1501 / 1450
+//   16 layers of width 256 / 512 / 1024 / 1536, bf16: 5 rows 572 / 467, 604 / 538, 637 / 556, 745 / 673; 32 rows 739 / 604, 790 / 626, 850 / 667, 1001 / 926
+// Up to 4 rows the norm inside the weight stream's kernel and its two to eight waves per row-tile win.
+bool gemv_in_regs(const LinearW& w, int M, size_t ws_bytes) {
+  if (M < 5 || M > 32) return false;
+  switch (w.wd) {
+    case MI_W_BF16: return gemv_regs_fits_wd<MI_W_BF16>(M, w.N, w.K, ws_bytes);
+    case MI_W_F8E4M3: return gemv_regs_fits_wd<MI_W_F8E4M3>(M, w.N, w.K, ws_bytes);
+    case MI_W_INT8: return gemv_regs_fits_wd<MI_W_INT8>(M, w.N, w.K, ws_bytes);
+  }
+  return false;
+}
+int launch_gemv_regs(const LinearW& w, int M, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s, float* ws, size_t ws_bytes, SlabSum* defer,
+                     bool split_as_deferred) {
+  if (defer) *defer = SlabSum();
+  MI_CHECK(M >= 1 && M <= 32 && w.N % 16 == 0 && w.K % 64 == 0 && ldx % 8 == 0, "gemv_regs: 1 .. 32 rows, N % 16 == 0, K % 64 == 0, row stride a multiple of 8");
+  switch (w.wd) {
+    case MI_W_BF16: return launch_gemv_regs_wd<MI_W_BF16>(w, M, x, ldx, epi, e, s, ws, ws_bytes, defer, split_as_deferred);
+    case MI_W_F8E4M3: return launch_gemv_regs_wd<MI_W_F8E4M3>(w, M, x, ldx, epi, e, s, ws, ws_bytes, defer, split_as_deferred);
+    case MI_W_INT8: return launch_gemv_regs_wd<MI_W_INT8>(w, M, x, ldx, epi, e, s, ws, ws_bytes, defer, split_as_deferred);
+  }
+  set_error("gemv_regs: bad weight dtype");
+  return MI_EINVAL;
+}
+
 size_t gemv_lds_bytes(int M, int K) { return gemv_image_lds_bytes(M, K); }
 bool gemv_fits(int M, int K) { (void)K; return gemv_rows_fit(M); }
 
 int launch_gemv(const LinearW& w, int M, int pro, const ProArgs& p, int epi, const EpiArgs& e, hipStream_t s) {
-  MI_CHECK(M >= 1 && M <= 32, "gemv: M must be 1..32");
+  MI_CHECK(M >= 1 && M <= 16, "gemv: M must be 1..16");
   MI_CHECK(w.N % 16 == 0 && w.K % 64 == 0, "gemv: N % 16 == 0 and K % 64 == 0 required");
   switch (w.wd) {
     case MI_W_BF16: return launch_gemv_wd<MI_W_BF16>(w, M, pro, p, epi, e, s);
@@ -637,8 +670,8 @@ static int gemm_wide_ks() {      // MI355X_GEMM_WIDE_KS: 1 = never split K in th
 }
 template <int WD>
 static int launch_gemm_wide_wd(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
-                               float* splitk_ws, size_t splitk_ws_bytes, SlabSum* defer, int force_bm, int force_ks) {
-  WidePlan pl = gemm_wide_plan(T, w.N, w.K, gemm_wide_ks() == 1 || !splitk_ws ? 0 : splitk_ws_bytes, w.wd, defer && (epi == EPI_RESID || epi == EPI_F32));
+                               float* splitk_ws, size_t splitk_ws_bytes, SlabSum* defer, int force_bm, int force_ks, bool split_as_deferred) {
+  WidePlan pl = gemm_wide_plan(T, w.N, w.K, gemm_wide_ks() == 1 || !splitk_ws ? 0 : splitk_ws_bytes, w.wd, split_as_deferred || (defer && (epi == EPI_RESID || epi == EPI_F32)));
   const int forced_bm = force_bm ? force_bm : gemm_wide_bm();
   if (forced_bm == 128 || forced_bm == 256) pl = WidePlan{forced_bm, 1};
   if (force_ks) {
@@ -661,22 +694,22 @@ static bool gemm_wide_wanted(const LinearW& w, int T, size_t ws_bytes) {
   return ws_bytes > 0 || ceil_div(T, 128) * ceil_div(w.N, kWideBN) >= 128;
 }
 int launch_gemm_wide(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
-                     float* splitk_ws, size_t splitk_ws_bytes, SlabSum* defer, int force_bm, int force_ks) {
+                     float* splitk_ws, size_t splitk_ws_bytes, SlabSum* defer, int force_bm, int force_ks, bool split_as_deferred) {
   if (defer) *defer = SlabSum();
   MI_CHECK(w.K % 64 == 0 && ldx % 8 == 0, "gemm_wide: K % 64 == 0");
   if (w.wd == MI_W_BF16)
-    return launch_gemm_wide_wd<MI_W_BF16>(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer, force_bm, force_ks);
+    return launch_gemm_wide_wd<MI_W_BF16>(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer, force_bm, force_ks, split_as_deferred);
   if (w.wd == MI_W_F8E4M3)
-    return launch_gemm_wide_wd<MI_W_F8E4M3>(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer, force_bm, force_ks);
-  return launch_gemm_wide_wd<MI_W_INT8>(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer, force_bm, force_ks);
+    return launch_gemm_wide_wd<MI_W_F8E4M3>(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer, force_bm, force_ks, split_as_deferred);
+  return launch_gemm_wide_wd<MI_W_INT8>(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer, force_bm, force_ks, split_as_deferred);
 }
 
 int launch_gemm(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
-                float* splitk_ws, size_t splitk_ws_bytes, SlabSum* defer) {
+                float* splitk_ws, size_t splitk_ws_bytes, SlabSum* defer, bool split_as_deferred) {
   if (defer) *defer = SlabSum();
   MI_CHECK(T >= 1, "gemm: T must be >= 1");
   if (gemm_wide_wanted(w, T, splitk_ws ? splitk_ws_bytes : 0) && ldx % 8 == 0)
-    return launch_gemm_wide(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer);
+    return launch_gemm_wide(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer, 0, 0, split_as_deferred);
   MI_CHECK(w.N % 16 == 0 && w.K % 64 == 0, "gemm: N % 16 == 0 and K % 64 == 0 required");
   MI_CHECK(ldx % 8 == 0, "gemm: x row stride must be a multiple of 8 elements");
   switch (w.wd) {
@@ -953,6 +986,18 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   const int m = q / nq, n0 = (q - m * nq) * 4;
   const float4 v = slab_sum4(slab + (size_t)m * N + n0, (size_t)T * N, KS);
   epilogue<EPI>(e, m, n0, f32x4_t{v.x, v.y, v.z, v.w});
+}
+
+int launch_splitk_reduce(const SlabSum& sl, int epi, const EpiArgs& e, hipStream_t s) {
+  const dim3 grid(ceil_div(sl.T * (sl.N / 4), 256));
+#define MI_S(EPI_) case EPI_: hipLaunchKernelGGL((splitk_reduce_kernel<EPI_>), grid, dim3(256), 0, s, sl.slab, sl.KS, sl.T, sl.N, e); break
+  switch (epi) {
+    MI_S(EPI_F32); MI_S(EPI_QKV); MI_S(EPI_SWIGLU); MI_S(EPI_RESID); MI_S(EPI_RELU2); MI_S(EPI_GLU_CLIP); MI_S(EPI_SOFTCAP);
+    default: set_error("splitk_reduce: unknown epilogue"); return MI_EINVAL;
+  }
+#undef MI_S
+  MI_HIP(hipGetLastError());
+  return MI_OK;
 }
 
 // sum a deferred K-split (SlabSum) the plain way: splitk_reduce + residual epilogue

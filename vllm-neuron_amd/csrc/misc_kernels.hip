@@ -76,7 +76,7 @@ template <bool FP8>
 __global__ __launch_bounds__(1024) void norm_rows_kernel(const float* __restrict__ resid_in, const float* __restrict__ partial,
                                                         float* __restrict__ resid_out, const float* __restrict__ gain,
                                                         int H, float eps, uint16_t* __restrict__ y,
-                                                        uint8_t* __restrict__ x8, float* __restrict__ row_scale, SlabSum sl) {
+                                                        uint8_t* __restrict__ x8, float* __restrict__ row_scale, float* __restrict__ rinv_out, SlabSum sl) {
   extern __shared__ __attribute__((aligned(16))) float hrow[];  // H floats + 32
   const int t = blockIdx.x, tid = threadIdx.x, nthr = blockDim.x;
   const size_t o = (size_t)t * H;
@@ -109,7 +109,11 @@ __global__ __launch_bounds__(1024) void norm_rows_kernel(const float* __restrict
   __syncthreads();
   ss = red[0];
   for (int w = 1; w < nthr >> 6; ++w) ss += red[w];
-  const float rinv = rsqrtf(ss / (float)H + eps);
+  float rinv = rsqrtf(ss / (float)H + eps);
+  if (rinv_out) {   // the projection's output takes the factor (gemv_row_rinv's arithmetic: the same roundings at every decode batch)
+    if (tid == 0) rinv_out[t] = rinv;
+    rinv = 1.f;
+  }
   float amax = 0.f;
   for (int c4 = tid; c4 < H / 4; c4 += nthr) {
     const float4 a = *reinterpret_cast<const float4*>(hrow + c4 * 4);
@@ -147,11 +151,11 @@ __global__ __launch_bounds__(1024) void norm_rows_kernel(const float* __restrict
 // up to 512 rows (two per CU): a float4 per thread, one round of requests; more rows: 256 threads, several rows per CU
 static int norm_threads(int T, int H) { return T <= 512 ? std::min(1024, ceil_div(H / 4, 64) * 64) : 256; }
 int launch_norm_rows(const float* resid_in, const float* partial, float* resid_out, const float* gain, int T,
-                     int H, float eps, uint16_t* y, hipStream_t s, const SlabSum* slabs) {
+                     int H, float eps, uint16_t* y, hipStream_t s, const SlabSum* slabs, float* rinv) {
   MI_CHECK(H % 4 == 0 && H <= 32768, "rmsnorm: H % 4 == 0 and H <= 32768 required");
   MI_CHECK(!slabs || (slabs->T == T && slabs->N == H && resid_out), "rmsnorm: pending K-split sum of another shape");
   hipLaunchKernelGGL(norm_rows_kernel<false>, dim3(T), dim3(norm_threads(T, H)), (H + 32) * sizeof(float), s, resid_in, partial, resid_out,
-                     gain, H, eps, y, nullptr, nullptr, slabs ? *slabs : SlabSum());
+                     gain, H, eps, y, nullptr, nullptr, rinv, slabs ? *slabs : SlabSum());
   MI_HIP(hipGetLastError());
   return MI_OK;
 }
@@ -160,7 +164,7 @@ int launch_norm_rows_fp8(const float* resid_in, const float* partial, float* res
   MI_CHECK(H % 128 == 0 && H <= 32768, "rmsnorm + fp8: H % 128 == 0 and H <= 32768 required");
   MI_CHECK(!slabs || (slabs->T == T && slabs->N == H && resid_out), "rmsnorm: pending K-split sum of another shape");
   hipLaunchKernelGGL(norm_rows_kernel<true>, dim3(T), dim3(norm_threads(T, H)), (H + 32) * sizeof(float), s, resid_in, partial, resid_out,
-                     gain, H, eps, nullptr, x8, row_scale, slabs ? *slabs : SlabSum());
+                     gain, H, eps, nullptr, x8, row_scale, nullptr, slabs ? *slabs : SlabSum());
   MI_HIP(hipGetLastError());
   return MI_OK;
 }

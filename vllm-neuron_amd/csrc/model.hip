@@ -98,16 +98,23 @@ int flush_pending(mi_ctx* c) {
 int run_linear(mi_ctx* c, const Linear& L, int rows, int pro, ProArgs p, int epi, EpiArgs e) {
   e.scale = L.scale;
   e.bias = L.bias;
-  if (gemv_fits(rows, L.K)) {
+  const bool regs = gemv_in_regs(L.view(), rows, c->splitk_ws_bytes);
+  if (!regs && gemv_fits(rows, L.K)) {
     if (!c->runs(MI_K_GEMV)) return MI_OK;
+    if (c->pend.slab) MI_TRY(flush_pending(c));
     Scope sc(c, MI_K_GEMV);
     if (c->prof.on) c->prof.gemv_bytes += (double)L.bytes();
     return launch_gemv(L.view(), rows, pro, p, epi, e, c->stream);
   }
   const uint16_t* x = p.x;
   int ldx = p.ldx;
-  const bool a8 = c->cfg.prefill_fp8_activations && gemm_a8_supported(L.view());
-  if (pro == PRO_NORM) {
+  const bool a8 = !regs && c->cfg.prefill_fp8_activations && gemm_a8_supported(L.view());
+  if (regs && pro == PRO_NORM) e.row_scale = c->row_rinv;
+  if (pro == PRO_NORM && !c->runs(MI_K_OTHER)) {   // (class-masked replay: what the norm would have left)
+    x = c->xn;
+    ldx = L.K;
+    c->pend = SlabSum();
+  } else if (pro == PRO_NORM) {
     Scope sc(c, MI_K_OTHER);
     // A K-split residual projection in front of this norm left its slabs unsummed: the norm sums them on the way
     // (sum, scale, bias, + residual: the arithmetic of splitk_reduce + epilogue) and writes the residual stream.
@@ -126,7 +133,7 @@ int run_linear(mi_ctx* c, const Linear& L, int rows, int pro, ProArgs p, int epi
     if (a8) {   // norm and per-token quantization in one pass over the row
       MI_TRY(launch_norm_rows_fp8(rin, p.partial, rout, p.gain, rows, L.K, p.eps, c->x8, c->x8_scale, c->stream, slabs));
     } else {
-      MI_TRY(launch_norm_rows(rin, p.partial, rout, p.gain, rows, L.K, p.eps, c->xn, c->stream, slabs));
+      MI_TRY(launch_norm_rows(rin, p.partial, rout, p.gain, rows, L.K, p.eps, c->xn, c->stream, slabs, regs ? c->row_rinv : nullptr));
       x = c->xn;
       ldx = L.K;
     }
@@ -138,9 +145,18 @@ int run_linear(mi_ctx* c, const Linear& L, int rows, int pro, ProArgs p, int epi
   //  the 8B model in fp8 2077 -> 2036 us, 242 tokens 3114 -> 3062, 300 tokens of TinyLlama 2602 -> 2520)
   static const int fuse_min_rows = [] { const char* v = getenv("MI355X_FUSE_SPLITK_MIN_ROWS"); return v ? atoi(v) : 0; }();
   SlabSum* defer = (fuse && epi == EPI_RESID && rows >= fuse_min_rows && !c->pend.slab) ? &c->pend : nullptr;
+  const bool as_deferred = fuse && c->collective() && epi == EPI_F32 && rows >= fuse_min_rows && &L != &c->lm_head;
   auto note_deferred = [&]() {
     if (defer && c->pend.slab) { c->pend_in = e.resid_in; c->pend_out = e.out_f32; }
   };
+  if (regs) {
+    if (!c->runs(MI_K_GEMV)) return MI_OK;
+    Scope sc(c, MI_K_GEMV);
+    if (c->prof.on) c->prof.gemv_bytes += (double)L.bytes();
+    MI_TRY(launch_gemv_regs(L.view(), rows, x, ldx, epi, e, c->stream, c->splitk_ws, c->splitk_ws_bytes, defer, as_deferred));
+    note_deferred();
+    return MI_OK;
+  }
   if (a8) {
     if (pro != PRO_NORM) {
       Scope sc(c, MI_K_OTHER);
@@ -153,7 +169,7 @@ int run_linear(mi_ctx* c, const Linear& L, int rows, int pro, ProArgs p, int epi
     return MI_OK;
   }
   Scope sc(c, MI_K_GEMM);
-  MI_TRY(launch_gemm(L.view(), rows, x, ldx, epi, e, c->stream, c->splitk_ws, c->splitk_ws_bytes, defer));
+  MI_TRY(launch_gemm(L.view(), rows, x, ldx, epi, e, c->stream, c->splitk_ws, c->splitk_ws_bytes, defer, as_deferred));
   note_deferred();
   return MI_OK;
 }
@@ -324,7 +340,8 @@ int run_trunk(mi_ctx* c, int rows, bool decode, int B, int MB, int q_pos0, const
       }
     }
   }
-  MI_TRY(flush_pending(c));   // the last down projection's K-split sum: the final norm reads other rows (or a gather of rows)
+  // the last down projection's K-split sum: the final norm takes it over where it reads the same rows and runs as a kernel of its own
+  if (!decode || !gemv_in_regs(c->lm_head.view(), rows, c->splitk_ws_bytes)) MI_TRY(flush_pending(c));
   c->tail_cur = cur;
   c->tail_partial = have_partial;
   return MI_OK;
@@ -387,7 +404,7 @@ int run_layers(mi_ctx* c, int rows, bool decode, int B, int MB, int q_pos0, int 
 // head, gap and copy took 87 + 19 + 37; 32 rows 369 against 127 + 19 + 300.  The GEMMs of larger batches, and shards, keep the copy.
 struct HeadToHost {
   mi_ctx* c;
-  HeadToHost(mi_ctx* c_, int nrows, bool wanted) : c(c_) { c->head_out = wanted && !c->collective() && gemv_fits(nrows, c->H) ? c->h_logits : nullptr; }
+  HeadToHost(mi_ctx* c_, int nrows, bool wanted) : c(c_) { c->head_out = wanted && !c->collective() && nrows <= 32 ? c->h_logits : nullptr; }
   ~HeadToHost() { c->head_out = nullptr; }
 };
 
@@ -855,7 +872,7 @@ int mi_ctx_destroy(mi_ctx* c) {
   fl(c->lm_head);
   void* ptrs[] = {c->g_final, c->embed, c->rowmax, c->kv_pool, c->rope_cos, c->rope_sin, c->stage_raw, c->stage_f32,
                   c->resid[0], c->resid[1], c->partial, c->xn, c->qbuf, c->attn_out, c->act, c->logits, c->logits_all,
-                  c->attn_scratch, c->d_inputs, c->d_dec, c->d_dec_bt, c->d_sparams, c->d_tokens, c->x8, c->x8_scale, c->splitk_ws, c->d_spec, c->d_sample_scratch};
+                  c->attn_scratch, c->d_inputs, c->d_dec, c->d_dec_bt, c->d_sparams, c->d_tokens, c->x8, c->x8_scale, c->row_rinv, c->splitk_ws, c->d_spec, c->d_sample_scratch};
   for (void* p : ptrs) hipFree(p);
   void* hptrs[] = {c->h_inputs, c->h_dec, c->h_dec_bt, c->h_sparams, c->h_tokens, c->h_logits, c->h_spec};
   for (void* p : hptrs) if (p) hipHostFree(p);
@@ -1191,6 +1208,7 @@ int mi_finalize(mi_ctx* c) {
     MI_TRY(dmalloc(&c->x8_scale, R, ws));
   }
   }
+  MI_TRY(dmalloc(&c->row_rinv, 32, ws));
   c->splitk_ws_bytes = (size_t)64 << 20;   // fp32 K-slice slabs of the short-prompt GEMMs
   MI_TRY(dmalloc(&c->splitk_ws, c->splitk_ws_bytes / 4, ws));
   MI_TRY(dmalloc(&c->logits, (size_t)k.max_num_seqs * c->V_l, ws));
@@ -2033,14 +2051,21 @@ int mi_op_qlinear(const void* x, int32_t M, const void* w_tiled, const float* sc
   e.scale = scale; e.bias = bias; e.out_f32 = y; e.ld_out = N;
   ProArgs p{};
   p.x = reinterpret_cast<const uint16_t*>(x); p.ldx = K;
-  const bool gemv = force_path == 1 || (force_path == 0 && gemv_fits(M, K));
-  if (gemv) return launch_gemv(W, M, PRO_BF16, p, EPI_F32, e, (hipStream_t)stream);
+  if (force_path == 1 || (force_path == 0 && M <= 32)) {
+    MI_CHECK(M >= 1 && M <= 32, "gemv: M must be 1..32");
+    for (int m0 = 0; m0 < M; m0 += 16) {   // (the kernels of a caller without a workspace take 16 rows)
+      p.x = reinterpret_cast<const uint16_t*>(x) + (size_t)m0 * K;
+      e.out_f32 = y + (size_t)m0 * N;
+      MI_TRY(launch_gemv(W, std::min(M - m0, 16), PRO_BF16, p, EPI_F32, e, (hipStream_t)stream));
+    }
+    return MI_OK;
+  }
   MI_CHECK(wd != MI_W_BF16 || force_path < 3 || force_path > 7, "qlinear: paths 3 .. 7 are for 1-byte weights");
   if (force_path == 8) {   // as the model runs it: with a workspace of the model's size for K slices
     float* slab = nullptr;
     const size_t bytes = (size_t)64 << 20;
     MI_HIP(hipMalloc(reinterpret_cast<void**>(&slab), bytes));
-    int rc = launch_gemm(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes);
+    int rc = M <= 4 ? launch_gemv(W, M, PRO_BF16, p, EPI_F32, e, (hipStream_t)stream) : gemv_in_regs(W, M, bytes) ? launch_gemv_regs(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes) : launch_gemm(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes);
     hipStreamSynchronize((hipStream_t)stream);
     hipFree(slab);
     return rc;

@@ -69,6 +69,7 @@ struct mi_ctx {
   float* partial = nullptr;
   uint16_t *xn = nullptr, *qbuf = nullptr, *attn_out = nullptr, *act = nullptr;
   uint8_t* x8 = nullptr;        // FP8-activation GEMM input [rows, K]
+  float* row_rinv = nullptr;    // 1 / rms of up to 32 rows, for the projection behind the norm
   float* x8_scale = nullptr;    // its per-token scales [rows]
   float* splitk_ws = nullptr;   // fp32 K-split slabs of short-prompt GEMMs
   mi::SlabSum pend;               // a residual projection's K-split sum left for the next row norm (run_linear)

@@ -81,10 +81,13 @@ int apply(mi_ctx* c, const StackMat& m, int rows, const void* x, int ldx, int ep
     Scope sc(c, MI_K_GEMM);
     return launch_linear_f32((const float*)m.L.w, m.N, m.K, (const float*)x, ldx, rows, epi, e, c->stream);
   }
-  if (gemv_fits(rows, m.K)) {
+  const bool regs = gemv_in_regs(m.L.view(), rows, c->splitk_ws_bytes);
+  if (regs || gemv_fits(rows, m.K)) {
     if (!c->runs(MI_K_GEMV)) return MI_OK;
     Scope sc(c, MI_K_GEMV);
     if (c->prof.on) c->prof.gemv_bytes += (double)m.N * m.K * 2;
+    if (regs)
+      return launch_gemv_regs(m.L.view(), rows, (const uint16_t*)x, ldx, epi, e, c->stream, c->splitk_ws, c->splitk_ws_bytes, defer);
     ProArgs p{};
     p.x = (const uint16_t*)x;
     p.ldx = ldx;
@@ -1357,8 +1360,8 @@ int latent_mixer(mi_ctx* c, const StackLayer& W, size_t kv_at, const Batch& b, R
   EpiArgs e{};
   e.out_f32 = S->qkv_out; e.ld_out = W.qkv.N;
   const bool token = b.decode && W.fast() && latent_token_supported(g);
-  SlabSum slabs;       // (many rows: a K-split's sum is left to the scatter; the token kernel reads summed rows)
-  MI_TRY(apply(c, W.qkv, b.rows, S->n1, S->Kd, EPI_F32, e, b.rows > 32 && !token ? &slabs : nullptr));
+  SlabSum slabs;       // (a K-split's sum is left to the scatter; the token kernel reads summed rows)
+  MI_TRY(apply(c, W.qkv, b.rows, S->n1, S->Kd, EPI_F32, e, token ? nullptr : &slabs));
   unsigned char* pool = reinterpret_cast<unsigned char*>(c->kv_pool) + kv_at * S->elem();
   const LatentRowsIn in{S->qkv_out, S->qkv_out + g.H * g.dk, W.qkv.N, W.qkv.N};
   if (token) {
@@ -1375,7 +1378,7 @@ int latent_mixer(mi_ctx* c, const StackLayer& W, size_t kv_at, const Batch& b, R
   EpiArgs o{};
   o.out_f32 = S->y; o.ld_out = S->ld;
   out.y = S->y; out.ld = S->ld;
-  return apply(c, W.out, b.rows, S->cat, S->cat_ld, EPI_F32, o, b.rows > 32 ? &out.slabs : nullptr);
+  return apply(c, W.out, b.rows, S->cat, S->cat_ld, EPI_F32, o, &out.slabs);
 }
 
 int gated_ff(mi_ctx* c, const StackLayer& W, int rows, RowSource& out) {
@@ -1387,7 +1390,7 @@ int gated_ff(mi_ctx* c, const StackLayer& W, int rows, RowSource& out) {
   EpiArgs o{};
   o.out_f32 = S->y; o.ld_out = S->ld;
   out.y = S->y; out.ld = S->ld;
-  return apply(c, W.down, rows, S->act, S->act_ld, EPI_F32, o, rows > 32 ? &out.slabs : nullptr);
+  return apply(c, W.down, rows, S->act, S->act_ld, EPI_F32, o, &out.slabs);
 }
 
 // few rows stream the weights of the experts they chose; many are grouped by expert
@@ -1566,7 +1569,7 @@ int one_norm_trunk(mi_ctx* c, const Batch& b, int& cur) {
     MI_TRY(W.s.mixer_kind == MI_MIX_DELTA ? one_norm_delta(c, W, S->state_at[i], b) : one_norm_latent(c, W, S->kv_at[i], b));
     EpiArgs e{};
     e.out_f32 = c->resid[cur ^ 1]; e.resid_in = c->resid[cur]; e.ld_out = S->ld;
-    MI_TRY(apply(c, W.out, b.rows, S->cat, S->cat_ld, EPI_RESID, e, b.rows > 32 ? &src.slabs : nullptr));
+    MI_TRY(apply(c, W.out, b.rows, S->cat, S->cat_ld, EPI_RESID, e, &src.slabs));
     if (!src.slabs.slab) cur ^= 1;
   }
   MI_TRY(row(nullptr));
@@ -1684,7 +1687,7 @@ int post_norm_trunk(mi_ctx* c, const Batch& b, int& cur) {
     e.out_f32 = S->y; e.ld_out = S->ld;
     src.y = S->y; src.ld = S->ld;
     w_post = w;
-    return apply(c, m, b.rows, x, ldx, EPI_F32, e, b.rows > 32 ? &src.slabs : nullptr);
+    return apply(c, m, b.rows, x, ldx, EPI_F32, e, &src.slabs);
   };
   for (size_t i = 0; i < S->runs.size(); ++i) {
     const StackLayer& W = S->layers[S->runs[i].layer];
@@ -1775,7 +1778,7 @@ int stack_trunk(mi_ctx* c, int rows, bool decode, int MB, const AttnSeg* segs, i
       EpiArgs e{};
       e.out_f32 = c->resid[cur ^ 1]; e.resid_in = c->resid[cur]; e.ld_out = S->ld;
       // (many rows: the K-split sum is left to the next norm, which passes over the row anyway)
-      MI_TRY(apply(c, W.out, rows, S->cat, S->cat_ld, EPI_RESID, e, rows > 32 && !S->residuals ? &S->pend : nullptr));
+      MI_TRY(apply(c, W.out, rows, S->cat, S->cat_ld, EPI_RESID, e, !S->residuals ? &S->pend : nullptr));
       cur ^= 1;
     }
     if (S->residuals)
