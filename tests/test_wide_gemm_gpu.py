@@ -44,6 +44,33 @@ def test_edges_of_the_wide_gemm(lib, wd, M, N, K):
     assert err < tol, (err, tol)
 
 
+# every tile, at shapes that leave none of its edges whole: a token and a 16-row weight tile past a block, K-steps fewer, as many and more than its stages,
+# three uneven slices
+@pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
+@pytest.mark.parametrize("bm", [64, 128, 192, 256])
+@pytest.mark.parametrize("ntw", [2, 3, 4])
+def test_every_tile_of_the_wide_gemm(lib, wd, bm, ntw):
+    if wd == "bf16" and bm + 64 * ntw > 384 and bm * ntw < 1024:
+        pytest.skip("not built: its stages do not fit the LDS three times")
+    for M, N, K, ks in ((bm + 1, 64 * ntw + 16, 64, 1), (bm - 1, 80, 320, 1), (2 * bm, 128 * ntw, 704, 1), (33, 8 * 64 * ntw + 32, 576, 1),
+                        (bm + 17, 64 * ntw + 16, 704, 3)):
+        g = torch.Generator().manual_seed(M + N + K)
+        w = torch.randn(N, K, generator=g) * 0.05
+        x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+        bias = torch.randn(N, generator=g) * 0.1
+        tiled, scale = quantize_on_device(lib, w, wd, "per_channel_symmetric")
+        wq = w.to(torch.bfloat16).float() if wd == "bf16" else dequantize_weight(*quantize_weight(w, wd, "per_channel_symmetric"))
+        ref = x.double() @ wq.double().t() + bias.double()
+        y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+        xd, bd = dev(x), dev(bias)
+        lib.check(lib.load_library().mi_op_qlinear(xd.data_ptr(), M, tiled.data_ptr(), scale.data_ptr(), bd.data_ptr(), N, K, WD[wd], y.data_ptr(),
+                                                   100 * bm + 10 * ntw + ks, None))
+        torch.cuda.synchronize()
+        err = (y.cpu().double() - ref).abs().max().item()
+        tol = 2e-5 * ref.abs().max().item() + 1e-5 * (K ** 0.5)
+        assert err < tol, (M, N, K, ks, err, tol)
+
+
 _CHILD = r"""
 import sys, torch
 sys.path.insert(0, %(root)r)

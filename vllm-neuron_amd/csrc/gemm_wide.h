@@ -1,0 +1,413 @@
+// The wide context-encoding GEMM (launched through linear_kernels.hip, instantiated per weight type).
+#pragma once
+#include <algorithm>
+
+#include "linear_device.h"
+#include "linear_kernels.h"
+
+namespace mi {
+
+// =====================================================================================
+// GEMM, wide-N tile with an LDS-DMA ring and two wave groups half a K-step apart (context encoding)
+// =====================================================================================
+// A 128 x 128 tile pulls 16 KiB of activations + 8 (16) KiB of weights per 64-deep K-step for 2.1 MFLOP.  A CU takes in 55 - 65 GB/s
+// once half of it comes from HBM (64 KiB of requests in flight, 1.2 us each; from L2 it takes 125 GB/s), so the tile grows: 128 tokens x 256
+// weight rows = 16 + 16 (32) KiB for 4.2 MFLOP, 256 x 256 = 32 + 16 (32) KiB for 8.4.  Smaller ones (64, 128, 192 tokens x 128, 192 weight rows) are for
+// what those leave idle: a grid of one and a bit rounds, token blocks mostly padding, few tokens, whose K then takes fewer slabs.  Eight waves as 2 (tokens) x 4 (weight
+// rows): activation fragments are shared by four waves, weight fragments by two.  Both operands arrive by LDS-DMA
+// (global_load_lds, 1 KiB per wave-instruction: the weight tiles land lane-linear = fragment
+// order; the activation rows land in an XOR-swizzled image (xs_swz), the swizzle being
+// applied to the per-lane SOURCE address) into a ring of stages: all but the one being multiplied are in
+// flight, retired by counted vmcnt waits in front of raw barriers -- no ordinary global
+// load in the loop, so hipcc has nothing to drain.  A wave's K-step is a READ phase (fragments LDS -> registers, then the requests of a later
+// K-step) and a MULTIPLY phase (MFMAs, the weight codes decoded between them), and the two waves of a SIMD are in opposite phases
+// (see "Schedule" in the kernel).
+// What it holds on full grids (gate|up of the 8B model, 2031 tokens): bf16 1.22, fp8 1.27, int8 1.22 PF/s (1.16 before the codes were decoded
+// between the MFMAs), where a library product of 8192^3 in bf16 runs at 1.28 on this card; 128-token blocks 1.13 / 1.18 / 1.05.
+
+// A work-group's tile: BM tokens x 64 NTW weight rows (NTW 16-row tiles for each of the four waves side by side).
+template <int WD, int NTW> constexpr int kWideWBytes = NTW * (WD == MI_W_BF16 ? 8 : 4) * 1024;   // the weight rows of a 64-deep K-step
+// as many stages as the LDS holds, eight at most
+template <int WD, int BM, int NTW> constexpr int kWideStages = std::min(8, 160 * 1024 / (kWideWBytes<WD, NTW> + BM * 128));
+
+// Waits until at most the youngest min(left, MOST) K-steps' DMAs (PER each) of this wave are in flight.
+template <int PER, int MOST>
+__device__ __forceinline__ void wait_dma(int left) {
+  if (left >= MOST) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER * MOST) : "memory");
+  else if constexpr (MOST > 0) wait_dma<PER, MOST - 1>(left);
+}
+
+// The tile of this work-group.  Work-group b runs on XCD b % 8: an XCD takes an eighth of the tiles, one after the other with the token
+// blocks of a weight slab in a row, so that a slab comes into its L2 once.  (Every eighth slab to an XCD, as in gemm_kernel, left the XCDs
+// up to a slab apart: 44 slabs of 11 token blocks put 66 work-groups on the 32 CUs of four of them, three rounds in place of two.)
+template <int BM, int NTW>
+__device__ __forceinline__ bool wide_tile(int T, int NT, int& m0, int& nt0) {
+  const int mtiles = ceil_div(T, BM), tiles = mtiles * ceil_div(NT, 4 * NTW), per = ceil_div(tiles, 8);
+  const int seq = blockIdx.x >> 3, t = (blockIdx.x & 7) * per + seq;
+  if (seq >= per || t >= tiles) return false;
+  nt0 = t / mtiles * (4 * NTW);
+  m0 = t % mtiles * BM;
+  return true;
+}
+// the K-steps of grid.z slice blockIdx.z: equal ones, the last may be shorter (the launch leaves none empty)
+template <bool SPLIT>
+__device__ __forceinline__ void wide_slice(int K, int& ks0, int& nks) {
+  const int all = K / 64, per = SPLIT ? ceil_div(all, (int)gridDim.z) : all;
+  ks0 = SPLIT ? (int)blockIdx.z * per : 0;
+  nks = min(per, all - ks0);
+}
+
+// A wave multiplies BM / 2 tokens x 16 NTW weight rows: NTW BM / 8 accumulator registers (256 x 256: 128, and 246 VGPRs
+// with the decoded fragments of one K-step).
+// SPLIT: grid.z K-slices write raw fp32 accumulators to slab[z][m][n] (see gemm_a8_kernel).
+template <int WD, int EPI, int BM, int NTW, bool SPLIT>
+__global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict__ W, int NT, int KT, int T, int K,
+                                                        const uint16_t* __restrict__ x, int ldx, EpiArgs e,
+                                                        float* __restrict__ slab) {
+  constexpr int kW = kWideWBytes<WD, NTW>, kStage = kW + BM * 128, kStages = kWideStages<WD, BM, NTW>;
+  static_assert(kStages >= 3, "the two wave groups need three stages");
+  // waves as 2 (tokens) x 4 (weight rows), each MT 16-token tiles x NTW 16-row weight tiles (4 x 2 waves would read 16 instead of 20 KiB of
+  // fragments per K-step at 256 x 256 but decode every weight code four times instead of twice)
+  constexpr int MT = BM / 32, WM = 2;
+  constexpr int XP = BM / 64;                 // 8-row activation pieces per wave and stage
+  constexpr int WPK = WD == MI_W_BF16 ? 2 : 1;   // 1 KiB weight tiles per 16 rows and K-step
+  // the 4 NTW WPK weight tiles of a stage over the waves: group 0 (waves 0-3) may bring one more each than group 1 (twelve tiles)
+  constexpr int WP0 = (NTW * WPK + 1) / 2, WP1 = NTW * WPK - WP0;
+  constexpr int kDma0 = WP0 + XP, kDma1 = WP1 + XP;   // DMAs per wave and stage
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int g = lane >> 4, c = lane & 15;
+  const int wm = wave % WM, wn = wave / WM;
+  int m0, ntb;
+  if (!wide_tile<BM, NTW>(T, NT, m0, ntb)) return;
+  int ks0, nks;                               // this slice's K-steps, from K-step ks0 on
+  wide_slice<SPLIT>(K, ks0, nks);
+
+  // this lane's DMA sources: weight tiles wt0 .. (fragment order) and XP 8-row pieces of the activation tile
+  const int grp = __builtin_amdgcn_readfirstlane(wave >> 2), wt0 = grp == 0 ? WP0 * wave : 4 * WP0 + WP1 * (wave - 4);
+  const uint4* wsrc[WP0];
+  const uint16_t* xsrc[XP];
+#pragma unroll
+  for (int i = 0; i < WP0; ++i) {   // tile (row tile / WPK, k tile % WPK); a group-1 wave without an i-th one does not use it
+    const int t = min(wt0 + i, 4 * NTW * WPK - 1);
+    wsrc[i] = W + ((size_t)min(ntb + t / WPK, NT - 1) * KT + ks0 * WPK + t % WPK) * 64 + lane;
+  }
+#pragma unroll
+  for (int i = 0; i < XP; ++i) {
+    const int r = (XP * wave + i) * 8 + (lane >> 3), sl = lane & 7;
+    xsrc[i] = x + (size_t)min(m0 + r, T - 1) * ldx + (size_t)ks0 * 64 + ((sl ^ xs_swz<WD>(r)) * 8);   // LDS slot sl of row r holds chunk sl ^ swz(r)
+  }
+  auto issue = [&](int ks, int stage) {
+    unsigned char* st = smem + stage * kStage;
+#pragma unroll
+    for (int i = 0; i < WP1; ++i) glds16(wsrc[i] + (size_t)ks * WPK * 64, st + (wt0 + i) * 1024);
+    if constexpr (WP0 > WP1) {
+      if (grp == 0) glds16(wsrc[WP1] + (size_t)ks * WPK * 64, st + (wt0 + WP1) * 1024);
+    }
+#pragma unroll
+    for (int i = 0; i < XP; ++i) glds16(xsrc[i] + (size_t)ks * 64, st + kW + (XP * wave + i) * 1024);
+  };
+
+  f32x4_t acc[NTW][MT];
+#pragma unroll
+  for (int i = 0; i < NTW; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  // Schedule.  A K-step of a wave is two phases: READ (its fragments, 20 KiB at BM = 256, from LDS into registers) and MULTIPLY
+  // (2 NTW MT MFMAs from registers).  With one barrier per K-step every wave is in the same phase at the same time, the two waves
+  // of a SIMD included, and LDS-read time and MFMA time add up: 1.7 us per K-step at BM = 256 against 1.0 us of MFMAs.  Here
+  // the two wave groups (waves 0-3 / 4-7 = the two waves of every SIMD) run half a K-step apart -- group 1 executes one
+  // barrier more at the start -- so one group multiplies while the other reads:
+  //     physical barrier:      P0        P1        P2        P3        P4  ...
+  //     group 0 (waves 0-3):   | READ 0  | MUL 0   | READ 1  | MUL 1   | ...
+  //     group 1 (waves 4-7):   |         | READ 0  | MUL 0   | READ 1  | MUL 1 ...
+  // Stage k is read in [P2k, P2k+2]; K-step k + kStages - 1 goes into the stage of K-step k - 1 (read until P2k), requested by every wave
+  // behind its top barrier of iteration k, kStages - 1 K-steps ahead of its first read.  A wave waits for ITS pieces of a
+  // stage before the barrier in front of the stage's first read by anyone (group 0: its top barrier; group 1: its second one).
+#pragma unroll
+  for (int k = 0; k + 1 < kStages; ++k)
+    if (k < nks) issue(k, k);
+  if (grp == 1) {   // its pieces of stage 0 are in before P0
+    wait_dma<kDma1, kStages - 2>(nks - 1);
+    __builtin_amdgcn_s_barrier();           // P0
+  }
+  int cur = 0, fill = kStages - 1;          // the stages of K-step ks and of K-step ks + kStages - 1
+  for (int ks = 0; ks < nks; ++ks) {
+    if (grp == 0) wait_dma<kDma0, kStages - 2>(nks - 1 - ks);   // own pieces of stage ks
+    __builtin_amdgcn_s_barrier();           // group 0: P2ks | group 1: P2ks+1 -- either way nobody reads stage ks - 1 any more
+    const unsigned char* st = smem + cur * kStage;
+    const uint4* xs = reinterpret_cast<const uint4*>(st + kW);
+    u32x4_t b0[MT], b1[MT], w0[NTW], w1[NTW];
+#pragma unroll
+    for (int i = 0; i < NTW; ++i) {
+      const u32x4_t* w = reinterpret_cast<const u32x4_t*>(st + (wn * NTW + i) * (WPK * 1024) + lane * 16);
+      w0[i] = w[0];
+      if constexpr (WD == MI_W_BF16) w1[i] = w[64];
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int r = wm * (BM / 2) + mt * 16 + c;
+      const int ch0 = WD == MI_W_BF16 ? g : 2 * g, ch1 = WD == MI_W_BF16 ? 4 + g : 2 * g + 1;
+      b0[mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + (ch0 ^ xs_swz<WD>(r))]);
+      b1[mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + (ch1 ^ xs_swz<WD>(r))]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (ks + kStages - 1 < nks) issue(ks + kStages - 1, fill);
+    __builtin_amdgcn_sched_barrier(0);
+    cur = cur + 1 == kStages ? 0 : cur + 1;
+    fill = fill + 1 == kStages ? 0 : fill + 1;
+    // the fragments are in registers (the empty asm takes them as operands: the compiler's wait for the reads sits in front of it)
+#pragma unroll
+    for (int i = 0; i < NTW; ++i) {
+      asm volatile("" : "+v"(w0[i]));
+      if constexpr (WD == MI_W_BF16) asm volatile("" : "+v"(w1[i]));
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) { asm volatile("" : "+v"(b0[mt])); asm volatile("" : "+v"(b1[mt])); }
+    if (grp == 1 && ks + 1 < nks) wait_dma<kDma1, kStages - 2>(nks - 2 - ks);   // own pieces of stage ks + 1: group 0 reads it behind the next barrier
+    __builtin_amdgcn_s_barrier();           // group 0: P2ks+1 | group 1: P2ks+2
+    __builtin_amdgcn_sched_barrier(0);
+    // the codes of weight tile i + 1 are decoded between the MFMAs of tile i, whose 16 cycles leave room for three vector instructions each
+    u32x4_t a[2], an[2];
+    auto piece = [&](const u32x4_t& w, int q) { const uint32_t v = w[q >> 1]; return decode2<WD>(v, q & 1); };
+    if constexpr (WD != MI_W_BF16) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) a[q >> 2][q & 3] = piece(w0[0], q);
+    }
+#pragma unroll
+    for (int i = 0; i < NTW; ++i) {
+      if constexpr (WD == MI_W_BF16) { a[0] = w0[i]; a[1] = w1[i]; }
+#pragma unroll
+      for (int m2 = 0; m2 < 2 * MT; ++m2) {   // both halves of a K-step one after the other: two MFMAs in a row never meet in an accumulator
+        const int h = m2 / MT, mt = m2 % MT;
+        acc[i][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[h]), __builtin_bit_cast(bf16x8_t, h ? b1[mt] : b0[mt]), acc[i][mt], 0, 0, 0);
+        if constexpr (WD != MI_W_BF16) {
+          if (i + 1 < NTW) {
+#pragma unroll
+            for (int q = m2 * 4 / MT; q < (m2 + 1) * 4 / MT; ++q) an[q >> 2][q & 3] = piece(w0[i + 1], q);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      if constexpr (WD != MI_W_BF16) { a[0] = an[0]; a[1] = an[1]; }
+    }
+  }
+  if (grp == 0) __builtin_amdgcn_s_barrier();   // the barrier group 1 executed first
+#pragma unroll
+  for (int i = 0; i < NTW; ++i) {
+    const int nt = ntb + wn * NTW + i;
+    if (nt >= NT) continue;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int m = m0 + wm * (BM / 2) + mt * 16 + c;
+      if (m >= T) continue;
+      if constexpr (SPLIT) {
+        *reinterpret_cast<float4*>(slab + ((size_t)blockIdx.z * T + m) * (NT * 16) + nt * 16 + g * 4) =
+            make_float4(acc[i][mt][0], acc[i][mt][1], acc[i][mt][2], acc[i][mt][3]);
+      } else {
+        epilogue<EPI>(e, m, nt * 16 + g * 4, acc[i][mt]);
+      }
+    }
+  }
+}
+
+// The same for bf16 weights at 256 tokens x 256 weight rows.  A 64-deep stage of it is 64 KiB, and the LDS holds two; the stagger
+// needs a third.  So a K-step is 32 deep (one weight tile per 16 rows; 32 MFMAs a wave), the weights ride in four stages of 16 KiB, and the
+// activations, whose rows are fetched 128 bytes at a time, in three of 64-deep pairs of K-steps (32 KiB): 160 KiB.  K-step s requests the weights
+// of s + 3 and one half of the rows of the pair behind the next, four DMAs a wave, so what K-step s reads was requested by K-step s - 3 at
+// the latest and eight younger DMAs stay in flight.
+template <int EPI, bool SPLIT>
+__global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restrict__ W, int NT, int KT, int T, int K,
+                                                          const uint16_t* __restrict__ x, int ldx, EpiArgs e,
+                                                          float* __restrict__ slab) {
+  constexpr int BM = 256, MT = 8, WM = 2, NTW = 4, kW = 16 * 1024, kX = 32 * 1024, kXs = 4 * kW;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int g = lane >> 4, c = lane & 15;
+  const int wm = wave % WM, wn = wave / WM;
+  int m0, ntb;
+  if (!wide_tile<BM, NTW>(T, NT, m0, ntb)) return;
+  int ks0, nks;
+  wide_slice<SPLIT>(K, ks0, nks);
+  const int s0 = 2 * ks0, n = 2 * nks;        // this slice's 32-deep K-steps
+
+  const uint4* wsrc[2];
+  const uint16_t* xsrc[4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) wsrc[i] = W + ((size_t)min(ntb + 2 * wave + i, NT - 1) * KT + s0) * 64 + lane;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = (4 * wave + i) * 8 + (lane >> 3), sl = lane & 7;
+    xsrc[i] = x + (size_t)min(m0 + r, T - 1) * ldx + (size_t)s0 * 32 + ((sl ^ xs_swz<MI_W_BF16>(r)) * 8);
+  }
+  auto issue_w = [&](int s) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) glds16(wsrc[i] + (size_t)s * 64, smem + (s & 3) * kW + (2 * wave + i) * 1024);
+  };
+  auto issue_x = [&](int p, int half, int stage) {   // half of this wave's rows of pair p
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int q = 2 * half + i;
+      glds16((half ? xsrc[2 + i] : xsrc[i]) + (size_t)p * 64, smem + kXs + stage * kX + (4 * wave + q) * 1024);
+    }
+  };
+  // own pieces of K-step s are in: the requests of the last two K-steps may be out, fewer of them at the end
+  auto wait_for = [&](int s) {
+    const int left = n - 1 - s;
+    if (left >= 3) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    else if (left == 2) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+    else if (left == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  };
+
+  f32x4_t acc[NTW][MT];
+#pragma unroll
+  for (int i = 0; i < NTW; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  const int grp = __builtin_amdgcn_readfirstlane(wave >> 2);
+  issue_x(0, 0, 0);
+  issue_x(0, 1, 0);
+  issue_w(0);
+  issue_w(1);
+  if (n > 2) {
+    issue_x(1, 0, 1);
+    issue_w(2);
+    issue_x(1, 1, 1);
+  }
+  if (grp == 1) {
+    wait_for(0);
+    __builtin_amdgcn_s_barrier();           // P0
+  }
+  auto step = [&](int s, int half, int xcur, int xfill) {
+    if (grp == 0) wait_for(s);
+    __builtin_amdgcn_s_barrier();           // group 0: P2s | group 1: P2s+1
+    const unsigned char* st = smem + (s & 3) * kW;
+    const uint4* xs = reinterpret_cast<const uint4*>(smem + kXs + xcur * kX);
+    u32x4_t b[MT], a[NTW];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int r = wm * (BM / 2) + mt * 16 + c;
+      b[mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + ((4 * half + g) ^ xs_swz<MI_W_BF16>(r))]);
+    }
+#pragma unroll
+    for (int i = 0; i < NTW; ++i) a[i] = *reinterpret_cast<const u32x4_t*>(st + (wn * NTW + i) * 1024 + lane * 16);
+    __builtin_amdgcn_sched_barrier(0);
+    if (s + 3 < n) issue_w(s + 3);
+    if ((s >> 1) + 2 < (n >> 1)) issue_x((s >> 1) + 2, half, xfill);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(b[mt]));
+#pragma unroll
+    for (int i = 0; i < NTW; ++i) asm volatile("" : "+v"(a[i]));
+    if (grp == 1 && s + 1 < n) wait_for(s + 1);
+    __builtin_amdgcn_s_barrier();           // group 0: P2s+1 | group 1: P2s+2
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NTW; ++i)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+        acc[i][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[i]), __builtin_bit_cast(bf16x8_t, b[mt]), acc[i][mt], 0, 0, 0);
+  };
+  int xcur = 0, xfill = 2;
+  for (int s = 0; s < n; s += 2) {
+    step(s, 0, xcur, xfill);
+    step(s + 1, 1, xcur, xfill);
+    xcur = xcur == 2 ? 0 : xcur + 1;
+    xfill = xfill == 2 ? 0 : xfill + 1;
+  }
+  if (grp == 0) __builtin_amdgcn_s_barrier();   // the barrier group 1 executed first
+#pragma unroll
+  for (int i = 0; i < NTW; ++i) {
+    const int nt = ntb + wn * NTW + i;
+    if (nt >= NT) continue;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int m = m0 + wm * (BM / 2) + mt * 16 + c;
+      if (m >= T) continue;
+      if constexpr (SPLIT) {
+        *reinterpret_cast<float4*>(slab + ((size_t)blockIdx.z * T + m) * (NT * 16) + nt * 16 + g * 4) =
+            make_float4(acc[i][mt][0], acc[i][mt][1], acc[i][mt][2], acc[i][mt][3]);
+      } else {
+        epilogue<EPI>(e, m, nt * 16 + g * 4, acc[i][mt]);
+      }
+    }
+  }
+}
+
+// The tiles there are.  bf16 weights: a 64-deep stage of 256 x 192, 256 x 256 or 192 x 256 fits the LDS twice only; 256 x 256 has its own kernel.
+template <int WD>
+constexpr bool wide_tile_built(int bm, int ntw) {
+  return (bm == 64 || bm == 128 || bm == 192 || bm == 256) && ntw >= 2 && ntw <= 4 && (WD != MI_W_BF16 || bm + 64 * ntw <= 384 || (bm == 256 && ntw == 4));
+}
+
+template <int WD, int EPI, int BM, int NTW, bool SPLIT>
+static int launch_gemm_wide_t(const LinearW& w, int T, const uint16_t* x, int ldx, const EpiArgs& e, hipStream_t s, int KS, float* slab) {
+  const int NT = w.N / 16, KT = w.K / tile_k(WD);
+  const dim3 grid(8 * ceil_div(ceil_div(T, BM) * ceil_div(NT, 4 * NTW), 8), 1, KS);
+  const uint4* W = reinterpret_cast<const uint4*>(w.w);
+  if constexpr (WD == MI_W_BF16 && BM == 256 && NTW == 4) {
+    const auto fn = gemm_wide16_kernel<EPI, SPLIT>;
+    MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), 160 * 1024));
+    hipLaunchKernelGGL(fn, grid, dim3(512), 160 * 1024, s, W, NT, KT, T, w.K, x, ldx, e, slab);
+  } else {
+    constexpr int lds = kWideStages<WD, BM, NTW> * (kWideWBytes<WD, NTW> + BM * 128);
+    const auto fn = gemm_wide_kernel<WD, EPI, BM, NTW, SPLIT>;
+    MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds));
+    hipLaunchKernelGGL(fn, grid, dim3(512), lds, s, W, NT, KT, T, w.K, x, ldx, e, slab);
+  }
+  MI_HIP(hipGetLastError());
+  return MI_OK;
+}
+
+template <int WD, int BM, int NTW>
+static int launch_gemm_wide_bm(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
+                               int KS, float* ws, SlabSum* defer) {
+  if constexpr (!wide_tile_built<WD>(BM, NTW)) {
+    set_error("gemm_wide: no such tile for this weight type");
+    return MI_EINVAL;
+  } else {
+    if (KS > 1) {
+      MI_TRY_((launch_gemm_wide_t<WD, EPI_F32, BM, NTW, true>(w, T, x, ldx, e, s, KS, ws)));
+      const SlabSum sum{ws, KS, T, w.N, e.scale, e.bias, e.row_scale};
+      if (defer && (epi == EPI_RESID || epi == EPI_F32)) { *defer = sum; return MI_OK; }
+      return launch_splitk_reduce(sum, epi, e, s);
+    }
+#define MI_GW(EPI_) return launch_gemm_wide_t<WD, EPI_, BM, NTW, false>(w, T, x, ldx, e, s, 1, nullptr)
+    switch (epi) {
+      case EPI_QKV: MI_GW(EPI_QKV);
+      case EPI_SWIGLU: MI_GW(EPI_SWIGLU);
+      case EPI_RESID: MI_GW(EPI_RESID);
+      case EPI_F32: MI_GW(EPI_F32);
+    }
+    if constexpr (WD == MI_W_BF16)
+      switch (epi) {
+        case EPI_RELU2: MI_GW(EPI_RELU2);
+        case EPI_GLU_CLIP: MI_GW(EPI_GLU_CLIP);
+        case EPI_SOFTCAP: MI_GW(EPI_SOFTCAP);
+        case EPI_HEADS_KV: MI_GW(EPI_HEADS_KV);
+      }
+#undef MI_GW
+    set_error("gemm_wide: this epilogue is not built for this weight type");
+    return MI_EINVAL;
+  }
+}
+
+// bm x 64 ntw tiles, K over ks slices (ks > 1: ws holds them)
+template <int WD>
+int launch_gemm_wide_wd(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s, int bm, int ntw, int ks, float* ws,
+                        SlabSum* defer) {
+#define MI_GT(BM_, NTW_) \
+  if (bm == BM_ && ntw == NTW_) return launch_gemm_wide_bm<WD, BM_, NTW_>(w, T, x, ldx, epi, e, s, ks, ws, defer)
+  MI_GT(64, 2); MI_GT(64, 3); MI_GT(64, 4);
+  MI_GT(128, 2); MI_GT(128, 3); MI_GT(128, 4);
+  MI_GT(192, 2); MI_GT(192, 3); MI_GT(192, 4);
+  MI_GT(256, 2); MI_GT(256, 3); MI_GT(256, 4);
+#undef MI_GT
+  set_error("gemm_wide: no such tile");
+  return MI_EINVAL;
+}
+
+}  // namespace mi

@@ -1,0 +1,6 @@
+// The wide context-encoding GEMM for int8 weights (gemm_wide.h).
+#include "gemm_wide.h"
+
+namespace mi {
+template int launch_gemm_wide_wd<MI_W_INT8>(const LinearW&, int, const uint16_t*, int, int, const EpiArgs&, hipStream_t, int, int, int, float*, SlabSum*);
+}

@@ -181,6 +181,15 @@ __device__ __forceinline__ void epilogue_pre(const EpiArgs& e, int m, int n0, co
   }
 }
 
+// XOR swizzle of the 16-byte chunks of a 128-byte activation row in LDS.  A ds_read_b128 is
+// serviced in four groups of 16 lanes ({0-3,12-15,20-27}, ...); with the
+// fragment addressing of the MFMA B operand (lane (g, c): row c, chunk 2g / 2g+1 for 1-byte weights,
+// g / 4+g for bf16 weights) the plain `chunk ^ (row & 7)` image is conflict-free for the bf16-weight
+// chunk order but puts every group of the 1-byte order two-deep on its banks; folding row bit 3 into
+// the key makes that order conflict-free too (enumerated over the lane groups).
+template <int WD>
+__device__ __forceinline__ int xs_swz(int r) { return WD == MI_W_BF16 ? (r & 7) : ((r & 7) ^ ((r >> 3) & 1)); }
+
 // =====================================================================================
 // GEMV (token generation)
 // =====================================================================================

@@ -14,18 +14,19 @@
 // k-steps per load for the 1-byte types).  Tiles of one 16-row group are contiguous along K,
 // so a wave streams a dense byte range.
 //
-// Decode (M <= 16): gemv_kernel — pure weight streaming, HBM-bound.  x lives in LDS in
+// Token generation of up to 4 rows: the kernels of linear_device.h — pure weight streaming, HBM-bound.  x lives in LDS in
 //   fragment order; every wave streams a K-slice of one row-tile with 2 x 8 KiB in flight;
 //   the MFMA does the dot products AND the cross-lane reduction; waves combine through LDS
-//   in a fixed order (deterministic, no atomics).
-// Prefill (M > 16): gemm_kernel — 128 x 128 tile, x through swizzled LDS, W straight
-//   from global in fragment order.
+//   in a fixed order (deterministic, no atomics).  5 .. 32 rows: gemv_regs.h, x in registers.
+// Context encoding: gemm_wide.h; gemm_kernel here (128 x 128 tile, x through swizzled LDS, W straight
+//   from global in fragment order) for what that does not take.
 //
-// Both share one epilogue on D[n = 4g + r][m = c] (lane = 16 g + c): dequant scale, bias,
+// All share one epilogue on D[n = 4g + r][m = c] (lane = 16 g + c): dequant scale, bias,
 // then fp32 store | RoPE + q/KV-pool scatter | SwiGLU.
 
 #include "linear_kernels.h"
 
+#include "gemm_wide.h"
 #include "linear_device.h"
 
 namespace mi {
@@ -93,14 +94,6 @@ int launch_gemv(const LinearW& w, int M, int pro, const ProArgs& p, int epi, con
 // straight from the pre-tiled global image.
 constexpr int kBM = 128, kBN = 128, kBK = 64;
 
-// XOR swizzle of the 16-byte chunks of a 128-byte activation row in LDS.  A ds_read_b128 is
-// serviced in four groups of 16 lanes ({0-3,12-15,20-27}, ...: MI355X_MICROARCH.md, LDS); with the
-// fragment addressing of the MFMA B operand (lane (g, c): row c, chunk 2g / 2g+1 for 1-byte weights,
-// g / 4+g for bf16 weights) the plain `chunk ^ (row & 7)` image is conflict-free for the bf16-weight
-// chunk order but puts every group of the 1-byte order two-deep on its banks; folding row bit 3 into
-// the key makes that order conflict-free too (enumerated over the lane groups).
-template <int WD>
-__device__ __forceinline__ int xs_swz(int r) { return WD == MI_W_BF16 ? (r & 7) : ((r & 7) ^ ((r >> 3) & 1)); }
 
 // SPLIT: grid.z K-slices write raw fp32 accumulators to slab[z][m][n] (see gemm_a8_kernel).
 // Registers are kept under 170 per lane so that three work-groups share a CU (the same lesson as
@@ -259,401 +252,52 @@ static int launch_gemm_wd(const LinearW& w, int T, const uint16_t* x, int ldx, i
 }
 
 
-// =====================================================================================
-// GEMM, wide-N tile with an LDS-DMA ring and two wave groups half a K-step apart (context encoding)
-// =====================================================================================
-// The 128 x 128 kernel above pulls 16 KiB of activations + 8 (16) KiB of weights per 64-deep K-step for 2.1 MFLOP.  A CU takes in 55 - 65 GB/s
-// once half of it comes from HBM (64 KiB of requests in flight, 1.2 us each; from L2 it takes 125 GB/s), so the tile grows: 128 tokens x 256
-// weight rows = 16 + 16 (32) KiB for 4.2 MFLOP, 256 x 256 = 32 + 16 (32) KiB for 8.4.  Eight waves as 2 (tokens) x 4 (weight
-// rows): activation fragments are shared by four waves, weight fragments by two.  Both operands arrive by LDS-DMA
-// (global_load_lds, 1 KiB per wave-instruction: the weight tiles land lane-linear = fragment
-// order; the activation rows land in the XOR-swizzled image of the kernel above, the swizzle being
-// applied to the per-lane SOURCE address) into a ring of stages: all but the one being multiplied are in
-// flight, retired by counted vmcnt waits in front of raw barriers -- no ordinary global
-// load in the loop, so hipcc has nothing to drain.  A wave's K-step is a READ phase (fragments LDS -> registers, then the requests of a later
-// K-step) and a MULTIPLY phase (MFMAs, the weight codes decoded between them), and the two waves of a SIMD are in opposite phases
-// (see "Schedule" in the kernel).
-// What it holds on full grids (gate|up of the 8B model, 2031 tokens): bf16 1.22, fp8 1.27, int8 1.22 PF/s (1.16 before the codes were decoded
-// between the MFMAs), where a library product of 8192^3 in bf16 runs at 1.28 on this card; 128-token blocks 1.13 / 1.18 / 1.05.
-constexpr int kWideBN = 256;
-template <int WD> constexpr int kWideWBytes = (WD == MI_W_BF16 ? 32 : 16) * 1024;   // 256 weight rows of a 64-deep K-step
-// as many stages as the LDS holds: 144 or 160 KiB
-template <int WD, int BM> constexpr int kWideStages = 160 * 1024 / (kWideWBytes<WD> + BM * 128);
+// instantiated in gemm_wide_bf16.hip / gemm_wide_f8.hip / gemm_wide_i8.hip
+extern template int launch_gemm_wide_wd<MI_W_BF16>(const LinearW&, int, const uint16_t*, int, int, const EpiArgs&, hipStream_t, int, int, int, float*, SlabSum*);
+extern template int launch_gemm_wide_wd<MI_W_F8E4M3>(const LinearW&, int, const uint16_t*, int, int, const EpiArgs&, hipStream_t, int, int, int, float*, SlabSum*);
+extern template int launch_gemm_wide_wd<MI_W_INT8>(const LinearW&, int, const uint16_t*, int, int, const EpiArgs&, hipStream_t, int, int, int, float*, SlabSum*);
 
-// Waits until at most the youngest min(left, MOST) K-steps' DMAs (PER each) of this wave are in flight.
-template <int PER, int MOST>
-__device__ __forceinline__ void wait_dma(int left) {
-  if (left >= MOST) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER * MOST) : "memory");
-  else if constexpr (MOST > 0) wait_dma<PER, MOST - 1>(left);
-}
-
-// The tile of this work-group.  Work-group b runs on XCD b % 8: an XCD takes an eighth of the tiles, one after the other with the token
-// blocks of a weight slab in a row, so that a slab comes into its L2 once.  (Every eighth slab to an XCD, as in gemm_kernel, left the XCDs
-// up to a slab apart: 44 slabs of 11 token blocks put 66 work-groups on the 32 CUs of four of them, three rounds in place of two.)
-template <int BM>
-__device__ __forceinline__ bool wide_tile(int T, int NT, int& m0, int& nt0) {
-  const int mtiles = ceil_div(T, BM), tiles = mtiles * ceil_div(NT, kWideBN / 16), per = ceil_div(tiles, 8);
-  const int seq = blockIdx.x >> 3, t = (blockIdx.x & 7) * per + seq;
-  if (seq >= per || t >= tiles) return false;
-  nt0 = t / mtiles * (kWideBN / 16);
-  m0 = t % mtiles * BM;
-  return true;
-}
-// the K-steps of grid.z slice blockIdx.z: equal ones, the last may be shorter (the launch leaves none empty)
-template <bool SPLIT>
-__device__ __forceinline__ void wide_slice(int K, int& ks0, int& nks) {
-  const int all = K / 64, per = SPLIT ? ceil_div(all, (int)gridDim.z) : all;
-  ks0 = SPLIT ? (int)blockIdx.z * per : 0;
-  nks = min(per, all - ks0);
-}
-
-// BM = 128: each wave 64 x 64 (64 accumulator registers).  BM = 256: each 128 x 64 (128 accumulator registers, 246 VGPRs
-// with the decoded fragments of one K-step).
-// SPLIT: grid.z K-slices write raw fp32 accumulators to slab[z][m][n] (see gemm_a8_kernel).
-template <int WD, int EPI, int BM, bool SPLIT>
-__global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict__ W, int NT, int KT, int T, int K,
-                                                        const uint16_t* __restrict__ x, int ldx, EpiArgs e,
-                                                        float* __restrict__ slab) {
-  static_assert(BM == 128 || (BM == 256 && WD != MI_W_BF16), "token block");   // 256 tokens of bf16 weights: gemm_wide16_kernel
-  // waves as 2 (tokens) x 4 (weight rows), each MT 16-token tiles x 4 16-row weight tiles (4 x 2 waves would read 16 instead of 20 KiB of
-  // fragments per K-step but decode every weight code four times instead of twice)
-  constexpr int MT = BM / 32;                 // 16-token tiles per wave
-  constexpr int WM = 2, NTW = 4;
-  constexpr int XP = BM / 64;                 // 8-row activation pieces per wave and stage
-  constexpr int WP = kWideWBytes<WD> / 8192;  // 1 KiB weight tiles per wave and stage
-  constexpr int WPK = WP / 2;                 // weight tiles per 16 rows and K-step
-  constexpr int kStages = kWideStages<WD, BM>, kStage = kWideWBytes<WD> + BM * 128;
-  constexpr int kDma = WP + XP;               // DMAs per wave and stage
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int g = lane >> 4, c = lane & 15;
-  const int wm = wave % WM, wn = wave / WM;
-  int m0, ntb;
-  if (!wide_tile<BM>(T, NT, m0, ntb)) return;
-  int ks0, nks;                               // this slice's K-steps, from K-step ks0 on
-  wide_slice<SPLIT>(K, ks0, nks);
-
-  // this lane's DMA sources: wave w brings weight tiles 2w, 2w + 1 of the work-group's 16 (fragment
-  // order) and XP 8-row pieces of the activation tile
-  const uint4* wsrc[2];
-  const uint16_t* xsrc[XP];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) wsrc[i] = W + ((size_t)min(ntb + 2 * wave + i, NT - 1) * KT + ks0 * WPK) * 64 + lane;
-#pragma unroll
-  for (int i = 0; i < XP; ++i) {
-    const int r = (XP * wave + i) * 8 + (lane >> 3), sl = lane & 7;
-    xsrc[i] = x + (size_t)min(m0 + r, T - 1) * ldx + (size_t)ks0 * 64 + ((sl ^ xs_swz<WD>(r)) * 8);   // LDS slot sl of row r holds chunk sl ^ swz(r)
-  }
-  auto issue = [&](int ks, int stage) {
-    unsigned char* st = smem + stage * kStage;
-#pragma unroll
-    for (int i = 0; i < WP; ++i)   // tile (row tile i / WPK, k tile i % WPK)
-      glds16(wsrc[i / WPK] + ((size_t)ks * WPK + i % WPK) * 64, st + (WP * wave + i) * 1024);
-#pragma unroll
-    for (int i = 0; i < XP; ++i) glds16(xsrc[i] + (size_t)ks * 64, st + kWideWBytes<WD> + (XP * wave + i) * 1024);
-  };
-
-  f32x4_t acc[NTW][MT];
-#pragma unroll
-  for (int i = 0; i < NTW; ++i)
-#pragma unroll
-    for (int j = 0; j < MT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  // Schedule.  A K-step of a wave is two phases: READ (its fragments, 20 KiB at BM = 256, from LDS into registers) and MULTIPLY
-  // (2 NTW MT MFMAs from registers).  With one barrier per K-step every wave is in the same phase at the same time, the two waves
-  // of a SIMD included, and LDS-read time and MFMA time add up: 1.7 us per K-step at BM = 256 against 1.0 us of MFMAs.  Here
-  // the two wave groups (waves 0-3 / 4-7 = the two waves of every SIMD) run half a K-step apart -- group 1 executes one
-  // barrier more at the start -- so one group multiplies while the other reads:
-  //     physical barrier:      P0        P1        P2        P3        P4  ...
-  //     group 0 (waves 0-3):   | READ 0  | MUL 0   | READ 1  | MUL 1   | ...
-  //     group 1 (waves 4-7):   |         | READ 0  | MUL 0   | READ 1  | MUL 1 ...
-  // Stage k is read in [P2k, P2k+2]; K-step k + kStages - 1 goes into the stage of K-step k - 1 (read until P2k), requested by every wave
-  // behind its top barrier of iteration k, kStages - 1 K-steps ahead of its first read.  A wave waits for ITS pieces of a
-  // stage before the barrier in front of the stage's first read by anyone (group 0: its top barrier; group 1: its second one).
-  const int grp = __builtin_amdgcn_readfirstlane(wave >> 2);
-#pragma unroll
-  for (int k = 0; k + 1 < kStages; ++k)
-    if (k < nks) issue(k, k);
-  if (grp == 1) {   // its pieces of stage 0 are in before P0
-    wait_dma<kDma, kStages - 2>(nks - 1);
-    __builtin_amdgcn_s_barrier();           // P0
-  }
-  int cur = 0, fill = kStages - 1;          // the stages of K-step ks and of K-step ks + kStages - 1
-  for (int ks = 0; ks < nks; ++ks) {
-    if (grp == 0) wait_dma<kDma, kStages - 2>(nks - 1 - ks);   // own pieces of stage ks
-    __builtin_amdgcn_s_barrier();           // group 0: P2ks | group 1: P2ks+1 -- either way nobody reads stage ks - 1 any more
-    const unsigned char* st = smem + cur * kStage;
-    const uint4* xs = reinterpret_cast<const uint4*>(st + kWideWBytes<WD>);
-    u32x4_t b0[MT], b1[MT], w0[NTW], w1[NTW];
-#pragma unroll
-    for (int i = 0; i < NTW; ++i) {
-      const u32x4_t* w = reinterpret_cast<const u32x4_t*>(st + (wn * NTW + i) * (WPK * 1024) + lane * 16);
-      w0[i] = w[0];
-      if constexpr (WD == MI_W_BF16) w1[i] = w[64];
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int r = wm * (BM / 2) + mt * 16 + c;
-      const int ch0 = WD == MI_W_BF16 ? g : 2 * g, ch1 = WD == MI_W_BF16 ? 4 + g : 2 * g + 1;
-      b0[mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + (ch0 ^ xs_swz<WD>(r))]);
-      b1[mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + (ch1 ^ xs_swz<WD>(r))]);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    if (ks + kStages - 1 < nks) issue(ks + kStages - 1, fill);
-    __builtin_amdgcn_sched_barrier(0);
-    cur = cur + 1 == kStages ? 0 : cur + 1;
-    fill = fill + 1 == kStages ? 0 : fill + 1;
-    // the fragments are in registers (the empty asm takes them as operands: the compiler's wait for the reads sits in front of it)
-#pragma unroll
-    for (int i = 0; i < NTW; ++i) {
-      asm volatile("" : "+v"(w0[i]));
-      if constexpr (WD == MI_W_BF16) asm volatile("" : "+v"(w1[i]));
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) { asm volatile("" : "+v"(b0[mt])); asm volatile("" : "+v"(b1[mt])); }
-    if (grp == 1 && ks + 1 < nks) wait_dma<kDma, kStages - 2>(nks - 2 - ks);   // own pieces of stage ks + 1: group 0 reads it behind the next barrier
-    __builtin_amdgcn_s_barrier();           // group 0: P2ks+1 | group 1: P2ks+2
-    __builtin_amdgcn_sched_barrier(0);
-    // the codes of weight tile i + 1 are decoded between the MFMAs of tile i, whose 16 cycles leave room for three vector instructions each
-    u32x4_t a[2], an[2];
-    auto piece = [&](const u32x4_t& w, int q) { const uint32_t v = w[q >> 1]; return decode2<WD>(v, q & 1); };
-    if constexpr (WD != MI_W_BF16) {
-#pragma unroll
-      for (int q = 0; q < 8; ++q) a[q >> 2][q & 3] = piece(w0[0], q);
-    }
-#pragma unroll
-    for (int i = 0; i < NTW; ++i) {
-      if constexpr (WD == MI_W_BF16) { a[0] = w0[i]; a[1] = w1[i]; }
-#pragma unroll
-      for (int m2 = 0; m2 < 2 * MT; ++m2) {   // both halves of a K-step one after the other: two MFMAs in a row never meet in an accumulator
-        const int h = m2 / MT, mt = m2 % MT;
-        acc[i][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[h]), __builtin_bit_cast(bf16x8_t, h ? b1[mt] : b0[mt]), acc[i][mt], 0, 0, 0);
-        if constexpr (WD != MI_W_BF16) {
-          if (i + 1 < NTW) {
-#pragma unroll
-            for (int q = m2 * 4 / MT; q < (m2 + 1) * 4 / MT; ++q) an[q >> 2][q & 3] = piece(w0[i + 1], q);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-      if constexpr (WD != MI_W_BF16) { a[0] = an[0]; a[1] = an[1]; }
-    }
-  }
-  if (grp == 0) __builtin_amdgcn_s_barrier();   // the barrier group 1 executed first
-#pragma unroll
-  for (int i = 0; i < NTW; ++i) {
-    const int nt = ntb + wn * NTW + i;
-    if (nt >= NT) continue;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int m = m0 + wm * (BM / 2) + mt * 16 + c;
-      if (m >= T) continue;
-      if constexpr (SPLIT) {
-        *reinterpret_cast<float4*>(slab + ((size_t)blockIdx.z * T + m) * (NT * 16) + nt * 16 + g * 4) =
-            make_float4(acc[i][mt][0], acc[i][mt][1], acc[i][mt][2], acc[i][mt][3]);
-      } else {
-        epilogue<EPI>(e, m, nt * 16 + g * 4, acc[i][mt]);
-      }
-    }
-  }
-}
-
-// The same for bf16 weights at 256 tokens x 256 weight rows.  A 64-deep stage of it is 64 KiB, and the LDS holds two; the stagger
-// needs a third.  So a K-step is 32 deep (one weight tile per 16 rows; 32 MFMAs a wave), the weights ride in four stages of 16 KiB, and the
-// activations, whose rows are fetched 128 bytes at a time, in three of 64-deep pairs of K-steps (32 KiB): 160 KiB.  K-step s requests the weights
-// of s + 3 and one half of the rows of the pair behind the next, four DMAs a wave, so what K-step s reads was requested by K-step s - 3 at
-// the latest and eight younger DMAs stay in flight.
-template <int EPI, bool SPLIT>
-__global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restrict__ W, int NT, int KT, int T, int K,
-                                                          const uint16_t* __restrict__ x, int ldx, EpiArgs e,
-                                                          float* __restrict__ slab) {
-  constexpr int BM = 256, MT = 8, WM = 2, NTW = 4, kW = 16 * 1024, kX = 32 * 1024, kXs = 4 * kW;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int g = lane >> 4, c = lane & 15;
-  const int wm = wave % WM, wn = wave / WM;
-  int m0, ntb;
-  if (!wide_tile<BM>(T, NT, m0, ntb)) return;
-  int ks0, nks;
-  wide_slice<SPLIT>(K, ks0, nks);
-  const int s0 = 2 * ks0, n = 2 * nks;        // this slice's 32-deep K-steps
-
-  const uint4* wsrc[2];
-  const uint16_t* xsrc[4];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) wsrc[i] = W + ((size_t)min(ntb + 2 * wave + i, NT - 1) * KT + s0) * 64 + lane;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = (4 * wave + i) * 8 + (lane >> 3), sl = lane & 7;
-    xsrc[i] = x + (size_t)min(m0 + r, T - 1) * ldx + (size_t)s0 * 32 + ((sl ^ xs_swz<MI_W_BF16>(r)) * 8);
-  }
-  auto issue_w = [&](int s) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) glds16(wsrc[i] + (size_t)s * 64, smem + (s & 3) * kW + (2 * wave + i) * 1024);
-  };
-  auto issue_x = [&](int p, int half, int stage) {   // half of this wave's rows of pair p
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int q = 2 * half + i;
-      glds16((half ? xsrc[2 + i] : xsrc[i]) + (size_t)p * 64, smem + kXs + stage * kX + (4 * wave + q) * 1024);
-    }
-  };
-  // own pieces of K-step s are in: the requests of the last two K-steps may be out, fewer of them at the end
-  auto wait_for = [&](int s) {
-    const int left = n - 1 - s;
-    if (left >= 3) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    else if (left == 2) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-    else if (left == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  };
-
-  f32x4_t acc[NTW][MT];
-#pragma unroll
-  for (int i = 0; i < NTW; ++i)
-#pragma unroll
-    for (int j = 0; j < MT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  const int grp = __builtin_amdgcn_readfirstlane(wave >> 2);
-  issue_x(0, 0, 0);
-  issue_x(0, 1, 0);
-  issue_w(0);
-  issue_w(1);
-  if (n > 2) {
-    issue_x(1, 0, 1);
-    issue_w(2);
-    issue_x(1, 1, 1);
-  }
-  if (grp == 1) {
-    wait_for(0);
-    __builtin_amdgcn_s_barrier();           // P0
-  }
-  auto step = [&](int s, int half, int xcur, int xfill) {
-    if (grp == 0) wait_for(s);
-    __builtin_amdgcn_s_barrier();           // group 0: P2s | group 1: P2s+1
-    const unsigned char* st = smem + (s & 3) * kW;
-    const uint4* xs = reinterpret_cast<const uint4*>(smem + kXs + xcur * kX);
-    u32x4_t b[MT], a[NTW];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int r = wm * (BM / 2) + mt * 16 + c;
-      b[mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + ((4 * half + g) ^ xs_swz<MI_W_BF16>(r))]);
-    }
-#pragma unroll
-    for (int i = 0; i < NTW; ++i) a[i] = *reinterpret_cast<const u32x4_t*>(st + (wn * NTW + i) * 1024 + lane * 16);
-    __builtin_amdgcn_sched_barrier(0);
-    if (s + 3 < n) issue_w(s + 3);
-    if ((s >> 1) + 2 < (n >> 1)) issue_x((s >> 1) + 2, half, xfill);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(b[mt]));
-#pragma unroll
-    for (int i = 0; i < NTW; ++i) asm volatile("" : "+v"(a[i]));
-    if (grp == 1 && s + 1 < n) wait_for(s + 1);
-    __builtin_amdgcn_s_barrier();           // group 0: P2s+1 | group 1: P2s+2
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < NTW; ++i)
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-        acc[i][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[i]), __builtin_bit_cast(bf16x8_t, b[mt]), acc[i][mt], 0, 0, 0);
-  };
-  int xcur = 0, xfill = 2;
-  for (int s = 0; s < n; s += 2) {
-    step(s, 0, xcur, xfill);
-    step(s + 1, 1, xcur, xfill);
-    xcur = xcur == 2 ? 0 : xcur + 1;
-    xfill = xfill == 2 ? 0 : xfill + 1;
-  }
-  if (grp == 0) __builtin_amdgcn_s_barrier();   // the barrier group 1 executed first
-#pragma unroll
-  for (int i = 0; i < NTW; ++i) {
-    const int nt = ntb + wn * NTW + i;
-    if (nt >= NT) continue;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int m = m0 + wm * (BM / 2) + mt * 16 + c;
-      if (m >= T) continue;
-      if constexpr (SPLIT) {
-        *reinterpret_cast<float4*>(slab + ((size_t)blockIdx.z * T + m) * (NT * 16) + nt * 16 + g * 4) =
-            make_float4(acc[i][mt][0], acc[i][mt][1], acc[i][mt][2], acc[i][mt][3]);
-      } else {
-        epilogue<EPI>(e, m, nt * 16 + g * 4, acc[i][mt]);
-      }
-    }
-  }
-}
-
-template <int WD, int EPI, int BM, bool SPLIT>
-static auto gemm_wide_fn() {
-  if constexpr (WD == MI_W_BF16 && BM == 256) return gemm_wide16_kernel<EPI, SPLIT>;
-  else return gemm_wide_kernel<WD, EPI, BM, SPLIT>;
-}
-
-template <int WD, int BM>
-static int launch_gemm_wide_bm(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
-                               int KS, float* splitk_ws, SlabSum* defer) {
-  const int NT = w.N / 16, KT = w.K / tile_k(WD);
-  dim3 grid(8 * ceil_div(ceil_div(T, BM) * ceil_div(w.N, kWideBN), 8), 1, KS);
-  const uint4* W = reinterpret_cast<const uint4*>(w.w);
-  constexpr int lds = WD == MI_W_BF16 && BM == 256 ? 160 * 1024 : kWideStages<WD, BM> * (kWideWBytes<WD> + BM * 128);
-#define MI_GW(EPI_) \
-  do { \
-    if (KS == 1) { \
-      const auto fn = gemm_wide_fn<WD, EPI_, BM, false>(); \
-      MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)); \
-      hipLaunchKernelGGL(fn, grid, dim3(512), lds, s, W, NT, KT, T, w.K, x, ldx, e, nullptr); \
-    } else { \
-      const auto fn = gemm_wide_fn<WD, EPI_, BM, true>(); \
-      MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)); \
-      hipLaunchKernelGGL(fn, grid, dim3(512), lds, s, W, NT, KT, T, w.K, x, ldx, e, splitk_ws); \
-      if (defer && (EPI_ == EPI_RESID || EPI_ == EPI_F32)) { *defer = SlabSum{splitk_ws, KS, T, w.N, e.scale, e.bias, e.row_scale}; } \
-      else hipLaunchKernelGGL((splitk_reduce_kernel<EPI_>), dim3(ceil_div(T * (w.N / 4), 256)), dim3(256), 0, s, splitk_ws, KS, T, w.N, e); \
-    } \
-  } while (0)
-  if (epi == EPI_QKV) MI_GW(EPI_QKV);
-  else if (epi == EPI_SWIGLU) MI_GW(EPI_SWIGLU);
-  else if (epi == EPI_RESID) MI_GW(EPI_RESID);
-  else if (epi >= EPI_RELU2) {
-    if constexpr (WD == MI_W_BF16) {
-      if (epi == EPI_RELU2) MI_GW(EPI_RELU2);
-      else if (epi == EPI_GLU_CLIP) MI_GW(EPI_GLU_CLIP);
-      else if (epi == EPI_SOFTCAP) MI_GW(EPI_SOFTCAP);
-      else MI_GW(EPI_HEADS_KV);
-    } else { set_error("gemm_wide: this epilogue is built for bf16 weights"); return MI_EINVAL; }
-  } else MI_GW(EPI_F32);
-#undef MI_GW
-  MI_HIP(hipGetLastError());
-  return MI_OK;
-}
-// Which token block and K-split: the cheapest of a model of the kernel, us, fitted to 113 shapes (60 .. 4000 tokens, the projections of TinyLlama,
-// Llama-8B, Qwen2.5-7B and of the layer stacks; every block and split of each timed; the choice is 1.3 % from the fastest, 18 % at worst).  The
-// kernel holds 144 - 160 KiB of LDS, i.e. ONE work-group per CU, so a launch is rounds of 32 work-groups on each of the eight XCDs: 6.5 us, and
-// a round 2.6 us of ramp and epilogue beside its K-steps.  Time per 64-deep K-step, on an almost empty and on a full chip:
-//     128 tokens: fp8 0.49 / 0.77, bf16 0.68 / 0.80, int8 0.66 / 0.88;  256 tokens: fp8 0.95 / 1.36, bf16 0.93 / 1.51, int8 0.99 / 1.43
-// A K-split writes its slabs, and a second launch sums them (0.215 us per MB both ways), or the row norm that follows reads them.
-// Against the rule before it and the 128 x 128 kernel, us: bf16 gate|up of the 8B model 1000 tokens 298 -> 200, 350 tokens 151 -> 104, 128 tokens
-// 80 -> 64; its down projection 1000 tokens 199 -> 98, 350 tokens 104 -> 62; fp8 gate|up 128 tokens 55 -> 44, 33 tokens 48 -> 36.
-struct WidePlan { int bm, ks; };   // bm 0: the shape has no plan
+// Which tile and K-split: the cheapest of a model of the kernel, us, fitted to 167 shapes (40 .. 4000 tokens, the projections of TinyLlama,
+// Llama-8B, Qwen2.5-7B and of the layer stacks; every tile and up to eight splits of each timed; the choice is 1.6 % from the fastest on average).  The
+// kernel holds more than half of a CU's LDS, i.e. ONE work-group per CU, so a launch is rounds of 32 work-groups on each of the eight XCDs: 4.1 us, and
+// a round a ramp and epilogue that grow with the tile, beside its K-steps.  us per 64-deep K-step on an almost empty and on a full chip:
+//     128 x 256: fp8 0.53 / 0.79, bf16 0.75 / 0.83, int8 0.75 / 0.89;  256 x 256: fp8 0.91 / 1.33, bf16 0.89 / 1.46, int8 0.88 / 1.37
+//     192 x 192: fp8 0.57 / 0.89, bf16 0.70 / 0.86, int8 0.67 / 0.95;   64 x 128: fp8 0.22 / 0.35, bf16 0.31 / 0.39, int8 0.39 / 0.43
+// A K-split writes its slabs, and a second launch sums them, or the row norm that follows reads them.
+// Against the best of 128 x 256 and 256 x 256 alone, us: int8 gate|up of the 7B model at 188 tokens 79 -> 60 (148 tiles of 256 x 256 on 256 CUs, 73 % of
+// each filled; 198 of 192 x 192), its down projection 41.6 -> 34.4; bf16 gate|up of TinyLlama 700 tokens 51.6 -> 35.4, 200 tokens 28.4 -> 21.4;
+// fp8 QKV of the 8B model 1400 tokens 82.6 -> 63.9; bf16 down projection of 2048 x 14336 at 100 tokens 26.4 -> 17.6.
+struct WidePlan { int bm, ntw, ks; };   // bm 0: the shape has no plan
 static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, bool deferred) {
   int cus = 256;
   if (device_num_cu(&cus) != MI_OK || cus < 8) cus = 256;
-  static const double kStep[3][2][2] = {{{0.68, 0.80}, {0.93, 1.51}}, {{0.49, 0.77}, {0.95, 1.36}}, {{0.66, 0.88}, {0.99, 1.43}}};
+  // us per 64-deep K-step on an almost empty chip and on a full one: {1, m ntw, m, ntw}, m = bm / 64
+  static const double kStep[3][2][4] = {{{0., 0.0310, 0.0289, 0.1119}, {0.0113, 0.0104, 0.1250, 0.1172}}, {{0.0923, 0.0475, 0., 0.0152}, {0.1645, 0.0627, 0.0207, 0.0208}},
+                                        {{0.0451, 0.0015, 0.0629, 0.1408}, {0.1990, 0.0565, 0.0129, 0.0542}}};
   const int nks = K / 64;
-  WidePlan best{0, 1};
+  const double mb = (double)T * N * 4e-6;
+  WidePlan best{0, 4, 1};
   double best_cost = 0.;
-  for (int bm = 128; bm <= 256; bm *= 2) {
-    const int tiles = ceil_div(T, bm) * ceil_div(N, kWideBN);
-    for (int ks = 1; ks <= 10; ++ks) {
-      const int per = ceil_div(nks, ks);
-      if (ks > 1 && (per < 4 || (ks - 1) * per >= nks || (size_t)ks * T * N * sizeof(float) > ws_bytes)) continue;
-      const double fill = std::min(1.0, (double)tiles * ks / cus), *st = kStep[wd][bm / 256];
-      const int rounds = ceil_div(ceil_div(tiles, 8) * ks, std::max(1, cus / 8));
-      double cost = 6.5 + rounds * (2.6 + per * (st[0] + (st[1] - st[0]) * fill));
-      const double mb = (double)T * N * 4e-6;
-      if (ks > 1) cost += deferred ? 0.15 * ks * mb : 2.7 + 0.215 * (ks + 1) * mb;
-      if (best.bm == 0 || cost < best_cost) { best = WidePlan{bm, ks}; best_cost = cost; }
+  for (int bm = 64; bm <= 256; bm += 64)
+    for (int ntw = 2; ntw <= 4; ++ntw) {
+      if (wd == MI_W_BF16 && !wide_tile_built<MI_W_BF16>(bm, ntw)) continue;
+      const double m = bm / 64, area = m * ntw;
+      const auto us = [&](const double (&k)[4]) { return k[0] + k[1] * area + k[2] * m + k[3] * ntw; };
+      double lo = us(kStep[wd][0]), hi = us(kStep[wd][1]);
+      if (wd == MI_W_BF16 && bm == 256 && ntw == 4) { lo = 0.893; hi = 1.456; }   // (the kernel with 32-deep K-steps)
+      if (bm == 192) hi *= 1.04;
+      const int tiles = ceil_div(T, bm) * ceil_div(N, 64 * ntw);
+      for (int ks = 1; ks <= 10; ++ks) {
+        const int per = ceil_div(nks, ks);
+        if (ks > 1 && (per < 4 || (ks - 1) * per >= nks || (size_t)ks * T * N * sizeof(float) > ws_bytes)) continue;
+        const int rounds = ceil_div(ceil_div(tiles, 8) * ks, std::max(1, cus / 8));
+        double body = rounds * (1.2 + 0.42 * area + per * (lo + (hi - lo) * std::min(1.0, (double)tiles * ks / cus)));
+        if (rounds * cus - tiles * ks < 6) body *= 1.028 + 0.0032 * area;   // no CU to spare: the slowest decides
+        double cost = 4.1 + body;
+        if (ks > 1) cost += deferred ? 0.144 * ks * mb : 2.65 + 0.179 * (ks + 1) * mb;
+        if (best.bm == 0 || cost < best_cost) { best = WidePlan{bm, ntw, ks}; best_cost = cost; }
+      }
     }
-  }
   return best;
 }
 static int gemm_wide_mode() {   // MI355X_GEMM_WIDE: 0 never, 1 whenever the shape allows, unset: by size
@@ -661,47 +305,37 @@ static int gemm_wide_mode() {   // MI355X_GEMM_WIDE: 0 never, 1 whenever the sha
   return m;
 }
 static int gemm_wide_bm() {      // MI355X_GEMM_WIDE_BM: 128 / 256 forces the token block (default: by grid size)
-  static const int m = [] { const char* v = getenv("MI355X_GEMM_WIDE_BM"); return v ? atoi(v) : 0; }();
+  static const int m = [] { const char* v = getenv("MI355X_GEMM_WIDE_BM"); const int b = v ? atoi(v) : 0; return b == 128 || b == 256 ? b : 0; }();
   return m;
 }
 static int gemm_wide_ks() {      // MI355X_GEMM_WIDE_KS: 1 = never split K in the wide kernel
   static const int m = [] { const char* v = getenv("MI355X_GEMM_WIDE_KS"); return v ? atoi(v) : 0; }();
   return m;
 }
-template <int WD>
-static int launch_gemm_wide_wd(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
-                               float* splitk_ws, size_t splitk_ws_bytes, SlabSum* defer, int force_bm, int force_ks, bool split_as_deferred) {
-  WidePlan pl = gemm_wide_plan(T, w.N, w.K, gemm_wide_ks() == 1 || !splitk_ws ? 0 : splitk_ws_bytes, w.wd, split_as_deferred || (defer && (epi == EPI_RESID || epi == EPI_F32)));
-  const int forced_bm = force_bm ? force_bm : gemm_wide_bm();
-  if (forced_bm == 128 || forced_bm == 256) pl = WidePlan{forced_bm, 1};
-  if (force_ks) {
-    MI_CHECK(force_ks >= 1 && (force_ks - 1) * ceil_div(w.K / 64, force_ks) < w.K / 64 && (force_ks == 1 || (splitk_ws && (size_t)force_ks * T * w.N * 4 <= splitk_ws_bytes)),
-             "gemm_wide: forced K-split must leave no slice empty and fit the workspace");
-    pl.ks = force_ks;
-  }
-  if (pl.bm == 256) return launch_gemm_wide_bm<WD, 256>(w, T, x, ldx, epi, e, s, pl.ks, splitk_ws, defer);
-  return launch_gemm_wide_bm<WD, 128>(w, T, x, ldx, epi, e, s, pl.ks, splitk_ws, defer);
-}
-// The 128 x 128 kernel keeps what is small on both sides: up to 128 tokens of a matrix of up to 17 M weights (33 .. 128 tokens, us: 4096 x 4096
-// fp8 16.3 / 18.4 / 19.5 against 15.8 / 18.8 / 20.9, 3584 x 3584 int8 15.3 / 17.3 / 20.9 against 16.2 / 18.8 / 22.7, 2560 x 2048 bf16
-// 12.6 / - / 17.4 against 12.1 / - / 18.1; 8448 x 2048 bf16 at 100 tokens is past it: 27.7 against 19.7), and grids of less than half the chip where there is no workspace to split K into.
+// The 128 x 128 kernel keeps single 16-row tiles and, where there is no workspace to split K into, grids of less than half the chip.  Everything else is the
+// wide kernel's (us at 60 / 100 - 128 tokens, 128 x 128 -> wide: 4096 x 4096 fp8 18.4 / 19.5 -> 9.4 / 11.8, 2560 x 2048 bf16 12.6 / 17.4 -> 11.0 / 11.6).
 static bool gemm_wide_wanted(const LinearW& w, int T, size_t ws_bytes) {
   if (w.K % 64 != 0 || (w.N / 16) < 2) return false;
   const int mode = gemm_wide_mode();
   if (mode == 1) return true;
   if (mode == 0) return false;
-  if (T <= 128 && (int64_t)w.N * w.K <= 17000000) return false;
-  return ws_bytes > 0 || ceil_div(T, 128) * ceil_div(w.N, kWideBN) >= 128;
+  return ws_bytes > 0 || ceil_div(T, 128) * ceil_div(w.N, 256) >= 128;
 }
 int launch_gemm_wide(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
-                     float* splitk_ws, size_t splitk_ws_bytes, SlabSum* defer, int force_bm, int force_ks, bool split_as_deferred) {
+                     float* splitk_ws, size_t splitk_ws_bytes, SlabSum* defer, bool split_as_deferred, int force_bm, int force_ntw, int force_ks) {
   if (defer) *defer = SlabSum();
   MI_CHECK(w.K % 64 == 0 && ldx % 8 == 0, "gemm_wide: K % 64 == 0");
-  if (w.wd == MI_W_BF16)
-    return launch_gemm_wide_wd<MI_W_BF16>(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer, force_bm, force_ks, split_as_deferred);
-  if (w.wd == MI_W_F8E4M3)
-    return launch_gemm_wide_wd<MI_W_F8E4M3>(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer, force_bm, force_ks, split_as_deferred);
-  return launch_gemm_wide_wd<MI_W_INT8>(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer, force_bm, force_ks, split_as_deferred);
+  WidePlan pl = gemm_wide_plan(T, w.N, w.K, gemm_wide_ks() == 1 || !splitk_ws ? 0 : splitk_ws_bytes, w.wd, split_as_deferred || (defer && (epi == EPI_RESID || epi == EPI_F32)));
+  const int forced_bm = force_bm ? force_bm : gemm_wide_bm();
+  if (forced_bm) pl = WidePlan{forced_bm, force_ntw ? force_ntw : 4, 1};
+  if (force_ks) {
+    MI_CHECK(force_ks >= 1 && (force_ks - 1) * ceil_div(w.K / 64, force_ks) < w.K / 64 && (force_ks == 1 || (splitk_ws && (size_t)force_ks * T * w.N * 4 <= splitk_ws_bytes)),
+             "gemm_wide: forced K-split must leave no slice empty and fit the workspace");
+    pl.ks = force_ks;
+  }
+  if (w.wd == MI_W_BF16) return launch_gemm_wide_wd<MI_W_BF16>(w, T, x, ldx, epi, e, s, pl.bm, pl.ntw, pl.ks, splitk_ws, defer);
+  if (w.wd == MI_W_F8E4M3) return launch_gemm_wide_wd<MI_W_F8E4M3>(w, T, x, ldx, epi, e, s, pl.bm, pl.ntw, pl.ks, splitk_ws, defer);
+  return launch_gemm_wide_wd<MI_W_INT8>(w, T, x, ldx, epi, e, s, pl.bm, pl.ntw, pl.ks, splitk_ws, defer);
 }
 
 int launch_gemm(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
@@ -709,7 +343,7 @@ int launch_gemm(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, co
   if (defer) *defer = SlabSum();
   MI_CHECK(T >= 1, "gemm: T must be >= 1");
   if (gemm_wide_wanted(w, T, splitk_ws ? splitk_ws_bytes : 0) && ldx % 8 == 0)
-    return launch_gemm_wide(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer, 0, 0, split_as_deferred);
+    return launch_gemm_wide(w, T, x, ldx, epi, e, s, splitk_ws, splitk_ws_bytes, defer, split_as_deferred);
   MI_CHECK(w.N % 16 == 0 && w.K % 64 == 0, "gemm: N % 16 == 0 and K % 64 == 0 required");
   MI_CHECK(ldx % 8 == 0, "gemm: x row stride must be a multiple of 8 elements");
   switch (w.wd) {
@@ -992,7 +626,7 @@ int launch_splitk_reduce(const SlabSum& sl, int epi, const EpiArgs& e, hipStream
   const dim3 grid(ceil_div(sl.T * (sl.N / 4), 256));
 #define MI_S(EPI_) case EPI_: hipLaunchKernelGGL((splitk_reduce_kernel<EPI_>), grid, dim3(256), 0, s, sl.slab, sl.KS, sl.T, sl.N, e); break
   switch (epi) {
-    MI_S(EPI_F32); MI_S(EPI_QKV); MI_S(EPI_SWIGLU); MI_S(EPI_RESID); MI_S(EPI_RELU2); MI_S(EPI_GLU_CLIP); MI_S(EPI_SOFTCAP);
+    MI_S(EPI_F32); MI_S(EPI_QKV); MI_S(EPI_SWIGLU); MI_S(EPI_RESID); MI_S(EPI_RELU2); MI_S(EPI_GLU_CLIP); MI_S(EPI_SOFTCAP); MI_S(EPI_HEADS_KV);
     default: set_error("splitk_reduce: unknown epilogue"); return MI_EINVAL;
   }
 #undef MI_S

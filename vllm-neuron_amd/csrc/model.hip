@@ -2071,13 +2071,15 @@ int mi_op_qlinear(const void* x, int32_t M, const void* w_tiled, const float* sc
     return rc;
   }
   if (force_path == 3) return launch_gemm_wide(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream);
-  if (force_path >= 4 && force_path <= 7) {   // the wide GEMM with its K dimension split: 4 / 5 = 2 / 4 slices at 128-token blocks, 6 / 7 at 256
-    const int ks = (force_path & 1) ? 4 : 2, bm = force_path >= 6 ? 256 : 128;
-    MI_CHECK(K / 64 % ks == 0, "qlinear: paths 4 .. 7 need K / 64 a multiple of their slices");
+  // the wide GEMM with its K dimension split: 4 / 5 = 2 / 4 slices at 128-token blocks, 6 / 7 at 256; 100 bm + 10 ntw + ks: tiles of bm tokens x 64 ntw rows, ks slices
+  const bool tile = force_path >= 6400;
+  if (tile || (force_path >= 4 && force_path <= 7)) {
+    const int ks = tile ? force_path % 10 : (force_path & 1) ? 4 : 2, bm = tile ? force_path / 100 : force_path >= 6 ? 256 : 128, ntw = tile ? force_path / 10 % 10 : 4;
+    MI_CHECK(ks >= 1 && (tile || K / 64 % ks == 0), "qlinear: paths 4 .. 7 need K / 64 a multiple of their slices");
     float* slab = nullptr;
     const size_t bytes = (size_t)ks * M * N * 4;
     MI_HIP(hipMalloc(reinterpret_cast<void**>(&slab), bytes));
-    int rc = launch_gemm_wide(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes, nullptr, bm, ks);
+    int rc = launch_gemm_wide(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes, nullptr, false, bm, ntw, ks);
     hipStreamSynchronize((hipStream_t)stream);
     hipFree(slab);
     return rc;
