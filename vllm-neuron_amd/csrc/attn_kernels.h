@@ -20,10 +20,12 @@ int attn_decode_splits(int B, int nkv);
 size_t attn_scratch_bytes(int B, int nh, int hd);
 
 // q [B, nh, hd] bf16 -> out [B, nh*hd] bf16.  ctx_lens[b] = number of keys (incl. the new one).
+// whether a grid too short for the chip still takes each (sequence, kv head) in one work-group, without partials: short contexts (max_ctx: the longest, 0 = not known)
+bool attn_decode_short(int B, int nkv, int hd, int max_ctx);
 int launch_attn_decode(const uint16_t* q, const uint16_t* kpool, const uint16_t* vpool, int block_size,
                        const int32_t* block_table, int MB, const int32_t* ctx_lens, int B, int nh,
                        int nkv, int hd, uint16_t* out, void* scratch, hipStream_t s, bool tickets_zeroed = false,
-                       int rows_per_seq = 1, int num_blocks = 0);
+                       int rows_per_seq = 1, int num_blocks = 0, int max_ctx = 0);
 // num_blocks > 0 (blocks of the pool): a wave's first K/V request does not wait for the context length (ids clamped into the pool)
 // rows_per_seq R > 1: batch rows b R .. b R + R - 1 are one sequence at consecutive positions (block_table row b R
 // serves them all); their heads share the MFMA columns and the sequence's K/V is read once

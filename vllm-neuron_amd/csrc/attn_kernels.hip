@@ -364,6 +364,12 @@ __global__ __launch_bounds__(HD) void attn_combine_kernel(const float* __restric
   out[((size_t)b * nh + head) * HD + d] = f32_to_bf16(L > 0.f ? acc / L : 0.f);   // empty context -> zeros
 }
 
+// Up to 128 tokens of 128-wide heads (256 of 64-wide ones) four waves of one work-group take at most one tile (two) each, and the combine launch costs more
+// than the split gains.  us per step, split + combine -> one launch: TinyLlama 1 row of 40 tokens 880 -> 822, of 250 892 -> 860; 8B fp8 4 rows
+// of 64 / 125 tokens 1160 -> 1115 / 1128, at 250 / 450 tokens 1166 -> 1164 / 1217; 7B int8 6 rows of 200 1300 -> 1293.
+bool attn_decode_short(int B, int nkv, int hd, int max_ctx) {
+  return max_ctx > 0 && max_ctx * hd <= 128 * 128 && attn_decode_splits(B, nkv) > 1;
+}
 int attn_decode_splits(int B, int nkv) {
   int ns = 256 / (B * nkv);  // ~one work-group per CU; >= 4 tiles (one per wave) each at 1k context
   return ns < 1 ? 1 : (ns > kAttnMaxSplits ? kAttnMaxSplits : ns);
@@ -387,7 +393,7 @@ static bool attn_merge_enabled() {
 template <int HD>
 static int launch_decode_t(const uint16_t* q, const uint16_t* kpool, const uint16_t* vpool, int bs,
                            const int32_t* bt, int MB, const int32_t* ctx, int B, int nh, int nkv,
-                           uint16_t* out, void* scratch, hipStream_t s, bool tickets_zeroed, int R, int num_blocks) {
+                           uint16_t* out, void* scratch, hipStream_t s, bool tickets_zeroed, int R, int num_blocks, int max_ctx) {
   const int G = nh / nkv, Bs = B / R, NS = attn_decode_splits(Bs, nkv);   // Bs sequences of R batch rows each
   // in-launch merge: needs every split's work-group resident on a CU of its own (grid <= CUs) and
   // the ticket counters at zero (the model keeps them so; the per-op entry cannot know)
@@ -402,11 +408,15 @@ static int launch_decode_t(const uint16_t* q, const uint16_t* kpool, const uint1
   constexpr size_t kMergeLds = 96 * 1024;   // more than half a CU's LDS: one work-group per CU (see the kernel comment)
   {
     int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(attn_decode_kernel<HD, 8, true>), (int)lds8);
+    if (rc == MI_OK) rc = ensure_dynamic_lds(reinterpret_cast<const void*>(attn_decode_kernel<HD, 4, true>), (int)lds4);
     if (rc == MI_OK) rc = ensure_dynamic_lds(reinterpret_cast<const void*>(attn_decode_kernel<HD, 4, false>), (int)lds4);
     if (rc == MI_OK) rc = ensure_dynamic_lds(reinterpret_cast<const void*>(attn_decode_kernel<HD, 4, false, true>), (int)kMergeLds);
     if (rc != MI_OK) return rc;
   }
-  if (NS == 1) {
+  if (attn_decode_short(Bs, nkv, HD, max_ctx)) {
+    hipLaunchKernelGGL((attn_decode_kernel<HD, 4, true>), dim3(1, nkv, Bs), dim3(256), lds4, s, q,
+                       kpool, vpool, bs, bt, MB, ctx, nh, nkv, G, 1, nullptr, nullptr, out, scale_log2e, nullptr, R, num_blocks);
+  } else if (NS == 1) {
     // Enough (sequence, kv head) pairs to fill the chip: one launch, no partials.  (Measured: a
     // single CU sustains only ~32 GB/s from HBM however many loads its waves keep in flight, so
     // a short grid must split the context over CUs -- the one-launch form at B x nkv = 32 took
@@ -428,14 +438,14 @@ static int launch_decode_t(const uint16_t* q, const uint16_t* kpool, const uint1
 int launch_attn_decode(const uint16_t* q, const uint16_t* kpool, const uint16_t* vpool, int block_size,
                        const int32_t* block_table, int MB, const int32_t* ctx_lens, int B, int nh,
                        int nkv, int hd, uint16_t* out, void* scratch, hipStream_t s, bool tickets_zeroed, int rows_per_seq,
-                       int num_blocks) {
+                       int num_blocks, int max_ctx) {
   MI_CHECK(hd == 64 || hd == 128, "attention: head_dim must be 64 or 128");
   MI_CHECK(rows_per_seq >= 1 && B % rows_per_seq == 0 && (nh / nkv) * rows_per_seq <= 16,
            "attention: rows_per_seq must divide the batch and q heads per kv head x rows_per_seq must be <= 16");
   MI_CHECK(nh % nkv == 0 && nh / nkv <= 16, "attention: q heads per kv head must be 1..16");
   MI_CHECK(block_size % 16 == 0, "attention: block_size must be a multiple of 16");
-  if (hd == 128) return launch_decode_t<128>(q, kpool, vpool, block_size, block_table, MB, ctx_lens, B, nh, nkv, out, scratch, s, tickets_zeroed, rows_per_seq, num_blocks);
-  return launch_decode_t<64>(q, kpool, vpool, block_size, block_table, MB, ctx_lens, B, nh, nkv, out, scratch, s, tickets_zeroed, rows_per_seq, num_blocks);
+  if (hd == 128) return launch_decode_t<128>(q, kpool, vpool, block_size, block_table, MB, ctx_lens, B, nh, nkv, out, scratch, s, tickets_zeroed, rows_per_seq, num_blocks, max_ctx);
+  return launch_decode_t<64>(q, kpool, vpool, block_size, block_table, MB, ctx_lens, B, nh, nkv, out, scratch, s, tickets_zeroed, rows_per_seq, num_blocks, max_ctx);
 }
 
 // =====================================================================================

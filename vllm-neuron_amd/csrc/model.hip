@@ -268,20 +268,21 @@ int run_trunk(mi_ctx* c, int rows, bool decode, int B, int MB, int q_pos0, const
       Scope sc(c, MI_K_ATTN_DECODE);
       MI_TRY(launch_attn_decode(c->qbuf, kpool, vpool, k.block_size, c->d_bt, MB, c->d_ctx, B, c->nh_l,
                                 c->nkv_l, c->hd, c->attn_out, c->attn_scratch, s, /*tickets_zeroed=*/true,
-                                c->attn_rows_per_seq, attn_early_kv() ? k.num_blocks : 0));
+                                c->attn_rows_per_seq, attn_early_kv() ? k.num_blocks : 0, c->attn_max_ctx));
     } else if (segs) {
       Scope sc(c, MI_K_ATTN_PREFILL);
       static const bool batch_decodes = [] { const char* v = getenv("MI355X_RAGGED_DECODE_ATTN"); return !v || v[0] != '0'; }();
       for (int i = 0; i < nseg;) {
         int j = i;
-        while (batch_decodes && j < nseg && segs[j].n == 1) ++j;
+        int ctx = 0;
+        for (; batch_decodes && j < nseg && segs[j].n == 1; ++j) ctx = std::max(ctx, segs[j].pos0 + 1);
         if (j > i) {
           // a run of requests that generate (one token each, consecutive rows and table rows): ONE split-context
           // decode-attention launch for all of them instead of a one-query context encoding per request
           MI_TRY(launch_attn_decode(c->qbuf + (size_t)segs[i].row0 * c->q_dim, kpool, vpool, k.block_size,
                                     c->d_bt + (size_t)i * MB, MB, c->d_seg_ctx + i, j - i, c->nh_l, c->nkv_l, c->hd,
                                     c->attn_out + (size_t)segs[i].row0 * c->q_dim, c->attn_scratch, s, false, 1,
-                                    attn_early_kv() ? k.num_blocks : 0));
+                                    attn_early_kv() ? k.num_blocks : 0, ctx));
           i = j;
           continue;
         }
@@ -571,7 +572,8 @@ float bf16_bits_to_f32(uint16_t h) {
 }
 
 int capture_or_launch_decode(mi_ctx* c, int B, int MB) {
-  const int64_t key = (int64_t)(uint32_t)((B * 65536 + MB) ^ (int)((c->class_mask & 0xff) << 24) ^ ((c->attn_rows_per_seq - 1) << 12)) | (int64_t)(c->head_out != nullptr) << 40;
+  const int64_t key = (int64_t)(uint32_t)((B * 65536 + MB) ^ (int)((c->class_mask & 0xff) << 24) ^ ((c->attn_rows_per_seq - 1) << 12)) | (int64_t)(c->head_out != nullptr) << 40 |
+                      (int64_t)(!c->stack && attn_decode_short(B / c->attn_rows_per_seq, c->nkv_l, c->hd, c->attn_max_ctx)) << 41;
   // a caller-supplied transport runs on the host thread: never captured
   if (!c->cfg.use_graphs || c->prof.on || c->xport_allreduce || (c->stack && c->stack->residuals)) return run_layers(c, B, true, B, MB, 0, B, 0);
   auto it = c->graphs.find(key);
@@ -1304,6 +1306,7 @@ static void decode_stage_begin(mi_ctx* c, int MB, int B, DecodeStage& st) {
     c->bt_shadow_MB = MB;
     std::fill(c->bt_checked.begin(), c->bt_checked.end(), 0);
   }
+  c->attn_max_ctx = 0;
   st.row_lo = B;   // rows whose device copy is stale: [row_lo, row_hi]
   st.row_hi = -1;
 }
@@ -1335,6 +1338,7 @@ static int decode_stage_row(mi_ctx* c, int b, int MB, int64_t id, int64_t pos, i
   c->h_pos[b] = (int32_t)pos;
   c->h_slots[b] = (int32_t)slot;
   c->h_ctx[b] = full;
+  c->attn_max_ctx = std::max(c->attn_max_ctx, full);
   return MI_OK;
 }
 static int decode_stage_push(mi_ctx* c, int MB, const DecodeStage& st) {   // 5 x max_num_seqs ints, + the table rows that changed

@@ -69,6 +69,7 @@ struct mi_ctx {
   float* partial = nullptr;
   uint16_t *xn = nullptr, *qbuf = nullptr, *attn_out = nullptr, *act = nullptr;
   uint8_t* x8 = nullptr;        // FP8-activation GEMM input [rows, K]
+  int attn_max_ctx = 0;         // longest context of the staged token-generation rows (0: none staged)
   float* row_rinv = nullptr;    // 1 / rms of up to 32 rows, for the projection behind the norm
   float* x8_scale = nullptr;    // its per-token scales [rows]
   float* splitk_ws = nullptr;   // fp32 K-split slabs of short-prompt GEMMs
