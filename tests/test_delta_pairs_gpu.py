@@ -1,0 +1,18 @@
+"""The delta rule's prompt scan with two chunks to a barrier (delta_scan_pairs_kernel): every number of chunks modulo its unrolled loop, whole and ragged
+last chunks, wave tiles past the last channel, and launches that end inside a segment, against the recurrence in 64 bits."""
+import pytest
+
+from tests.test_bokulorn_gpu import Delta, close, lib  # noqa: F401  (lib: the fixture)
+
+
+pytestmark = pytest.mark.gpu
+
+
+# one and two channel tiles a wave, all of them used, one and a half of the four waves idle, three of four idle
+@pytest.mark.parametrize("shape", [(2, 2, 128, 128, 4), (3, 1, 80, 48, 3), (2, 1, 64, 32, 2), (4, 4, 16, 200, 2)])
+@pytest.mark.parametrize("lengths,chunks", [([15, 16, 17, 32, 48], 64), ([64, 65, 80, 95, 112], 64), ([128, 129, 144, 193], 64), ([180, 33, 70], 5), ([200, 200], 9)])
+def test_chunks_in_pairs(lib, shape, lengths, chunks):  # noqa: F811
+    x = Delta(lib, *shape, lengths, seed=sum(shape) + sum(lengths))
+    close(*x.step([(i, n) for i, n in enumerate(lengths)], chunks=chunks), 1)
+    for i in range(len(lengths)):
+        x.check_state(i)

@@ -420,7 +420,7 @@ __global__ __launch_bounds__(256) void delta_factors_kernel(DeltaGeom g, DeltaIn
   }
 }
 
-// One work-group per (head, 16 value columns, segment): the chunks of the segment in order.  A wave holds NT 16-channel tiles of the
+// Keys of more than 128 numbers.  One work-group per (head, 16 value columns, segment): the chunks of the segment in order.  A wave holds NT 16-channel tiles of the
 // state as MFMA accumulators, which are the B operands of the next chunk's products as they stand; the partial sums of u and
 // o over the channels meet in LDS, once per chunk.
 template <int NT>
@@ -448,7 +448,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(DeltaGeom g, float* __r
   f32x4_t S[NT];
   // Factors and values of the next kAhead chunks are in flight.  Addresses: a uniform part that moves from chunk to chunk and lane
   // offsets (bytes) that do not.
-  constexpr int kAhead = NT <= 2 ? 4 : 2;
+  constexpr int kAhead = 2;
   struct Frag { f32x4_t w[NT], q[NT], k[NT], e[NT]; float t, m, x; };
   uint32_t off[NT], eoff[NT];
 #pragma unroll
@@ -580,6 +580,259 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(DeltaGeom g, float* __r
       if (wave * NT + t < tiles) S0[(size_t)((wave * NT + t) * 16 + 4 * g4 + r) * g.dvp] = S[t][r];
 }
 
+// The same for up to two tiles of channels a wave (keys of up to 128), two chunks to a barrier.  A chunk's chain is 26 matrix products of 32 cycles a wave,
+// then the meeting of the partial sums (write, barrier, read, add) with the matrix core idle: 0.84 us of which 0.39 are products (2048 tokens of 16 heads,
+// 108 us; half the chip's CUs have no work-group, and a head's state cannot be split further).  The second chunk's u needs the first one's state
+// S1 = e1 S + K1' u1, so with W2 e1 in place of W2 its product with S joins the first chunk's, and what is missing is (-W2 K1') u1, a 16 x 16 matrix
+// that does not depend on the state: it is made one pair ahead, while the partial sums of u come out of LDS.  One meeting and 64 products per
+// pair: 1.46 us, 94 us.  Two pairs of chunks are in registers; a load of the pair after the next is issued as soon as what it replaces is used up.
+// (Its own set of registers for a third pair, or the first chunk's o behind the barrier: 115 and 98 us.)
+constexpr int kOutside = 0x7fff0000;      // beyond any buffer of records
+template <typename F, int... I> __device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F&& f) { (f(std::integral_constant<int, I>()), ...); }
+template <int N, typename F> __device__ __forceinline__ void each(F&& f) { each_of(std::make_integer_sequence<int, N>(), f); }
+
+template <int NT>
+__global__ __launch_bounds__(256) void delta_scan_pairs_kernel(DeltaGeom g, float* __restrict__ state, const int32_t* __restrict__ slots,
+                                                               const AttnSeg* __restrict__ segs, int c0, int nchunks, int nvt, float* __restrict__ records) {
+  __shared__ f32x4_t ps[2][5][4][64];      // o of the pair before (two chunks), G, u1, what u2 has without G u1
+  int id = blockIdx.x, h, vt;
+  if (g.H % 8 == 0) {        // the column blocks of a head on one XCD: they read the same factors
+    const int k = id >> 3;
+    h = (id & 7) + 8 * (k / nvt);
+    vt = k % nvt;
+  } else {
+    h = id / nvt;
+    vt = id % nvt;
+  }
+  const int si = blockIdx.y;
+  const AttnSeg sg = segs[si];
+  if (sg.n < 2) return;
+  int first = 0;             // the segment's first chunk among all
+  for (int i = 0; i < si; ++i) first += segs[i].n < 2 ? 0 : ceil_div(segs[i].n, kC);
+  const int k0 = max(c0 - first, 0), k1 = min(c0 + nchunks - first, ceil_div(sg.n, kC));
+  if (k0 >= k1) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g4 = lane >> 4, c = lane & 15, tiles = g.dkp / 16;
+  const int n = k1 - k0, pairs = n / 4 * 2;      // pairs of chunks, an even number of them; up to three chunks by themselves
+  float* S0 = state + ((size_t)slots[sg.seq] * g.H + h) * g.dkp * g.dvp + vt * 16 + c;
+  struct Chunk { f32x4_t w[NT], q[NT], k[NT], e[NT]; float t, m, x; };
+  struct Pair { Chunk a, b; };
+  f32x4_t kt[NT];            // K' of the next pair's first chunk, with a token per lane
+  f32x4_t S[NT];
+  // The records of this segment's chunks as a buffer: a load is one instruction (lane offsets that do not change, a scalar one per chunk), and tiles
+  // past the last one lie outside of it, so that they read as zero and their part of S stays zero.
+  const size_t rec = record_floats(g.dkp, g.dvp) * sizeof(float);
+  float* const base = records + ((size_t)h * nchunks + (first + k0 - c0)) * (rec / sizeof(float));
+  const auto buf = __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)((k1 - k0) * rec), 0x00020000);
+  const int region = 16 * g.dkp * (int)sizeof(float);
+  int woff[NT], qoff[NT], koff[NT], eoff[NT], ktoff[NT];
+  bool live[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int tile = wave * NT + t, in_tile = (tile * 256 + c * 16 + 4 * g4) * 4;
+    live[t] = tile < tiles;
+    woff[t] = live[t] ? in_tile : kOutside;
+    qoff[t] = live[t] ? region + in_tile : kOutside;
+    koff[t] = live[t] ? 2 * region + in_tile : kOutside;
+    ktoff[t] = live[t] ? 2 * region + (tile * 256 + 4 * g4 * 16 + c) * 4 : kOutside;
+    eoff[t] = live[t] ? 3 * region + (tile * 16 + 4 * g4) * 4 : kOutside;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[t][r] = sg.pos0 + k0 > 0 && live[t] ? S0[(size_t)(tile * 16 + 4 * g4 + r) * g.dvp] : 0.f;
+  }
+  const int rest = 49 * g.dkp * (int)sizeof(float), toff = rest + (c * 16 + 4 * wave + g4) * 4, values = rest + 2048 + vt * 1024;
+  const int xoff = values + ((4 * wave + g4) * 16 + c) * 4, ooff = values + ((4 * g4 + wave) * 16 + c) * 4;
+  auto record = [&](int k) { return min(k, n - 1) * (int)rec; };      // (past the last chunk: its own factors again, not used)
+  auto load4 = [&](int at, int from) { return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(buf, at, from, 0)); };
+  auto load1 = [&](int at, int from) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buf, at, from, 0)); };
+  auto load_w = [&](int F, Chunk& f, int t) { f.w[t] = load4(woff[t], F); };
+  auto load_q = [&](int F, Chunk& f, int t) { f.q[t] = load4(qoff[t], F); };
+  auto load_k = [&](int F, Chunk& f, int t) { f.k[t] = load4(koff[t], F); };
+  auto load_e = [&](int F, Chunk& f, int t) { f.e[t] = load4(eoff[t], F); };
+  auto load_t = [&](int F, Chunk& f) { f.t = load1(toff, F); };
+  auto load_m = [&](int F, Chunk& f) { f.m = load1(toff + 1024, F); };
+  auto load_x = [&](int F, Chunk& f) { f.x = load1(xoff, F); };
+  auto load_kt = [&](int F, int t) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) kt[t][r] = load1(ktoff[t] + r * 64, F);
+  };
+  auto load_pair = [&](int p, Pair& f) {
+    const int A = record(2 * p), B = record(2 * p + 1);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      load_w(A, f.a, t); load_w(B, f.b, t); load_e(A, f.a, t); load_q(A, f.a, t); load_k(A, f.a, t); load_e(B, f.b, t); load_k(B, f.b, t); load_q(B, f.b, t);
+    }
+    load_t(A, f.a); load_x(A, f.a); load_m(A, f.a);
+    load_t(B, f.b); load_x(B, f.b); load_m(B, f.b);
+  };
+  auto meet = [] {      // LDS alone: the loads of later chunks stay in flight across the barrier
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto pin = [] { __builtin_amdgcn_sched_barrier(0x6); };       // (ALU instructions may cross)
+  struct Parts { f32x4_t v[4]; __device__ __forceinline__ f32x4_t sum() const { return f32x4_t{v[0][0] + v[1][0] + v[2][0] + v[3][0], v[0][1] + v[1][1] + v[2][1] + v[3][1], v[0][2] + v[1][2] + v[2][2] + v[3][2], v[0][3] + v[1][3] + v[2][3] + v[3][3]}; } };
+  auto parts = [&](const f32x4_t (&p)[4][64]) { return Parts{{p[0][lane], p[1][lane], p[2][lane], p[3][lane]}}; };
+  auto out_parts = [&](const f32x4_t (&p)[4][64]) {      // this thread's number of a chunk's output
+    const float* po = reinterpret_cast<const float*>(&p[0][0]) + lane * 4 + wave;
+    return f32x4_t{po[0], po[256], po[512], po[768]};
+  };
+  auto all4 = [](f32x4_t v) { return v[0] + v[1] + v[2] + v[3]; };
+  auto put_out = [&](int k, float v) { __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), buf, ooff, __builtin_amdgcn_readfirstlane(record(k)), 0); };      // in place of the chunk's values
+  auto coupling = [&](const Chunk& second, auto&& between) {      // this wave's part of (-W2 K1')^T: what it leaves in a lane is the A operand of G u1
+    f32x4_t gt = {0.f, 0.f, 0.f, 0.f};
+    each<4 * NT>([&](auto i) {
+      constexpr int t = decltype(i)::value / 4, r = decltype(i)::value % 4;
+      gt = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[t][r], second.w[t][r], gt, 0, 0, 0);
+      between(i);
+    });
+    return gt;
+  };
+  f32x4_t o1 = {0.f, 0.f, 0.f, 0.f}, o2 = o1, gt = o1;
+  Pair f[2];
+  auto step = [&](int p, Pair& now, Pair& next) {
+    const int b = p & 1, A = record(2 * p + 4), B = record(2 * p + 5), Bn = record(2 * p + 3);
+    const float xb = now.b.x;
+    ps[b][0][wave][lane] = o1;
+    ps[b][1][wave][lane] = o2;
+    ps[b][2][wave][lane] = gt;
+    f32x4_t u1 = {0.f, 0.f, 0.f, 0.f}, u2 = u1, Sg[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) now.b.w[t][r] *= now.a.e[t][r];
+    each<4 * NT>([&](auto i) {
+      constexpr int I = decltype(i)::value, t = I / 4, r = I % 4;
+      u1 = __builtin_amdgcn_mfma_f32_16x16x4f32(now.a.w[t][r], S[t][r], u1, 0, 0, 0);
+      u2 = __builtin_amdgcn_mfma_f32_16x16x4f32(now.b.w[t][r], S[t][r], u2, 0, 0, 0);
+      pin();
+      if (r == 0) load_q(Bn, next.b, t);       // (what the step before used up last)
+      if (r == 3) { load_w(B, now.b, t); load_w(A, now.a, t); }
+      pin();
+    });
+    u1 = __builtin_amdgcn_mfma_f32_16x16x4f32(now.a.t, now.a.x, u1, 0, 0, 0);
+    u2 = __builtin_amdgcn_mfma_f32_16x16x4f32(now.b.t, now.b.x, u2, 0, 0, 0);
+    ps[b][3][wave][lane] = u1;
+    ps[b][4][wave][lane] = u2;
+    pin();
+    o1 = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    each<4 * NT>([&](auto i) {
+      constexpr int I = decltype(i)::value, t = I / 4, r = I % 4;
+      o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(now.a.q[t][r], S[t][r], o1, 0, 0, 0);
+      pin();
+      if (I == 0) load_m(Bn, next.b);
+      if (I == 1) load_t(A, now.a);
+      if (I == 2) load_t(B, now.b);
+      if (r == 3) load_q(A, now.a, t);
+      pin();
+    });
+    o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(now.a.m, now.a.x, o1, 0, 0, 0);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) Sg[t] = f32x4_t{S[t][0] * now.a.e[t][0], S[t][1] * now.a.e[t][1], S[t][2] * now.a.e[t][2], S[t][3] * now.a.e[t][3]};
+    meet();
+    const Parts p1 = parts(ps[b][3]), pg = parts(ps[b][2]), p2 = parts(ps[b][4]);
+    const f32x4_t q1 = out_parts(ps[b][0]), q2 = out_parts(ps[b][1]);
+    __builtin_amdgcn_sched_barrier(0);         // (the reads leave together, and the products of the coupling run while they are on their way)
+    gt = coupling(next.b, [&](auto i) {
+      constexpr int I = decltype(i)::value;
+      pin();
+      if (I == 0) load_x(B, now.b);
+      if (I == 1) load_m(A, now.a);
+      if (I == 2) load_x(A, now.a);
+      if (I % 4 == 3) load_e(A, now.a, I / 4);
+      pin();
+    });
+    const float out1 = all4(q1), out2 = all4(q2);
+    u1 = p1.sum();
+    const f32x4_t G = pg.sum();
+    u2 = p2.sum();
+    each<4>([&](auto i) {
+      constexpr int r = decltype(i)::value;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) Sg[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.a.k[t][r], u1[r], Sg[t], 0, 0, 0);
+      u2 = __builtin_amdgcn_mfma_f32_16x16x4f32(G[r], u1[r], u2, 0, 0, 0);
+      pin();
+      if (r < NT) load_kt(A, r);
+      pin();
+    });
+#pragma unroll
+    for (int t = 0; t < NT; ++t) S[t] = f32x4_t{Sg[t][0] * now.b.e[t][0], Sg[t][1] * now.b.e[t][1], Sg[t][2] * now.b.e[t][2], Sg[t][3] * now.b.e[t][3]};
+    each<4>([&](auto i) {
+      constexpr int r = decltype(i)::value;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.b.k[t][r], u2[r], S[t], 0, 0, 0);
+      pin();
+      if (r < NT) load_k(A, now.a, r);
+      else if (r < 2 * NT) load_e(B, now.b, r - NT);
+      pin();
+    });
+    o2 = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    each<4 * NT>([&](auto i) {
+      constexpr int I = decltype(i)::value, t = I / 4, r = I % 4;
+      o2 = __builtin_amdgcn_mfma_f32_16x16x4f32(now.b.q[t][r], Sg[t][r], o2, 0, 0, 0);
+      pin();
+      if (r == 1) load_k(B, now.b, t);
+      pin();
+    });
+    o2 = __builtin_amdgcn_mfma_f32_16x16x4f32(now.b.m, xb, o2, 0, 0, 0);
+    if (p > 0) {
+      put_out(2 * p - 2, out1);
+      put_out(2 * p - 1, out2);
+    }
+  };
+  load_pair(0, f[0]);
+  load_pair(1, f[1]);
+  if (pairs > 0) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) load_kt(record(0), t);
+    gt = coupling(f[0].b, [](auto) {});
+#pragma unroll
+    for (int t = 0; t < NT; ++t) load_kt(record(2), t);
+    int p = 0;
+    do {
+      step(p, f[0], f[1]);
+      step(p + 1, f[1], f[0]);
+      p += 2;
+    } while (p < pairs);
+    ps[0][0][wave][lane] = o1;
+    ps[0][1][wave][lane] = o2;
+    __syncthreads();
+    put_out(2 * pairs - 2, all4(out_parts(ps[0][0])));
+    put_out(2 * pairs - 1, all4(out_parts(ps[0][1])));
+  }
+  auto single = [&](int k, int b, const Chunk& f) {
+    f32x4_t u = {0.f, 0.f, 0.f, 0.f}, o = u;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        u = __builtin_amdgcn_mfma_f32_16x16x4f32(f.w[t][r], S[t][r], u, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_16x16x4f32(f.q[t][r], S[t][r], o, 0, 0, 0);
+      }
+    u = __builtin_amdgcn_mfma_f32_16x16x4f32(f.t, f.x, u, 0, 0, 0);
+    o = __builtin_amdgcn_mfma_f32_16x16x4f32(f.m, f.x, o, 0, 0, 0);
+    ps[b][3][wave][lane] = u;
+    ps[b][4][wave][lane] = o;
+    __syncthreads();
+    u = parts(ps[b][3]).sum();
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      S[t] = f32x4_t{S[t][0] * f.e[t][0], S[t][1] * f.e[t][1], S[t][2] * f.e[t][2], S[t][3] * f.e[t][3]};
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.k[t][r], u[r], S[t], 0, 0, 0);
+    }
+    put_out(k, all4(out_parts(ps[b][4])));
+  };
+  if (2 * pairs < n) single(2 * pairs, 0, f[0].a);
+  if (2 * pairs + 1 < n) single(2 * pairs + 1, 1, f[0].b);
+  if (2 * pairs + 2 < n) single(2 * pairs + 2, 0, f[1].a);
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (live[t]) S0[(size_t)((wave * NT + t) * 16 + 4 * g4 + r) * g.dvp] = S[t][r];
+}
+
 // norm and gate: a wave per head, eight (four) of the chunk's tokens at a time; the work-groups of a segment's last chunk renew its ring
 template <typename T, int NV>
 __global__ __launch_bounds__(256) void delta_out_kernel(DeltaGeom g, DeltaIn in, const AttnSeg* __restrict__ segs, int nseg, int c0, float* __restrict__ records,
@@ -685,10 +938,12 @@ int launch_delta_prompt(const DeltaGeom& g, const DeltaIn& in, const AttnSeg* sd
       default: MI_DF(0);
     }
 #undef MI_DF
-    if (nt == 1) MI_DS(1);
-    else if (nt == 2) MI_DS(2);
-    else if (nt == 3) MI_DS(3);
+#define MI_DP(NT) hipLaunchKernelGGL((delta_scan_pairs_kernel<NT>), gs, dim3(256), 0, s, g, in.state, in.slots, sd, c0, n, nvt, records)
+    if (nt == 1) MI_DP(1);
+    else if (nt == 2) MI_DP(2);
+    else if (nt == 3) MI_DS(3);      // (three sets of two chunks do not fit the registers)
     else MI_DS(4);
+#undef MI_DP
 #undef MI_DS
 #define MI_DO(NV) \
     if (f32) hipLaunchKernelGGL((delta_out_kernel<float, NV>), go, dim3(256), 0, s, g, in, sd, nseg, c0, records, (float*)y, ldy); \
