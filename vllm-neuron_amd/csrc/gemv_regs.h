@@ -194,7 +194,8 @@ static int launch_gemv_regs_k(const LinearW& w, int M, const uint16_t* x, int ld
 }
 
 // Over how many slices K goes: what the registers need at least, and more where whole rows of K would leave CUs idle (2048 x 2048: 128 row-tiles) if the
-// sums have a taker.  us: a work-group's bytes at 24 GB/s, the slabs, and a launch that adds them where no row norm does.
+// sums have a taker.  us: a work-group's weights at 24 GB/s, its rows at 50 GB/s, the slabs both ways, and a launch that adds them where no row norm does.
+// (Without the rows' term, us a step: 8B fp8 32 rows 2150, 2099 with it; bf16 24 rows 2323, 2261; 7B int8 24 rows 1820, 1801; Rapodra 20 rows 731, 721.)
 template <int WD>
 static int gemv_regs_slices(int M, int N, int K, size_t ws_bytes, bool deferred, int num_cu) {
   const int NT = N / 16, KT = K / tile_k(WD);
@@ -203,8 +204,8 @@ static int gemv_regs_slices(int M, int N, int K, size_t ws_bytes, bool deferred,
   for (int z = ceil_div(KT, kGemvWaves * kRegsMaxTiles<WD>); z <= 8; ++z) {
     const int per = ceil_div(KT, z);
     if (z > 1 && ((z - 1) * per >= KT || (size_t)z * M * N * sizeof(float) > ws_bytes)) continue;
-    double cost = ceil_div(NT, std::max(1, num_cu / z)) * (per / 24.0 + 0.3);
-    if (z > 1) cost += (deferred ? 0.5 : 4.5) + z * (double)M * N * 8e-6 / 4.0;
+    double cost = ceil_div(NT, std::max(1, num_cu / z)) * (per / 24.0 + 0.3) + (double)M * per * tile_k(WD) * 4e-5;
+    if (z > 1) cost += (deferred ? 0.5 : 4.5) + z * (double)M * N * 1e-6;
     if (best == 0 || cost < best_cost) { best = z; best_cost = cost; }
   }
   return best;
