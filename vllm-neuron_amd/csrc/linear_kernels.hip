@@ -618,8 +618,14 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   const int nq = N >> 2;
   if (q >= T * nq) return;
   const int m = q / nq, n0 = (q - m * nq) * 4;
-  const float4 v = slab_sum4(slab + (size_t)m * N + n0, (size_t)T * N, KS);
-  epilogue<EPI>(e, m, n0, f32x4_t{v.x, v.y, v.z, v.w});
+  // what the epilogue needs is requested in front of the slabs, and what hangs off it (the rotary factors) behind their requests
+  EpiPre<EPI> pre;
+  epi_prefetch<EPI>(e, m, n0, pre);
+  const float4 sc = *reinterpret_cast<const float4*>(e.scale + n0), bi = e.bias ? *reinterpret_cast<const float4*>(e.bias + n0) : make_float4(0.f, 0.f, 0.f, 0.f);
+  const float rs = e.row_scale ? e.row_scale[m] : 1.f;
+  const float4 v = slab_sum4(slab + (size_t)m * N + n0, (size_t)T * N, KS, [&] { epi_prefetch_dependent<EPI>(e, n0, pre); });
+  const float sc4[4] = {sc.x, sc.y, sc.z, sc.w}, b4[4] = {bi.x, bi.y, bi.z, bi.w};
+  epilogue_pre<EPI>(e, m, n0, sc4, e.bias ? b4 : nullptr, f32x4_t{v.x, v.y, v.z, v.w}, pre, rs);
 }
 
 int launch_splitk_reduce(const SlabSum& sl, int epi, const EpiArgs& e, hipStream_t s) {

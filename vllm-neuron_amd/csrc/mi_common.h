@@ -184,13 +184,16 @@ struct SlabSum {
 #ifdef __HIPCC__
 // The sum of KS slabs' four numbers at p, `stride` numbers apart, in slice order.  Five requests leave before the first is waited for: one after the
 // other they cost a trip to memory each (the row norm over 8 slabs of 242 x 4096: 13.9 us that way, 9.3 now, of which the bytes take 6.3).
-__device__ __forceinline__ float4 slab_sum4(const float* __restrict__ p, size_t stride, int KS) {
+struct Nothing { __device__ __forceinline__ void operator()() const {} };
+template <typename F = Nothing>      // between(): other requests, behind the first slabs' ones
+__device__ __forceinline__ float4 slab_sum4(const float* __restrict__ p, size_t stride, int KS, F&& between = F()) {
   constexpr int U = 5;
   float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
   for (int z = 0; z < KS; z += U) {
     float4 q[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) q[u] = *reinterpret_cast<const float4*>(p + (size_t)min(z + u, KS - 1) * stride);
+    if (z == 0) between();
 #pragma unroll
     for (int u = 0; u < U; ++u)
       if (z + u < KS) { v.x += q[u].x; v.y += q[u].y; v.z += q[u].z; v.w += q[u].w; }

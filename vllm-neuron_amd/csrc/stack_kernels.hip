@@ -68,7 +68,8 @@ __global__ __launch_bounds__(256) void embed_pos_kernel(const int32_t* __restric
   }
 }
 
-template <typename T>
+// ONE: a float4 per thread, its weights requested with the row (else a trip to memory behind the two sums).
+template <typename T, bool ONE>
 __global__ __launch_bounds__(1024) void layernorm_rows_kernel(const float* __restrict__ resid_in, float* __restrict__ resid_out,
                                                              int D, int ld, float eps, NormOut na, NormOut nb, int ldy, SlabSum sl) {
   extern __shared__ __attribute__((aligned(16))) float hrow[];  // ld floats + 32
@@ -76,6 +77,12 @@ __global__ __launch_bounds__(1024) void layernorm_rows_kernel(const float* __res
   const size_t o = (size_t)t * ld;
   float* red = hrow + ld;
   float sum = 0.f;
+  float4 wa = make_float4(0.f, 0.f, 0.f, 0.f), ba = wa, wb = wa, bb = wa;
+  if constexpr (ONE) {
+    const int d = min(tid, ld / 4 - 1) * 4;
+    if (na.y) { wa = *reinterpret_cast<const float4*>(na.w + d); ba = *reinterpret_cast<const float4*>(na.b + d); }
+    if (nb.y) { wb = *reinterpret_cast<const float4*>(nb.w + d); bb = *reinterpret_cast<const float4*>(nb.b + d); }
+  }
   for (int c4 = tid; c4 < ld / 4; c4 += nthr) {
     float4 a = *reinterpret_cast<const float4*>(resid_in + o + c4 * 4);
     if (sl.slab) {   // slabs in slice order, scale, + residual: the arithmetic of splitk_reduce + the residual epilogue
@@ -102,13 +109,13 @@ __global__ __launch_bounds__(1024) void layernorm_rows_kernel(const float* __res
   const float rstd = 1.0f / sqrtf(block_sum(ss, red + 16) / (float)D + eps);
   for (int c4 = tid; c4 < ld / 4; c4 += nthr) {
     const float4 a = *reinterpret_cast<const float4*>(hrow + c4 * 4);
-    auto emit = [&](const NormOut& n) {
-      const float4 w = *reinterpret_cast<const float4*>(n.w + c4 * 4), b = *reinterpret_cast<const float4*>(n.b + c4 * 4);
+    auto emit = [&](const NormOut& n, const float4& w1, const float4& b1) {
+      const float4 w = ONE ? w1 : *reinterpret_cast<const float4*>(n.w + c4 * 4), b = ONE ? b1 : *reinterpret_cast<const float4*>(n.b + c4 * 4);
       put4(reinterpret_cast<T*>(n.y) + (size_t)t * ldy + c4 * 4, a.x * rstd * w.x + b.x, a.y * rstd * w.y + b.y,
            a.z * rstd * w.z + b.z, a.w * rstd * w.w + b.w);
     };
-    if (na.y) emit(na);
-    if (nb.y) emit(nb);
+    if (na.y) emit(na, wa, ba);
+    if (nb.y) emit(nb, wb, bb);
   }
 }
 
@@ -670,11 +677,14 @@ int launch_layernorm_rows(const float* resid_in, float* resid_out, int T, int D,
   // few rows (up to two per CU): one float4 per thread, the row is one round of loads; many rows: 256 threads, several rows per CU
   const int threads = T <= 512 ? std::min(1024, ceil_div(ld / 4, 64) * 64) : 256;
   const SlabSum sl = slabs ? *slabs : SlabSum();
-  if (lds > 64 * 1024)
-    MI_HIP(f32 ? hipFuncSetAttribute(reinterpret_cast<const void*>(layernorm_rows_kernel<float>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)
-               : hipFuncSetAttribute(reinterpret_cast<const void*>(layernorm_rows_kernel<uint16_t>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  if (f32) hipLaunchKernelGGL((layernorm_rows_kernel<float>), dim3(T), dim3(threads), lds, s, resid_in, resid_out, D, ld, eps, a, b, ldy, sl);
-  else hipLaunchKernelGGL((layernorm_rows_kernel<uint16_t>), dim3(T), dim3(threads), lds, s, resid_in, resid_out, D, ld, eps, a, b, ldy, sl);
+  const bool one = threads * 4 >= ld;
+#define MI_LN(T_, ONE_) do { \
+    if (lds > 64 * 1024) MI_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(layernorm_rows_kernel<T_, ONE_>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
+    hipLaunchKernelGGL((layernorm_rows_kernel<T_, ONE_>), dim3(T), dim3(threads), lds, s, resid_in, resid_out, D, ld, eps, a, b, ldy, sl); \
+  } while (0)
+  if (f32) { if (one) MI_LN(float, true); else MI_LN(float, false); }
+  else { if (one) MI_LN(uint16_t, true); else MI_LN(uint16_t, false); }
+#undef MI_LN
   MI_HIP(hipGetLastError());
   return MI_OK;
 }
