@@ -70,12 +70,12 @@ typedef __attribute__((ext_vector_type(4))) short s16x4_t;
 // CU: the launch pads its LDS request to keep it so).  The merge itself runs in split order, so the
 // result does not depend on which work-group performs it.  The counter is left at 0 for the next launch.
 template <int HD, int NW, bool FINAL, bool MERGE = false>
-__global__ __launch_bounds__(NW * 64) void attn_decode_kernel(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kpool, const uint16_t* __restrict__ vpool,
+__device__ __forceinline__ void attn_decode_body(
+    unsigned char* dsm, int split, int kvh, int seq, const uint16_t* __restrict__ q, const uint16_t* __restrict__ kpool, const uint16_t* __restrict__ vpool,
     int bs, const int32_t* __restrict__ block_table, int MB, const int32_t* __restrict__ ctx_lens,
     int nh, int nkv, int G, int NS, float* __restrict__ o_part, float* __restrict__ ml_part,
-    uint16_t* __restrict__ out, float scale_log2e, unsigned int* __restrict__ tickets = nullptr, int R = 1,
-    int num_blocks = 0) {
+    uint16_t* __restrict__ out, float scale_log2e, unsigned int* __restrict__ tickets, int R,
+    int num_blocks) {
   // R > 1 (the target's pass of a speculation step): batch rows b R .. b R + R - 1 are the SAME sequence
   // at consecutive positions (one block-table row, context lengths growing by one).  Their query heads
   // sit side by side in the 16 MFMA columns (column = row-in-sequence * G + head, G R <= 16) and each
@@ -85,11 +85,10 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(
   constexpr int KS = HD / 32, DN = HD / 16;
   constexpr int NV = 32 * CPR / 64; // 16-byte V loads per lane per tile
   constexpr int VT = 32 * KP;       // elements of one wave's V tile
-  extern __shared__ __attribute__((aligned(16))) unsigned char dsm[];
   uint16_t* Vs = reinterpret_cast<uint16_t*>(dsm);                       // [NW][32][KP] bf16
   float* sm_ml = reinterpret_cast<float*>(dsm + (size_t)NW * VT * 2);    // [NW][16][2]
 
-  const int split = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z * R;   // b: first batch row of the sequence
+  const int b = seq * R;                        // first batch row of the sequence
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int g = lane >> 4, c = lane & 15;
   const int Gc = G * R;                         // live MFMA columns
@@ -330,6 +329,17 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(
       }
     }
   }
+}
+template <int HD, int NW, bool FINAL, bool MERGE = false>
+__global__ __launch_bounds__(NW * 64) void attn_decode_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kpool, const uint16_t* __restrict__ vpool,
+    int bs, const int32_t* __restrict__ block_table, int MB, const int32_t* __restrict__ ctx_lens,
+    int nh, int nkv, int G, int NS, float* __restrict__ o_part, float* __restrict__ ml_part,
+    uint16_t* __restrict__ out, float scale_log2e, unsigned int* __restrict__ tickets = nullptr, int R = 1,
+    int num_blocks = 0) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char dsm[];
+  attn_decode_body<HD, NW, FINAL, MERGE>(dsm, blockIdx.x, blockIdx.y, blockIdx.z, q, kpool, vpool, bs, block_table, MB, ctx_lens, nh, nkv, G, NS, o_part, ml_part, out,
+                                         scale_log2e, tickets, R, num_blocks);
 }
 template <int HD, int NW>
 constexpr size_t attn_decode_lds() { return (size_t)NW * 32 * (HD + 8) * 2 + (size_t)NW * 16 * 2 * sizeof(float); }
@@ -747,8 +757,8 @@ __device__ __forceinline__ int kv_swz(int key) {   // XOR key of the 16-byte chu
 constexpr int kPrefillSlices = 6;   // of the keys, at most
 
 template <int HD, int NW>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill2_kernel(
-    const uint16_t* __restrict__ q, int T, int q_pos0, const uint16_t* __restrict__ kpool,
+__device__ __forceinline__ void attn_prefill2_body(
+    unsigned char* smem, int bx, int kvh, int bz, int nz, const uint16_t* __restrict__ q, int T, int q_pos0, const uint16_t* __restrict__ kpool,
     const uint16_t* __restrict__ vpool, int bs, int bs_shift, const int32_t* __restrict__ block_table, int nh, int nkv,
     int G, int Gp, int nblk, int paired, float* __restrict__ o_part, float* __restrict__ ml_part, uint16_t* __restrict__ out, float scale_log2e) {
   constexpr int TK = 64;                       // keys per tile
@@ -763,11 +773,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
   static_assert(NP % NW == 0, "pieces must divide over the waves");
   constexpr int CNT = 2 * PPW;                 // DMA instructions per wave and tile
   constexpr int KSTEPS = HD / 16, DB = HD / 32;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int kvh = blockIdx.y;
   const int QB = NW / Gp;
   const int hl = wave % Gp, slot = wave / Gp;
   const int head = kvh * G + min(hl, G - 1);
@@ -807,15 +815,15 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     int blk_q, pair;
     bool blk_ok;
     if (QB == 1 && !paired) {            // a work-group per block, the heavy ones first
-      pair = blockIdx.x;
+      pair = bx;
       blk_q = nblk - 1 - pair;
       blk_ok = pair < nblk;
-    } else if (QB == 1) {                // one block at a time: the heavy one of pair blockIdx.x, then the light one
-      pair = blockIdx.x;
+    } else if (QB == 1) {                // one block at a time: the heavy one of pair bx, then the light one
+      pair = bx;
       blk_q = pass == 0 ? nblk - 1 - pair : pair;
       blk_ok = pair < npair && !(pass == 1 && pair == nblk - 1 - pair);
     } else {
-      pair = (int)blockIdx.x * (QB >> 1) + (slot >> 1);
+      pair = bx * (QB >> 1) + (slot >> 1);
       blk_q = (slot & 1) ? nblk - 1 - pair : pair;
       blk_ok = pair < npair && !((slot & 1) && pair == nblk - 1 - pair);
     }
@@ -824,12 +832,12 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     // tiles: this wave's, and the work-group's (the heaviest block any of its waves owns)
     const int p_first = q_pos0 + min(q0, T - 1), p_last = q_pos0 + min(q0 + 31, T - 1);
     const int nt_wave = active ? p_last / TK + 1 : 0;
-    int wg_pair0 = QB == 1 ? (int)blockIdx.x : (int)blockIdx.x * (QB >> 1);
+    int wg_pair0 = QB == 1 ? bx : bx * (QB >> 1);
     int wg_blk = QB == 1 ? (pass == 0 ? nblk - 1 - wg_pair0 : wg_pair0) : nblk - 1 - wg_pair0;   // heaviest block of the work-group
     wg_blk = max(min(wg_blk, nblk - 1), 0);
     const int nt_all = (q_pos0 + min(wg_blk * 32 + 31, T - 1)) / TK + 1;
-    // this slice of them: all, or the blockIdx.z-th of gridDim.z slices of the keys
-    const int t_per = ceil_div(nt_all, (int)gridDim.z), t0 = (int)blockIdx.z * t_per, nt = min(nt_all, t0 + t_per);
+    // this slice of them: all, or the bz-th of nz slices of the keys
+    const int t_per = ceil_div(nt_all, nz), t0 = bz * t_per, nt = min(nt_all, t0 + t_per);
 
     // ---- Q fragments (B operand of S^T): Q[q0 + qq][16 ks + 8 h ..] ---------------------------------
     const int qi = min(q0 + qq, T - 1);
@@ -969,7 +977,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
       MI_VREAD(0); MI_VREAD(1); MI_VREAD(2); MI_VREAD(3);
       static_assert(kVAhead == 4, "the prefetch above is written out for 4");
       bf16x8_t pb[4];
-      const float m_exp = gridDim.z > 1 && m_used == -INFINITY ? 0.f : m_used;   // (a slice whose keys so far all lie ahead of this query)
+      const float m_exp = nz > 1 && m_used == -INFINITY ? 0.f : m_used;   // (a slice whose keys so far all lie ahead of this query)
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
         float pv[16];
@@ -1010,8 +1018,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     }
     const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
     const bool st_ok = active && q0 + qq < T;
-    if (gridDim.z > 1) {   // unnormalised, with its maximum and sum: attn_prefill_combine_kernel puts the slices together
-      const size_t row = ((size_t)blockIdx.z * T + q0 + qq) * nh + head;
+    if (nz > 1) {   // unnormalised, with its maximum and sum: attn_prefill_combine_kernel puts the slices together
+      const size_t row = ((size_t)bz * T + q0 + qq) * nh + head;
       if (st_ok && h == 0) *reinterpret_cast<float2*>(ml_part + 2 * row) = make_float2(m_used, lsum);
       if (st_ok && m_used != -INFINITY) {
 #pragma unroll
@@ -1040,6 +1048,33 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
         if (st_ok) *reinterpret_cast<u32x4_t*>(orow + 32 * db + 8 * (k2 + h)) = v;
       }
     __syncthreads();   // the ring is reused by the next pass
+  }
+}
+template <int HD, int NW>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill2_kernel(
+    const uint16_t* __restrict__ q, int T, int q_pos0, const uint16_t* __restrict__ kpool,
+    const uint16_t* __restrict__ vpool, int bs, int bs_shift, const int32_t* __restrict__ block_table, int nh, int nkv,
+    int G, int Gp, int nblk, int paired, float* __restrict__ o_part, float* __restrict__ ml_part, uint16_t* __restrict__ out, float scale_log2e) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  attn_prefill2_body<HD, NW>(smem, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk, paired, o_part,
+                             ml_part, out, scale_log2e);
+}
+
+// A prompt's chunk and the requests that generate beside it, in one launch: neither fills the chip, and one after the other they cost 11.1 + 8.0 us at 239 tokens
+// beside 3 contexts of up to 900 (8B model).  Work-groups (x, y) from `nd` on are the prompt's; those before it one (split, sequence) each of the others.
+struct DecodeSide { const uint16_t* q; const int32_t* block_table; const int32_t* ctx_lens; int MB, NS, nd, num_blocks; float *o_part, *ml_part; uint16_t* out; };
+template <int HD, bool FINAL>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_mixed_kernel(
+    const uint16_t* __restrict__ q, int T, int q_pos0, const uint16_t* __restrict__ kpool,
+    const uint16_t* __restrict__ vpool, int bs, int bs_shift, const int32_t* __restrict__ block_table, int nh, int nkv,
+    int G, int Gp, int nblk, int paired, float* __restrict__ o_part, float* __restrict__ ml_part, uint16_t* __restrict__ out, float scale_log2e, DecodeSide d) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  if ((int)blockIdx.x >= d.nd) {
+    attn_prefill2_body<HD, 8>(smem, (int)blockIdx.x - d.nd, blockIdx.y, blockIdx.z, gridDim.z, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk,
+                              paired, o_part, ml_part, out, scale_log2e);
+  } else if (blockIdx.z == 0) {
+    attn_decode_body<HD, 8, FINAL>(smem, (int)blockIdx.x % d.NS, blockIdx.y, (int)blockIdx.x / d.NS, d.q, kpool, vpool, bs, d.block_table, d.MB, d.ctx_lens, nh, nkv, G, d.NS,
+                                   d.o_part, d.ml_part, d.out, scale_log2e, nullptr, 1, d.num_blocks);
   }
 }
 
@@ -1078,6 +1113,41 @@ static bool attn_prefill_v1() {   // MI355X_ATTN_PREFILL_V1=1: the first-generat
   return on;
 }
 
+static int prefill_heads(int G) { return G <= 1 ? 1 : (G <= 2 ? 2 : (G <= 4 ? 4 : 8)); }
+struct PrefillPlan { int Gp, nblk, bs_shift, paired, gx, ns; float *o_part = nullptr, *ml_part = nullptr; };
+static PrefillPlan prefill_plan(int T, int q_pos0, int block_size, int nh, int nkv, int hd, float* ws, size_t ws_bytes) {
+  // second generation: 8 waves = (8 / Gp) query blocks x Gp heads; blocks in complementary pairs
+  PrefillPlan p;
+  p.Gp = prefill_heads(nh / nkv);
+  const int nblk = ceil_div(T, 32), npair = (nblk + 1) / 2, qb = 8 / p.Gp;
+  int bs_shift = -1;
+  for (int sh = 4; sh < 20; ++sh) if ((1 << sh) == block_size) bs_shift = sh;
+  // One block per work-group (5 .. 8 heads on a kv head): pairs only where single blocks would not all run at once.
+  const int paired = qb > 1 || nblk * nkv > 256;
+  const int gx = paired ? ceil_div(npair, qb >= 2 ? qb / 2 : 1) : nblk;
+  // A short prompt, or the rest of one behind cached keys, leaves most of the chip idle while each work-group walks its tiles, 1.75 us each:
+  // slices of the keys then, at least two tiles each, the cheapest by that and the second launch, which moves every slice's O out and in.
+  // 188 tokens behind 512 cached ones, 28 heads on 4: 40.8 us in 12 work-groups of two passes, 16.7 + 4.8 now.
+  int ns = 1;
+  const int tiles = ceil_div(q_pos0 + T, 64);
+  double best = 1.75 * tiles * ceil_div(gx * nkv, 256);
+  for (int z = 2; ws && z <= kPrefillSlices; ++z) {
+    const size_t part = (size_t)z * T * nh;
+    if (ceil_div(tiles, z) < 2 || part * (hd + 2) * sizeof(float) > ws_bytes) break;
+    const double cost = 1.75 * ceil_div(tiles, z) * ceil_div(gx * nkv * z, 256) + 4.5 + (double)part * hd * 8.0 / 4e6;
+    if (cost < best) { best = cost; ns = z; }
+  }
+  p.nblk = nblk; p.bs_shift = bs_shift; p.paired = paired; p.gx = gx; p.ns = ns;
+  if (ns > 1) { p.o_part = ws; p.ml_part = ws + (size_t)ns * T * nh * hd; }
+  return p;
+}
+static void launch_prefill_combine(const PrefillPlan& p, int T, int nh, int hd, uint16_t* out, hipStream_t s) {
+  if (p.ns <= 1) return;
+  const dim3 grid(ceil_div(T * nh * (hd / 4), 256));
+  if (hd == 128) hipLaunchKernelGGL((attn_prefill_combine_kernel<128>), grid, dim3(256), 0, s, p.o_part, p.ml_part, p.ns, T * nh, out);
+  else hipLaunchKernelGGL((attn_prefill_combine_kernel<64>), grid, dim3(256), 0, s, p.o_part, p.ml_part, p.ns, T * nh, out);
+}
+
 int launch_attn_prefill(const uint16_t* q, int T, int q_pos0, const uint16_t* kpool, const uint16_t* vpool,
                         int block_size, const int32_t* block_table, int nh, int nkv, int hd, uint16_t* out,
                         hipStream_t s, float* ws, size_t ws_bytes) {
@@ -1086,43 +1156,19 @@ int launch_attn_prefill(const uint16_t* q, int T, int q_pos0, const uint16_t* kp
   MI_CHECK(nh % nkv == 0 && nh / nkv <= 8, "attention: q heads per kv head must be 1..8");
   MI_CHECK(ceil_div(q_pos0 + T, block_size) <= kPrefillMaxBlocks, "attention: context spans more than 4096 blocks");
   const int G = nh / nkv;
-  const int Gp = G <= 1 ? 1 : (G <= 2 ? 2 : (G <= 4 ? 4 : 8));
   const float scale_log2e = 1.4426950408889634f / sqrtf((float)hd);
+  const int Gp = prefill_heads(G);
   if (!attn_prefill_v1()) {
-    // second generation: 8 waves = (8 / Gp) query blocks x Gp heads; blocks in complementary pairs
-    const int nblk = ceil_div(T, 32), npair = (nblk + 1) / 2, qb = 8 / Gp;
-    int bs_shift = -1;
-    for (int sh = 4; sh < 20; ++sh) if ((1 << sh) == block_size) bs_shift = sh;
-    // One block per work-group (5 .. 8 heads on a kv head): pairs only where single blocks would not all run at once.
-    const int paired = qb > 1 || nblk * nkv > 256;
-    const int gx = paired ? ceil_div(npair, qb >= 2 ? qb / 2 : 1) : nblk;
-    // A short prompt, or the rest of one behind cached keys, leaves most of the chip idle while each work-group walks its tiles, 1.75 us each:
-    // slices of the keys then, at least two tiles each, the cheapest by that and the second launch, which moves every slice's O out and in.
-    // 188 tokens behind 512 cached ones, 28 heads on 4: 40.8 us in 12 work-groups of two passes, 16.7 + 4.8 now.
-    int ns = 1;
-    const int tiles = ceil_div(q_pos0 + T, 64);
-    double best = 1.75 * tiles * ceil_div(gx * nkv, 256);
-    for (int z = 2; ws && z <= kPrefillSlices; ++z) {
-      const size_t part = (size_t)z * T * nh;
-      if (ceil_div(tiles, z) < 2 || part * (hd + 2) * sizeof(float) > ws_bytes) break;
-      const double cost = 1.75 * ceil_div(tiles, z) * ceil_div(gx * nkv * z, 256) + 4.5 + (double)part * hd * 8.0 / 4e6;
-      if (cost < best) { best = cost; ns = z; }
-    }
-    float *o_part = ns > 1 ? ws : nullptr, *ml_part = ns > 1 ? ws + (size_t)ns * T * nh * hd : nullptr;
-    const dim3 grid2(gx, nkv, ns);
-    if (hd == 128) {
-      constexpr int lds = 3 * 2 * 64 * 256;
-      MI_TRY_A(ensure_dynamic_lds(reinterpret_cast<const void*>(attn_prefill2_kernel<128, 8>), lds));
-      hipLaunchKernelGGL((attn_prefill2_kernel<128, 8>), grid2, dim3(512), lds, s, q, T, q_pos0, kpool, vpool, block_size, bs_shift,
-                         block_table, nh, nkv, G, Gp, nblk, paired, o_part, ml_part, out, scale_log2e);
-      if (ns > 1) hipLaunchKernelGGL((attn_prefill_combine_kernel<128>), dim3(ceil_div(T * nh * (128 / 4), 256)), dim3(256), 0, s, o_part, ml_part, ns, T * nh, out);
-    } else {
-      constexpr int lds = 3 * 2 * 64 * 128;
-      MI_TRY_A(ensure_dynamic_lds(reinterpret_cast<const void*>(attn_prefill2_kernel<64, 8>), lds));
-      hipLaunchKernelGGL((attn_prefill2_kernel<64, 8>), grid2, dim3(512), lds, s, q, T, q_pos0, kpool, vpool, block_size, bs_shift,
-                         block_table, nh, nkv, G, Gp, nblk, paired, o_part, ml_part, out, scale_log2e);
-      if (ns > 1) hipLaunchKernelGGL((attn_prefill_combine_kernel<64>), dim3(ceil_div(T * nh * (64 / 4), 256)), dim3(256), 0, s, o_part, ml_part, ns, T * nh, out);
-    }
+    const PrefillPlan p = prefill_plan(T, q_pos0, block_size, nh, nkv, hd, ws, ws_bytes);
+#define MI_P2(HD_) do { \
+      constexpr int lds = 3 * 2 * 64 * 2 * HD_; \
+      MI_TRY_A(ensure_dynamic_lds(reinterpret_cast<const void*>(attn_prefill2_kernel<HD_, 8>), lds)); \
+      hipLaunchKernelGGL((attn_prefill2_kernel<HD_, 8>), dim3(p.gx, nkv, p.ns), dim3(512), lds, s, q, T, q_pos0, kpool, vpool, block_size, p.bs_shift, \
+                         block_table, nh, nkv, G, p.Gp, p.nblk, p.paired, p.o_part, p.ml_part, out, scale_log2e); \
+    } while (0)
+    if (hd == 128) MI_P2(128); else MI_P2(64);
+#undef MI_P2
+    launch_prefill_combine(p, T, nh, hd, out, s);
     MI_HIP(hipGetLastError());
     return MI_OK;
   }
@@ -1136,6 +1182,46 @@ int launch_attn_prefill(const uint16_t* q, int T, int q_pos0, const uint16_t* kp
 #undef MI_PF
   MI_HIP(hipGetLastError());
   return MI_OK;
+}
+
+// (eight waves a work-group here, four in the launch of its own: half the splits)
+static int mixed_splits(const AttnMixed& m, int nkv, int hd) { return attn_decode_short(m.B, nkv, hd, m.max_ctx) ? 1 : ceil_div(attn_decode_splits(m.B, nkv), 2); }
+template <int HD>
+static int launch_mixed_t(const AttnMixed& m, const PrefillPlan& p, int T, int q_pos0, const uint16_t* q, const int32_t* bt, uint16_t* out, const uint16_t* kpool,
+                          const uint16_t* vpool, int bs, int nh, int nkv, hipStream_t s) {
+  const float scale_log2e = 1.4426950408889634f / sqrtf((float)HD);
+  float* ml_part = reinterpret_cast<float*>(reinterpret_cast<unsigned int*>(m.scratch) + kAttnTickets);
+  float* o_part = ml_part + (size_t)m.B * nh * kAttnMaxSplits * 2;
+  const int NS = mixed_splits(m, nkv, HD);
+  const DecodeSide d{m.q, m.block_table, m.ctx_lens, m.MB, NS, NS * m.B, m.num_blocks, o_part, ml_part, m.out};
+  constexpr int lds = std::max<int>(3 * 2 * 64 * 2 * HD, (int)attn_decode_lds<HD, 8>());
+  const auto fn = NS == 1 ? attn_mixed_kernel<HD, true> : attn_mixed_kernel<HD, false>;
+  MI_TRY_A(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds));
+  hipLaunchKernelGGL(fn, dim3(d.nd + p.gx, nkv, p.ns), dim3(512), lds, s, q, T, q_pos0, kpool, vpool, bs, p.bs_shift, bt, nh, nkv, nh / nkv, p.Gp, p.nblk, p.paired,
+                     p.o_part, p.ml_part, out, scale_log2e, d);
+  if (NS > 1) hipLaunchKernelGGL((attn_combine_kernel<HD>), dim3(nh, m.B), dim3(HD), 0, s, o_part, ml_part, NS, nh, m.out);
+  launch_prefill_combine(p, T, nh, HD, out, s);
+  MI_HIP(hipGetLastError());
+  return MI_OK;
+}
+int launch_attn_mixed(const AttnMixed& m, int T, int q_pos0, const uint16_t* q, const int32_t* block_table, uint16_t* out, const uint16_t* kpool, const uint16_t* vpool,
+                      int block_size, int nh, int nkv, int hd, hipStream_t s, float* ws, size_t ws_bytes) {
+  MI_CHECK(hd == 64 || hd == 128, "attention: head_dim must be 64 or 128");
+  MI_CHECK(block_size % 16 == 0, "attention: block_size must be a multiple of 16");
+  MI_CHECK(T >= 1 && q_pos0 >= 0 && m.B >= 1, "attention: bad T / q_pos0");
+  MI_CHECK(nh % nkv == 0 && nh / nkv <= 8, "attention: q heads per kv head must be 1..8");
+  MI_CHECK(ceil_div(q_pos0 + T, block_size) <= kPrefillMaxBlocks, "attention: context spans more than 4096 blocks");
+  // One launch where both sides find a CU for every work-group; beyond that the prompt's wait behind the others' (us per call, two launches -> one: 8B model
+  // 239 + 3 tokens 3105 -> 2980, 64 + 6 2205 -> 2108, TinyLlama 300 + 4 2385 -> 2245, 8B bf16 500 + 6 4862 -> 4724; 1900 + 3 13035 -> 13097).
+  int num_cu = 0;
+  if (device_num_cu(&num_cu) != MI_OK) return MI_EHIP;
+  const PrefillPlan p = prefill_plan(T, q_pos0, block_size, nh, nkv, hd, ws, ws_bytes);
+  if (attn_prefill_v1() || (p.gx * p.ns + mixed_splits(m, nkv, hd) * m.B) * nkv > num_cu) {
+    int rc = launch_attn_decode(m.q, kpool, vpool, block_size, m.block_table, m.MB, m.ctx_lens, m.B, nh, nkv, hd, m.out, m.scratch, s, false, 1, m.num_blocks, m.max_ctx);
+    return rc != MI_OK ? rc : launch_attn_prefill(q, T, q_pos0, kpool, vpool, block_size, block_table, nh, nkv, hd, out, s, ws, ws_bytes);
+  }
+  return hd == 128 ? launch_mixed_t<128>(m, p, T, q_pos0, q, block_table, out, kpool, vpool, block_size, nh, nkv, s)
+                   : launch_mixed_t<64>(m, p, T, q_pos0, q, block_table, out, kpool, vpool, block_size, nh, nkv, s);
 }
 
 // =====================================================================================

@@ -272,24 +272,43 @@ int run_trunk(mi_ctx* c, int rows, bool decode, int B, int MB, int q_pos0, const
     } else if (segs) {
       Scope sc(c, MI_K_ATTN_PREFILL);
       static const bool batch_decodes = [] { const char* v = getenv("MI355X_RAGGED_DECODE_ATTN"); return !v || v[0] != '0'; }();
-      for (int i = 0; i < nseg;) {
+      // runs of requests that generate (one token each, consecutive rows and table rows): ONE split-context decode-attention launch for all of
+      // a run instead of a one-query context encoding per request; the first run shares its launch with the first prompt segment
+      auto run_end = [&](int i, int& ctx) {
         int j = i;
-        int ctx = 0;
-        for (; batch_decodes && j < nseg && segs[j].n == 1; ++j) ctx = std::max(ctx, segs[j].pos0 + 1);
+        for (ctx = 0; batch_decodes && j < nseg && segs[j].n == 1; ++j) ctx = std::max(ctx, segs[j].pos0 + 1);
+        return j;
+      };
+      const uint16_t* q = c->qbuf;
+      auto rows_of = [&](uint16_t* p, int i) { return p + (size_t)segs[i].row0 * c->q_dim; };
+      int d0 = -1, d1 = -1, dctx = 0, pr = -1;
+      for (int i = 0; i < nseg;) {
+        int ctx;
+        const int j = run_end(i, ctx);
+        if (j > i) { if (d0 < 0) { d0 = i; d1 = j; dctx = ctx; } i = j; }
+        else { if (pr < 0) pr = i; ++i; }
+      }
+      if (d0 >= 0 && pr >= 0) {
+        const AttnMixed m{q + (size_t)segs[d0].row0 * c->q_dim, c->d_bt + (size_t)d0 * MB, c->d_seg_ctx + d0, MB, d1 - d0, dctx, attn_early_kv() ? k.num_blocks : 0,
+                          rows_of(c->attn_out, d0), c->attn_scratch};
+        MI_TRY(launch_attn_mixed(m, segs[pr].n, segs[pr].pos0, rows_of(c->qbuf, pr), c->d_bt + (size_t)pr * MB, rows_of(c->attn_out, pr), kpool, vpool, k.block_size,
+                                 c->nh_l, c->nkv_l, c->hd, s, c->splitk_ws, c->splitk_ws_bytes));
+      }
+      const bool mixed = d0 >= 0 && pr >= 0;
+      for (int i = 0; i < nseg;) {
+        int ctx;
+        const int j = run_end(i, ctx);
         if (j > i) {
-          // a run of requests that generate (one token each, consecutive rows and table rows): ONE split-context
-          // decode-attention launch for all of them instead of a one-query context encoding per request
-          MI_TRY(launch_attn_decode(c->qbuf + (size_t)segs[i].row0 * c->q_dim, kpool, vpool, k.block_size,
-                                    c->d_bt + (size_t)i * MB, MB, c->d_seg_ctx + i, j - i, c->nh_l, c->nkv_l, c->hd,
-                                    c->attn_out + (size_t)segs[i].row0 * c->q_dim, c->attn_scratch, s, false, 1,
-                                    attn_early_kv() ? k.num_blocks : 0, ctx));
+          if (!mixed || i != d0)
+            MI_TRY(launch_attn_decode(rows_of(c->qbuf, i), kpool, vpool, k.block_size, c->d_bt + (size_t)i * MB, MB, c->d_seg_ctx + i, j - i, c->nh_l, c->nkv_l, c->hd,
+                                      rows_of(c->attn_out, i), c->attn_scratch, s, false, 1, attn_early_kv() ? k.num_blocks : 0, ctx));
           i = j;
-          continue;
+        } else {
+          if (!mixed || i != pr)
+            MI_TRY(launch_attn_prefill(rows_of(c->qbuf, i), segs[i].n, segs[i].pos0, kpool, vpool, k.block_size, c->d_bt + (size_t)i * MB, c->nh_l, c->nkv_l, c->hd,
+                                       rows_of(c->attn_out, i), s, c->splitk_ws, c->splitk_ws_bytes));
+          ++i;
         }
-        MI_TRY(launch_attn_prefill(c->qbuf + (size_t)segs[i].row0 * c->q_dim, segs[i].n, segs[i].pos0, kpool, vpool,
-                                   k.block_size, c->d_bt + (size_t)i * MB, c->nh_l, c->nkv_l, c->hd,
-                                   c->attn_out + (size_t)segs[i].row0 * c->q_dim, s, c->splitk_ws, c->splitk_ws_bytes));
-        ++i;
       }
     } else {
       Scope sc(c, MI_K_ATTN_PREFILL);
