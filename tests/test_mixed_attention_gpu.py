@@ -18,6 +18,8 @@ STEPS = [
     ([1, 40, 0], [(0, 1), (1, 1), (2, 33)]),                        # a run, then a prompt; contexts of one tile
     ([600, 128, 129, 700], [(0, 20), (1, 1), (2, 1), (3, 1)]),      # a chunk far into its prompt (slices of its keys), then a run that needs splits
     ([126, 0, 127, 90], [(0, 1), (1, 70), (2, 1), (3, 2)]),         # two runs around a prompt, a second prompt of two tokens
+    ([255, 200, 0, 129], [(0, 1), (1, 1), (2, 65), (3, 1)]),        # a tile for each of eight waves
+    ([256, 200, 0], [(0, 1), (1, 1), (2, 65)]),                     # one token more
     ([500, 31, 0, 0, 300, 640], [(4, 1), (5, 1), (0, 1), (2, 96), (3, 17), (1, 1)]),
 ]
 

@@ -1184,8 +1184,10 @@ int launch_attn_prefill(const uint16_t* q, int T, int q_pos0, const uint16_t* kp
   return MI_OK;
 }
 
-// (eight waves a work-group here, four in the launch of its own: half the splits)
-static int mixed_splits(const AttnMixed& m, int nkv, int hd) { return attn_decode_short(m.B, nkv, hd, m.max_ctx) ? 1 : ceil_div(attn_decode_splits(m.B, nkv), 2); }
+// Eight waves a work-group here, four in the launch of its own: half the splits, and none (so no combine launch) up to 256 tokens of 128-wide heads, 512 of 64-wide
+// ones, twice the other's limit.  us per call, splits -> none: 8B fp8 239 + 3 of 250 tokens 2977 -> 2940, of 500 2974 -> 2988, of 1000 2979 -> 3114; 64 + 6 of 300
+// 2177 -> 2145, of 600 2197 -> 2215; TinyLlama 300 + 4 of 500 2234 -> 2178, of 1000 2228 -> 2296.
+static int mixed_splits(const AttnMixed& m, int nkv, int hd) { return m.max_ctx > 0 && m.max_ctx * hd <= 256 * 128 ? 1 : ceil_div(attn_decode_splits(m.B, nkv), 2); }
 template <int HD>
 static int launch_mixed_t(const AttnMixed& m, const PrefillPlan& p, int T, int q_pos0, const uint16_t* q, const int32_t* bt, uint16_t* out, const uint16_t* kpool,
                           const uint16_t* vpool, int bs, int nh, int nkv, hipStream_t s) {
