@@ -1021,7 +1021,7 @@ __device__ __forceinline__ void attn_prefill2_body(
     if (nz > 1) {   // unnormalised, with its maximum and sum: attn_prefill_combine_kernel puts the slices together
       const size_t row = ((size_t)bz * T + q0 + qq) * nh + head;
       if (st_ok && h == 0) *reinterpret_cast<float2*>(ml_part + 2 * row) = make_float2(m_used, lsum);
-      if (st_ok && m_used != -INFINITY) {
+      if (st_ok && (m_used != -INFINITY || lsum != 0.f)) {   // (a NaN score moves no maximum: the sum carries it)
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -1099,12 +1099,12 @@ __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(const float* 
   float l = 0.f;
 #pragma unroll
   for (int z = 0; z < kPrefillSlices; ++z) {
-    if (z >= ns || ml[z].x == -INFINITY) continue;   // (a slice without a key for this query wrote no O)
+    if (z >= ns || (ml[z].x == -INFINITY && ml[z].y == 0.f)) continue;   // (a slice without a key for this query wrote no O)
     const float w = fexp2(ml[z].x - M);
     l = fmaf(w, ml[z].y, l);
     v.x = fmaf(w, o[z].x, v.x); v.y = fmaf(w, o[z].y, v.y); v.z = fmaf(w, o[z].z, v.z); v.w = fmaf(w, o[z].w, v.w);
   }
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const float inv = 1.f / l;   // every query sees key 0: l is 0 only behind scores that are all -inf, whose row is 0 x inf, the NaN it is without slices
   *reinterpret_cast<uint2*>(out + (size_t)row * HD + d) = make_uint2(pack_bf16x2(v.x * inv, v.y * inv), pack_bf16x2(v.z * inv, v.w * inv));
 }
 
