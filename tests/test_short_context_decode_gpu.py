@@ -1,5 +1,7 @@
 """Decode attention of short contexts (one work-group per sequence and kv head, no partials) and the change to context splits as a batch outgrows it,
 with the captured graph of each form replayed, against the oracle."""
+import time
+
 import pytest
 import torch
 
@@ -32,27 +34,50 @@ def test_contexts_around_the_limit(name, lengths):
     model.close()
 
 
-def test_step_past_the_limit_is_no_pause():
-    """The step with which a batch outgrows the one-launch form has a graph of its own to capture, under the step itself: 1.05 - 1.1 of its neighbours'
-    time (1.4 - 1.8 where the capture waits for it).  The best of four batch sizes, so that a busy host does not count."""
-    import time
+L, BLOCK = 512, 32
+
+
+def _tinyllama():
+    """TinyLlama's decoder: a step long enough (0.9 ms) that a capture beside it, or in its way, tells"""
     from vllm_neuron_amd._native import MI_Q, MI_W, NativeModel
-    L, n = 512, 512 // 32
     model = NativeModel(num_layers=22, hidden_size=2048, num_heads=32, num_kv_heads=4, head_dim=64, intermediate_size=5632, vocab_size=4096, rms_norm_eps=1e-5,
-                        rope_theta=1e4, rope_type=0, rope_factor=1.0, num_blocks=1 + 4 * n, block_size=32, max_num_seqs=4, max_model_len=L,
+                        rope_theta=1e4, rope_type=0, rope_factor=1.0, num_blocks=1 + 4 * (L // BLOCK), block_size=BLOCK, max_num_seqs=4, max_model_len=L,
                         weight_dtype=MI_W["bf16"], quant_type=MI_Q["per_channel_symmetric"], quantize_lm_head=0, tp_degree=1, tp_rank=0, device_id=0,
                         use_graphs=1, ctx_buckets=[L])
     model.init_synthetic_weights(1, 0.02)
     model.finalize()
-    ratios = []
+    return model
+
+
+def _step(B, ctx):
+    n = L // BLOCK
+    return decode_inputs([5] * B, [ctx - 1] * B, [list(range(1 + i * n, 1 + (i + 1) * n)) for i in range(B)], BLOCK, L)
+
+
+def test_step_past_the_limit_is_no_pause():
+    """The step with which a batch outgrows the one-launch form has a graph of its own to capture, under the step itself: 1.05 - 1.1 of its neighbours'
+    time (1.4 - 1.8 where the capture waits for it).  The best of four batch sizes, so that a busy host does not count."""
+    model, ratios = _tinyllama(), []
     for B in (1, 2, 3, 4):
-        blocks = [list(range(1 + i * n, 1 + (i + 1) * n)) for i in range(B)]
         took = {}
         for ctx in range(245, 263):          # contexts of up to 256 tokens are short at 64-wide heads
-            inp = decode_inputs([5] * B, [ctx - 1] * B, blocks, 32, L)
+            inp = _step(B, ctx)
             start = time.perf_counter()
             model.forward(**inp)
             took[ctx] = time.perf_counter() - start
         ratios.append(took[257] / sorted(took[c] for c in took if c not in (245, 257))[8])
+    model.close()
+    assert min(ratios) < 1.3, ratios
+
+
+def test_first_replay_is_the_step_alone():
+    """The step replayed (its logits stay on the device) is another graph than that of the call in front of it (logits to the host): no capture in the
+    time it reports.  The best of four batch sizes again."""
+    model, ratios = _tinyllama(), []
+    for B in (1, 2, 3, 4):
+        ref = model.forward(**_step(B, 300)).clone()
+        first, later = model.replay_decode(2) / 2, model.replay_decode(20) / 20
+        ratios.append(first / later)
+        assert torch.equal(model.forward(**_step(B, 300)), ref)
     model.close()
     assert min(ratios) < 1.3, ratios

@@ -590,11 +590,17 @@ float bf16_bits_to_f32(uint16_t h) {
   return f;
 }
 
+// where the graph of this step is kept: its shape, and the forms that follow from where the logits go and from the staged contexts
+int64_t decode_graph_key(mi_ctx* c, int B, int MB) {
+  return (int64_t)(uint32_t)((B * 65536 + MB) ^ (int)((c->class_mask & 0xff) << 24) ^ ((c->attn_rows_per_seq - 1) << 12)) | (int64_t)(c->head_out != nullptr) << 40 |
+         (int64_t)(!c->stack && attn_decode_short(B / c->attn_rows_per_seq, c->nkv_l, c->hd, c->attn_max_ctx)) << 41;
+}
+// a caller-supplied transport runs on the host thread: never captured
+bool decode_captured(mi_ctx* c) { return c->cfg.use_graphs && !c->prof.on && !c->xport_allreduce && !(c->stack && c->stack->residuals); }
+
 int capture_or_launch_decode(mi_ctx* c, int B, int MB) {
-  const int64_t key = (int64_t)(uint32_t)((B * 65536 + MB) ^ (int)((c->class_mask & 0xff) << 24) ^ ((c->attn_rows_per_seq - 1) << 12)) | (int64_t)(c->head_out != nullptr) << 40 |
-                      (int64_t)(!c->stack && attn_decode_short(B / c->attn_rows_per_seq, c->nkv_l, c->hd, c->attn_max_ctx)) << 41;
-  // a caller-supplied transport runs on the host thread: never captured
-  if (!c->cfg.use_graphs || c->prof.on || c->xport_allreduce || (c->stack && c->stack->residuals)) return run_layers(c, B, true, B, MB, 0, B, 0);
+  if (!decode_captured(c)) return run_layers(c, B, true, B, MB, 0, B, 0);
+  const int64_t key = decode_graph_key(c, B, MB);
   auto it = c->graphs.find(key);
   if (it == c->graphs.end()) {
     // one eager pass first: sets every kernel's attributes outside of capture, which is host work alone and runs beside that pass.  The first step of
@@ -1900,6 +1906,8 @@ int mi_replay_decode(mi_ctx* c, int32_t steps, float* elapsed_ms) {
   MI_CHECK(steps >= 1, "steps must be >= 1");
   MI_HIP(hipSetDevice(c->cfg.device_id));
   set_input_views(c, true);
+  // (the step replayed leaves its logits on the device: behind steps whose head writes the host's buffer that graph is not there yet)
+  if (decode_captured(c) && !c->graphs.count(decode_graph_key(c, c->last_B, c->last_MB))) MI_TRY(capture_or_launch_decode(c, c->last_B, c->last_MB));
   hipEvent_t a, b;
   MI_HIP(hipEventCreate(&a));
   MI_HIP(hipEventCreate(&b));
