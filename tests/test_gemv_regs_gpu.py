@@ -68,3 +68,25 @@ def test_sums_left_to_the_next_norm(family, rows):
         worst = max([worst] + [T.error(o, refs[i % 3][p:p + 1]) for i, o in enumerate(outs)])
     assert worst <= T.LIMIT["bfloat16"], worst
     r.engine.close()
+
+
+@pytest.mark.parametrize("rows", [17, 32])
+def test_fp8_activations_stay_with_prompts(rows):
+    """A down projection deeper than eight slices of the registers (K > 32768) goes to the GEMM from 17 rows on: with bf16 activations there as well, whatever
+    prompts have."""
+    from oracle import DecoderConfig
+    from oracle.synth import make_weights
+    from tests.helpers import decode_inputs
+    from vllm_neuron_amd._native import MI_Q, MI_W, NativeModel
+    shape = dict(num_layers=1, hidden_size=128, num_heads=2, num_kv_heads=1, head_dim=64, intermediate_size=33792, vocab_size=256)
+    w = make_weights(DecoderConfig(**shape), seed=4)
+    out = []
+    for a8 in (0, 1):
+        model = NativeModel(**shape, rms_norm_eps=1e-5, rope_theta=1e4, rope_type=0, rope_factor=1.0, num_blocks=1 + rows, block_size=32, max_num_seqs=rows,
+                            max_model_len=32, weight_dtype=MI_W["f8e4m3"], quant_type=MI_Q["per_channel_symmetric"], quantize_lm_head=1, tp_degree=1, tp_rank=0,
+                            device_id=0, use_graphs=1, ctx_buckets=[32], prefill_fp8_activations=a8)
+        model.load_state_dict(w)
+        model.finalize()
+        out.append(model.forward(**decode_inputs(range(rows), [0] * rows, [[1 + i] for i in range(rows)], 32, 32)).clone())
+        model.close()
+    assert torch.equal(*out)

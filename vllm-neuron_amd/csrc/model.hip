@@ -108,7 +108,7 @@ int run_linear(mi_ctx* c, const Linear& L, int rows, int pro, ProArgs p, int epi
   }
   const uint16_t* x = p.x;
   int ldx = p.ldx;
-  const bool a8 = !regs && c->cfg.prefill_fp8_activations && gemm_a8_supported(L.view());
+  const bool a8 = rows > 32 && c->cfg.prefill_fp8_activations && gemm_a8_supported(L.view());   // (prompts' option: rows a token-generation batch can have keep bf16)
   if (regs && pro == PRO_NORM) e.row_scale = c->row_rinv;
   if (pro == PRO_NORM && !c->runs(MI_K_OTHER)) {   // (class-masked replay: what the norm would have left)
     x = c->xn;
