@@ -19,13 +19,13 @@ constexpr int kAttnMaxSplits = 16;
 int attn_decode_splits(int B, int nkv);
 size_t attn_scratch_bytes(int B, int nh, int hd);
 
-// q [B, nh, hd] bf16 -> out [B, nh*hd] bf16.  ctx_lens[b] = number of keys (incl. the new one).
 // launch_attn_decode of B rows and launch_attn_prefill of one sequence's T tokens in one launch (their outputs and partials are apart)
 struct AttnMixed { const uint16_t* q; const int32_t* block_table; const int32_t* ctx_lens; int MB, B, max_ctx, num_blocks; uint16_t* out; void* scratch; };
 int launch_attn_mixed(const AttnMixed& m, int T, int q_pos0, const uint16_t* q, const int32_t* block_table, uint16_t* out, const uint16_t* kpool, const uint16_t* vpool,
                       int block_size, int nh, int nkv, int hd, hipStream_t s, float* ws, size_t ws_bytes);
-// whether a grid too short for the chip still takes each (sequence, kv head) in one work-group, without partials: short contexts (max_ctx: the longest, 0 = not known)
+// whether a grid too short for the chip still takes each (sequence, kv head) in one work-group, without partials: short contexts
 bool attn_decode_short(int B, int nkv, int hd, int max_ctx);
+// q [B, nh, hd] bf16 -> out [B, nh*hd] bf16.  ctx_lens[b] = number of keys (incl. the new one); max_ctx: the longest, 0 = not known
 int launch_attn_decode(const uint16_t* q, const uint16_t* kpool, const uint16_t* vpool, int block_size,
                        const int32_t* block_table, int MB, const int32_t* ctx_lens, int B, int nh,
                        int nkv, int hd, uint16_t* out, void* scratch, hipStream_t s, bool tickets_zeroed = false,

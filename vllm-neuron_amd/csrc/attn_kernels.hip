@@ -1061,18 +1061,20 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 }
 
 // A prompt's chunk and the requests that generate beside it, in one launch: neither fills the chip, and one after the other they cost 11.1 + 8.0 us at 239 tokens
-// beside 3 contexts of up to 900 (8B model).  Work-groups (x, y) from `nd` on are the prompt's; those before it one (split, sequence) each of the others.
+// beside 3 contexts of up to 900 (8B model).  Work-groups x from `nd` on are the prompt's, gx of every slice of the keys; those before them one
+// (split, sequence) each of the others.
 struct DecodeSide { const uint16_t* q; const int32_t* block_table; const int32_t* ctx_lens; int MB, NS, nd, num_blocks; float *o_part, *ml_part; uint16_t* out; };
 template <int HD, bool FINAL>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_mixed_kernel(
     const uint16_t* __restrict__ q, int T, int q_pos0, const uint16_t* __restrict__ kpool,
     const uint16_t* __restrict__ vpool, int bs, int bs_shift, const int32_t* __restrict__ block_table, int nh, int nkv,
-    int G, int Gp, int nblk, int paired, float* __restrict__ o_part, float* __restrict__ ml_part, uint16_t* __restrict__ out, float scale_log2e, DecodeSide d) {
+    int G, int Gp, int nblk, int paired, int gx, int ns, float* __restrict__ o_part, float* __restrict__ ml_part, uint16_t* __restrict__ out, float scale_log2e, DecodeSide d) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   if ((int)blockIdx.x >= d.nd) {
-    attn_prefill2_body<HD, 8>(smem, (int)blockIdx.x - d.nd, blockIdx.y, blockIdx.z, gridDim.z, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk,
+    const int x = (int)blockIdx.x - d.nd;
+    attn_prefill2_body<HD, 8>(smem, x % gx, blockIdx.y, x / gx, ns, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk,
                               paired, o_part, ml_part, out, scale_log2e);
-  } else if (blockIdx.z == 0) {
+  } else {
     attn_decode_body<HD, 8, FINAL>(smem, (int)blockIdx.x % d.NS, blockIdx.y, (int)blockIdx.x / d.NS, d.q, kpool, vpool, bs, d.block_table, d.MB, d.ctx_lens, nh, nkv, G, d.NS,
                                    d.o_part, d.ml_part, d.out, scale_log2e, nullptr, 1, d.num_blocks);
   }
@@ -1199,8 +1201,8 @@ static int launch_mixed_t(const AttnMixed& m, const PrefillPlan& p, int T, int q
   constexpr int lds = std::max<int>(3 * 2 * 64 * 2 * HD, (int)attn_decode_lds<HD, 8>());
   const auto fn = NS == 1 ? attn_mixed_kernel<HD, true> : attn_mixed_kernel<HD, false>;
   MI_TRY_A(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds));
-  hipLaunchKernelGGL(fn, dim3(d.nd + p.gx, nkv, p.ns), dim3(512), lds, s, q, T, q_pos0, kpool, vpool, bs, p.bs_shift, bt, nh, nkv, nh / nkv, p.Gp, p.nblk, p.paired,
-                     p.o_part, p.ml_part, out, scale_log2e, d);
+  hipLaunchKernelGGL(fn, dim3(d.nd + p.gx * p.ns, nkv), dim3(512), lds, s, q, T, q_pos0, kpool, vpool, bs, p.bs_shift, bt, nh, nkv, nh / nkv, p.Gp, p.nblk, p.paired,
+                     p.gx, p.ns, p.o_part, p.ml_part, out, scale_log2e, d);
   if (NS > 1) hipLaunchKernelGGL((attn_combine_kernel<HD>), dim3(nh, m.B), dim3(HD), 0, s, o_part, ml_part, NS, nh, m.out);
   launch_prefill_combine(p, T, nh, HD, out, s);
   MI_HIP(hipGetLastError());
