@@ -15,7 +15,7 @@
  *                      vllm_neuron/worker/neuronx_distributed_model_loader.py:216-218,236
  *                      (fields: _get_default_neuron_config :725-793, overrides :870-900)
  *   mi_load_weight     checkpoint load + save_quantized_state_dict      loader.py:234-241
- *   mi_init_synthetic_weights   (bench only: no checkpoints exist offline; SURVEY.md §8d)
+ *   mi_init_synthetic_weights   (bench only: no checkpoints exist offline)
  *   mi_finalize        model.compile() + model.load()                    loader.py:240-241
  *   mi_forward         NxDI model __call__ + logits[:, -1, :]            loader.py:339-363
  *   mi_kv_stats        torch.classes.neuron.Runtime().get_vnc_memory_stats()
@@ -429,10 +429,12 @@ int mi_op_quantize_weight(const float* w, int32_t N, int32_t K, int32_t weight_d
 /* Inverse of the tiling for inspection: q_out row-major [N, K] (1 or 2 bytes/elem). */
 int mi_op_untile_weight(const void* tiled, int32_t N, int32_t K, int32_t weight_dtype,
                         void* q_out, void* stream);
-/* y[M, N] fp32 = (x[M, K] bf16 . Wq^T) * scale (+ bias).  M <= 16: weight-streaming GEMV;
- * else MFMA GEMM.  force_path: 0 auto, 1 GEMV, 2 GEMM (picked by size), 3 the wide-N LDS-DMA GEMM (1-byte weights),
- * 4 / 5 that GEMM with K split over 2 / 4 slices at 128-token blocks, 6 / 7 at 256-token blocks (K / 64 a multiple of the slices), 8 the model's GEMM:
- * picked by size with a workspace for K slices. */
+/* y[M, N] fp32 = (x[M, K] bf16 . Wq^T) * scale (+ bias).  force_path: 0 without a workspace: up to 32 rows the weight-streaming kernels of 16 rows
+ * (cut in two beyond), else the GEMM; 1 those kernels (M <= 32); 2 the GEMM (picked by size); 3 the wide LDS-DMA GEMM (1-byte weights);
+ * 4 / 5 that GEMM with K split over 2 / 4 slices at 128-token blocks, 6 / 7 at 256-token blocks (1-byte weights, K / 64 a multiple of the slices);
+ * 8 what the models run, with a workspace of their size for K slices: 5 to 32 rows in registers where K fits them, else up to 16 rows path 1's
+ * kernels, else the GEMM; 100 bm + 10 ntw + ks the wide GEMM in tiles of bm (64, 128, 192, 256) tokens x 64 ntw (2, 3, 4) weight rows and ks
+ * (1 .. 9) K slices. */
 int mi_op_qlinear(const void* x_bf16, int32_t M, const void* w_tiled, const float* scale,
                   const float* bias, int32_t N, int32_t K, int32_t weight_dtype, float* y,
                   int32_t force_path, void* stream);
@@ -443,6 +445,12 @@ int mi_op_qlinear_a8(const void* x_bf16, int32_t M, const void* w_tiled, const f
 /* y[T, H] bf16 = rmsnorm(x[T, H] fp32) * g */
 int mi_op_rmsnorm(const float* x, const float* g, int32_t T, int32_t H, float eps, void* y_bf16,
                   void* stream);
+/* The row norm behind a projection whose K slices are not summed yet: h[T, H] fp32 = resid_in + (sum of slab[KS][T][H]) * scale (* row_scale[t]) (+ bias),
+ * stored to resid_out; then, where y_bf16 is given, y = bf16(rmsnorm(h) * g), or with rinv [T] given, y = bf16(h * g) and rinv = 1 / rms; otherwise
+ * x8 [H / 128][T][128] e4m3 = bf16(rmsnorm(h) * g) / x8_scale[t] (amax / 448), which may be the array row_scale. */
+int mi_op_rmsnorm_slabs(const float* resid_in, const float* slab, int32_t KS, const float* scale, const float* bias,
+                        const float* row_scale, const float* g, int32_t T, int32_t H, float eps, float* resid_out,
+                        void* y_bf16, float* rinv, void* x8, float* x8_scale, void* stream);
 /* Paged KV write.  k, v [T, nkv, hd] bf16; slots [T] (int64; -1 skips).
  * pool layout (library-native): [2][num_blocks][nkv][block_size][hd] bf16. */
 int mi_op_kv_write(const void* k, const void* v, const int64_t* slots, int32_t T, int32_t nkv,

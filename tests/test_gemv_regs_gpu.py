@@ -17,10 +17,11 @@ def lib():
 
 
 # rows: the first and last of each column group; K: fewer k-tiles than waves, an odd share per wave, the first beyond 4 / 8 / 16 tiles a wave, two to eight
-# slices of uneven length; N: one row-tile, one more than the CUs, several passes, more than the passes whose scales fit
+# slices of uneven length, one k-tile more than eight slices hold (the kernels of 16 rows, and the GEMM); N: one row-tile, one more than the CUs, several
+# passes, more than the passes whose scales fit
 @pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
 @pytest.mark.parametrize("M", [5, 16, 17, 32])
-@pytest.mark.parametrize("N,K", [(16, 64), (4112, 320), (272, 1088), (528, 2112), (144, 4096), (48, 4160), (2048, 6208), (16, 28672), (263680, 64), (8208, 1152)])
+@pytest.mark.parametrize("N,K", [(16, 64), (4112, 320), (272, 1088), (528, 2112), (144, 4096), (48, 4160), (2048, 6208), (16, 28672), (263680, 64), (8208, 1152), (32, 32832)])
 def test_edges_of_the_register_gemv(lib, wd, M, N, K):
     g = torch.Generator().manual_seed(M + N + K)
     w = torch.randn(N, K, generator=g) * 0.05

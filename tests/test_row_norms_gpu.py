@@ -36,3 +36,45 @@ def test_layernorm(lib, T, D):  # noqa: F811
     ref = V.layer_norm(x[:, :D].double(), w[:D].double(), b[:D].double(), 1e-3)
     got = y.cpu().double()
     assert (got[:, D:] == 0).all() and ((got[:, :D] - ref).abs() <= 1e-5 * (1 + ref.abs())).all()
+
+
+# slabs: one, all of a batch of requests (5), the first of a second batch, two batches; rows: a float4 per thread, the loop of a long row, the loop of many rows
+@pytest.mark.parametrize("T,H", [(1, 128), (7, 4096), (5, 4224), (513, 256)])
+@pytest.mark.parametrize("KS", [1, 2, 5, 6, 8, 10])
+@pytest.mark.parametrize("form", ["bf16", "rinv", "fp8"])
+@pytest.mark.parametrize("bias,row_scale", [(False, False), (True, True)])
+def test_sums_of_k_slices(lib, T, H, KS, form, bias, row_scale):  # noqa: F811
+    g = torch.Generator().manual_seed(T + H + KS)
+    x, slab, sc = torch.randn(T, H, generator=g) * 3, torch.randn(KS, T, H, generator=g), 0.5 + torch.rand(H, generator=g)
+    w, b, rs = 1 + 0.1 * torch.randn(H, generator=g), torch.randn(H, generator=g), 0.5 + torch.rand(T, generator=g)
+    d = [dev(t) for t in (x, slab, sc, b, rs, w)]
+    out, y = torch.full((T, H), float("nan"), device="cuda"), torch.empty(T, H, dtype=torch.bfloat16, device="cuda")
+    rinv, x8 = torch.full((T,), float("nan"), device="cuda"), torch.zeros(H // 128, T, 128, dtype=torch.uint8, device="cuda")
+    scale8 = d[4] if row_scale else torch.empty(T, device="cuda")      # (the models read and write the same array)
+    lib.check(lib.load_library().mi_op_rmsnorm_slabs(
+        d[0].data_ptr(), d[1].data_ptr(), KS, d[2].data_ptr(), d[3].data_ptr() if bias else None, d[4].data_ptr() if row_scale else None, d[5].data_ptr(), T, H, 1e-5,
+        out.data_ptr(), None if form == "fp8" else y.data_ptr(), rinv.data_ptr() if form == "rinv" else None, x8.data_ptr() if form == "fp8" else None,
+        scale8.data_ptr() if form == "fp8" else None, None))
+    torch.cuda.synchronize()
+    x, slab, sc, b, rs, w = (t.double() for t in (x, slab, sc, b, rs, w))
+    if not bias:
+        b = torch.zeros_like(b)
+    if not row_scale:
+        rs = torch.ones_like(rs)
+    factor = sc * rs[:, None]
+    h, size = x + slab.sum(0) * factor + b, x.abs() + slab.abs().sum(0) * factor + b.abs()
+    got = out.cpu().double()
+    assert ((got - h).abs() <= (KS + 4) * 2.0 ** -24 * size).all()      # KS - 1 additions and four more operations, half a place of fp32 each
+    r = torch.rsqrt(got.pow(2).mean(-1, keepdim=True) + 1e-5)
+    if form == "rinv":
+        assert ((rinv.cpu().double() - r[:, 0]).abs() <= 1e-6 * r[:, 0]).all()
+        assert torch.equal(y.cpu(), (out.cpu() * w.float()).to(torch.bfloat16))
+        return
+    ref = got * r * w
+    if form == "bf16":
+        assert ((y.cpu().double() - ref).abs() <= 2.0 ** -8 * 1.01 * ref.abs()).all()      # one bf16 rounding of an fp32 result
+        return
+    s8 = scale8.cpu().double()
+    assert ((s8 - ref.abs().amax(-1) / 448).abs() <= 2.0 ** -8 * 1.01 * s8).all()
+    got8 = x8.cpu().view(torch.float8_e4m3fn).double().permute(1, 0, 2).reshape(T, H) * s8[:, None]
+    assert ((got8 - ref).abs() <= (2.0 ** -4 + 2.0 ** -8) * 1.01 * ref.abs() + 2.0 ** -10 * s8[:, None]).all()      # e4m3 of a bf16; half its least step below 2^-6

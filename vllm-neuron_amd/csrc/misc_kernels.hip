@@ -36,7 +36,7 @@ int ensure_dynamic_lds(const void* kernel, int bytes) {
   return MI_OK;
 }
 
-// resid[t, :] = fp32(E[ids[t], :])            (reference K1)
+// resid[t, :] = fp32(E[ids[t], :])
 __global__ void embed_kernel(const int32_t* __restrict__ ids, const uint16_t* __restrict__ table, int H,
                              float* __restrict__ resid) {
   const int t = blockIdx.x;
@@ -119,7 +119,7 @@ __global__ __launch_bounds__(1024) void norm_rows_kernel(const float* __restrict
   ss = red[0];
   for (int w = 1; w < nthr >> 6; ++w) ss += red[w];
   float rinv = rsqrtf(ss / (float)H + eps);
-  if (rinv_out) {   // the projection's output takes the factor (gemv_row_rinv's arithmetic: the same roundings at every decode batch)
+  if (rinv_out) {   // the projection's output takes the factor: what is rounded to bf16 is h * gain, as where the norm is part of the projection's kernel
     if (tid == 0) rinv_out[t] = rinv;
     rinv = 1.f;
   }

@@ -1862,7 +1862,7 @@ int mi_forward_spec(mi_ctx* t, mi_ctx* d, int32_t B, int32_t k, const int64_t* i
   // ---- tensor-parallel target: the same phases, every shard on its own thread ----
   hipEvent_t ids_ready = nullptr;
   if (!g->lockstep) {
-    MI_HIP(hipSetDevice(kt.device_id));   // the event is recorded on shard 0's stream: it belongs to shard 0's device (ADVICE r2)
+    MI_HIP(hipSetDevice(kt.device_id));   // the event is recorded on shard 0's stream: it belongs to shard 0's device
     MI_HIP(hipEventCreateWithFlags(&ids_ready, hipEventDisableTiming));
   }
   int rc = group_run(g, [&](mi_ctx* rcx, int r) -> int {
@@ -2098,7 +2098,8 @@ int mi_op_qlinear(const void* x, int32_t M, const void* w_tiled, const float* sc
     float* slab = nullptr;
     const size_t bytes = (size_t)64 << 20;
     MI_HIP(hipMalloc(reinterpret_cast<void**>(&slab), bytes));
-    int rc = M <= 4 ? launch_gemv(W, M, PRO_BF16, p, EPI_F32, e, (hipStream_t)stream) : gemv_in_regs(W, M, bytes) ? launch_gemv_regs(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes) : launch_gemm(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes);
+    int rc = gemv_in_regs(W, M, bytes) ? launch_gemv_regs(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes)
+             : gemv_fits(M, K) ? launch_gemv(W, M, PRO_BF16, p, EPI_F32, e, (hipStream_t)stream) : launch_gemm(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes);
     hipStreamSynchronize((hipStream_t)stream);
     hipFree(slab);
     return rc;
@@ -2228,6 +2229,14 @@ static int attn_op(const AttnSpec& a, const OutGate& gate, const void* q, const 
 int mi_op_rmsnorm(const float* x, const float* g, int32_t T, int32_t H, float eps, void* y, void* stream) {
   MI_CHECK(x && g && y, "null argument");
   return launch_norm_rows(x, nullptr, nullptr, g, T, H, eps, reinterpret_cast<uint16_t*>(y), (hipStream_t)stream);
+}
+int mi_op_rmsnorm_slabs(const float* resid_in, const float* slab, int32_t KS, const float* scale, const float* bias, const float* row_scale, const float* g, int32_t T,
+                        int32_t H, float eps, float* resid_out, void* y, float* rinv, void* x8, float* x8_scale, void* stream) {
+  MI_CHECK(resid_in && slab && KS >= 1 && scale && g && T >= 1 && H >= 4 && resid_out, "bad argument");
+  MI_CHECK(y ? !x8 : x8 && x8_scale && !rinv, "mi_op_rmsnorm_slabs: either bf16 rows (and 1 / rms) or an e4m3 image with its scales");
+  const SlabSum sum{slab, KS, T, H, scale, bias, row_scale};
+  if (y) return launch_norm_rows(resid_in, nullptr, resid_out, g, T, H, eps, reinterpret_cast<uint16_t*>(y), (hipStream_t)stream, &sum, rinv);
+  return launch_norm_rows_fp8(resid_in, nullptr, resid_out, g, T, H, eps, reinterpret_cast<uint8_t*>(x8), x8_scale, (hipStream_t)stream, &sum);
 }
 int mi_op_kv_write(const void* k, const void* v, const int64_t* slots, int32_t T, int32_t nkv, int32_t hd, void* pool,
                    int32_t num_blocks, int32_t block_size, void* stream) {
