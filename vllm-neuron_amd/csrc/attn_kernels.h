@@ -1,4 +1,4 @@
-// Block-layout paged-KV attention (reference K5/K6/K7 of SURVEY.md §2.2: the NxDI
+// Block-layout paged-KV attention (the NxDI
 // context-encoding and token-generation attention reached through
 // /root/reference/vllm_neuron/worker/neuronx_distributed_model_loader.py:339-348 with the
 // block_table / slot_mapping / *_context_lens contract of

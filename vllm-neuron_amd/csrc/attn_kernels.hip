@@ -65,9 +65,9 @@ typedef __attribute__((ext_vector_type(4))) short s16x4_t;
 // every storing wave drains them, one lane takes a ticket from an agent-scope counter, and the
 // work-group whose ticket is NS - 1 reads all NS partials back with sc1 loads (past its L1; no
 // other reader of these lines exists in the launch, so no L2 holds a stale copy) and writes the
-// bf16 output.  This is the hand-off form MI355X_MICROARCH.md lists as valid without fences
-// ("the workgroup whose add came last, told by the value its add returned"; one work-group per
-// CU: the launch pads its LDS request to keep it so).  The merge itself runs in split order, so the
+// bf16 output.  No fence is needed: the work-group whose add came last is told so by
+// the value its add returned, and there is one work-group per CU (the launch pads its LDS request to
+// keep it so).  The merge itself runs in split order, so the
 // result does not depend on which work-group performs it.  The counter is left at 0 for the next launch.
 template <int HD, int NW, bool FINAL, bool MERGE = false>
 __device__ __forceinline__ void attn_decode_body(
@@ -712,7 +712,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_prefill_kernel(
 // =====================================================================================
 // context encoding, second generation: 32x32x16 MFMAs, K/V tiles by LDS-DMA, two waves per SIMD
 // =====================================================================================
-// What the counters of the kernel above asked for (DESIGN.md 5.2: 17 % MFMA-busy at one wave per
+// What the counters of the kernel above asked for (17 % MFMA-busy at one wave per
 // SIMD, 408 registers, 144 accumulator moves and a ds_write staging pass per 64-key tile):
 //   * a wave owns ONE 32-query block of one q head: S^T[key][q] = K . Q^T on v_mfma_f32_32x32x16_bf16
 //     puts a query on a lane (its 32 scores of a 64-key tile in 32 registers of lanes l and l + 32), so
@@ -739,8 +739,8 @@ typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 constexpr float kDeferLog2 = 6.f;
 
 // {v of this lane, v of lane ^ 32} in some order (max / sum do not care): one v_permlane32_swap.  The elements of the
-// builtin's result are copied out before the bit cast: hipcc 7.2 reads element 0 for __builtin_bit_cast(float, r[1])
-// (hipcc notes) -- which made a row's sum 2 x (its lower half's sum).
+// builtin's result are copied out before the bit cast: hipcc 7.2 reads element 0 for __builtin_bit_cast(float, r[1]),
+// which made a row's sum 2 x (its lower half's sum).
 __device__ __forceinline__ f32x2_t swap32_pair(float v) {
   const unsigned a = __builtin_bit_cast(unsigned, v);
   const auto r = __builtin_amdgcn_permlane32_swap(a, a, false, false);
@@ -1117,7 +1117,7 @@ static bool attn_prefill_v1() {   // MI355X_ATTN_PREFILL_V1=1: the first-generat
 
 static int prefill_heads(int G) { return G <= 1 ? 1 : (G <= 2 ? 2 : (G <= 4 ? 4 : 8)); }
 struct PrefillPlan { int Gp, nblk, bs_shift, paired, gx, ns; float *o_part = nullptr, *ml_part = nullptr; };
-static PrefillPlan prefill_plan(int T, int q_pos0, int block_size, int nh, int nkv, int hd, float* ws, size_t ws_bytes) {
+static PrefillPlan prefill_plan(int T, int q_pos0, int block_size, int nh, int nkv, int hd, float* ws, size_t ws_bytes, int num_cu) {
   // second generation: 8 waves = (8 / Gp) query blocks x Gp heads; blocks in complementary pairs
   PrefillPlan p;
   p.Gp = prefill_heads(nh / nkv);
@@ -1125,18 +1125,18 @@ static PrefillPlan prefill_plan(int T, int q_pos0, int block_size, int nh, int n
   int bs_shift = -1;
   for (int sh = 4; sh < 20; ++sh) if ((1 << sh) == block_size) bs_shift = sh;
   // One block per work-group (5 .. 8 heads on a kv head): pairs only where single blocks would not all run at once.
-  const int paired = qb > 1 || nblk * nkv > 256;
+  const int paired = qb > 1 || nblk * nkv > num_cu;
   const int gx = paired ? ceil_div(npair, qb >= 2 ? qb / 2 : 1) : nblk;
   // A short prompt, or the rest of one behind cached keys, leaves most of the chip idle while each work-group walks its tiles, 1.75 us each:
   // slices of the keys then, at least two tiles each, the cheapest by that and the second launch, which moves every slice's O out and in.
   // 188 tokens behind 512 cached ones, 28 heads on 4: 40.8 us in 12 work-groups of two passes, 16.7 + 4.8 now.
   int ns = 1;
   const int tiles = ceil_div(q_pos0 + T, 64);
-  double best = 1.75 * tiles * ceil_div(gx * nkv, 256);
+  double best = 1.75 * tiles * ceil_div(gx * nkv, num_cu);
   for (int z = 2; ws && z <= kPrefillSlices; ++z) {
     const size_t part = (size_t)z * T * nh;
     if (ceil_div(tiles, z) < 2 || part * (hd + 2) * sizeof(float) > ws_bytes) break;
-    const double cost = 1.75 * ceil_div(tiles, z) * ceil_div(gx * nkv * z, 256) + 4.5 + (double)part * hd * 8.0 / 4e6;
+    const double cost = 1.75 * ceil_div(tiles, z) * ceil_div(gx * nkv * z, num_cu) + 4.5 + (double)part * hd * 8.0 / 4e6;
     if (cost < best) { best = cost; ns = z; }
   }
   p.nblk = nblk; p.bs_shift = bs_shift; p.paired = paired; p.gx = gx; p.ns = ns;
@@ -1161,7 +1161,9 @@ int launch_attn_prefill(const uint16_t* q, int T, int q_pos0, const uint16_t* kp
   const float scale_log2e = 1.4426950408889634f / sqrtf((float)hd);
   const int Gp = prefill_heads(G);
   if (!attn_prefill_v1()) {
-    const PrefillPlan p = prefill_plan(T, q_pos0, block_size, nh, nkv, hd, ws, ws_bytes);
+    int num_cu = 0;
+    MI_TRY_A(device_num_cu(&num_cu));
+    const PrefillPlan p = prefill_plan(T, q_pos0, block_size, nh, nkv, hd, ws, ws_bytes, num_cu);
 #define MI_P2(HD_) do { \
       constexpr int lds = 3 * 2 * 64 * 2 * HD_; \
       MI_TRY_A(ensure_dynamic_lds(reinterpret_cast<const void*>(attn_prefill2_kernel<HD_, 8>), lds)); \
@@ -1218,8 +1220,8 @@ int launch_attn_mixed(const AttnMixed& m, int T, int q_pos0, const uint16_t* q, 
   // One launch where both sides find a CU for every work-group; beyond that the prompt's wait behind the others' (us per call, two launches -> one: 8B model
   // 239 + 3 tokens 3105 -> 2980, 64 + 6 2205 -> 2108, TinyLlama 300 + 4 2385 -> 2245, 8B bf16 500 + 6 4862 -> 4724; 1900 + 3 13035 -> 13097).
   int num_cu = 0;
-  if (device_num_cu(&num_cu) != MI_OK) return MI_EHIP;
-  const PrefillPlan p = prefill_plan(T, q_pos0, block_size, nh, nkv, hd, ws, ws_bytes);
+  MI_TRY_A(device_num_cu(&num_cu));
+  const PrefillPlan p = prefill_plan(T, q_pos0, block_size, nh, nkv, hd, ws, ws_bytes, num_cu);
   if (attn_prefill_v1() || (p.gx * p.ns + mixed_splits(m, nkv, hd) * m.B) * nkv > num_cu) {
     int rc = launch_attn_decode(m.q, kpool, vpool, block_size, m.block_table, m.MB, m.ctx_lens, m.B, nh, nkv, hd, m.out, m.scratch, s, false, 1, m.num_blocks, m.max_ctx);
     return rc != MI_OK ? rc : launch_attn_prefill(q, T, q_pos0, kpool, vpool, block_size, block_table, nh, nkv, hd, out, s, ws, ws_bytes);
