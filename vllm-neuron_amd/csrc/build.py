@@ -58,9 +58,9 @@ def _compile(src, force=False):
     return obj, r.stderr
 
 
-def build(verbose=True):
+def build(verbose=True, force=False):
     os.makedirs(os.path.join(HERE, "build"), exist_ok=True)
-    force = "--force" in sys.argv or _flags_changed()
+    force = _flags_changed() or force or "--force" in sys.argv
     with cf.ThreadPoolExecutor(max_workers=min(len(SOURCES), int(os.environ.get("MAX_JOBS") or os.cpu_count() or 4))) as ex:
         results = list(ex.map(lambda src: _compile(src, force), SOURCES))
     objs = [o for o, _ in results]
