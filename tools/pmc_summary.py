@@ -2,9 +2,9 @@
 
     rocprofv3 --pmc FETCH_SIZE --output-format csv -d gpurun_out/pmc -o bench -- \
         python3 bench.py --steps 4 --warmup 1 --no-cpu-baseline --ttft-prompts 1
-    python tools/pmc_summary.py gpurun_out/pmc profiles/r01_gemv_traffic.json
+    python tools/pmc_summary.py gpurun_out/pmc profiles/gemv_traffic.json
 
-Correction per /opt/skills/guides/MI355X_MICROARCH.md (HBM): FETCH_SIZE is in KiB and on gfx950
+Correction: FETCH_SIZE is in KiB and on gfx950
 reports exactly half of the bytes of a wide coalesced streaming read -> bytes = value * 1024 * 2.
 """
 import collections, csv, glob, hashlib, json, os, sys
@@ -26,9 +26,9 @@ doc = {
     # the figure belongs to THESE kernels: bench.py flags it as stale when the source has changed since
     "kernel_source_sha1": hashlib.sha1(open(os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
                                                          "vllm-neuron_amd", "csrc", "linear_device.h"), "rb").read()).hexdigest(),
-    "counter": "FETCH_SIZE (KiB) x 1024 x 2: gfx950 tallies 128-B requests at 64 B (MI355X_MICROARCH.md, HBM)",
+    "counter": "FETCH_SIZE (KiB) x 1024 x 2: gfx950 tallies 128-B requests at 64 B (measured on a wide streaming read)",
     "command": "rocprofv3 --pmc FETCH_SIZE --output-format csv -- python3 bench.py --steps 4 --warmup 1 "
-               "--no-cpu-baseline --ttft-prompts 1",
+               "--no-cpu-baseline --ttft-prompts 1 --no-speculation",
 }
 json.dump(doc, open(out, "w"), indent=1)
 print(json.dumps(doc, indent=1))

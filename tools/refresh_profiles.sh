@@ -17,7 +17,7 @@ echo "[3] PMC pass (FETCH_SIZE only)"
 cd /tmp && rm -rf /tmp/pmc
 timeout -k 10 600 rocprofv3 --pmc FETCH_SIZE --output-format csv -d /tmp/pmc -o bench -- python3 /root/repo/bench.py --steps 4 --warmup 1 --no-cpu-baseline --ttft-prompts 1 --no-speculation > $OUT/pmc_bench.json 2> $OUT/pmc.err
 cd /root/repo
-python3 tools/pmc_summary.py /tmp/pmc $OUT/${R}_gemv_traffic.json > /dev/null
+python3 tools/pmc_summary.py /tmp/pmc $OUT/gemv_traffic.json > /dev/null
 echo "[4] Qwen2.5-7B INT8"; timeout -k 10 600 python3 bench.py --model qwen25_7b --no-cpu-baseline > $OUT/${R}_bench_n1_qwen25_7b_int8.json 2> $OUT/qwen.err
 for T in 2 4 8; do
   echo "[5] TP $T loopback kernel trace"

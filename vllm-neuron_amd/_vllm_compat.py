@@ -1,5 +1,5 @@
 # SPDX-License-Identifier: Apache-2.0
-"""vLLM 0.11 symbols this plugin is written against (SURVEY.md §8b).
+"""vLLM 0.11 symbols this plugin is written against.
 
 With vLLM installed the real classes are re-exported and the plugin is a drop-in
 out-of-tree backend.  This build image has no vLLM (and no network), so the same names

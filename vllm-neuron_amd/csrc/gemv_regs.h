@@ -8,15 +8,14 @@
 // of every row-tile in front of its requests (vector memory retires in order).  K beyond what fits the registers goes over grid.y: raw sums to
 // slabs, added by the next row norm or by splitk_reduce.
 // Bound by the weight bytes (117 MB of gate|up of the 8B model in fp8 in 22.7 us at 8 rows, 5.2 TB/s; 27.3 at 32).  us a launch, LDS kernels -> these,
-// 8B fp8 at 32 rows: gate|up 35.8 -> 27.3, QKV 23 -> 15.7, and 4.8 for each norm that was a part of them; 7B int8 at 24 rows: gate|up 57.8, lm_head 261
-// against 25.4 and 139 here at 5 rows (the logits' way over PCIe included).
+// 8B fp8 at 32 rows: gate|up 35.8 -> 27.3, QKV 23 -> 15.7, and 4.8 for each norm that was a part of them; 7B int8 at 24 rows: gate|up 57.8 -> 30.9.
 #pragma once
 #include "linear_device.h"
 
 namespace mi {
 
-// k-tiles a wave holds: 4 or 8 of 64 k (1-byte weights), 4, 8 or 16 of 32 k
 constexpr int kRegsMaxPasses = 64;   // row-tiles of a work-group: their scales and biases wait in LDS
+// k-tiles a wave holds at most: 4 or 8 of 64 k (1-byte weights), 4, 8 or 16 of 32 k
 template <int WD> constexpr int kRegsMaxTiles = WD == MI_W_BF16 ? 16 : 8;
 
 template <int WD, int EPI, int MG, int NK, bool SLAB>

@@ -1,5 +1,5 @@
-// Launch-side declarations of the weight-quantized linear layer (reference K3 of
-// the NxDI quantized QKV/O/MLP/lm_head linears reached through
+// Launch-side declarations of the weight-quantized linear layer (the
+// NxDI quantized QKV/O/MLP/lm_head linears reached through
 // /root/reference/vllm_neuron/worker/neuronx_distributed_model_loader.py:339-348).
 #pragma once
 #include "mi_common.h"

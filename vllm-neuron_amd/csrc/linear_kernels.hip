@@ -267,7 +267,7 @@ extern template int launch_gemm_wide_wd<MI_W_INT8>(const LinearW&, int, const ui
 // Against the best of 128 x 256 and 256 x 256 alone, us: int8 gate|up of the 7B model at 188 tokens 79 -> 60 (148 tiles of 256 x 256 on 256 CUs, 73 % of
 // each filled; 198 of 192 x 192), its down projection 41.6 -> 34.4; bf16 gate|up of TinyLlama 700 tokens 51.6 -> 35.4, 200 tokens 28.4 -> 21.4;
 // fp8 QKV of the 8B model 1400 tokens 82.6 -> 63.9; bf16 down projection of 2048 x 14336 at 100 tokens 26.4 -> 17.6.
-struct WidePlan { int bm, ntw, ks; };   // bm 0: the shape has no plan
+struct WidePlan { int bm, ntw, ks; };
 static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, bool deferred) {
   int cus = 256;
   if (device_num_cu(&cus) != MI_OK || cus < 8) cus = 256;
@@ -276,7 +276,7 @@ static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, boo
                                         {{0.0451, 0.0015, 0.0629, 0.1408}, {0.1990, 0.0565, 0.0129, 0.0542}}};
   const int nks = K / 64;
   const double mb = (double)T * N * 4e-6;
-  WidePlan best{0, 4, 1};
+  WidePlan best{0, 4, 1};   // (bm 0: none compared yet; one slice is always allowed, so there is one)
   double best_cost = 0.;
   for (int bm = 64; bm <= 256; bm += 64)
     for (int ntw = 2; ntw <= 4; ++ntw) {

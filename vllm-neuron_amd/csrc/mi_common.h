@@ -126,8 +126,8 @@ __device__ __forceinline__ uint4 nt_load16(const uint4* p) {
 
 // fp32 -> OCP e4m3fn, round-nearest-even, saturating at +-448: the hardware convert of gfx950 (v_cvt_pk_fp8_f32; OCP
 // formats on this chip).  The clamp in front makes the result independent of the instruction's own out-of-range rule; a NaN
-// input becomes +-448 like any other out-of-range value.  (Until round 3 this was ~20 integer / select instructions per value:
-// the per-token quantization passes of the FP8-activation path were VALU-bound on it.)
+// input becomes +-448 like any other out-of-range value.  (Written out it is ~20 integer / select instructions per value,
+// on which the per-token quantization passes of the FP8-activation path were VALU-bound.)
 __device__ __forceinline__ uint32_t f32_to_e4m3fn(float f) {
   const float c = __builtin_fminf(__builtin_fmaxf(f, -448.f), 448.f);
   return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(c, 0.f, 0, false) & 0xffu;

@@ -90,7 +90,7 @@ struct mi_ctx {
   // [context lengths][ids][positions][slots][state slots] (one H2D of 5 x max_num_seqs ints per step) and block
   // tables that STAY on the device: a row is re-sent only when the caller's row differs from the
   // host shadow of what the device holds (a new request in the row, a block appended), and only
-  // the entries that became live since the last call are validated (SURVEY 8f-2; the reference
+  // the entries that became live since the last call are validated (the reference
   // rebuilds and re-validates every table every step, runner.py:798-832, 887-917).
   int32_t *d_inputs = nullptr, *h_inputs = nullptr;      // context-encoding block
   size_t inputs_elems = 0;

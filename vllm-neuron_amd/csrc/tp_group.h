@@ -5,7 +5,7 @@
 // every core (/root/reference/vllm_neuron/platform.py:166-167, worker/neuron_worker.py:106-121,
 // tp_degree = tensor_parallel_size at worker/neuronx_distributed_model_loader.py:752-753).
 //
-// The exchange step of a row-parallel projection (SURVEY.md C1) is a hand-written all-reduce over
+// The exchange step of a row-parallel projection is a hand-written all-reduce over
 // peer-mapped device memory (xGMI between GPUs; plain device memory when every shard sits on one
 // GPU, which is how the single-GPU tests run the same kernels):
 //   publish   fp32 partial -> exchange buffer of this rank; system-scope release; one flag

@@ -532,7 +532,7 @@ int group_alloc_exchange(mi_ctx* c) {
     if (alloc_exchange_mem(&f1, fbytes, true) != MI_OK) return MI_EHIP;
     if (alloc_exchange_mem(&f2, fbytes, true) != MI_OK) return MI_EHIP;
     MI_HIP(hipMalloc(&ct, AR_WORDS * 4));
-    // EVERY exchange allocation is written by its owner before its address is published: round 2 lost the peers'
+    // EVERY exchange allocation is written by its owner before its address is published: an earlier form lost the peers'
     // contribution in the FIRST exchange after allocation (4 KiB-aligned ranges, data in place when the host looked later)
     // with never-written slots in uncached memory, and never with the flag blocks, which differed only in being cleared here.
     // What fits that evidence is the allocator's own (lazy, page-granular) initialisation of a fresh allocation landing

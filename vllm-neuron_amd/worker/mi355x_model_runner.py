@@ -7,7 +7,7 @@ continuous-batching path (with and without prefix caching): the persistent batch
 per-step argument record (``ModelInputForMI355X`` has the reference's fields and pad
 conventions: slot pad -1, block-table pad 0 / -1), the seq-id slot pool, CPU sampling through
 vLLM's ``Sampler`` and the ``ModelRunnerOutput`` assembly.  Chunked prefill, multimodal
-inputs, LoRA and speculative decoding raise ``NotImplementedError`` (out of scope, DESIGN.md).
+inputs, LoRA and speculative decoding raise ``NotImplementedError`` (out of scope).
 
 Differences that are deliberate: slot mappings are built with tensor ops instead of an
 O(max_model_len) Python list comprehension per prefill (reference runner.py:757-761), block
@@ -328,7 +328,7 @@ class MI355XModelRunner:
         return self._finalize_continuous_batching_inputs(data, is_prefill)
 
     def _prepare_decode_inputs_incremental(self, scheduler_output) -> ModelInputForMI355X:
-        """Token-generation inputs without rebuilding what did not change (SURVEY 8f-2).  Same
+        """Token-generation inputs without rebuilding what did not change.  Same
         record, same values as `_process_cached_request_*` + `_finalize_*` produce; the padded
         block-table rows persist across steps in one [max_num_seqs, MB] tensor -- a row is rewritten
         only when another request takes it or a block is appended (the reference pads, copies and
