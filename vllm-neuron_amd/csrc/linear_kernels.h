@@ -74,7 +74,7 @@ int launch_splitk_reduce(const SlabSum& sl, int epi, const EpiArgs& e, hipStream
 // M > 16 context-encoding path (MFMA-bound).  x is always bf16 [T, K].
 // defer != null: a K-split projection (EPI_RESID, EPI_F32) leaves its slabs unsummed and describes them in *defer
 // (slab == null: nothing deferred); the caller hands them to the next row norm or to launch_splitk_flush
-// split_as_deferred: K is split as if the sum were deferred, though it is not (a shard's partial sums: the same additions as one GPU's)
+// split_as_deferred: K is split as if the sum were deferred, though it is not (a communicator of one rank: the same additions as without one)
 int launch_gemm(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e,
                 hipStream_t s, float* splitk_ws = nullptr, size_t splitk_ws_bytes = 0, SlabSum* defer = nullptr, bool split_as_deferred = false);
 int launch_splitk_flush(const SlabSum& sl, const float* resid_in, float* out, int ld_out, hipStream_t s);

@@ -145,7 +145,8 @@ int run_linear(mi_ctx* c, const Linear& L, int rows, int pro, ProArgs p, int epi
   //  the 8B model in fp8 2077 -> 2036 us, 242 tokens 3114 -> 3062, 300 tokens of TinyLlama 2602 -> 2520)
   static const int fuse_min_rows = [] { const char* v = getenv("MI355X_FUSE_SPLITK_MIN_ROWS"); return v ? atoi(v) : 0; }();
   SlabSum* defer = (fuse && epi == EPI_RESID && rows >= fuse_min_rows && !c->pend.slab) ? &c->pend : nullptr;
-  const bool as_deferred = fuse && c->collective() && epi == EPI_F32 && rows >= fuse_min_rows && &L != &c->lm_head;
+  // (a communicator of one rank makes the additions of no communicator; a shard's K is another anyway, and its sum is a launch of its own in front of the exchange)
+  const bool as_deferred = fuse && c->collective() && c->cfg.tp_degree == 1 && epi == EPI_F32 && rows >= fuse_min_rows && &L != &c->lm_head;
   auto note_deferred = [&]() {
     if (defer && c->pend.slab) { c->pend_in = e.resid_in; c->pend_out = e.out_f32; }
   };
