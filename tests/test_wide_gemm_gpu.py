@@ -123,3 +123,47 @@ def test_stack_epilogues_agree_with_the_128x128_kernel(tmp_path):
     for k, want in got["0"].items():
         d = got["1"][k] - want
         assert torch.isfinite(d).all() and d.pow(2).mean().sqrt() < 0.02 * want.std(), k    # the bar of the other dispatch test
+
+
+_LLAMAS = r"""
+import sys, torch
+sys.path.insert(0, %(root)r)
+from vllm_neuron_amd._native import NativeModel, MI_W, MI_Q
+from tests.helpers import prefill_inputs
+out, hd, heads, kv, wd = sys.argv[1], *map(int, sys.argv[2:5]), sys.argv[5]
+m = NativeModel(num_layers=2, hidden_size=320, num_heads=heads, num_kv_heads=kv, head_dim=hd, intermediate_size=448, vocab_size=1008, rms_norm_eps=1e-5,
+                rope_theta=1e4, rope_type=0, qkv_bias=int(wd == "int8"), tie_word_embeddings=0, num_blocks=65, block_size=16, max_num_seqs=4,
+                max_model_len=1024, weight_dtype=MI_W[wd], quant_type=MI_Q["per_channel_symmetric"], quantize_lm_head=0, tp_degree=1, tp_rank=0, device_id=0,
+                use_graphs=1, prefill_fp8_activations=0)
+m.init_synthetic_weights(1, 0.05)
+m.finalize()
+g, res = torch.Generator().manual_seed(5), {}
+for n, cached in ((33, 0), (150, 0), (257, 0), (300, 112), (777, 0)):
+    prompt = torch.randint(0, 1000, (n,), generator=g).tolist()
+    blocks = list(range(1, 2 + n // 16))
+    if cached:
+        m.forward(**prefill_inputs(prompt[:cached], blocks, 16, 1024))
+    res[n] = m.forward(**prefill_inputs(prompt, blocks, 16, 1024, cached)).float().cpu().clone()
+    print(n, flush=True)
+m.close()
+torch.save(res, out)
+print("CHILD_OK", flush=True)
+"""
+
+
+# a wave's tiles that hold q and k, k and v; one and three heads a kv head; every row block with a remainder; planned tiles, and 128 and 256 tokens x 256 rows
+@pytest.mark.parametrize("hd,heads,kv,wd", [(64, 6, 2, "bf16"), (128, 1, 1, "int8"), (64, 3, 1, "f8e4m3")])
+def test_llama_epilogues_agree_with_the_128x128_kernel(tmp_path, hd, heads, kv, wd):
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    got = []
+    for i, env in enumerate((dict(MI355X_GEMM_WIDE="0"), dict(MI355X_GEMM_WIDE="1"), dict(MI355X_GEMM_WIDE="1", MI355X_GEMM_WIDE_BM="128"),
+                             dict(MI355X_GEMM_WIDE="1", MI355X_GEMM_WIDE_BM="256"))):
+        out = str(tmp_path / f"{i}.pt")
+        r = subprocess.run([sys.executable, "-c", _LLAMAS % {"root": root}, out, str(hd), str(heads), str(kv), wd], env=dict(os.environ, **env),
+                           capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0 and "CHILD_OK" in r.stdout, (r.stdout[-1500:], r.stderr[-1500:])
+        got.append(torch.load(out, weights_only=True))
+    for n, want in got[0].items():
+        for other in got[1:]:
+            d = other[n] - want
+            assert torch.isfinite(d).all() and d.pow(2).mean().sqrt() < 0.02 * want.std(), n    # the bar of the other dispatch test

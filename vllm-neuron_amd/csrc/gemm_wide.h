@@ -57,6 +57,20 @@ __device__ __forceinline__ void wide_slice(int K, int& ks0, int& nks) {
   nks = min(per, all - ks0);
 }
 
+// a wave's raw accumulators to its K-slice's slab [T][16 NT]
+template <int NTW, int MT>
+__device__ __forceinline__ void store_slab(float* __restrict__ slab, int T, int NT, int mb, int nb, int g, int c, const f32x4_t (&acc)[NTW][MT]) {
+#pragma unroll
+  for (int i = 0; i < NTW; ++i) {
+    if (nb + i >= NT) continue;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int m = mb + mt * 16 + c;
+      if (m < T) *reinterpret_cast<f32x4_t*>(slab + (size_t)m * (NT * 16) + (nb + i) * 16 + g * 4) = acc[i][mt];
+    }
+  }
+}
+
 // A wave multiplies BM / 2 tokens x 16 NTW weight rows: NTW BM / 8 accumulator registers (256 x 256: 128, and 246 VGPRs
 // with the decoded fragments of one K-step).
 // SPLIT: grid.z K-slices write raw fp32 accumulators to slab[z][m][n] (see gemm_a8_kernel).
@@ -194,22 +208,8 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
     }
   }
   if (grp == 0) __builtin_amdgcn_s_barrier();   // the barrier group 1 executed first
-#pragma unroll
-  for (int i = 0; i < NTW; ++i) {
-    const int nt = ntb + wn * NTW + i;
-    if (nt >= NT) continue;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int m = m0 + wm * (BM / 2) + mt * 16 + c;
-      if (m >= T) continue;
-      if constexpr (SPLIT) {
-        *reinterpret_cast<float4*>(slab + ((size_t)blockIdx.z * T + m) * (NT * 16) + nt * 16 + g * 4) =
-            make_float4(acc[i][mt][0], acc[i][mt][1], acc[i][mt][2], acc[i][mt][3]);
-      } else {
-        epilogue<EPI>(e, m, nt * 16 + g * 4, acc[i][mt]);
-      }
-    }
-  }
+  if constexpr (SPLIT) store_slab<NTW, MT>(slab + (size_t)blockIdx.z * T * (NT * 16), T, NT, m0 + wm * (BM / 2), ntb + wn * NTW, g, c, acc);
+  else epilogue_tile<EPI, NTW, MT>(e, T, NT, m0 + wm * (BM / 2), ntb + wn * NTW, g, c, acc);
 }
 
 // The same for bf16 weights at 256 tokens x 256 weight rows.  A 64-deep stage of it is 64 KiB, and the LDS holds two; the stagger
@@ -319,22 +319,8 @@ __global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restric
     xfill = xfill == 2 ? 0 : xfill + 1;
   }
   if (grp == 0) __builtin_amdgcn_s_barrier();   // the barrier group 1 executed first
-#pragma unroll
-  for (int i = 0; i < NTW; ++i) {
-    const int nt = ntb + wn * NTW + i;
-    if (nt >= NT) continue;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int m = m0 + wm * (BM / 2) + mt * 16 + c;
-      if (m >= T) continue;
-      if constexpr (SPLIT) {
-        *reinterpret_cast<float4*>(slab + ((size_t)blockIdx.z * T + m) * (NT * 16) + nt * 16 + g * 4) =
-            make_float4(acc[i][mt][0], acc[i][mt][1], acc[i][mt][2], acc[i][mt][3]);
-      } else {
-        epilogue<EPI>(e, m, nt * 16 + g * 4, acc[i][mt]);
-      }
-    }
-  }
+  if constexpr (SPLIT) store_slab<NTW, MT>(slab + (size_t)blockIdx.z * T * (NT * 16), T, NT, m0 + wm * (BM / 2), ntb + wn * NTW, g, c, acc);
+  else epilogue_tile<EPI, NTW, MT>(e, T, NT, m0 + wm * (BM / 2), ntb + wn * NTW, g, c, acc);
 }
 
 // The tiles there are.  bf16 weights: a 64-deep stage of 256 x 192, 256 x 256 or 192 x 256 fits the LDS twice only; 256 x 256 has its own kernel.
