@@ -71,6 +71,24 @@ def test_every_tile_of_the_wide_gemm(lib, wd, bm, ntw):
         assert err < tol, (M, N, K, ks, err, tol)
 
 
+# bf16 tiles by 32-deep K-steps: one pair of them, as many pairs as the ring of activations has, fewer and more; slices of two and of uneven length
+@pytest.mark.parametrize("bm,ntw", [(192, 4), (256, 3), (256, 4)])
+@pytest.mark.parametrize("M,N,K,ks", [(1, 16, 64, 1), (193, 208, 128, 1), (257, 272, 192, 1), (191, 400, 256, 1), (640, 560, 1088, 1), (300, 272, 128, 2), (255, 784, 704, 3)])
+def test_tiles_by_32_deep_steps(lib, bm, ntw, M, N, K, ks):
+    g = torch.Generator().manual_seed(M + N + K)
+    w = (torch.randn(N, K, generator=g) * 0.05).to(torch.bfloat16)
+    x, bias = torch.randn(M, K, generator=g).to(torch.bfloat16), torch.randn(N, generator=g) * 0.1
+    tiled, scale = quantize_on_device(lib, w.float(), "bf16", "per_channel_symmetric")
+    ref = x.double() @ w.double().t() + bias.double()
+    y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    xd, bd = dev(x), dev(bias)
+    lib.check(lib.load_library().mi_op_qlinear(xd.data_ptr(), M, tiled.data_ptr(), scale.data_ptr(), bd.data_ptr(), N, K, WD["bf16"], y.data_ptr(),
+                                               100 * bm + 10 * ntw + ks, None))
+    torch.cuda.synchronize()
+    err = (y.cpu().double() - ref).abs().max().item()
+    assert err < 2e-5 * ref.abs().max().item() + 1e-5 * (K ** 0.5), err      # as above
+
+
 _CHILD = r"""
 import sys, torch
 sys.path.insert(0, %(root)r)

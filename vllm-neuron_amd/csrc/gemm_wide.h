@@ -212,16 +212,21 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
   else epilogue_tile<EPI, NTW, MT>(e, T, NT, m0 + wm * (BM / 2), ntb + wn * NTW, g, c, acc);
 }
 
-// The same for bf16 weights at 256 tokens x 256 weight rows.  A 64-deep stage of it is 64 KiB, and the LDS holds two; the stagger
-// needs a third.  So a K-step is 32 deep (one weight tile per 16 rows; 32 MFMAs a wave), the weights ride in four stages of 16 KiB, and the
-// activations, whose rows are fetched 128 bytes at a time, in three of 64-deep pairs of K-steps (32 KiB): 160 KiB.  K-step s requests the weights
-// of s + 3 and one half of the rows of the pair behind the next, four DMAs a wave, so what K-step s reads was requested by K-step s - 3 at
-// the latest and eight younger DMAs stay in flight.
-template <int EPI, bool SPLIT>
+// The same for bf16 weights at 256 x 256, 256 x 192 and 192 x 256 (tokens x weight rows).  A 64-deep stage of these is 56 - 64 KiB, and the LDS holds
+// two; the stagger needs a third.  So a K-step is 32 deep (one weight tile per 16 rows; NTW MT MFMAs a wave), the weights ride in four stages, and the
+// activations, whose rows are fetched 128 bytes at a time, in three of 64-deep pairs of K-steps: 160 KiB at 256 x 256.  K-step s requests the weights
+// of s + 3 and a part of the rows of the pair behind the next, so what K-step s reads was requested by K-step s - 3 at
+// the latest and the DMAs of two K-steps stay in flight.
+// us a 64-deep K-step on a full chip: 256 x 256 1.46, the other two 1.2; 128 x 256 by 64 0.83.  12288 x 2048 at 777 tokens: 192 work-groups of 256 x 256 54.8,
+// 256 of 256 x 192 48.1, 240 of 192 x 256 46.0.
+template <int EPI, int BM, int NTW, bool SPLIT>
 __global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restrict__ W, int NT, int KT, int T, int K,
                                                           const uint16_t* __restrict__ x, int ldx, EpiArgs e,
                                                           float* __restrict__ slab) {
-  constexpr int BM = 256, MT = 8, WM = 2, NTW = 4, kW = 16 * 1024, kX = 32 * 1024, kXs = 4 * kW;
+  constexpr int MT = BM / 32, WM = 2, kW = NTW * 4096, kX = BM * 128, kXs = 4 * kW;
+  constexpr int XP = BM / 64, XH0 = (XP + 1) / 2, XH1 = XP - XH0;     // 8-row activation pieces per wave and pair, those of its first and its second K-step
+  constexpr int WP0 = (NTW + 1) / 2, WP1 = NTW - WP0;                 // weight tiles per wave and K-step: waves 0-3, waves 4-7
+  static_assert(4 * kW + 3 * kX <= 160 * 1024, "LDS");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int g = lane >> 4, c = lane & 15;
@@ -232,32 +237,35 @@ __global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restric
   wide_slice<SPLIT>(K, ks0, nks);
   const int s0 = 2 * ks0, n = 2 * nks;        // this slice's 32-deep K-steps
 
-  const uint4* wsrc[2];
-  const uint16_t* xsrc[4];
+  const int grp = __builtin_amdgcn_readfirstlane(wave >> 2), wt0 = grp == 0 ? WP0 * wave : 4 * WP0 + WP1 * (wave - 4);
+  const uint4* wsrc[WP0];
+  const uint16_t* xsrc[XP];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) wsrc[i] = W + ((size_t)min(ntb + 2 * wave + i, NT - 1) * KT + s0) * 64 + lane;
+  for (int i = 0; i < WP0; ++i) wsrc[i] = W + ((size_t)min(ntb + wt0 + i, NT - 1) * KT + s0) * 64 + lane;   // (a group-1 wave without an i-th one does not use it)
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = (4 * wave + i) * 8 + (lane >> 3), sl = lane & 7;
+  for (int i = 0; i < XP; ++i) {
+    const int r = (XP * wave + i) * 8 + (lane >> 3), sl = lane & 7;
     xsrc[i] = x + (size_t)min(m0 + r, T - 1) * ldx + (size_t)s0 * 32 + ((sl ^ xs_swz<MI_W_BF16>(r)) * 8);
   }
   auto issue_w = [&](int s) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) glds16(wsrc[i] + (size_t)s * 64, smem + (s & 3) * kW + (2 * wave + i) * 1024);
-  };
-  auto issue_x = [&](int p, int half, int stage) {   // half of this wave's rows of pair p
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int q = 2 * half + i;
-      glds16((half ? xsrc[2 + i] : xsrc[i]) + (size_t)p * 64, smem + kXs + stage * kX + (4 * wave + q) * 1024);
+    for (int i = 0; i < WP1; ++i) glds16(wsrc[i] + (size_t)s * 64, smem + (s & 3) * kW + (wt0 + i) * 1024);
+    if constexpr (WP0 > WP1) {
+      if (grp == 0) glds16(wsrc[WP1] + (size_t)s * 64, smem + (s & 3) * kW + (wt0 + WP1) * 1024);
     }
   };
-  // own pieces of K-step s are in: the requests of the last two K-steps may be out, fewer of them at the end
-  auto wait_for = [&](int s) {
+  auto issue_x = [&](int p, auto half, int stage) {   // a part of this wave's rows of pair p
+    constexpr int lo = decltype(half)::value ? XH0 : 0, hi = decltype(half)::value ? XP : XH0;
+#pragma unroll
+    for (int q = lo; q < hi; ++q) glds16(xsrc[q] + (size_t)p * 64, smem + kXs + stage * kX + (XP * wave + q) * 1024);
+  };
+  // own pieces of K-step s are in: the requests of the last two K-steps may be out, fewer of them at the end (w: weight tiles a K-step)
+  auto wait_at = [&](int s, auto w) {
+    constexpr int w1 = decltype(w)::value;
     const int left = n - 1 - s;
-    if (left >= 3) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    else if (left == 2) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-    else if (left == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+    if (left >= 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * w1 + XP) : "memory");
+    else if (left == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * w1 + XH1) : "memory");
+    else if (left == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(w1) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   };
 
@@ -267,22 +275,25 @@ __global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restric
 #pragma unroll
     for (int j = 0; j < MT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  const int grp = __builtin_amdgcn_readfirstlane(wave >> 2);
-  issue_x(0, 0, 0);
-  issue_x(0, 1, 0);
+  using First = std::integral_constant<int, 0>;
+  using Second = std::integral_constant<int, 1>;
+  using Tiles0 = std::integral_constant<int, WP0>;
+  using Tiles1 = std::integral_constant<int, WP1>;
+  issue_x(0, First(), 0);
+  issue_x(0, Second(), 0);
   issue_w(0);
   issue_w(1);
   if (n > 2) {
-    issue_x(1, 0, 1);
+    issue_x(1, First(), 1);
     issue_w(2);
-    issue_x(1, 1, 1);
+    issue_x(1, Second(), 1);
   }
   if (grp == 1) {
-    wait_for(0);
+    wait_at(0, Tiles1());
     __builtin_amdgcn_s_barrier();           // P0
   }
-  auto step = [&](int s, int half, int xcur, int xfill) {
-    if (grp == 0) wait_for(s);
+  auto step = [&](int s, auto half, int xcur, int xfill) {
+    if (grp == 0) wait_at(s, Tiles0());
     __builtin_amdgcn_s_barrier();           // group 0: P2s | group 1: P2s+1
     const unsigned char* st = smem + (s & 3) * kW;
     const uint4* xs = reinterpret_cast<const uint4*>(smem + kXs + xcur * kX);
@@ -290,7 +301,7 @@ __global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restric
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const int r = wm * (BM / 2) + mt * 16 + c;
-      b[mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + ((4 * half + g) ^ xs_swz<MI_W_BF16>(r))]);
+      b[mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + ((4 * decltype(half)::value + g) ^ xs_swz<MI_W_BF16>(r))]);
     }
 #pragma unroll
     for (int i = 0; i < NTW; ++i) a[i] = *reinterpret_cast<const u32x4_t*>(st + (wn * NTW + i) * 1024 + lane * 16);
@@ -302,7 +313,7 @@ __global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restric
     for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(b[mt]));
 #pragma unroll
     for (int i = 0; i < NTW; ++i) asm volatile("" : "+v"(a[i]));
-    if (grp == 1 && s + 1 < n) wait_for(s + 1);
+    if (grp == 1 && s + 1 < n) wait_at(s + 1, Tiles1());
     __builtin_amdgcn_s_barrier();           // group 0: P2s+1 | group 1: P2s+2
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -313,8 +324,8 @@ __global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restric
   };
   int xcur = 0, xfill = 2;
   for (int s = 0; s < n; s += 2) {
-    step(s, 0, xcur, xfill);
-    step(s + 1, 1, xcur, xfill);
+    step(s, First(), xcur, xfill);
+    step(s + 1, Second(), xcur, xfill);
     xcur = xcur == 2 ? 0 : xcur + 1;
     xfill = xfill == 2 ? 0 : xfill + 1;
   }
@@ -323,21 +334,19 @@ __global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restric
   else epilogue_tile<EPI, NTW, MT>(e, T, NT, m0 + wm * (BM / 2), ntb + wn * NTW, g, c, acc);
 }
 
-// The tiles there are.  bf16 weights: a 64-deep stage of 256 x 192, 256 x 256 or 192 x 256 fits the LDS twice only; 256 x 256 has its own kernel.
-template <int WD>
-constexpr bool wide_tile_built(int bm, int ntw) {
-  return (bm == 64 || bm == 128 || bm == 192 || bm == 256) && ntw >= 2 && ntw <= 4 && (WD != MI_W_BF16 || bm + 64 * ntw <= 384 || (bm == 256 && ntw == 4));
-}
+// bf16 tiles whose 64-deep stages fit the LDS twice only: 256 x 192, 192 x 256, 256 x 256
+constexpr bool wide_tile_by_32(int wd, int bm, int ntw) { return wd == MI_W_BF16 && bm + 64 * ntw > 384; }
 
 template <int WD, int EPI, int BM, int NTW, bool SPLIT>
 static int launch_gemm_wide_t(const LinearW& w, int T, const uint16_t* x, int ldx, const EpiArgs& e, hipStream_t s, int KS, float* slab) {
   const int NT = w.N / 16, KT = w.K / tile_k(WD);
   const dim3 grid(8 * ceil_div(ceil_div(T, BM) * ceil_div(NT, 4 * NTW), 8), 1, KS);
   const uint4* W = reinterpret_cast<const uint4*>(w.w);
-  if constexpr (WD == MI_W_BF16 && BM == 256 && NTW == 4) {
-    const auto fn = gemm_wide16_kernel<EPI, SPLIT>;
-    MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), 160 * 1024));
-    hipLaunchKernelGGL(fn, grid, dim3(512), 160 * 1024, s, W, NT, KT, T, w.K, x, ldx, e, slab);
+  if constexpr (wide_tile_by_32(WD, BM, NTW)) {
+    constexpr int lds = 4 * NTW * 4096 + 3 * BM * 128;
+    const auto fn = gemm_wide16_kernel<EPI, BM, NTW, SPLIT>;
+    MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds));
+    hipLaunchKernelGGL(fn, grid, dim3(512), lds, s, W, NT, KT, T, w.K, x, ldx, e, slab);
   } else {
     constexpr int lds = kWideStages<WD, BM, NTW> * (kWideWBytes<WD, NTW> + BM * 128);
     const auto fn = gemm_wide_kernel<WD, EPI, BM, NTW, SPLIT>;
@@ -351,34 +360,29 @@ static int launch_gemm_wide_t(const LinearW& w, int T, const uint16_t* x, int ld
 template <int WD, int BM, int NTW>
 static int launch_gemm_wide_bm(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
                                int KS, float* ws, SlabSum* defer) {
-  if constexpr (!wide_tile_built<WD>(BM, NTW)) {
-    set_error("gemm_wide: no such tile for this weight type");
-    return MI_EINVAL;
-  } else {
-    if (KS > 1) {
-      MI_TRY_((launch_gemm_wide_t<WD, EPI_F32, BM, NTW, true>(w, T, x, ldx, e, s, KS, ws)));
-      const SlabSum sum{ws, KS, T, w.N, e.scale, e.bias, e.row_scale};
-      if (defer && (epi == EPI_RESID || epi == EPI_F32)) { *defer = sum; return MI_OK; }
-      return launch_splitk_reduce(sum, epi, e, s);
-    }
-#define MI_GW(EPI_) return launch_gemm_wide_t<WD, EPI_, BM, NTW, false>(w, T, x, ldx, e, s, 1, nullptr)
-    switch (epi) {
-      case EPI_QKV: MI_GW(EPI_QKV);
-      case EPI_SWIGLU: MI_GW(EPI_SWIGLU);
-      case EPI_RESID: MI_GW(EPI_RESID);
-      case EPI_F32: MI_GW(EPI_F32);
-    }
-    if constexpr (WD == MI_W_BF16)
-      switch (epi) {
-        case EPI_RELU2: MI_GW(EPI_RELU2);
-        case EPI_GLU_CLIP: MI_GW(EPI_GLU_CLIP);
-        case EPI_SOFTCAP: MI_GW(EPI_SOFTCAP);
-        case EPI_HEADS_KV: MI_GW(EPI_HEADS_KV);
-      }
-#undef MI_GW
-    set_error("gemm_wide: this epilogue is not built for this weight type");
-    return MI_EINVAL;
+  if (KS > 1) {
+    MI_TRY_((launch_gemm_wide_t<WD, EPI_F32, BM, NTW, true>(w, T, x, ldx, e, s, KS, ws)));
+    const SlabSum sum{ws, KS, T, w.N, e.scale, e.bias, e.row_scale};
+    if (defer && (epi == EPI_RESID || epi == EPI_F32)) { *defer = sum; return MI_OK; }
+    return launch_splitk_reduce(sum, epi, e, s);
   }
+#define MI_GW(EPI_) return launch_gemm_wide_t<WD, EPI_, BM, NTW, false>(w, T, x, ldx, e, s, 1, nullptr)
+  switch (epi) {
+    case EPI_QKV: MI_GW(EPI_QKV);
+    case EPI_SWIGLU: MI_GW(EPI_SWIGLU);
+    case EPI_RESID: MI_GW(EPI_RESID);
+    case EPI_F32: MI_GW(EPI_F32);
+  }
+  if constexpr (WD == MI_W_BF16)
+    switch (epi) {
+      case EPI_RELU2: MI_GW(EPI_RELU2);
+      case EPI_GLU_CLIP: MI_GW(EPI_GLU_CLIP);
+      case EPI_SOFTCAP: MI_GW(EPI_SOFTCAP);
+      case EPI_HEADS_KV: MI_GW(EPI_HEADS_KV);
+    }
+#undef MI_GW
+  set_error("gemm_wide: this epilogue is not built for this weight type");
+  return MI_EINVAL;
 }
 
 // bm x 64 ntw tiles, K over ks slices (ks > 1: ws holds them)

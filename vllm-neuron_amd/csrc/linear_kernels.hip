@@ -267,6 +267,8 @@ extern template int launch_gemm_wide_wd<MI_W_INT8>(const LinearW&, int, const ui
 // Against the best of 128 x 256 and 256 x 256 alone, us: int8 gate|up of the 7B model at 188 tokens 79 -> 60 (148 tiles of 256 x 256 on 256 CUs, 73 % of
 // each filled; 198 of 192 x 192), its down projection 41.6 -> 34.4; bf16 gate|up of TinyLlama 700 tokens 51.6 -> 35.4, 200 tokens 28.4 -> 21.4;
 // fp8 QKV of the 8B model 1400 tokens 82.6 -> 63.9; bf16 down projection of 2048 x 14336 at 100 tokens 26.4 -> 17.6.
+// With 256 x 192 and 192 x 256 of bf16 weights (49 more shapes, the choice 0.5 % from the fastest): 12288 x 2048 777 tokens 54.8 -> 46.0, 1000 tokens
+// 55.1 -> 48.5, 3072 x 2048 4000 tokens 58.9 -> 50.2, 28672 x 4096 377 tokens 99.4 -> 82.0, 4096 x 14336 1500 tokens 175.9 -> 153.8.
 struct WidePlan { int bm, ntw, ks; };
 static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, bool deferred) {
   int cus = 256;
@@ -280,12 +282,11 @@ static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, boo
   double best_cost = 0.;
   for (int bm = 64; bm <= 256; bm += 64)
     for (int ntw = 2; ntw <= 4; ++ntw) {
-      if (wd == MI_W_BF16 && !wide_tile_built<MI_W_BF16>(bm, ntw)) continue;
       const double m = bm / 64, area = m * ntw;
       const auto us = [&](const double (&k)[4]) { return k[0] + k[1] * area + k[2] * m + k[3] * ntw; };
       double lo = us(kStep[wd][0]), hi = us(kStep[wd][1]);
-      if (wd == MI_W_BF16 && bm == 256 && ntw == 4) { lo = 0.893; hi = 1.456; }   // (the kernel with 32-deep K-steps)
       if (bm == 192) hi *= 1.04;
+      if (wide_tile_by_32(wd, bm, ntw)) { lo = area == 16 ? 0.893 : 0.95; hi = area == 16 ? 1.456 : 1.2; }   // (the kernel with 32-deep K-steps)
       const int tiles = ceil_div(T, bm) * ceil_div(N, 64 * ntw);
       for (int ks = 1; ks <= 10; ++ks) {
         const int per = ceil_div(nks, ks);
