@@ -39,6 +39,21 @@ def test_edges_of_the_register_gemv(lib, wd, M, N, K):
     assert err < tol, (err, tol)
 
 
+# up to 4 rows, where they go there: one row-tile a work-group, eight and more, one k-tile fewer than a wave has registers for, and one more (the LDS kernels)
+@pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
+@pytest.mark.parametrize("M", [1, 3, 4])
+@pytest.mark.parametrize("N,K", [(16, 64), (4096, 320), (4112, 320), (272, 2048), (528, 2112), (48, 4096), (48, 4160), (32768, 128)])
+def test_edges_of_few_rows(lib, wd, M, N, K):
+    test_edges_of_the_register_gemv(lib, wd, M, N, K)
+
+
+# the same sums at up to 4 rows: K of a narrow projection over several slices
+@pytest.mark.parametrize("rows", [1, 4])
+def test_sums_of_few_rows_left_to_the_next_norm(rows):
+    for family in (_rapodra, _vimesun):
+        test_sums_left_to_the_next_norm(family, rows)
+
+
 def _rapodra():
     from tests import test_rapodra_gpu as T
     from tests.rapodra_cases import config, dense, latent

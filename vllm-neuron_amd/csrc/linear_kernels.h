@@ -63,12 +63,14 @@ struct LinearW {
 // M <= 16 token-generation path (HBM-bound weight streaming).
 int launch_gemv(const LinearW& w, int M, int pro, const ProArgs& p, int epi, const EpiArgs& e,
                 hipStream_t s);
-// The same for 5 .. 32 rows of bf16 activations, with those in registers (gemv_regs.h).  ws: room for the slabs of a split K; defer as launch_gemm.
+// The same for up to 32 rows of bf16 activations, with those in registers (gemv_regs.h).  ws: room for the slabs of a split K; defer as launch_gemm.
 // EpiArgs::row_scale: a factor per row of the product (1 / rms where launch_norm_rows left it out).
 int launch_gemv_regs(const LinearW& w, int M, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s, float* ws, size_t ws_bytes,
                      SlabSum* defer = nullptr, bool split_as_deferred = false);
 // whether M rows of w take it (K beyond 8 slices of the registers, or slabs that do not fit: launch_gemv up to 16 rows, launch_gemm)
 bool gemv_in_regs(const LinearW& w, int M, size_t ws_bytes);
+// whether a projection of 1 .. 4 rows of bf16 activations takes it; deferred: its sums over K have a taker
+bool gemv_few_rows_in_regs(const LinearW& w, int M, size_t ws_bytes, bool deferred);
 // sums the slabs and runs the epilogue
 int launch_splitk_reduce(const SlabSum& sl, int epi, const EpiArgs& e, hipStream_t s);
 // M > 16 context-encoding path (MFMA-bound).  x is always bf16 [T, K].

@@ -42,6 +42,14 @@ template <int WD>
 int launch_gemv_regs_wd(const LinearW& w, int M, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s, float* ws, size_t ws_bytes, SlabSum* defer, bool split_as_deferred);
 template <int WD> bool gemv_regs_fits_wd(int M, int N, int K, size_t ws_bytes);
 
+static bool gemv_regs_fits(const LinearW& w, int M, size_t ws_bytes) {
+  switch (w.wd) {
+    case MI_W_BF16: return gemv_regs_fits_wd<MI_W_BF16>(M, w.N, w.K, ws_bytes);
+    case MI_W_F8E4M3: return gemv_regs_fits_wd<MI_W_F8E4M3>(M, w.N, w.K, ws_bytes);
+    case MI_W_INT8: return gemv_regs_fits_wd<MI_W_INT8>(M, w.N, w.K, ws_bytes);
+  }
+  return false;
+}
 // From 5 rows on (us per call; the LDS kernels with the norm in front of them / these behind a norm kernel; contexts of 500, TinyLlama 200):
 //   8B fp8, 16 layers:  8 rows 1472 / 1332, 16 rows 1758 / 1527, 32 rows 2282 / 2117;   4 rows 1191 / 1277
 //   8B bf16:            8 rows 1949 / 1857, 24 rows 2526 / 2298
@@ -49,14 +57,18 @@ template <int WD> bool gemv_regs_fits_wd(int M, int N, int K, size_t ws_bytes);
 //   TinyLlama bf16:     1 row 876 / 1034, 16 rows 1389 / 1210, 30 rows 1501 / 1450
 //   16 layers of width 256 / 512 / 1024 / 1536, bf16: 5 rows 572 / 467, 604 / 538, 637 / 556, 745 / 673; 32 rows 739 / 604, 790 / 626, 850 / 667, 1001 / 926
 // Up to 4 rows the norm inside the weight stream's kernel and its two to eight waves per row-tile win.
-bool gemv_in_regs(const LinearW& w, int M, size_t ws_bytes) {
-  if (M < 5 || M > 32) return false;
-  switch (w.wd) {
-    case MI_W_BF16: return gemv_regs_fits_wd<MI_W_BF16>(M, w.N, w.K, ws_bytes);
-    case MI_W_F8E4M3: return gemv_regs_fits_wd<MI_W_F8E4M3>(M, w.N, w.K, ws_bytes);
-    case MI_W_INT8: return gemv_regs_fits_wd<MI_W_INT8>(M, w.N, w.K, ws_bytes);
-  }
-  return false;
+bool gemv_in_regs(const LinearW& w, int M, size_t ws_bytes) { return M >= 5 && M <= 32 && gemv_regs_fits(w, M, ws_bytes); }
+// Up to 4 rows of bf16 activations (nothing to fuse in front).  They win where a wave's weights of a row-tile are one batch of requests and each work-group has one
+// row-tile (the chain to the first request is shorter: no staging) or eight and more (the tiles follow each other without a barrier on the way), and, where the sums have a
+// taker, on rows of at most half the CUs: K goes over the other half.  us a launch at 1 / 4 rows, LDS kernels -> these: 2048 x 2048 bf16 5.3 / 5.5 -> 4.3 / 4.3 with a
+// taker, 4.9 / 5.2 without; 2048 x 7680 bf16 9.0 / 9.3 -> 8.2 / 8.6 and 2048 x 14336 13.8 / 14.4 -> 12.5 / 12.7 with one; 4096 x 4096 fp8 7.4 -> 6.5, int8 7.7 -> 7.1;
+// 32768 x 2048 bf16 26.2 -> 23.7.  Not between: 8192 x 2048 bf16 8.1 -> 9.3, 15360 x 2048 12.7 -> 13.4, 5120 x 4096 fp8 7.1 -> 7.5; nor K in two batches: 3584 x 3584 bf16 7.6 -> 7.7.
+bool gemv_few_rows_in_regs(const LinearW& w, int M, size_t ws_bytes, bool deferred) {
+  int cus = 0;
+  if (M < 1 || M > 4 || device_num_cu(&cus) != MI_OK) return false;
+  const int NT = w.N / 16;
+  if (ceil_div(w.K / tile_k(w.wd), kGemvWaves) <= 8 && (NT <= cus || NT >= 8 * cus)) return true;
+  return deferred && 2 * NT <= cus && gemv_regs_fits(w, M, ws_bytes);
 }
 int launch_gemv_regs(const LinearW& w, int M, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s, float* ws, size_t ws_bytes, SlabSum* defer,
                      bool split_as_deferred) {

@@ -104,6 +104,7 @@ int run_linear(mi_ctx* c, const Linear& L, int rows, int pro, ProArgs p, int epi
     if (c->pend.slab) MI_TRY(flush_pending(c));
     Scope sc(c, MI_K_GEMV);
     if (c->prof.on) c->prof.gemv_bytes += (double)L.bytes();
+    if (pro == PRO_BF16 && gemv_few_rows_in_regs(L.view(), rows, 0, false)) return launch_gemv_regs(L.view(), rows, p.x, p.ldx, epi, e, c->stream, nullptr, 0);
     return launch_gemv(L.view(), rows, pro, p, epi, e, c->stream);
   }
   const uint16_t* x = p.x;
@@ -2099,7 +2100,7 @@ int mi_op_qlinear(const void* x, int32_t M, const void* w_tiled, const float* sc
     float* slab = nullptr;
     const size_t bytes = (size_t)64 << 20;
     MI_HIP(hipMalloc(reinterpret_cast<void**>(&slab), bytes));
-    int rc = gemv_in_regs(W, M, bytes) ? launch_gemv_regs(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes)
+    int rc = gemv_in_regs(W, M, bytes) || gemv_few_rows_in_regs(W, M, bytes, false) ? launch_gemv_regs(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes)
              : gemv_fits(M, K) ? launch_gemv(W, M, PRO_BF16, p, EPI_F32, e, (hipStream_t)stream) : launch_gemm(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes);
     hipStreamSynchronize((hipStream_t)stream);
     hipFree(slab);

@@ -81,7 +81,7 @@ int apply(mi_ctx* c, const StackMat& m, int rows, const void* x, int ldx, int ep
     Scope sc(c, MI_K_GEMM);
     return launch_linear_f32((const float*)m.L.w, m.N, m.K, (const float*)x, ldx, rows, epi, e, c->stream);
   }
-  const bool regs = gemv_in_regs(m.L.view(), rows, c->splitk_ws_bytes);
+  const bool regs = gemv_in_regs(m.L.view(), rows, c->splitk_ws_bytes) || gemv_few_rows_in_regs(m.L.view(), rows, c->splitk_ws_bytes, defer != nullptr);
   if (regs || gemv_fits(rows, m.K)) {
     if (!c->runs(MI_K_GEMV)) return MI_OK;
     Scope sc(c, MI_K_GEMV);
