@@ -106,3 +106,28 @@ def test_fp8_activations_stay_with_prompts(rows):
         out.append(model.forward(**decode_inputs(range(rows), [0] * rows, [[1 + i] for i in range(rows)], 32, 32)).clone())
         model.close()
     assert torch.equal(*out)
+
+
+# logits of 17 and more rows to the host: row-tiles four side by side, a number of them that four does and does not divide, one group and several a work-group
+@pytest.mark.parametrize("vocab", [16, 80, 1024, 16448])
+def test_logits_of_many_rows_to_the_host(vocab):
+    from oracle import DecoderConfig
+    from oracle.synth import make_weights
+    from tests.helpers import decode_inputs
+    from vllm_neuron_amd._native import MI_Q, MI_W, NativeModel
+    shape = dict(num_layers=1, hidden_size=128, num_heads=2, num_kv_heads=1, head_dim=64, intermediate_size=256, vocab_size=vocab)
+    w = make_weights(DecoderConfig(**shape), seed=4)
+    for wd in ("bf16", "f8e4m3"):
+        model = NativeModel(**shape, rms_norm_eps=1e-5, rope_theta=1e4, rope_type=0, rope_factor=1.0, num_blocks=33, block_size=32, max_num_seqs=32,
+                            max_model_len=32, weight_dtype=MI_W[wd], quant_type=MI_Q["per_channel_symmetric"], quantize_lm_head=1, tp_degree=1, tp_rank=0,
+                            device_id=0, use_graphs=1, ctx_buckets=[32])
+        model.load_state_dict(w)
+        model.finalize()
+        out = {}
+        for rows in (16, 17, 32):      # (16 rows: single row-tiles)
+            for _ in range(2):         # eager pass, then the graph
+                out[rows] = model.forward(**decode_inputs([i % vocab for i in range(rows)], [0] * rows, [[1 + i] for i in range(rows)], 32, 32)).clone()
+        # the same sums over K a row-tile, whoever stores them; the projections in front differ in low bits between 16 and 17 rows, as between any two kernels
+        std = out[32].std().item()
+        assert torch.isfinite(out[32]).all() and torch.equal(out[17], out[32][:17]) and (out[16] - out[32][:16]).abs().max().item() < 0.05 * std
+        model.close()

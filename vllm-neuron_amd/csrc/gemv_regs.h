@@ -18,7 +18,10 @@ constexpr int kRegsMaxPasses = 64;   // row-tiles of a work-group: their scales 
 // k-tiles a wave holds at most: 4 or 8 of 64 k (1-byte weights), 4, 8 or 16 of 32 k
 template <int WD> constexpr int kRegsMaxTiles = WD == MI_W_BF16 ? 16 : 8;
 
-template <int WD, int EPI, int MG, int NK, bool SLAB>
+// HOLD: a work-group takes HOLD row-tiles side by side, and the wave that sums them keeps their results until it has all: a row's HOLD x 64 bytes
+// leave together.  For results that go over PCIe: neighbouring 64 bytes that come from different work-groups take a packet each, 44 GB/s; 128 or 256 bytes
+// of one work-group 52 - 55, what a copy reaches.
+template <int WD, int EPI, int MG, int NK, bool SLAB, int HOLD = 1>
 __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4* __restrict__ W, int NT, int KT, int M, int G,
                                                                    const uint16_t* __restrict__ x, int ldx, EpiArgs e, float* __restrict__ slab) {
   constexpr int FR = WD == MI_W_BF16 ? 1 : 2;         // MFMAs per weight tile and column group
@@ -32,7 +35,9 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
   const int kper = ceil_div(KT, (int)gridDim.y), k_lo = (int)blockIdx.y * kper, k_hi = min(k_lo + kper, KT);
   const int ktw = ceil_div(k_hi - k_lo, kGemvWaves);
   const int kbeg = min(k_lo + wave * ktw, k_hi), kend = min(kbeg + ktw, k_hi), klast = max(kend - 1, k_lo);
-  const int passes = ceil_div(NT - (int)blockIdx.x, G);
+  const auto tile_of = [&](int pass) { return HOLD == 1 ? (int)blockIdx.x + pass * G : ((int)blockIdx.x + pass / HOLD * G) * HOLD + pass % HOLD; };
+  int passes = ceil_div(ceil_div(NT, HOLD) - (int)blockIdx.x, G) * HOLD;
+  if constexpr (HOLD > 1) passes -= max(tile_of(passes - 1) + 1 - NT, 0);       // (the last group may be short)
 
   // ---- this wave's activations: row c (and 16 + c) of every k-tile it owns; tiles it does not own multiply zeros ----
   u32x4_t xf[NK * FR * MG];
@@ -61,7 +66,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
   const int total = passes * NB;
   auto issue = [&](u32x4_t (&buf)[BT], int i) {
     const bool live = i < total;                      // (a batch that does not exist: one line, the same for every lane)
-    const int ii = min(i, total - 1), tile = (int)blockIdx.x + (ii / NB) * G, k0 = kbeg + (ii % NB) * BT;
+    const int ii = min(i, total - 1), tile = tile_of(ii / NB), k0 = kbeg + (ii % NB) * BT;
     const uint4* base = live ? W + (size_t)tile * KT * 64 : W;
     const int kstep = live ? 64 : 0;
     const unsigned at = live ? lane : 0;
@@ -86,7 +91,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
     for (int q = 0; q < kRegsMaxPasses * 16 / (kGemvWaves * 64); ++q) {
       const int i = tid + q * kGemvWaves * 64;
       if (i < n) {
-        const int at = ((int)blockIdx.x + (i >> 4) * G) * 16 + (i & 15);
+        const int at = tile_of(i >> 4) * 16 + (i & 15);
         sc_lds[i] = e.scale[at];
         bi_lds[i] = e.bias ? e.bias[at] : 0.f;
       }
@@ -124,17 +129,38 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
+  f32x4_t held[HOLD];
   auto finish = [&](int pass, int par) {
 #pragma unroll
     for (int mg = 0; mg < MG; ++mg) {
-      if (wave != ((pass * MG + mg) & (kGemvWaves - 1))) continue;
+      if (wave != ((pass / HOLD * MG + mg) & (kGemvWaves - 1))) continue;
       f32x4_t s = red[par][0][mg][lane];
 #pragma unroll
       for (int w = 1; w < kGemvWaves; ++w) {
         const f32x4_t t = red[par][w][mg][lane];
         s[0] += t[0]; s[1] += t[1]; s[2] += t[2]; s[3] += t[3];
       }
-      const int m = mg * 16 + c, n0 = ((int)blockIdx.x + pass * G) * 16 + g * 4;
+      const int m = mg * 16 + c, n0 = tile_of(pass) * 16 + g * 4;
+      if constexpr (HOLD > 1) {
+        static_assert(!SLAB && (EPI == EPI_F32 || EPI == EPI_SOFTCAP), "rows of fp32");
+        const float *sc4 = sc_lds + pass * 16 + g * 4, *b4 = bi_lds + pass * 16 + g * 4;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          s[r] *= sc4[r] * rmul[mg];
+          if (e.bias) s[r] += b4[r];
+          if constexpr (EPI == EPI_SOFTCAP) s[r] = e.softcap * tanhf(s[r] / e.softcap);
+        }
+        const int sub = pass % HOLD;
+#pragma unroll
+        for (int h = 0; h < HOLD; ++h)
+          if (h == sub) held[h] = s;
+        if (m < M && (sub == HOLD - 1 || pass == passes - 1)) {
+#pragma unroll
+          for (int h = 0; h < HOLD; ++h)
+            if (h <= sub) *reinterpret_cast<f32x4_t*>(e.out_f32 + (size_t)m * e.ld_out + n0 + (h - sub) * 16) = held[h];
+        }
+        continue;
+      }
       if (m >= M) continue;
       if constexpr (SLAB) {
         *reinterpret_cast<float4*>(slab + ((size_t)blockIdx.y * M + m) * (NT * 16) + n0) = make_float4(s[0], s[1], s[2], s[3]);
@@ -175,19 +201,19 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
   }
 }
 
-template <int WD, int EPI, int MG, bool SLAB>
+template <int WD, int EPI, int MG, bool SLAB, int HOLD = 1>
 static int launch_gemv_regs_k(const LinearW& w, int M, const uint16_t* x, int ldx, const EpiArgs& e, hipStream_t s, int slices, float* slab) {
   const int NT = w.N / 16, KT = w.K / tile_k(WD);
   int num_cu = 0;
   MI_TRY_(device_num_cu(&num_cu));
   const int tiles = ceil_div(ceil_div(KT, slices), kGemvWaves), per = std::max(1, num_cu / slices);
   // every work-group the same number of row-tiles, or one less; at most kRegsMaxPasses
-  const int G = ceil_div(NT, std::min(kRegsMaxPasses, ceil_div(NT, std::min(NT, per))));
+  const int groups = ceil_div(NT, HOLD), G = ceil_div(groups, std::min(kRegsMaxPasses / HOLD, ceil_div(groups, std::min(groups, per))));
   const dim3 grid(G, slices);
   const uint4* W = reinterpret_cast<const uint4*>(w.w);
-  if (tiles <= 4) hipLaunchKernelGGL((gemv_regs_kernel<WD, EPI, MG, 4, SLAB>), grid, dim3(kGemvWaves * 64), 0, s, W, NT, KT, M, G, x, ldx, e, slab);
-  else if (tiles <= 8) hipLaunchKernelGGL((gemv_regs_kernel<WD, EPI, MG, 8, SLAB>), grid, dim3(kGemvWaves * 64), 0, s, W, NT, KT, M, G, x, ldx, e, slab);
-  else if constexpr (WD == MI_W_BF16) hipLaunchKernelGGL((gemv_regs_kernel<WD, EPI, MG, 16, SLAB>), grid, dim3(kGemvWaves * 64), 0, s, W, NT, KT, M, G, x, ldx, e, slab);
+  if (tiles <= 4) hipLaunchKernelGGL((gemv_regs_kernel<WD, EPI, MG, 4, SLAB, HOLD>), grid, dim3(kGemvWaves * 64), 0, s, W, NT, KT, M, G, x, ldx, e, slab);
+  else if (tiles <= 8) hipLaunchKernelGGL((gemv_regs_kernel<WD, EPI, MG, 8, SLAB, HOLD>), grid, dim3(kGemvWaves * 64), 0, s, W, NT, KT, M, G, x, ldx, e, slab);
+  else if constexpr (WD == MI_W_BF16) hipLaunchKernelGGL((gemv_regs_kernel<WD, EPI, MG, 16, SLAB, HOLD>), grid, dim3(kGemvWaves * 64), 0, s, W, NT, KT, M, G, x, ldx, e, slab);
   MI_HIP(hipGetLastError());
   return MI_OK;
 }
@@ -223,6 +249,13 @@ int launch_gemv_regs_wd(const LinearW& w, int M, const uint16_t* x, int ldx, int
     const SlabSum sum{ws, slices, M, w.N, e.scale, e.bias, e.row_scale};
     if (deferred) { *defer = sum; return MI_OK; }
     return launch_splitk_reduce(sum, epi, e, s);
+  }
+  // (up to 16 rows the weights take longer than the way to the host, and single row-tiles deal them out more evenly: 8B fp8 8 rows 1266 us, 1280 with four;
+  //  24 rows 1695 and 1670, 7B int8 32 rows 1890 and 1830)
+  if (e.far_out && M > 16) {
+    if (epi == EPI_F32) return launch_gemv_regs_k<WD, EPI_F32, 2, false, 4>(w, M, x, ldx, e, s, 1, nullptr);
+    if constexpr (WD == MI_W_BF16)
+      if (epi == EPI_SOFTCAP) return launch_gemv_regs_k<WD, EPI_SOFTCAP, 2, false, 4>(w, M, x, ldx, e, s, 1, nullptr);
   }
 #define MI_R(EPI_) return M <= 16 ? launch_gemv_regs_k<WD, EPI_, 1, false>(w, M, x, ldx, e, s, 1, nullptr) : launch_gemv_regs_k<WD, EPI_, 2, false>(w, M, x, ldx, e, s, 1, nullptr)
   switch (epi) {

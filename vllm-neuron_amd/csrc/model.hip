@@ -394,6 +394,7 @@ int run_head(mi_ctx* c, int logits_rows, int logits_row0, bool gather) {
     p.gain = c->g_final; p.eps = k.rms_norm_eps;
     EpiArgs e{};
     e.out_f32 = c->head_out ? c->head_out : c->logits; e.ld_out = c->V_l;
+    e.far_out = c->head_out != nullptr;
     MI_TRY(run_linear(c, c->lm_head, logits_rows, PRO_NORM, p, EPI_F32, e));
   }
   if (c->grp) {

@@ -1802,6 +1802,7 @@ int stack_head(mi_ctx* c, const float* resid, int nrows) {
   EpiArgs e{};
   float* out = c->head_out ? c->head_out : c->logits;
   e.out_f32 = direct ? out : S->logits_pad;
+  e.far_out = direct && c->head_out;
   e.ld_out = S->head.N;
   e.softcap = S->cfg.logit_softcap;
   MI_TRY(apply(c, S->head, nrows, S->n1, S->Kd, e.softcap > 0.f ? EPI_SOFTCAP : EPI_F32, e));
