@@ -16,3 +16,13 @@ def test_chunks_in_pairs(lib, shape, lengths, chunks):  # noqa: F811
     close(*x.step([(i, n) for i, n in enumerate(lengths)], chunks=chunks), 1)
     for i in range(len(lengths)):
         x.check_state(i)
+
+
+# value columns: whole quads short of a tile, one past 64 and 128, no whole quad; keys of two rounds of lanes, of one past 128; bf16 and fp32 outputs
+@pytest.mark.parametrize("shape", [(2, 1, 32, 20, 4), (5, 5, 16, 68, 3), (2, 2, 48, 132, 1), (3, 1, 24, 30, 4), (2, 1, 144, 64, 4), (1, 1, 256, 128, 5)])
+def test_edges_of_columns(lib, shape):  # noqa: F811
+    for f32 in (0, 1):
+        x = Delta(lib, *shape, [40, 17, 2], seed=sum(shape))
+        close(*x.step([(0, 40), (1, 17), (2, 2)], f32), f32)
+        for i in range(3):
+            x.check_state(i)
