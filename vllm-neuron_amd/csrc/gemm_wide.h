@@ -28,7 +28,7 @@ namespace mi {
 // A work-group's tile: BM tokens x 64 NTW weight rows (NTW 16-row tiles for each of the four waves side by side).
 template <int WD, int NTW> constexpr int kWideWBytes = NTW * (WD == MI_W_BF16 ? 8 : 4) * 1024;   // the weight rows of a 64-deep K-step
 // as many stages as the LDS holds, eight at most
-template <int WD, int BM, int NTW> constexpr int kWideStages = std::min(8, 160 * 1024 / (kWideWBytes<WD, NTW> + BM * 128));
+template <int WD, int BM, int NTW, int KD = 1> constexpr int kWideStages = std::min(8, 160 * 1024 / (KD * (kWideWBytes<WD, NTW> + BM * 128)));
 
 // Waits until at most the youngest min(left, MOST) K-steps' DMAs (PER each) of this wave are in flight.
 template <int PER, int MOST>
@@ -50,9 +50,9 @@ __device__ __forceinline__ bool wide_tile(int T, int NT, int& m0, int& nt0) {
   return true;
 }
 // the K-steps of grid.z slice blockIdx.z: equal ones, the last may be shorter (the launch leaves none empty)
-template <bool SPLIT>
+template <bool SPLIT, int KD = 1>
 __device__ __forceinline__ void wide_slice(int K, int& ks0, int& nks) {
-  const int all = K / 64, per = SPLIT ? ceil_div(all, (int)gridDim.z) : all;
+  const int all = K / (64 * KD), per = SPLIT ? ceil_div(all, (int)gridDim.z) : all;
   ks0 = SPLIT ? (int)blockIdx.z * per : 0;
   nks = min(per, all - ks0);
 }
@@ -71,20 +71,24 @@ __device__ __forceinline__ void store_slab(float* __restrict__ slab, int T, int 
   }
 }
 
+// KD 64-deep parts to a K-step.  A phase (READ or MULTIPLY) costs some 340 cycles of barrier, LDS latency and requests even without its MFMAs; in the smallest tiles
+// of one-byte weights that is what a 64-deep K-step takes (us each at 128 work-groups, 64 x 128: fp8 0.325, 128-deep ones 0.294; int8 0.402, 0.326; 128 x 128: int8 0.472, 0.424).
+// The K-steps behind which another one is requested run in a loop of their own, without a count of what is left to wait for: us a K-step at 250 work-groups, one loop ->
+// two, 256 x 192 fp8 1.27 -> 1.14, int8 1.35 -> 1.20; 192 x 192 int8 1.14 -> 1.02; 64 x 128 fp8 0.388 -> 0.367.
 // A wave multiplies BM / 2 tokens x 16 NTW weight rows: NTW BM / 8 accumulator registers (256 x 256: 128, and 246 VGPRs
 // with the decoded fragments of one K-step).
 // SPLIT: grid.z K-slices write raw fp32 accumulators to slab[z][m][n] (see gemm_a8_kernel).
-template <int WD, int EPI, int BM, int NTW, bool SPLIT>
+template <int WD, int EPI, int BM, int NTW, bool SPLIT, int KD>
 __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict__ W, int NT, int KT, int T, int K,
                                                         const uint16_t* __restrict__ x, int ldx, EpiArgs e,
                                                         float* __restrict__ slab) {
-  constexpr int kW = kWideWBytes<WD, NTW>, kStage = kW + BM * 128, kStages = kWideStages<WD, BM, NTW>;
+  constexpr int kW = KD * kWideWBytes<WD, NTW>, kStage = kW + KD * BM * 128, kStages = kWideStages<WD, BM, NTW, KD>;
   static_assert(kStages >= 3, "the two wave groups need three stages");
   // waves as 2 (tokens) x 4 (weight rows), each MT 16-token tiles x NTW 16-row weight tiles (4 x 2 waves would read 16 instead of 20 KiB of
   // fragments per K-step at 256 x 256 but decode every weight code four times instead of twice)
   constexpr int MT = BM / 32, WM = 2;
-  constexpr int XP = BM / 64;                 // 8-row activation pieces per wave and stage
-  constexpr int WPK = WD == MI_W_BF16 ? 2 : 1;   // 1 KiB weight tiles per 16 rows and K-step
+  constexpr int XH = BM / 64, XP = KD * XH;   // 8-row activation pieces per wave and 64-deep part, and per stage
+  constexpr int WPH = WD == MI_W_BF16 ? 2 : 1, WPK = KD * WPH;   // 1 KiB weight tiles per 16 rows and 64-deep part, and per K-step
   // the 4 NTW WPK weight tiles of a stage over the waves: group 0 (waves 0-3) may bring one more each than group 1 (twelve tiles)
   constexpr int WP0 = (NTW * WPK + 1) / 2, WP1 = NTW * WPK - WP0;
   constexpr int kDma0 = WP0 + XP, kDma1 = WP1 + XP;   // DMAs per wave and stage
@@ -95,7 +99,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
   int m0, ntb;
   if (!wide_tile<BM, NTW>(T, NT, m0, ntb)) return;
   int ks0, nks;                               // this slice's K-steps, from K-step ks0 on
-  wide_slice<SPLIT>(K, ks0, nks);
+  wide_slice<SPLIT, KD>(K, ks0, nks);
 
   // this lane's DMA sources: weight tiles wt0 .. (fragment order) and XP 8-row pieces of the activation tile
   const int grp = __builtin_amdgcn_readfirstlane(wave >> 2), wt0 = grp == 0 ? WP0 * wave : 4 * WP0 + WP1 * (wave - 4);
@@ -108,8 +112,8 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
   }
 #pragma unroll
   for (int i = 0; i < XP; ++i) {
-    const int r = (XP * wave + i) * 8 + (lane >> 3), sl = lane & 7;
-    xsrc[i] = x + (size_t)min(m0 + r, T - 1) * ldx + (size_t)ks0 * 64 + ((sl ^ xs_swz<WD>(r)) * 8);   // LDS slot sl of row r holds chunk sl ^ swz(r)
+    const int r = (XH * wave + i % XH) * 8 + (lane >> 3), sl = lane & 7;
+    xsrc[i] = x + (size_t)min(m0 + r, T - 1) * ldx + (size_t)(ks0 * KD + i / XH) * 64 + ((sl ^ xs_swz<WD>(r)) * 8);   // LDS slot sl of row r holds chunk sl ^ swz(r)
   }
   auto issue = [&](int ks, int stage) {
     unsigned char* st = smem + stage * kStage;
@@ -119,7 +123,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
       if (grp == 0) glds16(wsrc[WP1] + (size_t)ks * WPK * 64, st + (wt0 + WP1) * 1024);
     }
 #pragma unroll
-    for (int i = 0; i < XP; ++i) glds16(xsrc[i] + (size_t)ks * 64, st + kW + (XP * wave + i) * 1024);
+    for (int i = 0; i < XP; ++i) glds16(xsrc[i] + (size_t)ks * (64 * KD), st + kW + (i / XH) * (BM * 128) + (XH * wave + i % XH) * 1024);
   };
 
   f32x4_t acc[NTW][MT];
@@ -147,66 +151,79 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
     __builtin_amdgcn_s_barrier();           // P0
   }
   int cur = 0, fill = kStages - 1;          // the stages of K-step ks and of K-step ks + kStages - 1
-  for (int ks = 0; ks < nks; ++ks) {
-    if (grp == 0) wait_dma<kDma0, kStages - 2>(nks - 1 - ks);   // own pieces of stage ks
+  auto step = [&](int ks, auto steady) {
+    constexpr bool more = decltype(steady)::value;         // K-step ks + kStages - 1 exists: no counting on the way
+    if (grp == 0) {                           // own pieces of stage ks
+      if constexpr (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kDma0 * (kStages - 2)) : "memory");
+      else wait_dma<kDma0, kStages - 2>(nks - 1 - ks);
+    }
     __builtin_amdgcn_s_barrier();           // group 0: P2ks | group 1: P2ks+1 -- either way nobody reads stage ks - 1 any more
     const unsigned char* st = smem + cur * kStage;
-    const uint4* xs = reinterpret_cast<const uint4*>(st + kW);
-    u32x4_t b0[MT], b1[MT], w0[NTW], w1[NTW];
+    u32x4_t b[KD][2][MT], w[NTW][WPK];
 #pragma unroll
-    for (int i = 0; i < NTW; ++i) {
-      const u32x4_t* w = reinterpret_cast<const u32x4_t*>(st + (wn * NTW + i) * (WPK * 1024) + lane * 16);
-      w0[i] = w[0];
-      if constexpr (WD == MI_W_BF16) w1[i] = w[64];
-    }
+    for (int i = 0; i < NTW; ++i)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int r = wm * (BM / 2) + mt * 16 + c;
-      const int ch0 = WD == MI_W_BF16 ? g : 2 * g, ch1 = WD == MI_W_BF16 ? 4 + g : 2 * g + 1;
-      b0[mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + (ch0 ^ xs_swz<WD>(r))]);
-      b1[mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + (ch1 ^ xs_swz<WD>(r))]);
+      for (int q = 0; q < WPK; ++q) w[i][q] = reinterpret_cast<const u32x4_t*>(st + (wn * NTW + i) * (WPK * 1024) + lane * 16)[q * 64];
+#pragma unroll
+    for (int d = 0; d < KD; ++d) {
+      const uint4* xs = reinterpret_cast<const uint4*>(st + kW + d * (BM * 128));
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const int r = wm * (BM / 2) + mt * 16 + c;
+        const int ch0 = WD == MI_W_BF16 ? g : 2 * g, ch1 = WD == MI_W_BF16 ? 4 + g : 2 * g + 1;
+        b[d][0][mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + (ch0 ^ xs_swz<WD>(r))]);
+        b[d][1][mt] = *reinterpret_cast<const u32x4_t*>(&xs[r * 8 + (ch1 ^ xs_swz<WD>(r))]);
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (ks + kStages - 1 < nks) issue(ks + kStages - 1, fill);
+    if constexpr (more) issue(ks + kStages - 1, fill);
     __builtin_amdgcn_sched_barrier(0);
     cur = cur + 1 == kStages ? 0 : cur + 1;
     fill = fill + 1 == kStages ? 0 : fill + 1;
     // the fragments are in registers (the empty asm takes them as operands: the compiler's wait for the reads sits in front of it)
 #pragma unroll
-    for (int i = 0; i < NTW; ++i) {
-      asm volatile("" : "+v"(w0[i]));
-      if constexpr (WD == MI_W_BF16) asm volatile("" : "+v"(w1[i]));
-    }
+    for (int i = 0; i < NTW; ++i)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) { asm volatile("" : "+v"(b0[mt])); asm volatile("" : "+v"(b1[mt])); }
-    if (grp == 1 && ks + 1 < nks) wait_dma<kDma1, kStages - 2>(nks - 2 - ks);   // own pieces of stage ks + 1: group 0 reads it behind the next barrier
+      for (int q = 0; q < WPK; ++q) asm volatile("" : "+v"(w[i][q]));
+#pragma unroll
+    for (int d = 0; d < KD; ++d)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) { asm volatile("" : "+v"(b[d][0][mt])); asm volatile("" : "+v"(b[d][1][mt])); }
+    if (grp == 1) {                           // own pieces of stage ks + 1: group 0 reads it behind the next barrier
+      if constexpr (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kDma1 * (kStages - 2)) : "memory");
+      else if (ks + 1 < nks) wait_dma<kDma1, kStages - 2>(nks - 2 - ks);
+    }
     __builtin_amdgcn_s_barrier();           // group 0: P2ks+1 | group 1: P2ks+2
     __builtin_amdgcn_sched_barrier(0);
     // the codes of weight tile i + 1 are decoded between the MFMAs of tile i, whose 16 cycles leave room for three vector instructions each
     u32x4_t a[2], an[2];
-    auto piece = [&](const u32x4_t& w, int q) { const uint32_t v = w[q >> 1]; return decode2<WD>(v, q & 1); };
+    auto piece = [&](const u32x4_t& v4, int q) { const uint32_t v = v4[q >> 1]; return decode2<WD>(v, q & 1); };
     if constexpr (WD != MI_W_BF16) {
 #pragma unroll
-      for (int q = 0; q < 8; ++q) a[q >> 2][q & 3] = piece(w0[0], q);
+      for (int q = 0; q < 8; ++q) a[q >> 2][q & 3] = piece(w[0][0], q);
     }
 #pragma unroll
-    for (int i = 0; i < NTW; ++i) {
-      if constexpr (WD == MI_W_BF16) { a[0] = w0[i]; a[1] = w1[i]; }
+    for (int t = 0; t < KD * NTW; ++t) {
+      const int d = t / NTW, i = t % NTW;
+      if constexpr (WD == MI_W_BF16) { a[0] = w[i][2 * d]; a[1] = w[i][2 * d + 1]; }
 #pragma unroll
-      for (int m2 = 0; m2 < 2 * MT; ++m2) {   // both halves of a K-step one after the other: two MFMAs in a row never meet in an accumulator
+      for (int m2 = 0; m2 < 2 * MT; ++m2) {   // both halves one after the other: two MFMAs in a row never meet in an accumulator
         const int h = m2 / MT, mt = m2 % MT;
-        acc[i][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[h]), __builtin_bit_cast(bf16x8_t, h ? b1[mt] : b0[mt]), acc[i][mt], 0, 0, 0);
+        acc[i][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[h]), __builtin_bit_cast(bf16x8_t, b[d][h][mt]), acc[i][mt], 0, 0, 0);
         if constexpr (WD != MI_W_BF16) {
-          if (i + 1 < NTW) {
+          if (t + 1 < KD * NTW) {
 #pragma unroll
-            for (int q = m2 * 4 / MT; q < (m2 + 1) * 4 / MT; ++q) an[q >> 2][q & 3] = piece(w0[i + 1], q);
+            for (int q = m2 * 4 / MT; q < (m2 + 1) * 4 / MT; ++q) an[q >> 2][q & 3] = piece(w[(t + 1) % NTW][(t + 1) / NTW], q);
           }
           __builtin_amdgcn_sched_barrier(0);
         }
       }
       if constexpr (WD != MI_W_BF16) { a[0] = an[0]; a[1] = an[1]; }
     }
-  }
+  };
+  int ks = 0;
+  for (; ks + kStages - 1 < nks; ++ks) step(ks, std::true_type());
+  for (; ks < nks; ++ks) step(ks, std::false_type());
   if (grp == 0) __builtin_amdgcn_s_barrier();   // the barrier group 1 executed first
   if constexpr (SPLIT) store_slab<NTW, MT>(slab + (size_t)blockIdx.z * T * (NT * 16), T, NT, m0 + wm * (BM / 2), ntb + wn * NTW, g, c, acc);
   else epilogue_tile<EPI, NTW, MT>(e, T, NT, m0 + wm * (BM / 2), ntb + wn * NTW, g, c, acc);
@@ -292,8 +309,12 @@ __global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restric
     wait_at(0, Tiles1());
     __builtin_amdgcn_s_barrier();           // P0
   }
-  auto step = [&](int s, auto half, int xcur, int xfill) {
-    if (grp == 0) wait_at(s, Tiles0());
+  auto step = [&](int s, auto half, int xcur, int xfill, auto steady) {
+    constexpr bool more = decltype(steady)::value;
+    if (grp == 0) {
+      if constexpr (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * WP0 + XP) : "memory");
+      else wait_at(s, Tiles0());
+    }
     __builtin_amdgcn_s_barrier();           // group 0: P2s | group 1: P2s+1
     const unsigned char* st = smem + (s & 3) * kW;
     const uint4* xs = reinterpret_cast<const uint4*>(smem + kXs + xcur * kX);
@@ -306,14 +327,17 @@ __global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restric
 #pragma unroll
     for (int i = 0; i < NTW; ++i) a[i] = *reinterpret_cast<const u32x4_t*>(st + (wn * NTW + i) * 1024 + lane * 16);
     __builtin_amdgcn_sched_barrier(0);
-    if (s + 3 < n) issue_w(s + 3);
-    if ((s >> 1) + 2 < (n >> 1)) issue_x((s >> 1) + 2, half, xfill);
+    if (more || s + 3 < n) issue_w(s + 3);
+    if (more || (s >> 1) + 2 < (n >> 1)) issue_x((s >> 1) + 2, half, xfill);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(b[mt]));
 #pragma unroll
     for (int i = 0; i < NTW; ++i) asm volatile("" : "+v"(a[i]));
-    if (grp == 1 && s + 1 < n) wait_at(s + 1, Tiles1());
+    if (grp == 1) {
+      if constexpr (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * WP1 + XP) : "memory");
+      else if (s + 1 < n) wait_at(s + 1, Tiles1());
+    }
     __builtin_amdgcn_s_barrier();           // group 0: P2s+1 | group 1: P2s+2
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -323,17 +347,22 @@ __global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restric
         acc[i][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[i]), __builtin_bit_cast(bf16x8_t, b[mt]), acc[i][mt], 0, 0, 0);
   };
   int xcur = 0, xfill = 2;
-  for (int s = 0; s < n; s += 2) {
-    step(s, First(), xcur, xfill);
-    step(s + 1, Second(), xcur, xfill);
+  auto pair = [&](int s, auto steady) {
+    step(s, First(), xcur, xfill, steady);
+    step(s + 1, Second(), xcur, xfill, steady);
     xcur = xcur == 2 ? 0 : xcur + 1;
     xfill = xfill == 2 ? 0 : xfill + 1;
-  }
+  };
+  int s = 0;
+  for (; s + 4 < n; s += 2) pair(s, std::true_type());      // both request, and two K-steps' DMAs are behind what they wait for
+  for (; s < n; s += 2) pair(s, std::false_type());
   if (grp == 0) __builtin_amdgcn_s_barrier();   // the barrier group 1 executed first
   if constexpr (SPLIT) store_slab<NTW, MT>(slab + (size_t)blockIdx.z * T * (NT * 16), T, NT, m0 + wm * (BM / 2), ntb + wn * NTW, g, c, acc);
   else epilogue_tile<EPI, NTW, MT>(e, T, NT, m0 + wm * (BM / 2), ntb + wn * NTW, g, c, acc);
 }
 
+// tiles of one-byte weights with 128-deep K-steps: what fits the LDS three times
+constexpr bool wide_tile_deep(int wd, int bm, int ntw) { return wd != MI_W_BF16 && 2 * (ntw * 4096 + bm * 128) * 3 <= 160 * 1024; }
 // bf16 tiles whose 64-deep stages fit the LDS twice only: 256 x 192, 192 x 256, 256 x 256
 constexpr bool wide_tile_by_32(int wd, int bm, int ntw) { return wd == MI_W_BF16 && bm + 64 * ntw > 384; }
 
@@ -348,10 +377,20 @@ static int launch_gemm_wide_t(const LinearW& w, int T, const uint16_t* x, int ld
     MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds));
     hipLaunchKernelGGL(fn, grid, dim3(512), lds, s, W, NT, KT, T, w.K, x, ldx, e, slab);
   } else {
-    constexpr int lds = kWideStages<WD, BM, NTW> * (kWideWBytes<WD, NTW> + BM * 128);
-    const auto fn = gemm_wide_kernel<WD, EPI, BM, NTW, SPLIT>;
-    MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds));
-    hipLaunchKernelGGL(fn, grid, dim3(512), lds, s, W, NT, KT, T, w.K, x, ldx, e, slab);
+    const auto launch = [&](auto deep) {
+      constexpr int KD = decltype(deep)::value, lds = kWideStages<WD, BM, NTW, KD> * KD * (kWideWBytes<WD, NTW> + BM * 128);
+      const auto fn = gemm_wide_kernel<WD, EPI, BM, NTW, SPLIT, KD>;
+      MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds));
+      hipLaunchKernelGGL(fn, grid, dim3(512), lds, s, W, NT, KT, T, w.K, x, ldx, e, slab);
+      return (int)MI_OK;
+    };
+    // 128-deep K-steps where a phase would be shorter than its reads: weights of a byte in the smallest tiles, if no slice of K stays empty by them
+    bool deep = false;
+    if constexpr (wide_tile_deep(WD, BM, NTW)) {
+      deep = w.K % 128 == 0 && (KS - 1) * ceil_div(w.K / 128, KS) < w.K / 128;
+      if (deep) MI_TRY_(launch(std::integral_constant<int, 2>()));
+    }
+    if (!deep) MI_TRY_(launch(std::integral_constant<int, 1>()));
   }
   MI_HIP(hipGetLastError());
   return MI_OK;
