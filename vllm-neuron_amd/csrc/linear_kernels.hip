@@ -24,6 +24,8 @@
 // All share one epilogue on D[n = 4g + r][m = c] (lane = 16 g + c): dequant scale, bias,
 // then fp32 store | RoPE + q/KV-pool scatter | SwiGLU.
 
+#include <cmath>
+
 #include "linear_kernels.h"
 
 #include "gemm_wide.h"
@@ -269,12 +271,14 @@ extern template int launch_gemm_wide_wd<MI_W_BF16>(const LinearW&, int, const ui
 extern template int launch_gemm_wide_wd<MI_W_F8E4M3>(const LinearW&, int, const uint16_t*, int, int, const EpiArgs&, hipStream_t, int, int, int, float*, SlabSum*);
 extern template int launch_gemm_wide_wd<MI_W_INT8>(const LinearW&, int, const uint16_t*, int, int, const EpiArgs&, hipStream_t, int, int, int, float*, SlabSum*);
 
-// Which tile and K-split: the cheapest of a model of the kernel, us, fitted to 167 shapes (40 .. 4000 tokens, the projections of TinyLlama,
-// Llama-8B, Qwen2.5-7B and of the layer stacks; every tile and up to eight splits of each timed; the choice is 1.6 % from the fastest on average).  The
-// kernel holds more than half of a CU's LDS, i.e. ONE work-group per CU, so a launch is rounds of 32 work-groups on each of the eight XCDs: 4.1 us, and
+// Which tile and K-split: the cheapest of a model of the kernel, us, fitted to 167 shapes for bf16 weights and 148 for those of a byte (40 .. 4000 tokens, the
+// projections of TinyLlama, Llama-8B, Qwen2.5-7B and of the layer stacks; every tile and up to ten slices of each timed; the choice is 2 % from the fastest on average).
+// The kernel holds more than half of a CU's LDS, i.e. ONE work-group per CU, so a launch is rounds of 32 work-groups on each of the eight XCDs:
 // a round a ramp and epilogue that grow with the tile, beside its K-steps.  us per 64-deep K-step on an almost empty and on a full chip:
-//     128 x 256: fp8 0.53 / 0.79, bf16 0.75 / 0.83, int8 0.75 / 0.89;  256 x 256: fp8 0.91 / 1.33, bf16 0.89 / 1.46, int8 0.88 / 1.37
-//     192 x 192: fp8 0.57 / 0.89, bf16 0.70 / 0.86, int8 0.67 / 0.95;   64 x 128: fp8 0.22 / 0.35, bf16 0.31 / 0.39, int8 0.39 / 0.43
+//     64 x 128: fp8 0.19 / 0.28, bf16 0.31 / 0.39, int8 0.31 / 0.39;  128 x 256: fp8 0.64 / 0.77, bf16 0.75 / 0.83, int8 0.81 / 0.92
+//     192 x 192: fp8 0.69 / 0.85, bf16 0.70 / 0.86, int8 0.72 / 0.95;  256 x 256: fp8 1.06 / 1.30, bf16 0.89 / 1.46, int8 0.99 / 1.37
+// For weights of a byte their stream has a term: with a slice for every CU it is memory that binds, and fewer slices are as fast (8B fp8 prompts of 75 / 140 / 430 tokens
+// 1823 -> 1750, 2229 -> 2134, 3754 -> 3654 us a call; with constants of the same kind bf16 gained 4 % in places and lost 1 % in others: left).
 // A K-split writes its slabs, and a second launch sums them, or the row norm that follows reads them.
 // Against the best of 128 x 256 and 256 x 256 alone, us: int8 gate|up of the 7B model at 188 tokens 79 -> 60 (148 tiles of 256 x 256 on 256 CUs, 73 % of
 // each filled; 198 of 192 x 192), its down projection 41.6 -> 34.4; bf16 gate|up of TinyLlama 700 tokens 51.6 -> 35.4, 200 tokens 28.4 -> 21.4;
@@ -286,10 +290,17 @@ static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, boo
   int cus = 256;
   if (device_num_cu(&cus) != MI_OK || cus < 8) cus = 256;
   // us per 64-deep K-step on an almost empty chip and on a full one: {1, m ntw, m, ntw}, m = bm / 64
-  static const double kStep[3][2][4] = {{{0., 0.0310, 0.0289, 0.1119}, {0.0113, 0.0104, 0.1250, 0.1172}}, {{0.0923, 0.0475, 0., 0.0152}, {0.1645, 0.0627, 0.0207, 0.0208}},
-                                        {{0.0451, 0.0015, 0.0629, 0.1408}, {0.1990, 0.0565, 0.0129, 0.0542}}};
+  static const double kStep[3][2][4] = {
+      {{0., 0.0310, 0.0289, 0.1119}, {0.0113, 0.0104, 0.1250, 0.1172}},
+      {{0.0421, 0.0428, 0.0357, 0.0463}, {0.0349, 0.0507, 0.0626, 0.0502}},
+      {{0.0813, 0.0177, 0.0187, 0.1367}, {0.0782, 0.0402, 0.0624, 0.0994}}};
+  // us: launch, a round's ramp and what it grows by with the tile, the factor of a grid without a CU to spare, slabs written, a launch that sums them
+  struct Rest { double launch, ramp, area, full, full_area, slab, sum, sum_mb; };
+  static const Rest kRest[2] = {{4.1, 1.2, 0.42, 1.028, 0.0032, 0., 2.65, 0.179}, {2.64, 0.56, 0.471, 1.065, 0., 0.092, 3.38, 0.113}};
+  const bool byte = wd != MI_W_BF16;
+  const Rest& r = kRest[byte];
   const int nks = K / 64;
-  const double mb = (double)T * N * 4e-6;
+  const double mb = (double)T * N * 4e-6, stream = byte ? (double)N * K / 6.67e6 : 0.;   // the weights at 6.7 TB/s
   WidePlan best{0, 4, 1};   // (bm 0: none compared yet; one slice is always allowed, so there is one)
   double best_cost = 0.;
   for (int bm = 64; bm <= 256; bm += 64)
@@ -297,17 +308,24 @@ static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, boo
       const double m = bm / 64, area = m * ntw;
       const auto us = [&](const double (&k)[4]) { return k[0] + k[1] * area + k[2] * m + k[3] * ntw; };
       double lo = us(kStep[wd][0]), hi = us(kStep[wd][1]);
-      if (bm == 192) hi *= 1.04;
-      if (wide_tile_by_32(wd, bm, ntw)) { lo = area == 16 ? 0.893 : 0.95; hi = area == 16 ? 1.456 : 1.2; }   // (the kernel with 32-deep K-steps)
+      if (wide_tile_by_32(wd, bm, ntw)) {   // (the kernel with 32-deep K-steps)
+        lo = area == 16 ? 0.893 : 0.95;
+        hi = area == 16 ? 1.456 : 1.2;
+      } else if (byte) {
+        if (wide_tile_deep(wd, bm, ntw)) { lo *= 0.75; hi *= 0.94; }
+        if (ntw == 3) { lo *= 1.022; hi *= 1.022; }
+      } else if (bm == 192) {
+        hi *= 1.04;
+      }
       const int tiles = ceil_div(T, bm) * ceil_div(N, 64 * ntw);
       for (int ks = 1; ks <= 10; ++ks) {
         const int per = ceil_div(nks, ks);
         if (ks > 1 && (per < 4 || (ks - 1) * per >= nks || (size_t)ks * T * N * sizeof(float) > ws_bytes)) continue;
         const int rounds = ceil_div(ceil_div(tiles, 8) * ks, std::max(1, cus / 8));
-        double body = rounds * (1.2 + 0.42 * area + per * (lo + (hi - lo) * std::min(1.0, (double)tiles * ks / cus)));
-        if (rounds * cus - tiles * ks < 6) body *= 1.028 + 0.0032 * area;   // no CU to spare: the slowest decides
-        double cost = 4.1 + body;
-        if (ks > 1) cost += deferred ? 0.144 * ks * mb : 2.65 + 0.179 * (ks + 1) * mb;
+        double body = rounds * (r.ramp + r.area * area + per * (lo + (hi - lo) * std::min(1.0, (double)tiles * ks / cus)));
+        if (rounds * cus - tiles * ks < 6) body *= r.full + r.full_area * area;   // no CU to spare: the slowest decides
+        double cost = r.launch + (byte ? std::sqrt(body * body + stream * stream) : body);
+        if (ks > 1) cost += r.slab * ks * mb + (deferred ? 0.144 * ks * mb : r.sum + r.sum_mb * (ks + 1) * mb);
         if (best.bm == 0 || cost < best_cost) { best = WidePlan{bm, ntw, ks}; best_cost = cost; }
       }
     }
