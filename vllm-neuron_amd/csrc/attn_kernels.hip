@@ -756,7 +756,14 @@ __device__ __forceinline__ int kv_swz(int key) {   // XOR key of the 16-byte chu
 
 constexpr int kPrefillSlices = 6;   // of the keys, at most
 
-template <int HD, int NW>
+// KH 2: the waves of a head are two, which take a step's two tiles of keys, one each, and put their sums together at the end: a work-group then has one query
+// block at a time (NW = 2 Gp).  KH 1: a wave takes every tile of its block, and a work-group has NW / Gp blocks.
+// A tile is a chain of LDS reads, products and exponentials, 1.6 us for a wave that has its SIMD to itself and 1.3 where two share it.  With 4 heads on a kv head two
+// blocks used to share a work-group: the wave of the light one left the other alone for most of the way, and up to 1000 tokens half of the CUs had none.
+// Alone, us, 32 heads of 128 on 8: 500 tokens 16.0 -> 13.6, 1000 26.8 -> 22.2, 900 behind 900 47.1 -> 33.9, 2031 49.3 -> 45.9 (60 tokens, one step: 7.1 -> 7.6).
+// Without the loads from memory 2031 tokens take 40.0, without the exponentials 44.5; half a step between the two parts (as in the wide GEMM): 53.4.
+// 16 waves for 8 heads do not fit the registers.
+template <int HD, int NW, int KH>
 __device__ __forceinline__ void attn_prefill2_body(
     unsigned char* smem, int bx, int kvh, int bz, int nz, const uint16_t* __restrict__ q, int T, int q_pos0, const uint16_t* __restrict__ kpool,
     const uint16_t* __restrict__ vpool, int bs, int bs_shift, const int32_t* __restrict__ block_table, int nh, int nkv,
@@ -767,17 +774,18 @@ __device__ __forceinline__ void attn_prefill2_body(
   constexpr int KPP = 1024 / ROWB;             // keys per 1 KiB DMA piece (4 / 8)
   constexpr int NP = TK / KPP;                 // pieces per K (or V) tile (16 / 8)
   constexpr int KBYTES = TK * ROWB;            // 16 / 8 KiB
-  constexpr int STAGE = 2 * KBYTES;
-  constexpr int NSTAGE = 3;
-  constexpr int PPW = NP / NW > 0 ? NP / NW : 1;   // K pieces per wave and tile (V the same)
-  static_assert(NP % NW == 0, "pieces must divide over the waves");
-  constexpr int CNT = 2 * PPW;                 // DMA instructions per wave and tile
-  constexpr int KSTEPS = HD / 16, DB = HD / 32;
+  constexpr int VAT = KH * KBYTES;             // a stage: the K of a step's KH tiles, then their V
+  constexpr int STAGE = 2 * VAT;
+  constexpr int NSTAGE = KH == 1 ? 3 : 2;
+  constexpr int PPW = KH * NP / NW;            // K pieces per wave and step (V the same)
+  static_assert(KH * NP % NW == 0, "pieces must divide over the waves");
+  constexpr int CNT = 2 * PPW;                 // DMA instructions per wave and step
+  constexpr int KSTEPS = HD / 16, DB = HD / 32, DW = DB / KH;   // (DW: 32-dim blocks of the output that a wave stores)
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int QB = NW / Gp;
-  const int hl = wave % Gp, slot = wave / Gp;
+  const int QB = KH == 1 ? NW / Gp : 1;
+  const int hl = wave % Gp, slot = KH == 1 ? wave / Gp : 0, part = KH == 1 ? 0 : wave / Gp;
   const int head = kvh * G + min(hl, G - 1);
   const bool head_ok = hl < G;
   const int kv_len = q_pos0 + T;
@@ -836,8 +844,8 @@ __device__ __forceinline__ void attn_prefill2_body(
     int wg_blk = QB == 1 ? (pass == 0 ? nblk - 1 - wg_pair0 : wg_pair0) : nblk - 1 - wg_pair0;   // heaviest block of the work-group
     wg_blk = max(min(wg_blk, nblk - 1), 0);
     const int nt_all = (q_pos0 + min(wg_blk * 32 + 31, T - 1)) / TK + 1;
-    // this slice of them: all, or the bz-th of nz slices of the keys
-    const int t_per = ceil_div(nt_all, nz), t0 = bz * t_per, nt = min(nt_all, t0 + t_per);
+    // steps of this slice of them: all, or the bz-th of nz slices of the keys
+    const int steps = ceil_div(nt_all, KH), s_per = ceil_div(steps, nz), s0 = bz * s_per, s1 = min(steps, s0 + s_per);
 
     // ---- Q fragments (B operand of S^T): Q[q0 + qq][16 ks + 8 h ..] ---------------------------------
     const int qi = min(q0 + qq, T - 1);
@@ -854,50 +862,51 @@ __device__ __forceinline__ void attn_prefill2_body(
       for (int r = 0; r < 16; ++r) o[db][r] = 0.f;
     float m_used = -INFINITY, lsum = 0.f;
 
-    // Block ids are fetched (scalar loads) one tile ahead of the DMAs that use them: the round trip to the scalar cache / L2
+    // Block ids are fetched (scalar loads) one step ahead of the DMAs that use them: the round trip to the scalar cache / L2
     // runs under a tile's arithmetic instead of in front of the global_load_lds it feeds.
     int pf_blk[PPW], pf_off[PPW];
     auto fetch_ids = [&](int t) {
 #pragma unroll
       for (int i = 0; i < PPW; ++i) {
-        const int k0 = min(t * TK + (wave + NW * i) * KPP, last_piece_key);   // rows past the context: the last piece again (masked by position)
+        const int k0 = min(t * KH * TK + (wave + NW * i) * KPP, last_piece_key);   // rows past the context: the last piece again (masked by position)
         int bi;
         if (bs_shift >= 0) { bi = k0 >> bs_shift; pf_off[i] = k0 & (bs - 1); }
         else { bi = k0 / bs; pf_off[i] = k0 - bi * bs; }
         pf_blk[i] = block_table[bi];
       }
     };
-    auto issue = [&](int st) {                  // the tile whose ids fetch_ids loaded last
+    auto issue = [&](int st) {                  // the step whose ids fetch_ids loaded last
       unsigned char* base = smem + st * STAGE;
 #pragma unroll
       for (int i = 0; i < PPW; ++i) {
         const int piece = wave + NW * i;
         const size_t row = ((size_t)pf_blk[i] * nkv + kvh) * bs + pf_off[i];
         glds16(kpool + row * HD + dma_lane_off, base + piece * 1024);
-        glds16(vpool + row * HD + dma_lane_off, base + KBYTES + piece * 1024);
+        glds16(vpool + row * HD + dma_lane_off, base + VAT + piece * 1024);
       }
     };
 
-    int st_issue = 0, st_read = 0;
-    if (t0 < nt) { fetch_ids(t0); issue(0); }
-    if (t0 + 1 < nt) { fetch_ids(t0 + 1); issue(1); }
-    fetch_ids(t0 + 2);
-    st_issue = 2;
+    constexpr int kAhead = NSTAGE - 1;          // steps in flight in front of the one that is read
+    int st_issue = kAhead, st_read = 0;
+    if (s0 < s1) { fetch_ids(s0); issue(0); }
+    if (kAhead > 1 && s0 + 1 < s1) { fetch_ids(s0 + 1); issue(1); }
+    fetch_ids(s0 + kAhead);
     // hipcc waits for a plain load at its first use -- inside the tile loop, as vmcnt(0) on every iteration, which would drain
     // the two tiles in flight each time.  Taking the Q fragments through an empty asm here puts that wait in front of the loop.
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) asm volatile("" : "+v"(qf[ks]));
-    for (int t = t0; t < nt; ++t) {
-      if (t + 1 < nt) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CNT) : "memory");
+    for (int step = s0; step < s1; ++step) {
+      if (kAhead > 1 && step + 1 < s1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CNT) : "memory");
       else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();            // every wave's pieces of tile t are in; everyone is done reading tile t - 1
-      if (t + 2 < nt) {
+      __builtin_amdgcn_s_barrier();            // every wave's pieces of this step are in; everyone is done reading the one before
+      if (step + kAhead < s1) {
         issue(st_issue);
         st_issue = st_issue == NSTAGE - 1 ? 0 : st_issue + 1;
-        fetch_ids(t + 3);
+        fetch_ids(step + kAhead + 1);
       }
-      const unsigned char* Kst = smem + st_read * STAGE;
-      const unsigned char* Vst = Kst + KBYTES;
+      const int t = step * KH + part;
+      const unsigned char* Kst = smem + st_read * STAGE + part * KBYTES;
+      const unsigned char* Vst = Kst + VAT;
       st_read = st_read == NSTAGE - 1 ? 0 : st_read + 1;
       if (t >= nt_wave) continue;                // wave-uniform: the tile lies in this block's future (or the slot is idle)
 
@@ -977,7 +986,7 @@ __device__ __forceinline__ void attn_prefill2_body(
       MI_VREAD(0); MI_VREAD(1); MI_VREAD(2); MI_VREAD(3);
       static_assert(kVAhead == 4, "the prefetch above is written out for 4");
       bf16x8_t pb[4];
-      const float m_exp = nz > 1 && m_used == -INFINITY ? 0.f : m_used;   // (a slice whose keys so far all lie ahead of this query)
+      const float m_exp = (KH > 1 || nz > 1) && m_used == -INFINITY ? 0.f : m_used;   // (a slice or part whose keys so far all lie ahead of this query)
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
         float pv[16];
@@ -1016,47 +1025,81 @@ __device__ __forceinline__ void attn_prefill2_body(
       const f32x2_t sw = swap32_pair(lsum);
       lsum = sw[0] + sw[1];
     }
-    const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
     const bool st_ok = active && q0 + qq < T;
-    if (nz > 1) {   // unnormalised, with its maximum and sum: attn_prefill_combine_kernel puts the slices together
-      const size_t row = ((size_t)bz * T + q0 + qq) * nh + head;
-      if (st_ok && h == 0) *reinterpret_cast<float2*>(ml_part + 2 * row) = make_float2(m_used, lsum);
-      if (st_ok && (m_used != -INFINITY || lsum != 0.f)) {   // (a NaN score moves no maximum: the sum carries it)
+    // the wave's blocks of dims, from d0 on; KH 2: behind the other part's sums for them, which come through the ring's LDS
+    auto finish = [&](auto d0c) {
+      constexpr int d0 = decltype(d0c)::value;
+      if constexpr (KH > 1) {
+        constexpr int other = DB - DW - d0, kPiece = DW * 4096 + 512;         // DW x 4 x [lane] f32x4, [lane] (m, l)
+        unsigned char* mine = smem + wave * kPiece;
+        const unsigned char* theirs = smem + (part == 0 ? wave + Gp : wave - Gp) * kPiece;
+        __syncthreads();                       // everyone is done reading the ring
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
+        for (int i = 0; i < DW * 4; ++i) {
+          const int db = other + i / 4, r = 4 * (i % 4);
+          *reinterpret_cast<f32x4_t*>(mine + i * 1024 + lane * 16) = f32x4_t{o[db][r], o[db][r + 1], o[db][r + 2], o[db][r + 3]};
+        }
+        *reinterpret_cast<f32x2_t*>(mine + DW * 4096 + lane * 8) = f32x2_t{m_used, lsum};
+        __syncthreads();
+        const f32x2_t ml = *reinterpret_cast<const f32x2_t*>(theirs + DW * 4096 + lane * 8);
+        // (a part without a key for this query counts nothing; a NaN score moves no maximum: the sum carries it)
+        const float M = fmaxf(m_used, ml[0]);
+        const float wa = m_used == -INFINITY && lsum == 0.f ? 0.f : fexp2(m_used - M), wb = ml[0] == -INFINITY && ml[1] == 0.f ? 0.f : fexp2(ml[0] - M);
+        lsum = lsum * wa + ml[1] * wb;
+        m_used = M;
 #pragma unroll
-          for (int k = 0; k < 4; ++k)
-            *reinterpret_cast<float4*>(o_part + row * HD + 32 * db + 8 * k + 4 * h) =
-                make_float4(o[db][4 * k], o[db][4 * k + 1], o[db][4 * k + 2], o[db][4 * k + 3]);
+        for (int i = 0; i < DW * 4; ++i) {
+          const f32x4_t v = *reinterpret_cast<const f32x4_t*>(theirs + i * 1024 + lane * 16);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) o[d0 + i / 4][4 * (i % 4) + k] = o[d0 + i / 4][4 * (i % 4) + k] * wa + v[k] * wb;
+        }
       }
-      __syncthreads();
-      continue;
-    }
-    uint16_t* orow = out + ((size_t)(q0 + qq) * nh + head) * HD;
+      if (nz > 1) {   // unnormalised, with its maximum and sum: attn_prefill_combine_kernel puts the slices together
+        const size_t row = ((size_t)bz * T + q0 + qq) * nh + head;
+        if (st_ok && h == 0 && part == 0) *reinterpret_cast<float2*>(ml_part + 2 * row) = make_float2(m_used, lsum);
+        if (st_ok && (m_used != -INFINITY || lsum != 0.f)) {
 #pragma unroll
-    for (int db = 0; db < DB; ++db)
+          for (int db = d0; db < d0 + DW; ++db)
 #pragma unroll
-      for (int k2 = 0; k2 < 4; k2 += 2) {      // dim groups k2, k2 + 1: dims 32 db + 8 k + 4 h + (0..3)
-        uint32_t a0 = pack_bf16x2(o[db][4 * k2 + 0] * inv, o[db][4 * k2 + 1] * inv);
-        uint32_t a1 = pack_bf16x2(o[db][4 * k2 + 2] * inv, o[db][4 * k2 + 3] * inv);
-        uint32_t b0 = pack_bf16x2(o[db][4 * k2 + 4] * inv, o[db][4 * k2 + 5] * inv);
-        uint32_t b1 = pack_bf16x2(o[db][4 * k2 + 6] * inv, o[db][4 * k2 + 7] * inv);
-        const auto x = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);
-        const auto y = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
-        // lower half: [own group k2 | upper's group k2] = dims 8 k2 .. 8 k2 + 7; upper half: [lower's k2 + 1 | own k2 + 1]
-        const u32x4_t v = {x[0], y[0], x[1], y[1]};
-        if (st_ok) *reinterpret_cast<u32x4_t*>(orow + 32 * db + 8 * (k2 + h)) = v;
+            for (int k = 0; k < 4; ++k)
+              *reinterpret_cast<float4*>(o_part + row * HD + 32 * db + 8 * k + 4 * h) =
+                  make_float4(o[db][4 * k], o[db][4 * k + 1], o[db][4 * k + 2], o[db][4 * k + 3]);
+        }
+        return;
       }
+      // (KH 2: a sum of 0 is one behind scores that are all -inf, whose row is 0 x inf, the NaN it is where one wave takes all tiles)
+      const float inv = KH > 1 || lsum > 0.f ? 1.f / lsum : 0.f;
+      uint16_t* orow = out + ((size_t)(q0 + qq) * nh + head) * HD;
+#pragma unroll
+      for (int db = d0; db < d0 + DW; ++db)
+#pragma unroll
+        for (int k2 = 0; k2 < 4; k2 += 2) {      // dim groups k2, k2 + 1: dims 32 db + 8 k + 4 h + (0..3)
+          uint32_t a0 = pack_bf16x2(o[db][4 * k2 + 0] * inv, o[db][4 * k2 + 1] * inv);
+          uint32_t a1 = pack_bf16x2(o[db][4 * k2 + 2] * inv, o[db][4 * k2 + 3] * inv);
+          uint32_t b0 = pack_bf16x2(o[db][4 * k2 + 4] * inv, o[db][4 * k2 + 5] * inv);
+          uint32_t b1 = pack_bf16x2(o[db][4 * k2 + 6] * inv, o[db][4 * k2 + 7] * inv);
+          const auto x = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);
+          const auto y = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
+          // lower half: [own group k2 | upper's group k2] = dims 8 k2 .. 8 k2 + 7; upper half: [lower's k2 + 1 | own k2 + 1]
+          const u32x4_t v = {x[0], y[0], x[1], y[1]};
+          if (st_ok) *reinterpret_cast<u32x4_t*>(orow + 32 * db + 8 * (k2 + h)) = v;
+        }
+    };
+    if (KH == 1 || part == 0) finish(std::integral_constant<int, 0>());
+    else finish(std::integral_constant<int, DB - DW>());
     __syncthreads();   // the ring is reused by the next pass
   }
 }
-template <int HD, int NW>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill2_kernel(
+template <int HD, int NW, int KH>
+constexpr int attn_prefill2_lds() { return std::max((KH == 1 ? 3 : 2) * KH * 2 * 64 * 2 * HD, KH == 1 ? 0 : NW * (HD / 64 * 4096 + 512)); }
+// The kv heads are the fastest of the grid: with 8 (4) of them an XCD's work-groups read the keys of one, and the heavy blocks of all start first.
+template <int HD, int NW, int KH>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4, NW / 4))) void attn_prefill2_kernel(
     const uint16_t* __restrict__ q, int T, int q_pos0, const uint16_t* __restrict__ kpool,
     const uint16_t* __restrict__ vpool, int bs, int bs_shift, const int32_t* __restrict__ block_table, int nh, int nkv,
     int G, int Gp, int nblk, int paired, float* __restrict__ o_part, float* __restrict__ ml_part, uint16_t* __restrict__ out, float scale_log2e) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  attn_prefill2_body<HD, NW>(smem, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk, paired, o_part,
+  attn_prefill2_body<HD, NW, KH>(smem, blockIdx.y, blockIdx.x, blockIdx.z, gridDim.z, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk, paired, o_part,
                              ml_part, out, scale_log2e);
 }
 
@@ -1064,7 +1107,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 // beside 3 contexts of up to 900 (8B model).  Work-groups x from `nd` on are the prompt's, gx of every slice of the keys; those before them one
 // (split, sequence) each of the others.
 struct DecodeSide { const uint16_t* q; const int32_t* block_table; const int32_t* ctx_lens; int MB, NS, nd, num_blocks; float *o_part, *ml_part; uint16_t* out; };
-template <int HD, bool FINAL>
+template <int HD, int KH, bool FINAL>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_mixed_kernel(
     const uint16_t* __restrict__ q, int T, int q_pos0, const uint16_t* __restrict__ kpool,
     const uint16_t* __restrict__ vpool, int bs, int bs_shift, const int32_t* __restrict__ block_table, int nh, int nkv,
@@ -1072,7 +1115,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   if ((int)blockIdx.x >= d.nd) {
     const int x = (int)blockIdx.x - d.nd;
-    attn_prefill2_body<HD, 8>(smem, x % gx, blockIdx.y, x / gx, ns, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk,
+    attn_prefill2_body<HD, 8, KH>(smem, x % gx, blockIdx.y, x / gx, ns, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk,
                               paired, o_part, ml_part, out, scale_log2e);
   } else {
     attn_decode_body<HD, 8, FINAL>(smem, (int)blockIdx.x % d.NS, blockIdx.y, (int)blockIdx.x / d.NS, d.q, kpool, vpool, bs, d.block_table, d.MB, d.ctx_lens, nh, nkv, G, d.NS,
@@ -1116,27 +1159,29 @@ static bool attn_prefill_v1() {   // MI355X_ATTN_PREFILL_V1=1: the first-generat
 }
 
 static int prefill_heads(int G) { return G <= 1 ? 1 : (G <= 2 ? 2 : (G <= 4 ? 4 : 8)); }
-struct PrefillPlan { int Gp, nblk, bs_shift, paired, gx, ns; float *o_part = nullptr, *ml_part = nullptr; };
+struct PrefillPlan { int Gp, kh, nblk, bs_shift, paired, gx, ns; float *o_part = nullptr, *ml_part = nullptr; };
 static PrefillPlan prefill_plan(int T, int q_pos0, int block_size, int nh, int nkv, int hd, float* ws, size_t ws_bytes, int num_cu) {
-  // second generation: 8 waves = (8 / Gp) query blocks x Gp heads; blocks in complementary pairs
+  // second generation: 8 waves = (8 / Gp) query blocks x Gp heads, blocks in complementary pairs; or a block of 4 heads, two waves each
   PrefillPlan p;
   p.Gp = prefill_heads(nh / nkv);
-  const int nblk = ceil_div(T, 32), npair = (nblk + 1) / 2, qb = 8 / p.Gp;
+  p.kh = p.Gp == 4 ? 2 : 1;
+  const int nblk = ceil_div(T, 32), npair = (nblk + 1) / 2, qb = p.kh == 2 ? 1 : 8 / p.Gp;
   int bs_shift = -1;
   for (int sh = 4; sh < 20; ++sh) if ((1 << sh) == block_size) bs_shift = sh;
   // One block per work-group (5 .. 8 heads on a kv head): pairs only where single blocks would not all run at once.
   const int paired = qb > 1 || nblk * nkv > num_cu;
   const int gx = paired ? ceil_div(npair, qb >= 2 ? qb / 2 : 1) : nblk;
-  // A short prompt, or the rest of one behind cached keys, leaves most of the chip idle while each work-group walks its tiles, 1.75 us each:
+  // A short prompt, or the rest of one behind cached keys, leaves most of the chip idle while each work-group walks its tiles, 1.75 us each (2.4 us two of them):
   // slices of the keys then, at least two tiles each, the cheapest by that and the second launch, which moves every slice's O out and in.
   // 188 tokens behind 512 cached ones, 28 heads on 4: 40.8 us in 12 work-groups of two passes, 16.7 + 4.8 now.
   int ns = 1;
-  const int tiles = ceil_div(q_pos0 + T, 64);
-  double best = 1.75 * tiles * ceil_div(gx * nkv, num_cu);
+  const int steps = ceil_div(q_pos0 + T, 64 * p.kh);
+  const double per_step = p.kh == 2 ? 2.4 : 1.75;
+  double best = per_step * steps * ceil_div(gx * nkv, num_cu);
   for (int z = 2; ws && z <= kPrefillSlices; ++z) {
     const size_t part = (size_t)z * T * nh;
-    if (ceil_div(tiles, z) < 2 || part * (hd + 2) * sizeof(float) > ws_bytes) break;
-    const double cost = 1.75 * ceil_div(tiles, z) * ceil_div(gx * nkv * z, num_cu) + 4.5 + (double)part * hd * 8.0 / 4e6;
+    if (ceil_div(steps, z) * p.kh < 2 || part * (hd + 2) * sizeof(float) > ws_bytes) break;
+    const double cost = per_step * ceil_div(steps, z) * ceil_div(gx * nkv * z, num_cu) + 4.5 + (double)part * hd * 8.0 / 4e6;
     if (cost < best) { best = cost; ns = z; }
   }
   p.nblk = nblk; p.bs_shift = bs_shift; p.paired = paired; p.gx = gx; p.ns = ns;
@@ -1164,13 +1209,14 @@ int launch_attn_prefill(const uint16_t* q, int T, int q_pos0, const uint16_t* kp
     int num_cu = 0;
     MI_TRY_A(device_num_cu(&num_cu));
     const PrefillPlan p = prefill_plan(T, q_pos0, block_size, nh, nkv, hd, ws, ws_bytes, num_cu);
-#define MI_P2(HD_) do { \
-      constexpr int lds = 3 * 2 * 64 * 2 * HD_; \
-      MI_TRY_A(ensure_dynamic_lds(reinterpret_cast<const void*>(attn_prefill2_kernel<HD_, 8>), lds)); \
-      hipLaunchKernelGGL((attn_prefill2_kernel<HD_, 8>), dim3(p.gx, nkv, p.ns), dim3(512), lds, s, q, T, q_pos0, kpool, vpool, block_size, p.bs_shift, \
+#define MI_P2(HD_, NW_, KH_) do { \
+      constexpr int lds = attn_prefill2_lds<HD_, NW_, KH_>(); \
+      MI_TRY_A(ensure_dynamic_lds(reinterpret_cast<const void*>(attn_prefill2_kernel<HD_, NW_, KH_>), lds)); \
+      hipLaunchKernelGGL((attn_prefill2_kernel<HD_, NW_, KH_>), dim3(nkv, p.gx, p.ns), dim3(NW_ * 64), lds, s, q, T, q_pos0, kpool, vpool, block_size, p.bs_shift, \
                          block_table, nh, nkv, G, p.Gp, p.nblk, p.paired, p.o_part, p.ml_part, out, scale_log2e); \
     } while (0)
-    if (hd == 128) MI_P2(128); else MI_P2(64);
+    if (p.kh == 1) { if (hd == 128) MI_P2(128, 8, 1); else MI_P2(64, 8, 1); }
+    else { if (hd == 128) MI_P2(128, 8, 2); else MI_P2(64, 8, 2); }
 #undef MI_P2
     launch_prefill_combine(p, T, nh, hd, out, s);
     MI_HIP(hipGetLastError());
@@ -1200,8 +1246,9 @@ static int launch_mixed_t(const AttnMixed& m, const PrefillPlan& p, int T, int q
   float* o_part = ml_part + (size_t)m.B * nh * kAttnMaxSplits * 2;
   const int NS = mixed_splits(m, nkv, HD);
   const DecodeSide d{m.q, m.block_table, m.ctx_lens, m.MB, NS, NS * m.B, m.num_blocks, o_part, ml_part, m.out};
-  constexpr int lds = std::max<int>(3 * 2 * 64 * 2 * HD, (int)attn_decode_lds<HD, 8>());
-  const auto fn = NS == 1 ? attn_mixed_kernel<HD, true> : attn_mixed_kernel<HD, false>;
+  const int lds = std::max<int>(p.kh == 2 ? attn_prefill2_lds<HD, 8, 2>() : attn_prefill2_lds<HD, 8, 1>(), (int)attn_decode_lds<HD, 8>());
+  const auto fn = p.kh == 2 ? (NS == 1 ? attn_mixed_kernel<HD, 2, true> : attn_mixed_kernel<HD, 2, false>)
+                            : (NS == 1 ? attn_mixed_kernel<HD, 1, true> : attn_mixed_kernel<HD, 1, false>);
   MI_TRY_A(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds));
   hipLaunchKernelGGL(fn, dim3(d.nd + p.gx * p.ns, nkv), dim3(512), lds, s, q, T, q_pos0, kpool, vpool, bs, p.bs_shift, bt, nh, nkv, nh / nkv, p.Gp, p.nblk, p.paired,
                      p.gx, p.ns, p.o_part, p.ml_part, out, scale_log2e, d);
