@@ -117,6 +117,26 @@ def test_unit_norm_and_kv_scatter(lib, H, G, dk, dv, unit, f32):
             written[s // bs, s % bs] = True
     assert (kp.permute(0, 2, 1, 3)[~written] == 7.0).all() and (vp.permute(0, 2, 1, 3)[~written] == 7.0).all()
 
+@pytest.mark.parametrize("T", [511, 514, 517])         # one token a thread, then four of them with one, two and three left over
+def test_scatter_of_many_tokens(lib, T):
+    torch.manual_seed(4)
+    H, G, dk, dv, bs = 3, 1, 52, 36, 16
+    ldq, nb = pad16((H + G) * dk + G * dv), 1 + -(-T // bs)
+    qkv, slots = torch.randn(T, ldq) * 3, (bs + torch.randperm(T)).int()
+    slots[5] = -1
+    q = torch.full((T, H, pad16(dk)), 7.0, device="cuda")
+    kp, vp = (torch.full((nb, G, bs, pad16(d)), 7.0, device="cuda") for d in (dk, dv))
+    a, b = dev(qkv), dev(slots)
+    lib.check(lib.load_library().mi_op_qkv_scatter(a.data_ptr(), ldq, T, spec_of(lib, H, G, dk, dv, 8, 1.0), 1e-3, b.data_ptr(), bs, q.data_ptr(), kp.data_ptr(),
+                                                   vp.data_ptr(), 1, None))
+    torch.cuda.synchronize()
+    heads = V.unit_rms(qkv[:, :(H + G) * dk].reshape(T, H + G, dk).double(), 1e-3)
+    v, live = qkv[:, (H + G) * dk:(H + G) * dk + dv].double(), slots >= 0
+    at = slots[live].long()
+    for got, ref, d in ((q.cpu(), heads[:, :H], dk), (kp.cpu()[at // bs, :, at % bs], heads[live, H:], dk), (vp.cpu()[at // bs, :, at % bs], v[live][:, None], dv)):
+        assert (got[..., d:] == 0).all() and ((got[..., :d].double() - ref).abs() <= 1e-5 * (1 + ref.abs())).all()
+    assert (kp[0] == 7).all() and (vp[0] == 7).all()
+
 
 class Paged:
     """One random sequence per request, its K / V scattered over shuffled pool blocks, and a ragged set of queries."""

@@ -564,6 +564,59 @@ __global__ __launch_bounds__(256) void qkv_scatter_kernel(const float* __restric
   }
 }
 
+// The same where a head's row is one quad a lane (LPH 16: heads of up to 64, 32: of up to 128): LPH lanes take a head of ROWS tokens, whose requests leave
+// together.  Bound by bytes: 4000 tokens of 32 + 8 + 8 heads of 64 move 74 MB, 27.1 us -> 16.5 (777 tokens 8.0 -> 6.9)
+// (a work-group per token, 32 lanes a head whose upper half was idle, and each value read again behind the norm).
+template <typename T, int LPH, int ROWS>
+__global__ __launch_bounds__(256) void qkv_scatter_quads_kernel(const float* __restrict__ qkv, int ldq, int rows, HeadGeom g, HeadRule rule, float eps,
+                                                                const int32_t* __restrict__ slots, int bs, T* __restrict__ q,
+                                                                T* __restrict__ kpool, T* __restrict__ vpool) {
+  const int t0 = blockIdx.x * ROWS, head = blockIdx.y * (256 / LPH) + threadIdx.x / LPH, d = threadIdx.x % LPH * 4;
+  if (head >= g.H + (rule.keys_as_values ? 1 : 2) * g.G) return;     // (whole group of lanes: the shuffles below stay inside it)
+  const bool is_q = head < g.H, is_v = head >= g.H + g.G;
+  const int kvh = is_v ? head - g.H - g.G : head - g.H;
+  const int d_n = is_v ? g.dv : g.dk, d_p = is_v ? g.dvp : g.dkp;
+  const float* src = qkv + (is_v ? (size_t)(g.H + g.G) * g.dk + (size_t)kvh * g.dv : (size_t)head * g.dk);
+  const float* w = is_v ? nullptr : is_q ? rule.q_norm : rule.k_norm;
+  const bool vec = (d_n & 3) == 0 && (((is_v ? (g.H + g.G) * g.dk : 0)) & 3) == 0;
+  auto get = [&](const float* p) -> float4 {
+    if (vec) return d < d_n ? *reinterpret_cast<const float4*>(p + d) : make_float4(0.f, 0.f, 0.f, 0.f);
+    return make_float4(d < d_n ? p[d] : 0.f, d + 1 < d_n ? p[d + 1] : 0.f, d + 2 < d_n ? p[d + 2] : 0.f, d + 3 < d_n ? p[d + 3] : 0.f);
+  };
+  float4 v[ROWS];
+  int slot[ROWS];
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    const int t = min(t0 + i, rows - 1);
+    v[i] = get(src + (size_t)t * ldq);
+    slot[i] = slots[t];
+  }
+  const float4 b = rule.bias && !is_v ? get(rule.bias + (size_t)head * g.dk) : make_float4(0.f, 0.f, 0.f, 0.f);
+  const float4 k = w ? get(w) : make_float4(1.f, 1.f, 1.f, 1.f);
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    const int t = t0 + i;
+    if (t >= rows || (!is_q && slot[i] < 0)) continue;               // (alike in all lanes of the group)
+    if (rule.bias && !is_v) v[i] = make_float4(v[i].x + b.x, v[i].y + b.y, v[i].z + b.z, v[i].w + b.w);
+    float f = 1.f;
+    if (!is_v && rule.unit_norm) {
+      float ss = (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
+#pragma unroll
+      for (int m = LPH / 2; m >= 1; m >>= 1) ss += __shfl_xor(ss, m);
+      f = 1.0f / sqrtf(ss / (float)d_n + eps);
+    }
+    if (d >= d_p) continue;
+    if (is_q) {
+      put4(q + ((size_t)t * g.H + head) * g.dkp + d, v[i].x * f * k.x, v[i].y * f * k.y, v[i].z * f * k.z, v[i].w * f * k.w);
+      continue;
+    }
+    const int blk = slot[i] / bs, off = slot[i] - blk * bs;
+    const size_t r = (((size_t)blk * g.G + kvh) * bs + off) * d_p + d;
+    put4((is_v ? vpool : kpool) + r, v[i].x * f * k.x, v[i].y * f * k.y, v[i].z * f * k.z, v[i].w * f * k.w);
+    if (rule.keys_as_values) put4(vpool + r, v[i].x, v[i].y, v[i].z, v[i].w);
+  }
+}
+
 // 64 x 64 tile, 4 x 4 outputs per thread, fp32 FMAs: the 32-bit mode is for checking, not for speed
 template <int EPI>
 __global__ __launch_bounds__(256) void linear_f32_kernel(const float* __restrict__ w, int N, int K, const float* __restrict__ x, int ldx,
@@ -811,7 +864,22 @@ int launch_qkv_scatter(const float* qkv, int ldq, int T, const HeadGeom& g, cons
   MI_CHECK(rule.unit_norm || (!rule.q_norm && !rule.k_norm), "qkv scatter: norm weights without a norm");
   MI_CHECK(ldq % 4 == 0 && ldq >= (g.H + g.G) * g.dk + (rule.keys_as_values ? 0 : g.G * g.dv) && g.dkp % 16 == 0 && g.dvp % 16 == 0 && g.dkp >= g.dk && g.dvp >= g.dv,
            "qkv scatter: geometry");
-  const dim3 grid(T, ceil_div(g.H + 2 * g.G, 8));
+  const int widest = std::max(g.dkp, g.dvp), heads = g.H + 2 * g.G;
+  // four tokens a thread where that leaves work-groups for the chip: a step of 3 rows takes 1 us more with them than with one
+#define MI_QUADS_R(T_, LPH_, ROWS_)                                                                                                                        \
+  hipLaunchKernelGGL((qkv_scatter_quads_kernel<T_, LPH_, ROWS_>), dim3(ceil_div(T, ROWS_), ceil_div(heads, 256 / LPH_)), dim3(256), 0, s, qkv, ldq, T, g, rule, \
+                     eps, slots, block_size, (T_*)q, (T_*)kpool, (T_*)vpool)
+#define MI_QUADS(LPH_) do {                                                                                          \
+    if (f32) { if (T >= 512) MI_QUADS_R(float, LPH_, 4); else MI_QUADS_R(float, LPH_, 1); }                          \
+    else { if (T >= 512) MI_QUADS_R(uint16_t, LPH_, 4); else MI_QUADS_R(uint16_t, LPH_, 1); }                        \
+    MI_HIP(hipGetLastError());                                                                                       \
+    return MI_OK;                                                                                                    \
+  } while (0)
+  if (T >= 1 && widest <= 64) MI_QUADS(16);
+  if (T >= 1 && widest <= 128) MI_QUADS(32);
+#undef MI_QUADS_R
+#undef MI_QUADS
+  const dim3 grid(T, ceil_div(heads, 8));
   if (f32) hipLaunchKernelGGL((qkv_scatter_kernel<float>), grid, dim3(256), 0, s, qkv, ldq, g, rule, eps, slots, block_size, (float*)q, (float*)kpool, (float*)vpool);
   else hipLaunchKernelGGL((qkv_scatter_kernel<uint16_t>), grid, dim3(256), 0, s, qkv, ldq, g, rule, eps, slots, block_size, (uint16_t*)q, (uint16_t*)kpool, (uint16_t*)vpool);
   MI_HIP(hipGetLastError());
