@@ -112,8 +112,12 @@ constexpr size_t prefill_lds() { return (size_t)64 * (DK + kPitch + DV + kPitch)
 
 // KS = 2: a second set of four waves takes every other key tile of the same queries (short grids, whose heaviest work-group is what
 // the launch waits for); the two sets' sums meet in LDS at the end.
+// Heads of 64: three or four waves a SIMD where the registers allow it, not two.  A tile is a chain of two barriers, LDS reads, products and exponentials, which two waves do not
+// fill.  us, 32 heads on 8, window 1024: 4000 tokens 68.2 -> 62.5, 1500 35.2 -> 28.8, chunks with a table 777 tokens 23.4 -> 22.5; four waves forced: 76.5.
+// Two column groups with tables (3000 tokens) 56.2 -> 57.6: left at two.
+constexpr bool more_waves(int dk, int dv, int ncg, bool ext) { return dk <= 64 && dv <= 64 && !(ext && ncg == 2); }
 template <int DK, int DV, int NCG, int KS2, bool FIXED, bool EXT>
-__global__ __launch_bounds__(256 * KS2) __attribute__((amdgpu_waves_per_eu(DK > 192 || DV > 128 ? KS2 : 2, DK > 192 || DV > 128 ? KS2 : 2))) void attn_window_prefill_kernel(AttnSpec a, const uint16_t* __restrict__ q, const uint16_t* __restrict__ kpool,
+__global__ __launch_bounds__(256 * KS2) __attribute__((amdgpu_waves_per_eu(DK > 192 || DV > 128 ? KS2 : 2, DK > 192 || DV > 128 ? KS2 : more_waves(DK, DV, NCG, EXT) ? 4 : 2))) void attn_window_prefill_kernel(AttnSpec a, const uint16_t* __restrict__ q, const uint16_t* __restrict__ kpool,
                                                                   const uint16_t* __restrict__ vpool, int bs, const int32_t* __restrict__ bt,
                                                                   int MB, const AttnSeg* __restrict__ segs, int nseg,
                                                                   uint16_t* __restrict__ out, int ldo, float s_max, int fold, int min_rows, int bs_shift, OutGate gt) {
