@@ -485,6 +485,19 @@ def test_state_space_duality(lib, H, P, N, G, f32):
         assert (s.state[1] == 1e4).all()
 
 
+# states in aligned pieces that fill no whole matrix operand (32), two and four tiles of them a wave, one and several groups: bf16 rows, whose fp32 factors go in parts
+@pytest.mark.parametrize("strong", [False, True])
+@pytest.mark.parametrize("H,P,N,G", [(4, 16, 104, 2), (8, 16, 72, 1), (2, 32, 200, 1), (8, 16, 136, 4)])
+def test_state_space_duality_of_bf16_rows(lib, H, P, N, G, strong):
+    for plan in PLANS:
+        s = Ssd(lib, H, P, N, G, H + P + N, slots=[3, 0, 2], strong=strong)
+        for live in plan:
+            close(*s.step(live, 0), 5e-5)
+        for i in range(3):
+            if s.st.at[i] == LENGTHS[i]:
+                s.check_state(i)
+
+
 @pytest.mark.parametrize("strong", [False, True])
 def test_state_space_duality_token_by_token_and_slots_used_again(lib, strong):
     s = Ssd(lib, 4, 24, 40, 2, 5, lengths=[70, 40, 200], slots=[0, 1, 0], strong=strong)

@@ -462,7 +462,31 @@ __device__ __forceinline__ void stage_rows(float* dst, int pitch, const T* src, 
   }
 }
 
-// Of every chunk: C B^T, a work-group per group (blockIdx.y < G), and the heads' steps, a wave per head
+// An fp32 number is the sum of three bf16 numbers (8 of its 24 bits each, cut off, so the differences are exact).  With a factor that is bf16 by itself the products of
+// the three are exact too, and only their sums round, in fp32: what the fp32 MFMAs do in 32 cycles per four terms, these do in 16 per 32 terms.
+typedef __attribute__((ext_vector_type(4))) short s16x4_t;
+struct Parts { u32x4_t hi, mid, lo; };
+__device__ __forceinline__ Parts in_parts(const float (&v)[8]) {
+  Parts p;
+  auto cut = [](float x) { return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x) & 0xffff0000u); };
+  auto upper = [](float a, float b) { return __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, b), __builtin_bit_cast(unsigned, a), 0x07060302u); };
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float a = v[2 * k], b = v[2 * k + 1], a1 = a - cut(a), b1 = b - cut(b);
+    p.hi[k] = upper(a, b);
+    p.mid[k] = upper(a1, b1);
+    p.lo[k] = upper(a1 - cut(a1), b1 - cut(b1));
+  }
+  return p;
+}
+__device__ __forceinline__ f32x4_t mfma32(u32x4_t a, u32x4_t b, f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4_t mfma32(u32x4_t a, const Parts& b, f32x4_t c) { return mfma32(a, b.hi, mfma32(a, b.mid, mfma32(a, b.lo, c))); }
+__device__ __forceinline__ f32x4_t mfma32(const Parts& a, u32x4_t b, f32x4_t c) { return mfma32(a.hi, b, mfma32(a.mid, b, mfma32(a.lo, b, c))); }
+
+// Of every chunk: C B^T, a work-group per group (blockIdx.y < G), and the heads' steps, a wave per head.  Rows of bf16 in whole aligned pieces of 8 are MFMA operands as they
+// lie in memory, and their products exact: through LDS, in fp32, a chunk of 128 states took as long as all the rest of the launch.  777 tokens of 64 heads: 11.8 us -> 5.2.
 template <typename T>
 __global__ __launch_bounds__(256) void ssd_chunk_kernel(SsdGeom g, SsdIn in, const AttnSeg* __restrict__ segs, int nseg, int c0, float* __restrict__ base) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
@@ -491,11 +515,32 @@ __global__ __launch_bounds__(256) void ssd_chunk_kernel(SsdGeom g, SsdIn in, con
   }
   const T* rows = reinterpret_cast<const T*>(in.xbc) + (size_t)(at.sg.row0 + at.t0) * in.ldx;
   const int grp = blockIdx.y, pitch = tall_pitch(g.Np);
+  float* out = rec.cb + ((size_t)blockIdx.x * g.G + grp) * kQ * kQ;
+  if constexpr (sizeof(T) == 2) {
+    if (((g.N | inner | in.ldx) & 7) == 0 && (reinterpret_cast<uintptr_t>(in.xbc) & 15) == 0) {
+      const T *B = rows + inner + grp * g.N, *C = B + g.G * g.N;
+      f32x4_t cb[4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+      auto eight = [&](const T* p, int t, int k) {       // (zeros behind the last token and the last state)
+        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(p + (size_t)min(t, at.n - 1) * in.ldx + min(k, g.N - 8));
+        return t < at.n && k < g.N ? v : u32x4_t{0, 0, 0, 0};
+      };
+#pragma unroll 4
+      for (int k = 8 * g4; k < g.Np + 8 * g4; k += 32) {
+        const u32x4_t a = eight(C, 16 * wave + c, k);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) cb[j] = mfma32(a, eight(B, 16 * j + c, k), cb[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[(16 * wave + 4 * g4 + r) * kQ + 16 * j + c] = cb[j][r];
+      return;
+    }
+  }
   float *Bs = sm, *Cs = sm + kQ * pitch;
   stage_rows(Bs, pitch, rows + inner + grp * g.N, in.ldx, at.n, g.N, g.Np);
   stage_rows(Cs, pitch, rows + inner + (g.G + grp) * g.N, in.ldx, at.n, g.N, g.Np);
   __syncthreads();
-  float* out = rec.cb + ((size_t)blockIdx.x * g.G + grp) * kQ * kQ;
   f32x4_t acc[4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
   for (int s = 0; s < g.Np / 4; ++s) {
     const float a = Cs[(16 * wave + c) * pitch + 4 * s + g4];
@@ -551,6 +596,11 @@ constexpr size_t scan_lds() { return 2 * 16 * 64 * 16 + 2 * sizeof(Steps) + 2 * 
 // n = 16 NT wave + NT rho + t: a lane's A operands of all tiles lie side by side, in C (registers, four rows of the tiles at a time) as in
 // B (through LDS, the wave's own columns).  The waves' shares of a chunk's outputs meet in LDS, one barrier per chunk; what the next
 // chunk needs is in flight meanwhile.  VEC: whole 16-byte pieces of rows, aligned.
+// In bf16, B, C and x are bf16 numbers; from two tiles a wave on the products take their fp32 factor (the state, weighted x, decayed C B^T) in parts: 777 tokens of 64 heads of
+// 64, 128 states, 46.8 us -> 38.0, and 35.5 with requests two chunks ahead; 3000 tokens 125 -> 99; error against 64 bits 1.30e-7 -> 1.08e-7, of the state 1.09e-7 -> 0.95e-7
+// (4.0e-8 -> 4.3e-8 where steps wipe the state within a chunk).  The state and the rest on waves of their own, two a SIMD: 40.3 (branches in front of what is in flight).
+// k-slot (g4, j) of a product over states is element 8 s + j of the lane's C; of one over tokens, token 32 s + (j < 4 ? 4 g4 + j : 16 + 4 g4 + j - 4), which transposed
+// reads of B give, whose tiles lie side by side in LDS for them.
 template <typename T, int NT, bool VEC>
 __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, const AttnSeg* __restrict__ segs, int c0, int nchunks, int nvt, float* __restrict__ base,
                                                        float* __restrict__ y, int ldy) {
@@ -559,6 +609,7 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, cons
   Steps* st = reinterpret_cast<Steps*>(dsm + 2 * 16 * 64 * 16);
   float* xs = reinterpret_cast<float*>(st + 2);
   constexpr int BP = b_pitch<T, NT>(), W = 16 / (int)sizeof(T), LPR = 16 * NT / W, RPL = 64 / LPR;    // elements per 16 bytes; lanes per row, rows per load of B
+  constexpr bool kParts = sizeof(T) == 2 && (NT == 2 || NT == 4);
   int id = blockIdx.x, h, vt;
   if (g.H % 8 == 0) {        // the column blocks of a head on one XCD
     const int k = id >> 3;
@@ -642,16 +693,28 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, cons
 #pragma unroll
         for (int e = 0; e < 4; ++e) v.v[0][e] = bn < g.N ? v.v[0][e] : 0u;
       }
-      v.store(Bs + (RPL * i + lane / LPR) * BP + (lane % LPR) * W);
+      T* row = Bs + (RPL * i + lane / LPR) * BP;
+      if constexpr (kParts && NT == 2) {
+        const unsigned a = v.v[0][0], b = v.v[0][1], cc = v.v[0][2], d2 = v.v[0][3];
+        *reinterpret_cast<uint2*>(row + 4 * (lane % LPR)) = make_uint2(__builtin_amdgcn_perm(b, a, 0x05040100u), __builtin_amdgcn_perm(d2, cc, 0x05040100u));
+        *reinterpret_cast<uint2*>(row + 16 + 4 * (lane % LPR)) = make_uint2(__builtin_amdgcn_perm(b, a, 0x07060302u), __builtin_amdgcn_perm(d2, cc, 0x07060302u));
+      } else if constexpr (kParts) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const unsigned a = v.v[0][t / 2], b = v.v[0][2 + t / 2];
+          *reinterpret_cast<unsigned*>(row + 16 * t + 2 * (lane % LPR)) = __builtin_amdgcn_perm(b, a, t & 1 ? 0x07060302u : 0x05040100u);
+        }
+      } else {
+        v.store(row + (lane % LPR) * W);
+      }
     }
   };
   const float skip = in.d[h];
-  auto step = [&](int k, Kept& f, Kept& next) {
-    const int b = (k - k0) & 1, n = min(kQ, sg.n - k * kQ);
+  // Two chunks ahead: with one, a chunk waits for memory longer than it computes.  `passed` goes to LDS at the end of the chunk before its own, `f` is used up in its own.
+  auto step = [&](int k, Kept& f, Passed& passed, Passed& d) {
+    const int b = (k - k0) & 1, n = min(kQ, sg.n - k * kQ), ahead = min(k + 2, k1 - 1);     // (behind the last chunk: that one again)
     const Steps& q = st[b];
-    Passed d;                  // (behind the last chunk: that one again)
-    load_passed(min(k + 1, k1 - 1), d);
-    load_kept(min(k + 1, k1 - 1), next);
+    load_passed(ahead, passed);
     __builtin_amdgcn_sched_barrier(0);
     float x[16];               // tokens 16 i + 4 g4 + r (past the last one: its weight and step are zero)
 #pragma unroll
@@ -660,41 +723,99 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, cons
     f32x4_t o[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if constexpr (kParts) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+      for (int s = 0; s < NT / 2; ++s) {
+        float v[8];
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
+        for (int j = 0; j < 8; ++j) v[j] = S[(8 * s + j) % NT][(8 * s + j) / NT];
+        const Parts sp = in_parts(v);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.c[i].at(NT * r + t), S[t][r], o[i], 0, 0, 0);
+        for (int i = 0; i < 4; ++i) o[i] = mfma32(f.c[i].v[s], sp, o[i]);
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.c[i].at(NT * r + t), S[t][r], o[i], 0, 0, 0);
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) ps[b][wave][i][lane] = o[i];
     // the state behind the chunk
     const float end = q.e[kQ - 1];
 #pragma unroll
     for (int t = 0; t < NT; ++t) S[t] = f32x4_t{S[t][0] * end, S[t][1] * end, S[t][2] * end, S[t][3] * end};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const f32x4_t w = *reinterpret_cast<const f32x4_t*>(q.w + 16 * i + 4 * g4);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float xw = x[4 * i + r] * w[r];
-        const Pack<T, NT> bv = *reinterpret_cast<const Pack<T, NT>*>(Bs + (16 * i + 4 * g4 + r) * BP + NT * c);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(to_f32(bv.v[t]), xw, S[t], 0, 0, 0);
-      }
-    }
-    // what the chunk's own tokens add: the wave's 16 tokens
-    f32x4_t own = {0.f, 0.f, 0.f, 0.f};
+    f32x4_t own = {0.f, 0.f, 0.f, 0.f};      // what the chunk's own tokens add: the wave's 16 tokens
     const float hi = q.hi[16 * wave + c], lo = q.lo[16 * wave + c];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (j > wave) break;
+    auto weights = [&](int j, float* v) {    // of tokens 16 j + 4 g4 + r
       const f32x4_t hj = *reinterpret_cast<const f32x4_t*>(q.hi + 16 * j + 4 * g4), lj = *reinterpret_cast<const f32x4_t*>(q.lo + 16 * j + 4 * g4),
                     dj = *reinterpret_cast<const f32x4_t*>(q.dt + 16 * j + 4 * g4);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float dt = 16 * j + 4 * g4 + r <= 16 * wave + c ? dj[r] : 0.f, e = __builtin_amdgcn_exp2f(fminf((hi - hj[r]) + (lo - lj[r]), 0.f));
-        own = __builtin_amdgcn_mfma_f32_16x16x4f32(f.cb[j][r] * e * dt, x[4 * j + r], own, 0, 0, 0);
+        v[r] = f.cb[j][r] * e * dt;
+      }
+    };
+    if constexpr (kParts) {
+      const T* bt = Bs + (4 * g4 + ((lane & 15) >> 2)) * BP + (lane & 3) * 4;
+      f32x4_t small[NT];                     // what the lower parts add, by itself: the state rounds once more for it, not once a product
+#pragma unroll
+      for (int t = 0; t < NT; ++t) small[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {          // 32 tokens
+        float xw[8];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const f32x4_t w = *reinterpret_cast<const f32x4_t*>(q.w + 32 * s + 16 * i + 4 * g4);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) xw[4 * i + r] = x[8 * s + 4 * i + r] * w[r];
+        }
+        const Parts xp = in_parts(xw);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const T* at = bt + 32 * s * BP + 16 * t;
+          const s16x4_t b0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4_t __attribute__((address_space(3)))*)at);
+          const s16x4_t b1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4_t __attribute__((address_space(3)))*)(at + 16 * BP));
+          const bf16x8_t a = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
+          const u32x4_t aw = __builtin_bit_cast(u32x4_t, a);
+          small[t] = mfma32(aw, xp.mid, mfma32(aw, xp.lo, small[t]));
+          S[t] = mfma32(aw, xp.hi, S[t]);
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) S[t] = f32x4_t{S[t][0] + small[t][0], S[t][1] + small[t][1], S[t][2] + small[t][2], S[t][3] + small[t][3]};
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        if (2 * s > wave) break;
+        float v[8];
+        weights(2 * s, v);
+        weights(2 * s + 1, v + 4);           // (of the next 16 tokens, wholly ahead of the wave's where 2 s is its own: zeros)
+        u32x4_t xb;                          // bf16 as they were
+#pragma unroll
+        for (int k = 0; k < 4; ++k) xb[k] = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, x[8 * s + 2 * k + 1]), __builtin_bit_cast(unsigned, x[8 * s + 2 * k]), 0x07060302u);
+        own = mfma32(in_parts(v), xb, own);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const f32x4_t w = *reinterpret_cast<const f32x4_t*>(q.w + 16 * i + 4 * g4);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float xw = x[4 * i + r] * w[r];
+          const Pack<T, NT> bv = *reinterpret_cast<const Pack<T, NT>*>(Bs + (16 * i + 4 * g4 + r) * BP + NT * c);
+#pragma unroll
+          for (int t = 0; t < NT; ++t) S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(to_f32(bv.v[t]), xw, S[t], 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (j > wave) break;
+        float v[4];
+        weights(j, v);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) own = __builtin_amdgcn_mfma_f32_16x16x4f32(v[r], x[4 * j + r], own, 0, 0, 0);
       }
     }
     float xo[4];
@@ -702,6 +823,7 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, cons
     for (int r = 0; r < 4; ++r) xo[r] = xs[(b * kQ + 16 * wave + 4 * g4 + r) * kXPitch + c];
     const f32x4_t e = *reinterpret_cast<const f32x4_t*>(q.e + 16 * wave + 4 * g4);
     __builtin_amdgcn_sched_barrier(0);
+    load_kept(ahead, f);
     post(d, b ^ 1);                     // (B: the wave's own reads of it are done)
     __syncthreads();
     f32x4_t sum = ps[b][0][wave][lane];
@@ -717,17 +839,20 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, cons
     }
   };
   Kept f[2];
-  {
-    Passed d;
-    load_passed(k0, d);
-    load_kept(k0, f[0]);
-    post(d, 0);
+  Passed d[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    load_passed(min(k0 + i, k1 - 1), d[i]);
+    load_kept(min(k0 + i, k1 - 1), f[i]);
   }
+  post(d[0], 0);
   __syncthreads();
-  for (int k = k0; k < k1; k += 2) {
-    step(k, f[0], f[1]);
-    if (k + 1 < k1) step(k + 1, f[1], f[0]);
+  int k = k0;
+  for (; k + 1 < k1; k += 2) {         // (a branch around the second step would make the first wait for requests it does not need)
+    step(k, f[0], d[0], d[1]);
+    step(k + 1, f[1], d[1], d[0]);
   }
+  if (k < k1) step(k, f[0], d[0], d[1]);
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
