@@ -71,6 +71,14 @@ def test_every_tile_of_the_wide_gemm(lib, wd, bm, ntw):
         assert err < tol, (M, N, K, ks, err, tol)
 
 
+# blocks of 96 and 160 tokens, whose activation pieces the two wave groups do not share evenly
+@pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
+@pytest.mark.parametrize("bm", [96, 160])
+@pytest.mark.parametrize("ntw", [2, 3, 4])
+def test_tiles_of_uneven_pieces(lib, wd, bm, ntw):
+    test_every_tile_of_the_wide_gemm(lib, wd, bm, ntw)
+
+
 # bf16 tiles by 32-deep K-steps: one pair of them, as many pairs as the ring of activations has, fewer and more; slices of two and of uneven length
 @pytest.mark.parametrize("bm,ntw", [(192, 4), (256, 3), (256, 4)])
 @pytest.mark.parametrize("M,N,K,ks", [(1, 16, 64, 1), (193, 208, 128, 1), (257, 272, 192, 1), (191, 400, 256, 1), (640, 560, 1088, 1), (300, 272, 128, 2), (255, 784, 704, 3)])

@@ -12,7 +12,7 @@ namespace mi {
 // =====================================================================================
 // A 128 x 128 tile pulls 16 KiB of activations + 8 (16) KiB of weights per 64-deep K-step for 2.1 MFLOP.  A CU takes in 55 - 65 GB/s
 // once half of it comes from HBM (64 KiB of requests in flight, 1.2 us each; from L2 it takes 125 GB/s), so the tile grows: 128 tokens x 256
-// weight rows = 16 + 16 (32) KiB for 4.2 MFLOP, 256 x 256 = 32 + 16 (32) KiB for 8.4.  Smaller ones (64, 128, 192 tokens x 128, 192 weight rows) are for
+// weight rows = 16 + 16 (32) KiB for 4.2 MFLOP, 256 x 256 = 32 + 16 (32) KiB for 8.4.  Smaller ones (64, 96, 128, 160, 192 tokens x 128, 192 weight rows) are for
 // what those leave idle: a grid of one and a bit rounds, token blocks mostly padding, few tokens, whose K then takes fewer slabs.  Eight waves as 2 (tokens) x 4 (weight
 // rows): activation fragments are shared by four waves, weight fragments by two.  Both operands arrive by LDS-DMA
 // (global_load_lds, 1 KiB per wave-instruction: the weight tiles land lane-linear = fragment
@@ -87,11 +87,11 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
   // waves as 2 (tokens) x 4 (weight rows), each MT 16-token tiles x NTW 16-row weight tiles (4 x 2 waves would read 16 instead of 20 KiB of
   // fragments per K-step at 256 x 256 but decode every weight code four times instead of twice)
   constexpr int MT = BM / 32, WM = 2;
-  constexpr int XH = BM / 64, XP = KD * XH;   // 8-row activation pieces per wave and 64-deep part, and per stage
+  constexpr int X0 = (MT + 1) / 2, X1 = MT - X0;                 // 8-row activation pieces per wave and 64-deep part: group 0, group 1
   constexpr int WPH = WD == MI_W_BF16 ? 2 : 1, WPK = KD * WPH;   // 1 KiB weight tiles per 16 rows and 64-deep part, and per K-step
-  // the 4 NTW WPK weight tiles of a stage over the waves: group 0 (waves 0-3) may bring one more each than group 1 (twelve tiles)
+  // the 4 NTW WPK weight tiles and BM / 8 activation pieces of a stage over the waves: group 0 (waves 0-3) may bring one more each than group 1
   constexpr int WP0 = (NTW * WPK + 1) / 2, WP1 = NTW * WPK - WP0;
-  constexpr int kDma0 = WP0 + XP, kDma1 = WP1 + XP;   // DMAs per wave and stage
+  constexpr int kDma0 = WP0 + KD * X0, kDma1 = WP1 + KD * X1;   // DMAs per wave and stage
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int g = lane >> 4, c = lane & 15;
@@ -103,17 +103,18 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
 
   // this lane's DMA sources: weight tiles wt0 .. (fragment order) and XP 8-row pieces of the activation tile
   const int grp = __builtin_amdgcn_readfirstlane(wave >> 2), wt0 = grp == 0 ? WP0 * wave : 4 * WP0 + WP1 * (wave - 4);
+  const int xp0 = grp == 0 ? X0 * wave : 4 * X0 + X1 * (wave - 4);
   const uint4* wsrc[WP0];
-  const uint16_t* xsrc[XP];
+  const uint16_t* xsrc[KD * X0];
 #pragma unroll
   for (int i = 0; i < WP0; ++i) {   // tile (row tile / WPK, k tile % WPK); a group-1 wave without an i-th one does not use it
     const int t = min(wt0 + i, 4 * NTW * WPK - 1);
     wsrc[i] = W + ((size_t)min(ntb + t / WPK, NT - 1) * KT + ks0 * WPK + t % WPK) * 64 + lane;
   }
 #pragma unroll
-  for (int i = 0; i < XP; ++i) {
-    const int r = (XH * wave + i % XH) * 8 + (lane >> 3), sl = lane & 7;
-    xsrc[i] = x + (size_t)min(m0 + r, T - 1) * ldx + (size_t)(ks0 * KD + i / XH) * 64 + ((sl ^ xs_swz<WD>(r)) * 8);   // LDS slot sl of row r holds chunk sl ^ swz(r)
+  for (int i = 0; i < KD * X0; ++i) {
+    const int r = min(xp0 + i % X0, BM / 8 - 1) * 8 + (lane >> 3), sl = lane & 7;
+    xsrc[i] = x + (size_t)min(m0 + r, T - 1) * ldx + (size_t)(ks0 * KD + i / X0) * 64 + ((sl ^ xs_swz<WD>(r)) * 8);   // LDS slot sl of row r holds chunk sl ^ swz(r)
   }
   auto issue = [&](int ks, int stage) {
     unsigned char* st = smem + stage * kStage;
@@ -122,8 +123,17 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
     if constexpr (WP0 > WP1) {
       if (grp == 0) glds16(wsrc[WP1] + (size_t)ks * WPK * 64, st + (wt0 + WP1) * 1024);
     }
+    auto bring_x = [&](int d, int i) { glds16(xsrc[d * X0 + i] + (size_t)ks * (64 * KD), st + kW + d * (BM * 128) + (xp0 + i) * 1024); };
 #pragma unroll
-    for (int i = 0; i < XP; ++i) glds16(xsrc[i] + (size_t)ks * (64 * KD), st + kW + (i / XH) * (BM * 128) + (XH * wave + i % XH) * 1024);
+    for (int d = 0; d < KD; ++d)
+#pragma unroll
+      for (int i = 0; i < X1; ++i) bring_x(d, i);
+    if constexpr (X0 > X1) {
+      if (grp == 0) {
+#pragma unroll
+        for (int d = 0; d < KD; ++d) bring_x(d, X1);
+      }
+    }
   };
 
   f32x4_t acc[NTW][MT];
@@ -364,7 +374,7 @@ __global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restric
 // tiles of one-byte weights with 128-deep K-steps: what fits the LDS three times
 constexpr bool wide_tile_deep(int wd, int bm, int ntw) { return wd != MI_W_BF16 && 2 * (ntw * 4096 + bm * 128) * 3 <= 160 * 1024; }
 // bf16 tiles whose 64-deep stages fit the LDS twice only: 256 x 192, 192 x 256, 256 x 256
-constexpr bool wide_tile_by_32(int wd, int bm, int ntw) { return wd == MI_W_BF16 && bm + 64 * ntw > 384; }
+constexpr bool wide_tile_by_32(int wd, int bm, int ntw) { return wd == MI_W_BF16 && 3 * (ntw * 8192 + bm * 128) > 160 * 1024; }
 
 template <int WD, int EPI, int BM, int NTW, bool SPLIT>
 static int launch_gemm_wide_t(const LinearW& w, int T, const uint16_t* x, int ldx, const EpiArgs& e, hipStream_t s, int KS, float* slab) {
@@ -431,7 +441,9 @@ int launch_gemm_wide_wd(const LinearW& w, int T, const uint16_t* x, int ldx, int
 #define MI_GT(BM_, NTW_) \
   if (bm == BM_ && ntw == NTW_) return launch_gemm_wide_bm<WD, BM_, NTW_>(w, T, x, ldx, epi, e, s, ks, ws, defer)
   MI_GT(64, 2); MI_GT(64, 3); MI_GT(64, 4);
+  MI_GT(96, 2); MI_GT(96, 3); MI_GT(96, 4);
   MI_GT(128, 2); MI_GT(128, 3); MI_GT(128, 4);
+  MI_GT(160, 2); MI_GT(160, 3); MI_GT(160, 4);
   MI_GT(192, 2); MI_GT(192, 3); MI_GT(192, 4);
   MI_GT(256, 2); MI_GT(256, 3); MI_GT(256, 4);
 #undef MI_GT

@@ -271,51 +271,48 @@ extern template int launch_gemm_wide_wd<MI_W_BF16>(const LinearW&, int, const ui
 extern template int launch_gemm_wide_wd<MI_W_F8E4M3>(const LinearW&, int, const uint16_t*, int, int, const EpiArgs&, hipStream_t, int, int, int, float*, SlabSum*);
 extern template int launch_gemm_wide_wd<MI_W_INT8>(const LinearW&, int, const uint16_t*, int, int, const EpiArgs&, hipStream_t, int, int, int, float*, SlabSum*);
 
-// Which tile and K-split: the cheapest of a model of the kernel, us, fitted to 167 shapes for bf16 weights and 148 for those of a byte (40 .. 4000 tokens, the
-// projections of TinyLlama, Llama-8B, Qwen2.5-7B and of the layer stacks; every tile and up to ten slices of each timed; the choice is 2 % from the fastest on average).
+// Which tile and K-split: the cheapest of a model of the kernel, us, fitted to 9334 launches: 24 projections of TinyLlama, Llama-8B, Qwen2.5-7B and the layer stacks, 70 ..
+// 2000 tokens, the tiles and up to nine slices whose cost came near the least, weights from memory (enough copies in turn to fill the caches).  The choice takes 1.1 % longer than the
+// fastest on average with bf16 weights, 0.8 % with fp8, 0.6 % with int8; with the constants before, 2.8, 1.1 and 0.9 %, and without blocks of 96 and 160 tokens 3.9, 2.5 and 3.5.
 // The kernel holds more than half of a CU's LDS, i.e. ONE work-group per CU, so a launch is rounds of 32 work-groups on each of the eight XCDs:
-// a round a ramp and epilogue that grow with the tile, beside its K-steps.  us per 64-deep K-step on an almost empty and on a full chip:
-//     64 x 128: fp8 0.19 / 0.28, bf16 0.31 / 0.39, int8 0.31 / 0.39;  128 x 256: fp8 0.64 / 0.77, bf16 0.75 / 0.83, int8 0.81 / 0.92
-//     192 x 192: fp8 0.69 / 0.85, bf16 0.70 / 0.86, int8 0.72 / 0.95;  256 x 256: fp8 1.06 / 1.30, bf16 0.89 / 1.46, int8 0.99 / 1.37
-// For weights of a byte their stream has a term: with a slice for every CU it is memory that binds, and fewer slices are as fast (8B fp8 prompts of 75 / 140 / 430 tokens
-// 1823 -> 1750, 2229 -> 2134, 3754 -> 3654 us a call; with constants of the same kind bf16 gained 4 % in places and lost 1 % in others: left).
+// a round a ramp and epilogue that grow with the tile, beside its K-steps, whose time grows from an almost empty to a full chip; and the weights' stream, where it binds.
 // A K-split writes its slabs, and a second launch sums them, or the row norm that follows reads them.
+// What blocks of 96 and 160 tokens are for, us, best of the others -> best: 28672 x 4096 bf16 300 tokens 77.5 -> 67.4, 777 tokens 174 -> 160, fp8 90 tokens 30.6 -> 26.8, 300
+// tokens 75.0 -> 66.6; 37888 x 3584 int8 90 tokens 49.2 -> 40.6, 777 tokens 211 -> 190; 12288 x 2048 bf16 777 tokens 47.2 -> 39.4.
 // Against the best of 128 x 256 and 256 x 256 alone, us: int8 gate|up of the 7B model at 188 tokens 79 -> 60 (148 tiles of 256 x 256 on 256 CUs, 73 % of
 // each filled; 198 of 192 x 192), its down projection 41.6 -> 34.4; bf16 gate|up of TinyLlama 700 tokens 51.6 -> 35.4, 200 tokens 28.4 -> 21.4;
 // fp8 QKV of the 8B model 1400 tokens 82.6 -> 63.9; bf16 down projection of 2048 x 14336 at 100 tokens 26.4 -> 17.6.
-// With 256 x 192 and 192 x 256 of bf16 weights (49 more shapes, the choice 0.5 % from the fastest): 12288 x 2048 777 tokens 54.8 -> 46.0, 1000 tokens
-// 55.1 -> 48.5, 3072 x 2048 4000 tokens 58.9 -> 50.2, 28672 x 4096 377 tokens 99.4 -> 82.0, 4096 x 14336 1500 tokens 175.9 -> 153.8.
 struct WidePlan { int bm, ntw, ks; };
 static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, bool deferred) {
   int cus = 256;
   if (device_num_cu(&cus) != MI_OK || cus < 8) cus = 256;
-  // us per 64-deep K-step on an almost empty chip and on a full one: {1, m ntw, m, ntw}, m = bm / 64
-  static const double kStep[3][2][4] = {
-      {{0., 0.0310, 0.0289, 0.1119}, {0.0113, 0.0104, 0.1250, 0.1172}},
-      {{0.0421, 0.0428, 0.0357, 0.0463}, {0.0349, 0.0507, 0.0626, 0.0502}},
-      {{0.0813, 0.0177, 0.0187, 0.1367}, {0.0782, 0.0402, 0.0624, 0.0994}}};
-  // us: launch, a round's ramp and what it grows by with the tile, the factor of a grid without a CU to spare, slabs written, a launch that sums them
-  struct Rest { double launch, ramp, area, full, full_area, slab, sum, sum_mb; };
-  static const Rest kRest[2] = {{4.1, 1.2, 0.42, 1.028, 0.0032, 0., 2.65, 0.179}, {2.64, 0.56, 0.471, 1.065, 0., 0.092, 3.38, 0.113}};
-  const bool byte = wd != MI_W_BF16;
-  const Rest& r = kRest[byte];
+  struct Model {
+    double lo[4], hi[4];           // us per 64-deep K-step on an almost empty chip and on a full one: {1, m ntw, m, ntw}, m = bm / 64
+    double deep[2], by_32[4];      // lo and hi: factors of 128-deep K-steps; of 256 x 256 and of the other two tiles with 32-deep K-steps (hi as inside long calls)
+    double launch, ramp, area;     // a launch; a round, and what it grows by with m ntw
+    double full, full_area;        // factor of a grid without a CU to spare: the slowest decides
+    double stream, slab;           // MB of weights a us; us per MB of slabs written
+  };
+  static const Model kModel[3] = {
+      {{0.0018, 0.0429, 0.0171, 0.0848}, {0.0016, 0.0208, 0.0944, 0.1035}, {1, 1}, {0.8862, 1.39, 0.7131, 1.13}, 3.405, 2.328, 0.3204, 1.0014, 0.0029, 6.604, 0.1129},
+      {{0.0094, 0.0435, 0.0163, 0.0335}, {0.0129, 0.0545, 0.0524, 0.0468}, {0.8062, 0.9204}, {0, 0, 0, 0}, 4.852, 1.738, 0.4059, 1.0135, 0.0021, 7.348, 0.0531},
+      {{0.0182, 0.0154, 0.0396, 0.1147}, {0.0296, 0.0403, 0.0633, 0.1088}, {0.7322, 0.949}, {0, 0, 0, 0}, 5.493, 1.132, 0.488, 1.0151, 0.0012, 7.284, 0.0479}};
+  const Model& r = kModel[wd];
   const int nks = K / 64;
-  const double mb = (double)T * N * 4e-6, stream = byte ? (double)N * K / 6.67e6 : 0.;   // the weights at 6.7 TB/s
+  const double mb = (double)T * N * 4e-6, stream = (double)N * K * elem_bytes(wd) * 1e-6 / r.stream;
   WidePlan best{0, 4, 1};   // (bm 0: none compared yet; one slice is always allowed, so there is one)
   double best_cost = 0.;
-  for (int bm = 64; bm <= 256; bm += 64)
+  for (const int bm : {64, 96, 128, 160, 192, 256})
     for (int ntw = 2; ntw <= 4; ++ntw) {
-      const double m = bm / 64, area = m * ntw;
+      const double m = bm / 64., area = m * ntw;
       const auto us = [&](const double (&k)[4]) { return k[0] + k[1] * area + k[2] * m + k[3] * ntw; };
-      double lo = us(kStep[wd][0]), hi = us(kStep[wd][1]);
-      if (wide_tile_by_32(wd, bm, ntw)) {   // (the kernel with 32-deep K-steps)
-        lo = area == 16 ? 0.893 : 0.95;
-        hi = area == 16 ? 1.456 : 1.2;
-      } else if (byte) {
-        if (wide_tile_deep(wd, bm, ntw)) { lo *= 0.75; hi *= 0.94; }
-        if (ntw == 3) { lo *= 1.022; hi *= 1.022; }
-      } else if (bm == 192) {
-        hi *= 1.04;
+      double lo = us(r.lo), hi = us(r.hi);
+      if (wide_tile_by_32(wd, bm, ntw)) {
+        lo = r.by_32[area == 16 ? 0 : 2];
+        hi = r.by_32[area == 16 ? 1 : 3];
+      } else if (wide_tile_deep(wd, bm, ntw) && K % 128 == 0) {
+        lo *= r.deep[0];
+        hi *= r.deep[1];
       }
       const int tiles = ceil_div(T, bm) * ceil_div(N, 64 * ntw);
       for (int ks = 1; ks <= 10; ++ks) {
@@ -323,9 +320,9 @@ static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, boo
         if (ks > 1 && (per < 4 || (ks - 1) * per >= nks || (size_t)ks * T * N * sizeof(float) > ws_bytes)) continue;
         const int rounds = ceil_div(ceil_div(tiles, 8) * ks, std::max(1, cus / 8));
         double body = rounds * (r.ramp + r.area * area + per * (lo + (hi - lo) * std::min(1.0, (double)tiles * ks / cus)));
-        if (rounds * cus - tiles * ks < 6) body *= r.full + r.full_area * area;   // no CU to spare: the slowest decides
-        double cost = r.launch + (byte ? std::sqrt(body * body + stream * stream) : body);
-        if (ks > 1) cost += r.slab * ks * mb + (deferred ? 0.144 * ks * mb : r.sum + r.sum_mb * (ks + 1) * mb);
+        if (rounds * cus - tiles * ks < 6) body *= r.full + r.full_area * area;
+        double cost = r.launch + std::sqrt(body * body + stream * stream);
+        if (ks > 1) cost += r.slab * ks * mb + (deferred ? 0.144 * ks * mb : 3.38 + 0.113 * (ks + 1) * mb);
         if (best.bm == 0 || cost < best_cost) { best = WidePlan{bm, ntw, ks}; best_cost = cost; }
       }
     }
