@@ -131,3 +131,26 @@ def test_logits_of_many_rows_to_the_host(vocab):
         std = out[32].std().item()
         assert torch.isfinite(out[32]).all() and torch.equal(out[17], out[32][:17]) and (out[16] - out[32][:16]).abs().max().item() < 0.05 * std
         model.close()
+
+
+# 17 .. 32 rows of one-byte weights leave the register kernel where deep K slices are summed by the next norm, and where unsplit K fills the chip (fp8 gate | up of 24576 rows)
+@pytest.mark.parametrize("wd,hidden,inter", [("f8e4m3", 256, 4096), ("f8e4m3", 3584, 12288), ("int8", 256, 16384)])
+def test_rows_on_both_sides_of_the_wide_gemm(wd, hidden, inter):
+    from oracle import DecoderConfig
+    from oracle.synth import make_weights
+    from tests.helpers import decode_inputs
+    from vllm_neuron_amd._native import MI_Q, MI_W, NativeModel
+    shape = dict(num_layers=2, hidden_size=hidden, num_heads=4, num_kv_heads=2, head_dim=64, intermediate_size=inter, vocab_size=512)
+    model = NativeModel(**shape, rms_norm_eps=1e-5, rope_theta=1e4, rope_type=0, rope_factor=1.0, num_blocks=34, block_size=32, max_num_seqs=33,
+                        max_model_len=32, weight_dtype=MI_W[wd], quant_type=MI_Q["per_channel_symmetric"], quantize_lm_head=1, tp_degree=1, tp_rank=0,
+                        device_id=0, use_graphs=1, ctx_buckets=[32])
+    model.load_state_dict(make_weights(DecoderConfig(**shape), seed=4))
+    model.finalize()
+    out = {}
+    for rows in (16, 17, 31, 32, 33):
+        for _ in range(2):             # eager pass, then the graph
+            out[rows] = model.forward(**decode_inputs([7 * i % 512 for i in range(rows)], [0] * rows, [[1 + i] for i in range(rows)], 32, 32)).clone()
+    std = out[16].std().item()
+    for rows in (17, 31, 32, 33):      # sums in another order, roundings of bf16 activations behind them: as between any two kernels
+        assert torch.isfinite(out[rows]).all() and (out[16] - out[rows][:16]).abs().max().item() < 0.05 * std and (out[33][:rows] - out[rows]).abs().max().item() < 0.05 * std
+    model.close()

@@ -71,9 +71,9 @@ def test_every_tile_of_the_wide_gemm(lib, wd, bm, ntw):
         assert err < tol, (M, N, K, ks, err, tol)
 
 
-# blocks of 96 and 160 tokens, whose activation pieces the two wave groups do not share evenly
+# blocks of 32, 96 and 160 tokens, whose activation pieces the two wave groups do not share evenly (32: the second has none)
 @pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
-@pytest.mark.parametrize("bm", [96, 160])
+@pytest.mark.parametrize("bm", [32, 96, 160])
 @pytest.mark.parametrize("ntw", [2, 3, 4])
 def test_tiles_of_uneven_pieces(lib, wd, bm, ntw):
     test_every_tile_of_the_wide_gemm(lib, wd, bm, ntw)

@@ -12,7 +12,7 @@ namespace mi {
 // =====================================================================================
 // A 128 x 128 tile pulls 16 KiB of activations + 8 (16) KiB of weights per 64-deep K-step for 2.1 MFLOP.  A CU takes in 55 - 65 GB/s
 // once half of it comes from HBM (64 KiB of requests in flight, 1.2 us each; from L2 it takes 125 GB/s), so the tile grows: 128 tokens x 256
-// weight rows = 16 + 16 (32) KiB for 4.2 MFLOP, 256 x 256 = 32 + 16 (32) KiB for 8.4.  Smaller ones (64, 96, 128, 160, 192 tokens x 128, 192 weight rows) are for
+// weight rows = 16 + 16 (32) KiB for 4.2 MFLOP, 256 x 256 = 32 + 16 (32) KiB for 8.4.  Smaller ones (32 by 32 to 192 tokens x 128, 192 weight rows) are for
 // what those leave idle: a grid of one and a bit rounds, token blocks mostly padding, few tokens, whose K then takes fewer slabs.  Eight waves as 2 (tokens) x 4 (weight
 // rows): activation fragments are shared by four waves, weight fragments by two.  Both operands arrive by LDS-DMA
 // (global_load_lds, 1 KiB per wave-instruction: the weight tiles land lane-linear = fragment
@@ -440,6 +440,7 @@ int launch_gemm_wide_wd(const LinearW& w, int T, const uint16_t* x, int ldx, int
                         SlabSum* defer) {
 #define MI_GT(BM_, NTW_) \
   if (bm == BM_ && ntw == NTW_) return launch_gemm_wide_bm<WD, BM_, NTW_>(w, T, x, ldx, epi, e, s, ks, ws, defer)
+  MI_GT(32, 2); MI_GT(32, 3); MI_GT(32, 4);
   MI_GT(64, 2); MI_GT(64, 3); MI_GT(64, 4);
   MI_GT(96, 2); MI_GT(96, 3); MI_GT(96, 4);
   MI_GT(128, 2); MI_GT(128, 3); MI_GT(128, 4);

@@ -155,7 +155,10 @@ int run_linear(mi_ctx* c, const Linear& L, int rows, int pro, ProArgs p, int epi
     if (!c->runs(MI_K_GEMV)) return MI_OK;
     Scope sc(c, MI_K_GEMV);
     if (c->prof.on) c->prof.gemv_bytes += (double)L.bytes();
-    MI_TRY(launch_gemv_regs(L.view(), rows, x, ldx, epi, e, c->stream, c->splitk_ws, c->splitk_ws_bytes, defer, as_deferred));
+    if (!e.far_out && ldx % 8 == 0 && gemm_wide_few_rows(L.view(), rows, defer || as_deferred))
+      MI_TRY(launch_gemm_wide(L.view(), rows, x, ldx, epi, e, c->stream, c->splitk_ws, c->splitk_ws_bytes, defer, as_deferred));
+    else
+      MI_TRY(launch_gemv_regs(L.view(), rows, x, ldx, epi, e, c->stream, c->splitk_ws, c->splitk_ws_bytes, defer, as_deferred));
     note_deferred();
     return MI_OK;
   }
@@ -2101,7 +2104,8 @@ int mi_op_qlinear(const void* x, int32_t M, const void* w_tiled, const float* sc
     float* slab = nullptr;
     const size_t bytes = (size_t)64 << 20;
     MI_HIP(hipMalloc(reinterpret_cast<void**>(&slab), bytes));
-    int rc = gemv_in_regs(W, M, bytes) || gemv_few_rows_in_regs(W, M, bytes, false) ? launch_gemv_regs(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes)
+    int rc = gemm_wide_few_rows(W, M, false) ? launch_gemm_wide(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes)
+             : gemv_in_regs(W, M, bytes) || gemv_few_rows_in_regs(W, M, bytes, false) ? launch_gemv_regs(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes)
              : gemv_fits(M, K) ? launch_gemv(W, M, PRO_BF16, p, EPI_F32, e, (hipStream_t)stream) : launch_gemm(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes);
     hipStreamSynchronize((hipStream_t)stream);
     hipFree(slab);
@@ -2109,7 +2113,7 @@ int mi_op_qlinear(const void* x, int32_t M, const void* w_tiled, const float* sc
   }
   if (force_path == 3) return launch_gemm_wide(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream);
   // the wide GEMM with its K dimension split: 4 / 5 = 2 / 4 slices at 128-token blocks, 6 / 7 at 256; 100 bm + 10 ntw + ks: tiles of bm tokens x 64 ntw rows, ks slices
-  const bool tile = force_path >= 6400;
+  const bool tile = force_path >= 3200;
   if (tile || (force_path >= 4 && force_path <= 7)) {
     const int ks = tile ? force_path % 10 : (force_path & 1) ? 4 : 2, bm = tile ? force_path / 100 : force_path >= 6 ? 256 : 128, ntw = tile ? force_path / 10 % 10 : 4;
     MI_CHECK(ks >= 1 && (tile || K / 64 % ks == 0), "qlinear: paths 4 .. 7 need K / 64 a multiple of their slices");
