@@ -756,16 +756,18 @@ __device__ __forceinline__ int kv_swz(int key) {   // XOR key of the 16-byte chu
 
 constexpr int kPrefillSlices = 6;   // of the keys, at most
 
+// A work-group has the heads of one kv head, or the sub-th of `subs` equal parts of them.
 // KH 2: the waves of a head are two, which take a step's two tiles of keys, one each, and put their sums together at the end: a work-group then has one query
 // block at a time (NW = 2 Gp).  KH 1: a wave takes every tile of its block, and a work-group has NW / Gp blocks.
 // A tile is a chain of LDS reads, products and exponentials, 1.6 us for a wave that has its SIMD to itself and 1.3 where two share it.  With 4 heads on a kv head two
 // blocks used to share a work-group: the wave of the light one left the other alone for most of the way, and up to 1000 tokens half of the CUs had none.
 // Alone, us, 32 heads of 128 on 8: 500 tokens 16.0 -> 13.6, 1000 26.8 -> 22.2, 900 behind 900 47.1 -> 33.9, 2031 49.3 -> 45.9 (60 tokens, one step: 7.1 -> 7.6).
 // Without the loads from memory 2031 tokens take 40.0, without the exponentials 44.5; half a step between the two parts (as in the wide GEMM): 53.4.
-// 16 waves for 8 heads do not fit the registers.
+// 16 waves for 8 heads do not fit the registers: 5 .. 8 heads on a kv head go to two work-groups, which both read its keys.  28 heads of 128 on 4, us: 500 tokens
+// 18.8 -> 14.0, 1000 32.0 -> 22.3, 188 behind 512 23.0 -> 16.5, 900 behind 900 51.7 -> 33.2, 2031 58.1 -> 44.0; 32 heads of 64 on 4: 239 8.6 -> 6.9, 1000 23.2 -> 15.1, 2031 42.6 -> 30.0.
 template <int HD, int NW, int KH>
 __device__ __forceinline__ void attn_prefill2_body(
-    unsigned char* smem, int bx, int kvh, int bz, int nz, const uint16_t* __restrict__ q, int T, int q_pos0, const uint16_t* __restrict__ kpool,
+    unsigned char* smem, int bx, int kvh, int sub, int subs, int bz, int nz, const uint16_t* __restrict__ q, int T, int q_pos0, const uint16_t* __restrict__ kpool,
     const uint16_t* __restrict__ vpool, int bs, int bs_shift, const int32_t* __restrict__ block_table, int nh, int nkv,
     int G, int Gp, int nblk, int paired, float* __restrict__ o_part, float* __restrict__ ml_part, uint16_t* __restrict__ out, float scale_log2e) {
   constexpr int TK = 64;                       // keys per tile
@@ -786,8 +788,9 @@ __device__ __forceinline__ void attn_prefill2_body(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int QB = KH == 1 ? NW / Gp : 1;
   const int hl = wave % Gp, slot = KH == 1 ? wave / Gp : 0, part = KH == 1 ? 0 : wave / Gp;
-  const int head = kvh * G + min(hl, G - 1);
-  const bool head_ok = hl < G;
+  const int per = ceil_div(G, subs), h0 = sub * per, hn = min(per, G - h0);      // this work-group's heads of the kv head's
+  const int head = kvh * G + h0 + min(hl, hn - 1);
+  const bool head_ok = hl < hn;
   const int kv_len = q_pos0 + T;
   const int last_piece_key = ((kv_len - 1) / KPP) * KPP;
   const int qq = lane & 31, h = lane >> 5;
@@ -1097,9 +1100,9 @@ template <int HD, int NW, int KH>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4, NW / 4))) void attn_prefill2_kernel(
     const uint16_t* __restrict__ q, int T, int q_pos0, const uint16_t* __restrict__ kpool,
     const uint16_t* __restrict__ vpool, int bs, int bs_shift, const int32_t* __restrict__ block_table, int nh, int nkv,
-    int G, int Gp, int nblk, int paired, float* __restrict__ o_part, float* __restrict__ ml_part, uint16_t* __restrict__ out, float scale_log2e) {
+    int G, int Gp, int subs, int nblk, int paired, float* __restrict__ o_part, float* __restrict__ ml_part, uint16_t* __restrict__ out, float scale_log2e) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  attn_prefill2_body<HD, NW, KH>(smem, blockIdx.y, blockIdx.x, blockIdx.z, gridDim.z, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk, paired, o_part,
+  attn_prefill2_body<HD, NW, KH>(smem, blockIdx.y, blockIdx.x / subs, blockIdx.x % subs, subs, blockIdx.z, gridDim.z, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk, paired, o_part,
                              ml_part, out, scale_log2e);
 }
 
@@ -1111,11 +1114,12 @@ template <int HD, int KH, bool FINAL>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_mixed_kernel(
     const uint16_t* __restrict__ q, int T, int q_pos0, const uint16_t* __restrict__ kpool,
     const uint16_t* __restrict__ vpool, int bs, int bs_shift, const int32_t* __restrict__ block_table, int nh, int nkv,
-    int G, int Gp, int nblk, int paired, int gx, int ns, float* __restrict__ o_part, float* __restrict__ ml_part, uint16_t* __restrict__ out, float scale_log2e, DecodeSide d) {
+    int G, int Gp, int subs, int nblk, int paired, int gx, int ns, float* __restrict__ o_part, float* __restrict__ ml_part, uint16_t* __restrict__ out, float scale_log2e, DecodeSide d) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   if ((int)blockIdx.x >= d.nd) {
     const int x = (int)blockIdx.x - d.nd;
-    attn_prefill2_body<HD, 8, KH>(smem, x % gx, blockIdx.y, x / gx, ns, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk,
+    const int y = x / subs;
+    attn_prefill2_body<HD, 8, KH>(smem, y % gx, blockIdx.y, x % subs, subs, y / gx, ns, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk,
                               paired, o_part, ml_part, out, scale_log2e);
   } else {
     attn_decode_body<HD, 8, FINAL>(smem, (int)blockIdx.x % d.NS, blockIdx.y, (int)blockIdx.x / d.NS, d.q, kpool, vpool, bs, d.block_table, d.MB, d.ctx_lens, nh, nkv, G, d.NS,
@@ -1159,29 +1163,33 @@ static bool attn_prefill_v1() {   // MI355X_ATTN_PREFILL_V1=1: the first-generat
 }
 
 static int prefill_heads(int G) { return G <= 1 ? 1 : (G <= 2 ? 2 : (G <= 4 ? 4 : 8)); }
-struct PrefillPlan { int Gp, kh, nblk, bs_shift, paired, gx, ns; float *o_part = nullptr, *ml_part = nullptr; };
+struct PrefillPlan { int Gp, kh, subs, nblk, bs_shift, paired, gx, ns; float *o_part = nullptr, *ml_part = nullptr; };
 static PrefillPlan prefill_plan(int T, int q_pos0, int block_size, int nh, int nkv, int hd, float* ws, size_t ws_bytes, int num_cu) {
-  // second generation: 8 waves = (8 / Gp) query blocks x Gp heads, blocks in complementary pairs; or a block of 4 heads, two waves each
+  // second generation: 8 waves = (8 / Gp) query blocks x Gp heads, blocks in complementary pairs; or, from 3 heads on a kv head on, a block of up to 4 heads, two waves each
   PrefillPlan p;
   p.Gp = prefill_heads(nh / nkv);
-  p.kh = p.Gp == 4 ? 2 : 1;
+  // (a single tile leaves the second wave of a head without one: 7.1 -> 7.6 us at 60 tokens)
+  p.kh = p.Gp >= 4 && q_pos0 + T > 64 ? 2 : 1;
+  p.subs = p.kh == 2 && p.Gp == 8 ? 2 : 1;
+  if (p.subs == 2) p.Gp = 4;
+  const int groups = nkv * p.subs;             // of heads: work-groups that read the same queries' keys
   const int nblk = ceil_div(T, 32), npair = (nblk + 1) / 2, qb = p.kh == 2 ? 1 : 8 / p.Gp;
   int bs_shift = -1;
   for (int sh = 4; sh < 20; ++sh) if ((1 << sh) == block_size) bs_shift = sh;
   // One block per work-group (5 .. 8 heads on a kv head): pairs only where single blocks would not all run at once.
-  const int paired = qb > 1 || nblk * nkv > num_cu;
+  const int paired = qb > 1 || nblk * groups > num_cu;
   const int gx = paired ? ceil_div(npair, qb >= 2 ? qb / 2 : 1) : nblk;
-  // A short prompt, or the rest of one behind cached keys, leaves most of the chip idle while each work-group walks its tiles, 1.75 us each (2.4 us two of them):
+  // A short prompt, or the rest of one behind cached keys, leaves most of the chip idle while each work-group walks its tiles, 1.75 us each (two of them by pairs of waves 2.4, 1.4 of 64-wide heads):
   // slices of the keys then, at least two tiles each, the cheapest by that and the second launch, which moves every slice's O out and in.
   // 188 tokens behind 512 cached ones, 28 heads on 4: 40.8 us in 12 work-groups of two passes, 16.7 + 4.8 now.
   int ns = 1;
   const int steps = ceil_div(q_pos0 + T, 64 * p.kh);
-  const double per_step = p.kh == 2 ? 2.4 : 1.75;
-  double best = per_step * steps * ceil_div(gx * nkv, num_cu);
+  const double per_step = p.kh == 1 ? 1.75 : hd == 128 ? 2.4 : 1.4;
+  double best = per_step * steps * ceil_div(gx * groups, num_cu);
   for (int z = 2; ws && z <= kPrefillSlices; ++z) {
     const size_t part = (size_t)z * T * nh;
     if (ceil_div(steps, z) * p.kh < 2 || part * (hd + 2) * sizeof(float) > ws_bytes) break;
-    const double cost = per_step * ceil_div(steps, z) * ceil_div(gx * nkv * z, num_cu) + 4.5 + (double)part * hd * 8.0 / 4e6;
+    const double cost = per_step * ceil_div(steps, z) * ceil_div(gx * groups * z, num_cu) + 4.5 + (double)part * hd * 8.0 / 4e6;
     if (cost < best) { best = cost; ns = z; }
   }
   p.nblk = nblk; p.bs_shift = bs_shift; p.paired = paired; p.gx = gx; p.ns = ns;
@@ -1212,8 +1220,8 @@ int launch_attn_prefill(const uint16_t* q, int T, int q_pos0, const uint16_t* kp
 #define MI_P2(HD_, NW_, KH_) do { \
       constexpr int lds = attn_prefill2_lds<HD_, NW_, KH_>(); \
       MI_TRY_A(ensure_dynamic_lds(reinterpret_cast<const void*>(attn_prefill2_kernel<HD_, NW_, KH_>), lds)); \
-      hipLaunchKernelGGL((attn_prefill2_kernel<HD_, NW_, KH_>), dim3(nkv, p.gx, p.ns), dim3(NW_ * 64), lds, s, q, T, q_pos0, kpool, vpool, block_size, p.bs_shift, \
-                         block_table, nh, nkv, G, p.Gp, p.nblk, p.paired, p.o_part, p.ml_part, out, scale_log2e); \
+      hipLaunchKernelGGL((attn_prefill2_kernel<HD_, NW_, KH_>), dim3(nkv * p.subs, p.gx, p.ns), dim3(NW_ * 64), lds, s, q, T, q_pos0, kpool, vpool, block_size, p.bs_shift, \
+                         block_table, nh, nkv, G, p.Gp, p.subs, p.nblk, p.paired, p.o_part, p.ml_part, out, scale_log2e); \
     } while (0)
     if (p.kh == 1) { if (hd == 128) MI_P2(128, 8, 1); else MI_P2(64, 8, 1); }
     else { if (hd == 128) MI_P2(128, 8, 2); else MI_P2(64, 8, 2); }
@@ -1250,7 +1258,7 @@ static int launch_mixed_t(const AttnMixed& m, const PrefillPlan& p, int T, int q
   const auto fn = p.kh == 2 ? (NS == 1 ? attn_mixed_kernel<HD, 2, true> : attn_mixed_kernel<HD, 2, false>)
                             : (NS == 1 ? attn_mixed_kernel<HD, 1, true> : attn_mixed_kernel<HD, 1, false>);
   MI_TRY_A(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds));
-  hipLaunchKernelGGL(fn, dim3(d.nd + p.gx * p.ns, nkv), dim3(512), lds, s, q, T, q_pos0, kpool, vpool, bs, p.bs_shift, bt, nh, nkv, nh / nkv, p.Gp, p.nblk, p.paired,
+  hipLaunchKernelGGL(fn, dim3(d.nd + p.gx * p.ns * p.subs, nkv), dim3(512), lds, s, q, T, q_pos0, kpool, vpool, bs, p.bs_shift, bt, nh, nkv, nh / nkv, p.Gp, p.subs, p.nblk, p.paired,
                      p.gx, p.ns, p.o_part, p.ml_part, out, scale_log2e, d);
   if (NS > 1) hipLaunchKernelGGL((attn_combine_kernel<HD>), dim3(nh, m.B), dim3(HD), 0, s, o_part, ml_part, NS, nh, m.out);
   launch_prefill_combine(p, T, nh, HD, out, s);
@@ -1269,7 +1277,7 @@ int launch_attn_mixed(const AttnMixed& m, int T, int q_pos0, const uint16_t* q, 
   int num_cu = 0;
   MI_TRY_A(device_num_cu(&num_cu));
   const PrefillPlan p = prefill_plan(T, q_pos0, block_size, nh, nkv, hd, ws, ws_bytes, num_cu);
-  if (attn_prefill_v1() || (p.gx * p.ns + mixed_splits(m, nkv, hd) * m.B) * nkv > num_cu) {
+  if (attn_prefill_v1() || (p.gx * p.ns * p.subs + mixed_splits(m, nkv, hd) * m.B) * nkv > num_cu) {
     int rc = launch_attn_decode(m.q, kpool, vpool, block_size, m.block_table, m.MB, m.ctx_lens, m.B, nh, nkv, hd, m.out, m.scratch, s, false, 1, m.num_blocks, m.max_ctx);
     return rc != MI_OK ? rc : launch_attn_prefill(q, T, q_pos0, kpool, vpool, block_size, block_table, nh, nkv, hd, out, s, ws, ws_bytes);
   }
