@@ -1181,7 +1181,8 @@ static PrefillPlan prefill_plan(int T, int q_pos0, int block_size, int nh, int n
   const int gx = paired ? ceil_div(npair, qb >= 2 ? qb / 2 : 1) : nblk;
   // A short prompt, or the rest of one behind cached keys, leaves most of the chip idle while each work-group walks its tiles, 1.75 us each (two of them by pairs of waves 2.4, 1.4 of 64-wide heads):
   // slices of the keys then, at least two tiles each, the cheapest by that and the second launch, which moves every slice's O out and in.
-  // 188 tokens behind 512 cached ones, 28 heads on 4: 40.8 us in 12 work-groups of two passes, 16.7 + 4.8 now.
+  // 188 tokens behind 512 cached ones, 28 heads on 4: 40.8 us in 12 work-groups of two passes, 16.7 + 4.8 in four slices, 13.8 + 4.8 in three by pairs of waves, 16.5 by
+  // pairs without: what slices cost whatever their number is more there.  (Not with 64-wide heads: 100 tokens behind 800, 32 heads on 4, 1439 us a call with slices, 1497 without.)
   int ns = 1;
   const int steps = ceil_div(q_pos0 + T, 64 * p.kh);
   const double per_step = p.kh == 1 ? 1.75 : hd == 128 ? 2.4 : 1.4;
@@ -1189,7 +1190,7 @@ static PrefillPlan prefill_plan(int T, int q_pos0, int block_size, int nh, int n
   for (int z = 2; ws && z <= kPrefillSlices; ++z) {
     const size_t part = (size_t)z * T * nh;
     if (ceil_div(steps, z) * p.kh < 2 || part * (hd + 2) * sizeof(float) > ws_bytes) break;
-    const double cost = per_step * ceil_div(steps, z) * ceil_div(gx * groups * z, num_cu) + 4.5 + (double)part * hd * 8.0 / 4e6;
+    const double cost = per_step * ceil_div(steps, z) * ceil_div(gx * groups * z, num_cu) + (p.kh == 2 && hd == 128 ? 6.0 : 4.5) + (double)part * hd * 8.0 / 4e6;
     if (cost < best) { best = cost; ns = z; }
   }
   p.nblk = nblk; p.bs_shift = bs_shift; p.paired = paired; p.gx = gx; p.ns = ns;
