@@ -1871,13 +1871,19 @@ int mi_forward_spec(mi_ctx* t, mi_ctx* d, int32_t B, int32_t k, const int64_t* i
     MI_HIP(hipSetDevice(kt.device_id));   // the event is recorded on shard 0's stream: it belongs to shard 0's device
     MI_HIP(hipEventCreateWithFlags(&ids_ready, hipEventDisableTiming));
   }
-  int rc = group_run(g, [&](mi_ctx* rcx, int r) -> int {
-    MI_TRY(stage_target(rcx));
+  auto draft = [&](int r) -> int {
     if (r != 0) return MI_OK;
     MI_TRY(draft_chain());
     if (ids_ready) MI_HIP(hipEventRecord(ids_ready, t0->stream));
     return MI_OK;
+  };
+  // Where the shards share a stream, every one has staged its rows before the draft starts: the draft's step may be captured on that stream, and what another thread
+  // puts on it meanwhile would go into the graph in place of running (or end the capture: "unjoined work").
+  int rc = group_run(g, [&](mi_ctx* rcx, int r) -> int {
+    MI_TRY(stage_target(rcx));
+    return g->lockstep ? (int)MI_OK : draft(r);
   });
+  if (rc == MI_OK && g->lockstep) rc = group_run(g, [&](mi_ctx*, int r) -> int { return draft(r); });
   if (rc == MI_OK)
     rc = group_run(g, [&](mi_ctx* rcx, int r) -> int {
       if (r != 0) {   // the candidates' ids: from shard 0's inputs into this shard's (one stream and GPU in loopback mode)
