@@ -76,12 +76,15 @@ bool gemv_few_rows_in_regs(const LinearW& w, int M, size_t ws_bytes, bool deferr
 // us a launch at 24 / 32 rows, register kernel -> blocks of 32 tokens, weights from memory: 4096 x 4096 fp8 11.8 / 13.0 -> 8.8 / 9.2, 4096 x 14336 fp8 16.0 / 17.2 -> 15.7 / 15.3,
 // 28672 x 4096 fp8 26.4 / 27.7 -> 24.8 / 25.5, 3584 x 18944 int8 23.6 / 25.2 -> 20.7 / 20.7.  Where the sum of K slices has a taker, or tiles of unsplit K fill the chip.  Not: int8
 // unsplit, whose codes the smallest tiles decode too often (37888 x 3584 32.0 / 34.2 -> 33.8 / 34.8), bf16 (28672 x 4096 42.8 / 44.0 -> 45.8 / 47.0), up to 16 rows (23.4 -> 23.8);
-// nor shallower K, where the norm behind reads more slabs for it (us a call: 8B int8 28 rows 1834 -> 1845, TinyLlama fp8 30 rows 1260 -> 1272).
-bool gemm_wide_few_rows(const LinearW& w, int M, bool deferred) {
+// Queries, keys and values of fp8 from 25 rows on, though a launch has to add their slices: 6144 x 4096 15.9 -> 10.8 + 4.1 at 32 rows (20 rows 13.8 -> 10.0 + 4.1: not).
+// Nor shallower K, where the norm behind reads more slabs for it (us a call: 8B int8 28 rows 1834 -> 1845, TinyLlama fp8 30 rows 1260 -> 1272).
+bool gemm_wide_few_rows(const LinearW& w, int M, int epi, bool deferred) {
   int cus = 0;
   if (M < 17 || M > 32 || w.wd == MI_W_BF16 || w.K % 64 != 0 || w.N < 32 || device_num_cu(&cus) != MI_OK) return false;
   if (w.wd == MI_W_INT8) return deferred && w.K >= 16384;
-  return w.K >= 3584 && (deferred || (w.N / 128 >= cus * 3 / 4 && w.N / 128 <= cus));
+  if (w.K < 3584) return false;
+  if (epi == EPI_QKV) return M >= 25;
+  return deferred || (w.N / 128 >= cus * 3 / 4 && w.N / 128 <= cus);
 }
 int launch_gemv_regs(const LinearW& w, int M, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s, float* ws, size_t ws_bytes, SlabSum* defer,
                      bool split_as_deferred) {
