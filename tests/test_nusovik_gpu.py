@@ -498,6 +498,30 @@ def test_state_space_duality_of_bf16_rows(lib, H, P, N, G, strong):
                 s.check_state(i)
 
 
+# A value that is not finite reaches what follows it and nothing else, and an infinity stays one: an infinite x in the first and in a later chunk (then in the state), an infinite B
+# (in every channel's state) and C (in its token alone), at the edges of tiles of 16 tokens, within which a zero weight times infinity is NaN; everything else positive and finite.
+@pytest.mark.parametrize("N", [128, 256])
+@pytest.mark.parametrize("where,at,value", [("x", 16, math.inf), ("x", 80, math.inf), ("x", 144, -math.inf), ("x", 16, math.nan), ("B", 48, math.inf), ("C", 95, math.inf)])
+def test_values_that_are_not_finite_in_bf16_rows(lib, N, where, at, value):
+    H, P = 2, 32
+    s = Ssd(lib, H, P, N, 1, 3, lengths=[200])
+    s.x[0].abs_()
+    s.x[0][at, {"x": 5, "B": H * P + 7, "C": H * P + N + 7}[where]] = value
+    s.d.abs_()
+    s.a_log[:] = -6.0                                    # (a decay of 0 would make NaN of what is infinite)
+    s.fixed[1:] = [dev(s.a_log), dev(s.d)]
+    x, b, c = s.x[0][:, :s.C].double().split([H * P, N, N], -1)
+    y, S = R.scan2(x.reshape(200, H, P), R.softplus(s.dt[0][:, :H].double() + s.bias.double()), s.a_log.double(), b.reshape(200, 1, N), c.reshape(200, 1, N), s.d.double())
+    s.ref = [y.reshape(200, -1)]
+    got, ref = s.step([(0, 200)], 0)
+    state = s.state[0].cpu().double()[:, :N, :P]
+    for g, r in ((got, ref), (state, S)):
+        finite = torch.isfinite(r)
+        assert finite.any() and torch.equal(torch.isfinite(g), finite) and torch.equal(torch.nan_to_num(g[~finite], nan=1.0), torch.nan_to_num(r[~finite], nan=1.0))
+        close(g[finite], r[finite], 5e-5)
+    assert torch.equal(torch.isfinite(ref).all(1), torch.arange(200) < at) or where == "C"
+
+
 @pytest.mark.parametrize("strong", [False, True])
 def test_state_space_duality_token_by_token_and_slots_used_again(lib, strong):
     s = Ssd(lib, 4, 24, 40, 2, 5, lengths=[70, 40, 200], slots=[0, 1, 0], strong=strong)

@@ -632,13 +632,6 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, cons
   T* Bs = reinterpret_cast<T*>(xs + 2 * kQ * kXPitch) + wave * kQ * BP;
   float* S0 = in.state + ((size_t)in.slots[sg.seq] * g.H + h) * g.Np * g.Pp + p;
   f32x4_t S[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int n = n0 + NT * (4 * g4 + r) + t;
-      S[t][r] = sg.pos0 + k0 > 0 && n < g.Np ? S0[(size_t)min(n, g.Np - 1) * g.Pp] : 0.f;
-    }
   const T* xbc = reinterpret_cast<const T*>(in.xbc) + (size_t)sg.row0 * in.ldx;
   const int at_b = g.H * g.P + grp * g.N, at_c = at_b + g.G * g.N, at_x = h * g.P + 16 * vt, bn = n0 + (lane % LPR) * W, xn = (tid & 3) * 4;
   struct Kept { Words<T, 4 * NT> c[4]; f32x4_t cb[4]; };                             // used from registers
@@ -677,7 +670,8 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, cons
       f.cb[i] = *reinterpret_cast<const f32x4_t*>(rec.cb + ((size_t)rc * g.G + grp) * kQ * kQ + (16 * wave + c) * kQ + 16 * min(i, wave) + 4 * g4);
     }
   };
-  auto post = [&](const Passed& d, int b) {
+  auto post = [&](const Passed& d, int b, auto in_parts_) {
+    constexpr bool kP = decltype(in_parts_)::value;
     float* s = reinterpret_cast<float*>(&st[b]);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -694,11 +688,11 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, cons
         for (int e = 0; e < 4; ++e) v.v[0][e] = bn < g.N ? v.v[0][e] : 0u;
       }
       T* row = Bs + (RPL * i + lane / LPR) * BP;
-      if constexpr (kParts && NT == 2) {
+      if constexpr (kP && NT == 2) {
         const unsigned a = v.v[0][0], b = v.v[0][1], cc = v.v[0][2], d2 = v.v[0][3];
         *reinterpret_cast<uint2*>(row + 4 * (lane % LPR)) = make_uint2(__builtin_amdgcn_perm(b, a, 0x05040100u), __builtin_amdgcn_perm(d2, cc, 0x05040100u));
         *reinterpret_cast<uint2*>(row + 16 + 4 * (lane % LPR)) = make_uint2(__builtin_amdgcn_perm(b, a, 0x07060302u), __builtin_amdgcn_perm(d2, cc, 0x07060302u));
-      } else if constexpr (kParts) {
+      } else if constexpr (kP) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           const unsigned a = v.v[0][t / 2], b = v.v[0][2 + t / 2];
@@ -710,11 +704,20 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, cons
     }
   };
   const float skip = in.d[h];
+  bool nan = false;
   // Two chunks ahead: with one, a chunk waits for memory longer than it computes.  `passed` goes to LDS at the end of the chunk before its own, `f` is used up in its own.
-  auto step = [&](int k, Kept& f, Passed& passed, Passed& d) {
+  auto step = [&](int k, auto& f, Passed& passed, Passed& d, auto in_parts_, auto ahead_) {
+    constexpr bool kP = decltype(in_parts_)::value, kAhead = decltype(ahead_)::value;
     const int b = (k - k0) & 1, n = min(kQ, sg.n - k * kQ), ahead = min(k + 2, k1 - 1);     // (behind the last chunk: that one again)
     const Steps& q = st[b];
-    load_passed(ahead, passed);
+    if constexpr (kAhead) {
+      load_passed(ahead, passed);
+    } else {
+      load_passed(k, d);
+      load_kept(k, f);
+      post(d, b, in_parts_);
+      __syncthreads();
+    }
     __builtin_amdgcn_sched_barrier(0);
     float x[16];               // tokens 16 i + 4 g4 + r (past the last one: its weight and step are zero)
 #pragma unroll
@@ -723,7 +726,7 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, cons
     f32x4_t o[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    if constexpr (kParts) {
+    if constexpr (kP) {
 #pragma unroll
       for (int s = 0; s < NT / 2; ++s) {
         float v[8];
@@ -758,7 +761,7 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, cons
         v[r] = f.cb[j][r] * e * dt;
       }
     };
-    if constexpr (kParts) {
+    if constexpr (kP) {
       const T* bt = Bs + (4 * g4 + ((lane & 15) >> 2)) * BP + (lane & 3) * 4;
       f32x4_t small[NT];                     // what the lower parts add, by itself: the state rounds once more for it, not once a product
 #pragma unroll
@@ -823,8 +826,10 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, cons
     for (int r = 0; r < 4; ++r) xo[r] = xs[(b * kQ + 16 * wave + 4 * g4 + r) * kXPitch + c];
     const f32x4_t e = *reinterpret_cast<const f32x4_t*>(q.e + 16 * wave + 4 * g4);
     __builtin_amdgcn_sched_barrier(0);
-    load_kept(ahead, f);
-    post(d, b ^ 1);                     // (B: the wave's own reads of it are done)
+    if constexpr (kAhead) {
+      load_kept(ahead, f);
+      post(d, b ^ 1, in_parts_);          // (B: the wave's own reads of it are done)
+    }
     __syncthreads();
     f32x4_t sum = ps[b][0][wave][lane];
 #pragma unroll
@@ -832,27 +837,64 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, cons
       const f32x4_t a = ps[b][w][wave][lane];
       sum[0] += a[0]; sum[1] += a[1]; sum[2] += a[2]; sum[3] += a[3];
     }
+    float out[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) out[r] = __builtin_fmaf(e[r], sum[r], __builtin_fmaf(skip, xo[r], own[r]));
+    if constexpr (kP) nan |= __builtin_isunordered(out[0], out[1]) | __builtin_isunordered(out[2], out[3]);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = 16 * wave + 4 * g4 + r;
-      if (i < n && p < g.P) y[(size_t)(sg.row0 + k * kQ + i) * ldy + h * g.P + p] = __builtin_fmaf(e[r], sum[r], __builtin_fmaf(skip, xo[r], own[r]));
+      if (i < n && p < g.P) y[(size_t)(sg.row0 + k * kQ + i) * ldy + h * g.P + p] = out[r];
     }
   };
-  Kept f[2];
-  Passed d[2];
+  auto load_state = [&] {
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    load_passed(min(k0 + i, k1 - 1), d[i]);
-    load_kept(min(k0 + i, k1 - 1), f[i]);
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int n = n0 + NT * (4 * g4 + r) + t;
+        S[t][r] = sg.pos0 + k0 > 0 && n < g.Np ? S0[(size_t)min(n, g.Np - 1) * g.Pp] : 0.f;
+      }
+  };
+  {
+    load_state();
+    const std::integral_constant<bool, kParts> in_parts_;
+    const std::true_type ahead;
+    Kept f[2];
+    Passed d[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      load_passed(min(k0 + i, k1 - 1), d[i]);
+      load_kept(min(k0 + i, k1 - 1), f[i]);
+    }
+    post(d[0], 0, in_parts_);
+    __syncthreads();
+    int k = k0;
+    for (; k + 1 < k1; k += 2) {         // (a branch around the second step would make the first wait for requests it does not need)
+      step(k, f[0], d[0], d[1], in_parts_, ahead);
+      step(k + 1, f[1], d[1], d[0], in_parts_, ahead);
+    }
+    if (k < k1) step(k, f[0], d[0], d[1], in_parts_, ahead);
   }
-  post(d[0], 0);
-  __syncthreads();
-  int k = k0;
-  for (; k + 1 < k1; k += 2) {         // (a branch around the second step would make the first wait for requests it does not need)
-    step(k, f[0], d[0], d[1]);
-    step(k + 1, f[1], d[1], d[0]);
+  if constexpr (kParts) {
+    // An infinite factor leaves a NaN among the sums of its parts (inf and inf - inf; an infinite bf16 factor meets parts that are 0), and what is not finite one behind a weight
+    // of zero; it stays in the state or shows in an output.  Then all chunks go through fp32 products, which leave the one an infinity and the other out.
+#pragma unroll
+    for (int t = 0; t < NT; ++t) nan |= __builtin_isunordered(S[t][0], S[t][1]) | __builtin_isunordered(S[t][2], S[t][3]);
+    int* any = reinterpret_cast<int*>(dsm);
+    __syncthreads();                     // (the last chunk's shares are read)
+    const bool here = __builtin_amdgcn_ballot_w64(nan) != 0;
+    if (lane == 0) any[wave] = here;
+    __syncthreads();
+    const bool again = any[0] | any[1] | any[2] | any[3];
+    __syncthreads();
+    if (again) {
+      load_state();
+      Kept f;
+      Passed d;
+      for (int k = k0; k < k1; ++k) step(k, f, d, d, std::false_type(), std::false_type());     // (nothing ahead, whose registers would leave one wave a SIMD)
+    }
   }
-  if (k < k1) step(k, f[0], d[0], d[1]);
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
