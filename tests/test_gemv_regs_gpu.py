@@ -1,5 +1,9 @@
 """Token generation of 5 .. 32 rows: the weight stream with the activations in registers (gemv_regs_kernel) at the edges of its splits, and the
 sums it leaves to the next norm inside the models."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -154,3 +158,37 @@ def test_rows_on_both_sides_of_the_wide_gemm(wd, hidden, inter):
     for rows in (17, 31, 32, 33):      # sums in another order, roundings of bf16 activations behind them: as between any two kernels
         assert torch.isfinite(out[rows]).all() and (out[16] - out[rows][:16]).abs().max().item() < 0.05 * std and (out[33][:rows] - out[rows]).abs().max().item() < 0.05 * std
     model.close()
+
+
+_OP = r"""
+import sys, torch
+sys.path.insert(0, %(root)r)
+from vllm_neuron_amd import _native as lib
+from tests.test_ops_gpu import WD, dev, quantize_on_device
+lib.load_library()
+for N, K in %(shapes)r:
+    g = torch.Generator().manual_seed(N + K)
+    tiled, scale = quantize_on_device(lib, torch.randn(N, K, generator=g) * 0.05, "f8e4m3", "per_channel_symmetric")
+    x, y = dev(torch.randn(32, K, generator=g).to(torch.bfloat16)), {}
+    for M in (16, 32):
+        y[M] = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+        lib.check(lib.load_library().mi_op_qlinear(x.data_ptr(), M, tiled.data_ptr(), scale.data_ptr(), None, N, K, WD["f8e4m3"], y[M].data_ptr(), 8, None))
+        torch.cuda.synchronize()
+    assert torch.isfinite(y[32]).all() and (y[32][:16] - y[16]).abs().max() < 1e-4 * y[16].std()
+    print("SAME" if torch.equal(y[32][:16], y[16]) else "OTHER", flush=True)
+"""
+
+
+def _kernels_of_32_rows(shapes, **env):
+    """Per shape: whether 32 rows have the bits of 16, i.e. take the register kernel, whose sums do not depend on the rows beside them."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", _OP % {"root": root, "shapes": shapes}], env=dict(os.environ, **env), capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, (r.stdout[-1500:], r.stderr[-1500:])
+    return [x == "SAME" for x in r.stdout.split()[-len(shapes):]]
+
+
+def test_switches_keep_32_rows_from_the_wide_gemm():
+    """fp8, 192 tiles of 128 weight rows: the wide GEMM by size, the register kernel where that one is switched off or its token blocks are forced."""
+    shape = [(24576, 3584)]
+    assert _kernels_of_32_rows(shape) == [False]
+    assert _kernels_of_32_rows(shape, MI355X_GEMM_WIDE="0") == [True] and _kernels_of_32_rows(shape, MI355X_GEMM_WIDE_BM="128") == [True]

@@ -72,6 +72,14 @@ bool gemv_few_rows_in_regs(const LinearW& w, int M, size_t ws_bytes, bool deferr
   if (ceil_div(w.K / tile_k(w.wd), kGemvWaves) <= 8 && (NT <= cus || NT >= 8 * cus)) return true;
   return deferred && 2 * NT <= cus && gemv_regs_fits(w, M, ws_bytes);
 }
+static int gemm_wide_mode() {   // MI355X_GEMM_WIDE: 0 never, 1 whenever the shape allows, unset: by size
+  static const int m = [] { const char* v = getenv("MI355X_GEMM_WIDE"); return v ? atoi(v) : -1; }();
+  return m;
+}
+static int gemm_wide_bm() {      // MI355X_GEMM_WIDE_BM: 128 / 256 forces the token block (default: by grid size)
+  static const int m = [] { const char* v = getenv("MI355X_GEMM_WIDE_BM"); const int b = v ? atoi(v) : 0; return b == 128 || b == 256 ? b : 0; }();
+  return m;
+}
 // Rows beside which the register kernel takes in more of the activations than of the weights' share of a CU, in front of the first weights; the wide GEMM brings both side by side.
 // us a launch at 24 / 32 rows, register kernel -> blocks of 32 tokens, weights from memory: 4096 x 4096 fp8 11.8 / 13.0 -> 8.8 / 9.2, 4096 x 14336 fp8 16.0 / 17.2 -> 15.7 / 15.3,
 // 28672 x 4096 fp8 26.4 / 27.7 -> 24.8 / 25.5, 3584 x 18944 int8 23.6 / 25.2 -> 20.7 / 20.7.  Where the sum of K slices has a taker, or tiles of unsplit K fill the chip.  Not: int8
@@ -80,6 +88,7 @@ bool gemv_few_rows_in_regs(const LinearW& w, int M, size_t ws_bytes, bool deferr
 // Nor shallower K, where the norm behind reads more slabs for it (us a call: 8B int8 28 rows 1834 -> 1845, TinyLlama fp8 30 rows 1260 -> 1272).
 bool gemm_wide_few_rows(const LinearW& w, int M, int epi, bool deferred) {
   int cus = 0;
+  if (gemm_wide_mode() == 0 || gemm_wide_bm()) return false;      // (128 tokens and more: none of these calls has them)
   if (M < 17 || M > 32 || w.wd == MI_W_BF16 || w.K % 64 != 0 || w.N < 32 || device_num_cu(&cus) != MI_OK) return false;
   if (w.wd == MI_W_INT8) return deferred && w.K >= 16384;
   if (w.K < 3584) return false;
@@ -342,14 +351,6 @@ static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, boo
       }
     }
   return best;
-}
-static int gemm_wide_mode() {   // MI355X_GEMM_WIDE: 0 never, 1 whenever the shape allows, unset: by size
-  static const int m = [] { const char* v = getenv("MI355X_GEMM_WIDE"); return v ? atoi(v) : -1; }();
-  return m;
-}
-static int gemm_wide_bm() {      // MI355X_GEMM_WIDE_BM: 128 / 256 forces the token block (default: by grid size)
-  static const int m = [] { const char* v = getenv("MI355X_GEMM_WIDE_BM"); const int b = v ? atoi(v) : 0; return b == 128 || b == 256 ? b : 0; }();
-  return m;
 }
 static int gemm_wide_ks() {      // MI355X_GEMM_WIDE_KS: 1 = never split K in the wide kernel
   static const int m = [] { const char* v = getenv("MI355X_GEMM_WIDE_KS"); return v ? atoi(v) : 0; }();
