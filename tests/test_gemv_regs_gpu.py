@@ -192,3 +192,9 @@ def test_switches_keep_32_rows_from_the_wide_gemm():
     shape = [(24576, 3584)]
     assert _kernels_of_32_rows(shape) == [False]
     assert _kernels_of_32_rows(shape, MI355X_GEMM_WIDE="0") == [True] and _kernels_of_32_rows(shape, MI355X_GEMM_WIDE_BM="128") == [True]
+
+
+def test_a_tile_more_than_the_chip_stays_in_registers():
+    """fp8, tiles of 128 weight rows, one work-group a CU: 257 of them on 256 CUs are a second round for one (a last tile of 16 rows counts)."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert _kernels_of_32_rows([(128 * cus + 16, 3584), (128 * cus, 3584)]) == [True, False]

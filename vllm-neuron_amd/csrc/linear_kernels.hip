@@ -93,7 +93,8 @@ bool gemm_wide_few_rows(const LinearW& w, int M, int epi, bool deferred) {
   if (w.wd == MI_W_INT8) return deferred && w.K >= 16384;
   if (w.K < 3584) return false;
   if (epi == EPI_QKV) return M >= 25;
-  return deferred || (w.N / 128 >= cus * 3 / 4 && w.N / 128 <= cus);
+  const int tiles = ceil_div(w.N, 128);      // of the wide GEMM, one work-group a CU
+  return deferred || (tiles >= cus * 3 / 4 && tiles <= cus);
 }
 int launch_gemv_regs(const LinearW& w, int M, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s, float* ws, size_t ws_bytes, SlabSum* defer,
                      bool split_as_deferred) {
