@@ -50,10 +50,12 @@ def test_edges_of_the_wide_gemm(lib, wd, M, N, K):
 @pytest.mark.parametrize("bm", [64, 128, 192, 256])
 @pytest.mark.parametrize("ntw", [2, 3, 4])
 def test_every_tile_of_the_wide_gemm(lib, wd, bm, ntw):
-    if wd == "bf16" and bm + 64 * ntw > 384 and bm * ntw < 1024:
-        pytest.skip("not built: its stages do not fit the LDS three times")
-    for M, N, K, ks in ((bm + 1, 64 * ntw + 16, 64, 1), (bm - 1, 80, 320, 1), (2 * bm, 128 * ntw, 704, 1), (33, 8 * 64 * ntw + 32, 576, 1),
-                        (bm + 17, 64 * ntw + 16, 704, 3)):
+    check_tile(lib, wd, bm, ntw, ((bm + 1, 64 * ntw + 16, 64, 1), (bm - 1, 80, 320, 1), (2 * bm, 128 * ntw, 704, 1), (33, 8 * 64 * ntw + 32, 576, 1),
+                                  (bm + 17, 64 * ntw + 16, 704, 3)))
+
+
+def check_tile(lib, wd, bm, ntw, shapes):
+    for M, N, K, ks in shapes:
         g = torch.Generator().manual_seed(M + N + K)
         w = torch.randn(N, K, generator=g) * 0.05
         x = torch.randn(M, K, generator=g).to(torch.bfloat16)
@@ -77,6 +79,17 @@ def test_every_tile_of_the_wide_gemm(lib, wd, bm, ntw):
 @pytest.mark.parametrize("ntw", [2, 3, 4])
 def test_tiles_of_uneven_pieces(lib, wd, bm, ntw):
     test_every_tile_of_the_wide_gemm(lib, wd, bm, ntw)
+
+
+# 128-deep K-steps (weights of a byte, tiles that fit the LDS three times by them, K a multiple of 128): one, two and three of them, as many as the ring of
+# three to six stages has, fewer and more; three uneven slices (4, 4 and 3 steps); four slices of 64-deep steps (3, 3, 3 and 1), whose last would be empty by
+# 128-deep ones; rows that fill a token block but for one, and the least of the calls that take blocks of 32
+@pytest.mark.parametrize("wd", ["f8e4m3", "int8"])
+@pytest.mark.parametrize("bm,ntw", [(32, 2), (32, 3), (32, 4), (64, 2), (64, 3), (64, 4), (96, 2), (96, 3), (128, 2)])
+def test_tiles_by_128_deep_steps(lib, wd, bm, ntw):
+    rows = (17, 31, 32) if bm == 32 else (bm - 1, bm, bm + 17)
+    steps = [(rows[i % 3], 64 * ntw * (1 + i % 2) + 16, 128 * n, 1) for i, n in enumerate((1, 2, 3, 4, 5, 6, 7, 8, 11))]
+    check_tile(lib, wd, bm, ntw, steps + [(m, 64 * ntw + 16, 1408, 3) for m in rows] + [(rows[0], 64 * ntw + 16, 640, 4), (rows[1], 208, 256, 2)])
 
 
 # bf16 tiles by 32-deep K-steps: one pair of them, as many pairs as the ring of activations has, fewer and more; slices of two and of uneven length
