@@ -137,8 +137,9 @@ def test_logits_of_many_rows_to_the_host(vocab):
         model.close()
 
 
-# 17 .. 32 rows of one-byte weights leave the register kernel where deep K slices are summed by the next norm, and where unsplit K fills the chip (fp8 gate | up of 24576 rows)
-@pytest.mark.parametrize("wd,hidden,inter", [("f8e4m3", 256, 4096), ("f8e4m3", 3584, 12288), ("int8", 256, 16384)])
+# 17 .. 32 rows of one-byte weights leave the register kernel where deep K slices are summed by the next norm (2048 wide), and where unsplit K fills the chip (fp8 gate | up
+# of 24576 rows); not for sums of 256 wide
+@pytest.mark.parametrize("wd,hidden,inter", [("f8e4m3", 256, 4096), ("f8e4m3", 3584, 12288), ("int8", 256, 16384), ("f8e4m3", 2048, 4096), ("int8", 2048, 17408)])
 def test_rows_on_both_sides_of_the_wide_gemm(wd, hidden, inter):
     from oracle import DecoderConfig
     from oracle.synth import make_weights
@@ -198,3 +199,45 @@ def test_a_tile_more_than_the_chip_stays_in_registers():
     """fp8, tiles of 128 weight rows, one work-group a CU: 257 of them on 256 CUs are a second round for one (a last tile of 16 rows counts)."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     assert _kernels_of_32_rows([(128 * cus + 16, 3584), (128 * cus, 3584)]) == [True, False]
+
+
+_ROUTES = r"""
+import sys, torch
+sys.path.insert(0, %(root)r)
+from vllm_neuron_amd._native import MI_Q, MI_W, NativeModel
+from tests.helpers import decode_inputs
+res = {}
+for wd, hidden, inter, heads, kv in %(shapes)r:
+    m = NativeModel(num_layers=1, hidden_size=hidden, num_heads=heads, num_kv_heads=kv, head_dim=128, intermediate_size=inter, vocab_size=512, rms_norm_eps=1e-5,
+                    rope_theta=1e4, rope_type=0, rope_factor=1.0, num_blocks=33, block_size=32, max_num_seqs=32, max_model_len=32, weight_dtype=MI_W[wd],
+                    quant_type=MI_Q["per_channel_symmetric"], quantize_lm_head=1, tp_degree=1, tp_rank=0, device_id=0, use_graphs=1, ctx_buckets=[32])
+    m.init_synthetic_weights(1, 0.02)
+    m.finalize()
+    for rows in (17, 28):
+        res[wd, hidden, inter, heads, kv, rows] = m.forward(**decode_inputs([7 * i %% 512 for i in range(rows)], [0] * rows, [[1 + i] for i in range(rows)], 32, 32)).clone()
+    m.close()
+torch.save(res, sys.argv[1])
+"""
+
+# (weights, hidden, feed-forward, heads, kv heads) -> whether 17 and 28 rows go through the register kernel alone
+_REGS_ALONE = {
+    ("int8", 2048, 16384, 16, 4): (True, True),             # of the waves' requests for the down projection's weights all are their own
+    ("int8", 2048, 17408, 16, 4): (False, False),           # 17 of 32
+    ("int8", 1536, 17408, 12, 2): (True, True),             # narrow
+    ("f8e4m3", 2048, 4096, 16, 4): (False, False),          # at most 4 of 8
+    ("f8e4m3", 1024, 4096, 8, 2): (True, True),             # narrow
+    ("f8e4m3", 2048, 14336, 16, 4): (True, True),           # 28 of 32, and 16 tiles of 128 rows times ten slices of K are 160 work-groups of the wide GEMM
+    ("f8e4m3", 3584, 3584, 28, 14): (True, True),           # K of 3584; queries, keys and values are twice the width
+    ("f8e4m3", 3584, 3584, 28, 28): (True, False)}          # three times: the wide GEMM from 25 rows on
+
+
+def test_which_calls_of_17_to_32_rows_leave_the_register_kernel(tmp_path):
+    root, got = os.path.dirname(os.path.dirname(os.path.abspath(__file__))), []
+    for i, env in enumerate(({}, dict(MI355X_GEMM_WIDE="0"))):
+        out = str(tmp_path / f"{i}.pt")
+        r = subprocess.run([sys.executable, "-c", _ROUTES % {"root": root, "shapes": list(_REGS_ALONE)}, out], env=dict(os.environ, **env), capture_output=True, text=True,
+                           timeout=300)
+        assert r.returncode == 0, (r.stdout[-1500:], r.stderr[-1500:])
+        got.append(torch.load(out, weights_only=True))
+    for k, want in _REGS_ALONE.items():
+        assert tuple(torch.equal(got[0][(*k, rows)], got[1][(*k, rows)]) for rows in (17, 28)) == want, k

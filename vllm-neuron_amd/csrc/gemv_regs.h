@@ -281,4 +281,14 @@ bool gemv_regs_fits_wd(int M, int N, int K, size_t ws_bytes) {
   return device_num_cu(&num_cu) == MI_OK && gemv_regs_slices<WD>(M, N, K, ws_bytes, false, num_cu) > 0;
 }
 
+// Which part of a wave's requests are k-tiles of its own, the sum of the slices having a taker: a row-tile's 4 or 8 go out whatever it owns.
+template <int WD>
+double gemv_regs_own_wd(int M, int N, int K, size_t ws_bytes) {
+  int num_cu = 0;
+  const int z = device_num_cu(&num_cu) == MI_OK ? gemv_regs_slices<WD>(M, N, K, ws_bytes, true, num_cu) : 0;
+  if (z == 0) return 1.;
+  const int KT = K / tile_k(WD), tiles = ceil_div(ceil_div(KT, z), kGemvWaves);
+  return (double)KT / (z * kGemvWaves * (tiles <= 4 ? 4 : 8));
+}
+
 }  // namespace mi

@@ -43,6 +43,7 @@ extern template int launch_gemv_wd<MI_W_INT8>(const LinearW&, int, int, const Pr
 template <int WD>
 int launch_gemv_regs_wd(const LinearW& w, int M, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s, float* ws, size_t ws_bytes, SlabSum* defer, bool split_as_deferred);
 template <int WD> bool gemv_regs_fits_wd(int M, int N, int K, size_t ws_bytes);
+template <int WD> double gemv_regs_own_wd(int M, int N, int K, size_t ws_bytes);
 
 static bool gemv_regs_fits(const LinearW& w, int M, size_t ws_bytes) {
   switch (w.wd) {
@@ -82,19 +83,33 @@ static int gemm_wide_bm() {      // MI355X_GEMM_WIDE_BM: 128 / 256 forces the to
 }
 // Rows beside which the register kernel takes in more of the activations than of the weights' share of a CU, in front of the first weights; the wide GEMM brings both side by side.
 // us a launch at 24 / 32 rows, register kernel -> blocks of 32 tokens, weights from memory: 4096 x 4096 fp8 11.8 / 13.0 -> 8.8 / 9.2, 4096 x 14336 fp8 16.0 / 17.2 -> 15.7 / 15.3,
-// 28672 x 4096 fp8 26.4 / 27.7 -> 24.8 / 25.5, 3584 x 18944 int8 23.6 / 25.2 -> 20.7 / 20.7.  Where the sum of K slices has a taker, or tiles of unsplit K fill the chip.  Not: int8
-// unsplit, whose codes the smallest tiles decode too often (37888 x 3584 32.0 / 34.2 -> 33.8 / 34.8), bf16 (28672 x 4096 42.8 / 44.0 -> 45.8 / 47.0), up to 16 rows (23.4 -> 23.8);
-// Queries, keys and values of fp8 from 25 rows on, though a launch has to add their slices: 6144 x 4096 15.9 -> 10.8 + 4.1 at 32 rows (20 rows 13.8 -> 10.0 + 4.1: not).
-// Nor shallower K, where the norm behind reads more slabs for it (us a call: 8B int8 28 rows 1834 -> 1845, TinyLlama fp8 30 rows 1260 -> 1272).
-bool gemm_wide_few_rows(const LinearW& w, int M, int epi, bool deferred) {
+// 28672 x 4096 fp8 26.4 / 27.7 -> 24.8 / 25.5, 3584 x 18944 int8 23.6 / 25.2 -> 20.7 / 20.7.  Not: int8 unsplit, whose codes the smallest tiles decode too often (37888 x 3584
+// 32.0 / 34.2 -> 33.8 / 34.8), bf16 (28672 x 4096 42.8 / 44.0 -> 45.8 / 47.0), up to 16 rows (23.4 -> 23.8); nor shallower K (us a call: 8B int8 28 rows 1834 -> 1845, TinyLlama
+// fp8 30 rows 1260 -> 1272).  The lines below are drawn through us a layer of 78 models of 1024 .. 8192 wide, feed-forwards of 3584 .. 28672, at 17 .. 32 rows, one projection after the
+// other moved to the wide GEMM in the same model:
+// K slices whose sum the next norm takes: by the share of a register wave's requests that are k-tiles of its own (they go out by 4 and 8, and those it does not have repeat the last).
+// fp8: up to 27 / 32 of them 0 .. 9 less; beyond that 0.5 .. 3 less where the wide GEMM's tiles times ten slices at most fill the chip (N of 3584, 4096, 4608), else up to 4 more
+// (7168 x 17408 17 rows; 6144 x 16384 1.4); 3584 x 3584 0.2 .. 1.7 more.  int8: up to 5 / 8 2 .. 8 less, beyond that between 3 less and 4 more (3072 x 24576; 7168 x 28672).  Where the
+// weights themselves take longest the register kernel streams them faster (fp8 7168 x 22016 4 more, 8192 x 28672 5, 8192 x 17408 5 .. 9 less), and narrow sums leave the wide GEMM
+// half of the chip and more (1536 x 11008 fp8 0.6 more, 1536 x 20480 int8 1.5, 1024 x 20480 2.8).
+// Unsplit gate | up of fp8 that fills three quarters of the chip in one round: 0.5 .. 12 less.
+// Queries, keys and values of fp8 from 25 rows on, though a launch has to add their slices (6144 x 4096 15.9 -> 10.8 + 4.1 at 32 rows; 20 rows 13.8 -> 10.0 + 4.1: not): a kv head for
+// four q heads and more 1 .. 4.5 less, one for each 2 .. 6; between, from 6 less (10240 x 5120) to 1.4 more (7168 x 3584); 8192 wide 0 (10240) and 4 more (12288).
+bool gemm_wide_few_rows(const LinearW& w, int M, int epi, size_t ws_bytes, bool deferred) {
   int cus = 0;
   if (gemm_wide_mode() == 0 || gemm_wide_bm()) return false;      // (128 tokens and more: none of these calls has them)
   if (M < 17 || M > 32 || w.wd == MI_W_BF16 || w.K % 64 != 0 || w.N < 32 || device_num_cu(&cus) != MI_OK) return false;
-  if (w.wd == MI_W_INT8) return deferred && w.K >= 16384;
-  if (w.K < 3584) return false;
-  if (epi == EPI_QKV) return M >= 25;
   const int tiles = ceil_div(w.N, 128);      // of the wide GEMM, one work-group a CU
-  return deferred || (tiles >= cus * 3 / 4 && tiles <= cus);
+  const bool fp8 = w.wd == MI_W_F8E4M3;
+  if (deferred) {
+    if (w.K < (fp8 ? 4096 : 16384) || w.N < 2048 || (size_t)w.N * w.K > 150000000) return false;
+    const double own = fp8 ? gemv_regs_own_wd<MI_W_F8E4M3>(M, w.N, w.K, ws_bytes) : gemv_regs_own_wd<MI_W_INT8>(M, w.N, w.K, ws_bytes);
+    if (own <= (fp8 ? 27. / 32. : 5. / 8.)) return true;
+    return fp8 && w.K >= 8192 && tiles * std::min(10, cus / tiles) * 16 > cus * 15;
+  }
+  if (!fp8 || w.K < 3584) return false;
+  if (epi == EPI_QKV) return M >= 25 && w.K <= 7168 && (2 * w.N <= 3 * w.K || w.N >= 3 * w.K);
+  return tiles >= cus * 3 / 4 && tiles <= cus;
 }
 int launch_gemv_regs(const LinearW& w, int M, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s, float* ws, size_t ws_bytes, SlabSum* defer,
                      bool split_as_deferred) {
