@@ -241,3 +241,34 @@ def test_which_calls_of_17_to_32_rows_leave_the_register_kernel(tmp_path):
         got.append(torch.load(out, weights_only=True))
     for k, want in _REGS_ALONE.items():
         assert tuple(torch.equal(got[0][(*k, rows)], got[1][(*k, rows)]) for rows in (17, 28)) == want, k
+
+
+# queries, keys and values by the wide GEMM from 25 rows on (their slices' sum rotates them and writes them to the pool, which the second step reads), the down
+# projection by it from 17 rows on, logits to the host in groups of four row-tiles of which the last has one: against the oracle, at the bar of the other dispatch tests
+@pytest.mark.parametrize("rows", [16, 17, 25, 32])
+def test_two_steps_of_many_rows_against_the_oracle(rows):
+    from oracle import DecoderConfig, PagedDecoderOracle
+    from oracle.synth import make_weights
+    from tests.helpers import decode_inputs
+    from vllm_neuron_amd._native import MI_Q, MI_W, NativeModel
+    shape = dict(num_layers=1, hidden_size=3584, num_heads=28, num_kv_heads=4, head_dim=128, intermediate_size=4096, vocab_size=1040)
+    if not _oracle:
+        cfg = DecoderConfig(**shape)
+        _oracle.append((cfg, make_weights(cfg, seed=4)))
+    cfg, w = _oracle[0]
+    oracle = PagedDecoderOracle(cfg, w, 34, 32, compute="bf16", quant=dict(quantized=True, quantization_dtype="f8e4m3", quantization_type="per_channel_symmetric"))
+    model = NativeModel(**shape, rms_norm_eps=cfg.rms_norm_eps, rope_theta=cfg.rope_theta, rope_type=0, rope_factor=1.0, num_blocks=34, block_size=32, max_num_seqs=32,
+                        max_model_len=32, weight_dtype=MI_W["f8e4m3"], quant_type=MI_Q["per_channel_symmetric"], quantize_lm_head=1, tp_degree=1, tp_rank=0, device_id=0,
+                        use_graphs=1, ctx_buckets=[32])
+    model.load_state_dict(w)
+    model.finalize()
+    for at in range(2):
+        inputs = decode_inputs([(31 * i + 7 * at) % 1040 for i in range(rows)], [at] * rows, [[1 + i] for i in range(rows)], 32, 32)
+        want = oracle.forward(**inputs).float()
+        for _ in range(2):             # eager pass, then the graph
+            d = model.forward(**inputs).float() - want
+            assert torch.isfinite(d).all() and d.pow(2).mean().sqrt() < 0.02 * want.std() and d.abs().max() < 0.1 * want.std()
+    model.close()
+
+
+_oracle = []
