@@ -432,9 +432,9 @@ int mi_op_untile_weight(const void* tiled, int32_t N, int32_t K, int32_t weight_
 /* y[M, N] fp32 = (x[M, K] bf16 . Wq^T) * scale (+ bias).  force_path: 0 without a workspace: up to 32 rows the weight-streaming kernels of 16 rows
  * (cut in two beyond), else the GEMM; 1 those kernels (M <= 32); 2 the GEMM (picked by size); 3 the wide LDS-DMA GEMM (1-byte weights);
  * 4 / 5 that GEMM with K split over 2 / 4 slices at 128-token blocks, 6 / 7 at 256-token blocks (1-byte weights, K / 64 a multiple of the slices);
- * 8 what the models run, with a workspace of their size for K slices: up to 32 rows in registers where K fits them (up to 4: and where that is faster), else up to 16 rows path 1's
- * kernels, else the GEMM; 100 bm + 10 ntw + ks the wide GEMM in tiles of bm (64, 128, 192, 256) tokens x 64 ntw (2, 3, 4) weight rows and ks
- * (1 .. 9) K slices. */
+ * 8 what the models run, with a workspace of their size for K slices: up to 32 rows in registers where K fits them (up to 4: and where that is faster; 17 to 32
+ * rows of 1-byte weights: the wide GEMM where that is faster), else up to 16 rows path 1's kernels, else the GEMM; 100 bm + 10 ntw + ks the wide GEMM in tiles of
+ * bm (32, 64, 96, 128, 160, 192, 256) tokens x 64 ntw (2, 3, 4) weight rows and ks (1 .. 9) K slices. */
 int mi_op_qlinear(const void* x_bf16, int32_t M, const void* w_tiled, const float* scale,
                   const float* bias, int32_t N, int32_t K, int32_t weight_dtype, float* y,
                   int32_t force_path, void* stream);

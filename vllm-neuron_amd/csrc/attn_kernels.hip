@@ -761,7 +761,7 @@ constexpr int kPrefillSlices = 6;   // of the keys, at most
 // block at a time (NW = 2 Gp).  KH 1: a wave takes every tile of its block, and a work-group has NW / Gp blocks.
 // A tile is a chain of LDS reads, products and exponentials, 1.6 us for a wave that has its SIMD to itself and 1.3 where two share it.  With 4 heads on a kv head two
 // blocks used to share a work-group: the wave of the light one left the other alone for most of the way, and up to 1000 tokens half of the CUs had none.
-// Alone, us, 32 heads of 128 on 8: 500 tokens 16.0 -> 13.6, 1000 26.8 -> 22.2, 900 behind 900 47.1 -> 33.9, 2031 49.3 -> 45.9 (60 tokens, one step: 7.1 -> 7.6).
+// Alone, us, 32 heads of 128 on 8: 500 tokens 16.0 -> 13.6, 1000 26.8 -> 22.2, 900 behind 900 47.1 -> 33.9, 2031 49.3 -> 45.9 (60 tokens, whose one tile leaves the second wave idle, 7.1 -> 7.6: those keep KH 1).
 // Without the loads from memory 2031 tokens take 40.0, without the exponentials 44.5; half a step between the two parts (as in the wide GEMM): 53.4.
 // 16 waves for 8 heads do not fit the registers: 5 .. 8 heads on a kv head go to two work-groups, which both read its keys.  28 heads of 128 on 4, us: 500 tokens
 // 18.8 -> 14.0, 1000 32.0 -> 22.3, 188 behind 512 23.0 -> 16.5, 900 behind 900 51.7 -> 33.2, 2031 58.1 -> 44.0; 32 heads of 64 on 4: 239 8.6 -> 6.9, 1000 23.2 -> 15.1, 2031 42.6 -> 30.0.
@@ -1176,7 +1176,7 @@ static PrefillPlan prefill_plan(int T, int q_pos0, int block_size, int nh, int n
   const int nblk = ceil_div(T, 32), npair = (nblk + 1) / 2, qb = p.kh == 2 ? 1 : 8 / p.Gp;
   int bs_shift = -1;
   for (int sh = 4; sh < 20; ++sh) if ((1 << sh) == block_size) bs_shift = sh;
-  // One block per work-group (5 .. 8 heads on a kv head): pairs only where single blocks would not all run at once.
+  // One block per work-group (from 3 heads on a kv head on): pairs only where single blocks would not all run at once.
   const int paired = qb > 1 || nblk * groups > num_cu;
   const int gx = paired ? ceil_div(npair, qb >= 2 ? qb / 2 : 1) : nblk;
   // A short prompt, or the rest of one behind cached keys, leaves most of the chip idle while each work-group walks its tiles, 1.75 us each (two of them by pairs of waves 2.4, 1.4 of 64-wide heads):

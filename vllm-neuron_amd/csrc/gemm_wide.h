@@ -101,7 +101,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
   int ks0, nks;                               // this slice's K-steps, from K-step ks0 on
   wide_slice<SPLIT, KD>(K, ks0, nks);
 
-  // this lane's DMA sources: weight tiles wt0 .. (fragment order) and XP 8-row pieces of the activation tile
+  // this lane's DMA sources: weight tiles wt0 .. (fragment order) and X0 (group 1: X1) 8-row pieces of each 64-deep part of the activation tile
   const int grp = __builtin_amdgcn_readfirstlane(wave >> 2), wt0 = grp == 0 ? WP0 * wave : 4 * WP0 + WP1 * (wave - 4);
   const int xp0 = grp == 0 ? X0 * wave : 4 * X0 + X1 * (wave - 4);
   const uint4* wsrc[WP0];

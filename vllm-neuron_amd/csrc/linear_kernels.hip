@@ -65,7 +65,8 @@ bool gemv_in_regs(const LinearW& w, int M, size_t ws_bytes) { return M >= 5 && M
 // row-tile (the chain to the first request is shorter: no staging) or eight and more (the tiles follow each other without a barrier on the way), and, where the sums have a
 // taker, on rows of at most half the CUs: K goes over the other half.  us a launch at 1 / 4 rows, LDS kernels -> these: 2048 x 2048 bf16 5.3 / 5.5 -> 4.3 / 4.3 with a
 // taker, 4.9 / 5.2 without; 2048 x 7680 bf16 9.0 / 9.3 -> 8.2 / 8.6 and 2048 x 14336 13.8 / 14.4 -> 12.5 / 12.7 with one; 4096 x 4096 fp8 7.4 -> 6.5, int8 7.7 -> 7.1;
-// 32768 x 2048 bf16 26.2 -> 23.7.  Not between: 8192 x 2048 bf16 8.1 -> 9.3, 15360 x 2048 12.7 -> 13.4, 5120 x 4096 fp8 7.1 -> 7.5; nor K in two batches: 3584 x 3584 bf16 7.6 -> 7.7.
+// 32768 x 2048 bf16 26.2 -> 23.7.  In whole calls, us a layer, rule off and on in turn: 2048 wide fp8 1.0 .. 1.3 of 33 - 37, int8 1.4 .. 1.7 of 35 - 39, bf16 nothing to 0.3; 3584 wide fp8 0.6 .. 1.3
+// of 70, 4096 wide bf16 1 .. 2 of 93, the others nothing to 0.6 (two models of the same weights differ by 0.3).  Not between: 8192 x 2048 bf16 8.1 -> 9.3, 15360 x 2048 12.7 -> 13.4, 5120 x 4096 fp8 7.1 -> 7.5; nor K in two batches: 3584 x 3584 bf16 7.6 -> 7.7.
 bool gemv_few_rows_in_regs(const LinearW& w, int M, size_t ws_bytes, bool deferred) {
   int cus = 0;
   if (M < 1 || M > 4 || device_num_cu(&cus) != MI_OK) return false;
@@ -88,9 +89,9 @@ static int gemm_wide_bm() {      // MI355X_GEMM_WIDE_BM: 128 / 256 forces the to
 // fp8 30 rows 1260 -> 1272).  The lines below are drawn through us a layer of 78 models of 1024 .. 8192 wide, feed-forwards of 3584 .. 28672, at 17 .. 32 rows, one projection after the
 // other moved to the wide GEMM in the same model:
 // K slices whose sum the next norm takes: by the share of a register wave's requests that are k-tiles of its own (they go out by 4 and 8, and those it does not have repeat the last).
-// fp8: up to 27 / 32 of them 0 .. 9 less; beyond that 0.5 .. 3 less where the wide GEMM's tiles times ten slices at most fill the chip (N of 3584, 4096, 4608), else up to 4 more
-// (7168 x 17408 17 rows; 6144 x 16384 1.4); 3584 x 3584 0.2 .. 1.7 more.  int8: up to 5 / 8 2 .. 8 less, beyond that between 3 less and 4 more (3072 x 24576; 7168 x 28672).  Where the
-// weights themselves take longest the register kernel streams them faster (fp8 7168 x 22016 4 more, 8192 x 28672 5, 8192 x 17408 5 .. 9 less), and narrow sums leave the wide GEMM
+// fp8: up to 27 / 32 of them 0 .. 9 less; beyond that 0.5 .. 3 less where the wide GEMM's tiles times ten slices at most fill the chip (N of 3584, 4096, 4608, 8192), else up to 4 more
+// (7168 x 17408 17 rows; 6144 x 16384 1.4); 3584 x 3584 0.2 .. 1.7 more.  int8: up to 5 / 8 0.7 .. 8 less, beyond that between 3 less and 2 more (3072 x 24576; 4608 x 16384).  Where the
+// weights themselves take longest the register kernel streams them faster (fp8 7168 x 22016 4 more, 8192 x 28672 5, int8 7168 x 28672 4; fp8 8192 x 17408 still 5 .. 9 less), and narrow sums leave the wide GEMM
 // half of the chip and more (1536 x 11008 fp8 0.6 more, 1536 x 20480 int8 1.5, 1024 x 20480 2.8).
 // Unsplit gate | up of fp8 that fills three quarters of the chip in one round: 0.5 .. 12 less.
 // Queries, keys and values of fp8 from 25 rows on, though a launch has to add their slices (6144 x 4096 15.9 -> 10.8 + 4.1 at 32 rows; 20 rows 13.8 -> 10.0 + 4.1: not): a kv head for
