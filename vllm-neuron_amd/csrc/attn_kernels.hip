@@ -788,7 +788,7 @@ __device__ __forceinline__ void attn_prefill2_body(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int QB = KH == 1 ? NW / Gp : 1;
   const int hl = wave % Gp, slot = KH == 1 ? wave / Gp : 0, part = KH == 1 ? 0 : wave / Gp;
-  const int per = ceil_div(G, subs), h0 = sub * per, hn = min(per, G - h0);      // this work-group's heads of the kv head's
+  const int per = subs == 2 ? (G + 1) >> 1 : G, h0 = subs == 2 ? sub * per : 0, hn = min(per, G - h0);      // this work-group's heads of the kv head's
   const int head = kvh * G + h0 + min(hl, hn - 1);
   const bool head_ok = hl < hn;
   const int kv_len = q_pos0 + T;
@@ -1102,7 +1102,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
     const uint16_t* __restrict__ vpool, int bs, int bs_shift, const int32_t* __restrict__ block_table, int nh, int nkv,
     int G, int Gp, int subs, int nblk, int paired, float* __restrict__ o_part, float* __restrict__ ml_part, uint16_t* __restrict__ out, float scale_log2e) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  attn_prefill2_body<HD, NW, KH>(smem, blockIdx.y, blockIdx.x / subs, blockIdx.x % subs, subs, blockIdx.z, gridDim.z, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk, paired, o_part,
+  const int two = KH > 1 && subs == 2, kvh = two ? blockIdx.x >> 1 : blockIdx.x;
+  attn_prefill2_body<HD, NW, KH>(smem, blockIdx.y, kvh, two ? blockIdx.x & 1 : 0, two ? 2 : 1, blockIdx.z, gridDim.z, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk, paired, o_part,
                              ml_part, out, scale_log2e);
 }
 
@@ -1118,8 +1119,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   if ((int)blockIdx.x >= d.nd) {
     const int x = (int)blockIdx.x - d.nd;
-    const int y = x / subs;
-    attn_prefill2_body<HD, 8, KH>(smem, y % gx, blockIdx.y, x % subs, subs, y / gx, ns, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk,
+    const int two = KH > 1 && subs == 2, y = two ? x >> 1 : x;
+    attn_prefill2_body<HD, 8, KH>(smem, y % gx, blockIdx.y, two ? x & 1 : 0, two ? 2 : 1, y / gx, ns, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk,
                               paired, o_part, ml_part, out, scale_log2e);
   } else {
     attn_decode_body<HD, 8, FINAL>(smem, (int)blockIdx.x % d.NS, blockIdx.y, (int)blockIdx.x / d.NS, d.q, kpool, vpool, bs, d.block_table, d.MB, d.ctx_lens, nh, nkv, G, d.NS,
@@ -1164,19 +1165,33 @@ static bool attn_prefill_v1() {   // MI355X_ATTN_PREFILL_V1=1: the first-generat
 
 static int prefill_heads(int G) { return G <= 1 ? 1 : (G <= 2 ? 2 : (G <= 4 ? 4 : 8)); }
 struct PrefillPlan { int Gp, kh, subs, nblk, bs_shift, paired, gx, ns; float *o_part = nullptr, *ml_part = nullptr; };
+// Where one wave a head takes less time, from 3 heads on a kv head on.  By two waves each, 5 to 8 heads are two work-groups, and 3 and 4 leave the second block of a pair to a second pass:
+// behind a long prefix, or in another round of work-groups, that can cost more than the waves save.  Tiles that a work-group walks, of its block or of a pair of blocks one after the other,
+// times the rounds (single waves of 3 and 4 heads: pairs side by side, the heavy ones first, so a later round is half as long); a step of two tiles by two waves takes 1.1 of a tile by one, where
+// that one shares its SIMD 1.4 (64-wide heads: never).  Of 400 shapes (4 to 16 kv heads, 100 .. 2048 tokens behind 0 .. 6000) the choice is 0.1 % from the faster on the average, 9 % at worst.
+// us, two waves -> one: 64 heads of 128 on 8, 1500 tokens 72 -> 57, 2048 92 -> 79; 64 of 64 on 8, 1500 43 -> 37; 32 of 128 on 8, 1500 behind 2000 98 -> 92; but 28 on 4, 1500 behind 2000 87 (97).
+static bool prefill_one_wave(int heads, int T, int q_pos0, int nkv, int hd, int num_cu) {
+  const int nblk = ceil_div(T, 32), npair = (nblk + 1) / 2, kv = q_pos0 + T;
+  const auto walk = [&](int kh) {
+    const int groups = nkv * (heads == 8 ? kh : 1), paired = nblk * groups > num_cu;
+    return (ceil_div(kv, 64 * kh) + (paired ? ceil_div(q_pos0 + 32, 64 * kh) : 0)) * ceil_div((paired ? npair : nblk) * groups, num_cu);
+  };
+  if (heads == 8) return walk(1) < 1.1 * walk(2);
+  return hd == 128 && ceil_div(kv, 64) + (ceil_div(npair * nkv, num_cu) - 1) * ceil_div(q_pos0 + T / 2, 64) < 1.4 * walk(2);
+}
 static PrefillPlan prefill_plan(int T, int q_pos0, int block_size, int nh, int nkv, int hd, float* ws, size_t ws_bytes, int num_cu) {
   // second generation: 8 waves = (8 / Gp) query blocks x Gp heads, blocks in complementary pairs; or, from 3 heads on a kv head on, a block of up to 4 heads, two waves each
   PrefillPlan p;
   p.Gp = prefill_heads(nh / nkv);
-  // (a single tile leaves the second wave of a head without one: 7.1 -> 7.6 us at 60 tokens)
-  p.kh = p.Gp >= 4 && q_pos0 + T > 64 ? 2 : 1;
+  // two waves a head from half a second tile on (81 keys, 17 tokens: 6.6 -> 7.2 us; 97: as fast)
+  p.kh = p.Gp >= 4 && q_pos0 + T > 96 && !prefill_one_wave(p.Gp, T, q_pos0, nkv, hd, num_cu) ? 2 : 1;
   p.subs = p.kh == 2 && p.Gp == 8 ? 2 : 1;
   if (p.subs == 2) p.Gp = 4;
   const int groups = nkv * p.subs;             // of heads: work-groups that read the same queries' keys
   const int nblk = ceil_div(T, 32), npair = (nblk + 1) / 2, qb = p.kh == 2 ? 1 : 8 / p.Gp;
   int bs_shift = -1;
   for (int sh = 4; sh < 20; ++sh) if ((1 << sh) == block_size) bs_shift = sh;
-  // One block per work-group (from 3 heads on a kv head on): pairs only where single blocks would not all run at once.
+  // One block per work-group (two waves a head, or 5 .. 8 heads): pairs only where single blocks would not all run at once.
   const int paired = qb > 1 || nblk * groups > num_cu;
   const int gx = paired ? ceil_div(npair, qb >= 2 ? qb / 2 : 1) : nblk;
   // A short prompt, or the rest of one behind cached keys, leaves most of the chip idle while each work-group walks its tiles, 1.75 us each (two of them by pairs of waves 2.4, 1.4 of 64-wide heads):
