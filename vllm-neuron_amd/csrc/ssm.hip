@@ -856,9 +856,13 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, cons
         S[t][r] = sg.pos0 + k0 > 0 && n < g.Np ? S0[(size_t)min(n, g.Np - 1) * g.Pp] : 0.f;
       }
   };
-  {
-    load_state();
-    const std::integral_constant<bool, kParts> in_parts_;
+  const std::integral_constant<bool, kParts> in_parts_;
+  load_state();
+  if (k1 - k0 == 1) {                    // (nothing to ask for ahead: 16 prompts of 64 tokens, 64 heads in 8 groups, 76 -> 58 us with the chunks' launch)
+    Kept f;
+    Passed d;
+    step(k0, f, d, d, in_parts_, std::false_type());
+  } else {
     const std::true_type ahead;
     Kept f[2];
     Passed d[2];
