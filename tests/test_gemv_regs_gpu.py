@@ -112,8 +112,8 @@ def test_fp8_activations_stay_with_prompts(rows):
     assert torch.equal(*out)
 
 
-# logits of 17 and more rows to the host: row-tiles four side by side, a number of them that four does and does not divide, one group and several a work-group
-@pytest.mark.parametrize("vocab", [16, 80, 1024, 16448])
+# logits of 17 and more rows to the host: single row-tiles, and from 8192 rows on (two of them a CU) four side by side: a last group of one, two, three and four, one and several a work-group
+@pytest.mark.parametrize("vocab", [16, 80, 1024, 16448, 8176, 8208, 8224, 12272])
 def test_logits_of_many_rows_to_the_host(vocab):
     from oracle import DecoderConfig
     from oracle.synth import make_weights
@@ -251,7 +251,7 @@ def test_two_steps_of_many_rows_against_the_oracle(rows):
     from oracle.synth import make_weights
     from tests.helpers import decode_inputs
     from vllm_neuron_amd._native import MI_Q, MI_W, NativeModel
-    shape = dict(num_layers=1, hidden_size=3584, num_heads=28, num_kv_heads=4, head_dim=128, intermediate_size=4096, vocab_size=1040)
+    shape = dict(num_layers=1, hidden_size=3584, num_heads=28, num_kv_heads=4, head_dim=128, intermediate_size=4096, vocab_size=8208)
     if not _oracle:
         cfg = DecoderConfig(**shape)
         _oracle.append((cfg, make_weights(cfg, seed=4)))
@@ -263,7 +263,7 @@ def test_two_steps_of_many_rows_against_the_oracle(rows):
     model.load_state_dict(w)
     model.finalize()
     for at in range(2):
-        inputs = decode_inputs([(31 * i + 7 * at) % 1040 for i in range(rows)], [at] * rows, [[1 + i] for i in range(rows)], 32, 32)
+        inputs = decode_inputs([(31 * i + 7 * at) % 8208 for i in range(rows)], [at] * rows, [[1 + i] for i in range(rows)], 32, 32)
         want = oracle.forward(**inputs).float()
         for _ in range(2):             # eager pass, then the graph
             d = model.forward(**inputs).float() - want

@@ -251,8 +251,9 @@ int launch_gemv_regs_wd(const LinearW& w, int M, const uint16_t* x, int ldx, int
     return launch_splitk_reduce(sum, epi, e, s);
   }
   // (up to 16 rows the weights take longer than the way to the host, and single row-tiles deal them out more evenly: 8B fp8 8 rows 1266 us, 1280 with four;
-  //  24 rows 1695 and 1670, 7B int8 32 rows 1890 and 1830)
-  if (e.far_out && M > 16) {
+  //  24 rows 1695 and 1670, 7B int8 32 rows 1890 and 1830; nor where less than half of the CUs would have a group: us a launch, 20 - 27 rows, 2048 and 4096 wide, single row-tiles
+  //  and four: 16384 rows of logits 52.9 and 46.4, 8192 29.5 and 27.2, fp8 26.4 and 25.8, 4096 21.2 and 24.8)
+  if (e.far_out && M > 16 && w.N / 16 >= 2 * num_cu) {
     if (epi == EPI_F32) return launch_gemv_regs_k<WD, EPI_F32, 2, false, 4>(w, M, x, ldx, e, s, 1, nullptr);
     if constexpr (WD == MI_W_BF16)
       if (epi == EPI_SOFTCAP) return launch_gemv_regs_k<WD, EPI_SOFTCAP, 2, false, 4>(w, M, x, ldx, e, s, 1, nullptr);
