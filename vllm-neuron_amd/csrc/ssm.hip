@@ -601,7 +601,8 @@ constexpr size_t scan_lds() { return 2 * 16 * 64 * 16 + 2 * sizeof(Steps) + 2 * 
 // (4.0e-8 -> 4.3e-8 where steps wipe the state within a chunk).  The state and the rest on waves of their own, two a SIMD: 40.3 (branches in front of what is in flight).
 // k-slot (g4, j) of a product over states is element 8 s + j of the lane's C; of one over tokens, token 32 s + (j < 4 ? 4 g4 + j : 16 + 4 g4 + j - 4), which transposed
 // reads of B give, whose tiles lie side by side in LDS for them.
-template <typename T, int NT, bool VEC>
+// ONE: no segment has a second chunk, and nothing is asked for ahead (16 prompts of 64 tokens, 64 heads in 8 groups, with the chunks' launch 76 -> 58 us).
+template <typename T, int NT, bool VEC, bool ONE>
 __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, const AttnSeg* __restrict__ segs, int c0, int nchunks, int nvt, float* __restrict__ base,
                                                        float* __restrict__ y, int ldy) {
   extern __shared__ __attribute__((aligned(16))) unsigned char dsm[];
@@ -858,7 +859,7 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdGeom g, SsdIn in, cons
   };
   const std::integral_constant<bool, kParts> in_parts_;
   load_state();
-  if (k1 - k0 == 1) {                    // (nothing to ask for ahead: 16 prompts of 64 tokens, 64 heads in 8 groups, 76 -> 58 us with the chunks' launch)
+  if constexpr (ONE) {
     Kept f;
     Passed d;
     step(k0, f, d, d, in_parts_, std::false_type());
@@ -1096,7 +1097,11 @@ int launch_ssd_prompt(const SsdGeom& g, const SsdIn& in, const AttnSeg* sd, cons
   if (rc != MI_OK) return rc;
   MI_CHECK(nseg >= 1 && nseg <= 65535 && records && max_chunks >= 1, "state-space duality: segments / workspace");
   int chunks = 0;
-  for (int i = 0; i < nseg; ++i) chunks += sh[i].n < 2 ? 0 : ceil_div(sh[i].n, kQ);
+  bool one = true;
+  for (int i = 0; i < nseg; ++i) {
+    chunks += sh[i].n < 2 ? 0 : ceil_div(sh[i].n, kQ);
+    one &= sh[i].n <= kQ;
+  }
   const size_t lds = (size_t)kQ * 2 * tall_pitch(g.Np) * 4;
   const int nvt = g.Pp / 16, nt = g.Np <= 64 ? 1 : g.Np <= 128 ? 2 : 4;
   // whole packs of B, C and x, rows and groups aligned to them
@@ -1108,7 +1113,7 @@ int launch_ssd_prompt(const SsdGeom& g, const SsdIn& in, const AttnSeg* sd, cons
 #define MI_SSD_CHUNK(T) { auto k = ssd_chunk_kernel<T>; \
       if (lds > 48 * 1024) { rc = ensure_dynamic_lds(reinterpret_cast<const void*>(k), (int)lds); if (rc != MI_OK) return rc; } \
       hipLaunchKernelGGL(k, gc, dim3(256), lds, s, g, in, sd, nseg, c0, records); }
-#define MI_SSD_SCAN(T, NT, VEC) { auto k = ssd_scan_kernel<T, NT, VEC>; constexpr size_t bytes = scan_lds<T, NT>(); \
+#define MI_SSD_SCAN(T, NT, VEC) { auto k = one ? ssd_scan_kernel<T, NT, VEC, true> : ssd_scan_kernel<T, NT, VEC, false>; constexpr size_t bytes = scan_lds<T, NT>(); \
       if (bytes > 64 * 1024) { rc = ensure_dynamic_lds(reinterpret_cast<const void*>(k), (int)bytes); if (rc != MI_OK) return rc; } \
       hipLaunchKernelGGL(k, gs, dim3(256), bytes, s, g, in, sd, c0, n, nvt, records, y, ldy); }
 #define MI_SSD_SCAN_V(T, NT) if (vec) MI_SSD_SCAN(T, NT, true) else MI_SSD_SCAN(T, NT, false)
