@@ -501,25 +501,26 @@ def test_state_space_duality_of_bf16_rows(lib, H, P, N, G, strong):
 # A value that is not finite reaches what follows it and nothing else, and an infinity stays one: an infinite x in the first and in a later chunk (then in the state), an infinite B
 # (in every channel's state) and C (in its token alone), at the edges of tiles of 16 tokens, within which a zero weight times infinity is NaN; everything else positive and finite.
 @pytest.mark.parametrize("N", [128, 256])
-@pytest.mark.parametrize("where,at,value", [("x", 16, math.inf), ("x", 80, math.inf), ("x", 144, -math.inf), ("x", 16, math.nan), ("B", 48, math.inf), ("C", 95, math.inf)])
-def test_values_that_are_not_finite_in_bf16_rows(lib, N, where, at, value):
+@pytest.mark.parametrize("T,where,at,value", [(200, "x", 16, math.inf), (200, "x", 80, math.inf), (200, "x", 144, -math.inf), (200, "x", 16, math.nan), (200, "B", 48, math.inf),
+                                              (200, "C", 95, math.inf), (64, "x", 32, math.inf), (50, "B", 16, math.inf)])
+def test_values_that_are_not_finite_in_bf16_rows(lib, N, T, where, at, value):
     H, P = 2, 32
-    s = Ssd(lib, H, P, N, 1, 3, lengths=[200])
+    s = Ssd(lib, H, P, N, 1, 3, lengths=[T])
     s.x[0].abs_()
     s.x[0][at, {"x": 5, "B": H * P + 7, "C": H * P + N + 7}[where]] = value
     s.d.abs_()
     s.a_log[:] = -6.0                                    # (a decay of 0 would make NaN of what is infinite)
     s.fixed[1:] = [dev(s.a_log), dev(s.d)]
     x, b, c = s.x[0][:, :s.C].double().split([H * P, N, N], -1)
-    y, S = R.scan2(x.reshape(200, H, P), R.softplus(s.dt[0][:, :H].double() + s.bias.double()), s.a_log.double(), b.reshape(200, 1, N), c.reshape(200, 1, N), s.d.double())
-    s.ref = [y.reshape(200, -1)]
-    got, ref = s.step([(0, 200)], 0)
+    y, S = R.scan2(x.reshape(T, H, P), R.softplus(s.dt[0][:, :H].double() + s.bias.double()), s.a_log.double(), b.reshape(T, 1, N), c.reshape(T, 1, N), s.d.double())
+    s.ref = [y.reshape(T, -1)]
+    got, ref = s.step([(0, T)], 0)
     state = s.state[0].cpu().double()[:, :N, :P]
     for g, r in ((got, ref), (state, S)):
         finite = torch.isfinite(r)
         assert finite.any() and torch.equal(torch.isfinite(g), finite) and torch.equal(torch.nan_to_num(g[~finite], nan=1.0), torch.nan_to_num(r[~finite], nan=1.0))
         close(g[finite], r[finite], 5e-5)
-    assert torch.equal(torch.isfinite(ref).all(1), torch.arange(200) < at) or where == "C"
+    assert torch.equal(torch.isfinite(ref).all(1), torch.arange(T) < at) or where == "C"
 
 
 @pytest.mark.parametrize("strong", [False, True])
