@@ -314,6 +314,8 @@ extern template int launch_gemm_wide_wd<MI_W_INT8>(const LinearW&, int, const ui
 // Which tile and K-split: the cheapest of a model of the kernel, us, fitted to 9334 launches: 24 projections of TinyLlama, Llama-8B, Qwen2.5-7B and the layer stacks, 70 ..
 // 2000 tokens, the tiles and up to nine slices whose cost came near the least, weights from memory (enough copies in turn to fill the caches).  The choice takes 1.1 % longer than the
 // fastest on average with bf16 weights, 0.8 % with fp8, 0.6 % with int8; with the constants before, 2.8, 1.1 and 0.9 %, and without blocks of 96 and 160 tokens 3.9, 2.5 and 3.5.
+// Over 50 projections, 30 of them others, 33 .. 2048 tokens: 1.4, 1.0 and 0.7 % where a norm takes the sum, 1.7, 1.6 and 1.5 % where a launch does (before: 3.4, 3.9, 2.0 and 2.5, 2.8, 1.7); fitted to
+// all of them it is no better.
 // The kernel holds more than half of a CU's LDS, i.e. ONE work-group per CU, so a launch is rounds of 32 work-groups on each of the eight XCDs:
 // a round a ramp and epilogue that grow with the tile, beside its K-steps, whose time grows from an almost empty to a full chip; and the weights' stream, where it binds.
 // A K-split writes its slabs, and a second launch sums them, or the row norm that follows reads them.
