@@ -319,6 +319,9 @@ extern template int launch_gemm_wide_wd<MI_W_INT8>(const LinearW&, int, const ui
 // The kernel holds more than half of a CU's LDS, i.e. ONE work-group per CU, so a launch is rounds of 32 work-groups on each of the eight XCDs:
 // a round a ramp and epilogue that grow with the tile, beside its K-steps, whose time grows from an almost empty to a full chip; and the weights' stream, where it binds.
 // A K-split writes its slabs, and a second launch sums them, or the row norm that follows reads them.
+// Unsplit tiles on half of the CUs at most take 12 % more than that, inside a call above all: prompts of 34 .. 300 tokens of ten models in the same process, factor 1, 1.06, 1.12, 1.2:
+// -, 0.2, 0.3, 0.2 us a layer less with bf16 weights, -, 0.4, 0.5, 0.3 with fp8, -, 0.04, 0.08, 0.11 with int8; 2560 wide bf16, 40 tokens, 475 -> 453 us a call (gate | up on 112 CUs -> 224).  Where a
+// launch sums the slices the choice is 1.7, 1.3 and 1.2 % from the fastest with it.
 // What blocks of 96 and 160 tokens are for, us, best of the others -> best: 28672 x 4096 bf16 300 tokens 77.5 -> 67.4, 777 tokens 174 -> 160, fp8 90 tokens 30.6 -> 26.8, 300
 // tokens 75.0 -> 66.6; 37888 x 3584 int8 90 tokens 49.2 -> 40.6, 777 tokens 211 -> 190; 12288 x 2048 bf16 777 tokens 47.2 -> 39.4.
 // Against the best of 128 x 256 and 256 x 256 alone, us: int8 gate|up of the 7B model at 188 tokens 79 -> 60 (148 tiles of 256 x 256 on 256 CUs, 73 % of
@@ -349,23 +352,22 @@ static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, boo
       if (bm == 32 && T > 32) break;
       const double m = bm / 64., area = m * ntw;
       const auto us = [&](const double (&k)[4]) { return k[0] + k[1] * area + k[2] * m + k[3] * ntw; };
-      double lo = us(r.lo), hi = us(r.hi);
-      if (wide_tile_by_32(wd, bm, ntw)) {
-        lo = r.by_32[area == 16 ? 0 : 2];
-        hi = r.by_32[area == 16 ? 1 : 3];
-      } else if (wide_tile_deep(wd, bm, ntw) && K % 128 == 0) {
-        lo *= r.deep[0];
-        hi *= r.deep[1];
-      }
+      const bool by_32 = wide_tile_by_32(wd, bm, ntw), deep_tile = wide_tile_deep(wd, bm, ntw) && K % 128 == 0;
       const int tiles = ceil_div(T, bm) * ceil_div(N, 64 * ntw);
       for (int ks = 1; ks <= 10; ++ks) {
         const int per = ceil_div(nks, ks);
         if (ks > 1 && (per < 4 || (ks - 1) * per >= nks || (size_t)ks * T * N * sizeof(float) > ws_bytes)) continue;
+        double lo = by_32 ? r.by_32[area == 16 ? 0 : 2] : us(r.lo), hi = by_32 ? r.by_32[area == 16 ? 1 : 3] : us(r.hi);
+        if (deep_tile && (ks - 1) * ceil_div(K / 128, ks) < K / 128) {   // (as the launch: where 128-deep K-steps leave no slice empty)
+          lo *= r.deep[0];
+          hi *= r.deep[1];
+        }
         const int rounds = ceil_div(ceil_div(tiles, 8) * ks, std::max(1, cus / 8));
         double body = rounds * (r.ramp + r.area * area + per * (lo + (hi - lo) * std::min(1.0, (double)tiles * ks / cus)));
         if (rounds * cus - tiles * ks < 6) body *= r.full + r.full_area * area;
         double cost = r.launch + std::sqrt(body * body + stream * stream);
         if (ks > 1) cost += r.slab * ks * mb + (deferred ? 0.144 * ks * mb : 3.38 + 0.113 * (ks + 1) * mb);
+        else if (2 * tiles <= cus) cost *= 1.12;   // (half of the CUs at most: longer inside a call than alone)
         if (best.bm == 0 || cost < best_cost) { best = WidePlan{bm, ntw, ks}; best_cost = cost; }
       }
     }
