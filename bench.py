@@ -767,7 +767,7 @@ def main():
         eng2.worker.model_runner.model.model.close()
         del eng2
 
-    # ---- prefix caching (BASELINE config 4: sequences sharing a 512-token prefix) ----------------
+    # ---- prefix caching (sequences sharing a 512-token prefix) ----------------
     prefix_ttft = None
     if args.model == "qwen25_7b":
         g = torch.Generator().manual_seed(7)
@@ -806,7 +806,7 @@ def main():
     engine_dev_sampled = engine_decode_rate(SamplingParams(temperature=0.8, top_k=50, top_p=0.9, max_tokens=128, ignore_eos=True))
     model_adapter.mi355x_config.on_device_sampling_config = None
 
-    # ---- the same loop under vLLM's native scheduler (chunked prefill on, SURVEY 8f-3): every step is a
+    # ---- the same loop under vLLM's native scheduler (chunked prefill on): every step is a
     #      ragged record; once all prompts are encoded the library runs it as a token-generation step
     engine_chunked = None
     if tp == 1 and args.model == "llama31_8b":
@@ -824,7 +824,7 @@ def main():
         engc.worker.model_runner.model.model.close()
         del engc
 
-    # ---- decode at other context lengths (SURVEY 8d: ctx 256 / 1024 / 2040), device-resident ---
+    # ---- decode at other context lengths (ctx 256 / 1024 / 2040), device-resident ---
     from tests.helpers import decode_inputs
     mb = MAX_MODEL_LEN // BLOCK_SIZE
     perm = (torch.randperm(PA_NUM_BLOCKS, generator=torch.Generator().manual_seed(2)) + 1).tolist()
@@ -894,7 +894,7 @@ def main():
             traffic_src = ("profiles/gemv_traffic.json (rocprofv3 --pmc FETCH_SIZE pass of this command, x2 gfx950 "
                            "correction: the counter tallies 128-B requests at 64 B)"
                            + ("" if fresh else " -- STALE: the GEMV source has changed since that pass"))
-        roofline = {"bound": "hbm", "kernel": "mi::gemv_kernel / gemv_priv_kernel (all projections + lm_head of a step)",
+        roofline = {"bound": "hbm", "kernel": "mi::gemv_kernel / gemv_priv_kernel / gemv_regs_kernel (all projections + lm_head of a step)",
                     "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic, "traffic_source": traffic_src,
                     "algorithmic_bytes_per_launch": round(gemv_bytes / max(gemv_n, 1)),
@@ -908,7 +908,7 @@ def main():
                     "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(step_bytes / (ms_per_step * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                     "traffic": None, "step_algorithmic_GB": round(step_bytes / 1e9, 3)}
 
-    # ---- fused speculation (SURVEY 8f-4 tail): what a speculation step costs next to a plain step --------
+    # ---- fused speculation: what a speculation step costs next to a plain step --------
     speculation = None
     if tp == 1 and args.model == "llama31_8b" and wd != "bf16" and not args.no_speculation:
         speculation = speculation_section(torch, HF, wd, ms_per_step, args.steps)
@@ -917,7 +917,7 @@ def main():
     if tp == 1 and not args.no_cpu_baseline:
         cpu = cpu_baseline(MODELS["llama31_8b"] if args.model != "qwen25_7b" else HF, MAX_NUM_SEQS, DECODE_CTX)
 
-    # ---- context encoding against the MFMA roofline (SURVEY 8d): algorithmic flops = 2 W N + 4 L nh hd N^2 / 2 ----
+    # ---- context encoding against the MFMA roofline: algorithmic flops = 2 W N + 4 L nh hd N^2 / 2 ----
     def prefill_flops(n):
         head = HF["vocab_size"] * HF["hidden_size"]                 # lm_head: one row (the last token) only
         body = weight_bytes_per_step(HF, 1, 1) - head
@@ -927,7 +927,7 @@ def main():
                  "fp8_activations": ({b: round(prefill_flops(int(b) - 17) / (t_ms * 1e-3) / (5.0e15 * tp), 4) for b, t_ms in ttft_a8.items()}
                                      if ttft_a8 else None),
                  "note": "whole TTFT (scheduler, H2D, every kernel of the bucket, logits D2H, CPU sampler) against the dense MFMA "
-                         "peak of the dtype; prompts are bucket - 17 tokens; flops = 2 (W - lm_head) N + 2 lm_head + 4 L nh hd N^2 / 2 (SURVEY 8d counts the lm_head for every token: 7 % more)"}
+                         "peak of the dtype; prompts are bucket - 17 tokens; flops = 2 (W - lm_head) N + 2 lm_head + 4 L nh hd N^2 / 2"}
 
     label = MODEL_LABEL[args.model]
     wname = {"f8e4m3": "FP8", "int8": "INT8", "bf16": "bf16"}[wd]

@@ -19,7 +19,7 @@ for r in csv.DictReader(open(f)):
 n = sum(len(v) for v in per.values())
 total = sum(sum(v) for v in per.values()) * 1024 * 2
 doc = {
-    "kernel": "mi::gemv_kernel / gemv_priv_kernel (all projections + lm_head of the decode steps in the pass)",
+    "kernel": "mi::gemv_kernel / gemv_priv_kernel / gemv_regs_kernel (all projections + lm_head of the decode steps in the pass)",
     "launches": n,
     "traffic_bytes_per_launch": round(total / n),
     "per_instantiation_median_bytes": {k: round(sorted(v)[len(v) // 2] * 2048) for k, v in per.items()},
