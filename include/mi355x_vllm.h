@@ -451,6 +451,10 @@ int mi_op_rmsnorm(const float* x, const float* g, int32_t T, int32_t H, float ep
 int mi_op_rmsnorm_slabs(const float* resid_in, const float* slab, int32_t KS, const float* scale, const float* bias,
                         const float* row_scale, const float* g, int32_t T, int32_t H, float eps, float* resid_out,
                         void* y_bf16, float* rinv, void* x8, float* x8_scale, void* stream);
+/* The same row over four work-groups, for the few rows of a token-generation step: h = resid_in (+ partial) (+ the slabs' sum), stored to resid_out where it is
+ * given; y = bf16(h * g), and ss[T][4] the sums of squares of h's quarters: the projection applies 1 / rms.  H % 16 == 0, up to 16384. */
+int mi_op_rmsnorm_parts(const float* resid_in, const float* partial, const float* slab, int32_t KS, const float* scale, const float* bias, const float* g,
+                        int32_t T, int32_t H, float* resid_out, void* y_bf16, float* ss, void* stream);
 /* Paged KV write.  k, v [T, nkv, hd] bf16; slots [T] (int64; -1 skips).
  * pool layout (library-native): [2][num_blocks][nkv][block_size][hd] bf16. */
 int mi_op_kv_write(const void* k, const void* v, const int64_t* slots, int32_t T, int32_t nkv,

@@ -78,3 +78,24 @@ def test_sums_of_k_slices(lib, T, H, KS, form, bias, row_scale):  # noqa: F811
     assert ((s8 - ref.abs().amax(-1) / 448).abs() <= 2.0 ** -8 * 1.01 * s8).all()
     got8 = x8.cpu().view(torch.float8_e4m3fn).double().permute(1, 0, 2).reshape(T, H) * s8[:, None]
     assert ((got8 - ref).abs() <= (2.0 ** -4 + 2.0 ** -8) * 1.01 * ref.abs() + 2.0 ** -10 * s8[:, None]).all()      # e4m3 of a bf16; half its least step below 2^-6
+
+
+# the row over four work-groups: one wave and one number a thread of it, the last wave partly idle, sixteen waves; one batch of slabs and two
+@pytest.mark.parametrize("T,H", [(1, 16), (5, 3584), (32, 4096), (3, 4112), (2, 16384)])
+@pytest.mark.parametrize("KS,bias,partial", [(0, False, False), (0, False, True), (1, True, False), (5, False, False), (8, True, False)])
+def test_row_parts(lib, T, H, KS, bias, partial):  # noqa: F811
+    g = torch.Generator().manual_seed(T + H + KS)
+    x, slab, sc = torch.randn(T, H, generator=g) * 3, torch.randn(max(KS, 1), T, H, generator=g), 0.5 + torch.rand(H, generator=g)
+    w, b, p = 1 + 0.1 * torch.randn(H, generator=g), torch.randn(H, generator=g), torch.randn(T, H, generator=g)
+    d = [dev(t) for t in (x, p, slab, sc, b, w)]
+    out, y, ss = torch.full((T, H), float("nan"), device="cuda"), torch.empty(T, H, dtype=torch.bfloat16, device="cuda"), torch.full((T, 4), float("nan"), device="cuda")
+    lib.check(lib.load_library().mi_op_rmsnorm_parts(
+        d[0].data_ptr(), d[1].data_ptr() if partial else None, d[2].data_ptr() if KS else None, KS, d[3].data_ptr(), d[4].data_ptr() if bias else None, d[5].data_ptr(), T, H,
+        out.data_ptr(), y.data_ptr(), ss.data_ptr(), None))
+    torch.cuda.synchronize()
+    h = x.double() + (p.double() if partial else 0) + (slab.double().sum(0) * sc.double() + (b.double() if bias else 0) if KS else 0)
+    assert ((out.cpu().double() - h).abs() <= 2e-6 * (1 + h.abs()) * max(KS, 1)).all()              # KS + 2 fp32 roundings of sums of this size
+    ref = h * w.double()
+    assert ((y.cpu().double() - ref).abs() <= 2.0 ** -8 * 1.01 * ref.abs() + 1e-5 * max(KS, 1)).all()
+    sq = h.reshape(T, 4, H // 4).pow(2).sum(-1)
+    assert ((ss.cpu().double() - sq).abs() <= 1e-5 * sq).all()

@@ -411,7 +411,7 @@ static int launch_gemm_wide_bm(const LinearW& w, int T, const uint16_t* x, int l
                                int KS, float* ws, SlabSum* defer) {
   if (KS > 1) {
     MI_TRY_((launch_gemm_wide_t<WD, EPI_F32, BM, NTW, true>(w, T, x, ldx, e, s, KS, ws)));
-    const SlabSum sum{ws, KS, T, w.N, e.scale, e.bias, e.row_scale};
+    const SlabSum sum{ws, KS, T, w.N, e.scale, e.bias, e.row_scale, e.rs_n, e.rs_eps};
     if (defer && (epi == EPI_RESID || epi == EPI_F32)) { *defer = sum; return MI_OK; }
     return launch_splitk_reduce(sum, epi, e, s);
   }

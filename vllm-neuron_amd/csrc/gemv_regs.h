@@ -52,9 +52,11 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
     }
   }
   __builtin_amdgcn_sched_barrier(0);
-  float rmul[MG];                                     // the row's own factor: 1 / rms where the norm left it to the output
+  RowFactor rfac[MG];                                 // the row's own factor: 1 / rms where the norm left it to the output
+  if constexpr (!SLAB) {
 #pragma unroll
-  for (int mg = 0; mg < MG; ++mg) rmul[mg] = !SLAB && e.row_scale ? e.row_scale[min(mg * 16 + c, M - 1)] : 1.f;
+    for (int mg = 0; mg < MG; ++mg) rfac[mg].request(e.row_scale ? e.row_scale : e.scale, e.row_scale ? min(mg * 16 + c, M - 1) : 0, e.rs_n);
+  }
   // operands of the epilogue of the first row-tile (every wave asks: see gemv_priv_kernel)
   constexpr bool kPre = !SLAB && !(EPI == EPI_QKV && MG == 2);   // (two groups' rotary factors would not fit the registers)
   EpiPre<kPre ? EPI : EPI_F32> epre[MG];
@@ -98,6 +100,9 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
     }
   }
   issue(bufB, 1);
+  float rmul[MG];
+#pragma unroll
+  for (int mg = 0; mg < MG; ++mg) rmul[mg] = !SLAB && e.row_scale ? rfac[mg].value(e.rs_n, e.rs_eps) : 1.f;
 
   f32x4_t acc[MG];
 #pragma unroll
@@ -246,7 +251,7 @@ int launch_gemv_regs_wd(const LinearW& w, int M, const uint16_t* x, int ldx, int
   MI_CHECK(slices > 0, "gemv_regs: no split of K fits the workspace");
   if (slices > 1) {
     MI_TRY_(M <= 16 ? (launch_gemv_regs_k<WD, EPI_F32, 1, true>(w, M, x, ldx, e, s, slices, ws)) : (launch_gemv_regs_k<WD, EPI_F32, 2, true>(w, M, x, ldx, e, s, slices, ws)));
-    const SlabSum sum{ws, slices, M, w.N, e.scale, e.bias, e.row_scale};
+    const SlabSum sum{ws, slices, M, w.N, e.scale, e.bias, e.row_scale, e.rs_n, e.rs_eps};
     if (deferred) { *defer = sum; return MI_OK; }
     return launch_splitk_reduce(sum, epi, e, s);
   }

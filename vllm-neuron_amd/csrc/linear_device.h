@@ -28,7 +28,9 @@ template <int EPI>
 __device__ __forceinline__ void epilogue(const EpiArgs& e, int m, int n0, f32x4_t v) {
   float4 sc = *reinterpret_cast<const float4*>(e.scale + n0);
   if (e.row_scale) {   // FP8 activations: the token's scale multiplies the channel's
-    const float rs = e.row_scale[m];
+    RowFactor f;
+    f.request(e.row_scale, m, e.rs_n);
+    const float rs = f.value(e.rs_n, e.rs_eps);
     sc.x *= rs; sc.y *= rs; sc.z *= rs; sc.w *= rs;
   }
   v[0] *= sc.x; v[1] *= sc.y; v[2] *= sc.z; v[3] *= sc.w;
@@ -249,6 +251,14 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& e, int T, int NT, i
   };
   Operands ops[2];
   request(ops[0], 0);
+  if (e.rs_n > 0.f) {       // (calls of few rows)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      RowFactor f;
+      f.request(e.row_scale, mb + row(mt), e.rs_n);
+      rs[mt] = f.value(e.rs_n, e.rs_eps);
+    }
+  }
 #pragma unroll
   for (int i = 0; i < NTW; ++i) {
     if (i + 1 < NTW) request(ops[(i + 1) & 1], i + 1);

@@ -14,6 +14,7 @@ enum { PRO_BF16 = 0, PRO_NORM = 1, PRO_NORM_PARTIAL = 2 };  // callers pass PRO_
 struct EpiArgs {
   const float* scale;  // [N] per-output-row dequant scale
   const float* row_scale;  // [M] factor per row (per-token activation scale of the FP8-activation GEMM; launch_gemv_regs) or nullptr
+  float rs_n, rs_eps;      // rs_n > 0: row_scale holds [M][kNormParts] sums of squares of rows of rs_n numbers, the factor is 1 / rms (launch_norm_parts)
   const float* bias;   // [N] or nullptr
   // EPI_F32: out[m * ld_out + n] = y;  EPI_RESID: out = resid_in[m * ld_out + n] + y
   float* out_f32;
@@ -65,7 +66,7 @@ struct LinearW {
 int launch_gemv(const LinearW& w, int M, int pro, const ProArgs& p, int epi, const EpiArgs& e,
                 hipStream_t s);
 // The same for up to 32 rows of bf16 activations, with those in registers (gemv_regs.h).  ws: room for the slabs of a split K; defer as launch_gemm.
-// EpiArgs::row_scale: a factor per row of the product (1 / rms where launch_norm_rows left it out).
+// EpiArgs::row_scale: a factor per row of the product (1 / rms where the norm left it out).
 int launch_gemv_regs(const LinearW& w, int M, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s, float* ws, size_t ws_bytes,
                      SlabSum* defer = nullptr, bool split_as_deferred = false);
 // whether M rows of w take it (K beyond 8 slices of the registers, or slabs that do not fit: launch_gemv up to 16 rows, launch_gemm)

@@ -687,10 +687,11 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   EpiPre<EPI> pre;
   epi_prefetch<EPI>(e, m, n0, pre);
   const float4 sc = *reinterpret_cast<const float4*>(e.scale + n0), bi = e.bias ? *reinterpret_cast<const float4*>(e.bias + n0) : make_float4(0.f, 0.f, 0.f, 0.f);
-  const float rs = e.row_scale ? e.row_scale[m] : 1.f;
+  RowFactor rf;
+  rf.request(e.row_scale ? e.row_scale : e.scale, e.row_scale ? m : 0, e.rs_n);
   const float4 v = slab_sum4(slab + (size_t)m * N + n0, (size_t)T * N, KS, [&] { epi_prefetch_dependent<EPI>(e, n0, pre); });
   const float sc4[4] = {sc.x, sc.y, sc.z, sc.w}, b4[4] = {bi.x, bi.y, bi.z, bi.w};
-  epilogue_pre<EPI>(e, m, n0, sc4, e.bias ? b4 : nullptr, f32x4_t{v.x, v.y, v.z, v.w}, pre, rs);
+  epilogue_pre<EPI>(e, m, n0, sc4, e.bias ? b4 : nullptr, f32x4_t{v.x, v.y, v.z, v.w}, pre, e.row_scale ? rf.value(e.rs_n, e.rs_eps) : 1.f);
 }
 
 int launch_splitk_reduce(const SlabSum& sl, int epi, const EpiArgs& e, hipStream_t s) {
@@ -708,7 +709,7 @@ int launch_splitk_reduce(const SlabSum& sl, int epi, const EpiArgs& e, hipStream
 // sum a deferred K-split (SlabSum) the plain way: splitk_reduce + residual epilogue
 int launch_splitk_flush(const SlabSum& sl, const float* resid_in, float* out, int ld_out, hipStream_t s) {
   EpiArgs e{};
-  e.scale = sl.scale; e.bias = sl.bias; e.row_scale = sl.row_scale;
+  e.scale = sl.scale; e.bias = sl.bias; e.row_scale = sl.row_scale; e.rs_n = sl.rs_n; e.rs_eps = sl.rs_eps;
   e.out_f32 = out; e.resid_in = resid_in; e.ld_out = ld_out;
   hipLaunchKernelGGL((splitk_reduce_kernel<EPI_RESID>), dim3(ceil_div(sl.T * (sl.N / 4), 256)), dim3(256), 0, s, sl.slab, sl.KS,
                      sl.T, sl.N, e);

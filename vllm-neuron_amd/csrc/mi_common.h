@@ -180,8 +180,22 @@ struct SlabSum {
   const float* scale = nullptr;     // [N]
   const float* bias = nullptr;      // [N] or null
   const float* row_scale = nullptr; // [T] or null (FP8 activations)
+  float rs_n = 0.f, rs_eps = 0.f;   // as EpiArgs
 };
+constexpr int kNormParts = 4;       // work-groups of a row in norm_parts_kernel, each with a sum of squares of its own
 #ifdef __HIPCC__
+// A row's factor: p[m], or (n > 0) 1 / rms of a row of n numbers from its parts' sums of squares p[kNormParts m ..].  Requests without a branch: what they stand
+// behind stays in flight.
+struct RowFactor {
+  float a, b, c, d;
+  __device__ __forceinline__ void request(const float* p, int m, float n) {
+    const bool parts = n > 0.f;
+    const float* q = p + (parts ? kNormParts * m : m);
+    const int step = parts ? 1 : 0;
+    a = q[0]; b = q[step]; c = q[2 * step]; d = q[3 * step];
+  }
+  __device__ __forceinline__ float value(float n, float eps) const { return n > 0.f ? rsqrtf(((a + b) + (c + d)) / n + eps) : a; }
+};
 // The sum of KS slabs' four numbers at p, `stride` numbers apart, in slice order.  Five requests leave before the first is waited for: one after the
 // other they cost a trip to memory each (the row norm over 8 slabs of 242 x 4096: 13.9 us that way, 9.3 now, of which the bytes take 6.3).
 struct Nothing { __device__ __forceinline__ void operator()() const {} };

@@ -157,6 +157,51 @@ __global__ __launch_bounds__(1024) void norm_rows_kernel(const float* __restrict
     }
   }
 }
+// The same for the few rows of a token-generation step, the row over kNormParts work-groups: a CU takes in some 35 GB/s of a row and its slabs (32 rows of 4096 behind
+// 8 slabs: 147 KB a work-group, 5.8 us a launch; 4.7 so, which is what the smallest launch takes that reads what others wrote: 5 rows 4.8 and 4.6).  Each leaves the sum of its squares; whoever takes the rows adds them up and applies 1 / rms
+// (RowFactor), so that what is rounded to bf16 is h * gain.
+__global__ __launch_bounds__(1024) void norm_parts_kernel(const float* __restrict__ resid_in, const float* __restrict__ partial, float* __restrict__ resid_out,
+                                                         const float* __restrict__ gain, int H, uint16_t* __restrict__ y, float* __restrict__ ss_out, SlabSum sl) {
+  __shared__ float red[16];
+  const int t = blockIdx.y, part = blockIdx.x, tid = threadIdx.x, mine = H / kNormParts;
+  const bool in = tid * 4 < mine;
+  const int col = part * mine + (in ? tid * 4 : 0);
+  const size_t o = (size_t)t * H + col;
+  const float4 g = *reinterpret_cast<const float4*>(gain + col);
+  float4 a = *reinterpret_cast<const float4*>(resid_in + o);
+  if (partial) {
+    const float4 p = *reinterpret_cast<const float4*>(partial + o);
+    a.x += p.x; a.y += p.y; a.z += p.z; a.w += p.w;
+  }
+  if (sl.slab) {
+    float4 sc = *reinterpret_cast<const float4*>(sl.scale + col), bb = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (sl.bias) bb = *reinterpret_cast<const float4*>(sl.bias + col);
+    const float rs = sl.row_scale ? sl.row_scale[t] : 1.f;
+    float4 v = slab_sum4(sl.slab + (size_t)t * sl.N + col, (size_t)sl.T * sl.N, sl.KS);
+    if (sl.row_scale) { sc.x *= rs; sc.y *= rs; sc.z *= rs; sc.w *= rs; }
+    v.x *= sc.x; v.y *= sc.y; v.z *= sc.z; v.w *= sc.w;
+    if (sl.bias) { v.x += bb.x; v.y += bb.y; v.z += bb.z; v.w += bb.w; }
+    a.x += v.x; a.y += v.y; a.z += v.z; a.w += v.w;
+  }
+  if (in) {
+    if (resid_out) *reinterpret_cast<float4*>(resid_out + o) = a;
+    *reinterpret_cast<uint2*>(y + o) = make_uint2(pack_bf16x2(a.x * g.x, a.y * g.y), pack_bf16x2(a.z * g.z, a.w * g.w));
+  }
+  float ss = wave_sum(in ? a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w : 0.f);
+  if ((tid & 63) == 0) red[tid >> 6] = ss;
+  __syncthreads();
+  if (tid) return;
+  for (int w = 1; w < (int)blockDim.x >> 6; ++w) ss += red[w];
+  ss_out[t * kNormParts + part] = ss;
+}
+bool norm_parts_fit(int H) { return H % (4 * kNormParts) == 0 && H <= 1024 * 4 * kNormParts; }
+int launch_norm_parts(const float* resid_in, const float* partial, float* resid_out, const float* gain, int T, int H, uint16_t* y, float* ss, hipStream_t s, const SlabSum* slabs) {
+  MI_CHECK(norm_parts_fit(H) && T >= 1 && T <= 65535, "rmsnorm: a float4 per thread of four work-groups a row");
+  MI_CHECK(!slabs || (slabs->T == T && slabs->N == H && resid_out && slabs->rs_n == 0.f), "rmsnorm: pending K-split sum of another shape");
+  hipLaunchKernelGGL(norm_parts_kernel, dim3(kNormParts, T), dim3(ceil_div(H / kNormParts, 256) * 64), 0, s, resid_in, partial, resid_out, gain, H, y, ss, slabs ? *slabs : SlabSum());
+  MI_HIP(hipGetLastError());
+  return MI_OK;
+}
 // up to 512 rows (two per CU): a float4 per thread, one round of requests; more rows: 256 threads, several rows per CU
 static int norm_threads(int T, int H) { return T <= 512 ? std::min(1024, ceil_div(H / 4, 64) * 64) : 256; }
 int launch_norm_rows(const float* resid_in, const float* partial, float* resid_out, const float* gain, int T,

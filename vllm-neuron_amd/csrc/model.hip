@@ -110,7 +110,11 @@ int run_linear(mi_ctx* c, const Linear& L, int rows, int pro, ProArgs p, int epi
   const uint16_t* x = p.x;
   int ldx = p.ldx;
   const bool a8 = rows > 32 && c->cfg.prefill_fp8_activations && gemm_a8_supported(L.view());   // (prompts' option: rows a token-generation batch can have keep bf16)
-  if (regs && pro == PRO_NORM) e.row_scale = c->row_rinv;
+  const bool parts = regs && norm_parts_fit(L.K);
+  if (regs && pro == PRO_NORM) {
+    e.row_scale = c->row_rinv;
+    if (parts) { e.rs_n = (float)L.K; e.rs_eps = p.eps; }
+  }
   if (pro == PRO_NORM && !c->runs(MI_K_OTHER)) {   // (class-masked replay: what the norm would have left)
     x = c->xn;
     ldx = L.K;
@@ -133,6 +137,10 @@ int run_linear(mi_ctx* c, const Linear& L, int rows, int pro, ProArgs p, int epi
     }
     if (a8) {   // norm and per-token quantization in one pass over the row
       MI_TRY(launch_norm_rows_fp8(rin, p.partial, rout, p.gain, rows, L.K, p.eps, c->x8, c->x8_scale, c->stream, slabs));
+    } else if (parts) {
+      MI_TRY(launch_norm_parts(rin, p.partial, rout, p.gain, rows, L.K, c->xn, c->row_rinv, c->stream, slabs));
+      x = c->xn;
+      ldx = L.K;
     } else {
       MI_TRY(launch_norm_rows(rin, p.partial, rout, p.gain, rows, L.K, p.eps, c->xn, c->stream, slabs, regs ? c->row_rinv : nullptr));
       x = c->xn;
@@ -1243,7 +1251,7 @@ int mi_finalize(mi_ctx* c) {
     MI_TRY(dmalloc(&c->x8_scale, R, ws));
   }
   }
-  MI_TRY(dmalloc(&c->row_rinv, 32, ws));
+  MI_TRY(dmalloc(&c->row_rinv, 32 * kNormParts, ws));
   c->splitk_ws_bytes = (size_t)64 << 20;   // fp32 K-slice slabs of the short-prompt GEMMs
   MI_TRY(dmalloc(&c->splitk_ws, c->splitk_ws_bytes / 4, ws));
   MI_TRY(dmalloc(&c->logits, (size_t)k.max_num_seqs * c->V_l, ws));
@@ -2250,6 +2258,12 @@ int mi_op_rmsnorm_slabs(const float* resid_in, const float* slab, int32_t KS, co
   const SlabSum sum{slab, KS, T, H, scale, bias, row_scale};
   if (y) return launch_norm_rows(resid_in, nullptr, resid_out, g, T, H, eps, reinterpret_cast<uint16_t*>(y), (hipStream_t)stream, &sum, rinv);
   return launch_norm_rows_fp8(resid_in, nullptr, resid_out, g, T, H, eps, reinterpret_cast<uint8_t*>(x8), x8_scale, (hipStream_t)stream, &sum);
+}
+int mi_op_rmsnorm_parts(const float* resid_in, const float* partial, const float* slab, int32_t KS, const float* scale, const float* bias, const float* g, int32_t T,
+                        int32_t H, float* resid_out, void* y, float* ss, void* stream) {
+  MI_CHECK(resid_in && g && T >= 1 && H >= 16 && y && ss && (!slab || (KS >= 1 && scale && resid_out)), "bad argument");
+  const SlabSum sum{slab, KS, T, H, scale, bias};
+  return launch_norm_parts(resid_in, partial, resid_out, g, T, H, reinterpret_cast<uint16_t*>(y), ss, (hipStream_t)stream, slab ? &sum : nullptr);
 }
 int mi_op_kv_write(const void* k, const void* v, const int64_t* slots, int32_t T, int32_t nkv, int32_t hd, void* pool,
                    int32_t num_blocks, int32_t block_size, void* stream) {
