@@ -26,3 +26,23 @@ def test_edges_of_columns(lib, shape):  # noqa: F811
         close(*x.step([(0, 40), (1, 17), (2, 2)], f32), f32)
         for i in range(3):
             x.check_state(i)
+
+
+# one long segment in two parts at the same time: the shortest that goes so, second parts of 0 .. 3 chunks by themselves and a ragged last one, one and two channel tiles a
+# wave with waves idle and not; the next segment starts from the joined state
+@pytest.mark.parametrize("shape", [(2, 2, 128, 128, 4), (16, 16, 128, 128, 4), (3, 1, 80, 80, 3), (4, 2, 64, 64, 2), (2, 1, 20, 20, 4), (1, 1, 7, 16, 1)])
+@pytest.mark.parametrize("first,second", [(1008, 1024), (1024, 1056), (1025, 1071), (1055, 1036), (1500, 2)])
+def test_long_segments_in_two_parts(lib, shape, first, second):  # noqa: F811
+    x = Delta(lib, *shape, [first + second], seed=sum(shape) + first, strong=shape[0] == 4)
+    close(*x.step([(0, first)], chunks=256), 1)
+    close(*x.step([(0, second)], 0, chunks=256), 0)
+    x.check_state(0)
+
+
+# pieces of a segment that the workspace holds: two of them in two parts, the rest not; beside it a sequence too short, and with another one neither goes in parts
+@pytest.mark.parametrize("lengths,chunks", [([2300], 70), ([1100, 40], 256), ([1100], 63)])
+def test_parts_and_pieces(lib, lengths, chunks):  # noqa: F811
+    x = Delta(lib, 4, 4, 128, 128, 4, lengths, seed=len(lengths) + chunks)
+    close(*x.step([(i, n) for i, n in enumerate(lengths)], chunks=chunks), 1)
+    for i in range(len(lengths)):
+        x.check_state(i)

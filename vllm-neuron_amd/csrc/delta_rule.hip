@@ -580,35 +580,19 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(DeltaGeom g, float* __r
 // 108 us; half the chip's CUs have no work-group, and a head's state cannot be split further).  The second chunk's u needs the first one's state
 // S1 = e1 S + K1' u1, so with W2 e1 in place of W2 its product with S joins the first chunk's, and what is missing is (-W2 K1') u1, a 16 x 16 matrix
 // that does not depend on the state: it is made one pair ahead, while the partial sums of u come out of LDS.  One meeting and 64 products per
-// pair: 1.46 us, 94 us.  Two pairs of chunks are in registers; a load of the pair after the next is issued as soon as what it replaces is used up.
+// pair: 1.46 us, 94 us.  Two pairs of chunks are in registers (248: a bound of two waves a SIMD keeps the compiler from moving some to the other file and back, 99 -> 96 us); a load of the pair after the next is issued as soon as what it replaces is used up.
 // (Its own set of registers for a third pair, or the first chunk's o behind the barrier: 115 and 98 us.)
 constexpr int kOutside = 0x7fff0000;      // beyond any buffer of records
 template <typename F, int... I> __device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F&& f) { (f(std::integral_constant<int, I>()), ...); }
 template <int N, typename F> __device__ __forceinline__ void each(F&& f) { each_of(std::make_integer_sequence<int, N>(), f); }
 
-template <int NT>
-__global__ __launch_bounds__(256) void delta_scan_pairs_kernel(DeltaGeom g, float* __restrict__ state, const int32_t* __restrict__ slots,
-                                                               const AttnSeg* __restrict__ segs, int c0, int nchunks, int nvt, float* __restrict__ records) {
-  __shared__ f32x4_t ps[2][5][4][64];      // o of the pair before (two chunks), G, u1, what u2 has without G u1
-  int id = blockIdx.x, h, vt;
-  if (g.H % 8 == 0) {        // the column blocks of a head on one XCD: they read the same factors
-    const int k = id >> 3;
-    h = (id & 7) + 8 * (k / nvt);
-    vt = k % nvt;
-  } else {
-    h = id / nvt;
-    vt = id % nvt;
-  }
-  const int si = blockIdx.y;
-  const AttnSeg sg = segs[si];
-  if (sg.n < 2) return;
-  int first = 0;             // the segment's first chunk among all
-  for (int i = 0; i < si; ++i) first += segs[i].n < 2 ? 0 : ceil_div(segs[i].n, kC);
-  const int k0 = max(c0 - first, 0), k1 = min(c0 + nchunks - first, ceil_div(sg.n, kC));
-  if (k0 >= k1) return;
+// The 16 columns vt of a head over n chunks from `base` on.  REPLY (the second part of a segment, delta_scan_split_kernel): columns of the identity in place of a
+// state and no values; what they answer goes to `replies`, their last state is the product of the chunks' transitions.
+using PairParts = f32x4_t[5][4][64];       // o of the pair before (two chunks), G, u1, what u2 has without G u1
+template <int NT, bool REPLY, typename Load, typename Store>
+__device__ __forceinline__ void delta_scan_pairs(PairParts* ps, const DeltaGeom& g, float* base, int n, int vt, float* replies, Load&& load_state, Store&& store_state) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g4 = lane >> 4, c = lane & 15, tiles = g.dkp / 16;
-  const int n = k1 - k0, pairs = n / 4 * 2;      // pairs of chunks, an even number of them; up to three chunks by themselves
-  float* S0 = state + ((size_t)slots[sg.seq] * g.H + h) * g.dkp * g.dvp + vt * 16 + c;
+  const int pairs = n / 4 * 2;                   // pairs of chunks, an even number of them; up to three chunks by themselves
   struct Chunk { f32x4_t w[NT], q[NT], k[NT], e[NT]; float t, m, x; };
   struct Pair { Chunk a, b; };
   f32x4_t kt[NT];            // K' of the next pair's first chunk, with a token per lane
@@ -616,8 +600,9 @@ __global__ __launch_bounds__(256) void delta_scan_pairs_kernel(DeltaGeom g, floa
   // The records of this segment's chunks as a buffer: a load is one instruction (lane offsets that do not change, a scalar one per chunk), and tiles
   // past the last one lie outside of it, so that they read as zero and their part of S stays zero.
   const size_t rec = record_floats(g.dkp, g.dvp) * sizeof(float);
-  float* const base = records + ((size_t)h * nchunks + (first + k0 - c0)) * (rec / sizeof(float));
-  const auto buf = __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)((k1 - k0) * rec), 0x00020000);
+  const auto buf = __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)(n * rec), 0x00020000);
+  const int reply = 16 * g.dkp * (int)sizeof(float);
+  const auto rbuf = __builtin_amdgcn_make_buffer_rsrc(replies, 0, REPLY ? n * reply : 0, 0x00020000);
   const int region = 16 * g.dkp * (int)sizeof(float);
   int woff[NT], qoff[NT], koff[NT], eoff[NT], ktoff[NT];
   bool live[NT];
@@ -631,7 +616,7 @@ __global__ __launch_bounds__(256) void delta_scan_pairs_kernel(DeltaGeom g, floa
     ktoff[t] = live[t] ? 2 * region + (tile * 256 + 4 * g4 * 16 + c) * 4 : kOutside;
     eoff[t] = live[t] ? 3 * region + (tile * 16 + 4 * g4) * 4 : kOutside;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) S[t][r] = sg.pos0 + k0 > 0 && live[t] ? S0[(size_t)(tile * 16 + 4 * g4 + r) * g.dvp] : 0.f;
+    for (int r = 0; r < 4; ++r) S[t][r] = live[t] ? load_state(tile * 16 + 4 * g4 + r, vt * 16 + c) : 0.f;
   }
   const int rest = 49 * g.dkp * (int)sizeof(float), toff = rest + (c * 16 + 4 * wave + g4) * 4, values = rest + 2048 + vt * 1024;
   const int xoff = values + ((4 * wave + g4) * 16 + c) * 4, ooff = values + ((4 * g4 + wave) * 16 + c) * 4;
@@ -642,9 +627,9 @@ __global__ __launch_bounds__(256) void delta_scan_pairs_kernel(DeltaGeom g, floa
   auto load_q = [&](int F, Chunk& f, int t) { f.q[t] = load4(qoff[t], F); };
   auto load_k = [&](int F, Chunk& f, int t) { f.k[t] = load4(koff[t], F); };
   auto load_e = [&](int F, Chunk& f, int t) { f.e[t] = load4(eoff[t], F); };
-  auto load_t = [&](int F, Chunk& f) { f.t = load1(toff, F); };
-  auto load_m = [&](int F, Chunk& f) { f.m = load1(toff + 1024, F); };
-  auto load_x = [&](int F, Chunk& f) { f.x = load1(xoff, F); };
+  auto load_t = [&](int F, Chunk& f) { if constexpr (!REPLY) f.t = load1(toff, F); };
+  auto load_m = [&](int F, Chunk& f) { if constexpr (!REPLY) f.m = load1(toff + 1024, F); };
+  auto load_x = [&](int F, Chunk& f) { if constexpr (!REPLY) f.x = load1(xoff, F); };
   auto load_kt = [&](int F, int t) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) kt[t][r] = load1(ktoff[t] + r * 64, F);
@@ -673,7 +658,13 @@ __global__ __launch_bounds__(256) void delta_scan_pairs_kernel(DeltaGeom g, floa
     return f32x4_t{po[0], po[256], po[512], po[768]};
   };
   auto all4 = [](f32x4_t v) { return v[0] + v[1] + v[2] + v[3]; };
-  auto put_out = [&](int k, float v) { __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), buf, ooff, __builtin_amdgcn_readfirstlane(record(k)), 0); };      // in place of the chunk's values
+  const int roff = (vt * 256 + (4 * g4 + wave) * 16 + c) * 4;
+  auto put_out = [&](int k, float v) {
+    if constexpr (REPLY) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rbuf, roff, __builtin_amdgcn_readfirstlane(k * reply), 0);
+    else __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), buf, ooff, __builtin_amdgcn_readfirstlane(record(k)), 0);      // in place of the chunk's values
+  };
+  // (REPLY: no values, so no products with them)
+  auto with_values = [&](float m, float x, f32x4_t& acc) { if constexpr (!REPLY) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(m, x, acc, 0, 0, 0); };
   auto coupling = [&](const Chunk& second, auto&& between) {      // this wave's part of (-W2 K1')^T: what it leaves in a lane is the A operand of G u1
     f32x4_t gt = {0.f, 0.f, 0.f, 0.f};
     each<4 * NT>([&](auto i) {
@@ -705,8 +696,8 @@ __global__ __launch_bounds__(256) void delta_scan_pairs_kernel(DeltaGeom g, floa
       if (r == 3) { load_w(B, now.b, t); load_w(A, now.a, t); }
       pin();
     });
-    u1 = __builtin_amdgcn_mfma_f32_16x16x4f32(now.a.t, now.a.x, u1, 0, 0, 0);
-    u2 = __builtin_amdgcn_mfma_f32_16x16x4f32(now.b.t, now.b.x, u2, 0, 0, 0);
+    with_values(now.a.t, now.a.x, u1);
+    with_values(now.b.t, now.b.x, u2);
     ps[b][3][wave][lane] = u1;
     ps[b][4][wave][lane] = u2;
     pin();
@@ -721,7 +712,7 @@ __global__ __launch_bounds__(256) void delta_scan_pairs_kernel(DeltaGeom g, floa
       if (r == 3) load_q(A, now.a, t);
       pin();
     });
-    o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(now.a.m, now.a.x, o1, 0, 0, 0);
+    with_values(now.a.m, now.a.x, o1);
 #pragma unroll
     for (int t = 0; t < NT; ++t) Sg[t] = f32x4_t{S[t][0] * now.a.e[t][0], S[t][1] * now.a.e[t][1], S[t][2] * now.a.e[t][2], S[t][3] * now.a.e[t][3]};
     meet();
@@ -769,7 +760,7 @@ __global__ __launch_bounds__(256) void delta_scan_pairs_kernel(DeltaGeom g, floa
       if (r == 1) load_k(B, now.b, t);
       pin();
     });
-    o2 = __builtin_amdgcn_mfma_f32_16x16x4f32(now.b.m, xb, o2, 0, 0, 0);
+    with_values(now.b.m, xb, o2);
     if (p > 0) {
       put_out(2 * p - 2, out1);
       put_out(2 * p - 1, out2);
@@ -804,8 +795,8 @@ __global__ __launch_bounds__(256) void delta_scan_pairs_kernel(DeltaGeom g, floa
         u = __builtin_amdgcn_mfma_f32_16x16x4f32(f.w[t][r], S[t][r], u, 0, 0, 0);
         o = __builtin_amdgcn_mfma_f32_16x16x4f32(f.q[t][r], S[t][r], o, 0, 0, 0);
       }
-    u = __builtin_amdgcn_mfma_f32_16x16x4f32(f.t, f.x, u, 0, 0, 0);
-    o = __builtin_amdgcn_mfma_f32_16x16x4f32(f.m, f.x, o, 0, 0, 0);
+    with_values(f.t, f.x, u);
+    with_values(f.m, f.x, o);
     ps[b][3][wave][lane] = u;
     ps[b][4][wave][lane] = o;
     __syncthreads();
@@ -823,24 +814,149 @@ __global__ __launch_bounds__(256) void delta_scan_pairs_kernel(DeltaGeom g, floa
   if (2 * pairs + 2 < n) single(2 * pairs + 2, 0, f[1].a);
 #pragma unroll
   for (int t = 0; t < NT; ++t)
+    if (live[t]) store_state(wave * NT + t, S[t]);
+}
+
+// the head and block of value columns of work-group id among H nvt: the column blocks of a head on one XCD, they read the same factors
+__device__ __forceinline__ void scan_columns(const DeltaGeom& g, int id, int nvt, int& h, int& vt) {
+  if (g.H % 8 == 0) {
+    const int k = id >> 3;
+    h = (id & 7) + 8 * (k / nvt);
+    vt = k % nvt;
+  } else {
+    h = id / nvt;
+    vt = id % nvt;
+  }
+}
+
+template <int NT>
+__global__ __launch_bounds__(256, 2) void delta_scan_pairs_kernel(DeltaGeom g, float* __restrict__ state, const int32_t* __restrict__ slots,
+                                                               const AttnSeg* __restrict__ segs, int c0, int nchunks, int nvt, float* __restrict__ records) {
+  __shared__ PairParts ps[2];
+  int h, vt;
+  scan_columns(g, blockIdx.x, nvt, h, vt);
+  const int si = blockIdx.y;
+  const AttnSeg sg = segs[si];
+  if (sg.n < 2) return;
+  int first = 0;             // the segment's first chunk among all
+  for (int i = 0; i < si; ++i) first += segs[i].n < 2 ? 0 : ceil_div(segs[i].n, kC);
+  const int k0 = max(c0 - first, 0), k1 = min(c0 + nchunks - first, ceil_div(sg.n, kC));
+  if (k0 >= k1) return;
+  const int lane = threadIdx.x & 63;
+  float* S0 = state + ((size_t)slots[sg.seq] * g.H + h) * g.dkp * g.dvp;
+  const bool begun = sg.pos0 + k0 > 0;
+  delta_scan_pairs<NT, false>(ps, g, records + ((size_t)h * nchunks + (first + k0 - c0)) * record_floats(g.dkp, g.dvp), k1 - k0, vt, nullptr,
+                          [&](int d, int v) { return begun ? S0[(size_t)d * g.dvp + v] : 0.f; },
+                          [&](int tile, const f32x4_t& s) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (live[t]) S0[(size_t)((wave * NT + t) * 16 + 4 * g4 + r) * g.dvp] = S[t][r];
+                            for (int r = 0; r < 4; ++r) S0[(size_t)(tile * 16 + 4 * (lane >> 4) + r) * g.dvp + vt * 16 + (lane & 15)] = s[r];
+                          });
+}
+
+// One long segment on a chip whose CUs the kernel above leaves half idle: its chunks in two parts at the same time.  The transition of a chunk is linear in the state:
+// with S1 the state between the parts, an output of the second one is the output from a state of zeros plus q^T (the product of the transitions so far) S1, and that
+// row of replies is what the same recurrence makes of the columns of the identity.  So the second part has two work-groups for 16 columns, which share a CU and take 2.7 us
+// a pair between them (fp32 matrix products leave no room for vector instructions beside them: 32 cycles and 5 - 9 for each of those), and it is the shorter one; the order of the
+// work-groups puts both on the CUs that the first part leaves.  delta_out_kernel adds replies S1 and makes the last state.  Everything stays fp32.
+// 16 heads of 128, 2048 tokens, us: scan 98 -> 68, output norm 15.5 -> 28; 4000 tokens 3988 -> 3639 a call.
+// Behind the records: [chunk][16 dkp] replies a head, those of the first part unused: there the states, S1 as fragments, the second part's own (L) and its transition (P).
+constexpr int kSplitChunks = 64;                 // of a segment at least: room for the three states, and below the joining costs what the halves save (us a call, one scan -> two: 900 tokens 1202 -> 1213, 1100 1395 -> 1359)
+__host__ __device__ __forceinline__ int split_first(int n) { return (n * 41 + 127) / 256 * 4; }     // chunks of the first part: 0.64 of them, whole turns of the loop
+struct SplitMem { float *replies, *s1, *l, *p; };
+__host__ __device__ __forceinline__ SplitMem split_mem(float* records, const DeltaGeom& g, int n, int h) {
+  float* r = records + (size_t)g.H * n * record_floats(g.dkp, g.dvp) + (size_t)h * n * 16 * g.dkp;
+  return SplitMem{r, r, r + g.dkp * g.dvp, r + 2 * g.dkp * g.dvp};
+}
+template <int NT>
+__global__ __launch_bounds__(256, 2) void delta_scan_split_kernel(DeltaGeom g, const float* __restrict__ state, const int32_t* __restrict__ slots,
+                                                                  const AttnSeg* __restrict__ segs, int c0, int n, int nvt, float* __restrict__ records) {
+  __shared__ PairParts ps[2];
+  const int cols = g.H * nvt, slot = (int)blockIdx.x / cols, part = slot == 0 ? 1 : slot == 1 ? 0 : 2, first = split_first(n), lane = threadIdx.x & 63, g4 = lane >> 4, c = lane & 15;
+  int h, vt;
+  scan_columns(g, (int)blockIdx.x - slot * cols, nvt, h, vt);
+  const AttnSeg sg = segs[0];
+  const SplitMem m = split_mem(records, g, n, h);
+  float* base = records + (size_t)h * n * record_floats(g.dkp, g.dvp);
+  auto put = [&](float* to, int tile, const f32x4_t& s) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) to[(size_t)(tile * 16 + 4 * g4 + r) * g.dvp + vt * 16 + c] = s[r];
+  };
+  if (part < 2) {
+    const float* S0 = state + ((size_t)slots[sg.seq] * g.H + h) * g.dkp * g.dvp;
+    const bool begun = part == 0 && sg.pos0 + c0 > 0;
+    const int at = part ? first : 0;
+    delta_scan_pairs<NT, false>(ps, g, base + (size_t)at * record_floats(g.dkp, g.dvp), part ? n - first : first, vt, nullptr,
+                                [&](int d, int v) { return begun ? S0[(size_t)d * g.dvp + v] : 0.f; },
+                                [&](int tile, const f32x4_t& s) {
+                                  if (part) put(m.l, tile, s);
+                                  else *reinterpret_cast<f32x4_t*>(m.s1 + ((vt * (g.dkp / 16) + tile) * 64 + lane) * 4) = s;
+                                });
+  } else {
+    delta_scan_pairs<NT, true>(ps, g, base + (size_t)first * record_floats(g.dkp, g.dvp), n - first, vt, m.replies + (size_t)first * 16 * g.dkp,
+                               [&](int d, int v) { return d == v ? 1.f : 0.f; }, [&](int tile, const f32x4_t& s) { put(m.p, tile, s); });
+  }
+}
+// the state behind a segment in two parts: L + P S1, a wave per 16 x 16 tile
+__device__ __forceinline__ void delta_join(const DeltaGeom& g, float* __restrict__ state, int slot, int n, float* __restrict__ records, int at) {
+  const int tiles = g.dkp / 16, lane = threadIdx.x & 63, g4 = lane >> 4, c = lane & 15, h = at / (tiles * tiles), rt = at / tiles % tiles, ct = at % tiles;
+  if (h >= g.H) return;
+  const SplitMem m = split_mem(records, g, n, h);
+  const float* l = m.l + (size_t)(rt * 16 + 4 * g4) * g.dvp + ct * 16 + c;
+  f32x4_t s = {l[0], l[g.dvp], l[2 * g.dvp], l[3 * g.dvp]};
+  for (int t = 0; t < tiles; ++t) {
+    const f32x4_t p = *reinterpret_cast<const f32x4_t*>(m.p + (size_t)(rt * 16 + c) * g.dvp + t * 16 + 4 * g4), s1 = *reinterpret_cast<const f32x4_t*>(m.s1 + ((ct * tiles + t) * 64 + lane) * 4);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s = __builtin_amdgcn_mfma_f32_16x16x4f32(p[r], s1[r], s, 0, 0, 0);
+  }
+  float* to = state + ((size_t)slot * g.H + h) * g.dkp * g.dvp + (size_t)(rt * 16 + 4 * g4) * g.dvp + ct * 16 + c;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) to[(size_t)r * g.dvp] = s[r];
 }
 
 // Norm and gate: a wave per head and chunk, a lane four columns of every value tile of one token, all of them requested together; the work-groups of a
 // segment's last chunk renew its ring.  WIDE: rows of z and y in 16 and 8 bytes.  Bound by memory: 16 heads of 128, 2048 tokens, 42 MB in 16.3 us (19.5 with
 // a lane per column and eight tokens after each other).
-template <typename T, int NT, bool WIDE>
-__global__ __launch_bounds__(256) void delta_out_kernel(DeltaGeom g, DeltaIn in, const AttnSeg* __restrict__ segs, int nseg, int c0, float* __restrict__ records,
+// SPLIT: a segment in two parts (delta_scan_split_kernel) -- chunks of the second one get their replies times S1, four of a head in a work-group, so that S1's
+// fragments come out of memory once for four waves; work-groups behind those make the last state.
+__host__ __device__ __forceinline__ int split_columns(int n, int H) { return ceil_div(ceil_div(n - split_first(n), 4) * H, ceil_div(H, 4)); }     // of the grid, for the second part
+template <typename T, int NT, bool WIDE, bool SPLIT = false>
+__global__ __launch_bounds__(256) void delta_out_kernel(DeltaGeom g, DeltaIn in, const AttnSeg* __restrict__ segs, int nseg, int c0, int n, float* __restrict__ records,
                                                         T* __restrict__ y, int ldy) {
-  const ChunkAt at = chunk_at(segs, nseg, c0 + blockIdx.x);
-  if (!at.ok) return;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, h = blockIdx.y * 4 + wave;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  int chunk = blockIdx.x, h = blockIdx.y * 4 + wave;
+  __shared__ f32x4_t s1[SPLIT ? NT * NT * 64 : 1];      // the state between the parts, as fragments: one round of requests
+  f32x4_t rep[SPLIT ? NT : 1];                           // the chunk's replies
+  if constexpr (SPLIT) {
+    const int first = split_first(n), columns = split_columns(n, g.H), x = (int)blockIdx.x - first - columns;      // (the second part takes longer: it comes first)
+    if (x >= 0) {
+      delta_join(g, in.state, in.slots[segs[0].seq], n, records, (x * (int)gridDim.y + (int)blockIdx.y) * 4 + wave);
+      return;
+    }
+    chunk -= columns;
+    if (chunk < 0) {
+      const int u = (int)blockIdx.x * (int)gridDim.y + (int)blockIdx.y;
+      chunk = first + u / g.H * 4 + wave;
+      h = u % g.H;
+      const SplitMem m = split_mem(records, g, n, h);
+      const float* replies = m.replies + (size_t)min(chunk, n - 1) * 16 * g.dkp + (lane & 15) * 16 + (lane >> 4) * 4;
+#pragma unroll
+      for (int d = 0; d < NT; ++d) rep[d] = *reinterpret_cast<const f32x4_t*>(replies + min(d, g.dkp / 16 - 1) * 256);
+      const f32x4_t* from = reinterpret_cast<const f32x4_t*>(m.s1);
+      const int all = g.dkp * g.dvp / 4;
+      f32x4_t v[NT * NT / 4];
+#pragma unroll
+      for (int i = 0; i < NT * NT / 4; ++i) v[i] = from[min(i * 256 + (int)threadIdx.x, all - 1)];
+#pragma unroll
+      for (int i = 0; i < NT * NT / 4; ++i) s1[i * 256 + threadIdx.x] = v[i];
+      __syncthreads();
+    }
+  }
+  const ChunkAt at = chunk_at(segs, nseg, c0 + chunk);
+  if (!at.ok || chunk >= n) return;
   if (h < g.H) {
     const int t = lane >> 2, q = (lane & 3) * 4, tiles = g.dvp / 16;
     const size_t row = at.sg.row0 + at.t0 + min(t, at.n - 1);
-    const float *src = factors_at(records, (size_t)h * gridDim.x + blockIdx.x, g.dkp, g.dvp).v, *zr = in.z + row * in.ldz + in.gate + h * g.dv;
+    const float *src = factors_at(records, (size_t)h * n + chunk, g.dkp, g.dvp).v, *zr = in.z + row * in.ldz + in.gate + h * g.dv;
     f32x4_t x[NT], z[NT];
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
@@ -848,6 +964,23 @@ __global__ __launch_bounds__(256) void delta_out_kernel(DeltaGeom g, DeltaIn in,
       x[i] = *reinterpret_cast<const f32x4_t*>(src + tile * 256 + lane * 4);
       if constexpr (WIDE) z[i] = *reinterpret_cast<const f32x4_t*>(zr + min(v, g.dv - 4));
       else z[i] = f32x4_t{zr[min(v, g.dv - 1)], zr[min(v + 1, g.dv - 1)], zr[min(v + 2, g.dv - 1)], zr[min(v + 3, g.dv - 1)]};
+    }
+    if constexpr (SPLIT) {
+      if (chunk >= split_first(n)) {     // the products leave a column's quad of token (lane & 15) in lane >> 4: four lanes trade places
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+          f32x4_t add[2] = {};
+#pragma unroll
+          for (int d = 0; d < NT; ++d) {
+            if (max(i, d) >= tiles) continue;
+            const f32x4_t f = s1[(i * tiles + d) * 64 + lane];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) add[d & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[r], rep[d][r], add[d & 1], 0, 0, 0);
+          }
+#pragma unroll
+          for (int r = 0; r < 4; ++r) x[i][r] += __shfl(add[0][r] + add[1][r], (lane & 3) * 16 + t);
+        }
+      }
     }
     float ss = 0.f;
 #pragma unroll
@@ -877,7 +1010,8 @@ __global__ __launch_bounds__(256) void delta_out_kernel(DeltaGeom g, DeltaIn in,
   if (!at.last) return;
   const int C = g.channels();
   float* ring = in.ring + (size_t)in.slots[at.sg.seq] * g.taps * C;
-  for (int ch = blockIdx.y * 256 + threadIdx.x; ch < C; ch += gridDim.y * 256)
+  const bool by_wave = SPLIT && chunk >= split_first(n);       // (one wave a head has the last chunk, not four work-groups)
+  for (int ch = by_wave ? h * 64 + lane : blockIdx.y * 256 + threadIdx.x; ch < C; ch += by_wave ? g.H * 64 : gridDim.y * 256)
     for (int i = max(0, at.sg.n - g.taps); i < at.sg.n; ++i)
       ring[(size_t)((at.sg.pos0 + i) % g.taps) * C + ch] = in.proj[(size_t)(at.sg.row0 + i) * in.ldp + ch];
 }
@@ -895,7 +1029,9 @@ int check_in(const DeltaGeom& g, const DeltaIn& in) {
 bool delta_supported(const DeltaGeom& g) {
   return g.H >= 1 && g.G >= 1 && g.H % g.G == 0 && g.dk >= 1 && g.dk <= 256 && g.dv >= 1 && g.dv <= 256 && g.taps >= 1 && g.taps <= 16;
 }
-size_t delta_chunk_floats(const DeltaGeom& g) { return (size_t)g.H * record_floats(g.dkp, g.dvp); }
+// whether a segment may go in two parts (delta_scan_split_kernel): states as wide as they are high, keys the paired scan takes
+static bool split_fits(const DeltaGeom& g) { return g.dkp == g.dvp && g.dkp <= 128; }
+size_t delta_chunk_floats(const DeltaGeom& g) { return (size_t)g.H * (record_floats(g.dkp, g.dvp) + (split_fits(g) ? 16 * g.dkp : 0)); }
 
 int launch_delta_token(const DeltaGeom& g, const DeltaIn& in, int rows, const AttnSeg* segs, void* y, int ldy, bool f32, hipStream_t s) {
   int rc = check_in(g, in);
@@ -924,10 +1060,14 @@ int launch_delta_prompt(const DeltaGeom& g, const DeltaIn& in, const AttnSeg* sd
   int chunks = 0;
   for (int i = 0; i < nseg; ++i) chunks += sh[i].n < 2 ? 0 : ceil_div(sh[i].n, kC);
   const int nvt = g.dvp / 16, nt = ceil_div(g.dkp / 16, 4);
+  int num_cu = 0;
+  if (device_num_cu(&num_cu) != MI_OK) return MI_EHIP;
   const size_t lds = (size_t)(3 * kC * (g.dkp + 4) + std::max(kC * (g.dkp + 4), kPairParts * kPairTiles * 8)) * sizeof(float);
   for (int c0 = 0; c0 < chunks; c0 += max_chunks) {
     const int n = std::min(max_chunks, chunks - c0);
-    const dim3 gf(n, g.H), gs(g.H * nvt, nseg), go(n, ceil_div(g.H, 4));
+    const bool split = nseg == 1 && split_fits(g) && n >= kSplitChunks && 2 * g.H * nvt <= num_cu;
+    const int joins = split ? ceil_div(g.H * nvt * nvt, 4 * ceil_div(g.H, 4)) : 0;       // work-groups for the last state
+    const dim3 gf(n, g.H), gs(g.H * nvt, nseg), go(split ? split_first(n) + split_columns(n, g.H) + joins : n, ceil_div(g.H, 4));
 #define MI_DF(TAPS) { \
     if (lds > 48 * 1024) { rc = ensure_dynamic_lds(reinterpret_cast<const void*>(delta_factors_kernel<TAPS>), (int)lds); if (rc != MI_OK) return rc; } \
     hipLaunchKernelGGL((delta_factors_kernel<TAPS>), gf, dim3(256), lds, s, g, in, sd, nseg, c0, records); }
@@ -941,17 +1081,20 @@ int launch_delta_prompt(const DeltaGeom& g, const DeltaIn& in, const AttnSeg* sd
     }
 #undef MI_DF
 #define MI_DP(NT) hipLaunchKernelGGL((delta_scan_pairs_kernel<NT>), gs, dim3(256), 0, s, g, in.state, in.slots, sd, c0, n, nvt, records)
-    if (nt == 1) MI_DP(1);
+    if (split && nt == 1) hipLaunchKernelGGL((delta_scan_split_kernel<1>), dim3(3 * g.H * nvt), dim3(256), 0, s, g, in.state, in.slots, sd, c0, n, nvt, records);
+    else if (split) hipLaunchKernelGGL((delta_scan_split_kernel<2>), dim3(3 * g.H * nvt), dim3(256), 0, s, g, in.state, in.slots, sd, c0, n, nvt, records);
+    else if (nt == 1) MI_DP(1);
     else if (nt == 2) MI_DP(2);
     else if (nt == 3) MI_DS(3);      // (three sets of two chunks do not fit the registers)
     else MI_DS(4);
 #undef MI_DP
 #undef MI_DS
-#define MI_DO(NT, WIDE) \
-    if (f32) hipLaunchKernelGGL((delta_out_kernel<float, NT, WIDE>), go, dim3(256), 0, s, g, in, sd, nseg, c0, records, (float*)y, ldy); \
-    else hipLaunchKernelGGL((delta_out_kernel<uint16_t, NT, WIDE>), go, dim3(256), 0, s, g, in, sd, nseg, c0, records, (uint16_t*)y, ldy)
+#define MI_DO(NT, ...) \
+    if (f32) hipLaunchKernelGGL((delta_out_kernel<float, NT, __VA_ARGS__>), go, dim3(256), 0, s, g, in, sd, nseg, c0, n, records, (float*)y, ldy); \
+    else hipLaunchKernelGGL((delta_out_kernel<uint16_t, NT, __VA_ARGS__>), go, dim3(256), 0, s, g, in, sd, nseg, c0, n, records, (uint16_t*)y, ldy)
     const bool wide = g.dv % 4 == 0 && in.ldz % 4 == 0 && in.gate % 4 == 0 && ldy % 4 == 0 && reinterpret_cast<uintptr_t>(in.z) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
-    if (!wide) { MI_DO(16, false); } else if (g.dv <= 64) { MI_DO(4, true); } else if (g.dv <= 128) { MI_DO(8, true); } else { MI_DO(16, true); }
+    if (split) { if (wide && g.dv <= 64) { MI_DO(4, true, true); } else if (wide) { MI_DO(8, true, true); } else { MI_DO(8, false, true); } }
+    else if (!wide) { MI_DO(16, false); } else if (g.dv <= 64) { MI_DO(4, true); } else if (g.dv <= 128) { MI_DO(8, true); } else { MI_DO(16, true); }
 #undef MI_DO
     MI_HIP(hipGetLastError());
   }
