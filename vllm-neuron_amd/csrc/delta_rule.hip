@@ -902,15 +902,15 @@ __device__ __forceinline__ void delta_join(const DeltaGeom& g, float* __restrict
   if (h >= g.H) return;
   const SplitMem m = split_mem(records, g, n, h);
   const float* l = m.l + (size_t)(rt * 16 + 4 * g4) * g.dvp + ct * 16 + c;
-  f32x4_t s = {l[0], l[g.dvp], l[2 * g.dvp], l[3 * g.dvp]};
+  f32x4_t a[4] = {};             // (short chains, added pairwise: the join adds little to the rounding of its parts)
   for (int t = 0; t < tiles; ++t) {
     const f32x4_t p = *reinterpret_cast<const f32x4_t*>(m.p + (size_t)(rt * 16 + c) * g.dvp + t * 16 + 4 * g4), s1 = *reinterpret_cast<const f32x4_t*>(m.s1 + ((ct * tiles + t) * 64 + lane) * 4);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) s = __builtin_amdgcn_mfma_f32_16x16x4f32(p[r], s1[r], s, 0, 0, 0);
+    for (int r = 0; r < 4; ++r) a[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[r], s1[r], a[r], 0, 0, 0);
   }
   float* to = state + ((size_t)slot * g.H + h) * g.dkp * g.dvp + (size_t)(rt * 16 + 4 * g4) * g.dvp + ct * 16 + c;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) to[(size_t)r * g.dvp] = s[r];
+  for (int r = 0; r < 4; ++r) to[(size_t)r * g.dvp] = l[(size_t)r * g.dvp] + ((a[0][r] + a[1][r]) + (a[2][r] + a[3][r]));
 }
 
 // Norm and gate: a wave per head and chunk, a lane four columns of every value tile of one token, all of them requested together; the work-groups of a
