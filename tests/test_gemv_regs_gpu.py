@@ -43,6 +43,14 @@ def test_edges_of_the_register_gemv(lib, wd, M, N, K):
     assert err < tol, (err, tol)
 
 
+# every number of k-tiles a wave holds that has a kernel of its own, whole and with a last tile or whole waves missing (one-byte weights 5 .. 8, bf16 5 .. 8, 12, 14, 16)
+@pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
+@pytest.mark.parametrize("M", [5, 32])
+@pytest.mark.parametrize("N,K", [(4096, K) for K in (1088, 1536, 1600, 1792, 2112, 2560, 2624, 3072, 3136, 3584, 3648)])
+def test_k_tiles_of_a_wave(lib, wd, M, N, K):
+    test_edges_of_the_register_gemv(lib, wd, M, N, K)
+
+
 # up to 4 rows, where they go there: one row-tile a work-group, eight and more, one k-tile fewer than a wave has registers for, and one more (the LDS kernels)
 @pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
 @pytest.mark.parametrize("M", [1, 3, 4])

@@ -15,7 +15,8 @@
 namespace mi {
 
 constexpr int kRegsMaxPasses = 64;   // row-tiles of a work-group: their scales and biases wait in LDS
-// k-tiles a wave holds at most: 4 or 8 of 64 k (1-byte weights), 4, 8 or 16 of 32 k
+// k-tiles a wave holds at most: 8 of 64 k (1-byte weights), 16 of 32 k.  There is a kernel for 4, 5, 6, 7, 8 (bf16 also 12, 14, 16): a row-tile's requests all go out, those a wave has no
+// tile for repeat its last one, and a CU's requests in flight are what bounds it.  With 4, 8 and 16 alone, us a step: 7B int8 5 rows 1243 -> 1196, bf16 1679 -> 1583, 8B fp8 8 rows 1230 -> 1207.
 template <int WD> constexpr int kRegsMaxTiles = WD == MI_W_BF16 ? 16 : 8;
 
 // HOLD: a work-group takes HOLD row-tiles side by side, and the wave that sums them keeps their results until it has all: a row's HOLD x 64 bytes
@@ -25,9 +26,9 @@ template <int WD, int EPI, int MG, int NK, bool SLAB, int HOLD = 1>
 __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4* __restrict__ W, int NT, int KT, int M, int G,
                                                                    const uint16_t* __restrict__ x, int ldx, EpiArgs e, float* __restrict__ slab) {
   constexpr int FR = WD == MI_W_BF16 ? 1 : 2;         // MFMAs per weight tile and column group
-  constexpr int BT = NK < 8 ? NK : 8, NB = NK / BT;   // weight tiles per request batch (8 KiB a wave), batches per row-tile
+  constexpr int NB = NK > 8 ? 2 : 1, BT = NK / NB;    // batches per row-tile, weight tiles per request batch (up to 8 KiB a wave)
   constexpr int TK = WD == MI_W_BF16 ? 32 : 64;
-  static_assert(NB == 1 || NB == 2, "one or two batches per row-tile");
+  static_assert(NB * BT == NK, "whole batches");
   __shared__ f32x4_t red[2][kGemvWaves][MG][64];
   __shared__ __attribute__((aligned(16))) float sc_lds[SLAB ? 4 : kRegsMaxPasses * 16], bi_lds[SLAB ? 4 : kRegsMaxPasses * 16];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -216,9 +217,18 @@ static int launch_gemv_regs_k(const LinearW& w, int M, const uint16_t* x, int ld
   const int groups = ceil_div(NT, HOLD), G = ceil_div(groups, std::min(kRegsMaxPasses / HOLD, ceil_div(groups, std::min(groups, per))));
   const dim3 grid(G, slices);
   const uint4* W = reinterpret_cast<const uint4*>(w.w);
-  if (tiles <= 4) hipLaunchKernelGGL((gemv_regs_kernel<WD, EPI, MG, 4, SLAB, HOLD>), grid, dim3(kGemvWaves * 64), 0, s, W, NT, KT, M, G, x, ldx, e, slab);
-  else if (tiles <= 8) hipLaunchKernelGGL((gemv_regs_kernel<WD, EPI, MG, 8, SLAB, HOLD>), grid, dim3(kGemvWaves * 64), 0, s, W, NT, KT, M, G, x, ldx, e, slab);
-  else if constexpr (WD == MI_W_BF16) hipLaunchKernelGGL((gemv_regs_kernel<WD, EPI, MG, 16, SLAB, HOLD>), grid, dim3(kGemvWaves * 64), 0, s, W, NT, KT, M, G, x, ldx, e, slab);
+#define MI_K(NK_) hipLaunchKernelGGL((gemv_regs_kernel<WD, EPI, MG, NK_, SLAB, HOLD>), grid, dim3(kGemvWaves * 64), 0, s, W, NT, KT, M, G, x, ldx, e, slab)
+  if (tiles <= 4) MI_K(4);
+  else if (tiles == 5) MI_K(5);
+  else if (tiles == 6) MI_K(6);
+  else if (tiles == 7) MI_K(7);
+  else if (tiles == 8) MI_K(8);
+  else if constexpr (WD == MI_W_BF16) {
+    if (tiles <= 12) MI_K(12);
+    else if (tiles <= 14) MI_K(14);
+    else MI_K(16);
+  }
+#undef MI_K
   MI_HIP(hipGetLastError());
   return MI_OK;
 }
@@ -287,14 +297,14 @@ bool gemv_regs_fits_wd(int M, int N, int K, size_t ws_bytes) {
   return device_num_cu(&num_cu) == MI_OK && gemv_regs_slices<WD>(M, N, K, ws_bytes, false, num_cu) > 0;
 }
 
-// Which part of a wave's requests are k-tiles of its own, the sum of the slices having a taker: a row-tile's 4 or 8 go out whatever it owns.
+// Which part of a wave's requests are k-tiles of its own, the sum of the slices having a taker: a row-tile's 4 .. 8 go out whatever it owns (by_fours: as if they were 4 or 8).
 template <int WD>
-double gemv_regs_own_wd(int M, int N, int K, size_t ws_bytes) {
+double gemv_regs_own_wd(int M, int N, int K, size_t ws_bytes, bool by_fours) {
   int num_cu = 0;
   const int z = device_num_cu(&num_cu) == MI_OK ? gemv_regs_slices<WD>(M, N, K, ws_bytes, true, num_cu) : 0;
   if (z == 0) return 1.;
   const int KT = K / tile_k(WD), tiles = ceil_div(ceil_div(KT, z), kGemvWaves);
-  return (double)KT / (z * kGemvWaves * (tiles <= 4 ? 4 : 8));
+  return (double)KT / (z * kGemvWaves * (tiles <= 4 ? 4 : by_fours ? 8 : tiles));
 }
 
 }  // namespace mi

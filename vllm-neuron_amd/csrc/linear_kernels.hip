@@ -43,7 +43,7 @@ extern template int launch_gemv_wd<MI_W_INT8>(const LinearW&, int, int, const Pr
 template <int WD>
 int launch_gemv_regs_wd(const LinearW& w, int M, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s, float* ws, size_t ws_bytes, SlabSum* defer, bool split_as_deferred);
 template <int WD> bool gemv_regs_fits_wd(int M, int N, int K, size_t ws_bytes);
-template <int WD> double gemv_regs_own_wd(int M, int N, int K, size_t ws_bytes);
+template <int WD> double gemv_regs_own_wd(int M, int N, int K, size_t ws_bytes, bool by_fours);
 
 static bool gemv_regs_fits(const LinearW& w, int M, size_t ws_bytes) {
   switch (w.wd) {
@@ -88,9 +88,11 @@ static int gemm_wide_bm() {      // MI355X_GEMM_WIDE_BM: 128 / 256 forces the to
 // 32.0 / 34.2 -> 33.8 / 34.8), bf16 (28672 x 4096 42.8 / 44.0 -> 45.8 / 47.0), up to 16 rows (23.4 -> 23.8); nor shallower K (us a call: 8B int8 28 rows 1834 -> 1845, TinyLlama
 // fp8 30 rows 1260 -> 1272).  The lines below are drawn through us a layer of 78 models of 1024 .. 8192 wide, feed-forwards of 3584 .. 28672, at 17 .. 32 rows, one projection after the
 // other moved to the wide GEMM in the same model:
-// K slices whose sum the next norm takes: by the share of a register wave's requests that are k-tiles of its own (they go out by 4 and 8, and those it does not have repeat the last).
+// K slices whose sum the next norm takes: by the share of a register wave's requests that are k-tiles of its own (counted as if they went out by 4 and 8, as they did when the
+// lines were drawn; those it does not have repeat the last).
 // fp8: up to 27 / 32 of them 0 .. 9 less; beyond that 0.5 .. 3 less where the wide GEMM's tiles times ten slices at most fill the chip (N of 3584, 4096, 4608, 8192), else up to 4 more
-// (7168 x 17408 17 rows; 6144 x 16384 1.4); 3584 x 3584 0.2 .. 1.7 more.  int8: up to 5 / 8 0.7 .. 8 less, beyond that between 3 less and 2 more (3072 x 24576; 4608 x 16384).  Where the
+// (7168 x 17408 17 rows; 6144 x 16384 1.4); 3584 x 3584 0.2 .. 1.7 more.  int8: up to 5 / 8 0.7 .. 8 less, beyond that between 3 less and 2 more (3072 x 24576; 4608 x 16384); since 5 .. 7 have kernels
+// of their own the register kernel is the faster one where more than 0.86 of what goes out is its own (3584 x 18944, 17 / 20 / 28 / 32 rows a step of the 7B model 1410 -> 1376, 1486 -> 1452, 1637 -> 1596, 1725 -> 1686).  Where the
 // weights themselves take longest the register kernel streams them faster (fp8 7168 x 22016 4 more, 8192 x 28672 5, int8 7168 x 28672 4; fp8 8192 x 17408 still 5 .. 9 less), and narrow sums leave the wide GEMM
 // half of the chip and more (1536 x 11008 fp8 0.6 more, 1536 x 20480 int8 1.5, 1024 x 20480 2.8).
 // Unsplit gate | up of fp8 that fills three quarters of the chip in one round: 0.5 .. 12 less.
@@ -104,8 +106,8 @@ bool gemm_wide_few_rows(const LinearW& w, int M, int epi, size_t ws_bytes, bool 
   const bool fp8 = w.wd == MI_W_F8E4M3;
   if (deferred) {
     if (w.K < (fp8 ? 4096 : 16384) || w.N < 2048 || (size_t)w.N * w.K > 150000000) return false;
-    const double own = fp8 ? gemv_regs_own_wd<MI_W_F8E4M3>(M, w.N, w.K, ws_bytes) : gemv_regs_own_wd<MI_W_INT8>(M, w.N, w.K, ws_bytes);
-    if (own <= (fp8 ? 27. / 32. : 5. / 8.)) return true;
+    const auto own = [&](bool by_fours) { return fp8 ? gemv_regs_own_wd<MI_W_F8E4M3>(M, w.N, w.K, ws_bytes, by_fours) : gemv_regs_own_wd<MI_W_INT8>(M, w.N, w.K, ws_bytes, by_fours); };
+    if (own(true) <= (fp8 ? 27. / 32. : 5. / 8.) && (fp8 || own(false) <= 0.86)) return true;
     return fp8 && w.K >= 8192 && tiles * std::min(10, cus / tiles) * 16 > cus * 15;
   }
   if (!fp8 || w.K < 3584) return false;
