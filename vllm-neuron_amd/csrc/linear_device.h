@@ -774,7 +774,8 @@ __device__ __forceinline__ void pin_gemv_args(const uint4* W, int NT, int KT, in
 constexpr int kPrivJ = 4;       // 16-byte chunks per lane per activation row (slice <= 2048 elements)
 constexpr int kPrivJNorm = 2;   // norm prologues hold fp32 rows: slice <= 1024 elements
 
-template <int WD, int PRO, int EPI, int KS>
+// U: weight tiles to a batch (priv_batch)
+template <int WD, int PRO, int EPI, int KS, int U>
 __global__ __launch_bounds__(kGemvWaves * 64) void gemv_priv_kernel(const uint4* __restrict__ W, int NT, int KT,
                                                                     int M, int K, int G, ProArgs p, EpiArgs e) {
   // G = the grid size as an argument: the builtin reads the dispatch packet (two more dependent scalar loads)
@@ -797,23 +798,23 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_priv_kernel(const uint4*
   const int ktw = ceil_div(KT, KS);
   const int kbeg = min(kslice * ktw, KT), kend = min(kbeg + ktw, KT);
   const int klast = max(kend - 1, 0);
-  const int nb = ceil_div(ktw, kGemvU);
+  const int nb = ceil_div(ktw, U);
   const int units = ceil_div(NT, TP);
   const int my_units = (int)blockIdx.x < units ? ceil_div(units - (int)blockIdx.x, G) : 0;
   const bool col_ok = c < M;
   MI_TRACE_BEGIN();
   MI_STAMP(0);
 
-  u32x4_t bufA[kGemvU], bufB[kGemvU];
+  u32x4_t bufA[U], bufB[U];
   int is_pass = 0, is_b = 0;     // the next batch to request
-  auto issue = [&](u32x4_t (&buf)[kGemvU]) {
+  auto issue = [&](u32x4_t (&buf)[U]) {
     const bool live = is_pass < my_units;
     const int tile = min((int)(blockIdx.x + is_pass * G) * TP + tsub, NT - 1);
-    const int kt0 = kbeg + is_b * kGemvU;
+    const int kt0 = kbeg + is_b * U;
     const uint4* base = live ? W + (size_t)tile * KT * 64 + lane : W;
     const size_t kstep = live ? 64 : 0;
 #pragma unroll
-    for (int u = 0; u < kGemvU; ++u) stream_load16(buf[u], base + (size_t)min(kt0 + u, klast) * kstep);
+    for (int u = 0; u < U; ++u) stream_load16(buf[u], base + (size_t)min(kt0 + u, klast) * kstep);
     if (++is_b == nb) { is_b = 0; ++is_pass; }
   };
 
@@ -934,10 +935,10 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_priv_kernel(const uint4*
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
   int parity = 0;
   int pr_pass = 0, pr_b = 0;     // the batch being multiplied
-  auto process = [&](u32x4_t (&buf)[kGemvU]) {
-    const int kt0 = kbeg + pr_b * kGemvU;
+  auto process = [&](u32x4_t (&buf)[U]) {
+    const int kt0 = kbeg + pr_b * U;
 #pragma unroll
-    for (int u = 0; u < kGemvU; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int kt = kt0 + u;
       const bool ok = col_ok && kt < kend;
       const u32x4_t w = buf[u];
@@ -1015,12 +1016,17 @@ static bool gemv_priv_ok(int M, int KT, int ks, int tp) {
   return nch <= 64 * (PRO == PRO_BF16 ? kPrivJ : kPrivJNorm);
 }
 
-template <int WD, int PRO, int EPI, int KS>
-static int launch_gemv_priv(const LinearW& w, int M, const ProArgs& p, const EpiArgs& e, hipStream_t s, int num_cu) {
+// Weight tiles to a batch for a wave's slice of `ktw`: all requests of a batch go out, those beyond the slice for its last tile once more, so the slice is spread
+// evenly over as many batches as there would be of 8 (more batches of fewer would keep fewer requests in flight; below 6 the same).  Measured at batches of 8 ->
+// here: the down projection 14336 deep of one-byte weights (28 tiles a wave) 13.3 -> 12.9 us, int8 3584 deep (14) 9.4 -> 8.7 us for the 4608 rows of
+// QKV and 125.6 -> 121.4 us for a head of 152064, both at 4 rows; whole passes of TinyLlama fp8 (5632 deep: 11) at 2 rows 709 -> 680 us.
+static int priv_batch(int ktw) { return max(6, ceil_div(ktw, ceil_div(ktw, 8))); }
+template <int WD, int PRO, int EPI, int KS, int U>
+static int launch_gemv_priv_u(const LinearW& w, int M, const ProArgs& p, const EpiArgs& e, hipStream_t s, int num_cu) {
   constexpr int TP = kGemvWaves / KS;
   const int NT = w.N / 16, KT = w.K / tile_k(WD);
   const size_t lds = gemv_image_lds_bytes(M, w.K);
-  auto kern = gemv_priv_kernel<WD, PRO, EPI, KS>;
+  auto kern = gemv_priv_kernel<WD, PRO, EPI, KS, U>;
   MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(kern), 160 * 1024));
   const int units = ceil_div(NT, TP);
   int grid = min(units, num_cu);
@@ -1029,6 +1035,14 @@ static int launch_gemv_priv(const LinearW& w, int M, const ProArgs& p, const Epi
                      w.K, grid, p, e);
   MI_HIP(hipGetLastError());
   return MI_OK;
+}
+template <int WD, int PRO, int EPI, int KS>
+static int launch_gemv_priv(const LinearW& w, int M, const ProArgs& p, const EpiArgs& e, hipStream_t s, int num_cu) {
+  switch (priv_batch(ceil_div(w.K / tile_k(WD), KS))) {
+    case 6: return launch_gemv_priv_u<WD, PRO, EPI, KS, 6>(w, M, p, e, s, num_cu);
+    case 7: return launch_gemv_priv_u<WD, PRO, EPI, KS, 7>(w, M, p, e, s, num_cu);
+    default: return launch_gemv_priv_u<WD, PRO, EPI, KS, 8>(w, M, p, e, s, num_cu);
+  }
 }
 
 // (KS, TP) for NT row-tiles of KT k-tiles on `slots` resident work-groups: fewest k-tiles on the
