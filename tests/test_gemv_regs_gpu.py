@@ -67,6 +67,29 @@ def test_batches_of_the_few_row_kernels(lib, wd, M, N, K):
     test_edges_of_the_register_gemv(lib, wd, M, N, K)
 
 
+# ... with the norms in front, where slices of 2 .. 16 tiles go to 1, 2, 4 and 8 waves: against 5 rows, whose weights the register kernel reads (the same products
+# in another order; bf16 roundings of the activations in between make 2^-8 of a value, and as between any two kernels of this file 5 % of the spread is far beyond)
+@pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
+@pytest.mark.parametrize("hidden,inter,vocab", [(1024, 1088, 16), (1280, 6208, 12304), (2048, 5632, 32000), (2304, 2112, 8208), (3584, 4736, 16400), (4096, 14336, 4112)])
+def test_norms_in_front_of_few_rows(wd, hidden, inter, vocab):
+    from oracle import DecoderConfig
+    from oracle.synth import make_weights
+    from tests.helpers import decode_inputs
+    from vllm_neuron_amd._native import MI_Q, MI_W, NativeModel
+    shape = dict(num_layers=1, hidden_size=hidden, num_heads=hidden // 64, num_kv_heads=hidden // 256, head_dim=64, intermediate_size=inter, vocab_size=vocab)
+    w = make_weights(DecoderConfig(**shape), seed=4)
+    model = NativeModel(**shape, rms_norm_eps=1e-5, rope_theta=1e4, rope_type=0, rope_factor=1.0, num_blocks=33, block_size=32, max_num_seqs=8,
+                        max_model_len=32, weight_dtype=MI_W[wd], quant_type=MI_Q["per_channel_symmetric"], quantize_lm_head=1, tp_degree=1, tp_rank=0,
+                        device_id=0, use_graphs=1, ctx_buckets=[32])
+    model.load_state_dict(w)
+    model.finalize()
+    out = {rows: model.forward(**decode_inputs([i % vocab for i in range(rows)], [0] * rows, [[1 + i] for i in range(rows)], 32, 32)).clone() for rows in (5, 4, 1)}
+    std = out[5].std().item()
+    for rows in (4, 1):
+        assert torch.isfinite(out[rows]).all() and (out[rows] - out[5][:rows]).abs().max().item() < 0.05 * std
+    model.close()
+
+
 # the same sums at up to 4 rows: K of a narrow projection over several slices
 @pytest.mark.parametrize("rows", [1, 4])
 def test_sums_of_few_rows_left_to_the_next_norm(rows):

@@ -1007,20 +1007,19 @@ static bool gemv_priv_enabled() {
   static const bool on = [] { const char* v = getenv("MI355X_GEMV_PRIV"); return !(v && v[0] == '0'); }();
   return on;
 }
-// wave-private staging applies when all 8 waves stream (TP = 8 / KS), at most 4 rows, and a wave's
-// K-slice fits the per-lane register budget of the prologue
+// wave-private staging applies when all 8 waves stream (TP = 8 / KS), at most 4 rows, and a wave's K-slice fits the per-lane register budget of the prologue:
+// the most k-tiles of such a slice
 template <int WD, int PRO>
-static bool gemv_priv_ok(int M, int KT, int ks, int tp) {
-  if (!gemv_priv_enabled() || ks < 2 || ks * tp != kGemvWaves || M > 4) return false;
-  const int nch = ceil_div(KT, ks) * (tile_k(WD) / 8);
-  return nch <= 64 * (PRO == PRO_BF16 ? kPrivJ : kPrivJNorm);
+static int gemv_priv_kt(int M) {
+  return gemv_priv_enabled() && M <= 4 ? 64 * (PRO == PRO_BF16 ? kPrivJ : kPrivJNorm) / (tile_k(WD) / 8) : 0;
 }
 
 // Weight tiles to a batch for a wave's slice of `ktw`: all requests of a batch go out, those beyond the slice for its last tile once more, so the slice is spread
-// evenly over as many batches as there would be of 8 (more batches of fewer would keep fewer requests in flight; below 6 the same).  Measured at batches of 8 ->
+// evenly over as many batches as there would be of 8 (more batches of fewer would keep fewer requests in flight).  Measured at batches of 8 ->
 // here: the down projection 14336 deep of one-byte weights (28 tiles a wave) 13.3 -> 12.9 us, int8 3584 deep (14) 9.4 -> 8.7 us for the 4608 rows of
-// QKV and 125.6 -> 121.4 us for a head of 152064, both at 4 rows; whole passes of TinyLlama fp8 (5632 deep: 11) at 2 rows 709 -> 680 us.
-static int priv_batch(int ktw) { return max(6, ceil_div(ktw, ceil_div(ktw, 8))); }
+// QKV and 125.6 -> 121.4 us for a head of 152064, both at 4 rows; whole passes of TinyLlama fp8 at
+// 2 rows 709 -> 680 us with the down projection's 11 tiles in 6 + 5, and 670 -> 637 with gate | up, QKV (2048 deep: 4) in batches of 4 instead of 6.
+static int priv_batch(int ktw) { return max(4, ceil_div(ktw, ceil_div(ktw, 8))); }
 template <int WD, int PRO, int EPI, int KS, int U>
 static int launch_gemv_priv_u(const LinearW& w, int M, const ProArgs& p, const EpiArgs& e, hipStream_t s, int num_cu) {
   constexpr int TP = kGemvWaves / KS;
@@ -1039,30 +1038,33 @@ static int launch_gemv_priv_u(const LinearW& w, int M, const ProArgs& p, const E
 template <int WD, int PRO, int EPI, int KS>
 static int launch_gemv_priv(const LinearW& w, int M, const ProArgs& p, const EpiArgs& e, hipStream_t s, int num_cu) {
   switch (priv_batch(ceil_div(w.K / tile_k(WD), KS))) {
+    case 4: return launch_gemv_priv_u<WD, PRO, EPI, KS, 4>(w, M, p, e, s, num_cu);
+    case 5: return launch_gemv_priv_u<WD, PRO, EPI, KS, 5>(w, M, p, e, s, num_cu);
     case 6: return launch_gemv_priv_u<WD, PRO, EPI, KS, 6>(w, M, p, e, s, num_cu);
     case 7: return launch_gemv_priv_u<WD, PRO, EPI, KS, 7>(w, M, p, e, s, num_cu);
     default: return launch_gemv_priv_u<WD, PRO, EPI, KS, 8>(w, M, p, e, s, num_cu);
   }
 }
 
-// (KS, TP) for NT row-tiles of KT k-tiles on `slots` resident work-groups: fewest k-tiles on the
-// busiest CU (passes x TP x KT/KS x KS), then the fewest passes, then the most streaming waves,
-// then the smallest K split.
+// (KS, TP) for NT row-tiles of KT k-tiles on `slots` resident work-groups: fewest k-tiles on the busiest CU (passes x TP x KT/KS x KS), then the most streaming
+// waves, then slices that the waves stage for themselves (of at most `priv_kt` k-tiles, 0: none) and of them the shortest that fill a batch, else the smallest K split.
+// Waves used to come behind the number of passes: the gate | up rows of the 7B shape (37888: 2368 row-tiles, ten on the busiest CU either way) went as 1 x 5, five
+// waves and two passes, at 4 rows int8 31.1 us and with bf16 47.4 (2 rows); as 4 x 2 they take 26.2 and 42.7.  28672 rows x 4096 fp8 (1 x 7 -> 8 x 1) 22.8 -> 21.6 us,
+// the head of 128256 rows beside it (1 x 8 -> 8 x 1, 8 tiles a slice) 106 -> 94; of 152064 x 3584 the slices of 14 tiles keep 121 us against 133 with slices of 7.
 struct GemvShape { int ks, tp; };
-static GemvShape gemv_pick_shape(int NT, int KT, int slots) {
+static GemvShape gemv_pick_shape(int NT, int KT, int slots, int priv_kt) {
   GemvShape best{8, 1};
   long best_load = 1L << 60;
-  int best_pass = 1 << 30, best_waves = 0;
+  int best_waves = 0, best_rank = 0;
   for (int ks = 1; ks <= 8; ks *= 2) {
     if (KT < ks) break;
     for (int tp = 1; tp * ks <= kGemvWaves; ++tp) {
-      const int units = ceil_div(NT, tp);
-      const int passes = ceil_div(units, slots);
-      const long load = (long)passes * tp * ceil_div(KT, ks) * ks;
-      const int waves = tp * ks;
-      const bool better = load < best_load || (load == best_load && (passes < best_pass ||
-                          (passes == best_pass && (waves > best_waves))));
-      if (better) { best = {ks, tp}; best_load = load; best_pass = passes; best_waves = waves; }
+      const int slice = ceil_div(KT, ks), waves = tp * ks;
+      const long load = (long)ceil_div(ceil_div(NT, tp), slots) * tp * slice * ks;
+      const bool priv = ks > 1 && waves == kGemvWaves && slice <= priv_kt;
+      const int rank = !priv ? 8 - ks : slice < 8 ? 16 - ks : 16 + ks;
+      const bool better = load < best_load || (load == best_load && (waves > best_waves || (waves == best_waves && rank > best_rank)));
+      if (better) { best = {ks, tp}; best_load = load; best_waves = waves; best_rank = rank; }
     }
   }
   return best;
@@ -1104,8 +1106,9 @@ static int launch_gemv_t(const LinearW& w, int M, const ProArgs& p, const EpiArg
   //  per Llama-8B pass)
   int num_cu = 0;
   MI_TRY_(device_num_cu(&num_cu));
-  const GemvShape sh = gemv_pick_shape(w.N / 16, w.K / tile_k(WD), num_cu);
-  if (gemv_priv_ok<WD, PRO>(M, w.K / tile_k(WD), sh.ks, sh.tp)) {
+  const int KT = w.K / tile_k(WD), priv_kt = gemv_priv_kt<WD, PRO>(M);
+  const GemvShape sh = gemv_pick_shape(w.N / 16, KT, num_cu, priv_kt);
+  if (sh.ks > 1 && sh.ks * sh.tp == kGemvWaves && ceil_div(KT, sh.ks) <= priv_kt) {
     switch (sh.ks) {
       case 2: return launch_gemv_priv<WD, PRO, EPI, 2>(w, M, p, e, s, num_cu);
       case 4: return launch_gemv_priv<WD, PRO, EPI, 4>(w, M, p, e, s, num_cu);
