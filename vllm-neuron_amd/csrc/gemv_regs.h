@@ -68,13 +68,8 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
   u32x4_t bufA[BT], bufB[BT];
   const int total = passes * NB;
   auto issue = [&](u32x4_t (&buf)[BT], int i) {
-    const bool live = i < total;                      // (a batch that does not exist: one line, the same for every lane)
-    const int ii = min(i, total - 1), tile = tile_of(ii / NB), k0 = kbeg + (ii % NB) * BT;
-    const uint4* base = live ? W + (size_t)tile * KT * 64 : W;
-    const int kstep = live ? 64 : 0;
-    const unsigned at = live ? lane : 0;
-#pragma unroll
-    for (int u = 0; u < BT; ++u) stream_load16(buf[u], base + (size_t)(min(k0 + u, klast) * kstep) + at);
+    const int ii = min(i, total - 1), k0 = kbeg + (ii % NB) * BT;      // (behind the last batch, and beyond the slice: no request.  O of the 1B shape 5.2 -> 4.7 us, of the 7B 6.4 -> 6.0)
+    stream_batch(buf, W, tile_of(ii / NB) * KT + k0, i < total ? kend - k0 : 0, lane);
   };
   issue(bufA, 0);
   __builtin_amdgcn_sched_barrier(0);

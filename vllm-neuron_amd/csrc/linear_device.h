@@ -811,10 +811,16 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_priv_kernel(const uint4*
     const bool live = is_pass < my_units;
     const int tile = min((int)(blockIdx.x + is_pass * G) * TP + tsub, NT - 1);
     const int kt0 = kbeg + is_b * U;
-    const uint4* base = live ? W + (size_t)tile * KT * 64 + lane : W;
-    const size_t kstep = live ? 64 : 0;
+    // zeros without a request beyond the slice, and behind the last row-tile, where the loop asks for two batches more: down projections 5632 x 2048 bf16 7.9 -> 7.5 us.
+    // (with norms in front, 4 batches and more a wave, it measured the same or slower in batches of 8: gate | up of the 1B shape 9.8 -> 10.4, 8B fp8 21.8 either way)
+    if constexpr (PRO == PRO_BF16) {
+      stream_batch(buf, W, tile * KT + kt0, live ? kend - kt0 : 0, lane);
+    } else {
+      const uint4* base = live ? W + (size_t)tile * KT * 64 + lane : W;
+      const size_t kstep = live ? 64 : 0;
 #pragma unroll
-    for (int u = 0; u < U; ++u) stream_load16(buf[u], base + (size_t)min(kt0 + u, klast) * kstep);
+      for (int u = 0; u < U; ++u) stream_load16(buf[u], base + (size_t)min(kt0 + u, klast) * kstep);
+    }
     if (++is_b == nb) { is_b = 0; ++is_pass; }
   };
 
@@ -1014,10 +1020,9 @@ static int gemv_priv_kt(int M) {
   return gemv_priv_enabled() && M <= 4 ? 64 * (PRO == PRO_BF16 ? kPrivJ : kPrivJNorm) / (tile_k(WD) / 8) : 0;
 }
 
-// Weight tiles to a batch for a wave's slice of `ktw`: all requests of a batch go out, those beyond the slice for its last tile once more, so the slice is spread
-// evenly over as many batches as there would be of 8 (more batches of fewer would keep fewer requests in flight).  Measured at batches of 8 ->
-// here: the down projection 14336 deep of one-byte weights (28 tiles a wave) 13.3 -> 12.9 us, int8 3584 deep (14) 9.4 -> 8.7 us for the 4608 rows of
-// QKV and 125.6 -> 121.4 us for a head of 152064, both at 4 rows; whole passes of TinyLlama fp8 at
+// Weight tiles to a batch for a wave's slice of `ktw`: as many batches as there would be of 8, the slice spread evenly over them (more batches of fewer would keep fewer
+// requests in flight).  With norms in front the tiles of a batch beyond the slice are requests for its last tile once more.  Measured at batches of 8 -> here: int8
+// 3584 deep (14 tiles a wave) 9.4 -> 8.7 us for the 4608 rows of QKV and 125.6 -> 121.4 us for a head of 152064, both at 4 rows; whole passes of TinyLlama fp8 at
 // 2 rows 709 -> 680 us with the down projection's 11 tiles in 6 + 5, and 670 -> 637 with gate | up, QKV (2048 deep: 4) in batches of 4 instead of 6.
 static int priv_batch(int ktw) { return max(4, ceil_div(ktw, ceil_div(ktw, 8))); }
 template <int WD, int PRO, int EPI, int KS, int U>
