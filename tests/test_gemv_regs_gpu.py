@@ -59,10 +59,11 @@ def test_edges_of_few_rows(lib, wd, M, N, K):
     test_edges_of_the_register_gemv(lib, wd, M, N, K)
 
 
-# up to 4 rows in the LDS kernels with K over the waves: batches of 6, 7 and 8 tiles, whole, and with tiles of the last wave missing; one and several passes
+# up to 4 rows in the LDS kernels with K over the waves: batches of 5 .. 8 tiles, whole, and with tiles of the last wave missing; one and several passes; K beyond 16384
+# and what the LDS holds: activations beside the weights, an odd and an even number of sub-chunks, waves with a part of one and with none of the last
 @pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
 @pytest.mark.parametrize("M", [1, 4])
-@pytest.mark.parametrize("N,K", [(16, 4608), (4112, 5632), (144, 5568), (272, 6656), (4096, 7168), (16, 7104), (48, 9216), (4112, 14336), (528, 14272), (16, 16384)])
+@pytest.mark.parametrize("N,K", [(16, 4608), (4112, 5632), (144, 5568), (272, 6656), (4096, 7168), (16, 7104), (48, 9216), (4112, 14336), (528, 14272), (16, 16384), (48, 16448), (4112, 17472), (16, 18944), (8208, 20480), (272, 28672)])
 def test_batches_of_the_few_row_kernels(lib, wd, M, N, K):
     test_edges_of_the_register_gemv(lib, wd, M, N, K)
 

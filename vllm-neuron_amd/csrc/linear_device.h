@@ -1005,6 +1005,12 @@ __device__ __forceinline__ void glds16(const void* g, unsigned char* l) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g,
                                    (__attribute__((address_space(3))) void*)l, 16, 0, 0);
 }
+// the same through a buffer descriptor, `at` in bytes: past the descriptor's end zeros, and no request.  (hipcc counts loads to registers beside it; beside
+// global_load_lds it waits for all that are in flight)
+__device__ __forceinline__ void blds16(const void* p, int bytes, int at, unsigned char* l) {
+  const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)l, 16, at, 0, 0, 0);
+}
 static bool gemv_kstream_enabled() {
   static const bool on = [] { const char* v = getenv("MI355X_GEMV_KSTREAM"); return !(v && v[0] == '0'); }();
   return on;
@@ -1113,6 +1119,10 @@ static int launch_gemv_t(const LinearW& w, int M, const ProArgs& p, const EpiArg
   MI_TRY_(device_num_cu(&num_cu));
   const int KT = w.K / tile_k(WD), priv_kt = gemv_priv_kt<WD, PRO>(M);
   const GemvShape sh = gemv_pick_shape(w.N / 16, KT, num_cu, priv_kt);
+  // slices too long to be staged by their wave: beside the weights (bit for bit the same sums; 3584 x 18944 int8 at 2 rows 17.4 -> 16.6 us, bf16 24.3 -> 23.5, at 1 row
+  // the same)
+  if constexpr (PRO == PRO_BF16 && (EPI == EPI_F32 || EPI == EPI_RESID || EPI >= EPI_RELU2))
+    if (sh.ks == 8 && ceil_div(KT, 8) > priv_kt && M >= 2 && M <= 4 && gemv_kstream_enabled()) return launch_gemv_kstream<WD, EPI>(w, M, p, e, s);
   if (sh.ks > 1 && sh.ks * sh.tp == kGemvWaves && ceil_div(KT, sh.ks) <= priv_kt) {
     switch (sh.ks) {
       case 2: return launch_gemv_priv<WD, PRO, EPI, 2>(w, M, p, e, s, num_cu);
@@ -1327,17 +1337,18 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_bigk_kernel(const uint4*
 // Llama-8B down_proj at 16 rows, the target's pass of a speculation step: 35 us for 59 MB).  The K
 // dimension of a row-tile is split over the 8 waves as everywhere, so a wave only ever multiplies ITS
 // K-slice: here it also stages that slice for itself, a sub-chunk of U k-tiles at a time, by LDS-DMA
-// (global_load_lds: no registers, no arithmetic -- hence bf16 activations only) into a double buffer of
+// (no registers, no arithmetic -- hence bf16 activations only) into a double buffer of
 // its own, two sub-chunks ahead together with the weight batch of the same k-tiles.  No work-group
 // barrier before the K-slice reduction of a row-tile.  The lane -> source-address map of the DMA does
 // the transpose into the MFMA B-fragment image (xfrag_slot: [k-chunk][row] 16-byte slots); a sub-chunk is always
 // 4 or 8 DMA instructions (U = 8 / 8 / 4 k-tiles for up to 4 / 8 / 16 rows), so the waits are
-// counted at compile time.  Same K-slices and MFMA order as gemv_bigk_kernel's chunks of one wave:
-// the products differ from it only in the association of the per-wave partial sums (none: each wave
+// counted at compile time; hipcc counts the weights beside them if the DMAs go through a descriptor and no load is
+// behind a branch of the loop (with either, it waited for all requests once per pair of sub-chunks: 20.4 us).
+// Same K-slices and MFMA order as gemv_bigk_kernel's chunks of one wave: the products differ from it only in the association of the per-wave partial sums (none: each wave
 // still adds its k-tiles in order, the waves are combined in wave order).
 constexpr int kKsBuf = 8 * 1024;                   // bytes of one wave-private activation buffer (<= 8 DMA instructions)
 // reduction buffer: [2 parities][waves 1..7][64 lanes] (wave 0 finishes from its own registers)
-constexpr size_t kGemvKstreamLds = (size_t)kGemvWaves * 2 * kKsBuf + 2 * (kGemvWaves - 1) * 64 * 16 + 64 * 4 + 16;
+constexpr size_t kGemvKstreamLds = (size_t)kGemvWaves * 2 * kKsBuf + 2 * (kGemvWaves - 1) * 64 * 16 + 2 * kGemvMaxTilesPerWg * 16 * 4 + 16;
 
 template <int WD, int EPI, int U, int kKsDma>   // U k-tiles and kKsDma DMA instructions (64 slots each) per sub-chunk
 __global__ __launch_bounds__(kGemvWaves * 64) void gemv_kstream_kernel(const uint4* __restrict__ W, int NT, int KT, int M,
@@ -1352,8 +1363,9 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_kstream_kernel(const uin
   unsigned char* tail = smem + (size_t)kGemvWaves * 2 * kKsBuf;
   constexpr int RW = kGemvWaves - 1;                                     // waves that hand their partial sums over
   f32x4_t* red = reinterpret_cast<f32x4_t*>(tail);                       // [2 parities][waves 1..7][64 lanes]
-  float* sc_lds = reinterpret_cast<float*>(tail + 2 * RW * 64 * 16);   // [2 parities][scale 16 | bias 16]
-  uint4* zero = reinterpret_cast<uint4*>(sc_lds + 64);
+  float* sc_lds = reinterpret_cast<float*>(tail + 2 * RW * 64 * 16);   // scales and biases of this work-group's row-tiles
+  float* bi_lds = sc_lds + kGemvMaxTilesPerWg * 16;
+  uint4* zero = reinterpret_cast<uint4*>(bi_lds + kGemvMaxTilesPerWg * 16);
   pin_sgpr(W); pin_sgpr(NT); pin_sgpr(KT); pin_sgpr(M); pin_sgpr(K); pin_sgpr(G); pin_sgpr(p.x); pin_sgpr(p.ldx);
   pin_sgpr(e.scale); pin_sgpr(e.bias); pin_sgpr(e.out_f32); pin_sgpr(e.ld_out);
   if constexpr (EPI == EPI_RESID) pin_sgpr(e.resid_in);
@@ -1378,49 +1390,49 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_kstream_kernel(const uin
     src_off[d] = sl < slots ? r * p.ldx + ch * 8 : -1;
     src_k[d] = ch * 8;
   }
-  auto issue_x = [&](int sel, int i) {
-    const bool live = i < total;
-    const int j = live ? i % nsc : 0;
-    const int k0 = (kbeg + j * U) * TK;                // first element of the sub-chunk
-    const int klim = kend * TK;
-#pragma unroll
-    for (int d = 0; d < kKsDma; ++d) {
-      // a slot past the wave's slice (or no slot at all) fetches the first line of x: never multiplied
-      const int off = src_off[d];
-      const bool ok = live && off >= 0 && k0 + src_k[d] < klim;
-      glds16(p.x + (ok ? (size_t)k0 + off : 0), xb + sel * kKsBuf + d * 1024);
-    }
-  };
+  const int xbytes = ((M - 1) * p.ldx + K) * 2;
+  int is_tile = 0, is_j = 0;                           // the next sub-chunk to request
   u32x4_t bufA[U], bufB[U];
-  auto issue_w = [&](u32x4_t (&buf)[U], int i) {
-    const bool live = i < total && kbeg < kend;
-    const int ii = min(i, max(total - 1, 0));
-    const int it = ii / nsc, j = ii - it * nsc;
-    const int tile = min((int)blockIdx.x + it * G, NT - 1);
-    const int klast = max(kend - 1, kbeg);
-    const uint4* base = live ? W + (size_t)tile * KT * 64 + lane : W;
-    const size_t kstep = live ? 64 : 0;
+  auto issue = [&](u32x4_t (&buf)[U], int sel) {
+    const bool live = is_tile < my_tiles;
+    const int kt0 = kbeg + is_j * U;
+    const int k0 = kt0 * TK;                           // first element of the sub-chunk
+    const int kn = live ? kend * TK - k0 : 0;
 #pragma unroll
-    for (int u = 0; u < U; ++u) stream_load16(buf[u], base + (size_t)min(kbeg + j * U + u, min(klast, KT - 1)) * kstep);
+    for (int d = 0; d < kKsDma; ++d) {                 // (a slot past the wave's slice, or no slot at all: zeros, and no request)
+      const int off = src_off[d];
+      blds16(p.x, xbytes, off >= 0 && src_k[d] < kn ? (k0 + off) * 2 : xbytes, xb + sel * kKsBuf + d * 1024);
+    }
+    stream_batch(buf, W, min((int)blockIdx.x + is_tile * G, NT - 1) * KT + kt0, live ? kend - kt0 : 0, lane);
+    if (++is_j == nsc) { is_j = 0; ++is_tile; }
   };
 
-  if (tid == 0) *zero = make_uint4(0, 0, 0, 0);
-  issue_x(0, 0);
-  issue_w(bufA, 0);
-  issue_x(1, 1);
-  issue_w(bufB, 1);
-  float scv = 0.f, biv = 0.f;                          // scale / bias of the row-tile in flight (threads 0..15)
-  __syncthreads();                                     // the zero slot
+  // asked for before the first sub-chunks and looked at behind them; a load inside the loop, under a branch, and hipcc waits for everything at its end
+  float scv[2] = {0.f, 0.f}, biv[2] = {0.f, 0.f};
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int jc = min(tid + q * kGemvWaves * 64, max(my_tiles * 16 - 1, 0));
+    const int at = min((int)blockIdx.x + (jc >> 4) * G, NT - 1) * 16 + (jc & 15);
+    scv[q] = e.scale[at];
+    biv[q] = e.bias ? e.bias[at] : 0.f;
+  }
+  EpiPre<EPI> epre{};
+  epi_prefetch<EPI>(e, min(c, M - 1), min((int)blockIdx.x, NT - 1) * 16 + g * 4, epre);
+  if (lane == 0) *zero = make_uint4(0, 0, 0, 0);       // (every wave the same: no barrier for it)
+  __builtin_amdgcn_sched_barrier(0);
+  issue(bufA, 0);
+  issue(bufB, 1);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    sc_lds[tid + q * kGemvWaves * 64] = scv[q];
+    bi_lds[tid + q * kGemvWaves * 64] = biv[q];
+  }
 
   f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
   int parity = 0;
-  auto process = [&](u32x4_t (&buf)[U], int sel, int i) {
-    const int it = i / nsc, j = i - it * nsc;
-    const int tile = (int)blockIdx.x + it * G;
-    if (j == 0 && tid < 16) {
-      scv = e.scale[tile * 16 + tid];
-      biv = e.bias ? e.bias[tile * 16 + tid] : 0.f;
-    }
+  int it = 0, j = 0;                                   // the sub-chunk being multiplied
+  auto process = [&](u32x4_t (&buf)[U], int sel) {
     // everything but the DMAs and weight loads of the NEXT sub-chunk has landed
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kKsDma + U) : "memory");
     const uint4* xf = reinterpret_cast<const uint4*>(xb + sel * kKsBuf);
@@ -1441,36 +1453,36 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_kstream_kernel(const uin
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(decode8<WD>(w[2], w[3]), b1, acc, 0, 0, 0);
       }
     }
-    if (j == nsc - 1) {   // row-tile done: combine the K-slices in wave order (wave 0's own partial first, then waves 1..7)
+    if (++j == nsc && it < my_tiles) {   // row-tile done: combine the K-slices in wave order (wave 0's own partial first, then waves 1..7)
+      const int tile = (int)blockIdx.x + it * G;
       if (wave > 0) red[(parity * RW + wave - 1) * 64 + lane] = acc;
-      if (tid < 16) { sc_lds[parity * 32 + tid] = scv; sc_lds[parity * 32 + 16 + tid] = biv; }
-      __syncthreads();
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (__syncthreads waits for the DMAs too, which no other wave reads)
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
       if (wave == 0 && tile < NT && col_ok) {
 #pragma unroll
         for (int w2 = 0; w2 < RW; ++w2) {
           const f32x4_t t = red[(parity * RW + w2) * 64 + lane];
           acc[0] += t[0]; acc[1] += t[1]; acc[2] += t[2]; acc[3] += t[3];
         }
-        epilogue_lds<EPI>(e, c, tile * 16 + g * 4, sc_lds + parity * 32 + g * 4, e.bias ? sc_lds + parity * 32 + 16 + g * 4 : nullptr, acc, 1.f);
+        const float* b4 = e.bias ? bi_lds + it * 16 + g * 4 : nullptr;
+        if (it == 0) epilogue_pre<EPI>(e, c, tile * 16 + g * 4, sc_lds + g * 4, b4, acc, epre);
+        else epilogue_lds<EPI>(e, c, tile * 16 + g * 4, sc_lds + it * 16 + g * 4, b4, acc, 1.f);
       }
       parity ^= 1;
+      j = 0;
+      ++it;
       acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
     // the buffer is re-filled next: its fragment reads must have returned
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
-  for (int i = 0; i < total; i += 2) {
-    process(bufA, 0, i);
-    issue_x(0, i + 2);
-    issue_w(bufA, i + 2);
-    if (i + 1 < total) {
-      process(bufB, 1, i + 1);
-    } else {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kKsDma + U) : "memory");   // keep the DMA / wait pairing of the loop
-    }
-    issue_x(1, i + 3);
-    issue_w(bufB, i + 3);
+  for (int i = 0; i < total; i += 2) {                 // (behind an odd number one of zeros that nobody keeps, instead of a branch)
+    process(bufA, 0);
+    issue(bufA, 0);
+    process(bufB, 1);
+    issue(bufB, 1);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // no DMA may land after the work-group has gone
 }
@@ -1484,7 +1496,7 @@ static int launch_gemv_kstream_u(const LinearW& w, int M, const ProArgs& p, cons
   int num_cu = 0;
   MI_TRY_(device_num_cu(&num_cu));
   int grid = NT;
-  if (NT > num_cu) grid = ceil_div(NT, ceil_div(NT, num_cu));
+  if (NT > num_cu) grid = ceil_div(NT, min(ceil_div(NT, num_cu), kGemvMaxTilesPerWg));
   hipLaunchKernelGGL(kern, dim3(grid), dim3(kGemvWaves * 64), kGemvKstreamLds, s, reinterpret_cast<const uint4*>(w.w), NT,
                      KT, M, w.K, grid, p, e);
   MI_HIP(hipGetLastError());
