@@ -58,13 +58,11 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
 #pragma unroll
     for (int mg = 0; mg < MG; ++mg) rfac[mg].request(e.row_scale ? e.row_scale : e.scale, e.row_scale ? min(mg * 16 + c, M - 1) : 0, e.rs_n);
   }
-  // operands of the epilogue of the first row-tile (every wave asks: see gemv_priv_kernel)
-  constexpr bool kPre = !SLAB && !(EPI == EPI_QKV && MG == 2);   // (two groups' rotary factors would not fit the registers)
-  EpiPre<kPre ? EPI : EPI_F32> epre[MG];
-  if constexpr (kPre) {
-#pragma unroll
-    for (int mg = 0; mg < MG; ++mg) epi_prefetch<EPI>(e, min(mg * 16 + c, M - 1), (int)blockIdx.x * 16 + g * 4, epre[mg]);
-  }
+  // operands of the epilogue of the first row-tile (and column group) that this wave finishes
+  constexpr bool kPre = !SLAB && HOLD == 1;
+  EpiPre<kPre ? EPI : EPI_F32> epre;
+  const int pre_pass = wave / MG, pre_m = min(wave % MG * 16 + c, M - 1), pre_n = tile_of(min(pre_pass, passes - 1)) * 16 + g * 4;
+  if constexpr (kPre) epi_prefetch<EPI>(e, pre_m, pre_n, epre);
   u32x4_t bufA[BT], bufB[BT];
   const int total = passes * NB;
   auto issue = [&](u32x4_t (&buf)[BT], int i) {
@@ -79,10 +77,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
 #pragma unroll
       for (int q = 0; q < FR * MG; ++q) xf[j * FR * MG + q] = u32x4_t{0, 0, 0, 0};
     }
-  if constexpr (kPre) {
-#pragma unroll
-    for (int mg = 0; mg < MG; ++mg) epi_prefetch_dependent<EPI>(e, (int)blockIdx.x * 16 + g * 4, epre[mg]);
-  }
+  if constexpr (kPre) epi_prefetch_dependent<EPI>(e, pre_n, epre);
   if constexpr (!SLAB) {
     const int n = passes * 16;
 #pragma unroll
@@ -169,7 +164,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
         const float *sc4 = sc_lds + pass * 16 + g * 4, *b4 = e.bias ? bi_lds + pass * 16 + g * 4 : nullptr;
         bool done = false;
         if constexpr (kPre) {
-          if (pass == 0) { epilogue_pre<EPI>(e, m, n0, sc4, b4, s, epre[mg], rmul[mg]); done = true; }
+          if (pass == pre_pass) { epilogue_pre<EPI>(e, m, n0, sc4, b4, s, epre, rmul[mg]); done = true; }
         }
         if (!done) epilogue_lds<EPI>(e, m, n0, sc4, b4, s, rmul[mg]);
       }

@@ -869,7 +869,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_priv_kernel(const uint4*
       biv[q] = e.bias ? e.bias[tile * 16 + r] : 0.f;
     }
   }
-  const int tile0 = min((int)blockIdx.x * TP + tsub, NT - 1);
+  const int tile0 = min((int)(blockIdx.x + kslice * G) * TP + tsub, NT - 1);   // the first that this wave finishes
   EpiPre<EPI> epre{};
   // unconditional (every wave asks, the finishers use it): under a branch hipcc waits for the load
   // at the merge point -- vmcnt(0) in front of the first weight request
@@ -964,11 +964,12 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_priv_kernel(const uint4*
       const int tile = (int)(blockIdx.x + pass * G) * TP + tsub;
       red[(parity * kGemvWaves + wave) * 64 + lane] = acc;
       __syncthreads();
-      if (kslice == 0 && col_ok && tile < NT) {
-        f32x4_t sum = red[(parity * kGemvWaves + wave) * 64 + lane];
+      if (kslice == (pass & (KS - 1)) && col_ok && tile < NT) {   // (in turn: what a wave's first row-tile needs is here by then;
+                                                                  // always the first wave: 8B fp8 1 row 1003 us, so 977, bf16 2 rows 1586 and 1554)
+        f32x4_t sum = red[(parity * kGemvWaves + tsub * KS) * 64 + lane];
 #pragma unroll
         for (int w = 1; w < KS; ++w) {
-          const f32x4_t t = red[(parity * kGemvWaves + wave + w) * 64 + lane];
+          const f32x4_t t = red[(parity * kGemvWaves + tsub * KS + w) * 64 + lane];
           sum[0] += t[0]; sum[1] += t[1]; sum[2] += t[2]; sum[3] += t[3];
         }
         float rmul = 1.f;
@@ -981,7 +982,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_priv_kernel(const uint4*
         const int lslot = (pass * TP + tsub) * 16 + g * 4;
         const float* sc4 = sc_lds + lslot;
         const float* b4 = e.bias ? bi_lds + lslot : nullptr;
-        if (pass == 0) epilogue_pre<EPI>(e, c, tile * 16 + g * 4, sc4, b4, sum, epre, rmul);
+        if (pass == kslice) epilogue_pre<EPI>(e, c, tile * 16 + g * 4, sc4, b4, sum, epre, rmul);
         else epilogue_lds<EPI>(e, c, tile * 16 + g * 4, sc4, b4, sum, rmul);
       }
       parity ^= 1;
