@@ -206,3 +206,22 @@ def test_llama_epilogues_agree_with_the_128x128_kernel(tmp_path, hd, heads, kv, 
         for other in got[1:]:
             d = other[n] - want
             assert torch.isfinite(d).all() and d.pow(2).mean().sqrt() < 0.02 * want.std(), n    # the bar of the other dispatch test
+
+
+# Small whole numbers: the slices' sum is exact in fp32 in any order, so scale and bias are all that rounds, and the launch that adds slices makes one fused multiply-add of them.
+# (Two roundings, half a unit each of numbers twice the result's size, would be off by more than half a unit of the result in a part of the rows.)
+@pytest.mark.parametrize("M,N,K,ks", [(33, 272, 704, 3), (100, 1040, 1984, 8), (188, 528, 320, 2)])
+def test_sums_of_slices_round_once(lib, M, N, K, ks):
+    g = torch.Generator().manual_seed(M + N + K)
+    q = torch.randint(-20, 21, (N, K), generator=g).float()
+    q[:, 0] = 127                                                     # int8 codes are these numbers
+    x = torch.randint(-3, 4, (M, K), generator=g).to(torch.bfloat16)
+    bias = torch.randn(N, generator=g) * 20
+    tiled, scale = quantize_on_device(lib, q * (0.3 + torch.rand(N, 1, generator=g)) / 127, "int8", "per_channel_symmetric")
+    y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    xd, bd = dev(x), dev(bias)
+    lib.check(lib.load_library().mi_op_qlinear(xd.data_ptr(), M, tiled.data_ptr(), scale.data_ptr(), bd.data_ptr(), N, K, WD["int8"], y.data_ptr(), 6420 + ks, None))
+    torch.cuda.synchronize()
+    ref = (x.double() @ q.double().t()) * scale.cpu().double() + bias.double()      # 48 bits and a sum: 64-bit rounding is 2^-29 of a unit here
+    unit = 2.0 ** (torch.frexp(ref.abs())[1].double() - 24)
+    assert ((y.cpu().double() - ref).abs() <= 0.50001 * unit).all()

@@ -211,6 +211,9 @@ struct RowFactor {
   }
   __device__ __forceinline__ float value(float n, float eps) const { return n > 0.f ? rsqrtf(((a + b) + (c + d)) / n + eps) : a; }
 };
+// the same in two steps where the parts are known to be there
+__device__ __forceinline__ float4 row_parts(const float* p, int m) { return *reinterpret_cast<const float4*>(p + kNormParts * m); }
+__device__ __forceinline__ float row_rinv(float4 ss, float n, float eps) { return rsqrtf(((ss.x + ss.y) + (ss.z + ss.w)) / n + eps); }
 // The sum of KS slabs' four numbers at p, `stride` numbers apart, in slice order.  Five requests leave before the first is waited for: one after the
 // other they cost a trip to memory each (the row norm over 8 slabs of 242 x 4096: 13.9 us that way, 9.3 now, of which the bytes take 6.3).
 struct Nothing { __device__ __forceinline__ void operator()() const {} };
