@@ -409,6 +409,7 @@ static int launch_gemm_wide_t(const LinearW& w, int T, const uint16_t* x, int ld
 template <int WD, int BM, int NTW>
 static int launch_gemm_wide_bm(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
                                int KS, float* ws, SlabSum* defer) {
+  MI_CHECK(e.rs_n == 0.f || BM == 32 || KS > 1, "gemm_wide: the parts of a norm are for blocks of 32 tokens");
   if (KS > 1) {
     MI_TRY_((launch_gemm_wide_t<WD, EPI_F32, BM, NTW, true>(w, T, x, ldx, e, s, KS, ws)));
     const SlabSum sum{ws, KS, T, w.N, e.scale, e.bias, e.row_scale, e.rs_n, e.rs_eps};

@@ -28,9 +28,7 @@ template <int EPI>
 __device__ __forceinline__ void epilogue(const EpiArgs& e, int m, int n0, f32x4_t v) {
   float4 sc = *reinterpret_cast<const float4*>(e.scale + n0);
   if (e.row_scale) {   // FP8 activations: the token's scale multiplies the channel's
-    RowFactor f;
-    f.request(e.row_scale, m, e.rs_n);
-    const float rs = f.value(e.rs_n, e.rs_eps);
+    const float rs = e.row_scale[m];
     sc.x *= rs; sc.y *= rs; sc.z *= rs; sc.w *= rs;
   }
   v[0] *= sc.x; v[1] *= sc.y; v[2] *= sc.z; v[3] *= sc.w;
@@ -216,6 +214,7 @@ __device__ __forceinline__ void epilogue_pre(const EpiArgs& e, int m, int n0, co
 // tile of 32-byte pieces in 6 us longer than one of 64-byte pieces, which are as fast as whole lines through LDS.
 // us, before -> now, in turn: 12288 x 2048 squared relu, 777 tokens 62.4 -> 56.4, 4000 tokens 226 -> 203; gate|up of the 8B model, bf16 1000 tokens 246 -> 238,
 // fp8 242 tokens 64.7 -> 62.5 (without any store 50, 184, 224, 59).
+// MT = 1 (blocks of 32 tokens) may have the rows' factors as the parts of a norm; larger blocks do not: the requests for them cost 256 x 256 a register it had not.
 template <int EPI, int NTW, int MT>
 __device__ __forceinline__ void epilogue_tile(const EpiArgs& e, int T, int NT, int mb, int nb, int g, int c, f32x4_t (&acc)[NTW][MT]) {
   if (mb >= T) return;
@@ -251,13 +250,8 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& e, int T, int NT, i
   };
   Operands ops[2];
   request(ops[0], 0);
-  if (e.rs_n > 0.f) {       // (calls of few rows)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      RowFactor f;
-      f.request(e.row_scale, mb + row(mt), e.rs_n);
-      rs[mt] = f.value(e.rs_n, e.rs_eps);
-    }
+  if constexpr (MT == 1) {
+    if (e.rs_n > 0.f) rs[0] = row_rinv(row_parts(e.row_scale, mb + row(0)), e.rs_n, e.rs_eps);
   }
 #pragma unroll
   for (int i = 0; i < NTW; ++i) {

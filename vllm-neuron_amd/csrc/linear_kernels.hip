@@ -351,7 +351,7 @@ static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, boo
   double best_cost = 0.;
   for (const int bm : {32, 64, 96, 128, 160, 192, 256})
     for (int ntw = 2; ntw <= 4; ++ntw) {
-      if (bm == 32 && T > 32) break;
+      if ((bm == 32) != (T <= 32)) break;        // (32 tokens are the cheapest block that holds them: every term grows with m)
       const double m = bm / 64., area = m * ntw;
       const auto us = [&](const double (&k)[4]) { return k[0] + k[1] * area + k[2] * m + k[3] * ntw; };
       const bool by_32 = wide_tile_by_32(wd, bm, ntw), deep_tile = wide_tile_deep(wd, bm, ntw) && K % 128 == 0;
