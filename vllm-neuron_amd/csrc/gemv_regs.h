@@ -31,6 +31,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
   static_assert(NB * BT == NK, "whole batches");
   __shared__ f32x4_t red[2][kGemvWaves][MG][64];
   __shared__ __attribute__((aligned(16))) float sc_lds[SLAB ? 4 : kRegsMaxPasses * 16], bi_lds[SLAB ? 4 : kRegsMaxPasses * 16];
+  __shared__ float rf_lds[SLAB ? 1 : 16 * MG];        // the rows' own factors: 1 / rms where the norm left it to the output
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int g = lane >> 4, c = lane & 15;
   const int kper = ceil_div(KT, (int)gridDim.y), k_lo = (int)blockIdx.y * kper, k_hi = min(k_lo + kper, KT);
@@ -53,13 +54,8 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
     }
   }
   __builtin_amdgcn_sched_barrier(0);
-  RowFactor rfac[MG];                                 // the row's own factor: 1 / rms where the norm left it to the output
-  if constexpr (!SLAB) {
-#pragma unroll
-    for (int mg = 0; mg < MG; ++mg) rfac[mg].request(e.row_scale ? e.row_scale : e.scale, e.row_scale ? min(mg * 16 + c, M - 1) : 0, e.rs_n);
-  }
   // operands of the epilogue of the first row-tile (and column group) that this wave finishes
-  constexpr bool kPre = !SLAB && HOLD == 1;
+  constexpr bool kPre = !SLAB && HOLD == 1 && !(EPI == EPI_QKV && MG == 2);   // (two groups' rotary factors would not fit the registers)
   EpiPre<kPre ? EPI : EPI_F32> epre;
   const int pre_pass = wave / MG, pre_m = min(wave % MG * 16 + c, M - 1), pre_n = tile_of(min(pre_pass, passes - 1)) * 16 + g * 4;
   if constexpr (kPre) epi_prefetch<EPI>(e, pre_m, pre_n, epre);
@@ -79,6 +75,8 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
     }
   if constexpr (kPre) epi_prefetch_dependent<EPI>(e, pre_n, epre);
   if constexpr (!SLAB) {
+    RowFactor rf;                                     // (a thread a row; all ask, so that no branch waits for it)
+    rf.request(e.row_scale ? e.row_scale : e.scale, e.row_scale ? min(tid, M - 1) : 0, e.rs_n);
     const int n = passes * 16;
 #pragma unroll
     for (int q = 0; q < kRegsMaxPasses * 16 / (kGemvWaves * 64); ++q) {
@@ -89,11 +87,9 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
         bi_lds[i] = e.bias ? e.bias[at] : 0.f;
       }
     }
+    if (tid < 16 * MG) rf_lds[tid] = e.row_scale ? rf.value(e.rs_n, e.rs_eps) : 1.f;
   }
   issue(bufB, 1);
-  float rmul[MG];
-#pragma unroll
-  for (int mg = 0; mg < MG; ++mg) rmul[mg] = !SLAB && e.row_scale ? rfac[mg].value(e.rs_n, e.rs_eps) : 1.f;
 
   f32x4_t acc[MG];
 #pragma unroll
@@ -139,10 +135,10 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
       const int m = mg * 16 + c, n0 = tile_of(pass) * 16 + g * 4;
       if constexpr (HOLD > 1) {
         static_assert(!SLAB && (EPI == EPI_F32 || EPI == EPI_SOFTCAP), "rows of fp32");
-        const float *sc4 = sc_lds + pass * 16 + g * 4, *b4 = bi_lds + pass * 16 + g * 4;
+        const float *sc4 = sc_lds + pass * 16 + g * 4, *b4 = bi_lds + pass * 16 + g * 4, rmul = rf_lds[m];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          s[r] *= sc4[r] * rmul[mg];
+          s[r] *= sc4[r] * rmul;
           if (e.bias) s[r] += b4[r];
           if constexpr (EPI == EPI_SOFTCAP) s[r] = e.softcap * tanhf(s[r] / e.softcap);
         }
@@ -161,12 +157,12 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
       if constexpr (SLAB) {
         *reinterpret_cast<float4*>(slab + ((size_t)blockIdx.y * M + m) * (NT * 16) + n0) = make_float4(s[0], s[1], s[2], s[3]);
       } else {
-        const float *sc4 = sc_lds + pass * 16 + g * 4, *b4 = e.bias ? bi_lds + pass * 16 + g * 4 : nullptr;
+        const float *sc4 = sc_lds + pass * 16 + g * 4, *b4 = e.bias ? bi_lds + pass * 16 + g * 4 : nullptr, rmul = rf_lds[m];
         bool done = false;
         if constexpr (kPre) {
-          if (pass == pre_pass) { epilogue_pre<EPI>(e, m, n0, sc4, b4, s, epre, rmul[mg]); done = true; }
+          if (pass == pre_pass) { epilogue_pre<EPI>(e, m, n0, sc4, b4, s, epre, rmul); done = true; }
         }
-        if (!done) epilogue_lds<EPI>(e, m, n0, sc4, b4, s, rmul[mg]);
+        if (!done) epilogue_lds<EPI>(e, m, n0, sc4, b4, s, rmul);
       }
     }
   };
