@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from oracle.nusovik import bucket
 from tests.helpers import pool_to_native
 from tests.test_ops_gpu import _make_pool, dev, lib, ref_attention  # noqa: F401  (lib: the fixture)
 from tests.test_vimesun_gpu import spec_of
@@ -74,3 +75,31 @@ def test_long_windows(lib, d, bs, tiles, window):  # noqa: F811
         s = torch.einsum("hd,nhd->hn", q[b, :, :d].double(), K.repeat_interleave(2, 1)) * d ** -0.5
         ref = torch.einsum("hn,nhd->hd", torch.softmax(s, -1), W.repeat_interleave(2, 1)).flatten()
         assert (out[b, :16 * d].cpu().double() - ref).abs().max().item() < 0.02, (b, ctx[b])      # as above
+
+
+# chunked attention with its distance table and sinks, so many kv heads that one work-group's four waves take a whole context (128 tokens to each of their tiles): no tile, one, two and three for a wave, the last of a look, the first of the next, a third look
+@pytest.mark.parametrize("n", [1, 33, 128, 129, 257, 300, 400, 128 * 31 + 5, 128 * 32, 128 * 32 + 1, 128 * 33, 128 * 63 + 20])
+def test_tables_and_tiles(lib, n):  # noqa: F811
+    H, G, d, bs, mult = 130, 130, 32, 32, 0.7
+    MB = -(-n // bs) + 1
+    bt, nb = _tables([n], bs, MB, 0)
+    g = torch.Generator().manual_seed(n)
+    k, v = (torch.randn(nb, G, bs, d, generator=g).to(torch.bfloat16) for _ in range(2))
+    k[0], v[0] = 50., 50.                                  # (nobody's block)
+    q = torch.randn(1, H, d, generator=g).to(torch.bfloat16)
+    rel, sink, gate = torch.randn(16, H, generator=g) * 2, torch.randn(H, generator=g) + 1, torch.randn(1, H, generator=g)
+    out = torch.zeros(1, H * d, dtype=torch.bfloat16, device="cuda")
+    spec = lib.layer_spec(dict(num_heads=H, num_kv_heads=G, qk_dim=d, v_dim=d, chunk=8200, scale=0.1, rel_rows=16, rel_far=200, softmax_sink=2))
+    pos = torch.tensor([n - 1], dtype=torch.int32)
+    x = [dev(t) for t in (sink, rel, gate, q, k, v, bt, pos, pos + 1)]
+    segs = torch.tensor([(0, 1, n - 1, 0)], dtype=torch.int32).contiguous()
+    lib.check(lib.load_library().mi_op_chunk_attn(spec, x[0].data_ptr(), x[1].data_ptr(), x[2].data_ptr(), H, mult, x[3].data_ptr(), x[4].data_ptr(), x[5].data_ptr(), bs,
+                                                  x[6].data_ptr(), MB, x[7].data_ptr(), x[8].data_ptr(), segs.data_ptr(), 1, 1, n, out.data_ptr(), H * d, 0, 0, None))
+    torch.cuda.synchronize()
+    idx = torch.arange(n)
+    blk = bt[0, idx // bs].long()
+    K, V = (t[blk, :, idx % bs].double().repeat_interleave(H // G, 1) for t in (k, v))
+    rows = torch.tensor([bucket(n - 1 - i, 16, 200) for i in range(n)])
+    s = torch.cat([torch.einsum("hd,nhd->hn", q[0].double(), K) * 0.1 + rel.double()[rows].t(), sink.double()[:, None]], 1)
+    ref = torch.einsum("hn,nhd->hd", torch.softmax(s, -1)[:, :n], V) * mult * torch.sigmoid(gate[0].double())[:, None]
+    assert ((out.cpu().double().reshape(H, d) - ref).abs() <= 1.5e-2 * (1 + ref.abs())).all()      # as the tests of chunked attention
