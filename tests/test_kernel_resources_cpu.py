@@ -32,7 +32,7 @@ def kernels():
     return found
 
 
-@pytest.mark.parametrize("kernel", ["splitk_reduce_kernel", "gemm_wide", "gemv_"])
+@pytest.mark.parametrize("kernel", ["splitk_reduce_kernel", "gemm_wide", "gemv_", "attn_window_decode_kernel", "attn_decode_kernel"])
 def test_nothing_in_scratch(kernel):
     mine = {n: k for n, k in kernels().items() if kernel in n}
     assert mine

@@ -606,8 +606,9 @@ __global__ __launch_bounds__(NW * 64) void attn_window_decode_kernel(AttnSpec a,
   };
 
   // a single tile by itself: requests without bytes take their time too (4 kv heads of 64, us a launch: 40 tokens 4.5 -> 3.8; with a table, whose
-  // requests behind the context are left out as well, 5.5 -> 4.8, 3000 tokens in chunks of 256 8.7 -> 8.1)
-  if (mine == 1) update(kA, vA, bA, t_first);
+  // requests behind the context are left out as well, 5.5 -> 4.8, 3000 tokens in chunks of 256 8.7 -> 8.1).  (heads of 256: a third copy of the update does not
+  // fit the registers)
+  if (DK + DV < 512 && mine == 1) update(kA, vA, bA, t_first);
   else for (int i = 0; i < mine; i += 2) {
     if (i + 3 > i_base + kIds) {
       i_base = i;
