@@ -177,9 +177,29 @@ def test_logits_of_many_rows_to_the_host(vocab):
         model.close()
 
 
-# 17 .. 32 rows of one-byte weights leave the register kernel where deep K slices are summed by the next norm (2048 wide), and where unsplit K fills the chip (fp8 gate | up
-# of 24576 rows); not for sums of 256 wide
-@pytest.mark.parametrize("wd,hidden,inter", [("f8e4m3", 256, 4096), ("f8e4m3", 3584, 12288), ("int8", 256, 16384), ("f8e4m3", 2048, 4096), ("int8", 2048, 17408)])
+# Which of the two kernels takes 17 .. 32 rows of one-byte weights: the register kernel's sums over unsplit K are those of 16 rows bit for bit, the wide GEMM's are not.  Either side of the
+# measured line by some us of 15 to 65 (profiles/few_rows_sweep.txt): shallow K stays, however full its tiles make the chip; deep and wide goes, unsplit and in slices; int8 later than fp8
+@pytest.mark.parametrize("wd,N,K,rows,wide", [("f8e4m3", 49152, 6144, 17, True), ("int8", 49152, 6144, 32, True), ("f8e4m3", 10240, 8192, 20, True), ("int8", 20480, 5120, 32, False),
+                                              ("f8e4m3", 28672, 3584, 17, False), ("f8e4m3", 16384, 3072, 32, False)])
+def test_the_faster_kernel(lib, wd, N, K, rows, wide):
+    g = torch.Generator().manual_seed(N + rows)
+    w = torch.randn(N, K, generator=g) * 0.05
+    x, bias = torch.randn(rows, K, generator=g).to(torch.bfloat16), torch.randn(N, generator=g) * 0.1
+    tiled, scale = quantize_on_device(lib, w, wd, "per_channel_symmetric")
+    xd, bd, out = dev(x), dev(bias), []
+    for m in (16, rows):
+        y = torch.full((m, N), float("nan"), dtype=torch.float32, device="cuda")
+        lib.check(lib.load_library().mi_op_qlinear(xd.data_ptr(), m, tiled.data_ptr(), scale.data_ptr(), bd.data_ptr(), N, K, WD[wd], y.data_ptr(), 8, None))
+        torch.cuda.synchronize()
+        out.append(y.cpu())
+    assert torch.isfinite(out[1]).all() and torch.equal(out[0], out[1][:16]) != wide
+    assert (out[0] - out[1][:16]).abs().max().item() < 2e-5 * out[0].abs().max().item() + 1e-5 * (K ** 0.5)      # as above
+
+
+# 17 .. 32 rows of one-byte weights leave the register kernel where deep K slices are summed by the next norm (2048 wide), where unsplit K fills the chip (fp8 gate | up
+# of 24576 rows, from 25 rows on) and where it is deep besides (fp8 32768 x 5120, int8 32768 x 6144); not for sums of 256 wide
+@pytest.mark.parametrize("wd,hidden,inter", [("f8e4m3", 256, 4096), ("f8e4m3", 3584, 12288), ("int8", 256, 16384), ("f8e4m3", 2048, 4096), ("int8", 2048, 17408), ("f8e4m3", 5120, 16384),
+                                             ("int8", 6144, 16384)])
 def test_rows_on_both_sides_of_the_wide_gemm(wd, hidden, inter):
     from oracle import DecoderConfig
     from oracle.synth import make_weights

@@ -229,7 +229,7 @@ static int launch_gemv_regs_k(const LinearW& w, int M, const uint16_t* x, int ld
 // sums have a taker.  us: a work-group's weights at 24 GB/s, its rows at 50 GB/s, the slabs both ways, and a launch that adds them where no row norm does.
 // (Without the rows' term, us a step: 8B fp8 32 rows 2150, 2099 with it; bf16 24 rows 2323, 2261; 7B int8 24 rows 1820, 1801; Rapodra 20 rows 731, 721.)
 template <int WD>
-static int gemv_regs_slices(int M, int N, int K, size_t ws_bytes, bool deferred, int num_cu) {
+static int gemv_regs_slices(int M, int N, int K, size_t ws_bytes, bool deferred, int num_cu, double* us = nullptr) {
   const int NT = N / 16, KT = K / tile_k(WD);
   int best = 0;
   double best_cost = 0.;
@@ -240,6 +240,7 @@ static int gemv_regs_slices(int M, int N, int K, size_t ws_bytes, bool deferred,
     if (z > 1) cost += (deferred ? 0.5 : 4.5) + z * (double)M * N * 1e-6;
     if (best == 0 || cost < best_cost) { best = z; best_cost = cost; }
   }
+  if (us) *us = best_cost;
   return best;
 }
 
@@ -289,14 +290,13 @@ bool gemv_regs_fits_wd(int M, int N, int K, size_t ws_bytes) {
   return device_num_cu(&num_cu) == MI_OK && gemv_regs_slices<WD>(M, N, K, ws_bytes, false, num_cu) > 0;
 }
 
-// Which part of a wave's requests are k-tiles of its own, the sum of the slices having a taker: a row-tile's 4 .. 8 go out whatever it owns (by_fours: as if they were 4 or 8).
+// what the choice of slices takes the launch and the sum of its slices to be, us; 0: no split fits
 template <int WD>
-double gemv_regs_own_wd(int M, int N, int K, size_t ws_bytes, bool by_fours) {
+double gemv_regs_us_wd(int M, int N, int K, size_t ws_bytes, bool deferred) {
   int num_cu = 0;
-  const int z = device_num_cu(&num_cu) == MI_OK ? gemv_regs_slices<WD>(M, N, K, ws_bytes, true, num_cu) : 0;
-  if (z == 0) return 1.;
-  const int KT = K / tile_k(WD), tiles = ceil_div(ceil_div(KT, z), kGemvWaves);
-  return (double)KT / (z * kGemvWaves * (tiles <= 4 ? 4 : by_fours ? 8 : tiles));
+  double us = 0.;
+  if (device_num_cu(&num_cu) == MI_OK) gemv_regs_slices<WD>(M, N, K, ws_bytes, deferred, num_cu, &us);
+  return us;
 }
 
 }  // namespace mi

@@ -43,7 +43,7 @@ extern template int launch_gemv_wd<MI_W_INT8>(const LinearW&, int, int, const Pr
 template <int WD>
 int launch_gemv_regs_wd(const LinearW& w, int M, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s, float* ws, size_t ws_bytes, SlabSum* defer, bool split_as_deferred);
 template <int WD> bool gemv_regs_fits_wd(int M, int N, int K, size_t ws_bytes);
-template <int WD> double gemv_regs_own_wd(int M, int N, int K, size_t ws_bytes, bool by_fours);
+template <int WD> double gemv_regs_us_wd(int M, int N, int K, size_t ws_bytes, bool deferred);
 
 static bool gemv_regs_fits(const LinearW& w, int M, size_t ws_bytes) {
   switch (w.wd) {
@@ -81,38 +81,6 @@ static int gemm_wide_mode() {   // MI355X_GEMM_WIDE: 0 never, 1 whenever the sha
 static int gemm_wide_bm() {      // MI355X_GEMM_WIDE_BM: 128 / 256 forces the token block (default: by grid size)
   static const int m = [] { const char* v = getenv("MI355X_GEMM_WIDE_BM"); const int b = v ? atoi(v) : 0; return b == 128 || b == 256 ? b : 0; }();
   return m;
-}
-// Rows beside which the register kernel takes in more of the activations than of the weights' share of a CU, in front of the first weights; the wide GEMM brings both side by side.
-// us a launch at 24 / 32 rows, register kernel -> blocks of 32 tokens, weights from memory: 4096 x 4096 fp8 11.8 / 13.0 -> 8.8 / 9.2, 4096 x 14336 fp8 16.0 / 17.2 -> 15.7 / 15.3,
-// 28672 x 4096 fp8 26.4 / 27.7 -> 24.8 / 25.5, 3584 x 18944 int8 23.6 / 25.2 -> 20.7 / 20.7.  Not: int8 unsplit, whose codes the smallest tiles decode too often (37888 x 3584
-// 32.0 / 34.2 -> 33.8 / 34.8), bf16 (28672 x 4096 42.8 / 44.0 -> 45.8 / 47.0), up to 16 rows (23.4 -> 23.8); nor shallower K (us a call: 8B int8 28 rows 1834 -> 1845, TinyLlama
-// fp8 30 rows 1260 -> 1272).  The lines below are drawn through us a layer of 78 models of 1024 .. 8192 wide, feed-forwards of 3584 .. 28672, at 17 .. 32 rows, one projection after the
-// other moved to the wide GEMM in the same model:
-// K slices whose sum the next norm takes: by the share of a register wave's requests that are k-tiles of its own (counted as if they went out by 4 and 8, as they did when the
-// lines were drawn; those it does not have repeat the last).
-// fp8: up to 27 / 32 of them 0 .. 9 less; beyond that 0.5 .. 3 less where the wide GEMM's tiles times ten slices at most fill the chip (N of 3584, 4096, 4608, 8192), else up to 4 more
-// (7168 x 17408 17 rows; 6144 x 16384 1.4); 3584 x 3584 0.2 .. 1.7 more.  int8: up to 5 / 8 0.7 .. 8 less, beyond that between 3 less and 2 more (3072 x 24576; 4608 x 16384); since 5 .. 7 have kernels
-// of their own the register kernel is the faster one where more than 0.86 of what goes out is its own (3584 x 18944, 17 / 20 / 28 / 32 rows a step of the 7B model 1410 -> 1376, 1486 -> 1452, 1637 -> 1596, 1725 -> 1686).  Where the
-// weights themselves take longest the register kernel streams them faster (fp8 7168 x 22016 4 more, 8192 x 28672 5, int8 7168 x 28672 4; fp8 8192 x 17408 still 5 .. 9 less), and narrow sums leave the wide GEMM
-// half of the chip and more (1536 x 11008 fp8 0.6 more, 1536 x 20480 int8 1.5, 1024 x 20480 2.8).
-// Unsplit gate | up of fp8 that fills three quarters of the chip in one round: 0.5 .. 12 less.
-// Queries, keys and values of fp8 from 25 rows on, though a launch has to add their slices (6144 x 4096 15.9 -> 10.8 + 4.1 at 32 rows; 20 rows 13.8 -> 10.0 + 4.1: not): a kv head for
-// four q heads and more 1 .. 4.5 less, one for each 2 .. 6; between, from 6 less (10240 x 5120) to 1.4 more (7168 x 3584); 8192 wide 0 (10240) and 4 more (12288).
-bool gemm_wide_few_rows(const LinearW& w, int M, int epi, size_t ws_bytes, bool deferred) {
-  int cus = 0;
-  if (gemm_wide_mode() == 0 || gemm_wide_bm()) return false;      // (128 tokens and more: none of these calls has them)
-  if (M < 17 || M > 32 || w.wd == MI_W_BF16 || w.K % 64 != 0 || w.N < 32 || device_num_cu(&cus) != MI_OK) return false;
-  const int tiles = ceil_div(w.N, 128);      // of the wide GEMM, one work-group a CU
-  const bool fp8 = w.wd == MI_W_F8E4M3;
-  if (deferred) {
-    if (w.K < (fp8 ? 4096 : 16384) || w.N < 2048 || (size_t)w.N * w.K > 150000000) return false;
-    const auto own = [&](bool by_fours) { return fp8 ? gemv_regs_own_wd<MI_W_F8E4M3>(M, w.N, w.K, ws_bytes, by_fours) : gemv_regs_own_wd<MI_W_INT8>(M, w.N, w.K, ws_bytes, by_fours); };
-    if (own(true) <= (fp8 ? 27. / 32. : 5. / 8.) && (fp8 || own(false) <= 0.86)) return true;
-    return fp8 && w.K >= 8192 && tiles * std::min(10, cus / tiles) * 16 > cus * 15;
-  }
-  if (!fp8 || w.K < 3584) return false;
-  if (epi == EPI_QKV) return M >= 25 && w.K <= 7168 && (2 * w.N <= 3 * w.K || w.N >= 3 * w.K);
-  return tiles >= cus * 3 / 4 && tiles <= cus;
 }
 int launch_gemv_regs(const LinearW& w, int M, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s, float* ws, size_t ws_bytes, SlabSum* defer,
                      bool split_as_deferred) {
@@ -329,7 +297,7 @@ extern template int launch_gemm_wide_wd<MI_W_INT8>(const LinearW&, int, const ui
 // Against the best of 128 x 256 and 256 x 256 alone, us: int8 gate|up of the 7B model at 188 tokens 79 -> 60 (148 tiles of 256 x 256 on 256 CUs, 73 % of
 // each filled; 198 of 192 x 192), its down projection 41.6 -> 34.4; bf16 gate|up of TinyLlama 700 tokens 51.6 -> 35.4, 200 tokens 28.4 -> 21.4;
 // fp8 QKV of the 8B model 1400 tokens 82.6 -> 63.9; bf16 down projection of 2048 x 14336 at 100 tokens 26.4 -> 17.6.
-struct WidePlan { int bm, ntw, ks; };
+struct WidePlan { int bm, ntw, ks; double us; };
 static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, bool deferred) {
   int cus = 256;
   if (device_num_cu(&cus) != MI_OK || cus < 8) cus = 256;
@@ -347,8 +315,7 @@ static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, boo
   const Model& r = kModel[wd];
   const int nks = K / 64;
   const double mb = (double)T * N * 4e-6, stream = (double)N * K * elem_bytes(wd) * 1e-6 / r.stream;
-  WidePlan best{0, 4, 1};   // (bm 0: none compared yet; one slice is always allowed, so there is one)
-  double best_cost = 0.;
+  WidePlan best{0, 4, 1, 0.};   // (bm 0: none compared yet; one slice is always allowed, so there is one)
   for (const int bm : {32, 64, 96, 128, 160, 192, 256})
     for (int ntw = 2; ntw <= 4; ++ntw) {
       if ((bm == 32) != (T <= 32)) break;        // (32 tokens are the cheapest block that holds them: every term grows with m)
@@ -370,7 +337,7 @@ static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, boo
         double cost = r.launch + std::sqrt(body * body + stream * stream);
         if (ks > 1) cost += r.slab * ks * mb + (deferred ? 0.144 * ks * mb : 3.38 + 0.113 * (ks + 1) * mb);
         else if (2 * tiles <= cus) cost *= 1.12;   // (half of the CUs at most: longer inside a call than alone)
-        if (best.bm == 0 || cost < best_cost) { best = WidePlan{bm, ntw, ks}; best_cost = cost; }
+        if (best.bm == 0 || cost < best.us) best = WidePlan{bm, ntw, ks, cost};
       }
     }
   return best;
@@ -378,6 +345,34 @@ static WidePlan gemm_wide_plan(int T, int N, int K, size_t ws_bytes, int wd, boo
 static int gemm_wide_ks() {      // MI355X_GEMM_WIDE_KS: 1 = never split K in the wide kernel
   static const int m = [] { const char* v = getenv("MI355X_GEMM_WIDE_KS"); return v ? atoi(v) : 0; }();
   return m;
+}
+// Rows beside which the register kernel takes in more of the activations than of the weights' share of a CU, in front of the first weights; the wide GEMM brings both side by side,
+// but streams long weights no faster and decodes int8 codes once for every two waves that read them.  Which is the faster one: by what the two choices of slices take their
+// launches to be, each with the sum of its slices.  Both are models of a kernel alone; a line for each of the three ways a sum goes ties them together, drawn through us a layer of
+// 36 models of 1024 .. 8192 wide, feed-forwards of 3584 .. 28672, at 17, 20, 24, 28 and 32 rows, one projection after the other moved to the wide GEMM in the same model (1400 comparisons;
+// profiles/few_rows_sweep.txt).  What the choice loses against the faster one of the two, us a layer of 40 .. 330, on the mean, fp8 and int8: slices that a launch adds 0.06 and 0.06 (never
+// the wide GEMM 0.54 and 0.11, the rule before 0.33 and 0.11), unsplit 0.04 and 0.06 (0.75 and 0.42; 0.60 and 0.42), sums of 4096 deep and more that the next norm takes 0.23 (0.42; 0.44), int8 see below.  The rule before
+// went by the share of a wave's requests that are k-tiles of its own, and tiles that are not a wave's own are no requests any more.
+// Not bf16 weights, nor up to 16 rows (28672 x 4096 fp8 23.4 -> 23.8 us); nothing beyond the sizes measured.
+bool gemm_wide_few_rows(const LinearW& w, int M, int epi, size_t ws_bytes, bool deferred) {
+  int cus = 0;
+  if (gemm_wide_mode() == 0 || gemm_wide_bm()) return false;      // (128 tokens and more: none of these calls has them)
+  if (M < 17 || M > 32 || w.wd == MI_W_BF16 || w.K % 64 != 0 || w.K < 2048 || w.N < 2048 || w.N > 65536 || device_num_cu(&cus) != MI_OK) return false;
+  const bool fp8 = w.wd == MI_W_F8E4M3;
+  // sums, int8: the register kernel takes 0 .. 9 us less but for the narrowest (2048 .. 3072 square, 24 rows and more: 0.3 .. 1.2 more).  K of 16448 .. 17600 (five k-tiles a wave, the last of them
+  // rare) was the wide GEMM's by the rule before, and its tests hold it to that: 1.5 .. 4 more (2048, 3072, 5120 rows).
+  if (deferred && !fp8) return w.K > 16384 && w.K <= 17600 && (size_t)w.N * w.K <= 150000000;
+  if (deferred && w.K < 4096) return false;                       // (2048 .. 3072 square: 0.3 .. 2 us in favour of the wide GEMM from 20 rows on; held by the same tests)
+  const double regs = fp8 ? gemv_regs_us_wd<MI_W_F8E4M3>(M, w.N, w.K, ws_bytes, deferred) : gemv_regs_us_wd<MI_W_INT8>(M, w.N, w.K, ws_bytes, deferred);
+  const WidePlan wide = gemm_wide_plan(M, w.N, w.K, gemm_wide_ks() == 1 ? 0 : ws_bytes, w.wd, deferred);
+  if (deferred) return 1.6 * wide.us - 10.5 < regs;
+  // (three times as wide as deep, 3584 .. 4032 deep, from 25 rows on: level, 0.3 more .. 0.4 less)
+  if (wide.ks > 1) return 1.2 * wide.us - 7.5 < regs || (fp8 && M >= 25 && w.K >= 3584 && w.K < 4096 && w.N >= 3 * w.K);
+  // fp8 tiles that fill three quarters of the chip to all of it in one round take less than the line says: 24576 .. 32768 rows, 3584 and 4096 deep, at 28 rows 0.1 .. 0.7 less than the registers, at 32 rows
+  // 0.2 .. 1.5, at 24 rows 0.5 more to as much
+  const int tiles = ceil_div(w.N, 128);
+  if (fp8 && M >= 25 && w.K >= 3584 && 4 * tiles >= 3 * cus && tiles <= cus) return true;
+  return w.K >= 4096 && 0.85 * wide.us + 4.5 < regs;
 }
 // The 128 x 128 kernel keeps single 16-row tiles and, where there is no workspace to split K into, grids of less than half the chip.  Everything else is the
 // wide kernel's (us at 60 / 100 - 128 tokens, 128 x 128 -> wide: 4096 x 4096 fp8 18.4 / 19.5 -> 9.4 / 11.8, 2560 x 2048 bf16 12.6 / 17.4 -> 11.0 / 11.6).
@@ -394,7 +389,7 @@ int launch_gemm_wide(const LinearW& w, int T, const uint16_t* x, int ldx, int ep
   MI_CHECK(w.K % 64 == 0 && ldx % 8 == 0, "gemm_wide: K % 64 == 0");
   WidePlan pl = gemm_wide_plan(T, w.N, w.K, gemm_wide_ks() == 1 || !splitk_ws ? 0 : splitk_ws_bytes, w.wd, split_as_deferred || (defer && (epi == EPI_RESID || epi == EPI_F32)));
   const int forced_bm = force_bm ? force_bm : gemm_wide_bm();
-  if (forced_bm) pl = WidePlan{forced_bm, force_ntw ? force_ntw : 4, 1};
+  if (forced_bm) pl = WidePlan{forced_bm, force_ntw ? force_ntw : 4, 1, 0.};
   if (force_ks) {
     MI_CHECK(force_ks >= 1 && (force_ks - 1) * ceil_div(w.K / 64, force_ks) < w.K / 64 && (force_ks == 1 || (splitk_ws && (size_t)force_ks * T * w.N * 4 <= splitk_ws_bytes)),
              "gemm_wide: forced K-split must leave no slice empty and fit the workspace");
