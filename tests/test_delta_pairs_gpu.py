@@ -46,3 +46,10 @@ def test_parts_and_pieces(lib, lengths, chunks):  # noqa: F811
     close(*x.step([(i, n) for i, n in enumerate(lengths)], chunks=chunks), 1)
     for i in range(len(lengths)):
         x.check_state(i)
+
+
+# heads of 128 on more CUs than three parts leave: a chunk below the line (one scan), on it, and one above
+@pytest.mark.parametrize("heads", [12, 16])
+@pytest.mark.parametrize("first,second", [(1136, 1152), (1152, 1168), (1151, 1153)])
+def test_two_parts_that_share_cus(lib, heads, first, second):  # noqa: F811
+    test_long_segments_in_two_parts(lib, (heads, heads, 128, 128, 4), first, second)

@@ -860,7 +860,11 @@ __global__ __launch_bounds__(256, 2) void delta_scan_pairs_kernel(DeltaGeom g, f
 // work-groups puts both on the CUs that the first part leaves.  delta_out_kernel adds replies S1 and makes the last state.  Everything stays fp32.
 // 16 heads of 128, 2048 tokens, us: scan 98 -> 68, output norm 15.5 -> 28; 4000 tokens 3988 -> 3639 a call.
 // Behind the records: [chunk][16 dkp] replies a head, those of the first part unused: there the states, S1 as fragments, the second part's own (L) and its transition (P).
-constexpr int kSplitChunks = 64;                 // of a segment at least: room for the three states, and below the joining costs what the halves save (us a call, one scan -> two: 900 tokens 1202 -> 1213, 1100 1395 -> 1359)
+constexpr int kSplitChunks = 64;                 // of a segment at least: room for the three states
+// ... and below, the joining costs what the parts save where they share CUs and states are 112 and 128 high (a work-group stages 50 and 64 KB of S1).  us of all kernels, one scan -> two parts: 16 heads
+// of 128, 1024 tokens 95 -> 98, 1136 109.5 -> 106.4; 12 heads 88 -> 92, 97.9 -> 95.0; 14 heads 93.8 -> 94.4, 99.8 -> 101.3, 1200 tokens 107.6 -> 108.2; 10 heads, which share none, 85.9 -> 82.8; 20 heads of 96 97 -> 91;
+// 32 of 64 85 -> 79
+static int split_chunks(const DeltaGeom& g, int num_cu) { return g.dkp > 96 && 3 * g.H * (g.dvp / 16) > num_cu ? 72 : kSplitChunks; }
 __host__ __device__ __forceinline__ int split_first(int n) { return (n * 41 + 127) / 256 * 4; }     // chunks of the first part: 0.64 of them, whole turns of the loop
 struct SplitMem { float *replies, *s1, *l, *p; };
 __host__ __device__ __forceinline__ SplitMem split_mem(float* records, const DeltaGeom& g, int n, int h) {
@@ -1029,9 +1033,11 @@ int check_in(const DeltaGeom& g, const DeltaIn& in) {
 bool delta_supported(const DeltaGeom& g) {
   return g.H >= 1 && g.G >= 1 && g.H % g.G == 0 && g.dk >= 1 && g.dk <= 256 && g.dv >= 1 && g.dv <= 256 && g.taps >= 1 && g.taps <= 16;
 }
-// whether a segment may go in two parts (delta_scan_split_kernel): states as wide as they are high, keys the paired scan takes
-static bool split_fits(const DeltaGeom& g) { return g.dkp == g.dvp && g.dkp <= 128; }
-size_t delta_chunk_floats(const DeltaGeom& g) { return (size_t)g.H * (record_floats(g.dkp, g.dvp) + (split_fits(g) ? 16 * g.dkp : 0)); }
+// whether a segment may go in two parts (delta_scan_split_kernel): states as wide as they are high, keys the paired scan takes, CUs for both parts
+static bool split_fits(const DeltaGeom& g, int num_cu) { return g.dkp == g.dvp && g.dkp <= 128 && 2 * g.H * (g.dvp / 16) <= num_cu; }
+size_t delta_chunk_floats(const DeltaGeom& g) {
+  return (size_t)g.H * (record_floats(g.dkp, g.dvp) + (g.dkp == g.dvp && g.dkp <= 128 ? 16 * g.dkp : 0));
+}
 
 int launch_delta_token(const DeltaGeom& g, const DeltaIn& in, int rows, const AttnSeg* segs, void* y, int ldy, bool f32, hipStream_t s) {
   int rc = check_in(g, in);
@@ -1065,7 +1071,7 @@ int launch_delta_prompt(const DeltaGeom& g, const DeltaIn& in, const AttnSeg* sd
   const size_t lds = (size_t)(3 * kC * (g.dkp + 4) + std::max(kC * (g.dkp + 4), kPairParts * kPairTiles * 8)) * sizeof(float);
   for (int c0 = 0; c0 < chunks; c0 += max_chunks) {
     const int n = std::min(max_chunks, chunks - c0);
-    const bool split = nseg == 1 && split_fits(g) && n >= kSplitChunks && 2 * g.H * nvt <= num_cu;
+    const bool split = nseg == 1 && split_fits(g, num_cu) && n >= split_chunks(g, num_cu);
     const int joins = split ? ceil_div(g.H * nvt * nvt, 4 * ceil_div(g.H, 4)) : 0;       // work-groups for the last state
     const dim3 gf(n, g.H), gs(g.H * nvt, nseg), go(split ? split_first(n) + split_columns(n, g.H) + joins : n, ceil_div(g.H, 4));
 #define MI_DF(TAPS) { \
