@@ -1033,10 +1033,11 @@ int check_in(const DeltaGeom& g, const DeltaIn& in) {
 bool delta_supported(const DeltaGeom& g) {
   return g.H >= 1 && g.G >= 1 && g.H % g.G == 0 && g.dk >= 1 && g.dk <= 256 && g.dv >= 1 && g.dv <= 256 && g.taps >= 1 && g.taps <= 16;
 }
-// whether a segment may go in two parts (delta_scan_split_kernel): states as wide as they are high, keys the paired scan takes, CUs for both parts
+// whether a segment may go in two parts (delta_scan_split_kernel): states as wide as they are high, keys the paired scan takes, CUs for both parts (32 heads of 128 have none to spare, and no replies)
 static bool split_fits(const DeltaGeom& g, int num_cu) { return g.dkp == g.dvp && g.dkp <= 128 && 2 * g.H * (g.dvp / 16) <= num_cu; }
 size_t delta_chunk_floats(const DeltaGeom& g) {
-  return (size_t)g.H * (record_floats(g.dkp, g.dvp) + (g.dkp == g.dvp && g.dkp <= 128 ? 16 * g.dkp : 0));
+  int num_cu = 0;
+  return (size_t)g.H * (record_floats(g.dkp, g.dvp) + (device_num_cu(&num_cu) != MI_OK || split_fits(g, num_cu) ? 16 * g.dkp : 0));
 }
 
 int launch_delta_token(const DeltaGeom& g, const DeltaIn& in, int rows, const AttnSeg* segs, void* y, int ldy, bool f32, hipStream_t s) {
