@@ -53,3 +53,26 @@ def test_parts_and_pieces(lib, lengths, chunks):  # noqa: F811
 @pytest.mark.parametrize("first,second", [(1136, 1152), (1152, 1168), (1151, 1153)])
 def test_two_parts_that_share_cus(lib, heads, first, second):  # noqa: F811
     test_long_segments_in_two_parts(lib, (heads, heads, 128, 128, 4), first, second)
+
+
+# the replies' rooms of a second part: 16 dkp numbers a head and chunk, for heads that have CUs for one (16 of 128 on 256 CUs), and not for one head more
+def test_rooms_for_replies(lib):  # noqa: F811
+    import torch
+    from tests.bokulorn_cases import config, delta
+    from vllm_neuron_amd._native import NativeModel
+    from vllm_neuron_amd.models import config_from_dict, fill_sizes
+    heads, length = torch.cuda.get_device_properties(0).multi_processor_count // 16, 4096
+
+    def workspace(n):
+        c = config_from_dict(config(256, 256, [delta(n, n, 128, 128, 4)]))
+        fill_sizes(c, lambda name: (128, 256))
+        m = NativeModel(stack=dict(c.stack, compute_dtype=1), ctx_buckets=[length], num_blocks=129, block_size=32, max_num_seqs=1, max_model_len=length, device_id=0, use_graphs=0)
+        m.init_synthetic_weights(1, 0.02)
+        m.finalize()
+        got = m.kv_stats()["workspace_bytes"]
+        m.close()
+        return got
+    at = {n: workspace(n) for n in (heads - 1, heads, heads + 1, heads + 2)}
+    chunks = length // 16 + 1
+    # what a head takes besides is the same either way (a row's columns come in sixteens: none of the pairs crosses one)
+    assert (at[heads] - at[heads - 1]) - (at[heads + 2] - at[heads + 1]) == chunks * 16 * 128 * 4
