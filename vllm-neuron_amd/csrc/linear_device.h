@@ -1006,9 +1006,10 @@ __device__ __forceinline__ void blds16(const void* p, int bytes, int at, unsigne
   const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)l, 16, at, 0, 0, 0);
 }
-static bool gemv_kstream_enabled() {
-  static const bool on = [] { const char* v = getenv("MI355X_GEMV_KSTREAM"); return !(v && v[0] == '0'); }();
-  return on;
+// MI355X_GEMV_KSTREAM=0: never; MI355X_GEMV_KSTREAM_MIN_M: from so many rows on
+static bool gemv_kstream_enabled(int M) {
+  static const int min_m = [] { const char *v = getenv("MI355X_GEMV_KSTREAM"), *n = getenv("MI355X_GEMV_KSTREAM_MIN_M"); return v && v[0] == '0' ? 1 << 30 : n ? atoi(n) : 1; }();
+  return M >= min_m;
 }
 static bool gemv_priv_enabled() {
   static const bool on = [] { const char* v = getenv("MI355X_GEMV_PRIV"); return !(v && v[0] == '0'); }();
@@ -1103,8 +1104,7 @@ template <int WD, int PRO, int EPI>
 static int launch_gemv_t(const LinearW& w, int M, const ProArgs& p, const EpiArgs& e, hipStream_t s) {
   if (!gemv_fits_whole(M, w.K)) {
     if constexpr (PRO == PRO_BF16 && (EPI == EPI_F32 || EPI == EPI_RESID || EPI >= EPI_RELU2)) {
-      static const int min_m = [] { const char* v = getenv("MI355X_GEMV_KSTREAM_MIN_M"); return v ? atoi(v) : 1; }();
-      if (gemv_kstream_enabled() && M >= min_m) return launch_gemv_kstream<WD, EPI>(w, M, p, e, s);
+      if (gemv_kstream_enabled(M)) return launch_gemv_kstream<WD, EPI>(w, M, p, e, s);
     }
     return launch_gemv_bigk_t<WD, PRO, EPI>(w, M, p, e, s);
   }
@@ -1116,7 +1116,7 @@ static int launch_gemv_t(const LinearW& w, int M, const ProArgs& p, const EpiArg
   // slices too long to be staged by their wave: beside the weights (bit for bit the same sums; 3584 x 18944 int8 at 2 rows 17.4 -> 16.6 us, bf16 24.3 -> 23.5, at 1 row
   // the same)
   if constexpr (PRO == PRO_BF16 && (EPI == EPI_F32 || EPI == EPI_RESID || EPI >= EPI_RELU2))
-    if (sh.ks == 8 && ceil_div(KT, 8) > priv_kt && M >= 2 && M <= 4 && gemv_kstream_enabled()) return launch_gemv_kstream<WD, EPI>(w, M, p, e, s);
+    if (sh.ks == 8 && ceil_div(KT, 8) > priv_kt && M >= 2 && M <= 4 && gemv_kstream_enabled(M)) return launch_gemv_kstream<WD, EPI>(w, M, p, e, s);
   if (sh.ks > 1 && sh.ks * sh.tp == kGemvWaves && ceil_div(KT, sh.ks) <= priv_kt) {
     switch (sh.ks) {
       case 2: return launch_gemv_priv<WD, PRO, EPI, 2>(w, M, p, e, s, num_cu);
