@@ -25,56 +25,79 @@ def _tables(ctx, bs, MB, pad):
 @pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("tiles", [29, 30, 31, 32, 33, 63])
 def test_long_contexts(lib, hd, bs, tiles):  # noqa: F811
-    ctx = [3 + i for i in range(32)]
-    ctx[5], ctx[30] = 256 * tiles + 1, 256 * tiles - 20
+    _long_contexts(lib, hd, bs, tiles, 32)
+
+
+# 16 sequences: two slices of four waves to each, 256 tokens to each of a wave's tiles again, and a launch that puts the slices together
+@pytest.mark.parametrize("hd,bs", [(64, 48), (128, 16)])
+@pytest.mark.parametrize("tiles", [30, 31, 32, 33, 63])
+def test_long_contexts_in_slices(lib, hd, bs, tiles):  # noqa: F811
+    _long_contexts(lib, hd, bs, tiles, 16)
+
+
+def _long_contexts(lib, hd, bs, tiles, rows):  # noqa: F811
+    ctx = [3 + i for i in range(rows)]
+    ctx[5], ctx[-2] = 256 * tiles + 1, 256 * tiles - 20
     MB = -(-max(ctx) // bs) + 3
     bt, nb = _tables(ctx, bs, MB, -1)                      # pad -1: must never be read
     k, v = _make_pool(nb, bs, 8, hd, 4)
-    q = torch.randn(32, 16, hd, generator=torch.Generator().manual_seed(6)).to(torch.bfloat16)
-    out = torch.empty(32, 16 * hd, dtype=torch.bfloat16, device="cuda")
+    q = torch.randn(rows, 16, hd, generator=torch.Generator().manual_seed(6)).to(torch.bfloat16)
+    out = torch.empty(rows, 16 * hd, dtype=torch.bfloat16, device="cuda")
     L = lib.load_library()
-    scratch = torch.empty(L.mi_op_attn_scratch_bytes(32, 16, hd), dtype=torch.uint8, device="cuda")
+    scratch = torch.empty(L.mi_op_attn_scratch_bytes(rows, 16, hd), dtype=torch.uint8, device="cuda")
     d = [dev(t) for t in (q, pool_to_native(k, v, nb, bs), bt, torch.tensor(ctx, dtype=torch.int32))]
-    lib.check(L.mi_op_paged_attn_decode(d[0].data_ptr(), d[1].data_ptr(), nb, bs, d[2].data_ptr(), MB, d[3].data_ptr(), 32, 16, 8, hd, out.data_ptr(),
+    lib.check(L.mi_op_paged_attn_decode(d[0].data_ptr(), d[1].data_ptr(), nb, bs, d[2].data_ptr(), MB, d[3].data_ptr(), rows, 16, 8, hd, out.data_ptr(),
                                         scratch.data_ptr(), None))
     torch.cuda.synchronize()
     kk, vv = k.float().reshape(nb, bs, 8, hd), v.float().reshape(nb, bs, 8, hd)
-    for b in (0, 5, 30, 31):
+    for b in (0, 5, rows - 2, rows - 1):
         idx = torch.arange(ctx[b])
         blk = bt[b, idx // bs].long()
         ref = ref_attention(q[b:b + 1].float(), kk[blk, idx % bs], vv[blk, idx % bs], torch.tensor([ctx[b] - 1]))
         assert (out[b].cpu().float() - ref[0]).abs().max().item() < 0.02, (b, ctx[b])      # bf16 output rounding of O(1) values
 
 
-# the windowed kernel's: four waves a work-group, 128 tokens to each of their tiles; a window that starts inside a tile
+# the windowed kernel's, a launch a sequence here: 16 slices of four waves to each of 8 kv heads, one tile a wave to four; a window that starts inside a tile
 @pytest.mark.parametrize("d,bs", [(64, 32), (100, 16)])
 @pytest.mark.parametrize("tiles,window", [(30, 0), (31, 0), (32, 0), (33, 4000), (63, 0)])
 def test_long_windows(lib, d, bs, tiles, window):  # noqa: F811
-    dp, ctx = -(-d // 16) * 16, [3 + i for i in range(32)]
+    ctx = [3 + i for i in range(32)]
     ctx[5], ctx[30] = 128 * tiles + 1, 128 * tiles - 20
+    _long_windows(lib, 16, 8, d, bs, ctx, window, tiles, (0, 5, 30, 31))
+
+
+# ... and with 130 kv heads, where the four waves of one work-group take a whole context, 128 tokens to each of their tiles: more of them than a look holds
+@pytest.mark.parametrize("d,bs", [(32, 32), (20, 16)])
+@pytest.mark.parametrize("tiles,window", [(30, 0), (31, 0), (32, 0), (33, 4000), (63, 0)])
+def test_long_windows_of_one_work_group(lib, d, bs, tiles, window):  # noqa: F811
+    _long_windows(lib, 130, 130, d, bs, [128 * tiles + 1, 128 * tiles - 20, 7], window, tiles, (0, 1, 2))
+
+
+def _long_windows(lib, H, G, d, bs, ctx, window, seed, checked):  # noqa: F811
+    dp, B = -(-d // 16) * 16, len(ctx)
     MB = -(-max(ctx) // bs) + 1
     bt, nb = _tables(ctx, bs, MB, 0)
-    g = torch.Generator().manual_seed(tiles)
-    k, v = (torch.zeros(nb, 8, bs, dp, dtype=torch.bfloat16) for _ in range(2))
-    k[..., :d], v[..., :d] = torch.randn(nb, 8, bs, d, generator=g), torch.randn(nb, 8, bs, d, generator=g)
-    q = torch.zeros(32, 16, dp, dtype=torch.bfloat16)
-    q[..., :d] = torch.randn(32, 16, d, generator=g)
-    ldo = (16 * d + 63) // 64 * 64
-    out = torch.zeros(32, ldo, dtype=torch.bfloat16, device="cuda")
+    g = torch.Generator().manual_seed(seed)
+    k, v = (torch.zeros(nb, G, bs, dp, dtype=torch.bfloat16) for _ in range(2))
+    k[..., :d], v[..., :d] = torch.randn(nb, G, bs, d, generator=g), torch.randn(nb, G, bs, d, generator=g)
+    q = torch.zeros(B, H, dp, dtype=torch.bfloat16)
+    q[..., :d] = torch.randn(B, H, d, generator=g)
+    ldo = (H * d + 63) // 64 * 64
+    out = torch.zeros(B, ldo, dtype=torch.bfloat16, device="cuda")
     pos = torch.tensor([n - 1 for n in ctx], dtype=torch.int32)
-    x = [dev(t) for t in (torch.zeros(16), q, k, v, bt, pos, pos + 1)]
+    x = [dev(t) for t in (torch.zeros(H), q, k, v, bt, pos, pos + 1)]
     segs = torch.tensor([(i, 1, n - 1, i) for i, n in enumerate(ctx)], dtype=torch.int32).contiguous()
-    spec = spec_of(lib, 16, 8, d, d, window, d ** -0.5, bias=0, sink=0, unit=0)
+    spec = spec_of(lib, H, G, d, d, window, d ** -0.5, bias=0, sink=0, unit=0)
     lib.check(lib.load_library().mi_op_window_attn(spec, x[0].data_ptr(), x[1].data_ptr(), x[2].data_ptr(), x[3].data_ptr(), bs, x[4].data_ptr(), MB, x[5].data_ptr(),
-                                                   x[6].data_ptr(), segs.data_ptr(), 32, 32, max(ctx), out.data_ptr(), ldo, 0, 0, None))
+                                                   x[6].data_ptr(), segs.data_ptr(), B, B, max(ctx), out.data_ptr(), ldo, 0, 0, None))
     torch.cuda.synchronize()
-    for b in (0, 5, 30, 31):
+    for b in checked:
         idx = torch.arange(max(0, ctx[b] - window) if window else 0, ctx[b])
         blk = bt[b, idx // bs].long()
         K, W = (t[blk, :, idx % bs, :d].double() for t in (k, v))
-        s = torch.einsum("hd,nhd->hn", q[b, :, :d].double(), K.repeat_interleave(2, 1)) * d ** -0.5
-        ref = torch.einsum("hn,nhd->hd", torch.softmax(s, -1), W.repeat_interleave(2, 1)).flatten()
-        assert (out[b, :16 * d].cpu().double() - ref).abs().max().item() < 0.02, (b, ctx[b])      # as above
+        s = torch.einsum("hd,nhd->hn", q[b, :, :d].double(), K.repeat_interleave(H // G, 1)) * d ** -0.5
+        ref = torch.einsum("hn,nhd->hd", torch.softmax(s, -1), W.repeat_interleave(H // G, 1)).flatten()
+        assert (out[b, :H * d].cpu().double() - ref).abs().max().item() < 0.02, (b, ctx[b])      # as above
 
 
 # chunked attention with its distance table and sinks, so many kv heads that one work-group's four waves take a whole context (128 tokens to each of their tiles): no tile, one, two and three for a wave, the last of a look, the first of the next, a third look

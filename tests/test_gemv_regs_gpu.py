@@ -46,7 +46,7 @@ def test_edges_of_the_register_gemv(lib, wd, M, N, K):
 # every number of k-tiles a wave holds that has a kernel of its own, whole and with a last tile or whole waves missing (one-byte weights 5 .. 8, bf16 5 .. 8, 12, 14, 16)
 @pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
 @pytest.mark.parametrize("M", [5, 32])
-@pytest.mark.parametrize("N,K", [(4096, K) for K in (1088, 1536, 1600, 1792, 2112, 2560, 2624, 3072, 3136, 3584, 3648)])
+@pytest.mark.parametrize("N,K", [(4096, K) for K in (1088, 1536, 1600, 1792, 1856, 2048, 2112, 2560, 2624, 3072, 3136, 3584, 3648, 4096)])
 def test_k_tiles_of_a_wave(lib, wd, M, N, K):
     test_edges_of_the_register_gemv(lib, wd, M, N, K)
 
@@ -68,25 +68,35 @@ def test_batches_of_the_few_row_kernels(lib, wd, M, N, K):
     test_edges_of_the_register_gemv(lib, wd, M, N, K)
 
 
-# ... with the norms in front, where slices of 2 .. 16 tiles go to 1, 2, 4 and 8 waves: against 5 rows, whose weights the register kernel reads (the same products
-# in another order; bf16 roundings of the activations in between make 2^-8 of a value, and as between any two kernels of this file 5 % of the spread is far beyond)
+def _quant(wd):
+    return None if wd == "bf16" else dict(quantized=True, quantization_dtype=wd, quantization_type="per_channel_symmetric")
+
+
+# ... with the norms in front, where slices of 2 .. 16 tiles go to 1, 2, 4 and 8 waves: against the oracle, at the bar of the other dispatch tests, and against 5 rows, whose weights the
+# register kernel reads (the same products in another order; bf16 roundings of the activations in between make 2^-8 of a value, and as between any two kernels of this file 5 % of the spread
+# is far beyond)
 @pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
 @pytest.mark.parametrize("hidden,inter,vocab", [(1024, 1088, 16), (1280, 6208, 12304), (2048, 5632, 32000), (2304, 2112, 8208), (3584, 4736, 16400), (4096, 14336, 4112)])
 def test_norms_in_front_of_few_rows(wd, hidden, inter, vocab):
-    from oracle import DecoderConfig
+    from oracle import DecoderConfig, PagedDecoderOracle
     from oracle.synth import make_weights
     from tests.helpers import decode_inputs
     from vllm_neuron_amd._native import MI_Q, MI_W, NativeModel
     shape = dict(num_layers=1, hidden_size=hidden, num_heads=hidden // 64, num_kv_heads=hidden // 256, head_dim=64, intermediate_size=inter, vocab_size=vocab)
-    w = make_weights(DecoderConfig(**shape), seed=4)
-    model = NativeModel(**shape, rms_norm_eps=1e-5, rope_theta=1e4, rope_type=0, rope_factor=1.0, num_blocks=33, block_size=32, max_num_seqs=8,
+    cfg = DecoderConfig(**shape)
+    w = make_weights(cfg, seed=4)
+    model = NativeModel(**shape, rms_norm_eps=cfg.rms_norm_eps, rope_theta=cfg.rope_theta, rope_type=0, rope_factor=1.0, num_blocks=33, block_size=32, max_num_seqs=8,
                         max_model_len=32, weight_dtype=MI_W[wd], quant_type=MI_Q["per_channel_symmetric"], quantize_lm_head=1, tp_degree=1, tp_rank=0,
                         device_id=0, use_graphs=1, ctx_buckets=[32])
     model.load_state_dict(w)
     model.finalize()
-    out = {rows: model.forward(**decode_inputs([i % vocab for i in range(rows)], [0] * rows, [[1 + i] for i in range(rows)], 32, 32)).clone() for rows in (5, 4, 1)}
+    inputs = {rows: decode_inputs([i % vocab for i in range(rows)], [0] * rows, [[1 + i] for i in range(rows)], 32, 32) for rows in (5, 4, 1)}
+    out = {rows: model.forward(**x).clone() for rows, x in inputs.items()}
     std = out[5].std().item()
+    want = PagedDecoderOracle(cfg, w, 33, 32, compute="bf16", quant=_quant(wd)).forward(**inputs[4]).float()
     for rows in (4, 1):
+        d = out[rows] - want[:rows]
+        assert d.pow(2).mean().sqrt() < 0.02 * want.std() and d.abs().max() < 0.1 * want.std()
         assert torch.isfinite(out[rows]).all() and (out[rows] - out[5][:rows]).abs().max().item() < 0.05 * std
     model.close()
 
@@ -281,12 +291,12 @@ torch.save(res, sys.argv[1])
 
 # (weights, hidden, feed-forward, heads, kv heads) -> whether 17 and 28 rows go through the register kernel alone
 _REGS_ALONE = {
-    ("int8", 2048, 16384, 16, 4): (True, True),             # of the waves' requests for the down projection's weights all are their own
-    ("int8", 2048, 17408, 16, 4): (False, False),           # 17 of 32
+    ("int8", 2048, 16384, 16, 4): (True, True),             # sums of int8 stay, up to K of 16384
+    ("int8", 2048, 17408, 16, 4): (False, False),           # a little beyond
     ("int8", 1536, 17408, 12, 2): (True, True),             # narrow
-    ("f8e4m3", 2048, 4096, 16, 4): (False, False),          # at most 4 of 8
+    ("f8e4m3", 2048, 4096, 16, 4): (False, False),          # a sum of 4096 deep
     ("f8e4m3", 1024, 4096, 8, 2): (True, True),             # narrow
-    ("f8e4m3", 2048, 14336, 16, 4): (True, True),           # 28 of 32, and 16 tiles of 128 rows times ten slices of K are 160 work-groups of the wide GEMM
+    ("f8e4m3", 2048, 14336, 16, 4): (True, True),           # deep and narrow: ten slices of K are 160 work-groups of the wide GEMM
     ("f8e4m3", 3584, 3584, 28, 14): (True, True),           # K of 3584; queries, keys and values are twice the width
     ("f8e4m3", 3584, 3584, 28, 28): (True, False)}          # three times: the wide GEMM from 25 rows on
 
@@ -303,7 +313,7 @@ def test_which_calls_of_17_to_32_rows_leave_the_register_kernel(tmp_path):
         assert tuple(torch.equal(got[0][(*k, rows)], got[1][(*k, rows)]) for rows in (17, 28)) == want, k
 
 
-# queries, keys and values by the wide GEMM from 25 rows on (their slices' sum rotates them and writes them to the pool, which the second step reads), the down
+# queries, keys and values by the wide GEMM from 25 rows on and earlier (their slices' sum rotates them and writes them to the pool, which the second step reads), the down
 # projection by it from 17 rows on, logits to the host in groups of four row-tiles of which the last has one: against the oracle, at the bar of the other dispatch tests
 @pytest.mark.parametrize("rows", [16, 17, 25, 32])
 def test_two_steps_of_many_rows_against_the_oracle(rows):
@@ -328,6 +338,34 @@ def test_two_steps_of_many_rows_against_the_oracle(rows):
         for _ in range(2):             # eager pass, then the graph
             d = model.forward(**inputs).float() - want
             assert torch.isfinite(d).all() and d.pow(2).mean().sqrt() < 0.02 * want.std() and d.abs().max() < 0.1 * want.std()
+    model.close()
+
+
+
+# two row-tiles a work-group and more, of which the first has its epilogue's operands asked for ahead and the others do not: rotated queries and keys (384 row-tiles of 512), residual sums
+# unsplit (272 of 256); one and two column groups, the last one with a single row
+@pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
+@pytest.mark.parametrize("rows", [5, 16, 17, 32])
+@pytest.mark.parametrize("hidden,heads,kv,dim,inter", [(512, 32, 8, 128, 256), (4352, 4, 2, 64, 256)])
+def test_epilogues_of_several_row_tiles(wd, rows, hidden, heads, kv, dim, inter):
+    from oracle import DecoderConfig, PagedDecoderOracle
+    from oracle.synth import make_weights
+    from tests.helpers import decode_inputs
+    from vllm_neuron_amd._native import MI_Q, MI_W, NativeModel
+    shape = dict(num_layers=1, hidden_size=hidden, num_heads=heads, num_kv_heads=kv, head_dim=dim, intermediate_size=inter, vocab_size=512)
+    cfg = DecoderConfig(**shape)
+    w = make_weights(cfg, seed=4)
+    oracle = PagedDecoderOracle(cfg, w, 34, 32, compute="bf16", quant=_quant(wd))
+    model = NativeModel(**shape, rms_norm_eps=cfg.rms_norm_eps, rope_theta=cfg.rope_theta, rope_type=0, rope_factor=1.0, num_blocks=34, block_size=32, max_num_seqs=32,
+                        max_model_len=32, weight_dtype=MI_W[wd], quant_type=MI_Q["per_channel_symmetric"], quantize_lm_head=1, tp_degree=1, tp_rank=0, device_id=0,
+                        use_graphs=1, ctx_buckets=[32])
+    model.load_state_dict(w)
+    model.finalize()
+    for at in range(3):                # (positions that turn)
+        inputs = decode_inputs([(31 * i + 7 * at) % 512 for i in range(rows)], [at] * rows, [[1 + i] for i in range(rows)], 32, 32)
+        want = oracle.forward(**inputs).float()
+        d = model.forward(**inputs).float() - want
+        assert torch.isfinite(d).all() and d.pow(2).mean().sqrt() < 0.02 * want.std() and d.abs().max() < 0.1 * want.std()
     model.close()
 
 
