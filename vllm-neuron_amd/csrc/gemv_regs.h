@@ -63,7 +63,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
   const int total = passes * NB;
   auto issue = [&](u32x4_t (&buf)[BT], int i) {
     const int ii = min(i, total - 1), k0 = kbeg + (ii % NB) * BT;      // (behind the last batch, and beyond the slice: no request.  O of the 1B shape 5.2 -> 4.7 us, of the 7B 6.4 -> 6.0)
-    stream_batch(buf, W, tile_of(ii / NB) * KT + k0, i < total ? kend - k0 : 0, lane);
+    stream_batch<MG == 2>(buf, W, tile_of(ii / NB) * KT + k0, i < total ? kend - k0 : 0, lane);
   };
   issue(bufA, 0);
   __builtin_amdgcn_sched_barrier(0);

@@ -167,18 +167,19 @@ __device__ __forceinline__ void stream_wait(u32x4_t&) {}
 #endif
 
 // A batch of 1 KiB weight tiles from the `first` of W on, of which there are `n` (both the same for the whole wave): what lies beyond is zeros and no request to
-// memory.  Two descriptors, 4 KiB apart: an instruction's own offset ends there, and a second offset register is one too many for the kernels of two column groups.
-template <int U>
+// memory.  TWO: two descriptors, 4 KiB apart, where a second offset register is one too many (an instruction's own offset ends at 4095).
+template <bool TWO = false, int U>
 __device__ __forceinline__ void stream_batch(u32x4_t (&buf)[U], const uint4* W, int first, int n, int lane) {
   int bytes = min(max(n, 0), U) * 1024;
   asm("" : "+v"(first), "+v"(bytes));   // (else hipcc folds the two below away, keeps some in vector registers and loops over the lanes for the descriptor)
   const uint4* at = W + (size_t)(unsigned)__builtin_amdgcn_readfirstlane(first) * 64;
   const int size = __builtin_amdgcn_readfirstlane(bytes);
+  constexpr int S = TWO ? 4 : U;
   const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(at), 0, size, 0x00020000);
   const auto r4 = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(at + 256), 0, max(size - 4096, 0), 0x00020000);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    buf[u] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(u < 4 ? r : r4, lane * 16 + u % 4 * 1024, 0, 2));   // (2: streaming, nt)
+    buf[u] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(u < S ? r : r4, lane * 16 + u % S * 1024, 0, 2));   // (2: streaming, nt)
     __builtin_amdgcn_sched_barrier(0x3cf);   // in the order they are multiplied: a wait for one is a wait for all requested before it
   }
 }
