@@ -858,7 +858,8 @@ __global__ __launch_bounds__(256, 2) void delta_scan_pairs_kernel(DeltaGeom g, f
 // row of replies is what the same recurrence makes of the columns of the identity.  So the second part has two work-groups for 16 columns, which share a CU and take 2.7 us
 // a pair between them (fp32 matrix products leave no room for vector instructions beside them: 32 cycles and 5 - 9 for each of those), and it is the shorter one; the order of the
 // work-groups puts both on the CUs that the first part leaves.  delta_out_kernel adds replies S1 and makes the last state.  Everything stays fp32.
-// 16 heads of 128, 2048 tokens, us: scan 98 -> 68, output norm 15.5 -> 28; 4000 tokens 3988 -> 3639 a call.
+// 16 heads of 128, 2048 tokens, us: scan 98 -> 66, output norm 15.5 -> 31, a call 2142 -> 2020; 3000 tokens 2993 -> 2768.  The cut is for parts that share CUs (16 heads of 128 take 256 of them); where each
+// has its own, one half would be the even one.  All kernels of a launch of 8 heads there: 2048 tokens 139 -> 116, 4096 251 -> 200; 2 heads 119 -> 96, 215 -> 160.
 // Behind the records: [chunk][16 dkp] replies a head, those of the first part unused: there the states, S1 as fragments, the second part's own (L) and its transition (P).
 constexpr int kSplitChunks = 64;                 // of a segment at least: room for the three states
 // ... and below, the joining costs what the parts save where they share CUs and states are 112 and 128 high (a work-group stages 50 and 64 KB of S1).  us of all kernels, one scan -> two parts: 16 heads

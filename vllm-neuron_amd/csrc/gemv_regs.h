@@ -15,8 +15,9 @@
 namespace mi {
 
 constexpr int kRegsMaxPasses = 64;   // row-tiles of a work-group: their scales and biases wait in LDS
-// k-tiles a wave holds at most: 8 of 64 k (1-byte weights), 16 of 32 k.  There is a kernel for 4, 5, 6, 7, 8 (bf16 also 12, 14, 16): a row-tile's requests all go out, those a wave has no
-// tile for repeat its last one, and a CU's requests in flight are what bounds it.  With 4, 8 and 16 alone, us a step: 7B int8 5 rows 1243 -> 1196, bf16 1679 -> 1583, 8B fp8 8 rows 1230 -> 1207.
+// k-tiles a wave holds at most: 8 of 64 k (1-byte weights), 16 of 32 k.  There is a kernel for 4, 5, 6, 7, 8 (bf16 also 12, 14, 16), since a wave asks for
+// the activations of all of them and multiplies all of them, its own or not; weights that are not its own are zeros without a request (stream_batch).  With 4, 8 and 16 alone, when they were
+// requests for its last tile again, us a step: 7B int8 5 rows 1243 -> 1196, bf16 1679 -> 1583, 8B fp8 8 rows 1230 -> 1207.
 template <int WD> constexpr int kRegsMaxTiles = WD == MI_W_BF16 ? 16 : 8;
 
 // HOLD: a work-group takes HOLD row-tiles side by side, and the wave that sums them keeps their results until it has all: a row's HOLD x 64 bytes

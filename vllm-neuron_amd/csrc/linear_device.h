@@ -1057,7 +1057,10 @@ static int launch_gemv_priv(const LinearW& w, int M, const ProArgs& p, const Epi
 // waves, then slices that the waves stage for themselves (of at most `priv_kt` k-tiles, 0: none) and of them the shortest that fill a batch, else the smallest K split.
 // Waves used to come behind the number of passes: the gate | up rows of the 7B shape (37888: 2368 row-tiles, ten on the busiest CU either way) went as 1 x 5, five
 // waves and two passes, at 4 rows int8 31.1 us and with bf16 47.4 (2 rows); as 4 x 2 they take 26.2 and 42.7.  28672 rows x 4096 fp8 (1 x 7 -> 8 x 1) 22.8 -> 21.6 us,
-// the head of 128256 rows beside it (1 x 8 -> 8 x 1, 8 tiles a slice) 106 -> 94; of 152064 x 3584 the slices of 14 tiles keep 121 us against 133 with slices of 7.
+// the head of 128256 rows beside it (1 x 8 -> 8 x 1, 8 tiles a slice) 106 -> 96; of 152064 x 3584 the slices of 14 tiles keep 121 us against 133 with slices of 7.
+// Over 53 projections and heads of 12 models 1024 .. 8192 wide, three weight types, 1, 2 and 4 rows (profiles/gemv_split_sweep.txt): the choice takes 2.6 % longer than the fastest split, 10 % less than
+// the passes first and the kernels of that time did; one in fifteen is 2 to 8 % slower than then (bf16 6144 x 6144 13.1 -> 14.1, 152064 x 3584 157 -> 161), no step of those models is.  Far from the
+// fastest: K that four waves divide evenly and eight do not (fp8 4096 x 11008 14.4 with 4 x 1, 10.8 with 8 x 1).
 struct GemvShape { int ks, tp; };
 static GemvShape gemv_pick_shape(int NT, int KT, int slots, int priv_kt) {
   GemvShape best{8, 1};

@@ -72,7 +72,7 @@ int launch_gemv_regs(const LinearW& w, int M, const uint16_t* x, int ldx, int ep
 // whether M rows of w take it (K beyond 8 slices of the registers, or slabs that do not fit: launch_gemv up to 16 rows, launch_gemm)
 bool gemv_in_regs(const LinearW& w, int M, size_t ws_bytes);
 // where launch_gemm_wide takes less time than launch_gemv_regs (17 .. 32 rows); deferred: the sum of K slices has a taker
-bool gemm_wide_few_rows(const LinearW& w, int M, int epi, size_t ws_bytes, bool deferred);
+bool gemm_wide_few_rows(const LinearW& w, int M, size_t ws_bytes, bool deferred);
 // whether a projection of 1 .. 4 rows of bf16 activations takes it; deferred: its sums over K have a taker
 bool gemv_few_rows_in_regs(const LinearW& w, int M, size_t ws_bytes, bool deferred);
 // sums the slabs and runs the epilogue

@@ -354,7 +354,7 @@ static int gemm_wide_ks() {      // MI355X_GEMM_WIDE_KS: 1 = never split K in th
 // the wide GEMM 0.54 and 0.11, the rule before 0.33 and 0.11), unsplit 0.04 and 0.06 (0.75 and 0.42; 0.60 and 0.42), sums of 4096 deep and more that the next norm takes 0.23 (0.42; 0.44), int8 see below.  The rule before
 // went by the share of a wave's requests that are k-tiles of its own, and tiles that are not a wave's own are no requests any more.
 // Not bf16 weights, nor up to 16 rows (28672 x 4096 fp8 23.4 -> 23.8 us); nothing beyond the sizes measured.
-bool gemm_wide_few_rows(const LinearW& w, int M, int epi, size_t ws_bytes, bool deferred) {
+bool gemm_wide_few_rows(const LinearW& w, int M, size_t ws_bytes, bool deferred) {
   int cus = 0;
   if (gemm_wide_mode() == 0 || gemm_wide_bm()) return false;      // (128 tokens and more: none of these calls has them)
   if (M < 17 || M > 32 || w.wd == MI_W_BF16 || w.K % 64 != 0 || w.K < 2048 || w.N < 2048 || w.N > 65536 || device_num_cu(&cus) != MI_OK) return false;

@@ -158,7 +158,7 @@ __global__ __launch_bounds__(1024) void norm_rows_kernel(const float* __restrict
   }
 }
 // The same for the few rows of a token-generation step, the row over kNormParts work-groups: a CU takes in some 35 GB/s of a row and its slabs (32 rows of 4096 behind
-// 8 slabs: 147 KB a work-group, 5.8 us a launch; 4.7 so, which is what the smallest launch takes that reads what others wrote: 5 rows 4.8 and 4.6).  Each leaves the sum of its squares; whoever takes the rows adds them up and applies 1 / rms
+// 8 slabs: 147 KB a work-group, 5.8 us a launch; 4.7 so, which is what the smallest launch takes that reads what others wrote: 24 rows 5.1 and 4.8, 5 rows 4.8 and 4.6).  Each leaves the sum of its squares; whoever takes the rows adds them up and applies 1 / rms
 // (RowFactor), so that what is rounded to bf16 is h * gain.
 __global__ __launch_bounds__(1024) void norm_parts_kernel(const float* __restrict__ resid_in, const float* __restrict__ partial, float* __restrict__ resid_out,
                                                          const float* __restrict__ gain, int H, uint16_t* __restrict__ y, float* __restrict__ ss_out, SlabSum sl) {

@@ -163,7 +163,7 @@ int run_linear(mi_ctx* c, const Linear& L, int rows, int pro, ProArgs p, int epi
     if (!c->runs(MI_K_GEMV)) return MI_OK;
     Scope sc(c, MI_K_GEMV);
     if (c->prof.on) c->prof.gemv_bytes += (double)L.bytes();
-    if (!e.far_out && ldx % 8 == 0 && gemm_wide_few_rows(L.view(), rows, epi, c->splitk_ws_bytes, defer || as_deferred))
+    if (!e.far_out && ldx % 8 == 0 && gemm_wide_few_rows(L.view(), rows, c->splitk_ws_bytes, defer || as_deferred))
       MI_TRY(launch_gemm_wide(L.view(), rows, x, ldx, epi, e, c->stream, c->splitk_ws, c->splitk_ws_bytes, defer, as_deferred));
     else
       MI_TRY(launch_gemv_regs(L.view(), rows, x, ldx, epi, e, c->stream, c->splitk_ws, c->splitk_ws_bytes, defer, as_deferred));
@@ -2118,7 +2118,7 @@ int mi_op_qlinear(const void* x, int32_t M, const void* w_tiled, const float* sc
     float* slab = nullptr;
     const size_t bytes = (size_t)64 << 20;
     MI_HIP(hipMalloc(reinterpret_cast<void**>(&slab), bytes));
-    int rc = gemm_wide_few_rows(W, M, EPI_F32, bytes, false) ? launch_gemm_wide(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes)
+    int rc = gemm_wide_few_rows(W, M, bytes, false) ? launch_gemm_wide(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes)
              : gemv_in_regs(W, M, bytes) || gemv_few_rows_in_regs(W, M, bytes, false) ? launch_gemv_regs(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes)
              : gemv_fits(M, K) ? launch_gemv(W, M, PRO_BF16, p, EPI_F32, e, (hipStream_t)stream) : launch_gemm(W, M, p.x, K, EPI_F32, e, (hipStream_t)stream, slab, bytes);
     hipStreamSynchronize((hipStream_t)stream);
