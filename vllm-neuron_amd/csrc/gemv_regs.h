@@ -267,7 +267,12 @@ int launch_gemv_regs_wd(const LinearW& w, int M, const uint16_t* x, int ldx, int
     if constexpr (WD == MI_W_BF16)
       if (epi == EPI_SOFTCAP) return launch_gemv_regs_k<WD, EPI_SOFTCAP, 2, false, 4>(w, M, x, ldx, e, s, 1, nullptr);
   }
-#define MI_R(EPI_) return M <= 16 ? launch_gemv_regs_k<WD, EPI_, 1, false>(w, M, x, ldx, e, s, 1, nullptr) : launch_gemv_regs_k<WD, EPI_, 2, false>(w, M, x, ldx, e, s, 1, nullptr)
+  // (far results are stored through up to 16 rows: left in L2 they cross PCIe when the weights are done.  Steps of half-depth models, us: 8B fp8 4 rows 1116 -> 1095, 8 rows 1147 -> 1120,
+  //  16 rows 1299 -> 1288, 7B int8 5 rows 1138 -> 1088, 2048 wide 2 - 16 rows 0.2 - 3 %.  From 17 on PCIe is what bounds them, and pieces of 64 bytes are best put together by the L2: 24 rows of 8B
+  //  in groups of four row-tiles 1507, single ones stored through 1535, 32 rows 1606 and 1650)
+  EpiArgs near = e;
+  near.far_out = false;
+#define MI_R(EPI_) return M <= 16 ? launch_gemv_regs_k<WD, EPI_, 1, false>(w, M, x, ldx, e, s, 1, nullptr) : launch_gemv_regs_k<WD, EPI_, 2, false>(w, M, x, ldx, near, s, 1, nullptr)
   switch (epi) {
     case EPI_QKV: MI_R(EPI_QKV);
     case EPI_SWIGLU: MI_R(EPI_SWIGLU);

@@ -95,8 +95,8 @@ __device__ __forceinline__ void epilogue_put(const EpiArgs& e, int m, int n, int
 template <int EPI>
 __device__ __forceinline__ void epilogue_store(const EpiArgs& e, int m, int n0, f32x4_t v) {
   if constexpr (EPI == EPI_F32) {
-    *reinterpret_cast<float4*>(e.out_f32 + (size_t)m * e.ld_out + n0) =
-        make_float4(v[0], v[1], v[2], v[3]);
+    if (e.far_out) store_through(e.out_f32, ((uint32_t)m * e.ld_out + n0) * 4u, v);
+    else *reinterpret_cast<f32x4_t*>(e.out_f32 + (size_t)m * e.ld_out + n0) = v;
   } else if constexpr (EPI == EPI_RESID) {  // residual stream: out = resid_in + y (fp32)
     const float4 r = *reinterpret_cast<const float4*>(e.resid_in + (size_t)m * e.ld_out + n0);
     *reinterpret_cast<float4*>(e.out_f32 + (size_t)m * e.ld_out + n0) =
@@ -104,8 +104,7 @@ __device__ __forceinline__ void epilogue_store(const EpiArgs& e, int m, int n0, 
   } else if constexpr (EPI == EPI_SWIGLU || EPI == EPI_GLU_CLIP) {
     *reinterpret_cast<uint32_t*>(e.act_out + (size_t)m * e.ld_act + (n0 >> 1)) = epilogue_half<EPI>(e, v);
   } else if constexpr (EPI == EPI_SOFTCAP) {
-    *reinterpret_cast<float4*>(e.out_f32 + (size_t)m * e.ld_out + n0) =
-        make_float4(e.softcap * tanhf(v[0] / e.softcap), e.softcap * tanhf(v[1] / e.softcap), e.softcap * tanhf(v[2] / e.softcap), e.softcap * tanhf(v[3] / e.softcap));
+    epilogue_store<EPI_F32>(e, m, n0, f32x4_t{e.softcap * tanhf(v[0] / e.softcap), e.softcap * tanhf(v[1] / e.softcap), e.softcap * tanhf(v[2] / e.softcap), e.softcap * tanhf(v[3] / e.softcap)});
   } else if constexpr (EPI == EPI_RELU2 || EPI == EPI_HEADS_KV) {
     epilogue_put<EPI>(e, m, n0, 0, epilogue_whole<EPI>(v));
   } else {  // EPI_QKV

@@ -19,7 +19,7 @@ struct EpiArgs {
   // EPI_F32: out[m * ld_out + n] = y;  EPI_RESID: out = resid_in[m * ld_out + n] + y
   float* out_f32;
   int ld_out;
-  bool far_out;        // out_f32 is host memory (launch_gemv_regs, EPI_F32 and EPI_SOFTCAP: results leave in larger pieces)
+  bool far_out;        // out_f32 is host memory (launch_gemv, launch_gemv_regs, EPI_F32 and EPI_SOFTCAP: results are stored through L2, or leave in larger pieces)
   const float* resid_in;
   // EPI_QKV: rows [0,q_dim) -> RoPE -> q_out; [q_dim, q_dim+kv_dim) -> RoPE -> K pool;
   // the rest -> V pool.  Rows of every q/k head are stored pair-interleaved

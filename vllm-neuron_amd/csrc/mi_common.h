@@ -124,6 +124,13 @@ __device__ __forceinline__ uint4 nt_load16(const uint4* p) {
   return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
+// A 16-byte store to `at` bytes behind `base` (the same for the whole wave) that does not stay in this XCD's L2 (sc1).  What a kernel leaves dirty there is written out when
+// the kernel ends, in front of the next one's start; written through it leaves while the kernel still works.  (A builtin: the results of MFMAs that are still
+// on their way are waited for in front of an instruction the compiler knows, and not in front of inline asm.)
+__device__ __forceinline__ void store_through(void* base, uint32_t at, f32x4_t v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), __builtin_amdgcn_make_buffer_rsrc(base, 0, 0xffffffffu, 0x00020000), at, 0, 16);
+}
+
 // fp32 -> OCP e4m3fn, round-nearest-even, saturating at +-448: the hardware convert of gfx950 (v_cvt_pk_fp8_f32; OCP
 // formats on this chip).  The clamp in front makes the result independent of the instruction's own out-of-range rule; a NaN
 // input becomes +-448 like any other out-of-range value.  (Written out it is ~20 integer / select instructions per value,
