@@ -225,3 +225,9 @@ def test_sums_of_slices_round_once(lib, M, N, K, ks):
     ref = (x.double() @ q.double().t()) * scale.cpu().double() + bias.double()      # 48 bits and a sum: 64-bit rounding is 2^-29 of a unit here
     unit = 2.0 ** (torch.frexp(ref.abs())[1].double() - 24)
     assert ((y.cpu().double() - ref).abs() <= 0.50001 * unit).all()
+
+
+# slabs of 24 MiB (written through), one row more than that, and twice as much, whole token blocks and a short last one
+@pytest.mark.parametrize("M,N,K,bm,ntw,ks", [(1024, 2048, 128, 128, 2, 3), (1025, 2048, 192, 128, 3, 3), (2048, 2064, 192, 256, 4, 3), (1024, 3072, 128, 256, 4, 2)])
+def test_slabs_left_in_l2_and_written_through(lib, M, N, K, bm, ntw, ks):
+    check_tile(lib, "bf16", bm, ntw, ((M, N, K, min(ks, K // 64)),))
