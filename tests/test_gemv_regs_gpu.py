@@ -370,3 +370,30 @@ def test_epilogues_of_several_row_tiles(wd, rows, hidden, heads, kv, dim, inter)
 
 
 _oracle = []
+
+
+# norms that a residual projection hands on to the next one: 3, 32, 33 and 64 requests of 4 parts for a row (the second 32 are a thread's second request), down projections that
+# keep K in one piece (their norm is handed on too, the last one's to the head) and one that does not, a width whose next projection splits K; the fewest rows, the most, one more
+@pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
+@pytest.mark.parametrize("hidden,inter", [(192, 320), (2048, 4096), (2112, 4160), (4096, 1024), (4160, 512)])
+def test_norms_handed_on(wd, hidden, inter):
+    from oracle import DecoderConfig, PagedDecoderOracle
+    from oracle.synth import make_weights
+    from tests.helpers import decode_inputs
+    from vllm_neuron_amd._native import MI_Q, MI_W, NativeModel
+    shape = dict(num_layers=2, hidden_size=hidden, num_heads=4, num_kv_heads=2, head_dim=64, intermediate_size=inter, vocab_size=528)
+    cfg = DecoderConfig(**shape)
+    w = make_weights(cfg, seed=5)
+    model = NativeModel(**shape, rms_norm_eps=cfg.rms_norm_eps, rope_theta=cfg.rope_theta, rope_type=0, rope_factor=1.0, num_blocks=34, block_size=32, max_num_seqs=32,
+                        max_model_len=32, weight_dtype=MI_W[wd], quant_type=MI_Q["per_channel_symmetric"], quantize_lm_head=1, tp_degree=1, tp_rank=0, device_id=0,
+                        use_graphs=1, ctx_buckets=[32])
+    model.load_state_dict(w)
+    model.finalize()
+    for rows in (5, 16, 17):
+        oracle = PagedDecoderOracle(cfg, w, 34, 32, compute="bf16", quant=_quant(wd))
+        for at in range(3):                # the call that is captured, and two replays
+            inputs = decode_inputs([(31 * i + 7 * at) % 528 for i in range(rows)], [at] * rows, [[1 + i] for i in range(rows)], 32, 32)
+            want = oracle.forward(**inputs).float()
+            d = model.forward(**inputs).float() - want
+            assert torch.isfinite(d).all() and d.pow(2).mean().sqrt() < 0.02 * want.std() and d.abs().max() < 0.1 * want.std()       # as above
+    model.close()

@@ -15,10 +15,6 @@
 namespace mi {
 
 constexpr int kRegsMaxPasses = 64;   // row-tiles of a work-group: their scales and biases wait in LDS
-// k-tiles a wave holds at most: 8 of 64 k (1-byte weights), 16 of 32 k.  There is a kernel for 4, 5, 6, 7, 8 (bf16 also 12, 14, 16), since a wave asks for
-// the activations of all of them and multiplies all of them, its own or not; weights that are not its own are zeros without a request (stream_batch).  With 4, 8 and 16 alone, when they were
-// requests for its last tile again, us a step: 7B int8 5 rows 1243 -> 1196, bf16 1679 -> 1583, 8B fp8 8 rows 1230 -> 1207.
-template <int WD> constexpr int kRegsMaxTiles = WD == MI_W_BF16 ? 16 : 8;
 
 // HOLD: a work-group takes HOLD row-tiles side by side, and the wave that sums them keeps their results until it has all: a row's HOLD x 64 bytes
 // leave together.  For results that go over PCIe: neighbouring 64 bytes that come from different work-groups take a packet each, 44 GB/s; 128 or 256 bytes
@@ -33,6 +29,8 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
   __shared__ f32x4_t red[2][kGemvWaves][MG][64];
   __shared__ __attribute__((aligned(16))) float sc_lds[SLAB ? 4 : kRegsMaxPasses * 16], bi_lds[SLAB ? 4 : kRegsMaxPasses * 16];
   __shared__ float rf_lds[SLAB ? 1 : 16 * MG];        // the rows' own factors: 1 / rms where the norm left it to the output
+  constexpr bool kNext = !SLAB && EPI == EPI_RESID && MG == 1;
+  __shared__ __attribute__((aligned(16))) float ga_lds[kNext ? kRegsMaxPasses * 16 : 4];   // the gains of the norm behind
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int g = lane >> 4, c = lane & 15;
   const int kper = ceil_div(KT, (int)gridDim.y), k_lo = (int)blockIdx.y * kper, k_hi = min(k_lo + kper, KT);
@@ -53,6 +51,22 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
 #pragma unroll
       for (int f = 0; f < FR; ++f) xf[(j * FR + f) * MG + mg] = *reinterpret_cast<const u32x4_t*>(row + (size_t)kt * TK + f * 8);
     }
+  }
+  // The rows' own factors (no residual has one).  Everybody asks, so that no branch waits; in front of the weights, whose second batch would wait for them behind the first
+  // (sums of squares over 16 columns, 16 rows of 4096: gate | up of the 8B shape 23.3 us that way, 22.3 now; QKV 10.4 and 9.7; scales and biases asked for up here gained nothing).
+  constexpr bool kFactor = !SLAB && EPI != EPI_RESID;
+  RowFactor rf;
+  float4 ss0, ss1;                                    // 16 rows: 32 threads a row, up to 8 parts each
+  const bool parts = e.rs_n > 0.f;
+  const int n4 = parts ? e.rs_parts >> 2 : 1, pl = tid & 31;
+  if constexpr (kFactor && MG == 1) {
+    const float* q = e.row_scale ? e.row_scale : e.scale;
+    const float* p4 = parts ? q + (size_t)min(tid >> 5, M - 1) * e.rs_parts : e.scale;
+    rf.a = q[e.row_scale && !parts ? min(tid >> 5, M - 1) : 0];
+    ss0 = reinterpret_cast<const float4*>(p4)[min(pl, n4 - 1)];
+    ss1 = reinterpret_cast<const float4*>(p4)[min(pl + 32, n4 - 1)];
+  } else if constexpr (kFactor) {
+    rf.request(e.row_scale ? e.row_scale : e.scale, e.row_scale ? min(tid, M - 1) : 0, e.rs_n);   // (a thread a row)
   }
   __builtin_amdgcn_sched_barrier(0);
   // operands of the epilogue of the first row-tile (and column group) that this wave finishes
@@ -76,8 +90,6 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
     }
   if constexpr (kPre) epi_prefetch_dependent<EPI>(e, pre_n, epre);
   if constexpr (!SLAB) {
-    RowFactor rf;                                     // (a thread a row; all ask, so that no branch waits for it)
-    rf.request(e.row_scale ? e.row_scale : e.scale, e.row_scale ? min(tid, M - 1) : 0, e.rs_n);
     const int n = passes * 16;
 #pragma unroll
     for (int q = 0; q < kRegsMaxPasses * 16 / (kGemvWaves * 64); ++q) {
@@ -86,9 +98,20 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
         const int at = tile_of(i >> 4) * 16 + (i & 15);
         sc_lds[i] = e.scale[at];
         bi_lds[i] = e.bias ? e.bias[at] : 0.f;
+        if constexpr (kNext) ga_lds[i] = e.next_x ? e.next_gain[at] : 0.f;
       }
     }
-    if (tid < 16 * MG) rf_lds[tid] = e.row_scale ? rf.value(e.rs_n, e.rs_eps) : 1.f;
+    if constexpr (!kFactor) {
+      if (tid < 16 * MG) rf_lds[tid] = 1.f;
+    } else if constexpr (MG == 1) {
+      float ss = pl < n4 ? (ss0.x + ss0.y) + (ss0.z + ss0.w) : 0.f;
+      if (pl + 32 < n4) ss += (ss1.x + ss1.y) + (ss1.z + ss1.w);
+      ss = group_sum<16>(ss);
+      ss += __shfl_xor(ss, 16);
+      if (pl == 0) rf_lds[tid >> 5] = !e.row_scale ? 1.f : parts ? rsqrtf(ss / e.rs_n + e.rs_eps) : rf.a;
+    } else {
+      if (tid < 16 * MG) rf_lds[tid] = e.row_scale ? rf.value(e.rs_n, e.rs_eps) : 1.f;
+    }
   }
   issue(bufB, 1);
 
@@ -160,6 +183,28 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
       } else {
         const float *sc4 = sc_lds + pass * 16 + g * 4, *b4 = e.bias ? bi_lds + pass * 16 + g * 4 : nullptr, rmul = rf_lds[m];
         bool done = false;
+        if constexpr (kNext) {
+          f32x4_t r = __builtin_bit_cast(f32x4_t, epre.r);
+          asm volatile("" : "+v"(r));                 // (else the two places it comes from become one load, and the first of them memory)
+          if (pass != pre_pass) r = *reinterpret_cast<const f32x4_t*>(e.resid_in + (size_t)m * e.ld_out + n0);
+          const float4 sc = *reinterpret_cast<const float4*>(sc4);
+          s[0] *= sc.x * rmul; s[1] *= sc.y * rmul; s[2] *= sc.z * rmul; s[3] *= sc.w * rmul;
+          if (b4) {
+            const float4 b = *reinterpret_cast<const float4*>(b4);
+            s[0] += b.x; s[1] += b.y; s[2] += b.z; s[3] += b.w;
+          }
+          const float4 o = make_float4(r[0] + s[0], r[1] + s[1], r[2] + s[2], r[3] + s[3]);
+          *reinterpret_cast<float4*>(e.out_f32 + (size_t)m * e.ld_out + n0) = o;
+          if (e.next_x) {
+            const float4 ga = *reinterpret_cast<const float4*>(ga_lds + pass * 16 + g * 4);
+            *reinterpret_cast<uint2*>(e.next_x + (size_t)m * e.ld_out + n0) = make_uint2(pack_bf16x2(o.x * ga.x, o.y * ga.y), pack_bf16x2(o.z * ga.z, o.w * ga.w));
+            float ss = o.x * o.x + o.y * o.y + o.z * o.z + o.w * o.w;
+            ss += __shfl_xor(ss, 16);
+            ss += __shfl_xor(ss, 32);
+            if (g == 0) e.next_ss[m * NT + tile_of(pass)] = ss;
+          }
+          continue;
+        }
         if constexpr (kPre) {
           if (pass == pre_pass) { epilogue_pre<EPI>(e, m, n0, sc4, b4, s, epre, rmul); done = true; }
         }
@@ -234,7 +279,7 @@ static int gemv_regs_slices(int M, int N, int K, size_t ws_bytes, bool deferred,
   const int NT = N / 16, KT = K / tile_k(WD);
   int best = 0;
   double best_cost = 0.;
-  for (int z = ceil_div(KT, kGemvWaves * kRegsMaxTiles<WD>); z <= 8; ++z) {
+  for (int z = ceil_div(KT, kGemvWaves * regs_max_tiles(WD)); z <= 8; ++z) {
     const int per = ceil_div(KT, z);
     if (z > 1 && ((z - 1) * per >= KT || (size_t)z * M * N * sizeof(float) > ws_bytes)) continue;
     double cost = ceil_div(NT, std::max(1, num_cu / z)) * (per / 24.0 + 0.3) + (double)M * per * tile_k(WD) * 4e-5;
@@ -251,8 +296,12 @@ int launch_gemv_regs_wd(const LinearW& w, int M, const uint16_t* x, int ldx, int
   int num_cu = 0;
   MI_TRY_(device_num_cu(&num_cu));
   const bool deferred = defer && (epi == EPI_RESID || epi == EPI_F32);
-  const int slices = gemv_regs_slices<WD>(M, w.N, w.K, ws ? ws_bytes : 0, deferred || split_as_deferred, num_cu);
+  // (where the norm behind is left to its projection, an unsplit K saves that norm's launch: 4.7 us against the 0.3 - 1 that half-empty CUs cost)
+  const int slices = e.next_x ? 1 : gemv_regs_slices<WD>(M, w.N, w.K, ws ? ws_bytes : 0, deferred || split_as_deferred, num_cu);
   MI_CHECK(slices > 0, "gemv_regs: no split of K fits the workspace");
+  MI_CHECK(!e.next_x || (epi == EPI_RESID && M <= 16 && gemv_regs_holds(w)), "gemv_regs: a norm handed on is for residuals of up to 16 rows, K in one slice");
+  MI_CHECK(epi != EPI_RESID || !e.row_scale || slices > 1, "gemv_regs: no residual takes a factor a row");
+  MI_CHECK(e.rs_n == 0.f || e.rs_parts == kNormParts || (M <= 16 && slices == 1 && e.rs_parts % 4 == 0 && e.rs_parts > 0 && e.rs_parts <= 256), "gemv_regs: a norm's parts");
   if (slices > 1) {
     MI_TRY_(M <= 16 ? (launch_gemv_regs_k<WD, EPI_F32, 1, true>(w, M, x, ldx, e, s, slices, ws)) : (launch_gemv_regs_k<WD, EPI_F32, 2, true>(w, M, x, ldx, e, s, slices, ws)));
     const SlabSum sum{ws, slices, M, w.N, e.scale, e.bias, e.row_scale, e.rs_n, e.rs_eps};
@@ -294,6 +343,12 @@ template <int WD>
 bool gemv_regs_fits_wd(int M, int N, int K, size_t ws_bytes) {
   int num_cu = 0;
   return device_num_cu(&num_cu) == MI_OK && gemv_regs_slices<WD>(M, N, K, ws_bytes, false, num_cu) > 0;
+}
+
+template <int WD>
+bool gemv_regs_whole_wd(int M, int N, int K, size_t ws_bytes) {
+  int num_cu = 0;
+  return device_num_cu(&num_cu) == MI_OK && gemv_regs_slices<WD>(M, N, K, ws_bytes, false, num_cu) == 1;
 }
 
 // what the choice of slices takes the launch and the sum of its slices to be, us; 0: no split fits

@@ -14,13 +14,19 @@ enum { PRO_BF16 = 0, PRO_NORM = 1, PRO_NORM_PARTIAL = 2 };  // callers pass PRO_
 struct EpiArgs {
   const float* scale;  // [N] per-output-row dequant scale
   const float* row_scale;  // [M] factor per row (per-token activation scale of the FP8-activation GEMM; launch_gemv_regs) or nullptr
-  float rs_n, rs_eps;      // rs_n > 0: row_scale holds [M][kNormParts] sums of squares of rows of rs_n numbers, the factor is 1 / rms (launch_norm_parts)
+  float rs_n, rs_eps;      // rs_n > 0: row_scale holds [M][rs_parts] sums of squares of rows of rs_n numbers, the factor is 1 / rms (launch_norm_parts)
+  int rs_parts;            // kNormParts; launch_gemv_regs of an unsplit K and up to 16 rows: any multiple of 4 up to 256
   const float* bias;   // [N] or nullptr
   // EPI_F32: out[m * ld_out + n] = y;  EPI_RESID: out = resid_in[m * ld_out + n] + y
   float* out_f32;
   int ld_out;
   bool far_out;        // out_f32 is host memory (launch_gemv, launch_gemv_regs, EPI_F32 and EPI_SOFTCAP: results are stored through L2, or leave in larger pieces)
   const float* resid_in;
+  // EPI_RESID, launch_gemv_regs, up to 16 rows, or null: the norm behind is left to its projection, which takes next_x[m * ld_out + n] = bf16(out next_gain[n]) and 1 / rms
+  //   from next_ss [M][N / 16], the sums of squares of out over 16 columns.  K is not split then (gemv_regs_holds)
+  const float* next_gain;
+  uint16_t* next_x;
+  float* next_ss;
   // EPI_QKV: rows [0,q_dim) -> RoPE -> q_out; [q_dim, q_dim+kv_dim) -> RoPE -> K pool;
   // the rest -> V pool.  Rows of every q/k head are stored pair-interleaved
   // (2i <- d=i, 2i+1 <- d=i+hd/2) so a lane owns both halves of a rotation.
@@ -71,6 +77,13 @@ int launch_gemv_regs(const LinearW& w, int M, const uint16_t* x, int ldx, int ep
                      SlabSum* defer = nullptr, bool split_as_deferred = false);
 // whether M rows of w take it (K beyond 8 slices of the registers, or slabs that do not fit: launch_gemv up to 16 rows, launch_gemm)
 bool gemv_in_regs(const LinearW& w, int M, size_t ws_bytes);
+// k-tiles a wave holds at most: 8 of 64 k (1-byte weights), 16 of 32 k.  There is a kernel for 4, 5, 6, 7, 8 (bf16 also 12, 14, 16), since a wave asks for
+// the activations of all of them and multiplies all of them, its own or not; weights that are not its own are zeros without a request (stream_batch).  With 4, 8 and 16 alone, when they were
+// requests for its last tile again, us a step: 7B int8 5 rows 1243 -> 1196, bf16 1679 -> 1583, 8B fp8 8 rows 1230 -> 1207.
+constexpr int regs_max_tiles(int wd) { return wd == MI_W_BF16 ? 16 : 8; }
+// whether all of K fits the registers of a work-group, and whether K goes unsplit by launch_gemv_regs' own choice where nobody takes the slices' sum
+bool gemv_regs_holds(const LinearW& w);
+bool gemv_regs_whole(const LinearW& w, int M, size_t ws_bytes);
 // where launch_gemm_wide takes less time than launch_gemv_regs (17 .. 32 rows); deferred: the sum of K slices has a taker
 bool gemm_wide_few_rows(const LinearW& w, int M, size_t ws_bytes, bool deferred);
 // whether a projection of 1 .. 4 rows of bf16 activations takes it; deferred: its sums over K have a taker

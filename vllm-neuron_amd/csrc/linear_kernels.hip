@@ -53,6 +53,16 @@ static bool gemv_regs_fits(const LinearW& w, int M, size_t ws_bytes) {
   }
   return false;
 }
+template <int WD> bool gemv_regs_whole_wd(int M, int N, int K, size_t ws_bytes);
+bool gemv_regs_whole(const LinearW& w, int M, size_t ws_bytes) {
+  switch (w.wd) {
+    case MI_W_BF16: return gemv_regs_whole_wd<MI_W_BF16>(M, w.N, w.K, ws_bytes);
+    case MI_W_F8E4M3: return gemv_regs_whole_wd<MI_W_F8E4M3>(M, w.N, w.K, ws_bytes);
+    case MI_W_INT8: return gemv_regs_whole_wd<MI_W_INT8>(M, w.N, w.K, ws_bytes);
+  }
+  return false;
+}
+bool gemv_regs_holds(const LinearW& w) { return ceil_div(w.K / tile_k(w.wd), kGemvWaves) <= regs_max_tiles(w.wd); }
 // From 5 rows on (us per call; the LDS kernels with the norm in front of them / these behind a norm kernel; contexts of 500, TinyLlama 200):
 //   8B fp8, 16 layers:  8 rows 1472 / 1332, 16 rows 1758 / 1527, 32 rows 2282 / 2117;   4 rows 1191 / 1277
 //   8B bf16:            8 rows 1949 / 1857, 24 rows 2526 / 2298

@@ -8,10 +8,10 @@ int launch_embed(const int32_t* ids, const uint16_t* table, int T, int H, float*
 // splitk_reduce + residual epilogue followed by this kernel
 int launch_norm_rows(const float* resid_in, const float* partial, float* resid_out, const float* gain, int T,
                      int H, float eps, uint16_t* y, hipStream_t s, const SlabSum* slabs = nullptr, float* rinv = nullptr);
-// for the few rows of a token-generation step: y = bf16(h * gain) and ss = [T][kNormParts] sums of squares of h (EpiArgs::rs_n)
+// for the few rows of a token-generation step: y = bf16(h * gain) and ss = [T][kNormParts] sums of squares of h (EpiArgs::rs_n); fine: [T][H / 16]
 bool norm_parts_fit(int H);
 int launch_norm_parts(const float* resid_in, const float* partial, float* resid_out, const float* gain, int T, int H, uint16_t* y, float* ss, hipStream_t s,
-                      const SlabSum* slabs);
+                      const SlabSum* slabs, bool fine = false);
 // the same row, emitted as the FP8 GEMM's input: bf16-rounded, then e4m3 with scale amax / 448,
 // K-step-major image [H / 128][T][128 B] + row_scale[T]
 int launch_norm_rows_fp8(const float* resid_in, const float* partial, float* resid_out, const float* gain, int T,

@@ -161,7 +161,7 @@ __global__ __launch_bounds__(1024) void norm_rows_kernel(const float* __restrict
 // 8 slabs: 147 KB a work-group, 5.8 us a launch; 4.7 so, which is what the smallest launch takes that reads what others wrote: 24 rows 5.1 and 4.8, 5 rows 4.8 and 4.6).  Each leaves the sum of its squares; whoever takes the rows adds them up and applies 1 / rms
 // (RowFactor), so that what is rounded to bf16 is h * gain.
 __global__ __launch_bounds__(1024) void norm_parts_kernel(const float* __restrict__ resid_in, const float* __restrict__ partial, float* __restrict__ resid_out,
-                                                         const float* __restrict__ gain, int H, uint16_t* __restrict__ y, float* __restrict__ ss_out, SlabSum sl) {
+                                                         const float* __restrict__ gain, int H, uint16_t* __restrict__ y, float* __restrict__ ss_out, int fine, SlabSum sl) {
   __shared__ float red[16];
   const int t = blockIdx.y, part = blockIdx.x, tid = threadIdx.x, mine = H / kNormParts;
   const bool in = tid * 4 < mine;
@@ -187,7 +187,13 @@ __global__ __launch_bounds__(1024) void norm_parts_kernel(const float* __restric
     if (resid_out) *reinterpret_cast<float4*>(resid_out + o) = a;
     *reinterpret_cast<uint2*>(y + o) = make_uint2(pack_bf16x2(a.x * g.x, a.y * g.y), pack_bf16x2(a.z * g.z, a.w * g.w));
   }
-  float ss = wave_sum(in ? a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w : 0.f);
+  float ss = in ? a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w : 0.f;
+  if (fine) {          // a part for 16 columns, as the residual projection leaves them that hands its norm on
+    ss = group_sum<4>(ss);
+    if (in && (tid & 3) == 0) ss_out[t * (H / 16) + (col >> 4)] = ss;
+    return;
+  }
+  ss = wave_sum(ss);
   if ((tid & 63) == 0) red[tid >> 6] = ss;
   __syncthreads();
   if (tid) return;
@@ -195,10 +201,10 @@ __global__ __launch_bounds__(1024) void norm_parts_kernel(const float* __restric
   ss_out[t * kNormParts + part] = ss;
 }
 bool norm_parts_fit(int H) { return H % (4 * kNormParts) == 0 && H <= 1024 * 4 * kNormParts; }
-int launch_norm_parts(const float* resid_in, const float* partial, float* resid_out, const float* gain, int T, int H, uint16_t* y, float* ss, hipStream_t s, const SlabSum* slabs) {
-  MI_CHECK(norm_parts_fit(H) && T >= 1 && T <= 65535, "rmsnorm: a float4 per thread of four work-groups a row");
+int launch_norm_parts(const float* resid_in, const float* partial, float* resid_out, const float* gain, int T, int H, uint16_t* y, float* ss, hipStream_t s, const SlabSum* slabs, bool fine) {
+  MI_CHECK((!fine || H % 64 == 0) && norm_parts_fit(H) && T >= 1 && T <= 65535, "rmsnorm: a float4 per thread of four work-groups a row");
   MI_CHECK(!slabs || (slabs->T == T && slabs->N == H && resid_out && slabs->rs_n == 0.f), "rmsnorm: pending K-split sum of another shape");
-  hipLaunchKernelGGL(norm_parts_kernel, dim3(kNormParts, T), dim3(ceil_div(H / kNormParts, 256) * 64), 0, s, resid_in, partial, resid_out, gain, H, y, ss, slabs ? *slabs : SlabSum());
+  hipLaunchKernelGGL(norm_parts_kernel, dim3(kNormParts, T), dim3(ceil_div(H / kNormParts, 256) * 64), 0, s, resid_in, partial, resid_out, gain, H, y, ss, (int)fine, slabs ? *slabs : SlabSum());
   MI_HIP(hipGetLastError());
   return MI_OK;
 }

@@ -70,7 +70,8 @@ struct mi_ctx {
   uint16_t *xn = nullptr, *qbuf = nullptr, *attn_out = nullptr, *act = nullptr;
   uint8_t* x8 = nullptr;        // FP8-activation GEMM input [rows, K]
   int attn_max_ctx = 0;         // longest context of the staged token-generation rows (0: none staged)
-  float* row_rinv = nullptr;    // up to 32 rows, for the projection behind the norm: [32][kNormParts] sums of squares, or (norm_parts_fit says no) 1 / rms
+  float* row_rinv = nullptr;    // up to 32 rows, for the projection behind the norm: [32][kNormParts] or [16][H / 16] sums of squares, or (norm_parts_fit says no) 1 / rms
+  struct { const float *resid = nullptr, *gain = nullptr; int rows = 0; } handed;   // the norm that the last residual projection left in xn and row_rinv (run_linear)
   float* x8_scale = nullptr;    // its per-token scales [rows]
   float* splitk_ws = nullptr;   // fp32 K-split slabs of short-prompt GEMMs
   mi::SlabSum pend;               // a residual projection's K-split sum left for the next row norm (run_linear)
