@@ -373,9 +373,10 @@ _oracle = []
 
 
 # norms that a residual projection hands on to the next one: 3, 32, 33 and 64 requests of 4 parts for a row (the second 32 are a thread's second request), down projections that
-# keep K in one piece (their norm is handed on too, the last one's to the head) and one that does not, a width whose next projection splits K; the fewest rows, the most, one more
+# keep K in one piece (their norm is handed on too, the last one's to the head) and some that do not (up to 4 rows every kernel hands it on), a width whose next projection splits K; the rows on
+# both sides of each kernel
 @pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
-@pytest.mark.parametrize("hidden,inter", [(192, 320), (2048, 4096), (2112, 4160), (4096, 1024), (4160, 512)])
+@pytest.mark.parametrize("hidden,inter", [(192, 320), (2048, 4096), (2112, 4160), (4096, 1024), (4160, 512), (1024, 19008)])
 def test_norms_handed_on(wd, hidden, inter):
     from oracle import DecoderConfig, PagedDecoderOracle
     from oracle.synth import make_weights
@@ -389,7 +390,7 @@ def test_norms_handed_on(wd, hidden, inter):
                         use_graphs=1, ctx_buckets=[32])
     model.load_state_dict(w)
     model.finalize()
-    for rows in (5, 16, 17):
+    for rows in (1, 2, 4, 5, 16, 17):
         oracle = PagedDecoderOracle(cfg, w, 34, 32, compute="bf16", quant=_quant(wd))
         for at in range(3):                # the call that is captured, and two replays
             inputs = decode_inputs([(31 * i + 7 * at) % 528 for i in range(rows)], [at] * rows, [[1 + i] for i in range(rows)], 32, 32)

@@ -22,6 +22,7 @@ constexpr int kRegsMaxPasses = 64;   // row-tiles of a work-group: their scales 
 template <int WD, int EPI, int MG, int NK, bool SLAB, int HOLD = 1>
 __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4* __restrict__ W, int NT, int KT, int M, int G,
                                                                    const uint16_t* __restrict__ x, int ldx, EpiArgs e, float* __restrict__ slab) {
+  if constexpr (MG == 2) e.next_x = nullptr;          // (up to 16 rows; the registers of 32 leave no room for it)
   constexpr int FR = WD == MI_W_BF16 ? 1 : 2;         // MFMAs per weight tile and column group
   constexpr int NB = NK > 8 ? 2 : 1, BT = NK / NB;    // batches per row-tile, weight tiles per request batch (up to 8 KiB a wave)
   constexpr int TK = WD == MI_W_BF16 ? 32 : 64;
@@ -29,8 +30,6 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
   __shared__ f32x4_t red[2][kGemvWaves][MG][64];
   __shared__ __attribute__((aligned(16))) float sc_lds[SLAB ? 4 : kRegsMaxPasses * 16], bi_lds[SLAB ? 4 : kRegsMaxPasses * 16];
   __shared__ float rf_lds[SLAB ? 1 : 16 * MG];        // the rows' own factors: 1 / rms where the norm left it to the output
-  constexpr bool kNext = !SLAB && EPI == EPI_RESID && MG == 1;
-  __shared__ __attribute__((aligned(16))) float ga_lds[kNext ? kRegsMaxPasses * 16 : 4];   // the gains of the norm behind
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int g = lane >> 4, c = lane & 15;
   const int kper = ceil_div(KT, (int)gridDim.y), k_lo = (int)blockIdx.y * kper, k_hi = min(k_lo + kper, KT);
@@ -98,7 +97,6 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
         const int at = tile_of(i >> 4) * 16 + (i & 15);
         sc_lds[i] = e.scale[at];
         bi_lds[i] = e.bias ? e.bias[at] : 0.f;
-        if constexpr (kNext) ga_lds[i] = e.next_x ? e.next_gain[at] : 0.f;
       }
     }
     if constexpr (!kFactor) {
@@ -183,28 +181,6 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
       } else {
         const float *sc4 = sc_lds + pass * 16 + g * 4, *b4 = e.bias ? bi_lds + pass * 16 + g * 4 : nullptr, rmul = rf_lds[m];
         bool done = false;
-        if constexpr (kNext) {
-          f32x4_t r = __builtin_bit_cast(f32x4_t, epre.r);
-          asm volatile("" : "+v"(r));                 // (else the two places it comes from become one load, and the first of them memory)
-          if (pass != pre_pass) r = *reinterpret_cast<const f32x4_t*>(e.resid_in + (size_t)m * e.ld_out + n0);
-          const float4 sc = *reinterpret_cast<const float4*>(sc4);
-          s[0] *= sc.x * rmul; s[1] *= sc.y * rmul; s[2] *= sc.z * rmul; s[3] *= sc.w * rmul;
-          if (b4) {
-            const float4 b = *reinterpret_cast<const float4*>(b4);
-            s[0] += b.x; s[1] += b.y; s[2] += b.z; s[3] += b.w;
-          }
-          const float4 o = make_float4(r[0] + s[0], r[1] + s[1], r[2] + s[2], r[3] + s[3]);
-          *reinterpret_cast<float4*>(e.out_f32 + (size_t)m * e.ld_out + n0) = o;
-          if (e.next_x) {
-            const float4 ga = *reinterpret_cast<const float4*>(ga_lds + pass * 16 + g * 4);
-            *reinterpret_cast<uint2*>(e.next_x + (size_t)m * e.ld_out + n0) = make_uint2(pack_bf16x2(o.x * ga.x, o.y * ga.y), pack_bf16x2(o.z * ga.z, o.w * ga.w));
-            float ss = o.x * o.x + o.y * o.y + o.z * o.z + o.w * o.w;
-            ss += __shfl_xor(ss, 16);
-            ss += __shfl_xor(ss, 32);
-            if (g == 0) e.next_ss[m * NT + tile_of(pass)] = ss;
-          }
-          continue;
-        }
         if constexpr (kPre) {
           if (pass == pre_pass) { epilogue_pre<EPI>(e, m, n0, sc4, b4, s, epre, rmul); done = true; }
         }

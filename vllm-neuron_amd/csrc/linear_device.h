@@ -39,6 +39,20 @@ __device__ __forceinline__ void epilogue(const EpiArgs& e, int m, int n0, f32x4_
   epilogue_store<EPI>(e, m, n0, v);
 }
 
+// The residual stream's new numbers, columns n0 .. n0 + 3 of row m, and what the norm behind would make of them where it is handed on (EpiArgs::next_x).  The four lanes c, c + 16,
+// c + 32, c + 48 of a wave hold the 16 columns of a row-tile.  Only the weight-streaming kernels come here.
+__device__ __forceinline__ void put_resid(const EpiArgs& e, int m, int n0, float4 r, f32x4_t v, float4 ga) {
+  const float4 o = make_float4(r.x + v[0], r.y + v[1], r.z + v[2], r.w + v[3]);
+  *reinterpret_cast<float4*>(e.out_f32 + (size_t)m * e.ld_out + n0) = o;
+  if (e.next_x) {
+    *reinterpret_cast<uint2*>(e.next_x + (size_t)m * e.ld_out + n0) = make_uint2(pack_bf16x2(o.x * ga.x, o.y * ga.y), pack_bf16x2(o.z * ga.z, o.w * ga.w));
+    float ss = o.x * o.x + o.y * o.y + o.z * o.z + o.w * o.w;
+    ss += __shfl_xor(ss, 16);
+    ss += __shfl_xor(ss, 32);
+    if ((n0 & 15) == 0) e.next_ss[m * (e.ld_out >> 4) + (n0 >> 4)] = ss;
+  }
+}
+
 // GEMV form: the scales / biases of the row-tiles a work-group owns were copied to LDS at
 // kernel start, so the epilogue never queues a global load behind the weight stream (vmcnt
 // retires in order: a late scale load would drain the whole prefetch).
@@ -51,7 +65,10 @@ __device__ __forceinline__ void epilogue_lds(const EpiArgs& e, int m, int n0, co
     const float4 b = *reinterpret_cast<const float4*>(b4);
     v[0] += b.x; v[1] += b.y; v[2] += b.z; v[3] += b.w;
   }
-  epilogue_store<EPI>(e, m, n0, v);
+  if constexpr (EPI == EPI_RESID)
+    put_resid(e, m, n0, *reinterpret_cast<const float4*>(e.resid_in + (size_t)m * e.ld_out + n0), v, *reinterpret_cast<const float4*>((e.next_x ? e.next_gain : e.scale) + n0));
+  else
+    epilogue_store<EPI>(e, m, n0, v);
 }
 
 // four accumulators -> the results that are stored as bf16: two of a gated unit, else four
@@ -140,7 +157,7 @@ __device__ __forceinline__ void epilogue_store(const EpiArgs& e, int m, int n0, 
 // first row-tile in its prologue, so that the end of the kernel is not a chain of dependent
 // L2 round trips (position -> cos/sin -> store) behind the last weight batch.
 template <int EPI> struct EpiPre {};
-template <> struct EpiPre<EPI_RESID> { float4 r; };
+template <> struct EpiPre<EPI_RESID> { float4 r, ga; };
 template <> struct EpiPre<EPI_QKV> { float2 cs, sn; int pos, slot; };
 
 // independent loads (requested with the kernel's first operands) ...
@@ -148,6 +165,7 @@ template <int EPI>
 __device__ __forceinline__ void epi_prefetch(const EpiArgs& e, int m, int n0, EpiPre<EPI>& p) {
   if constexpr (EPI == EPI_RESID) {
     p.r = *reinterpret_cast<const float4*>(e.resid_in + (size_t)m * e.ld_out + n0);
+    p.ga = *reinterpret_cast<const float4*>((e.next_x ? e.next_gain : e.scale) + n0);
   } else if constexpr (EPI == EPI_QKV) {
     p.pos = e.pos[m];
     p.slot = e.slots[m];
@@ -179,8 +197,7 @@ __device__ __forceinline__ void epilogue_pre(const EpiArgs& e, int m, int n0, co
       v[0] += b.x; v[1] += b.y; v[2] += b.z; v[3] += b.w;
     }
     if constexpr (EPI == EPI_RESID) {
-      *reinterpret_cast<float4*>(e.out_f32 + (size_t)m * e.ld_out + n0) =
-          make_float4(p.r.x + v[0], p.r.y + v[1], p.r.z + v[2], p.r.w + v[3]);
+      put_resid(e, m, n0, p.r, v, p.ga);
     } else {
       const int qk_end = e.q_dim + e.kv_dim;
       if (n0 < qk_end) {

@@ -22,8 +22,8 @@ struct EpiArgs {
   int ld_out;
   bool far_out;        // out_f32 is host memory (launch_gemv, launch_gemv_regs, EPI_F32 and EPI_SOFTCAP: results are stored through L2, or leave in larger pieces)
   const float* resid_in;
-  // EPI_RESID, launch_gemv_regs, up to 16 rows, or null: the norm behind is left to its projection, which takes next_x[m * ld_out + n] = bf16(out next_gain[n]) and 1 / rms
-  //   from next_ss [M][N / 16], the sums of squares of out over 16 columns.  K is not split then (gemv_regs_holds)
+  // EPI_RESID, launch_gemv and launch_gemv_regs, up to 16 rows, ld_out = N, or null: the norm behind is left to its projection, which takes next_x[m * ld_out + n] = bf16(out next_gain[n]) and 1 / rms
+  //   from next_ss [M][N / 16], the sums of squares of out over 16 columns.  launch_gemv_regs does not split K then (gemv_regs_holds)
   const float* next_gain;
   uint16_t* next_x;
   float* next_ss;

@@ -95,33 +95,46 @@ int flush_pending(mi_ctx* c) {
   return launch_splitk_flush(sl, c->pend_in, c->pend_out, sl.N, c->stream);
 }
 
-// next, next_gain: the projection behind a residual one and the gain of the norm between them.  From 5 to 16 rows, where both keep K in one piece, the residual projection leaves what the
-// norm would have (its rows times the gain, a sum of squares for 16 columns) and no norm is launched: 7B int8 5 rows 1088 -> 1048 us a step of 14 layers, 7B bf16 12 rows 1740 -> 1655, 8B fp8 6 rows 1150 -> 1103, 16 rows 1350 -> 1330.
+// next, next_gain: the projection behind a residual one and the gain of the norm between them.  Up to 16 rows, where the next one keeps K in the registers (and from 5 on the residual one
+// does, too: the kernels that stream rows beside the weights took 1 - 10 % of a step longer than slices and a norm), the residual projection leaves what the norm would have: its rows times the gain
+// and a sum of squares for 16 columns.  From 5 rows on that saves a launch, up to 4 it keeps fp32 rows and gains out of the next projection, which goes to the register kernel.  Half-depth
+// models, us a step: 8B fp8 1 row 1048 -> 1014, 4 rows 1095 -> 1070, 6 rows 1150 -> 1103, 16 rows 1350 -> 1330; bf16 1 - 4 rows 0.5 - 0.8 %; 7B int8 1 row 1026 -> 985, 4 rows 1071 -> 1023,
+// 5 rows 1088 -> 1048; 7B bf16 4 rows 1562 -> 1525, 12 rows 1740 -> 1655; TinyLlama bf16 1 row 753 -> 735, fp8 700 -> 669 at 4 rows.
 int run_linear(mi_ctx* c, const Linear& L, int rows, int pro, ProArgs p, int epi, EpiArgs e, const Linear* next = nullptr, const float* next_gain = nullptr) {
   e.scale = L.scale;
   e.bias = L.bias;
   const auto handed = c->handed;
   c->handed = {};
-  const bool regs = gemv_in_regs(L.view(), rows, c->splitk_ws_bytes);
+  // whether l takes the norm in front of it from sums of squares over 16 columns
+  const auto takes = [&](const Linear& l) {
+    return rows <= 16 && l.K <= c->H && l.K <= 4096 && norm_parts_fit(l.K) && (rows <= 4 || gemv_in_regs(l.view(), rows, c->splitk_ws_bytes)) &&
+           gemv_regs_whole(l.view(), rows, c->splitk_ws_bytes);
+  };
+  const bool alone = c->collective() && c->cfg.tp_degree == 1;      // a communicator of one rank makes the additions of none
+  const bool ready = pro == PRO_NORM && handed.resid == p.resid_in && handed.gain == p.gain && handed.rows == rows && !p.partial && !p.resid_out && takes(L);
+  bool hand = epi == EPI_RESID && next && next->K == L.N && e.ld_out == L.N && takes(*next);
+  if (hand) { e.next_gain = next_gain; e.next_x = c->xn; e.next_ss = c->row_rinv; }
+  const bool regs = gemv_in_regs(L.view(), rows, c->splitk_ws_bytes) || (rows <= 4 && (ready || (alone && pro == PRO_NORM && p.partial == c->partial && handed.gain == p.gain && handed.rows == rows && takes(L))));
   if (!regs && gemv_fits(rows, L.K)) {
     if (!c->runs(MI_K_GEMV)) return MI_OK;
     if (c->pend.slab) MI_TRY(flush_pending(c));
     Scope sc(c, MI_K_GEMV);
     if (c->prof.on) c->prof.gemv_bytes += (double)L.bytes();
-    if (pro == PRO_BF16 && gemv_few_rows_in_regs(L.view(), rows, 0, false)) return launch_gemv_regs(L.view(), rows, p.x, p.ldx, epi, e, c->stream, nullptr, 0);
-    return launch_gemv(L.view(), rows, pro, p, epi, e, c->stream);
+    if (pro == PRO_BF16 && gemv_few_rows_in_regs(L.view(), rows, 0, false)) MI_TRY(launch_gemv_regs(L.view(), rows, p.x, p.ldx, epi, e, c->stream, nullptr, 0));
+    else MI_TRY(launch_gemv(L.view(), rows, pro, p, epi, e, c->stream));
+    if (hand || (alone && epi == EPI_F32 && next)) c->handed = {e.out_f32, next_gain, rows};
+    return MI_OK;
   }
   const uint16_t* x = p.x;
   int ldx = p.ldx;
   const bool a8 = rows > 32 && c->cfg.prefill_fp8_activations && gemm_a8_supported(L.view());   // (prompts' option: rows a token-generation batch can have keep bf16)
   const bool parts = regs && norm_parts_fit(L.K);
-  const auto takes_fine = [&](const Linear& l) { return rows <= 16 && l.K <= c->H && l.K <= 4096 && gemv_in_regs(l.view(), rows, c->splitk_ws_bytes) && gemv_regs_whole(l.view(), rows, c->splitk_ws_bytes); };
-  const bool fine = pro == PRO_NORM && parts && takes_fine(L);
+  const bool fine = pro == PRO_NORM && parts && takes(L);
   if (regs && pro == PRO_NORM) {
     e.row_scale = c->row_rinv;
     if (parts) { e.rs_n = (float)L.K; e.rs_eps = p.eps; e.rs_parts = fine ? L.K / 16 : kNormParts; }
   }
-  if (fine && handed.resid == p.resid_in && handed.gain == p.gain && handed.rows == rows && !p.partial && !p.resid_out) {
+  if (ready) {
     x = c->xn;
     ldx = L.K;
   } else if (pro == PRO_NORM && !c->runs(MI_K_OTHER)) {   // (class-masked replay: what the norm would have left)
@@ -162,11 +175,11 @@ int run_linear(mi_ctx* c, const Linear& L, int rows, int pro, ProArgs p, int epi
   // (at every length: with the slabs' requests in flight together the sum inside the norm costs less than a launch of its own; prompts of 70 tokens of
   //  the 8B model in fp8 2077 -> 2036 us, 242 tokens 3114 -> 3062, 300 tokens of TinyLlama 2602 -> 2520)
   static const int fuse_min_rows = [] { const char* v = getenv("MI355X_FUSE_SPLITK_MIN_ROWS"); return v ? atoi(v) : 0; }();
-  const bool hand = regs && epi == EPI_RESID && next && next->K == L.N && e.ld_out == L.N && norm_parts_fit(next->K) && gemv_regs_holds(L.view()) && takes_fine(*next);
-  if (hand) { e.next_gain = next_gain; e.next_x = c->xn; e.next_ss = c->row_rinv; }
+  if (hand && !gemv_regs_holds(L.view())) { hand = false; e.next_x = nullptr; }
   SlabSum* defer = (fuse && !hand && epi == EPI_RESID && rows >= fuse_min_rows && !c->pend.slab) ? &c->pend : nullptr;
-  // (a communicator of one rank makes the additions of no communicator; a shard's K is another anyway, and its sum is a launch of its own in front of the exchange)
-  const bool as_deferred = fuse && c->collective() && c->cfg.tp_degree == 1 && epi == EPI_F32 && rows >= fuse_min_rows && &L != &c->lm_head;
+  // (a shard's K is another anyway, and its sum is a launch of its own in front of the exchange)
+  const bool as_deferred = fuse && alone && epi == EPI_F32 && rows >= fuse_min_rows && &L != &c->lm_head;
+  const bool as_handed = as_deferred && next && takes(*next) && gemv_regs_holds(L.view());
   auto note_deferred = [&]() {
     if (defer && c->pend.slab) { c->pend_in = e.resid_in; c->pend_out = e.out_f32; }
   };
@@ -177,7 +190,7 @@ int run_linear(mi_ctx* c, const Linear& L, int rows, int pro, ProArgs p, int epi
     if (!e.far_out && ldx % 8 == 0 && gemm_wide_few_rows(L.view(), rows, c->splitk_ws_bytes, defer || as_deferred))
       MI_TRY(launch_gemm_wide(L.view(), rows, x, ldx, epi, e, c->stream, c->splitk_ws, c->splitk_ws_bytes, defer, as_deferred));
     else
-      MI_TRY(launch_gemv_regs(L.view(), rows, x, ldx, epi, e, c->stream, c->splitk_ws, c->splitk_ws_bytes, defer, as_deferred));
+      MI_TRY(launch_gemv_regs(L.view(), rows, x, ldx, epi, e, c->stream, as_handed ? nullptr : c->splitk_ws, c->splitk_ws_bytes, defer, as_deferred));
     if (hand) c->handed = {e.out_f32, next_gain, rows};
     note_deferred();
     return MI_OK;
@@ -350,7 +363,7 @@ int run_trunk(mi_ctx* c, int rows, bool decode, int B, int MB, int q_pos0, const
       e.ld_out = c->H;
       if (tp) {
         e.out_f32 = c->partial;
-        MI_TRY(run_linear(c, W.o, rows, PRO_BF16, p, EPI_F32, e));
+        MI_TRY(run_linear(c, W.o, rows, PRO_BF16, p, EPI_F32, e, &W.gu, W.g_post));
         MI_TRY(all_reduce_partial(c, rows));
       } else {
         e.out_f32 = c->resid[cur ^ 1]; e.resid_in = c->resid[cur];
@@ -370,19 +383,21 @@ int run_trunk(mi_ctx* c, int rows, bool decode, int B, int MB, int q_pos0, const
       if (tp) cur ^= 1;
     }
     {  // down projection
+      const bool last = l + 1 == k.num_layers;
+      const Linear* next = last ? &c->lm_head : &c->layers[l + 1].qkv;
+      const float* next_gain = last ? c->g_final : c->layers[l + 1].g_in;
       ProArgs p{};
       p.x = c->act; p.ldx = c->I_l;
       EpiArgs e{};
       e.ld_out = c->H;
       if (tp) {
         e.out_f32 = c->partial;
-        MI_TRY(run_linear(c, W.down, rows, PRO_BF16, p, EPI_F32, e));
+        MI_TRY(run_linear(c, W.down, rows, PRO_BF16, p, EPI_F32, e, next, next_gain));
         MI_TRY(all_reduce_partial(c, rows));
         have_partial = true;
       } else {
         e.out_f32 = c->resid[cur ^ 1]; e.resid_in = c->resid[cur];
-        const bool last = l + 1 == k.num_layers;
-        MI_TRY(run_linear(c, W.down, rows, PRO_BF16, p, EPI_RESID, e, last ? &c->lm_head : &c->layers[l + 1].qkv, last ? c->g_final : c->layers[l + 1].g_in));
+        MI_TRY(run_linear(c, W.down, rows, PRO_BF16, p, EPI_RESID, e, next, next_gain));
         cur ^= 1;
       }
     }
