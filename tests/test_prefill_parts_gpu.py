@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
     (4, 1, 64, 1, 0), (4, 1, 128, 1, 63), (4, 1, 128, 1, 64), (3, 1, 64, 33, 95), (3, 1, 128, 64, 64), (4, 1, 64, 65, 127), (8, 2, 128, 31, 321), (3, 1, 64, 129, 256),
     (5, 1, 128, 33, 40), (6, 1, 64, 70, 0), (7, 1, 128, 129, 130), (8, 1, 64, 65, 63), (14, 2, 64, 200, 300), (28, 4, 128, 1061, 0), (32, 4, 64, 1030, 31), (20, 4, 128, 1025, 0),
     (32, 8, 128, 1023, 0), (32, 8, 64, 1030, 0), (24, 8, 128, 1057, 70), (4, 1, 128, 33, 64), (3, 1, 64, 32, 64), (4, 1, 64, 33, 63),
-    (40, 8, 64, 1200, 0), (32, 8, 128, 1057, 2000)])      # (the last two: one wave a head, where two would be a second round, and behind a long prefix)
+    (40, 8, 64, 1200, 0), (32, 8, 128, 1057, 2000),       # (these two: one wave a head, where two would be a second round, and behind a long prefix)
+    (32, 8, 128, 512, 0), (32, 8, 64, 513, 0), (24, 4, 128, 512, 5), (20, 4, 64, 513, 0), (5, 1, 64, 97, 0)])      # two heads to a work-group up to 512 tokens here; a third (two) of the groups empty
 def test_two_waves_a_head(lib, nh, nkv, hd, T, pos0):  # noqa: F811
     bs, kv_len = 16, pos0 + T
     MB = -(-kv_len // bs) + 1

@@ -777,8 +777,8 @@ __device__ __forceinline__ void attn_prefill2_body(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int QB = KH == 1 ? NW / Gp : 1;
   const int hl = wave % Gp, slot = KH == 1 ? wave / Gp : 0, part = KH == 1 ? 0 : wave / Gp;
-  const int per = subs == 2 ? (G + 1) >> 1 : G, h0 = subs == 2 ? sub * per : 0, hn = min(per, G - h0);      // this work-group's heads of the kv head's
-  const int head = kvh * G + h0 + min(hl, hn - 1);
+  const int per = ceil_div(G, subs), h0 = min(sub * per, G - 1), hn = min(per, G - sub * per);      // this work-group's heads of the kv head's (hn <= 0: none)
+  const int head = kvh * G + h0 + max(min(hl, hn - 1), 0);
   const bool head_ok = hl < hn;
   const int kv_len = q_pos0 + T;
   const int last_piece_key = ((kv_len - 1) / KPP) * KPP;
@@ -1086,13 +1086,13 @@ template <int HD, int NW, int KH>
 constexpr int attn_prefill2_lds() { return std::max((KH == 1 ? 3 : 2) * KH * 2 * 64 * 2 * HD, KH == 1 ? 0 : NW * (HD / 64 * 4096 + 512)); }
 // The kv heads are the fastest of the grid: with 8 (4) of them an XCD's work-groups read the keys of one, and the heavy blocks of all start first.
 template <int HD, int NW, int KH>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4, NW / 4))) void attn_prefill2_kernel(
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill2_kernel(
     const uint16_t* __restrict__ q, int T, int q_pos0, const uint16_t* __restrict__ kpool,
     const uint16_t* __restrict__ vpool, int bs, int bs_shift, const int32_t* __restrict__ block_table, int nh, int nkv,
     int G, int Gp, int subs, int nblk, int paired, float* __restrict__ o_part, float* __restrict__ ml_part, uint16_t* __restrict__ out, float scale_log2e) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int two = KH > 1 && subs == 2, kvh = two ? blockIdx.x >> 1 : blockIdx.x;
-  attn_prefill2_body<HD, NW, KH>(smem, blockIdx.y, kvh, two ? blockIdx.x & 1 : 0, two ? 2 : 1, blockIdx.z, gridDim.z, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk, paired, o_part,
+  const int parts = KH > 1 ? subs : 1, kvh = (int)blockIdx.x / parts;
+  attn_prefill2_body<HD, NW, KH>(smem, blockIdx.y, kvh, (int)blockIdx.x - kvh * parts, parts, blockIdx.z, gridDim.z, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk, paired, o_part,
                              ml_part, out, scale_log2e);
 }
 
@@ -1108,7 +1108,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   if ((int)blockIdx.x >= d.nd) {
     const int x = (int)blockIdx.x - d.nd;
-    const int two = KH > 1 && subs == 2, y = two ? x >> 1 : x;
+    const int two = KH > 1 && subs == 2, y = two ? x >> 1 : x;      // (four sub-groups: not here)
     attn_prefill2_body<HD, 8, KH>(smem, y % gx, blockIdx.y, two ? x & 1 : 0, two ? 2 : 1, y / gx, ns, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk,
                               paired, o_part, ml_part, out, scale_log2e);
   } else {
@@ -1153,7 +1153,7 @@ static bool attn_prefill_v1() {   // MI355X_ATTN_PREFILL_V1=1: the first-generat
 }
 
 static int prefill_heads(int G) { return G <= 1 ? 1 : (G <= 2 ? 2 : (G <= 4 ? 4 : 8)); }
-struct PrefillPlan { int Gp, kh, subs, nblk, bs_shift, paired, gx, ns; float *o_part = nullptr, *ml_part = nullptr; };
+struct PrefillPlan { int Gp, kh, nw, subs, nblk, bs_shift, paired, gx, ns; float *o_part = nullptr, *ml_part = nullptr; };
 // Where one wave a head takes less time, from 3 heads on a kv head on.  By two waves each, 5 to 8 heads are two work-groups, and 3 and 4 leave the second block of a pair to a second pass:
 // behind a long prefix, or in another round of work-groups, that can cost more than the waves save.  Tiles that a work-group walks, of its block or of a pair of blocks one after the other,
 // times the rounds (single waves of 3 and 4 heads: pairs side by side, the heavy ones first, so a later round is half as long); a step of two tiles by two waves takes 1.1 of a tile by one, where
@@ -1168,7 +1168,7 @@ static bool prefill_one_wave(int heads, int T, int q_pos0, int nkv, int hd, int 
   if (heads == 8) return walk(1) < 1.1 * walk(2);
   return hd == 128 && ceil_div(kv, 64) + (ceil_div(npair * nkv, num_cu) - 1) * ceil_div(q_pos0 + T / 2, 64) < 1.4 * walk(2);
 }
-static PrefillPlan prefill_plan(int T, int q_pos0, int block_size, int nh, int nkv, int hd, float* ws, size_t ws_bytes, int num_cu) {
+static PrefillPlan prefill_plan(int T, int q_pos0, int block_size, int nh, int nkv, int hd, float* ws, size_t ws_bytes, int num_cu, bool mixed = false) {
   // second generation: 8 waves = (8 / Gp) query blocks x Gp heads, blocks in complementary pairs; or, from 3 heads on a kv head on, a block of up to 4 heads, two waves each
   PrefillPlan p;
   p.Gp = prefill_heads(nh / nkv);
@@ -1176,6 +1176,7 @@ static PrefillPlan prefill_plan(int T, int q_pos0, int block_size, int nh, int n
   p.kh = p.Gp >= 4 && q_pos0 + T > 96 && !prefill_one_wave(p.Gp, T, q_pos0, nkv, hd, num_cu) ? 2 : 1;
   p.subs = p.kh == 2 && p.Gp == 8 ? 2 : 1;
   if (p.subs == 2) p.Gp = 4;
+  p.nw = 8;
   const int groups = nkv * p.subs;             // of heads: work-groups that read the same queries' keys
   const int nblk = ceil_div(T, 32), npair = (nblk + 1) / 2, qb = p.kh == 2 ? 1 : 8 / p.Gp;
   int bs_shift = -1;
@@ -1196,6 +1197,15 @@ static PrefillPlan prefill_plan(int T, int q_pos0, int block_size, int nh, int n
     if (ceil_div(steps, z) * p.kh < 2 || part * (hd + 2) * sizeof(float) > ws_bytes) break;
     const double cost = per_step * ceil_div(steps, z) * ceil_div(gx * groups * z, num_cu) + (p.kh == 2 && hd == 128 ? 6.0 : 4.5) + (double)part * hd * 8.0 / 4e6;
     if (cost < best) { best = cost; ns = z; }
+  }
+  // Where twice the work-groups find a CU each: two heads to a work-group of four waves.  A wave then has its SIMD to itself, and a work-group half the results to put together: some 1 us less and 0.2 a
+  // step.  us a call: 7B int8 188 behind 512 tokens 2276 -> 2253, 300 tokens 3301 -> 3272, 8B fp8 100 1938 -> 1911, 400 3717 -> 3679, TinyLlama 300 1711 -> 1686, bf16 100 behind 800 1653 -> 1629.  Not in
+  // place of slices: 8B 136 tokens behind 864 2287 in slices, 2325 in fewer slices of these; 236 behind 1664 2758 and 2800.
+  if (!mixed && p.kh == 2 && nblk * groups * 2 <= num_cu && (per_step - 0.2) * steps - 1.0 < best) {
+    p.nw = 4;
+    p.Gp = 2;
+    p.subs *= 2;
+    ns = 1;
   }
   p.nblk = nblk; p.bs_shift = bs_shift; p.paired = paired; p.gx = gx; p.ns = ns;
   if (ns > 1) { p.o_part = ws; p.ml_part = ws + (size_t)ns * T * nh * hd; }
@@ -1229,6 +1239,7 @@ int launch_attn_prefill(const uint16_t* q, int T, int q_pos0, const uint16_t* kp
                          block_table, nh, nkv, G, p.Gp, p.subs, p.nblk, p.paired, p.o_part, p.ml_part, out, scale_log2e); \
     } while (0)
     if (p.kh == 1) { if (hd == 128) MI_P2(128, 8, 1); else MI_P2(64, 8, 1); }
+    else if (p.nw == 4) { if (hd == 128) MI_P2(128, 4, 2); else MI_P2(64, 4, 2); }
     else { if (hd == 128) MI_P2(128, 8, 2); else MI_P2(64, 8, 2); }
 #undef MI_P2
     launch_prefill_combine(p, T, nh, hd, out, s);
@@ -1281,7 +1292,7 @@ int launch_attn_mixed(const AttnMixed& m, int T, int q_pos0, const uint16_t* q, 
   // 239 + 3 tokens 3105 -> 2980, 64 + 6 2205 -> 2108, TinyLlama 300 + 4 2385 -> 2245, 8B bf16 500 + 6 4862 -> 4724; 1900 + 3 13035 -> 13097).
   int num_cu = 0;
   MI_TRY_A(device_num_cu(&num_cu));
-  const PrefillPlan p = prefill_plan(T, q_pos0, block_size, nh, nkv, hd, ws, ws_bytes, num_cu);
+  const PrefillPlan p = prefill_plan(T, q_pos0, block_size, nh, nkv, hd, ws, ws_bytes, num_cu, true);
   if (attn_prefill_v1() || (p.gx * p.ns * p.subs + mixed_splits(m, nkv, hd) * m.B) * nkv > num_cu) {
     int rc = launch_attn_decode(m.q, kpool, vpool, block_size, m.block_table, m.MB, m.ctx_lens, m.B, nh, nkv, hd, m.out, m.scratch, s, false, 1, m.num_blocks, m.max_ctx);
     return rc != MI_OK ? rc : launch_attn_prefill(q, T, q_pos0, kpool, vpool, block_size, block_table, nh, nkv, hd, out, s, ws, ws_bytes);
