@@ -761,7 +761,8 @@ int launch_sandwich_rows(const float* resid_in, float* resid_out, const RowSourc
     if (rc != MI_OK) return rc;
     cs = *conv;
   }
-  if (T <= 32 && (w_pre || as_is) && ld <= 4096 && ld == D && (D / groups) % 256 == 0 && (!conv || conv->taps <= 4)) {
+  // (rows of prompts too, where no convolution's state rides along: the general kernel waits for memory twice and more.  us a call: Bokulorn 2048 tokens 2166 -> 2150, Nusovik 777 2157 -> 2151)
+  if ((T <= 32 || !conv) && (w_pre || as_is) && ld <= 4096 && ld == D && (D / groups) % 256 == 0 && (!conv || conv->taps <= 4)) {
     const int gs = D / groups;      // (one wave and more)
 #define MI_TOKEN(TAPS) \
     if (f32) hipLaunchKernelGGL((sandwich_token_kernel<float, TAPS>), dim3(T, groups), dim3(gs / 4), 0, s, resid_in, resid_out, src, w_post, w_pre, D, ld, gs, eps, cs, (float*)y, ldy); \
