@@ -60,7 +60,12 @@ __device__ __forceinline__ void wide_slice(int K, int& ks0, int& nks) {
 // Slabs are written through while they fit the eight L2s (4 MiB each) with room for the rows and weights that come in beside them: left there, they go out when the kernel
 // ends, and the norm behind waits.  us a launch, left -> through: 8 slabs of 188 x 3584 (21.6 MB) 34.3 -> 32.8, 4 of 242 x 4096 (15.9 MB) 31.7 -> 30.2, 3 of 188 x 4608 15.0 -> 14.0, 8 of
 // 32 x 4096 8.7 -> 7.5.  Larger ones mostly leave on the way, and pieces of 64 bytes cost more than lines: 2 of 1000 x 4096 (32.8 MB) 107.3 -> 107.9, 2 of 2031 x 4096 181 -> 185.
+// Nor where the weights are more than four times the slabs and keep the memory busy to the end: bf16 14336 x 2048, 100 tokens 19.6 -> 20.8, 3584 x 4608 14.7 -> 15.7, fp8 14336 x 4096, 60 tokens
+// 17.7 -> 18.2, 100 (4.5 times) 25.5 -> 25.6; 8B bf16, 60 tokens 2127 -> 2155 a call.
 constexpr size_t kSlabThroughBytes = (size_t)24 << 20;
+__device__ __forceinline__ bool slab_through(int slices, int T, int NT, int K, int weight_bytes) {
+  return (size_t)slices * T * NT * 64 <= kSlabThroughBytes && (size_t)K * weight_bytes <= (size_t)16 * slices * T;
+}
 // a wave's raw accumulators to its K-slice's slab [T][16 NT]
 template <int NTW, int MT>
 __device__ __forceinline__ void store_slab(float* __restrict__ slab, bool through, int T, int NT, int mb, int nb, int g, int c, const f32x4_t (&acc)[NTW][MT]) {
@@ -241,7 +246,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
   for (; ks + kStages - 1 < nks; ++ks) step(ks, std::true_type());
   for (; ks < nks; ++ks) step(ks, std::false_type());
   if (grp == 0) __builtin_amdgcn_s_barrier();   // the barrier group 1 executed first
-  if constexpr (SPLIT) store_slab<NTW, MT>(slab + (size_t)blockIdx.z * T * (NT * 16), (size_t)gridDim.z * T * NT * 64 <= kSlabThroughBytes, T, NT, m0 + wm * (BM / 2), ntb + wn * NTW, g, c, acc);
+  if constexpr (SPLIT) store_slab<NTW, MT>(slab + (size_t)blockIdx.z * T * (NT * 16), slab_through(gridDim.z, T, NT, K, WD == MI_W_BF16 ? 2 : 1), T, NT, m0 + wm * (BM / 2), ntb + wn * NTW, g, c, acc);
   else epilogue_tile<EPI, NTW, MT>(e, T, NT, m0 + wm * (BM / 2), ntb + wn * NTW, g, c, acc);
 }
 
@@ -373,7 +378,7 @@ __global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restric
   for (; s + 4 < n; s += 2) pair(s, std::true_type());      // both request, and two K-steps' DMAs are behind what they wait for
   for (; s < n; s += 2) pair(s, std::false_type());
   if (grp == 0) __builtin_amdgcn_s_barrier();   // the barrier group 1 executed first
-  if constexpr (SPLIT) store_slab<NTW, MT>(slab + (size_t)blockIdx.z * T * (NT * 16), (size_t)gridDim.z * T * NT * 64 <= kSlabThroughBytes, T, NT, m0 + wm * (BM / 2), ntb + wn * NTW, g, c, acc);
+  if constexpr (SPLIT) store_slab<NTW, MT>(slab + (size_t)blockIdx.z * T * (NT * 16), slab_through(gridDim.z, T, NT, K, 2), T, NT, m0 + wm * (BM / 2), ntb + wn * NTW, g, c, acc);
   else epilogue_tile<EPI, NTW, MT>(e, T, NT, m0 + wm * (BM / 2), ntb + wn * NTW, g, c, acc);
 }
 
