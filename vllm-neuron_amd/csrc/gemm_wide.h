@@ -37,24 +37,51 @@ __device__ __forceinline__ void wait_dma(int left) {
   else if constexpr (MOST > 0) wait_dma<PER, MOST - 1>(left);
 }
 
+// What a work-group needs in front of its first request, in one line of kernel arguments and taken in one go (wide_args): a kernel's arguments come from memory, and hipcc fetches
+// each where it is first used.  Divisions are the host's.  (A work-group took 1.6 - 3.1 us to the
+// last request of its ring.)  us a launch, before -> now: int8 188 x 4608 in 3 slices 14.2 -> 13.6, x 3584 in 4 12.1 -> 11.6, 18944 deep in 8 33.0 -> 32.4; calls of 32 .. 1000 tokens 0.8 - 1.3 %.
+struct WideArgs {
+  const uint4* W;
+  const uint16_t* x;
+  float* slab;
+  int NT, KT, T, K, ldx;
+  int mtiles, per;           // token blocks; tiles of an XCD
+  unsigned by_mtiles;        // 2^32 / mtiles, rounded down
+  int kper;                  // K-steps of a slice
+};
+static_assert(sizeof(WideArgs) <= 64, "a line");
+__device__ __forceinline__ void wide_args(const WideArgs& a) {
+  asm volatile("" ::"s"(a.W), "s"(a.x), "s"(a.slab), "s"(a.NT), "s"(a.KT), "s"(a.T), "s"(a.K), "s"(a.ldx), "s"(a.mtiles), "s"(a.per), "s"(a.by_mtiles), "s"(a.kper));
+}
+// ... and what its epilogue needs, asked for behind those requests
+template <int EPI, bool SPLIT>
+__device__ __forceinline__ void wide_epi_args(const EpiArgs& e) {
+  if constexpr (SPLIT) return;
+  asm volatile("" ::"s"(e.scale), "s"(e.bias), "s"(e.row_scale));
+  if constexpr (EPI == EPI_F32 || EPI == EPI_RESID || EPI == EPI_SOFTCAP) asm volatile("" ::"s"(e.out_f32), "s"(e.ld_out));
+  if constexpr (EPI == EPI_RESID) asm volatile("" ::"s"(e.resid_in));
+  if constexpr (EPI == EPI_SWIGLU || EPI == EPI_GLU_CLIP || EPI == EPI_RELU2) asm volatile("" ::"s"(e.act_out), "s"(e.ld_act));
+  if constexpr (EPI == EPI_QKV) asm volatile("" ::"s"(e.q_out), "s"(e.q_dim), "s"(e.kv_dim), "s"(e.hd), "s"(e.nkv), "s"(e.pos), "s"(e.slots), "s"(e.rope_cos), "s"(e.rope_sin), "s"(e.kpool), "s"(e.vpool), "s"(e.block_size));
+}
 // The tile of this work-group.  Work-group b runs on XCD b % 8: an XCD takes an eighth of the tiles, one after the other with the token
 // blocks of a weight slab in a row, so that a slab comes into its L2 once.  (Every eighth slab to an XCD, as in gemm_kernel, left the XCDs
 // up to a slab apart: 44 slabs of 11 token blocks put 66 work-groups on the 32 CUs of four of them, three rounds in place of two.)
 template <int BM, int NTW>
-__device__ __forceinline__ bool wide_tile(int T, int NT, int& m0, int& nt0) {
-  const int mtiles = ceil_div(T, BM), tiles = mtiles * ceil_div(NT, 4 * NTW), per = ceil_div(tiles, 8);
-  const int seq = blockIdx.x >> 3, t = (blockIdx.x & 7) * per + seq;
-  if (seq >= per || t >= tiles) return false;
-  nt0 = t / mtiles * (4 * NTW);
-  m0 = t % mtiles * BM;
+__device__ __forceinline__ bool wide_tile(const WideArgs& a, int& m0, int& nt0) {
+  const unsigned seq = blockIdx.x >> 3, t = (blockIdx.x & 7) * a.per + seq;
+  if (seq >= (unsigned)a.per || t >= (unsigned)(a.mtiles * ceil_div(a.NT, 4 * NTW))) return false;
+  unsigned q = __umulhi(t, a.by_mtiles);     // t / mtiles, or one less
+  if (t - q * a.mtiles >= (unsigned)a.mtiles) ++q;
+  nt0 = (int)q * (4 * NTW);
+  m0 = (int)(t - q * a.mtiles) * BM;
   return true;
 }
 // the K-steps of grid.z slice blockIdx.z: equal ones, the last may be shorter (the launch leaves none empty)
 template <bool SPLIT, int KD = 1>
-__device__ __forceinline__ void wide_slice(int K, int& ks0, int& nks) {
-  const int all = K / (64 * KD), per = SPLIT ? ceil_div(all, (int)gridDim.z) : all;
-  ks0 = SPLIT ? (int)blockIdx.z * per : 0;
-  nks = min(per, all - ks0);
+__device__ __forceinline__ void wide_slice(const WideArgs& a, int& ks0, int& nks) {
+  const int all = a.K / (64 * KD);
+  ks0 = SPLIT ? (int)blockIdx.z * a.kper : 0;
+  nks = SPLIT ? min(a.kper, all - ks0) : all;
 }
 
 // Slabs are written through while they fit the eight L2s (4 MiB each) with room for the rows and weights that come in beside them: left there, they go out when the kernel
@@ -67,19 +94,23 @@ __device__ __forceinline__ bool slab_through(int slices, int T, int NT, int K, i
   return (size_t)slices * T * NT * 64 <= kSlabThroughBytes && (size_t)K * weight_bytes <= (size_t)16 * slices * T;
 }
 // a wave's raw accumulators to its K-slice's slab [T][16 NT]
+// (One branch for all, and rows behind the last dropped by the descriptor: this code runs once a launch and is fetched from
+// memory then.)
 template <int NTW, int MT>
 __device__ __forceinline__ void store_slab(float* __restrict__ slab, bool through, int T, int NT, int mb, int nb, int g, int c, const f32x4_t (&acc)[NTW][MT]) {
+  const auto r = __builtin_amdgcn_make_buffer_rsrc(slab, 0, (uint32_t)T * NT * 64u, 0x00020000);
+  const uint32_t at = ((uint32_t)(mb + c) * NT + nb) * 64u + g * 16u;
+  const auto put = [&](auto aux) {
 #pragma unroll
-  for (int i = 0; i < NTW; ++i) {
-    if (nb + i >= NT) continue;
+    for (int i = 0; i < NTW; ++i) {
+      if (nb + i >= NT) break;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int m = mb + mt * 16 + c;
-      if (m >= T) continue;
-      if (through) store_through(slab, ((uint32_t)m * NT * 16 + (nb + i) * 16 + g * 4) * 4, acc[i][mt]);
-      else *reinterpret_cast<f32x4_t*>(slab + (size_t)m * (NT * 16) + (nb + i) * 16 + g * 4) = acc[i][mt];
+      for (int mt = 0; mt < MT; ++mt)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[i][mt]), r, at + (uint32_t)mt * NT * 1024u + i * 64u, 0, decltype(aux)::value);
     }
-  }
+  };
+  if (through) put(std::integral_constant<int, 16>());
+  else put(std::integral_constant<int, 0>());
 }
 
 // KD 64-deep parts to a K-step.  A phase (READ or MULTIPLY) costs some 340 cycles of barrier, LDS latency and requests even without its MFMAs; in the smallest tiles
@@ -90,9 +121,12 @@ __device__ __forceinline__ void store_slab(float* __restrict__ slab, bool throug
 // with the decoded fragments of one K-step).
 // SPLIT: grid.z K-slices write raw fp32 accumulators to slab[z][m][n] (see gemm_a8_kernel).
 template <int WD, int EPI, int BM, int NTW, bool SPLIT, int KD>
-__global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict__ W, int NT, int KT, int T, int K,
-                                                        const uint16_t* __restrict__ x, int ldx, EpiArgs e,
-                                                        float* __restrict__ slab) {
+__global__ __launch_bounds__(512) void gemm_wide_kernel(WideArgs a, EpiArgs e) {
+  wide_args(a);
+  const uint4* __restrict__ W = a.W;
+  const uint16_t* __restrict__ x = a.x;
+  float* __restrict__ slab = a.slab;
+  const int NT = a.NT, KT = a.KT, T = a.T, K = a.K, ldx = a.ldx;
   constexpr int kW = KD * kWideWBytes<WD, NTW>, kStage = kW + KD * BM * 128, kStages = kWideStages<WD, BM, NTW, KD>;
   static_assert(kStages >= 3, "the two wave groups need three stages");
   // waves as 2 (tokens) x 4 (weight rows), each MT 16-token tiles x NTW 16-row weight tiles (4 x 2 waves would read 16 instead of 20 KiB of
@@ -108,9 +142,9 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
   const int g = lane >> 4, c = lane & 15;
   const int wm = wave % WM, wn = wave / WM;
   int m0, ntb;
-  if (!wide_tile<BM, NTW>(T, NT, m0, ntb)) return;
+  if (!wide_tile<BM, NTW>(a, m0, ntb)) return;
   int ks0, nks;                               // this slice's K-steps, from K-step ks0 on
-  wide_slice<SPLIT, KD>(K, ks0, nks);
+  wide_slice<SPLIT, KD>(a, ks0, nks);
 
   // this lane's DMA sources: weight tiles wt0 .. (fragment order) and X0 (group 1: X1) 8-row pieces of each 64-deep part of the activation tile
   const int grp = __builtin_amdgcn_readfirstlane(wave >> 2), wt0 = grp == 0 ? WP0 * wave : 4 * WP0 + WP1 * (wave - 4);
@@ -167,6 +201,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
 #pragma unroll
   for (int k = 0; k + 1 < kStages; ++k)
     if (k < nks) issue(k, k);
+  wide_epi_args<EPI, SPLIT>(e);
   if (grp == 1) {   // its pieces of stage 0 are in before P0
     wait_dma<kDma1, kStages - 2>(nks - 1);
     __builtin_amdgcn_s_barrier();           // P0
@@ -258,9 +293,12 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const uint4* __restrict_
 // us a 64-deep K-step on a full chip: 256 x 256 1.46, the other two 1.2; 128 x 256 by 64 0.83.  12288 x 2048 at 777 tokens: 192 work-groups of 256 x 256 54.8,
 // 256 of 256 x 192 48.1, 240 of 192 x 256 46.0.
 template <int EPI, int BM, int NTW, bool SPLIT>
-__global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restrict__ W, int NT, int KT, int T, int K,
-                                                          const uint16_t* __restrict__ x, int ldx, EpiArgs e,
-                                                          float* __restrict__ slab) {
+__global__ __launch_bounds__(512) void gemm_wide16_kernel(WideArgs a, EpiArgs e) {
+  wide_args(a);
+  const uint4* __restrict__ W = a.W;
+  const uint16_t* __restrict__ x = a.x;
+  float* __restrict__ slab = a.slab;
+  const int NT = a.NT, KT = a.KT, T = a.T, K = a.K, ldx = a.ldx;
   constexpr int MT = BM / 32, WM = 2, kW = NTW * 4096, kX = BM * 128, kXs = 4 * kW;
   constexpr int XP = BM / 64, XH0 = (XP + 1) / 2, XH1 = XP - XH0;     // 8-row activation pieces per wave and pair, those of its first and its second K-step
   constexpr int WP0 = (NTW + 1) / 2, WP1 = NTW - WP0;                 // weight tiles per wave and K-step: waves 0-3, waves 4-7
@@ -270,9 +308,9 @@ __global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restric
   const int g = lane >> 4, c = lane & 15;
   const int wm = wave % WM, wn = wave / WM;
   int m0, ntb;
-  if (!wide_tile<BM, NTW>(T, NT, m0, ntb)) return;
+  if (!wide_tile<BM, NTW>(a, m0, ntb)) return;
   int ks0, nks;
-  wide_slice<SPLIT>(K, ks0, nks);
+  wide_slice<SPLIT>(a, ks0, nks);
   const int s0 = 2 * ks0, n = 2 * nks;        // this slice's 32-deep K-steps
 
   const int grp = __builtin_amdgcn_readfirstlane(wave >> 2), wt0 = grp == 0 ? WP0 * wave : 4 * WP0 + WP1 * (wave - 4);
@@ -326,6 +364,7 @@ __global__ __launch_bounds__(512) void gemm_wide16_kernel(const uint4* __restric
     issue_w(2);
     issue_x(1, Second(), 1);
   }
+  wide_epi_args<EPI, SPLIT>(e);
   if (grp == 1) {
     wait_at(0, Tiles1());
     __builtin_amdgcn_s_barrier();           // P0
@@ -389,20 +428,22 @@ constexpr bool wide_tile_by_32(int wd, int bm, int ntw) { return wd == MI_W_BF16
 
 template <int WD, int EPI, int BM, int NTW, bool SPLIT>
 static int launch_gemm_wide_t(const LinearW& w, int T, const uint16_t* x, int ldx, const EpiArgs& e, hipStream_t s, int KS, float* slab) {
-  const int NT = w.N / 16, KT = w.K / tile_k(WD);
-  const dim3 grid(8 * ceil_div(ceil_div(T, BM) * ceil_div(NT, 4 * NTW), 8), 1, KS);
-  const uint4* W = reinterpret_cast<const uint4*>(w.w);
+  const int NT = w.N / 16, mtiles = ceil_div(T, BM), per = ceil_div(mtiles * ceil_div(NT, 4 * NTW), 8);
+  const dim3 grid(8 * per, 1, KS);
+  WideArgs a{reinterpret_cast<const uint4*>(w.w), x, slab, NT, w.K / tile_k(WD), T, w.K, ldx, mtiles, per, mtiles == 1 ? ~0u : (unsigned)((1ull << 32) / mtiles), 0};
   if constexpr (wide_tile_by_32(WD, BM, NTW)) {
     constexpr int lds = 4 * NTW * 4096 + 3 * BM * 128;
     const auto fn = gemm_wide16_kernel<EPI, BM, NTW, SPLIT>;
     MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds));
-    hipLaunchKernelGGL(fn, grid, dim3(512), lds, s, W, NT, KT, T, w.K, x, ldx, e, slab);
+    a.kper = ceil_div(w.K / 64, KS);
+    hipLaunchKernelGGL(fn, grid, dim3(512), lds, s, a, e);
   } else {
     const auto launch = [&](auto deep) {
       constexpr int KD = decltype(deep)::value, lds = kWideStages<WD, BM, NTW, KD> * KD * (kWideWBytes<WD, NTW> + BM * 128);
       const auto fn = gemm_wide_kernel<WD, EPI, BM, NTW, SPLIT, KD>;
       MI_TRY_(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds));
-      hipLaunchKernelGGL(fn, grid, dim3(512), lds, s, W, NT, KT, T, w.K, x, ldx, e, slab);
+      a.kper = ceil_div(w.K / (64 * KD), KS);
+      hipLaunchKernelGGL(fn, grid, dim3(512), lds, s, a, e);
       return (int)MI_OK;
     };
     // 128-deep K-steps where a phase would be shorter than its reads: weights of a byte in the smallest tiles, if no slice of K stays empty by them
