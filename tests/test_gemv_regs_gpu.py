@@ -178,13 +178,63 @@ def test_logits_of_many_rows_to_the_host(vocab):
         model.load_state_dict(w)
         model.finalize()
         out = {}
-        for rows in (16, 17, 32):      # (16 rows: single row-tiles)
+        for rows in (16, 17, 32):
             for _ in range(2):         # eager pass, then the graph
                 out[rows] = model.forward(**decode_inputs([i % vocab for i in range(rows)], [0] * rows, [[1 + i] for i in range(rows)], 32, 32)).clone()
         # the same sums over K a row-tile, whoever stores them; the projections in front differ in low bits between 16 and 17 rows, as between any two kernels
         std = out[32].std().item()
         assert torch.isfinite(out[32]).all() and torch.equal(out[17], out[32][:17]) and (out[16] - out[32][:16]).abs().max().item() < 0.05 * std
         model.close()
+
+
+# logits of 5 to 16 rows to the host, four row-tiles side by side from 8192 rows on: a last group of four, one, two and three.  The bar is that of the test above: the rows' first
+# 4 come from another kernel, and a row is the same however many stand beside it
+@pytest.mark.parametrize("vocab", [8176, 8192, 8208, 8224, 12272])
+def test_logits_of_few_rows_to_the_host(vocab):
+    from oracle import DecoderConfig
+    from oracle.synth import make_weights
+    from tests.helpers import decode_inputs
+    from vllm_neuron_amd._native import MI_Q, MI_W, NativeModel
+    shape = dict(num_layers=1, hidden_size=192, num_heads=3, num_kv_heads=1, head_dim=64, intermediate_size=256, vocab_size=vocab)
+    w = make_weights(DecoderConfig(**shape), seed=4)
+    for wd in ("bf16", "f8e4m3", "int8"):
+        model = NativeModel(**shape, rms_norm_eps=1e-5, rope_theta=1e4, rope_type=0, rope_factor=1.0, num_blocks=33, block_size=32, max_num_seqs=16,
+                            max_model_len=32, weight_dtype=MI_W[wd], quant_type=MI_Q["per_channel_symmetric"], quantize_lm_head=1, tp_degree=1, tp_rank=0,
+                            device_id=0, use_graphs=1, ctx_buckets=[32])
+        model.load_state_dict(w)
+        model.finalize()
+        out = {}
+        for rows in (4, 5, 11, 16):
+            for _ in range(2):         # eager pass, then the graph
+                out[rows] = model.forward(**decode_inputs([i % vocab for i in range(rows)], [0] * rows, [[1 + i] for i in range(rows)], 32, 32)).clone()
+        std = out[16].std().item()
+        assert torch.isfinite(out[16]).all() and torch.equal(out[5], out[16][:5]) and torch.equal(out[11], out[16][:11])
+        assert (out[4] - out[16][:4]).abs().max().item() < 0.05 * std
+        model.close()
+
+
+def _rapodra_of_many_words():
+    from tests import test_rapodra_gpu as T
+    from tests.rapodra_cases import config, dense, latent
+    return T, config(256, 8208, [latent(4, 32, 32, 64, 40, dense(256))], groups=2)
+
+
+# ... and bounded (bf16): groups of four with the last of one row-tile, against the oracle
+@pytest.mark.parametrize("rows", [5, 16, 17])
+def test_bounded_logits_to_the_host(rows):
+    T, cfg = _rapodra_of_many_words()
+    w = T.weights(cfg, 9)
+    r = T.replay(cfg, w, "bfloat16", max_tokens=rows * 48, max_live=rows)
+    toks = [T.tokens(cfg, w, n, 7000 + n) for n in (30, 31, 32)]
+    refs = [T.reference(f"words{i}", cfg, w, t, "bfloat16") for i, t in enumerate(toks)]
+    ids = [T.uid() for _ in range(rows)]
+    r.step([{"id": rid, "tokens": toks[i % 3][:20], "want": []} for i, rid in enumerate(ids)], [])
+    worst = 0.0
+    for p in range(20, 24):
+        outs = r.step([{"id": rid, "tokens": [toks[i % 3][p]], "want": [0]} for i, rid in enumerate(ids)], ids if p == 23 else [])
+        worst = max([worst] + [T.error(o, refs[i % 3][p:p + 1]) for i, o in enumerate(outs)])
+    assert worst <= T.LIMIT["bfloat16"], worst
+    r.engine.close()
 
 
 # Which of the two kernels takes 17 .. 32 rows of one-byte weights: the register kernel's sums over unsplit K are those of 16 rows bit for bit, the wide GEMM's are not.  Either side of the

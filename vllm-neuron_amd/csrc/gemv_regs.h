@@ -16,9 +16,10 @@ namespace mi {
 
 constexpr int kRegsMaxPasses = 64;   // row-tiles of a work-group: their scales and biases wait in LDS
 
-// HOLD: a work-group takes HOLD row-tiles side by side, and the wave that sums them keeps their results until it has all: a row's HOLD x 64 bytes
-// leave together.  For results that go over PCIe: neighbouring 64 bytes that come from different work-groups take a packet each, 44 GB/s; 128 or 256 bytes
-// of one work-group 52 - 55, what a copy reaches.
+// HOLD: a work-group takes HOLD row-tiles side by side, and the wave that sums them puts their results together in LDS until it has all: a row's HOLD x 64 bytes
+// leave with one request.  For results that go over PCIe, whose packets are what one request writes side by side: 32 rows of 128256 in pieces of 64 bytes
+// take 370 us (44 GB/s), of 128 bytes 320, of 256 and more 299 (55 GB/s, a copy 303).  The head of the 8B shape at 32 rows 333 us with four requests of 64 bytes
+// from registers, III now.
 template <int WD, int EPI, int MG, int NK, bool SLAB, int HOLD = 1>
 __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4* __restrict__ W, int NT, int KT, int M, int G,
                                                                    const uint16_t* __restrict__ x, int ldx, EpiArgs e, float* __restrict__ slab) {
@@ -30,6 +31,8 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
   __shared__ f32x4_t red[2][kGemvWaves][MG][64];
   __shared__ __attribute__((aligned(16))) float sc_lds[SLAB ? 4 : kRegsMaxPasses * 16], bi_lds[SLAB ? 4 : kRegsMaxPasses * 16];
   __shared__ float rf_lds[SLAB ? 1 : 16 * MG];        // the rows' own factors: 1 / rms where the norm left it to the output
+  constexpr int kOutPitch = HOLD * 16 + 4;
+  __shared__ __attribute__((aligned(16))) float out_lds[HOLD == 1 ? 4 : 16 * MG * kOutPitch];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int g = lane >> 4, c = lane & 15;
   const int kper = ceil_div(KT, (int)gridDim.y), k_lo = (int)blockIdx.y * kper, k_hi = min(k_lo + kper, KT);
@@ -143,7 +146,6 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  f32x4_t held[HOLD];
   auto finish = [&](int pass, int par) {
 #pragma unroll
     for (int mg = 0; mg < MG; ++mg) {
@@ -165,13 +167,15 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4*
           if constexpr (EPI == EPI_SOFTCAP) s[r] = e.softcap * tanhf(s[r] / e.softcap);
         }
         const int sub = pass % HOLD;
+        *reinterpret_cast<f32x4_t*>(out_lds + m * kOutPitch + sub * 16 + g * 4) = s;
+        if (sub < HOLD - 1 && pass < passes - 1) continue;
+        // (this wave's own; the next group's wave writes here behind a barrier that this one comes to with its results read)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-        for (int h = 0; h < HOLD; ++h)
-          if (h == sub) held[h] = s;
-        if (m < M && (sub == HOLD - 1 || pass == passes - 1)) {
-#pragma unroll
-          for (int h = 0; h < HOLD; ++h)
-            if (h <= sub) *reinterpret_cast<f32x4_t*>(e.out_f32 + (size_t)m * e.ld_out + n0 + (h - sub) * 16) = held[h];
+        for (int j = 0; j < HOLD; ++j) {
+          const int i = j * 64 + lane, row = mg * 16 + i / (HOLD * 4), q = i % (HOLD * 4);
+          const f32x4_t v = *reinterpret_cast<const f32x4_t*>(out_lds + row * kOutPitch + q * 4);
+          if (row < M && q < sub * 4 + 4) store_through(e.out_f32, ((uint32_t)row * e.ld_out + (tile_of(pass) - sub) * 16 + q * 4) * 4u, v);
         }
         continue;
       }
@@ -284,17 +288,22 @@ int launch_gemv_regs_wd(const LinearW& w, int M, const uint16_t* x, int ldx, int
     if (deferred) { *defer = sum; return MI_OK; }
     return launch_splitk_reduce(sum, epi, e, s);
   }
-  // (up to 16 rows the weights take longer than the way to the host, and single row-tiles deal them out more evenly: 8B fp8 8 rows 1266 us, 1280 with four;
-  //  24 rows 1695 and 1670, 7B int8 32 rows 1890 and 1830; nor where less than half of the CUs would have a group: us a launch, 20 - 27 rows, 2048 and 4096 wide, single row-tiles
-  //  and four: 16384 rows of logits 52.9 and 46.4, 8192 29.5 and 27.2, fp8 26.4 and 25.8, 4096 21.2 and 24.8)
-  if (e.far_out && M > 16 && w.N / 16 >= 2 * num_cu) {
-    if (epi == EPI_F32) return launch_gemv_regs_k<WD, EPI_F32, 2, false, 4>(w, M, x, ldx, e, s, 1, nullptr);
+  // (Logits to the host in groups of four row-tiles where their way, in pieces of 64 bytes, takes as long as the weights do or nearly so; below, single row-tiles deal the weights out more evenly.
+  //  Steps of half-depth models, us, single -> four: 8B fp8 6 rows 1123 -> 1121, 9 1199 -> 1188, 16 1403 -> 1382, bf16 5 rows 1710 -> 1714, 12 1839 -> 1856, 14 1870 -> 1877, 16 1940 -> 1919,
+  //  7B bf16 12 rows 1665 -> 1668, 14 1714 -> 1686, int8 5 rows 1029 -> 1030, 8 1095 -> 1085, 12 1207 -> 1179, 2048 wide 6 rows 522 -> 522, 16 591 -> 585; groups of two gain half of that.
+  //  Not where less than half of the CUs would have a group: us a launch, 20 - 27 rows, 2048 and 4096 wide, single row-tiles and four: 16384 rows of logits 52.9 and 46.4, 8192 29.5 and 27.2,
+  //  fp8 26.4 and 25.8, 4096 21.2 and 24.8)
+  const bool four = M * 540 >= w.K * (WD == MI_W_BF16 ? 2 : 1) && w.N / 16 >= 2 * num_cu;
+#define MI_R4(EPI_) return M <= 16 ? launch_gemv_regs_k<WD, EPI_, 1, false, 4>(w, M, x, ldx, e, s, 1, nullptr) : launch_gemv_regs_k<WD, EPI_, 2, false, 4>(w, M, x, ldx, e, s, 1, nullptr)
+  if (e.far_out && four) {
+    if (epi == EPI_F32) MI_R4(EPI_F32);
     if constexpr (WD == MI_W_BF16)
-      if (epi == EPI_SOFTCAP) return launch_gemv_regs_k<WD, EPI_SOFTCAP, 2, false, 4>(w, M, x, ldx, e, s, 1, nullptr);
+      if (epi == EPI_SOFTCAP) MI_R4(EPI_SOFTCAP);
   }
-  // (far results are stored through up to 16 rows: left in L2 they cross PCIe when the weights are done.  Steps of half-depth models, us: 8B fp8 4 rows 1116 -> 1095, 8 rows 1147 -> 1120,
-  //  16 rows 1299 -> 1288, 7B int8 5 rows 1138 -> 1088, 2048 wide 2 - 16 rows 0.2 - 3 %.  From 17 on PCIe is what bounds them, and pieces of 64 bytes are best put together by the L2: 24 rows of 8B
-  //  in groups of four row-tiles 1507, single ones stored through 1535, 32 rows 1606 and 1650)
+#undef MI_R4
+  // (Far results are stored through: left in L2 they cross PCIe when the weights are done.  Steps of half-depth models, us: 8B fp8 4 rows 1116 -> 1095, 8 rows 1147 -> 1120,
+  //  16 rows 1299 -> 1288, 7B int8 5 rows 1138 -> 1088, 2048 wide 2 - 16 rows 0.2 - 3 %; groups of four, 8B fp8 9 rows 1230 -> 1188, 32 rows 1790 -> 1768.  Not single row-tiles of 17 and more rows:
+  //  PCIe bounds them, and the L2 puts some of their pieces together, 24 rows of 8B 1535 through)
   EpiArgs near = e;
   near.far_out = false;
 #define MI_R(EPI_) return M <= 16 ? launch_gemv_regs_k<WD, EPI_, 1, false>(w, M, x, ldx, e, s, 1, nullptr) : launch_gemv_regs_k<WD, EPI_, 2, false>(w, M, x, ldx, near, s, 1, nullptr)
