@@ -922,47 +922,55 @@ __device__ __forceinline__ void delta_join(const DeltaGeom& g, float* __restrict
 // segment's last chunk renew its ring.  WIDE: rows of z and y in 16 and 8 bytes.  Bound by memory: 16 heads of 128, 2048 tokens, 42 MB in 16.3 us (19.5 with
 // a lane per column and eight tokens after each other).
 // SPLIT: a segment in two parts (delta_scan_split_kernel) -- chunks of the second one get their replies times S1, four of a head in a work-group, so that S1's
-// fragments come out of memory once for four waves; work-groups behind those make the last state.
-__host__ __device__ __forceinline__ int split_columns(int n, int H) { return ceil_div(ceil_div(n - split_first(n), 4) * H, ceil_div(H, 4)); }     // of the grid, for the second part
+// fragments come out of memory once for four waves; the second part takes longer and comes first, then the first one's chunks, four a work-group whatever the number of
+// heads, then those that make the last state.  Bound by the round of requests and the fp32 products behind it: everything that a wave needs from memory is asked for in front of the
+// barrier, S1 goes to LDS without registers, and where every tile is there no branch stands around a product.  16 heads of 128, 2048 tokens: 31.2 -> 21.2 us a launch; eight chunks to one S1
+// 24.7 (half as many CUs multiply; 28.8 with registers for two such work-groups a CU, which spill).
+constexpr int kOutWaves = 4;
+__device__ __forceinline__ void lds_dma16(const void* g, void* l) {      // 16 bytes a lane, to l + 16 lane
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g, (__attribute__((address_space(3))) void*)l, 16, 0, 0);
+}
+__host__ __device__ __forceinline__ int split_groups(int n, int H) { return ceil_div(n - split_first(n), kOutWaves) * H; }     // work-groups of the second part
+__host__ __device__ __forceinline__ int first_groups(int n, int H) { return ceil_div(split_first(n) * H, kOutWaves); }         // and of the first
 template <typename T, int NT, bool WIDE, bool SPLIT = false>
-__global__ __launch_bounds__(256) void delta_out_kernel(DeltaGeom g, DeltaIn in, const AttnSeg* __restrict__ segs, int nseg, int c0, int n, float* __restrict__ records,
-                                                        T* __restrict__ y, int ldy) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+__global__ __launch_bounds__(SPLIT ? kOutWaves * 64 : 256, SPLIT ? 2 : 1) void delta_out_kernel(DeltaGeom g, DeltaIn in, const AttnSeg* __restrict__ segs, int nseg, int c0, int n,
+                                                                                                 float* __restrict__ records, T* __restrict__ y, int ldy) {
+  const int wave = SPLIT ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6, lane = threadIdx.x & 63;
   int chunk = blockIdx.x, h = blockIdx.y * 4 + wave;
   __shared__ f32x4_t s1[SPLIT ? NT * NT * 64 : 1];      // the state between the parts, as fragments: one round of requests
   f32x4_t rep[SPLIT ? NT : 1];                           // the chunk's replies
+  bool second = false;
   if constexpr (SPLIT) {
-    const int first = split_first(n), columns = split_columns(n, g.H), x = (int)blockIdx.x - first - columns;      // (the second part takes longer: it comes first)
-    if (x >= 0) {
-      delta_join(g, in.state, in.slots[segs[0].seq], n, records, (x * (int)gridDim.y + (int)blockIdx.y) * 4 + wave);
+    const int first = split_first(n), seconds = split_groups(n, g.H), firsts = first_groups(n, g.H), b = blockIdx.x;
+    if (b >= seconds + firsts) {
+      delta_join(g, in.state, in.slots[segs[0].seq], n, records, (b - seconds - firsts) * kOutWaves + wave);
       return;
     }
-    chunk -= columns;
-    if (chunk < 0) {
-      const int u = (int)blockIdx.x * (int)gridDim.y + (int)blockIdx.y;
-      chunk = first + u / g.H * 4 + wave;
-      h = u % g.H;
+    second = b < seconds;
+    const int unit = (b - seconds) * kOutWaves + wave;
+    chunk = second ? first + b / g.H * kOutWaves + wave : unit / g.H;
+    h = second ? b % g.H : unit % g.H;
+    if (!second && chunk >= first) return;
+    if (second) {
       const SplitMem m = split_mem(records, g, n, h);
       const float* replies = m.replies + (size_t)min(chunk, n - 1) * 16 * g.dkp + (lane & 15) * 16 + (lane >> 4) * 4;
-#pragma unroll
-      for (int d = 0; d < NT; ++d) rep[d] = *reinterpret_cast<const f32x4_t*>(replies + min(d, g.dkp / 16 - 1) * 256);
       const f32x4_t* from = reinterpret_cast<const f32x4_t*>(m.s1);
       const int all = g.dkp * g.dvp / 4;
-      f32x4_t v[NT * NT / 4];
 #pragma unroll
-      for (int i = 0; i < NT * NT / 4; ++i) v[i] = from[min(i * 256 + (int)threadIdx.x, all - 1)];
+      for (int i = 0; i < NT * NT / kOutWaves; ++i)
+        lds_dma16(from + min(i * kOutWaves * 64 + (int)threadIdx.x, all - 1), s1 + i * kOutWaves * 64 + wave * 64);
 #pragma unroll
-      for (int i = 0; i < NT * NT / 4; ++i) s1[i * 256 + threadIdx.x] = v[i];
-      __syncthreads();
+      for (int d = 0; d < NT; ++d) rep[d] = *reinterpret_cast<const f32x4_t*>(replies + min(d, g.dkp / 16 - 1) * 256);
     }
   }
-  const ChunkAt at = chunk_at(segs, nseg, c0 + chunk);
-  if (!at.ok || chunk >= n) return;
+  const int known = min(chunk, n - 1);
+  const ChunkAt at = chunk_at(segs, nseg, c0 + known);
+  if (!SPLIT && (!at.ok || chunk >= n)) return;
+  const int t = lane >> 2, q = (lane & 3) * 4, tiles = g.dvp / 16;
+  const size_t row = at.sg.row0 + at.t0 + min(t, at.n - 1);
+  f32x4_t x[NT], z[NT];
   if (h < g.H) {
-    const int t = lane >> 2, q = (lane & 3) * 4, tiles = g.dvp / 16;
-    const size_t row = at.sg.row0 + at.t0 + min(t, at.n - 1);
-    const float *src = factors_at(records, (size_t)h * n + chunk, g.dkp, g.dvp).v, *zr = in.z + row * in.ldz + in.gate + h * g.dv;
-    f32x4_t x[NT], z[NT];
+    const float *src = factors_at(records, (size_t)h * n + known, g.dkp, g.dvp).v, *zr = in.z + row * in.ldz + in.gate + h * g.dv;
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
       const int tile = min(i, tiles - 1), v = tile * 16 + q;
@@ -970,21 +978,34 @@ __global__ __launch_bounds__(256) void delta_out_kernel(DeltaGeom g, DeltaIn in,
       if constexpr (WIDE) z[i] = *reinterpret_cast<const f32x4_t*>(zr + min(v, g.dv - 4));
       else z[i] = f32x4_t{zr[min(v, g.dv - 1)], zr[min(v + 1, g.dv - 1)], zr[min(v + 2, g.dv - 1)], zr[min(v + 3, g.dv - 1)]};
     }
+  }
+  if constexpr (SPLIT) {
+    if (second) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+    }
+    if (chunk >= n) return;
+  }
+  if (h < g.H) {
     if constexpr (SPLIT) {
-      if (chunk >= split_first(n)) {     // the products leave a column's quad of token (lane & 15) in lane >> 4: four lanes trade places
+      if (second) {     // the products leave a column's quad of token (lane & 15) in lane >> 4: four lanes trade places
+        auto products = [&](auto whole) {      // (every tile there: no branch around a product)
 #pragma unroll
-        for (int i = 0; i < NT; ++i) {
-          f32x4_t add[2] = {};
+          for (int i = 0; i < NT; ++i) {
+            f32x4_t add[2] = {};
 #pragma unroll
-          for (int d = 0; d < NT; ++d) {
-            if (max(i, d) >= tiles) continue;
-            const f32x4_t f = s1[(i * tiles + d) * 64 + lane];
+            for (int d = 0; d < NT; ++d) {
+              if (!decltype(whole)::value && max(i, d) >= tiles) continue;
+              const f32x4_t f = s1[(i * (decltype(whole)::value ? NT : tiles) + d) * 64 + lane];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) add[d & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[r], rep[d][r], add[d & 1], 0, 0, 0);
+              for (int r = 0; r < 4; ++r) add[d & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[r], rep[d][r], add[d & 1], 0, 0, 0);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[i][r] += __shfl(add[0][r] + add[1][r], (lane & 3) * 16 + t);
           }
-#pragma unroll
-          for (int r = 0; r < 4; ++r) x[i][r] += __shfl(add[0][r] + add[1][r], (lane & 3) * 16 + t);
-        }
+        };
+        if (tiles == NT) products(std::true_type());
+        else products(std::false_type());
       }
     }
     float ss = 0.f;
@@ -1015,8 +1036,8 @@ __global__ __launch_bounds__(256) void delta_out_kernel(DeltaGeom g, DeltaIn in,
   if (!at.last) return;
   const int C = g.channels();
   float* ring = in.ring + (size_t)in.slots[at.sg.seq] * g.taps * C;
-  const bool by_wave = SPLIT && chunk >= split_first(n);       // (one wave a head has the last chunk, not four work-groups)
-  for (int ch = by_wave ? h * 64 + lane : blockIdx.y * 256 + threadIdx.x; ch < C; ch += by_wave ? g.H * 64 : gridDim.y * 256)
+  // (SPLIT: the last chunk is of the second part, and a wave a head has it, not ceil(H / 4) work-groups)
+  for (int ch = SPLIT ? h * 64 + lane : blockIdx.y * 256 + threadIdx.x; ch < C; ch += SPLIT ? g.H * 64 : gridDim.y * 256)
     for (int i = max(0, at.sg.n - g.taps); i < at.sg.n; ++i)
       ring[(size_t)((at.sg.pos0 + i) % g.taps) * C + ch] = in.proj[(size_t)(at.sg.row0 + i) * in.ldp + ch];
 }
@@ -1074,8 +1095,8 @@ int launch_delta_prompt(const DeltaGeom& g, const DeltaIn& in, const AttnSeg* sd
   for (int c0 = 0; c0 < chunks; c0 += max_chunks) {
     const int n = std::min(max_chunks, chunks - c0);
     const bool split = nseg == 1 && split_fits(g, num_cu) && n >= split_chunks(g, num_cu);
-    const int joins = split ? ceil_div(g.H * nvt * nvt, 4 * ceil_div(g.H, 4)) : 0;       // work-groups for the last state
-    const dim3 gf(n, g.H), gs(g.H * nvt, nseg), go(split ? split_first(n) + split_columns(n, g.H) + joins : n, ceil_div(g.H, 4));
+    const int joins = ceil_div(g.H * nvt * nvt, kOutWaves);       // work-groups for the last state
+    const dim3 gf(n, g.H), gs(g.H * nvt, nseg), go(split ? split_groups(n, g.H) + first_groups(n, g.H) + joins : n, split ? 1 : ceil_div(g.H, 4));
 #define MI_DF(TAPS) { \
     if (lds > 48 * 1024) { rc = ensure_dynamic_lds(reinterpret_cast<const void*>(delta_factors_kernel<TAPS>), (int)lds); if (rc != MI_OK) return rc; } \
     hipLaunchKernelGGL((delta_factors_kernel<TAPS>), gf, dim3(256), lds, s, g, in, sd, nseg, c0, records); }
@@ -1098,8 +1119,8 @@ int launch_delta_prompt(const DeltaGeom& g, const DeltaIn& in, const AttnSeg* sd
 #undef MI_DP
 #undef MI_DS
 #define MI_DO(NT, ...) \
-    if (f32) hipLaunchKernelGGL((delta_out_kernel<float, NT, __VA_ARGS__>), go, dim3(256), 0, s, g, in, sd, nseg, c0, n, records, (float*)y, ldy); \
-    else hipLaunchKernelGGL((delta_out_kernel<uint16_t, NT, __VA_ARGS__>), go, dim3(256), 0, s, g, in, sd, nseg, c0, n, records, (uint16_t*)y, ldy)
+    if (f32) hipLaunchKernelGGL((delta_out_kernel<float, NT, __VA_ARGS__>), go, dim3(split ? kOutWaves * 64 : 256), 0, s, g, in, sd, nseg, c0, n, records, (float*)y, ldy); \
+    else hipLaunchKernelGGL((delta_out_kernel<uint16_t, NT, __VA_ARGS__>), go, dim3(split ? kOutWaves * 64 : 256), 0, s, g, in, sd, nseg, c0, n, records, (uint16_t*)y, ldy)
     const bool wide = g.dv % 4 == 0 && in.ldz % 4 == 0 && in.gate % 4 == 0 && ldy % 4 == 0 && reinterpret_cast<uintptr_t>(in.z) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
     if (split) { if (wide && g.dv <= 64) { MI_DO(4, true, true); } else if (wide) { MI_DO(8, true, true); } else { MI_DO(8, false, true); } }
     else if (!wide) { MI_DO(16, false); } else if (g.dv <= 64) { MI_DO(4, true); } else if (g.dv <= 128) { MI_DO(8, true); } else { MI_DO(16, true); }
