@@ -28,7 +28,7 @@ def test_edges_of_columns(lib, shape):  # noqa: F811
             x.check_state(i)
 
 
-# one long segment in two parts at the same time: the shortest that goes so, second parts of 0 .. 3 chunks by themselves and a ragged last one, one and two channel tiles a
+# one long segment in two parts at the same time: second parts of 0 .. 3 chunks by themselves and a ragged last one, one and two channel tiles a
 # wave with waves idle and not; the next segment starts from the joined state
 @pytest.mark.parametrize("shape", [(2, 2, 128, 128, 4), (16, 16, 128, 128, 4), (3, 1, 80, 80, 3), (4, 2, 64, 64, 2), (2, 1, 20, 20, 4), (1, 1, 7, 16, 1)])
 @pytest.mark.parametrize("first,second", [(1008, 1024), (1024, 1056), (1025, 1071), (1055, 1036), (1500, 2)])
@@ -48,11 +48,21 @@ def test_parts_and_pieces(lib, lengths, chunks):  # noqa: F811
         x.check_state(i)
 
 
-# heads of 128 on more CUs than three parts leave: a chunk below the line (one scan), on it, and one above
+# heads of 128 on more CUs than three parts leave
 @pytest.mark.parametrize("heads", [12, 16])
 @pytest.mark.parametrize("first,second", [(1136, 1152), (1152, 1168), (1151, 1153)])
 def test_two_parts_that_share_cus(lib, heads, first, second):  # noqa: F811
     test_long_segments_in_two_parts(lib, (heads, heads, 128, 128, 4), first, second)
+
+
+# a chunk below the line (one scan), on it, and a ragged one above; a workspace that holds just so many, and one less
+@pytest.mark.parametrize("shape", [(16, 16, 128, 128, 4), (3, 1, 128, 128, 2), (4, 4, 64, 64, 4), (20, 20, 96, 96, 3), (1, 1, 7, 16, 1)])
+@pytest.mark.parametrize("first,second,chunks", [(752, 768, 256), (753, 770, 256), (768, 1000, 48), (800, 769, 47)])
+def test_line_of_two_parts(lib, shape, first, second, chunks):  # noqa: F811
+    x = Delta(lib, *shape, [first + second], seed=sum(shape) + first)
+    close(*x.step([(0, first)], chunks=chunks), 1)
+    close(*x.step([(0, second)], 0, chunks=chunks), 0)
+    x.check_state(0)
 
 
 # the replies' rooms of a second part: 16 dkp numbers a head and chunk, for heads that have CUs for one (16 of 128 on 256 CUs), and not for one head more

@@ -858,14 +858,13 @@ __global__ __launch_bounds__(256, 2) void delta_scan_pairs_kernel(DeltaGeom g, f
 // row of replies is what the same recurrence makes of the columns of the identity.  So the second part has two work-groups for 16 columns, which share a CU and take 2.7 us
 // a pair between them (fp32 matrix products leave no room for vector instructions beside them: 32 cycles and 5 - 9 for each of those), and it is the shorter one; the order of the
 // work-groups puts both on the CUs that the first part leaves.  delta_out_kernel adds replies S1 and makes the last state.  Everything stays fp32.
-// 16 heads of 128, 2048 tokens, us: scan 98 -> 66, output norm 15.5 -> 31, a call 2142 -> 2020; 3000 tokens 2993 -> 2768.  The cut is for parts that share CUs (16 heads of 128 take 256 of them); where each
+// 16 heads of 128, 2048 tokens, us: scan 98 -> 66, output norm 15.5 -> 21 (31 at first, a call 2142 -> 2020; 3000 tokens 2993 -> 2768).  The cut is for parts that share CUs (16 heads of 128 take 256 of them); where each
 // has its own, one half would be the even one.  All kernels of a launch of 8 heads there: 2048 tokens 139 -> 116, 4096 251 -> 200; 2 heads 119 -> 96, 215 -> 160.
 // Behind the records: [chunk][16 dkp] replies a head, those of the first part unused: there the states, S1 as fragments, the second part's own (L) and its transition (P).
-constexpr int kSplitChunks = 64;                 // of a segment at least: room for the three states
-// ... and below, the joining costs what the parts save where they share CUs and states are 112 and 128 high (a work-group stages 50 and 64 KB of S1).  us of all kernels, one scan -> two parts: 16 heads
-// of 128, 1024 tokens 95 -> 98, 1136 109.5 -> 106.4; 12 heads 88 -> 92, 97.9 -> 95.0; 14 heads 93.8 -> 94.4, 99.8 -> 101.3, 1200 tokens 107.6 -> 108.2; 10 heads, which share none, 85.9 -> 82.8; 20 heads of 96 97 -> 91;
-// 32 of 64 85 -> 79
-static int split_chunks(const DeltaGeom& g, int num_cu) { return g.dkp > 96 && 3 * g.H * (g.dvp / 16) > num_cu ? 72 : kSplitChunks; }
+// From 48 chunks on (16 dkp numbers each: room for the three states in those of the first part): below, the joining costs what the parts save.  us of all kernels, one scan -> two parts,
+// 640, 768, 1008 tokens: 16 heads of 128 69.5 -> 70.1, 75.8 -> 74.7, 91.5 -> 84.1; 12 heads 64.4 -> 67.1, 73.8 -> 72.4, 86.0 -> 80.8; 2 heads 53.3 -> 53.3, 59.2 -> 58.6, 71.4 -> 64.7;
+// 20 heads of 96 66.7 -> 68.4, 74.4 -> 73.1, 91.3 -> 86.7; 32 of 64 61.4 -> 56.5, 64.8 -> 63.4, 81.0 -> 73.0.  8 layers of 16 heads of 128, 1100 tokens: 1445 -> 1377 a call.
+constexpr int kSplitChunks = 48;
 __host__ __device__ __forceinline__ int split_first(int n) { return (n * 41 + 127) / 256 * 4; }     // chunks of the first part: 0.64 of them, whole turns of the loop
 struct SplitMem { float *replies, *s1, *l, *p; };
 __host__ __device__ __forceinline__ SplitMem split_mem(float* records, const DeltaGeom& g, int n, int h) {
@@ -1094,7 +1093,7 @@ int launch_delta_prompt(const DeltaGeom& g, const DeltaIn& in, const AttnSeg* sd
   const size_t lds = (size_t)(3 * kC * (g.dkp + 4) + std::max(kC * (g.dkp + 4), kPairParts * kPairTiles * 8)) * sizeof(float);
   for (int c0 = 0; c0 < chunks; c0 += max_chunks) {
     const int n = std::min(max_chunks, chunks - c0);
-    const bool split = nseg == 1 && split_fits(g, num_cu) && n >= split_chunks(g, num_cu);
+    const bool split = nseg == 1 && split_fits(g, num_cu) && n >= kSplitChunks;
     const int joins = ceil_div(g.H * nvt * nvt, kOutWaves);       // work-groups for the last state
     const dim3 gf(n, g.H), gs(g.H * nvt, nseg), go(split ? split_groups(n, g.H) + first_groups(n, g.H) + joins : n, split ? 1 : ceil_div(g.H, 4));
 #define MI_DF(TAPS) { \
