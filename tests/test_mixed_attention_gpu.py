@@ -58,3 +58,30 @@ def test_runs_beside_prompts(monkeypatch, name, step):
         worst = max(worst, (got[i] - ref[0]).abs().max().item())
     assert worst < 0.06, worst            # as the other comparisons with the oracle's bf16 rounding points
     model.close()
+
+
+# the splits of a run are merged by the work-group that ends last, which leaves the counters as it found them: a batch gives the same numbers again, whatever runs between
+@pytest.mark.parametrize("rows", [1, 5])
+def test_merged_splits_again(monkeypatch, rows):
+    for key, value in dict(BS=BS, MAXLEN=MAXLEN, NSEQ=NSEQ, NB=1 + NSEQ * MB).items():
+        monkeypatch.setattr(M, key, value)
+    cfg = zoo_config("llama31_like")
+    model = M.native_model(cfg, make_weights(cfg, seed=1))
+    g = torch.Generator().manual_seed(rows)
+    seqs = [torch.randint(0, cfg.vocab_size, (700 - 3 * r,), generator=g).tolist() for r in range(6)]
+    blocks = [[1 + i * MB + j for j in range(MB)] for i in range(6)]
+    for r in range(6):
+        model.forward(**prefill_inputs(seqs[r], blocks[r], BS, MAXLEN, 0))
+
+    def call(run, chunk):
+        batch = [(r, len(seqs[r]) - 1, len(seqs[r])) for r in run] + [(5, 0, chunk)]
+        ids = [t for r, lo, hi in batch for t in seqs[r][lo:hi]]
+        pos = [p for r, lo, hi in batch for p in range(lo, hi)]
+        slots = [blocks[r][p // BS] * BS + p % BS for r, lo, hi in batch for p in range(lo, hi)]
+        return model.forward_chunked(torch.tensor(ids), torch.tensor(pos), torch.tensor(slots), torch.tensor([blocks[r] for r, _, _ in batch]),
+                                     torch.tensor([hi for _, _, hi in batch]), torch.tensor([lo for _, lo, _ in batch]))
+    first, other = call(range(rows), 40), call([2], 70)
+    assert torch.isfinite(first).all()
+    for _ in range(20):
+        assert torch.equal(first, call(range(rows), 40)) and torch.equal(other, call([2], 70))
+    model.close()

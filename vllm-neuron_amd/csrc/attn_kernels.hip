@@ -380,7 +380,7 @@ constexpr int kAttnTickets = 1024;
 size_t attn_scratch_bytes(int B, int nh, int hd) {
   return kAttnTickets * sizeof(unsigned int) + (size_t)B * nh * kAttnMaxSplits * (hd + 2) * sizeof(float);
 }
-// Off by default: measured on Llama-3.1-8B decode (B 4, ctx 1024) the in-launch merge costs the
+// In launches of decode rows alone off by default: measured on Llama-3.1-8B decode (B 4, ctx 1024) the in-launch merge costs the
 // last work-group ~5.4 us (write-through drain + returning atomic + sc1 read-back are three
 // dependent trips to memory) against 4.8 us for the separate combine launch: 2.157 vs 2.138 ms per
 // step.  MI355X_ATTN_MERGE=1 selects it (same results: tests/test_model_gpu.py runs both).
@@ -1099,7 +1099,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 // A prompt's chunk and the requests that generate beside it, in one launch: neither fills the chip, and one after the other they cost 11.1 + 8.0 us at 239 tokens
 // beside 3 contexts of up to 900 (8B model).  Work-groups x from `nd` on are the prompt's, gx of every slice of the keys; those before them one
 // (split, sequence) each of the others.
-struct DecodeSide { const uint16_t* q; const int32_t* block_table; const int32_t* ctx_lens; int MB, NS, nd, num_blocks; float *o_part, *ml_part; uint16_t* out; };
+struct DecodeSide { const uint16_t* q; const int32_t* block_table; const int32_t* ctx_lens; int MB, NS, nd, num_blocks; float *o_part, *ml_part; uint16_t* out; unsigned int* tickets; };
 template <int HD, int KH, bool FINAL>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_mixed_kernel(
     const uint16_t* __restrict__ q, int T, int q_pos0, const uint16_t* __restrict__ kpool,
@@ -1112,8 +1112,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     attn_prefill2_body<HD, 8, KH>(smem, y % gx, blockIdx.y, two ? x & 1 : 0, two ? 2 : 1, y / gx, ns, q, T, q_pos0, kpool, vpool, bs, bs_shift, block_table, nh, nkv, G, Gp, nblk,
                               paired, o_part, ml_part, out, scale_log2e);
   } else {
-    attn_decode_body<HD, 8, FINAL>(smem, (int)blockIdx.x % d.NS, blockIdx.y, (int)blockIdx.x / d.NS, d.q, kpool, vpool, bs, d.block_table, d.MB, d.ctx_lens, nh, nkv, G, d.NS,
-                                   d.o_part, d.ml_part, d.out, scale_log2e, nullptr, 1, d.num_blocks);
+    attn_decode_body<HD, 8, FINAL, !FINAL>(smem, (int)blockIdx.x % d.NS, blockIdx.y, (int)blockIdx.x / d.NS, d.q, kpool, vpool, bs, d.block_table, d.MB, d.ctx_lens, nh, nkv, G, d.NS,
+                                   d.o_part, d.ml_part, d.out, scale_log2e, d.tickets, 1, d.num_blocks);
   }
 }
 
@@ -1261,6 +1261,9 @@ int launch_attn_prefill(const uint16_t* q, int T, int q_pos0, const uint16_t* kp
 // Eight waves a work-group here, four in the launch of its own: half the splits, and none (so no combine launch) up to 256 tokens of 128-wide heads, 512 of 64-wide
 // ones, twice the other's limit.  us per call, splits -> none: 8B fp8 239 + 3 of 250 tokens 2977 -> 2940, of 500 2974 -> 2988, of 1000 2979 -> 3114; 64 + 6 of 300
 // 2177 -> 2145, of 600 2197 -> 2215; TinyLlama 300 + 4 of 500 2234 -> 2178, of 1000 2228 -> 2296.
+// Splits are merged in this launch by whichever ends last (MERGE): what that takes is hidden by the prompt's work-groups, where a launch of one's own behind both was in line.  A work-group has its CU
+// to itself (two waves a SIMD).  us a call, combine launch -> merged: 8B fp8 239 + 3 2649 -> 2617 (a layer 10.6 + 4.7 -> 12.2), 64 + 6 1939 -> 1922, 500 + 1 3971 -> 3916, TinyLlama 300 + 4 1991 -> 1960,
+// 7B int8 200 + 3 2515 -> 2506.
 static int mixed_splits(const AttnMixed& m, int nkv, int hd) { return m.max_ctx > 0 && m.max_ctx * hd <= 256 * 128 ? 1 : ceil_div(attn_decode_splits(m.B, nkv), 2); }
 template <int HD>
 static int launch_mixed_t(const AttnMixed& m, const PrefillPlan& p, int T, int q_pos0, const uint16_t* q, const int32_t* bt, uint16_t* out, const uint16_t* kpool,
@@ -1269,14 +1272,13 @@ static int launch_mixed_t(const AttnMixed& m, const PrefillPlan& p, int T, int q
   float* ml_part = reinterpret_cast<float*>(reinterpret_cast<unsigned int*>(m.scratch) + kAttnTickets);
   float* o_part = ml_part + (size_t)m.B * nh * kAttnMaxSplits * 2;
   const int NS = mixed_splits(m, nkv, HD);
-  const DecodeSide d{m.q, m.block_table, m.ctx_lens, m.MB, NS, NS * m.B, m.num_blocks, o_part, ml_part, m.out};
+  const DecodeSide d{m.q, m.block_table, m.ctx_lens, m.MB, NS, NS * m.B, m.num_blocks, o_part, ml_part, m.out, reinterpret_cast<unsigned int*>(m.scratch)};
   const int lds = std::max<int>(p.kh == 2 ? attn_prefill2_lds<HD, 8, 2>() : attn_prefill2_lds<HD, 8, 1>(), (int)attn_decode_lds<HD, 8>());
   const auto fn = p.kh == 2 ? (NS == 1 ? attn_mixed_kernel<HD, 2, true> : attn_mixed_kernel<HD, 2, false>)
                             : (NS == 1 ? attn_mixed_kernel<HD, 1, true> : attn_mixed_kernel<HD, 1, false>);
   MI_TRY_A(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds));
   hipLaunchKernelGGL(fn, dim3(d.nd + p.gx * p.ns * p.subs, nkv), dim3(512), lds, s, q, T, q_pos0, kpool, vpool, bs, p.bs_shift, bt, nh, nkv, nh / nkv, p.Gp, p.subs, p.nblk, p.paired,
                      p.gx, p.ns, p.o_part, p.ml_part, out, scale_log2e, d);
-  if (NS > 1) hipLaunchKernelGGL((attn_combine_kernel<HD>), dim3(nh, m.B), dim3(HD), 0, s, o_part, ml_part, NS, nh, m.out);
   launch_prefill_combine(p, T, nh, HD, out, s);
   MI_HIP(hipGetLastError());
   return MI_OK;
