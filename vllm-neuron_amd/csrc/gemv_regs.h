@@ -1,4 +1,4 @@
-// Token-generation weight stream for 5 .. 32 rows: the activations live in registers.
+// Token-generation weight stream for 5 .. 32 rows, and for up to 4 where no norm is left to do in front: the activations live in registers.
 //
 // The kernels of linear_device.h keep the activations in LDS.  From 5 rows on that is what their time goes to: rows x K does not fit
 // beside the reduction buffers, so it is staged in chunks between barriers, or streamed beside the weights and read back by every wave.  Here a

@@ -14,10 +14,10 @@
 // k-steps per load for the 1-byte types).  Tiles of one 16-row group are contiguous along K,
 // so a wave streams a dense byte range.
 //
-// Token generation of up to 4 rows: the kernels of linear_device.h — pure weight streaming, HBM-bound.  x lives in LDS in
+// Token generation of up to 4 rows, where no norm was handed on and gemv_few_rows_in_regs says no: the kernels of linear_device.h — pure weight streaming, HBM-bound.  x lives in LDS in
 //   fragment order; every wave streams a K-slice of one row-tile with 2 x 8 KiB in flight;
 //   the MFMA does the dot products AND the cross-lane reduction; waves combine through LDS
-//   in a fixed order (deterministic, no atomics).  5 .. 32 rows: gemv_regs.h, x in registers.
+//   in a fixed order (deterministic, no atomics).  5 .. 32 rows, and up to 4 behind a norm that was handed on: gemv_regs.h, x in registers.
 // Context encoding: gemm_wide.h; gemm_kernel here (128 x 128 tile, x through swizzled LDS, W straight
 //   from global in fragment order) for what that does not take.
 //
@@ -69,7 +69,7 @@ bool gemv_regs_holds(const LinearW& w) { return ceil_div(w.K / tile_k(w.wd), kGe
 //   7B int8, 14 layers: 5 rows 1454 / 1330, 14 rows 1699 / 1446, 24 rows 2332 / 1789
 //   TinyLlama bf16:     1 row 876 / 1034, 16 rows 1389 / 1210, 30 rows 1501 / 1450
 //   16 layers of width 256 / 512 / 1024 / 1536, bf16: 5 rows 572 / 467, 604 / 538, 637 / 556, 745 / 673; 32 rows 739 / 604, 790 / 626, 850 / 667, 1001 / 926
-// Up to 4 rows the norm inside the weight stream's kernel and its two to eight waves per row-tile win.
+// Up to 4 rows the norm inside the weight stream's kernel and its two to eight waves per row-tile win, unless the projection in front has handed that norm on (run_linear).
 bool gemv_in_regs(const LinearW& w, int M, size_t ws_bytes) { return M >= 5 && M <= 32 && gemv_regs_fits(w, M, ws_bytes); }
 // Up to 4 rows of bf16 activations (nothing to fuse in front).  They win where a wave's weights of a row-tile are one batch of requests and each work-group has one
 // row-tile (the chain to the first request is shorter: no staging) or eight and more (the tiles follow each other without a barrier on the way), and, where the sums have a

@@ -8,11 +8,12 @@
 // Per decoder layer (token generation, 6 launches, captured in a hipGraph per batch size):
 //   gemv[norm -> QKV -> bias -> RoPE -> q buffer + KV-pool scatter]
 //   paged attention (split) ; combine
-//   gemv[O proj -> fp32 partial]                     (+ RCCL all-reduce when tp_degree > 1)
-//   gemv[residual add + norm -> gate|up -> SwiGLU]
-//   gemv[down proj -> fp32 partial]                  (+ RCCL all-reduce)
-// The residual stream is fp32 and ping-pongs between two buffers: the norm prologue of the
-// NEXT kernel folds in the previous partial, so a row-parallel output needs no extra pass.
+//   gemv[O proj -> residual add, or fp32 partial + RCCL all-reduce when tp_degree > 1]
+//   gemv[norm -> gate|up -> SwiGLU]
+//   gemv[down proj -> as O proj]
+// The residual stream is fp32 and ping-pongs between two buffers: with shards the norm prologue of the
+// NEXT kernel folds in the previous partial, so a row-parallel output needs no extra pass.  Up to 16 rows a residual projection
+// hands the norm behind it on (run_linear): rows times the gain and the parts of their sums of squares; from there to 32 rows a norm kernel stands in front.
 
 #include <chrono>
 #include <cmath>
@@ -463,8 +464,8 @@ int run_layers(mi_ctx* c, int rows, bool decode, int B, int MB, int q_pos0, int 
 }
 
 // Where the head of a call for `nrows` rows of host logits writes: straight into the pinned buffer the caller reads, over PCIe under its own weight stream.
-// The weight-streaming kernels' 64-byte pieces go out at 40 - 44 GB/s (a copy kernel: 42 - 55), so 4 rows of 128256 take 51 us under the head's 87 where
-// head, gap and copy took 87 + 19 + 37; 32 rows 369 against 127 + 19 + 300.  The GEMMs of larger batches, and shards, keep the copy.
+// A PCIe packet holds what one request writes side by side: 44 GB/s in pieces of 64 bytes, 55 of 256 (a copy: 54), which gemv_regs.h writes where that matters.  So 4 rows of 128256 take 51 us under
+// the head's 87 where head, gap and copy took 87 + 19 + 37; 32 rows 313 (369 in pieces of 64) against 127 + 19 + 300.  The GEMMs of larger batches, and shards, keep the copy.
 struct HeadToHost {
   mi_ctx* c;
   HeadToHost(mi_ctx* c_, int nrows, bool wanted) : c(c_) { c->head_out = wanted && !c->collective() && nrows <= 32 ? c->h_logits : nullptr; }
