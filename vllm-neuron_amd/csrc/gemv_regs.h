@@ -19,7 +19,7 @@ constexpr int kRegsMaxPasses = 64;   // row-tiles of a work-group: their scales 
 // HOLD: a work-group takes HOLD row-tiles side by side, and the wave that sums them puts their results together in LDS until it has all: a row's HOLD x 64 bytes
 // leave with one request.  For results that go over PCIe, whose packets are what one request writes side by side: 32 rows of 128256 in pieces of 64 bytes
 // take 370 us (44 GB/s), of 128 bytes 320, of 256 and more 299 (55 GB/s, a copy 303).  The head of the 8B shape at 32 rows 333 us with four requests of 64 bytes
-// from registers, III now.
+// from registers, 313 now.
 template <int WD, int EPI, int MG, int NK, bool SLAB, int HOLD = 1>
 __global__ __launch_bounds__(kGemvWaves * 64) void gemv_regs_kernel(const uint4* __restrict__ W, int NT, int KT, int M, int G,
                                                                    const uint16_t* __restrict__ x, int ldx, EpiArgs e, float* __restrict__ slab) {
