@@ -20,7 +20,7 @@ struct EpiArgs {
   // EPI_F32: out[m * ld_out + n] = y;  EPI_RESID: out = resid_in[m * ld_out + n] + y
   float* out_f32;
   int ld_out;
-  bool far_out;        // out_f32 is host memory (launch_gemv, launch_gemv_regs, EPI_F32 and EPI_SOFTCAP: results are stored through L2, or leave in larger pieces)
+  bool far_out;        // out_f32 is host memory (launch_gemv, launch_gemv_regs of an unsplit K, EPI_F32 and EPI_SOFTCAP: results are stored through L2, or leave in larger pieces; elsewhere: as any)
   const float* resid_in;
   // EPI_RESID, launch_gemv and launch_gemv_regs, up to 16 rows, ld_out = N, or null: the norm behind is left to its projection, which takes next_x[m * ld_out + n] = bf16(out next_gain[n]) and 1 / rms
   //   from next_ss [M][N / 16], the sums of squares of out over 16 columns.  launch_gemv_regs does not split K then (gemv_regs_holds)
