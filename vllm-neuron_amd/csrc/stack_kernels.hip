@@ -245,7 +245,7 @@ template <> struct Raw4<float> { typedef float4 type; };
 __device__ __forceinline__ float4 widen(uint2 v) { return make_float4(bf16lo_to_f32(v.x), bf16hi_to_f32(v.x), bf16lo_to_f32(v.y), bf16hi_to_f32(v.y)); }
 __device__ __forceinline__ float4 widen(float4 v) { return v; }
 
-// Token generation, rows of up to 4096: one float4 per thread and everything the row needs requested at once -- the sublayer's output,
+// Token generation, and prompts without a convolution's state (launch_sandwich_rows), rows of up to 4096: one float4 per thread and everything the row needs requested at once -- the sublayer's output,
 // the stream, both weights, the convolution's taps and state -- so that the two norms wait for memory once.  D / G a multiple of
 // 256; a norm's part is a work-group of its own (nothing crosses parts): a CU takes in some 35 GB/s, and a row of 2048 behind eight slabs is 74 KB.
 // 4 rows of 2048 in 4 parts 6.0 -> 4.7 us a launch.
@@ -761,9 +761,12 @@ int launch_sandwich_rows(const float* resid_in, float* resid_out, const RowSourc
     if (rc != MI_OK) return rc;
     cs = *conv;
   }
-  // (rows of prompts too, where no convolution's state rides along: the general kernel waits for memory twice and more.  us a call: Bokulorn 2048 tokens 2166 -> 2150, Nusovik 777 2157 -> 2151)
-  if ((T <= 32 || !conv) && (w_pre || as_is) && ld <= 4096 && ld == D && (D / groups) % 256 == 0 && (!conv || conv->taps <= 4)) {
-    const int gs = D / groups;      // (one wave and more)
+  // Rows of prompts too, where no convolution's state rides along: the general kernel waits for memory twice and more.  Up to 512 rows always (us a launch with both norms, general -> this one: 4096 wide
+  // 128 rows 7.9 -> 5.4, 512 rows 14.7 -> 9.3).  Beyond, the general kernel has 256 threads a row, several float4 each, and more rows on a CU: up to 2048 wide this one is still as fast or faster (1024 rows
+  // 9.9 -> 8.7, 2048 rows 16.8 -> 16.3; a call of Bokulorn 2048 tokens 2166 -> 2150, Nusovik 777 2157 -> 2151, 4000 7852 -> 7806), wider rows only in parts of a wave, which wait for no other (4096 in 16
+  // parts, 1024 rows 16.6 -> 14.8, 4096 rows 43.4 -> 42.4; in 8, 1500 rows 18.7 -> 19.8; in 1, 1024 rows 15.1 -> 16.9, 4096 rows 40.4 -> 47.9; 2560 in 1, 1500 rows 14.1 -> 17.8).
+  const int gs = D / groups;      // (one wave and more)
+  if ((T <= 32 || (!conv && (T <= 512 || ld <= 2048 || gs == 256))) && (w_pre || as_is) && ld <= 4096 && ld == D && gs % 256 == 0 && (!conv || conv->taps <= 4)) {
 #define MI_TOKEN(TAPS) \
     if (f32) hipLaunchKernelGGL((sandwich_token_kernel<float, TAPS>), dim3(T, groups), dim3(gs / 4), 0, s, resid_in, resid_out, src, w_post, w_pre, D, ld, gs, eps, cs, (float*)y, ldy); \
     else hipLaunchKernelGGL((sandwich_token_kernel<uint16_t, TAPS>), dim3(T, groups), dim3(gs / 4), 0, s, resid_in, resid_out, src, w_post, w_pre, D, ld, gs, eps, cs, (uint16_t*)y, ldy)
