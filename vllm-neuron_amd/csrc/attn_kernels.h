@@ -21,6 +21,7 @@ size_t attn_scratch_bytes(int B, int nh, int hd);
 
 // launch_attn_decode of B rows and launch_attn_prefill of one sequence's T tokens in one launch (their outputs and partials are apart); scratch as launch_attn_decode's with tickets_zeroed
 struct AttnMixed { const uint16_t* q; const int32_t* block_table; const int32_t* ctx_lens; int MB, B, max_ctx, num_blocks; uint16_t* out; void* scratch; };
+int attn_mixed_lds(int hd, int kh, int splits);   // bytes its launch asks for: kh waves a head of the prompt's, splits of a request's context
 int launch_attn_mixed(const AttnMixed& m, int T, int q_pos0, const uint16_t* q, const int32_t* block_table, uint16_t* out, const uint16_t* kpool, const uint16_t* vpool,
                       int block_size, int nh, int nkv, int hd, hipStream_t s, float* ws, size_t ws_bytes);
 // whether a grid too short for the chip still takes each (sequence, kv head) in one work-group, without partials: short contexts

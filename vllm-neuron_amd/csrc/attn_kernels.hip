@@ -67,8 +67,8 @@ constexpr int kNt = 2;   // a buffer load's `nt`: lines nobody reads again
 // work-group whose ticket is NS - 1 reads all NS partials back with sc1 loads (past its L1; no
 // other reader of these lines exists in the launch, so no L2 holds a stale copy) and writes the
 // bf16 output.  No fence is needed: the work-group whose add came last is told so by
-// the value its add returned, and there is one work-group per CU (the launch pads its LDS request to
-// keep it so).  The merge itself runs in split order, so the
+// the value its add returned, and there is one work-group per CU (the launches that merge ask for
+// kMergeLds of LDS to keep it so).  The merge itself runs in split order, so the
 // result does not depend on which work-group performs it.  The counter is left at 0 for the next launch.
 template <int HD, int NW, bool FINAL, bool MERGE = false>
 __device__ __forceinline__ void attn_decode_body(
@@ -332,6 +332,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(
 }
 template <int HD, int NW>
 constexpr size_t attn_decode_lds() { return (size_t)NW * 32 * (HD + 8) * 2 + (size_t)NW * 16 * 2 * sizeof(float); }
+constexpr size_t kMergeLds = 96 * 1024;   // of a launch that merges: more than half a CU's LDS, so that no two of its work-groups share a CU
 
 // Merge the context splits of one (sequence, head) in split order.  All partials are
 // fetched before the first use (kAttnMaxSplits is a compile-time bound), so the kernel is
@@ -404,7 +405,6 @@ static int launch_decode_t(const uint16_t* q, const uint16_t* kpool, const uint1
   float* o_part = ml_part + (size_t)B * nh * kAttnMaxSplits * 2;
   const float scale_log2e = 1.4426950408889634f / sqrtf((float)HD);
   constexpr size_t lds8 = attn_decode_lds<HD, 8>(), lds4 = attn_decode_lds<HD, 4>();
-  constexpr size_t kMergeLds = 96 * 1024;   // more than half a CU's LDS: one work-group per CU (see the kernel comment)
   {
     int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(attn_decode_kernel<HD, 8, true>), (int)lds8);
     if (rc == MI_OK) rc = ensure_dynamic_lds(reinterpret_cast<const void*>(attn_decode_kernel<HD, 4, true>), (int)lds4);
@@ -1262,9 +1262,15 @@ int launch_attn_prefill(const uint16_t* q, int T, int q_pos0, const uint16_t* kp
 // ones, twice the other's limit.  us per call, splits -> none: 8B fp8 239 + 3 of 250 tokens 2977 -> 2940, of 500 2974 -> 2988, of 1000 2979 -> 3114; 64 + 6 of 300
 // 2177 -> 2145, of 600 2197 -> 2215; TinyLlama 300 + 4 of 500 2234 -> 2178, of 1000 2228 -> 2296.
 // Splits are merged in this launch by whichever ends last (MERGE): what that takes is hidden by the prompt's work-groups, where a launch of one's own behind both was in line.  A work-group has its CU
-// to itself (two waves a SIMD).  us a call, combine launch -> merged: 8B fp8 239 + 3 2649 -> 2617 (a layer 10.6 + 4.7 -> 12.2), 64 + 6 1939 -> 1922, 500 + 1 3971 -> 3916, TinyLlama 300 + 4 1991 -> 1960,
+// to itself (kMergeLds; two waves a SIMD).  us a call, combine launch -> merged: 8B fp8 239 + 3 2649 -> 2617 (a layer 10.6 + 4.7 -> 12.2), 64 + 6 1939 -> 1922, 500 + 1 3971 -> 3916, TinyLlama 300 + 4 1991 -> 1960,
 // 7B int8 200 + 3 2515 -> 2506.
 static int mixed_splits(const AttnMixed& m, int nkv, int hd) { return m.max_ctx > 0 && m.max_ctx * hd <= 256 * 128 ? 1 : ceil_div(attn_decode_splits(m.B, nkv), 2); }
+template <int HD>
+static int mixed_lds(int kh, int splits) {
+  const int need = std::max<int>(kh == 2 ? attn_prefill2_lds<HD, 8, 2>() : attn_prefill2_lds<HD, 8, 1>(), (int)attn_decode_lds<HD, 8>());
+  return splits > 1 ? std::max<int>(need, kMergeLds) : need;
+}
+int attn_mixed_lds(int hd, int kh, int splits) { return hd == 128 ? mixed_lds<128>(kh, splits) : mixed_lds<64>(kh, splits); }
 template <int HD>
 static int launch_mixed_t(const AttnMixed& m, const PrefillPlan& p, int T, int q_pos0, const uint16_t* q, const int32_t* bt, uint16_t* out, const uint16_t* kpool,
                           const uint16_t* vpool, int bs, int nh, int nkv, hipStream_t s) {
@@ -1273,7 +1279,7 @@ static int launch_mixed_t(const AttnMixed& m, const PrefillPlan& p, int T, int q
   float* o_part = ml_part + (size_t)m.B * nh * kAttnMaxSplits * 2;
   const int NS = mixed_splits(m, nkv, HD);
   const DecodeSide d{m.q, m.block_table, m.ctx_lens, m.MB, NS, NS * m.B, m.num_blocks, o_part, ml_part, m.out, reinterpret_cast<unsigned int*>(m.scratch)};
-  const int lds = std::max<int>(p.kh == 2 ? attn_prefill2_lds<HD, 8, 2>() : attn_prefill2_lds<HD, 8, 1>(), (int)attn_decode_lds<HD, 8>());
+  const int lds = attn_mixed_lds(HD, p.kh, NS);
   const auto fn = p.kh == 2 ? (NS == 1 ? attn_mixed_kernel<HD, 2, true> : attn_mixed_kernel<HD, 2, false>)
                             : (NS == 1 ? attn_mixed_kernel<HD, 1, true> : attn_mixed_kernel<HD, 1, false>);
   MI_TRY_A(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds));
