@@ -279,7 +279,7 @@ int launch_gemv_regs_wd(const LinearW& w, int M, const uint16_t* x, int ldx, int
   // (where the norm behind is left to its projection, an unsplit K saves that norm's launch: 4.7 us against the 0.3 - 1 that half-empty CUs cost)
   const int slices = e.next_x ? 1 : gemv_regs_slices<WD>(M, w.N, w.K, ws ? ws_bytes : 0, deferred || split_as_deferred, num_cu);
   MI_CHECK(slices > 0, "gemv_regs: no split of K fits the workspace");
-  MI_CHECK(!e.next_x || (epi == EPI_RESID && M <= 16 && gemv_regs_holds(w)), "gemv_regs: a norm handed on is for residuals of up to 16 rows, K in one slice");
+  MI_CHECK(!e.next_x || (epi == EPI_RESID && e.ld_out == w.N && M <= 16 && gemv_regs_holds(w)), "gemv_regs: a norm handed on is for residuals of up to 16 rows side by side, K in one slice");
   MI_CHECK(epi != EPI_RESID || !e.row_scale || slices > 1, "gemv_regs: no residual takes a factor a row");
   MI_CHECK(e.rs_n == 0.f || e.rs_parts == kNormParts || (M <= 16 && slices == 1 && e.rs_parts % 4 == 0 && e.rs_parts > 0 && e.rs_parts <= 256), "gemv_regs: a norm's parts");
   if (slices > 1) {

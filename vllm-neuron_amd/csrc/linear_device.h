@@ -40,7 +40,7 @@ __device__ __forceinline__ void epilogue(const EpiArgs& e, int m, int n0, f32x4_
 }
 
 // The residual stream's new numbers, columns n0 .. n0 + 3 of row m, and what the norm behind would make of them where it is handed on (EpiArgs::next_x).  The four lanes c, c + 16,
-// c + 32, c + 48 of a wave hold the 16 columns of a row-tile.  Only the weight-streaming kernels come here.
+// c + 32, c + 48 of a wave hold the 16 columns of a row-tile: so it is in the weight-streaming kernels, whose launches alone take next_x (splitk_reduce_kernel comes here without).
 __device__ __forceinline__ void put_resid(const EpiArgs& e, int m, int n0, float4 r, f32x4_t v, float4 ga) {
   const float4 o = make_float4(r.x + v[0], r.y + v[1], r.z + v[2], r.w + v[3]);
   *reinterpret_cast<float4*>(e.out_f32 + (size_t)m * e.ld_out + n0) = o;

@@ -110,6 +110,7 @@ bool gemv_fits(int M, int K) { (void)K; return gemv_rows_fit(M); }
 
 int launch_gemv(const LinearW& w, int M, int pro, const ProArgs& p, int epi, const EpiArgs& e, hipStream_t s) {
   MI_CHECK(M >= 1 && M <= 16, "gemv: M must be 1..16");
+  MI_CHECK(!e.next_x || (epi == EPI_RESID && e.ld_out == w.N), "gemv: a norm handed on is for residuals, rows side by side");
   MI_CHECK(w.N % 16 == 0 && w.K % 64 == 0, "gemv: N % 16 == 0 and K % 64 == 0 required");
   switch (w.wd) {
     case MI_W_BF16: return launch_gemv_wd<MI_W_BF16>(w, M, pro, p, epi, e, s);
@@ -396,6 +397,7 @@ static bool gemm_wide_wanted(const LinearW& w, int T, size_t ws_bytes) {
 int launch_gemm_wide(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
                      float* splitk_ws, size_t splitk_ws_bytes, SlabSum* defer, bool split_as_deferred, int force_bm, int force_ntw, int force_ks) {
   if (defer) *defer = SlabSum();
+  MI_CHECK(!e.next_x, "gemm_wide: hands no norm on");
   MI_CHECK(w.K % 64 == 0 && ldx % 8 == 0, "gemm_wide: K % 64 == 0");
   WidePlan pl = gemm_wide_plan(T, w.N, w.K, gemm_wide_ks() == 1 || !splitk_ws ? 0 : splitk_ws_bytes, w.wd, split_as_deferred || (defer && (epi == EPI_RESID || epi == EPI_F32)));
   const int forced_bm = force_bm ? force_bm : gemm_wide_bm();
@@ -413,6 +415,7 @@ int launch_gemm_wide(const LinearW& w, int T, const uint16_t* x, int ldx, int ep
 int launch_gemm(const LinearW& w, int T, const uint16_t* x, int ldx, int epi, const EpiArgs& e, hipStream_t s,
                 float* splitk_ws, size_t splitk_ws_bytes, SlabSum* defer, bool split_as_deferred) {
   if (defer) *defer = SlabSum();
+  MI_CHECK(!e.next_x, "gemm: hands no norm on");
   if (e.far_out) {      // (nothing here stores through L2)
     EpiArgs near = e;
     near.far_out = false;
@@ -715,6 +718,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 // (Sums for the host stay in L2: a wave stores 1 KiB of a row with one request, which gains nothing by being stored through and waits.  24 rows of 32000 words, bf16 5120 deep:
 //  56.8 us, 60.0 through)
 int launch_splitk_reduce(const SlabSum& sl, int epi, const EpiArgs& args, hipStream_t s) {
+  MI_CHECK(!args.next_x, "splitk_reduce: hands no norm on");      // (its lanes hold other columns than put_resid adds up)
   EpiArgs e = args;
   e.far_out = false;
   const dim3 grid(ceil_div(sl.T * (sl.N / 4), 256));
@@ -746,6 +750,7 @@ bool gemm_a8_supported(const LinearW& w) {
 int launch_gemm_a8(const LinearW& w, int T, const uint8_t* x8, int ldx, int epi, const EpiArgs& e, hipStream_t s,
                    float* splitk_ws, size_t splitk_ws_bytes, SlabSum* defer) {
   if (defer) *defer = SlabSum();
+  MI_CHECK(!e.next_x, "gemm_a8: hands no norm on");
   MI_CHECK(e.rs_n == 0.f, "gemm_a8: no rows with the parts of a norm");
   MI_CHECK(T >= 1, "gemm_a8: T must be >= 1");
   MI_CHECK(gemm_a8_supported(w), "gemm_a8: needs fp8 weights, K % 128 == 0, N % 16 == 0");
