@@ -162,55 +162,59 @@ def test_fp8_activations_stay_with_prompts(rows):
     assert torch.equal(*out)
 
 
-# logits of 17 and more rows to the host: single row-tiles, and from 8192 rows on (two of them a CU) four side by side: a last group of one, two, three and four, one and several a work-group
-@pytest.mark.parametrize("vocab", [16, 80, 1024, 16448, 8176, 8208, 8224, 12272])
+def _logits_to_the_host(shape, wd, rows_of, max_rows=32):
+    """Logits of the first step of a one-layer model, per number of rows, against the oracle at the bar of the other dispatch tests (a row-tile or a row in another place is off by the
+    spread itself)."""
+    from oracle import DecoderConfig, PagedDecoderOracle
+    from oracle.synth import make_weights
+    from tests.helpers import decode_inputs
+    from vllm_neuron_amd._native import MI_Q, MI_W, NativeModel
+    cfg, vocab = DecoderConfig(**shape), shape["vocab_size"]
+    w = make_weights(cfg, seed=4)
+    model = NativeModel(**shape, rms_norm_eps=cfg.rms_norm_eps, rope_theta=cfg.rope_theta, rope_type=0, rope_factor=1.0, num_blocks=33, block_size=32, max_num_seqs=max_rows,
+                        max_model_len=32, weight_dtype=MI_W[wd], quant_type=MI_Q["per_channel_symmetric"], quantize_lm_head=1, tp_degree=1, tp_rank=0,
+                        device_id=0, use_graphs=1, ctx_buckets=[32])
+    model.load_state_dict(w)
+    model.finalize()
+    inputs = {rows: decode_inputs([i % vocab for i in range(rows)], [0] * rows, [[1 + i] for i in range(rows)], 32, 32) for rows in rows_of}
+    want = PagedDecoderOracle(cfg, w, 33, 32, compute="bf16", quant=_quant(wd)).forward(**inputs[max(rows_of)]).float()
+    out = {}
+    for rows, x in inputs.items():
+        for _ in range(2):         # eager pass, then the graph
+            out[rows] = model.forward(**x).clone()
+            d = out[rows] - want[:rows]
+            assert torch.isfinite(d).all() and d.pow(2).mean().sqrt() < 0.02 * want.std() and d.abs().max() < 0.1 * want.std(), (wd, rows)
+    model.close()
+    return out
+
+
+# logits of 16 and more rows to the host: single row-tiles, and from 8192 rows on (two of them a CU) four side by side: a last group of one, two, three and four, one and several a work-group
+@pytest.mark.parametrize("vocab", [16, 80, 1024, 16448, 8176, 8192, 8208, 8224, 12272])
 def test_logits_of_many_rows_to_the_host(vocab):
-    from oracle import DecoderConfig
-    from oracle.synth import make_weights
-    from tests.helpers import decode_inputs
-    from vllm_neuron_amd._native import MI_Q, MI_W, NativeModel
     shape = dict(num_layers=1, hidden_size=128, num_heads=2, num_kv_heads=1, head_dim=64, intermediate_size=256, vocab_size=vocab)
-    w = make_weights(DecoderConfig(**shape), seed=4)
-    for wd in ("bf16", "f8e4m3"):
-        model = NativeModel(**shape, rms_norm_eps=1e-5, rope_theta=1e4, rope_type=0, rope_factor=1.0, num_blocks=33, block_size=32, max_num_seqs=32,
-                            max_model_len=32, weight_dtype=MI_W[wd], quant_type=MI_Q["per_channel_symmetric"], quantize_lm_head=1, tp_degree=1, tp_rank=0,
-                            device_id=0, use_graphs=1, ctx_buckets=[32])
-        model.load_state_dict(w)
-        model.finalize()
-        out = {}
-        for rows in (16, 17, 32):
-            for _ in range(2):         # eager pass, then the graph
-                out[rows] = model.forward(**decode_inputs([i % vocab for i in range(rows)], [0] * rows, [[1 + i] for i in range(rows)], 32, 32)).clone()
-        # the same sums over K a row-tile, whoever stores them; the projections in front differ in low bits between 16 and 17 rows, as between any two kernels
-        std = out[32].std().item()
-        assert torch.isfinite(out[32]).all() and torch.equal(out[17], out[32][:17]) and (out[16] - out[32][:16]).abs().max().item() < 0.05 * std
-        model.close()
-
-
-# logits of 5 to 16 rows to the host, four row-tiles side by side from 8192 rows on: a last group of four, one, two and three.  The bar is that of the test above: the rows' first
-# 4 come from another kernel, and a row is the same however many stand beside it
-@pytest.mark.parametrize("vocab", [8176, 8192, 8208, 8224, 12272])
-def test_logits_of_few_rows_to_the_host(vocab):
-    from oracle import DecoderConfig
-    from oracle.synth import make_weights
-    from tests.helpers import decode_inputs
-    from vllm_neuron_amd._native import MI_Q, MI_W, NativeModel
-    shape = dict(num_layers=1, hidden_size=192, num_heads=3, num_kv_heads=1, head_dim=64, intermediate_size=256, vocab_size=vocab)
-    w = make_weights(DecoderConfig(**shape), seed=4)
     for wd in ("bf16", "f8e4m3", "int8"):
-        model = NativeModel(**shape, rms_norm_eps=1e-5, rope_theta=1e4, rope_type=0, rope_factor=1.0, num_blocks=33, block_size=32, max_num_seqs=16,
-                            max_model_len=32, weight_dtype=MI_W[wd], quant_type=MI_Q["per_channel_symmetric"], quantize_lm_head=1, tp_degree=1, tp_rank=0,
-                            device_id=0, use_graphs=1, ctx_buckets=[32])
-        model.load_state_dict(w)
-        model.finalize()
-        out = {}
-        for rows in (4, 5, 11, 16):
-            for _ in range(2):         # eager pass, then the graph
-                out[rows] = model.forward(**decode_inputs([i % vocab for i in range(rows)], [0] * rows, [[1 + i] for i in range(rows)], 32, 32)).clone()
-        std = out[16].std().item()
-        assert torch.isfinite(out[16]).all() and torch.equal(out[5], out[16][:5]) and torch.equal(out[11], out[16][:11])
-        assert (out[4] - out[16][:4]).abs().max().item() < 0.05 * std
-        model.close()
+        out = _logits_to_the_host(shape, wd, (16, 17, 32))
+        # the same sums over K a row-tile, however many rows stand beside it; the projections in front differ in low bits between 16 and 17 rows, as between any two kernels
+        assert torch.equal(out[17], out[32][:17]) and (out[16] - out[32][:16]).abs().max() < 0.05 * out[32].std()
+
+
+# logits of up to 16 rows to the host: K so shallow that all go in groups of four row-tiles, and so deep that the line between those and single ones (rows * 540 >= bytes of a weight row) lies
+# between 5 and 6 rows (bf16: 11 and 12); a last group of four, one, two and three, and below two row-tiles a CU
+@pytest.mark.parametrize("vocab", [8176, 8192, 8208, 8224, 12272])
+@pytest.mark.parametrize("hidden", [192, 3072])
+def test_logits_of_few_rows_to_the_host(hidden, vocab):
+    shape = dict(num_layers=1, hidden_size=hidden, num_heads=3, num_kv_heads=1, head_dim=64, intermediate_size=256, vocab_size=vocab)
+    for wd in ("bf16", "f8e4m3", "int8"):
+        out = _logits_to_the_host(shape, wd, (4, 5, 6, 11, 12, 16), 16)
+        # single tiles and four have the same sums over K; the projections in front split theirs by the number of rows (bf16 3072 deep from 10 on)
+        assert torch.equal(out[5], out[6][:5]) and torch.equal(out[11], out[12][:11])
+        assert all((out[rows] - out[16][:rows]).abs().max() < 0.05 * out[16].std() for rows in out)
+
+
+# ... and where they are sums of K slices
+@pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
+def test_logits_of_slices_to_the_host(wd):
+    _logits_to_the_host(dict(num_layers=1, hidden_size=4224, num_heads=4, num_kv_heads=1, head_dim=64, intermediate_size=256, vocab_size=8208), wd, (4, 5, 16, 17, 32))
 
 
 def _rapodra_of_many_words():
