@@ -261,6 +261,29 @@ def test_collective_path_single_rank_equals_fused_path():
         assert torch.equal(a, b)
 
 
+# ... for every weight type, where norms are handed on (up to 16 rows) and where they are not: widths of 12 to 256 parts of a norm, down projections that keep K in one piece and some that do not,
+# a width whose next projection splits K
+@pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
+@pytest.mark.parametrize("hidden,inter", [(192, 320), (2048, 4096), (2112, 4160), (4096, 1024), (4160, 512), (1024, 19008), (512, 33024)])
+def test_one_rank_gives_the_bits_of_none(wd, hidden, inter):
+    from vllm_neuron_amd._native import MI_Q, MI_W, NativeModel
+    from tests.helpers import decode_inputs
+    outs = []
+    for with_comm in (False, True):
+        m = NativeModel(num_layers=2, hidden_size=hidden, num_heads=4, num_kv_heads=2, head_dim=64, intermediate_size=inter, vocab_size=528, rms_norm_eps=1e-5, rope_theta=1e4, rope_type=0,
+                        rope_factor=1.0, num_blocks=34, block_size=32, max_num_seqs=32, max_model_len=32, weight_dtype=MI_W[wd], quant_type=MI_Q["per_channel_symmetric"],
+                        quantize_lm_head=1, tp_degree=1, tp_rank=0, device_id=0, use_graphs=0)
+        if with_comm:
+            m.tp_init(m.tp_unique_id())
+        m.init_synthetic_weights(7, 0.05)
+        m.finalize()
+        outs.append({(rows, at): m.forward(**decode_inputs([(31 * i + 7 * at) % 528 for i in range(rows)], [at] * rows, [[1 + i] for i in range(rows)], 32, 32)).clone()
+                     for rows in (1, 2, 4, 5, 12, 16, 17, 32) for at in range(2)})
+        m.close()
+    wrong = [k for k in outs[0] if not torch.isfinite(outs[0][k]).all() or not torch.equal(outs[0][k], outs[1][k])]
+    assert not wrong, wrong
+
+
 def test_in_launch_attention_merge_matches_oracle():
     """MI355X_ATTN_MERGE=1: the context splits of decode attention are merged by the last
     work-group to finish instead of a combine launch (off by default: measured slower).  The
