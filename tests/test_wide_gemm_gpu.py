@@ -227,7 +227,11 @@ def test_sums_of_slices_round_once(lib, M, N, K, ks):
     assert ((y.cpu().double() - ref).abs() <= 0.50001 * unit).all()
 
 
-# slabs of 24 MiB (written through), one row more than that, and twice as much, whole token blocks and a short last one
-@pytest.mark.parametrize("M,N,K,bm,ntw,ks", [(1024, 2048, 128, 128, 2, 3), (1025, 2048, 192, 128, 3, 3), (2048, 2064, 192, 256, 4, 3), (1024, 3072, 128, 256, 4, 2)])
-def test_slabs_left_in_l2_and_written_through(lib, M, N, K, bm, ntw, ks):
-    check_tile(lib, "bf16", bm, ntw, ((M, N, K, min(ks, K // 64)),))
+# slabs of 24 MiB (written through) and one row more than that, in two and three slices; twice as much; whole token blocks and a short last one.  Weights of four times the slabs (through) and 64 of K more,
+# in bf16 and in a byte
+@pytest.mark.parametrize("wd", ["bf16", "f8e4m3", "int8"])
+@pytest.mark.parametrize("M,N,K,bm,ntw,ks", [(1024, 2048, 192, 128, 2, 3), (1025, 2048, 192, 128, 3, 3), (1024, 3072, 128, 256, 4, 2), (1025, 3072, 128, 192, 4, 2), (2048, 2064, 192, 256, 4, 3),
+                                             (32, 528, 512, 64, 2, 2), (32, 528, 576, 64, 3, 2), (32, 528, 1024, 64, 4, 2), (32, 528, 1088, 96, 2, 2), (48, 272, 1152, 64, 2, 3), (48, 272, 1216, 64, 2, 3),
+                                             (48, 272, 2304, 64, 3, 3), (48, 272, 2368, 64, 3, 3)])
+def test_slabs_left_in_l2_and_written_through(lib, wd, M, N, K, bm, ntw, ks):
+    check_tile(lib, wd, bm, ntw, ((M, N, K, ks),))
