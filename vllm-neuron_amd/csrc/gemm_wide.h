@@ -39,7 +39,7 @@ __device__ __forceinline__ void wait_dma(int left) {
 
 // What a work-group needs in front of its first request, in one line of kernel arguments and taken in one go (wide_args): a kernel's arguments come from memory, and hipcc fetches
 // each where it is first used.  Divisions are the host's.  (A work-group took 1.6 - 3.1 us to the
-// last request of its ring.)  us a launch, before -> now: int8 188 x 4608 in 3 slices 14.2 -> 13.6, x 3584 in 4 12.1 -> 11.6, 18944 deep in 8 33.0 -> 32.4; calls of 32 .. 1000 tokens 0.8 - 1.3 %.
+// last request of its ring.)  us a launch, before -> now: int8 188 x 4608 in 3 slices 14.2 -> 13.6, x 3584 in 4 12.1 -> 11.6, 18944 deep in 8 33.0 -> 32.4; calls of 32 .. 250 rows 0.8 - 1.3 %, of 1000 tokens and more nothing.
 struct WideArgs {
   const uint4* W;
   const uint16_t* x;

@@ -291,7 +291,7 @@ int launch_gemv_regs_wd(const LinearW& w, int M, const uint16_t* x, int ldx, int
   // (Logits to the host in groups of four row-tiles where their way, in pieces of 64 bytes, takes as long as the weights do or nearly so; below, single row-tiles deal the weights out more evenly.
   //  Steps of half-depth models, us, single -> four: 8B fp8 6 rows 1123 -> 1121, 9 1199 -> 1188, 16 1403 -> 1382, bf16 5 rows 1710 -> 1714, 12 1839 -> 1856, 14 1870 -> 1877, 16 1940 -> 1919,
   //  7B bf16 12 rows 1665 -> 1668, 14 1714 -> 1686, int8 5 rows 1029 -> 1030, 8 1095 -> 1085, 12 1207 -> 1179, 2048 wide 6 rows 522 -> 522, 16 591 -> 585; groups of two gain half of that.
-  //  Not where less than half of the CUs would have a group: us a launch, 20 - 27 rows, 2048 and 4096 wide, single row-tiles and four: 16384 rows of logits 52.9 and 46.4, 8192 29.5 and 27.2,
+  //  From 17 rows on all of K that the registers hold (4096) lies above.  Not where less than half of the CUs would have a group: us a launch, 20 - 27 rows, 2048 and 4096 wide, single row-tiles and four: 16384 rows of logits 52.9 and 46.4, 8192 29.5 and 27.2,
   //  fp8 26.4 and 25.8, 4096 21.2 and 24.8)
   const bool four = M * 540 >= w.K * (WD == MI_W_BF16 ? 2 : 1) && w.N / 16 >= 2 * num_cu;
 #define MI_R4(EPI_) return M <= 16 ? launch_gemv_regs_k<WD, EPI_, 1, false, 4>(w, M, x, ldx, e, s, 1, nullptr) : launch_gemv_regs_k<WD, EPI_, 2, false, 4>(w, M, x, ldx, e, s, 1, nullptr)
