@@ -302,8 +302,9 @@ int launch_gemv_regs_wd(const LinearW& w, int M, const uint16_t* x, int ldx, int
   }
 #undef MI_R4
   // (Far results are stored through: left in L2 they cross PCIe when the weights are done.  Steps of half-depth models, us: 8B fp8 4 rows 1116 -> 1095, 8 rows 1147 -> 1120,
-  //  16 rows 1299 -> 1288, 7B int8 5 rows 1138 -> 1088, 2048 wide 2 - 16 rows 0.2 - 3 %; groups of four, 8B fp8 9 rows 1230 -> 1188, 32 rows 1790 -> 1768.  Not single row-tiles of 17 and more rows:
-  //  PCIe bounds them, and the L2 puts some of their pieces together, 24 rows of 8B 1535 through)
+  //  16 rows 1299 -> 1288, 7B int8 5 rows 1138 -> 1088, 2048 wide 2 - 16 rows 0.2 - 3 %; groups of four, 8B fp8 9 rows 1230 -> 1188, 32 rows 1790 -> 1768.  Single row-tiles of 17 and more rows, which only heads of
+  //  less than two a CU have, are still left in L2; what going through would give there is little: one layer, 24 rows, left -> through, 4096 wide and 8000 words bf16 101.3 -> 96.6, fp8 103.3 -> 101.6,
+  //  4096 words 88.8 -> 87.7 and 92.3 -> 92.7, 2048 wide and 4096 words 82.5 -> 81.6 and 83.2 -> 83.3)
   EpiArgs near = e;
   near.far_out = false;
 #define MI_R(EPI_) return M <= 16 ? launch_gemv_regs_k<WD, EPI_, 1, false>(w, M, x, ldx, e, s, 1, nullptr) : launch_gemv_regs_k<WD, EPI_, 2, false>(w, M, x, ldx, near, s, 1, nullptr)
